@@ -598,10 +598,206 @@ __global__ __launch_bounds__(256) void resize_aa_v_kernel(const float* __restric
   dst[i] = (uint8_t)rintf(acc);                 // [T][3][Hout][Wout]
 }
 
+// Both passes in one launch over output tiles of 64 columns x TH rows x 3 channels: the source window of a tile is staged in LDS by aligned
+// dwords, the width pass leaves its fp32 rows in LDS, the height pass reads them there.  Same products in the same order as the two kernels
+// above, so the same bytes.  Bound by vector instructions and the latency of a tile's three stages, not by bytes (a 720p pair is 5.5 MB in,
+// 1.7 MB out).  The two launches spent 18.9 us on byte-wise global loads of the width pass (27 per output column) and 14.4 us on the height
+// pass over an fp32 tensor of 12.6 MB that nothing else reads.  Here a lane owns a column and keeps its K weights (zero behind its own count)
+// in registers for all rows of the tile, its 3 K source bytes are K dword reads shifted into place, and the height pass takes four columns a
+// lane.  Two 720p frames to 392 x 728: 33.3 -> 11.6 us (rows x channels one column a lane: 15.9); two of 300 x 500: 15 -> 9.6; 24 of
+// 1080p to 280 x 504 (17 taps, half of a tile's rows are its neighbour's too): 391 -> 138.
+// The tables are the caller's: a tile whose window does not fit what the host sized from the scale is computed tap by tap (same values).
+constexpr int RS_COLS = 64;
+constexpr int RS_WAVES = 8;
+constexpr int RS_LDS_MAX = 80 * 1024;          // two blocks on a compute unit
+template <int K, bool PLANAR>
+__global__ __launch_bounds__(RS_WAVES * 64) void resize_aa_tile_kernel(const uint8_t* __restrict__ src, int T, int Hin, int Win, uint8_t* __restrict__ dst,
+                                                             int Hout, int Wout, const int32_t* __restrict__ xmin,
+                                                             const int32_t* __restrict__ xsize, const float* __restrict__ wx,
+                                                             const int32_t* __restrict__ ymin, const int32_t* __restrict__ ysize,
+                                                             const float* __restrict__ wy, int ky, int TH, int rows_cap, int seg_dw) {
+  constexpr int PX = PLANAR ? 1 : 3, NSEG = PLANAR ? 3 : 1;       // bytes from a pixel to the next; staged pieces of a source row
+  extern __shared__ __attribute__((aligned(16))) float wrow[];    // [TH][ky up to 4s], then mid [rows_cap][3][64], then the pieces [rows_cap * NSEG][seg_dw]
+  __shared__ int tap0[16], taps[16];
+  float* mid = wrow + TH * ((ky + 3) & ~3);
+  unsigned* raw = reinterpret_cast<unsigned*>(mid + (size_t)rows_cap * 3 * RS_COLS);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tiles_x = (Wout + RS_COLS - 1) / RS_COLS, tiles_y = (Hout + TH - 1) / TH;
+  const int tx = blockIdx.x % tiles_x, ty = (blockIdx.x / tiles_x) % tiles_y, t = blockIdx.x / (tiles_x * tiles_y);
+  const int y0t = ty * TH, nrow = min(TH, Hout - y0t);
+  const int xo = min(tx * RS_COLS + lane, Wout - 1), yl = y0t + min(lane, nrow - 1);
+  const int x0 = xmin[xo], n = xsize[xo], yy = ymin[yl], yn = ysize[yl];
+  int lo = x0, hi = x0, nmax = n, nymax = yn, rlo = yy, rhi = yy + max(yn, 1);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = min(lo, __shfl_xor(lo, o, 64)); hi = max(hi, __shfl_xor(hi, o, 64)); nmax = max(nmax, __shfl_xor(nmax, o, 64)); nymax = max(nymax, __shfl_xor(nymax, o, 64));
+    rlo = min(rlo, __shfl_xor(rlo, o, 64)); rhi = max(rhi, __shfl_xor(rhi, o, 64));
+  }
+  lo = __builtin_amdgcn_readfirstlane(lo); hi = __builtin_amdgcn_readfirstlane(hi); nmax = __builtin_amdgcn_readfirstlane(nmax); nymax = __builtin_amdgcn_readfirstlane(nymax);
+  rlo = __builtin_amdgcn_readfirstlane(rlo); rhi = __builtin_amdgcn_readfirstlane(rhi);
+  const int cols = hi - lo + K, rows = rhi - rlo;
+  const uint8_t* frame = src + (size_t)t * 3 * Hin * Win;
+  const size_t plane = (size_t)Hin * Win;
+  const bool live = tx * RS_COLS + lane < Wout;
+  if (rows > rows_cap || nymax > ky || nymax < 1 || cols * PX + 8 > seg_dw * 4 || nmax > K) {      // block-uniform: every wave reduced the same values
+    for (int it = wave; it < nrow * 3; it += RS_WAVES) {
+      const int yo = y0t + it / 3, c = it - it / 3 * 3, ys = ymin[yo], ny = ysize[yo];
+      float acc = 0.f;
+      for (int i = 0; i < max(ny, 1); ++i) {
+        const uint8_t* p = PLANAR ? frame + c * plane + (size_t)(ys + i) * Win + x0 : frame + ((size_t)(ys + i) * Win + x0) * 3 + c;
+        float h = __fmul_rn((float)p[0], wx[xo]);
+        for (int j = 1; j < n; ++j) h = fmaf((float)p[j * PX], wx[(size_t)j * Wout + xo], h);
+        const float w = wy[(size_t)yo * ky + i];
+        acc = i == 0 ? __fmul_rn(h, w) : fmaf(h, w, acc);
+      }
+      if (live) dst[(((size_t)t * 3 + c) * Hout + yo) * Wout + xo] = (uint8_t)rintf(fminf(fmaxf(acc, 0.f), 255.f));
+    }
+    return;
+  }
+  float w[K];
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    const float f = wx[(size_t)j * Wout + xo];
+    w[j] = (j == 0 || j < n) ? f : 0.f;                   // a tap behind the count adds 0 x byte: exact
+  }
+  // source window -> LDS.  A piece starts at the dword that holds its first byte and ends with the one that holds its last: every dword read
+  // shares its word with a byte of the picture.
+  const int nbytes = (min(lo + cols, Win) - lo) * PX, nseg = rows * NSEG;
+  auto piece = [&](int sg) { return PLANAR ? frame + (sg % 3) * plane + (size_t)(rlo + sg / 3) * Win + lo : frame + ((size_t)(rlo + sg) * Win + lo) * 3; };
+  for (int d0 = 0; d0 < seg_dw; d0 += 128)
+    for (int s0 = wave; s0 < nseg; s0 += 8 * RS_WAVES) {
+      unsigned v[8][2];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {                       // sixteen loads in flight per wave, clamped instead of predicated: a 720p tile arrives
+        const uint8_t* p = piece(min(s0 + RS_WAVES * q, nseg - 1));          // in one round trip
+        const unsigned sh = (unsigned)((uintptr_t)p & 3);
+        const unsigned* pw = reinterpret_cast<const unsigned*>(p - sh);
+        const int last = ((int)sh + nbytes - 1) >> 2;
+        v[q][0] = pw[min(d0 + lane, last)];
+        v[q][1] = pw[min(d0 + lane + 64, last)];
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int sg = s0 + RS_WAVES * q;
+        if (sg < nseg) {
+          if (d0 + lane < seg_dw) raw[sg * seg_dw + d0 + lane] = v[q][0];
+          if (d0 + lane + 64 < seg_dw) raw[sg * seg_dw + d0 + lane + 64] = v[q][1];
+        }
+      }
+    }
+  // the height pass's weights, and where each row's taps begin and how many they are
+  const int kyp = (ky + 3) & ~3;
+  for (int i = threadIdx.x; i < nrow * kyp; i += RS_WAVES * 64) {
+    const int r = i / kyp, j = i - r * kyp;
+    wrow[i] = j < max(ysize[y0t + r], 1) ? wy[(size_t)(y0t + r) * ky + j] : 0.f;
+  }
+  if (wave == 0 && lane < nrow) { tap0[lane] = yy - rlo; taps[lane] = max(yn, 1); }
+#pragma unroll
+  for (int j = 0; j < K; ++j) asm volatile("" ::"v"(w[j]));          // the weights arrive under the staging, not behind it
+  __syncthreads();
+  for (int r = wave; r < rows; r += RS_WAVES) {
+    float a[3];
+    if constexpr (PLANAR) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const int b = (int)((uintptr_t)piece(r * 3 + c) & 3) + (x0 - lo);
+        const unsigned* p = raw + (r * 3 + c) * seg_dw + (b >> 2);
+        constexpr int ND = (K + 3) / 4;
+        unsigned d[ND + 1];
+#pragma unroll
+        for (int i = 0; i <= ND; ++i) d[i] = p[i];
+#pragma unroll
+        for (int i = 0; i < ND; ++i) d[i] = __builtin_amdgcn_alignbyte(d[i + 1], d[i], b & 3);
+        float f = __fmul_rn((float)(d[0] & 255u), w[0]);
+#pragma unroll
+        for (int j = 1; j < K; ++j) f = fmaf((float)((d[j >> 2] >> (8 * (j & 3))) & 255u), w[j], f);
+        a[c] = f;
+      }
+    } else {
+      const int b = (int)((uintptr_t)piece(r) & 3) + (x0 - lo) * 3;
+      const unsigned* p = raw + r * seg_dw + (b >> 2);
+      constexpr int ND = (3 * K + 3) / 4;
+      unsigned d[ND + 1];
+#pragma unroll
+      for (int i = 0; i <= ND; ++i) d[i] = p[i];
+#pragma unroll
+      for (int i = 0; i < ND; ++i) d[i] = __builtin_amdgcn_alignbyte(d[i + 1], d[i], b & 3);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        float f = __fmul_rn((float)((d[0] >> (8 * c)) & 255u), w[0]);
+#pragma unroll
+        for (int j = 1; j < K; ++j) { const int e = 3 * j + c; f = fmaf((float)((d[e >> 2] >> (8 * (e & 3))) & 255u), w[j], f); }
+        a[c] = f;
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) mid[(r * 3 + c) * RS_COLS + lane] = a[c];
+  }
+  __syncthreads();
+  // four columns a lane, sixteen lanes a row and channel: one 16-byte read and four products per tap
+  const bool words = ((Wout & 3) | (int)((uintptr_t)dst & 3)) == 0;
+  for (int task = threadIdx.x; task < nrow * 48; task += RS_WAVES * 64) {
+    const int it = task >> 4, r = it / 3, c = it - r * 3, col = (task & 15) * 4, ny = taps[r];
+    const float* wr = wrow + r * kyp;
+    const float* p = mid + (tap0[r] * 3 + c) * RS_COLS + col;
+    f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int j0 = 0; j0 < nymax; j0 += 4) {
+      const f32x4 w4 = *reinterpret_cast<const f32x4*>(wr + j0);
+      f32x4 m[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) m[j] = *reinterpret_cast<const f32x4*>(p + min(j0 + j, ny - 1) * 3 * RS_COLS);      // behind the count: 0 x the last tap
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = fmaf(m[j][e], w4[j], acc[e]);
+    }
+    unsigned o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (unsigned)rintf(fminf(fmaxf(acc[e], 0.f), 255.f));      // the bicubic overshoot is clamped, then half to even
+    uint8_t* q = dst + (((size_t)t * 3 + c) * Hout + y0t + r) * Wout + tx * RS_COLS + col;
+    const int left = Wout - (tx * RS_COLS + col);
+    if (words) {
+      if (left > 0) *reinterpret_cast<unsigned*>(q) = o[0] | (o[1] << 8) | (o[2] << 16) | (o[3] << 24);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (e < left) q[e] = (uint8_t)o[e];
+    }
+  }
+}
+
+template <int K>
+static void launch_resize_tile(const uint8_t* src, int layout, int T, int Hin, int Win, uint8_t* dst, int Hout, int Wout, const int32_t* xmin,
+                               const int32_t* xsize, const float* wx, const int32_t* ymin, const int32_t* ysize, const float* wy, int ky, int TH,
+                               int rows_cap, int seg_dw, size_t lds, hipStream_t st) {
+  const dim3 grid((unsigned)((size_t)T * ((Hout + TH - 1) / TH) * ((Wout + RS_COLS - 1) / RS_COLS)));
+  static DeviceOnce attr_set;   // per instantiation
+  if (attr_set.first()) {
+    (void)hipFuncSetAttribute((const void*)resize_aa_tile_kernel<K, false>, hipFuncAttributeMaxDynamicSharedMemorySize, RS_LDS_MAX);
+    (void)hipFuncSetAttribute((const void*)resize_aa_tile_kernel<K, true>, hipFuncAttributeMaxDynamicSharedMemorySize, RS_LDS_MAX);
+  }
+  if (layout == 0)
+    resize_aa_tile_kernel<K, false><<<grid, dim3(RS_WAVES * 64), lds, st>>>(src, T, Hin, Win, dst, Hout, Wout, xmin, xsize, wx, ymin, ysize, wy, ky, TH, rows_cap, seg_dw);
+  else
+    resize_aa_tile_kernel<K, true><<<grid, dim3(RS_WAVES * 64), lds, st>>>(src, T, Hin, Win, dst, Hout, Wout, xmin, xsize, wx, ymin, ysize, wy, ky, TH, rows_cap, seg_dw);
+}
+
 int resize_bicubic_aa_u8(const uint8_t* src, int layout, int T, int Hin, int Win, uint8_t* dst, int Hout, int Wout,
                          const int32_t* xmin, const int32_t* xsize, const float* wx, int kx, const int32_t* ymin,
                          const int32_t* ysize, const float* wy, int ky, float* tmp, hipStream_t st) {
   if (T <= 0 || Hin <= 0 || Win <= 0 || Hout <= 0 || Wout <= 0 || kx <= 0 || ky <= 0 || (layout != 0 && layout != 1)) return LCC_ERR_SHAPE;
+  // one launch while a tile's window fits RS_LDS_MAX with at least 8 rows: scales up to about 4 (tap tables of 5 to 17 columns); wider filters
+  // take the two passes, whose work does not grow with the overlap of neighbouring tiles
+  const double sx = (double)Win / Wout, sy = (double)Hin / Hout;
+  const int seg_dw = (((int)(63 * sx) + 2 + kx) * (layout == 0 ? 3 : 1) + 8 + 3) / 4;
+  for (int TH = 16; TH >= 8; TH >>= 1) {
+    const int rows_cap = (int)((TH - 1) * sy + 4 * std::max(sy, 1.0)) + 3;
+    const size_t lds = ((size_t)rows_cap * (3 * RS_COLS + (layout == 0 ? 1 : 3) * seg_dw) + TH * ((ky + 3) & ~3)) * 4;
+    if ((kx & 1) == 0 || kx < 5 || kx > 17 || lds > RS_LDS_MAX) continue;
+#define LCC_RS(KX) case KX: launch_resize_tile<KX>(src, layout, T, Hin, Win, dst, Hout, Wout, xmin, xsize, wx, ymin, ysize, wy, ky, TH, rows_cap, seg_dw, lds, st); return 0
+    switch (kx) { LCC_RS(5); LCC_RS(7); LCC_RS(9); LCC_RS(11); LCC_RS(13); LCC_RS(15); LCC_RS(17); }
+#undef LCC_RS
+  }
   const size_t n1 = (size_t)T * Hin * Wout, n2 = (size_t)T * 3 * Hout * Wout;
   resize_aa_h_kernel<<<dim3((unsigned)((n1 + 255) / 256)), dim3(256), 0, st>>>(src, layout, T, Hin, Win, Wout, xmin, xsize, wx, kx, tmp);
   resize_aa_v_kernel<<<dim3((unsigned)((n2 + 255) / 256)), dim3(256), 0, st>>>(tmp, T, Hin, Hout, Wout, ymin, ysize, wy, ky, dst);

@@ -83,3 +83,18 @@ def test_live_cc_from_video_paces_like_the_reference(dev):
     assert all(b - a in (1.0, 3.0) for a, b in spans)
     assert state.get("video_end") is True
     state["past_key_values"].release()
+
+
+# tile edges: one column / row past a multiple of the tile (64 columns, 16 or 8 rows), every tap count the one-launch kernel is built for
+# (5 to 17), the first scale it leaves to the two passes, a width where a frame ends off a dword
+@pytest.mark.parametrize("T,hi,wi,ho,wo", [(1, 31, 65, 33, 65), (2, 45, 91, 33, 63), (3, 97, 255, 49, 129), (1, 131, 131, 57, 56), (1, 90, 171, 32, 64),
+                                          (2, 101, 333, 29, 97), (1, 115, 509, 29, 128), (1, 121, 260, 30, 64), (1, 700, 65, 90, 65), (1, 1, 1, 1, 1)])
+@pytest.mark.parametrize("layout", ["THWC", "TCHW"])
+def test_resize_one_launch_at_tile_edges(dev, T, hi, wi, ho, wo, layout):
+    from livecc_amd import resize as R
+    from oracle import resize_ref as O
+    g = torch.Generator().manual_seed(hi + 1000 * wi)
+    tchw = torch.randint(0, 256, (T + 1, 3, hi, wi), dtype=torch.uint8, generator=g)
+    src = tchw.permute(0, 2, 3, 1).contiguous() if layout == "THWC" else tchw
+    got = R.resize_bicubic_aa(src.to(dev)[1:], ho, wo, layout).cpu()          # a view: its first byte may lie inside a dword
+    assert torch.equal(got, O.resize_ref(tchw[1:].contiguous(), ho, wo))
