@@ -76,11 +76,11 @@ int lcc_debug_set_gemv_variant(int variant);
  * gate/up GEMM of 8 co-scheduled chunks: 12 x 148 tiles instead of 13 x 148); 15 = the SMALL variable-height class (row tiles of 128 / 144
  * rows) for split-K slabs of 64 < M <= 448 wherever legal, else as 4 -- the default picks it by score for the o / down / q|k|v projections
  * of one streaming chunk (M = 386: 3 row tiles instead of 4, 6 / 6 / 4 splits; LCC_GEMM_VH_SMALL=0 restores the 128-row tiles and their
- * 4 / 4 / 3 splits).  Every tile shape produces the same bits for the same split count. */
+ * 4 / 4 / 3 splits); 16 = 128 x 128 tiles (bf16 weights).  Every tile shape produces the same bits for the same split count. */
 int lcc_debug_set_gemm_variant(int variant);
 /* Host logic only (no launch; works without a GPU): which kernel family serves a packed-weight GEMM of this shape under the current
  * variant -- *tile_rows = 16 weight-streaming GEMV, 448 tall, 272 / 144 variable-height tiles (big / small class), 256 / 192 / 128 the
- * 8-wave tile of that height, 64 a 4-wave tile kernel; nsplit > 0 asks for the split-K slab form -- and *engine_splits = the split count
+ * 8-wave tile of that height x 256 columns, 129 the 128 x 128 tile, 64 the 64 x 128 tile; nsplit > 0 asks for the split-K slab form -- and *engine_splits = the split count
  * the engine's prefill asks for at this shape (what csrc/engine_llm.hip passes as nsplit for the o / down / q|k|v projections).
  * w_fp8 != 0: *tile_rows = 0 (fp8 weights route inside their own entry point), *engine_splits as for fp8 weights. */
 int lcc_debug_gemm_plan(int M, int N, int K, int epilogue, int nsplit, int w_fp8, int32_t* tile_rows, int32_t* engine_splits);

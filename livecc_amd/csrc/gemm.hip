@@ -7,7 +7,8 @@
 //                          (BM 256 / 192 / 128), LDS-DMA for both operands, optional fp8-e4m3 W converted after the LDS read.
 //  * gemm_vh_kernel      : the same pipeline over row tiles of 256 / 272 / 288 rows (no ragged last row tile; round 5).
 //  * gemm_tall_kernel    : one block row covers all of M (256 < M <= 448: one streaming chunk's gate/up).
-//  * gemm_glds_kernel /   : shapes with few 256-column tiles, row-major W, K % 64 != 0.  64x128x64 (128x128x64) tile, 4 waves,
+//  * gemm_mid_kernel     : shapes with few 256-column tiles.  64x128x64 (128x128x64) tile, 8 waves, 6- (4-) stage LDS-DMA ring.
+//  * gemm_glds_kernel /   : row-major W, K % 64 != 0.  64x128x64 (128x128x64) tile, 4 waves,
 //    gemm_tiled_kernel     LDS-DMA 3-stage ring / register-staged double buffer with an XOR swizzle, XCD-aware block remap.
 //  * gemv_skinny_kernel  : M <= 64 (decode, lm_head; MG = ceil(M / 16) activation fragments per weight fragment).  HBM-bound weight streaming.  4 waves per block share 16 (or 32) W rows,
 //                          each wave a slice of K; W fragments go straight from HBM into the MFMA operand registers (no LDS
@@ -439,6 +440,134 @@ __global__ __launch_bounds__(256) void gemm_glds_kernel(
     }
   }
   tile_epilogue<EPI, MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, (n0 + wn * 64) / 2, li, g, bias, residual, ldr, C, ldc, M, N, partial, wscale);
+  if (vb + (int)gridDim.x < nblk) __syncthreads();     // the next tile's DMA reuses the stages
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// 64 x 128 x 64 (128 x 128 x 64) tile on EIGHT waves with a deep LDS-DMA ring: shapes whose 256-column tiles leave most of the chip idle
+// ------------------------------------------------------------------------------------------------
+// One streaming chunk's vision fc2 / proj (M = 1456, N = 1280) is 230 tiles of 64 x 128, one per compute unit: the time is the chain of K / 64
+// steps of one block, and a split of K would give another summation order.  gemm_glds_kernel spent 0.92 us a step on it (four waves, two
+// stages in flight: DMA round trip, fragment reads and MFMAs one after the other).  Here
+//   * five stages (120 KB) are in flight, so a step never waits for a round trip that is longer than four steps;
+//   * the fragments of tile kt + 1 are read into a second register set under the MFMAs of tile kt, behind the same barrier;
+//   * eight waves, each 32 (BM 128: 64) rows x 32 columns.
+// What bounds it now: LDS.  A step of the 64-row tile reads 64 KB of fragments and takes 24 KB from the DMA = 704 clocks at 128 B/clk against
+// 256 clocks of MFMA per SIMD; measured 0.33 us a step with 120 blocks, 0.40 with 230.  The 128-row tile reads 96 KB for twice the work.
+// Same summation order as every other tile kernel of this file.  Measured (us, gemm_glds_kernel or the tile chosen before -> here):
+// 1456 x 1280, K 5120 73 -> 31; K 1280 22 -> 12; 720 x 1280, K 5120 72 -> 28; 390 x 3584, K 3584 without a split 23 (128 x 256 tiles: 50);
+// 128-row tile: 1000 x 3584, K 22528 285 -> 196; 2000 x 1280, K 5120 55 -> 41.
+// NST 6 / 4 stages (64- / 128-row tile): one block on a compute unit.  NST 3 (72 KB, two blocks): more than 256 blocks of the 64-row tile
+// (2912 x 1280, K 5120: 57 us, gemm_glds_kernel 77).
+// Requires packed bf16 W, K % 64 == 0.
+template <int BM, int EPI, int NST>
+__global__ __launch_bounds__(512) void gemm_mid_kernel(
+    const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual,
+    int ldr, bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n, float* __restrict__ partial, int kt_per_split,
+    const float* __restrict__ wscale, int raster) {
+  constexpr int BN = 128, BK = 64, MT = BM / 32, NT = 2;
+  constexpr int A_UNITS = BM * 8, STAGE = A_UNITS + 16 * 64;      // 16-byte units: [BM rows][8 chunks] (XOR-swizzled) + 16 weight sub-tiles = 24 / 32 KB
+  constexpr int APW = BM / 64, P = APW + 2;                       // DMA pieces of a wave per k-tile: 8 activation rows each, then the weights
+  extern __shared__ __attribute__((aligned(16))) u32x4 dsmem[];
+
+  const int nblk = tiles_m * tiles_n;
+  for (int vb = blockIdx.x; vb < nblk; vb += gridDim.x) {     // one tile per block, or a persistent walk under the grid cap
+  int bid = vb;
+  {
+    const int q = nblk >> 3, r = nblk & 7, xcd = bid & 7, idx = bid >> 3;
+    bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
+  }
+  int tn, tm;                                     // tile order: see gemm_big_kernel
+  if (raster > 0) {
+    const int band = bid / (raster * tiles_m), rem = bid - band * raster * tiles_m;
+    const int bw = min(raster, tiles_n - band * raster);
+    tm = rem / bw;
+    tn = band * raster + (rem - tm * bw);
+  } else {
+    tn = bid / tiles_m;
+    tm = bid - tn * tiles_m;
+  }
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 2, wn = wave & 3;
+  const int li = lane & 15, g = lane >> 4;
+  const int K32 = K >> 5, nfrag = (N + 15) >> 4;
+
+  // this wave's DMA pieces of a k-tile: 8 activation rows each, and both 32-k blocks of weight fragment row `wave`
+  const bf16_t* asrc[APW];
+#pragma unroll
+  for (int q = 0; q < APW; ++q) asrc[q] = A + (size_t)min(m0 + (wave + 8 * q) * 8 + (lane >> 3), M - 1) * lda + (((lane & 7) ^ (lane >> 3)) << 3);
+  const bf16_t* bsrc = W + (size_t)min((n0 >> 4) + wave, nfrag - 1) * K32 * 512 + lane * 8;
+  const unsigned lds0 = lds_addr(dsmem);
+  const int nkt_all = K / BK;
+  const int kt0 = (EPI == EPI_PARTIAL) ? blockIdx.y * kt_per_split : 0;
+  const int nkt = (EPI == EPI_PARTIAL) ? min(nkt_all, kt0 + kt_per_split) : nkt_all;
+  auto issue = [&](int kt, int stage) {           // past the last tile: the source is clamped, the copy lands in a stage nobody reads any more
+    const int k = min(kt, nkt - 1);
+    const unsigned base = lds0 + (unsigned)(stage * STAGE) * 16u;
+#pragma unroll
+    for (int q = 0; q < APW; ++q) glds16(asrc[q] + (size_t)k * BK, base + (wave + 8 * q) * 1024u);
+    glds16(bsrc + (size_t)k * 1024, base + (A_UNITS + wave * 128) * 16u);
+    glds16(bsrc + (size_t)k * 1024 + 512, base + (A_UNITS + wave * 128 + 64) * 16u);
+  };
+
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  int aoff[2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) aoff[kk] = (wm * (BM / 2) + li) * 8 + ((kk * 4 + g) ^ (li & 7));
+  const int boff = A_UNITS + wn * 4 * 64 + lane;
+  struct Frag { bf16x8 a[2][MT], b[2][NT]; };
+  auto read = [&](Frag& f, int stage) {
+    const u32x4* s = dsmem + stage * STAGE;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) f.a[kk][i] = as_bf16x8(s[aoff[kk] + i * 128]);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) f.b[kk][j] = as_bf16x8(s[boff + (j * 2 + kk) * 64]);
+    }
+  };
+  auto mul = [&](const Frag& f) {
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = mfma16(f.b[kk][j], f.a[kk][i], acc[i][j]);
+  };
+  // tile kt + 1 has landed (this wave's pieces; NST - 3 newer tiles may stay in flight) -> barrier -> DMA of tile kt + NST - 1 into the stage
+  // of tile kt - 1 (its fragments were in registers before the barrier) -> fragment reads of tile kt + 1 -> MFMAs of tile kt
+  auto step = [&](const Frag& cur, Frag& nxt, int kt, int st) {          // st = stage of tile kt
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(P * (NST - 3)) : "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);          // pinned: left alone, hipcc moves the MFMAs of tile kt + 1 up behind its reads
+    read(nxt, st == NST - 1 ? 0 : st + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    issue(kt + NST - 1, st == 0 ? NST - 1 : st - 1);
+    mul(cur);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int p = 0; p < NST - 1; ++p) issue(kt0 + p, p);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(P * (NST - 2)) : "memory");
+  __builtin_amdgcn_s_barrier();
+  Frag f0, f1;
+  read(f0, 0);
+  int st = 0, kt = kt0;
+  for (; kt + 1 < nkt; kt += 2) {
+    step(f0, f1, kt, st);
+    st = st == NST - 1 ? 0 : st + 1;
+    step(f1, f0, kt + 1, st);
+    st = st == NST - 1 ? 0 : st + 1;
+  }
+  if (kt < nkt) mul(f0);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the clamped copies
+  tile_epilogue<EPI, MT, NT>(acc, m0 + wm * (BM / 2), n0 + wn * 32, (n0 + wn * 32) / 2, li, g, bias, residual, ldr, C, ldc, M, N, partial, wscale);
   if (vb + (int)gridDim.x < nblk) __syncthreads();     // the next tile's DMA reuses the stages
   }
 }
@@ -1020,8 +1149,24 @@ static int g_gemm_variant = 2;
 static int g_gemm_sched = 1;   // fragment-read schedule of gemm_big_kernel: 0 compiler order, 1 pinned software pipeline
 void set_gemm_variant(int v);
 
+static inline int raster_for(int tiles_m);
+template <int BM, int EPI, int NST>
+static void launch_mid(const GemmArgs& a, hipStream_t st) {
+  const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + 127) / 128, nkt = a.K / 64, S = (EPI == EPI_PARTIAL) ? a.nsplit : 1;
+  constexpr size_t lds = (size_t)NST * (BM * 128 + 16384);
+  static DeviceOnce attr_set;   // per instantiation
+  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_mid_kernel<BM, EPI, NST>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  gemm_mid_kernel<BM, EPI, NST><<<dim3(capped_grid((long)tiles_m * tiles_n), S), dim3(512), lds, st>>>(
+      a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.partial, (nkt + S - 1) / S, a.wscale, raster_for(tiles_m));
+}
 template <int BM, int EPI>
 static void launch_tiled(const GemmArgs& a, hipStream_t st) {
+  if constexpr (BM == 64) {
+    if ((g_gemm_variant == 2 || g_gemm_variant == 7) && a.w_packed && (a.K & 63) == 0) {
+      const long blocks = (long)capped_grid((long)((a.M + 63) / 64) * ((a.N + 127) / 128)) * (EPI == EPI_PARTIAL ? a.nsplit : 1);
+      return blocks <= 256 ? launch_mid<64, EPI, 6>(a, st) : launch_mid<64, EPI, 3>(a, st);
+    }
+  }
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + 127) / 128;
   const int nkt = (a.K + 63) / 64, S = (EPI == EPI_PARTIAL) ? a.nsplit : 1;
   if (g_gemm_variant == 1 || ((g_gemm_variant == 2 || g_gemm_variant == 7) && BM == 64)) {   // 7: auto without the 8-wave kernel
@@ -1090,6 +1235,7 @@ static void launch_big(const GemmArgs& a, hipStream_t st) {
   else launch_big_s<BM, EPI, 0, false>(a, st);
 }
 // 13: the 192-row tile wherever eligible (bf16 weights); 14: variable-height row tiles (gemm_vh_kernel) wherever legal, else as 3;
+// 16: 128 x 128 tiles (gemm_mid_kernel) wherever eligible, bf16 weights
 // 15: the small variable-height class (8 / 9 fragments) for split-K slabs wherever legal, else as 4
 void set_gemm_variant(int v) {
   g_gemm_variant = v;
@@ -1134,30 +1280,37 @@ static int big_tile_rows(const GemmArgs& a, int S) {
   if (g_gemm_variant == 4 || g_gemm_variant == 6) return 128;
   if (g_gemm_variant == 13) return a.w_fp8 ? 256 : 192;
   if (g_gemm_variant == 15) return (a.partial != nullptr && vh_small_shape(a.M, a.K) && vh_legal(a, true)) ? 144 : 128;
+  if (g_gemm_variant == 16) return a.w_fp8 ? 128 : 129;
   if (g_gemm_variant != 2) return 0;
   const float s256 = tile_score(a.M, a.N, S, 256, 256, 256, 1.0f, true);
   static const int allow192 = [] { const char* v = getenv("LCC_GEMM_192"); return v ? atoi(v) : 1; }();     // A/B: 0 = round-3 tile choice
   const float s192 = (a.w_fp8 || !allow192) ? 0.f : tile_score(a.M, a.N, S, 192, 256, 256, 0.93f, true);
   const float s128 = tile_score(a.M, a.N, S, 128, 256, 256, 0.85f, true);
-  const float s64 = tile_score(a.M, a.N, S, 64, 128, 512, 0.55f, false);
+  // gemm_mid_kernel: 0.38 / 0.52 us a step of 64 x 128 / 128 x 128 against 0.85 of 128 x 256, one tile a compute unit at a time (two 64-row
+  // tiles side by side take twice as long).  Returned as 0 / 129.  The 128-row form wins where its blocks fill one round and the 64-row
+  // form's need two; beyond a round the 256-column tiles do (shapes around the lines: 1000 x 3584, K 3584: 43 / 34 / 52 us for 64 x 128 /
+  // 128 x 128 / 128 x 256; 1456 x 3584: 73 / 61 / 52; 520 x 3584: 25 / 33 / 50).  fp8 weights: the 64-row tile means a pass that
+  // dequantises first, scored as measured with it.
+  const float s64 = a.w_fp8 ? tile_score(a.M, a.N, S, 64, 128, 512, 0.55f, false) : tile_score(a.M, a.N, S, 64, 128, 256, 0.48f, false);
+  const float s128m = a.w_fp8 ? 0.f : tile_score(a.M, a.N, S, 128, 128, 256, 0.70f, false);
   static const int allow_vh = [] { const char* v = getenv("LCC_GEMM_VH"); return v ? atoi(v) : 1; }();
   if (allow_vh && vh_legal(a) && (((a.M + 15) >> 4) & 15) != 0) {      // F % 16 == 0: the 256-row tiles are the same thing
     const int F = (a.M + 15) >> 4, t = F >> 4, maxf = (F + t - 1) / t;
     const long blocks = (long)t * ((a.N + 255) / 256) * S;
     const float svh = (float)a.M / (float)(t * maxf * 16) * (float)blocks / (float)((blocks + 255) / 256 * 256);
-    if (svh > s256 && svh > s192 && svh > s128 && svh > s64) return 272;
+    if (svh > s256 && svh > s192 && svh > s128 && svh > s128m && svh > s64) return 272;
   }
   // small class (returned as 144): split-K slabs of one streaming chunk's projections, where the 128-row tiles leave a nearly empty last row tile
   if (vh_small_on() && a.partial != nullptr && vh_small_shape(a.M, a.K) && vh_legal(a, true)) {
     const int F = (a.M + 15) >> 4, t = F >> 3, maxf = (F + t - 1) / t;
     const long blocks = (long)t * ((a.N + 255) / 256) * S;
     const float svs = 0.85f * (float)a.M / (float)(t * maxf * 16) * (float)blocks / (float)((blocks + 255) / 256 * 256);
-    if (svs > s256 && svs > s192 && svs > s128 && svs > s64) return 144;
+    if (svs > s256 && svs > s192 && svs > s128 && svs > s128m && svs > s64) return 144;
   }
-  if (s256 >= s192 && s256 >= s128 && s256 >= s64) return 256;
-  if (s192 >= s128 && s192 >= s64) return 192;
-  if (s128 >= s64) return 128;
-  return 0;
+  if (s256 >= s192 && s256 >= s128 && s256 >= s128m && s256 >= s64) return 256;
+  if (s192 >= s128 && s192 >= s128m && s192 >= s64) return 192;
+  if (s128 >= s128m && s128 >= s64) return 128;
+  return s128m > s64 ? 129 : 0;
 }
 
 // The tall kernel serves one-block-row problems whose column tiles fill most of ONE round of the chip (7B gate/up at a streaming
@@ -1199,6 +1352,7 @@ static void launch_tiled_bm(const GemmArgs& a, hipStream_t st) {
     if (tall_wanted(a)) return launch_tall<EPI>(a, st);
   }
   const int big = big_tile_rows(a, 1);
+  if (big == 129) return launch_mid<128, EPI, 4>(a, st);
   if (big == 272) return launch_vh<EPI>(a, st);
   if (big == 256) return launch_big<256, EPI>(a, st);
   if (big == 192) return launch_big<192, EPI>(a, st);
@@ -1212,7 +1366,7 @@ static void launch_tiled_bm(const GemmArgs& a, hipStream_t st) {
 
 // Which kernel family serves a packed-weight GEMM of this shape under the current variant (host logic only: no launch, no GPU needed):
 // 16 = weight-streaming GEMV, 448 = tall, 272 / 144 = variable-height tiles (big / small class), 256 / 192 / 128 = the 8-wave tile of
-// that height, 64 = a 4-wave tile kernel.  `nsplit` > 0: the split-K slab form with that many splits (as the engine asks: gemm_tiled_num_splits).
+// that height x 256 columns, 129 = 128 x 128, 64 = 64 x 128.  `nsplit` > 0: the split-K slab form with that many splits (as the engine asks: gemm_tiled_num_splits).
 int gemm_plan(int M, int N, int K, int epilogue, int nsplit, bool w_fp8) {
   GemmArgs a; a.M = M; a.N = N; a.K = K; a.w_packed = 1; a.w_fp8 = w_fp8 ? 1 : 0; a.epilogue = epilogue; a.nsplit = nsplit;
   static float dummy;
@@ -1769,7 +1923,7 @@ int gemm_bf16(const GemmArgs& a, hipStream_t st) {
     if ((v && ((uintptr_t)q.vt & 7) != 0) || (a.bias != nullptr && ((uintptr_t)a.bias & 7) != 0)) return LCC_ERR_ALIGN;
     g_launch_counts[LC_GEMM_VIT_QKV]++;
     int big = big_tile_rows(a, 1);
-    if (big == 272) big = 256;      // the rotation / transposed-V epilogues live on the fixed-height tiles
+    if (big == 272) big = 256;      // the rotation / transposed-V epilogues live on the fixed-height 256-column tiles (129: the 128-row one)
     if (a.epilogue == EPI_VIT_QKV) {
       if (big == 256) launch_big_s<256, EPI_VIT_QKV, 6, false>(a, st);
       else if (big == 192) launch_big_s<192, EPI_VIT_QKV, 6, false>(a, st);
@@ -1817,6 +1971,7 @@ int gemm_bf16(const GemmArgs& a, hipStream_t st) {
     else if (big == 256) launch_big<256, EPI_PARTIAL>(a, st);
     else if (big == 192) launch_big<192, EPI_PARTIAL>(a, st);
     else if (big == 128) launch_big<128, EPI_PARTIAL>(a, st);
+    else if (big == 129) launch_mid<128, EPI_PARTIAL, 4>(a, st);
     else launch_tiled<64, EPI_PARTIAL>(a, st);
     return 0;
   }

@@ -151,6 +151,45 @@ def test_gemm_variable_height_tiles_are_bit_identical_to_the_256_row_tiles(dev, 
     assert_bf16_close(got, exp, f"gemm_vh[{M}x{N}x{K},epi{epi}]", max_ulp=1.0, max_frac=5e-3, atol=atol)
 
 
+@pytest.mark.parametrize("M,N,K,epi,variant", [
+    (65, 144, 64, 0, 7), (64, 128, 128, 3, 7), (127, 272, 192, 2, 7), (720, 1280, 448, 3, 7), (1456, 1280, 5120, 3, 2), (100, 512, 320, 4, 7),
+    (2912, 1280, 192, 3, 7), (1031, 2320, 256, 1, 7), (65, 144, 64, 0, 16), (129, 272, 128, 3, 16), (257, 144, 192, 2, 16), (720, 1280, 448, 1, 16),
+    (100, 544, 320, 4, 16), (1000, 3584, 1536, 3, 2)])
+def test_gemm_128_column_tiles_are_bit_identical_to_the_256_row_tiles(dev, M, N, K, epi, variant):
+    """64 x 128 tiles (6 stages up to 256 tiles, 3 stages beyond: 2912 x 1280, 1031 x 2320) and 128 x 128 tiles (variant 16): one k-tile, fewer
+    k-tiles than stages, odd and even counts, one row past a tile, a ragged last column tile, every epilogue; the summation order is that of
+    the 256-row tiles."""
+    from livecc_amd import ops
+    x, w, b = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.05, 2), _rand((N,), dev, 0.1, 3)
+    res = _rand((M, N), dev, 1.0, 4) if epi == 3 else None
+    wp = ops.pack_weight(w)
+    try:
+        ops.set_gemm_variant(3)
+        ref = ops.linear(x, wp, None if epi == 4 else b, epi, res, packed_shape=(N, K))
+        ops.set_gemm_variant(variant)
+        if variant != 7:
+            assert ops.gemm_plan(M, N, K, epi)[0] == (129 if M != 1456 else 64)
+        got = ops.linear(x, wp, None if epi == 4 else b, epi, res, packed_shape=(N, K))
+    finally:
+        ops.set_gemm_variant(ops.GEMM_DEFAULT_VARIANT)
+    assert torch.equal(got, ref), f"{int((got != ref).sum())} of {got.numel()} outputs differ from the 256-row tiles"
+
+
+@pytest.mark.parametrize("M,N,K,S,variant", [(72, 144, 320, 4, 7), (122, 1536, 8960, 4, 2), (390, 1536, 576, 8, 7), (200, 272, 320, 4, 16), (1000, 3584, 1024, 1, 2)])
+def test_gemm_128_column_tiles_give_the_slabs_of_the_128_row_tiles(dev, M, N, K, S, variant):
+    """Split-K slabs: uneven k-tile counts, a split without a k-tile (5 k-tiles in 4 splits: zeros)."""
+    from livecc_amd import ops
+    x, wp = _rand((M, K), dev, 1.0, 1), ops.pack_weight(_rand((N, K), dev, 0.05, 2))
+    try:
+        ops.set_gemm_variant(4)
+        ref = ops.linear_partial(x, wp, S, packed_shape=(N, K))
+        ops.set_gemm_variant(variant)
+        got = ops.linear_partial(x, wp, S, packed_shape=(N, K))
+    finally:
+        ops.set_gemm_variant(ops.GEMM_DEFAULT_VARIANT)
+    assert torch.equal(got, ref)
+
+
 @pytest.mark.parametrize("M,N,K,S", [(386, 3584, 18944, 6), (386, 4608, 3584, 4), (386, 3584, 3584, 6), (400, 3600, 1024, 2), (130, 512, 512, 2),
                                      (272, 1024, 1024, 4), (144, 256, 4096, 8), (391, 1536, 8960, 5)])
 def test_gemm_small_variable_height_tiles_give_the_slabs_of_the_128_row_tiles(dev, M, N, K, S):
