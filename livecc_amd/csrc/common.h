@@ -102,34 +102,34 @@ LCC_DEVICE float block_sum(float v, float* red) {
   return t;
 }
 
-// activations, with HF's bf16 rounding points (inputs are already-rounded bf16 values held in fp32).
-// exp and the reciprocal use the hardware units (v_exp_f32, v_rcp_f32) with the error terms folded back in:
-//   exp(t): t*log2(e) split into hi + lo (FMA residual), exp2(hi) * (1 + lo*ln2)      -> ~1 ulp of fp32
-//   1/d   : v_rcp_f32 + one Newton step                                              -> ~0.5 ulp of fp32
-// i.e. 10 VALU instructions instead of ~30 for libm expf + IEEE division; the fp32 result is then rounded to bf16 (2^-9
-// relative), so it differs from the correctly rounded activation in ~5e-5 of the elements by one bf16 ulp -- two orders of
-// magnitude below the effect of the fp32 summation order of the GEMM that feeds it.  (The epilogue was 9 % of the SwiGLU
-// gate/up GEMM and ~25 % of the ViT fc1 GEMM.)
-LCC_DEVICE float exp_fast(float t) {
-  const float L2E_HI = 1.4426950216293335f, L2E_LO = 1.9259629911266175e-8f;   // log2(e) = hi + lo
-  const float hi = t * L2E_HI;
-  const float lo = fmaf(t, L2E_HI, -hi) + t * L2E_LO;
-  return __builtin_amdgcn_exp2f(hi) * fmaf(lo, 0.6931471805599453f, 1.0f);
+// two values after rounding to bf16: one conversion for the pair
+LCC_DEVICE void rbf2(float& a, float& b) {
+  const unsigned u = pack2(a, b);
+  a = lo2f(u); b = hi2f(u);
 }
-LCC_DEVICE float rcp_fast(float d) {
-  const float r = __builtin_amdgcn_rcpf(d);
-  return fmaf(fmaf(-d, r, 1.0f), r, r);
-}
-// quick_gelu: HF activations.py QuickGELUActivation: input * sigmoid(1.702 * input) on bf16 tensors
-LCC_DEVICE float quick_gelu_bf16(float x) {
-  float t = rbf(1.702f * x);
-  float s = rbf(rcp_fast(1.0f + exp_fast(-t)));
-  return rbf(x * s);
+
+// activations, with HF's bf16 rounding points (inputs are already-rounded bf16 values held in fp32).  exp and the reciprocal are the
+// hardware units (v_exp_f32, v_rcp_f32), as few instructions around them as give the rounded double-precision result on EVERY finite bf16
+// input (all 65,280 were compared): they are what bounds the epilogues of the short products (ViT fc1: 37 us of 205 at 15,840 patches with
+// the error-corrected exponential and reciprocal this replaces, which also gave NaN below -52 / -88).
+constexpr float LOG2E = 1.4426950408889634f;
+// quick_gelu: HF activations.py QuickGELUActivation: input * sigmoid(1.702 * input) on bf16 tensors; two at a time.  The products are left
+// unrounded: the caller packs them.
+LCC_DEVICE void quick_gelu2(float& x0, float& x1) {
+  float t0 = 1.702f * x0, t1 = 1.702f * x1;
+  rbf2(t0, t1);
+  float s0 = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t0 * -LOG2E)), s1 = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t1 * -LOG2E));
+  rbf2(s0, s1);
+  x0 *= s0; x1 *= s1;
 }
 // exact (erf) GELU: torch gelu on bf16 computes in fp32 and rounds once
 LCC_DEVICE float gelu_erf_bf16(float x) { return rbf(0.5f * x * (1.0f + erff(x * 0.70710678118654752440f))); }
-// silu on bf16: x / (1 + exp(-x)) in fp32, rounded once
-LCC_DEVICE float silu_bf16(float x) { return rbf(x * rcp_fast(1.0f + exp_fast(-x))); }
+// silu on bf16: x / (1 + exp(-x)) in fp32, rounded once.  One Newton step on the reciprocal (without it one input rounds the other way); the
+// maximum turns the NaN of an infinite denominator into a step from 0 to 0.
+LCC_DEVICE float silu_bf16(float x) {
+  const float d = 1.0f + __builtin_amdgcn_exp2f(x * -LOG2E), r = __builtin_amdgcn_rcpf(d);
+  return rbf(x * fmaf(__builtin_fmaxf(fmaf(-d, r, 1.0f), -1.0f), r, r));
+}
 
 enum Epilogue : int {
   EPI_NONE = 0,        // C = bf16(acc + bias)

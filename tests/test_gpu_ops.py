@@ -175,6 +175,54 @@ def test_gemm_128_column_tiles_are_bit_identical_to_the_256_row_tiles(dev, M, N,
     assert torch.equal(got, ref), f"{int((got != ref).sum())} of {got.numel()} outputs differ from the 256-row tiles"
 
 
+@pytest.mark.parametrize("variant", [3, 4, 13, 14, 16, 7])
+@pytest.mark.parametrize("epi", [0, 1, 2, 3])
+def test_gemm_epilogue_rows_of_16_byte_pieces_and_others_give_the_same_bits(dev, variant, epi):
+    """A ragged row tile and a last column tile of 16 columns, rows of C and of the residual that are whole 16-byte pieces (the stores of whole
+    rows) or not (the plain form), a residual that starts off a piece; nothing is written beside the columns."""
+    from livecc_amd import _lib, ops
+    M, N, K = 281, 528, 128
+    x, w, b, r = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.05, 2), _rand((N,), dev, 0.1, 3), _rand((M, N), dev, 1.0, 4)
+    wp, lib = ops.pack_weight(w), _lib.load()
+    outs = []
+    ops.set_gemm_variant(variant)
+    try:
+        for ldc, ldr, off in ((N, N, 0), (N + 8, N + 8, 0), (N + 4, N, 0), (N, N + 4, 0), (N, N, 4)):
+            C = torch.full((M, ldc), 7.0, dtype=torch.bfloat16, device=dev)
+            R = torch.zeros(M * ldr + 16, dtype=torch.bfloat16, device=dev)
+            R[off:off + M * ldr].view(M, ldr)[:, :N] = r
+            _lib.check(lib.lcc_gemm_bf16(x.data_ptr(), K, wp.data_ptr(), K, 1, b.data_ptr(), R.data_ptr() + 2 * off if epi == 3 else None, ldr,
+                                         C.data_ptr(), ldc, M, N, K, epi, None, 0, torch.cuda.current_stream(dev).cuda_stream), "lcc_gemm_bf16")
+            assert bool((C[:, N:] == 7.0).all())
+            outs.append(C[:, :N].contiguous())
+    finally:
+        ops.set_gemm_variant(ops.GEMM_DEFAULT_VARIANT)
+    for o in outs[1:]:
+        assert torch.equal(outs[0], o)
+    ref, atol = _ref_linear(x, w, b, epi, r if epi == 3 else None, with_atol=True)
+    assert_bf16_close(outs[0], ref, f"gemm rows[{variant},epi{epi}]", max_ulp=1.0, max_frac=5e-3, atol=atol)
+
+
+def test_activations_round_like_double_precision_on_every_finite_bf16_input(dev):
+    """quick_gelu (the rounding points of its three bf16 operations) and silu: the rounded double-precision value for all 65,280 inputs."""
+    from livecc_amd import ops
+    x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    x = x[torch.isfinite(x.float())].view(1020, 64)
+    eye = torch.eye(64, dtype=torch.bfloat16)
+    d = x.double()
+    t = (1.702 * x.float()).to(torch.bfloat16)                # torch multiplies a bf16 tensor by a scalar in fp32
+    want = (d * (1 / (1 + torch.exp(-t.double()))).to(torch.bfloat16).double()).to(torch.bfloat16)
+    got = ops.linear(x.to(dev), ops.pack_weight(eye.to(dev)), None, ops.EPI_QUICK_GELU, packed_shape=(64, 64)).cpu()
+    normal = want.float().abs() > 1e-30                       # the matrix cores flush subnormal inputs and outputs
+    assert not torch.isnan(got.float()).any() and torch.equal(got[normal], want[normal])
+    assert float(got[~normal].float().abs().max()) < 2e-30
+    want = (d / (1 + torch.exp(-d))).to(torch.bfloat16)
+    got = ops.swiglu(x.to(dev), torch.ones_like(x).to(dev)).cpu()
+    normal = want.float().abs() > 1e-30
+    assert not torch.isnan(got.float()).any() and torch.equal(got[normal], want[normal])
+    assert float(got[~normal].float().abs().max()) < 2e-30
+
+
 @pytest.mark.parametrize("M,N,K,S,variant", [(72, 144, 320, 4, 7), (122, 1536, 8960, 4, 2), (390, 1536, 576, 8, 7), (200, 272, 320, 4, 16), (1000, 3584, 1024, 1, 2)])
 def test_gemm_128_column_tiles_give_the_slabs_of_the_128_row_tiles(dev, M, N, K, S, variant):
     """Split-K slabs: uneven k-tile counts, a split without a k-tile (5 k-tiles in 4 splits: zeros)."""
