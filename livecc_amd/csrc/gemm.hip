@@ -201,6 +201,40 @@ LCC_DEVICE void tile_epilogue_wide(const f32x4 (&acc)[MT][NT], int mbase, int nb
   }
 }
 
+// fp32 slabs the same way: 32 rows of 256 bytes at a time (lds: 8 KB, wave-private)
+template <int MT, int NT>
+LCC_DEVICE void tile_slab_wide(const f32x4 (&acc)[MT][NT], int mbase, int nbase, int lane, int M, int N, float* __restrict__ partial,
+                               const float* __restrict__ wscale, unsigned char* lds) {
+  static_assert(NT == 4, "64 columns a wave");
+  const int li = lane & 15, g = lane >> 4;
+  f32x4 sc[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) sc[j] = (f32x4){1.f, 1.f, 1.f, 1.f};
+  if (wscale != nullptr) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j) sc[j] = *reinterpret_cast<const f32x4*>(wscale + min(nbase + j * 16 + g * 4, N - 4));
+  }
+  const int sr = lane >> 4, schk = lane & 15, scol = nbase + schk * 4;
+  float* out = partial + (size_t)blockIdx.y * M * N + scol;
+#pragma unroll
+  for (int i0 = 0; i0 < MT; i0 += 2) {
+#pragma unroll
+    for (int ii = 0; ii < 2; ++ii) {
+      if (i0 + ii >= MT) continue;
+      const int r = ii * 16 + li;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) *reinterpret_cast<f32x4*>(lds + r * 256 + (((j * 4 + g) ^ (r & 15)) * 16)) = acc[i0 + ii][j] * sc[j];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      if (i0 * 16 + q * 4 >= MT * 16) continue;
+      const int r = q * 4 + sr, m = mbase + i0 * 16 + r;
+      const f32x4 v = *reinterpret_cast<const f32x4*>(lds + r * 256 + ((schk ^ (r & 15)) * 16));
+      if (m < M && scol < N) *reinterpret_cast<f32x4*>(out + (size_t)m * N) = v;
+    }
+  }
+}
+
 // ------------------------------------------------------------------------------------------------
 // EPI_VIT_QK / EPI_VIT_V (round 4): the vision tower's q|k|v projection writes what its attention kernels read -- q and k rotated (2-D
 // RoPE, HF modeling_qwen2_vl.py:225-248) at their natural columns of C, V blocked-transposed into vt[head][32-key block][80][32] -- instead
@@ -845,6 +879,9 @@ LCC_DEVICE void gemm_big_body(
     vit_qk_epilogue<MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, wm * WM, li, g, bias, C, ldc, M, N, vq.E, lcs, lcs + UNITS * 4);
   } else if constexpr (EPI == EPI_VIT_V) {
     vit_v_epilogue<MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, li, g, bias, M, N, vq);
+  } else if constexpr (EPI == EPI_PARTIAL) {
+    __builtin_amdgcn_s_barrier();          // every wave is done with the stages, and its DMA pieces have landed
+    tile_slab_wide<MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, lane, M, N, partial, wscale, reinterpret_cast<unsigned char*>(dsmem) + wave * 8192);
   } else if (wide_rows<EPI>(C, ldc, residual, ldr)) {
     __builtin_amdgcn_s_barrier();          // every wave is done with the stages, and its DMA pieces have landed
     tile_epilogue_wide<EPI, MT, NT, !(W8 && BM == 256)>(acc, m0 + wm * WM, n0 + wn * 64, lane, bias, residual, ldr, C, ldc, M, N, wscale,
@@ -1057,9 +1094,11 @@ __global__ __launch_bounds__(512) void gemm_vh_kernel(
       }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the clamped copies of the last iteration
-    const bool wide = wide_rows<EPI>(C, ldc, residual, ldr);          // block-uniform
+    const bool wide = EPI == EPI_PARTIAL || wide_rows<EPI>(C, ldc, residual, ldr);          // block-uniform
     if (wide) __builtin_amdgcn_s_barrier();          // every wave is done with the stages, and its DMA pieces have landed
-    if constexpr (MTW > 0) {
+    if constexpr (MTW > 0 && EPI == EPI_PARTIAL) {
+      tile_slab_wide<MTW, NT>(acc, m0 + my_row0, n0 + wn * 64, lane, M, N, partial, nullptr, reinterpret_cast<unsigned char*>(dsmem) + wave * 8192);
+    } else if constexpr (MTW > 0) {
       if (wide)
         tile_epilogue_wide<EPI, MTW, NT, false>(acc, m0 + my_row0, n0 + wn * 64, lane, bias, residual, ldr, C, ldc, M, N, nullptr,
                                          reinterpret_cast<unsigned char*>(dsmem) + wave * 8192);
