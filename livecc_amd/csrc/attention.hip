@@ -639,28 +639,43 @@ __global__ __launch_bounds__(64, 2) void attn_decode_kernel(
 // instead of ~51 leave few enough partials to merge them in the o-projection's prologue instead of a combine launch.  Decode step 2930 -> 3134 us
 // with 8 splits (32 blocks), 3012 with 16, 3390 with 4: a CU pulls ~35 GB/s of K / V however many waves it runs, so the 13.4 MB of a launch
 // need all 204 CUs' worth of one-wave blocks -- and with it the 51 partials.  profiles/r06/decode_attn_multiwave_ab.jsonl.)
-// grid = (Hq, B), 256 threads = 8 split groups x 32 lanes (4 consecutive d each).  Group q merges splits q, q+8, ...
-// with all its loads in flight at once; the 8 partial (m, num, den) triples are merged through LDS.
+// grid = (Hq, B), 256 threads = 8 split groups x 32 lanes (4 consecutive d each).  Group q merges splits q, q+8, ...; the 8 partial
+// (m, num, den) triples are merged through LDS.  What bounds it is the trip to the partials other XCDs wrote (they come from beyond the
+// L2): all 24 loads of up to 64 splits go out together (one running maximum per split, each iteration's loads behind the last one's use,
+// took two to eight trips).
 __global__ __launch_bounds__(256) void attn_decode_combine_kernel(
     const float* __restrict__ ws_o, const float* __restrict__ ws_ml, bf16_t* __restrict__ out, int n_q_heads,
     int n_kv_heads, int nsplit) {
-  constexpr int D = 128, NG = 8;
+  constexpr int D = 128, NG = 8, U = 8;
   __shared__ float sm[NG][32][6];
   const int hq = blockIdx.x, b = blockIdx.y, t = threadIdx.x, dl = t & 31, grp = t >> 5;
   const int G = n_q_heads / n_kv_heads, hk = hq / G, j = hq % G;
   const size_t slot0 = (((size_t)b * n_kv_heads + hk) * nsplit) * 16 + j;
   float M = -INFINITY, den = 0.f;
   f32x4 num = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-  for (int s = grp; s < nsplit; s += NG) {
-    const size_t slot = slot0 + (size_t)s * 16;
-    const float m = ws_ml[slot * 2], l = ws_ml[slot * 2 + 1];
-    const f32x4 o = *reinterpret_cast<const f32x4*>(ws_o + slot * D + dl * 4);
-    const float Mn = fmaxf(M, m);
+  for (int s0 = grp; s0 < nsplit; s0 += NG * U) {
+    f32x2_t ml[U];
+    f32x4 o[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const size_t slot = slot0 + (size_t)min(s0 + u * NG, nsplit - 1) * 16;
+      ml[u] = *reinterpret_cast<const f32x2_t*>(ws_ml + slot * 2);
+      o[u] = *reinterpret_cast<const f32x4*>(ws_o + slot * D + dl * 4);
+    }
+    float Mn = M;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (s0 + u * NG >= nsplit) ml[u][0] = -INFINITY;
+      Mn = fmaxf(Mn, ml[u][0]);
+    }
     const float a = (M == -INFINITY) ? 0.f : exp2f(M - Mn);
-    const float w = (m == -INFINITY) ? 0.f : exp2f(m - Mn);
-    num = num * a + o * w;
-    den = den * a + w * l;
+    num *= a; den *= a;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float w = (ml[u][0] == -INFINITY) ? 0.f : exp2f(ml[u][0] - Mn);
+      num += o[u] * w;
+      den += ml[u][1] * w;
+    }
     M = Mn;
   }
   sm[grp][dl][0] = M; sm[grp][dl][1] = den;
