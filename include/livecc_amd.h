@@ -122,7 +122,9 @@ int lcc_debug_set_decode_path(int path);
  * CU) and for <= 2 streams; 0 (default) = separate launches.  A hand-off that times out fails the call (lcc_slot_read_tokens) and disables it. */
 int lcc_debug_set_decode_chain(int on);
 /* Block shape of the o_proj / down_proj decode GEMV (lcc_dgemv_resid): 0 = 8 waves per block, 1 (default) = 16 waves for bf16 weights with
- * K >= 8192 (the down projection: half the dependent chain of load stages per wave), 2 = 16 waves for every call.  Returns the old mode.
+ * K >= 8192 (the down projection: half the dependent chain of load stages per wave), 2 = 16 waves for every call, 3 = blocks of 8 output
+ * rows (N <= 2048, M <= 8, bf16 weights: what the engine takes by itself under mode 1 where 16-row blocks would leave half the chip idle;
+ * lcc_dgemv_resid then writes one statistic per 8 outputs, [M, N/8]).  Returns the old mode.
  * The K split across the waves of a block -- and so the fp32 summation order -- differs between the two shapes. */
 int lcc_debug_set_resid_waves(int mode);
 /* Largest M (16..64, default 64) served by the weight-streaming GEMV kernels of lcc_gemm_bf16 and by the engine's decode step: with 17..64

@@ -451,6 +451,123 @@ __global__ __launch_bounds__(512, 2) void dgemv_latent_q_kernel(DgArgs a, Latent
   else latent_row<512, false>(row, (int)blockIdx.x - nb, reinterpret_cast<float*>(red));
 }
 
+// ---- eight output rows a block: products of few output rows (N <= 2048) ----
+// Blocks of 16 rows put the 2B o / down projections (N = 1536) on 96 of the 256 compute units, and a unit pulls about 37 GB/s however many
+// waves it runs: down's 27.5 MB took 11.2 us.  Here a block owns 8 rows and the other half of the MFMA's A operand carries the NEXT 32 k of
+// the same rows: operand row i + 8 multiplies columns j + 8 of B, which hold the activations of that k, so D[i][j] + D[i + 8][j + 8] is the
+// product (the other two quarters are not used) and every load still brings 1 KB.  Up to 8 activation rows, kept in LDS (staged while the
+// first twelve loads of a wave are in flight; no registers for them, so that 8,960 k are all requested at once).  Decode step of a 2B
+// model, one stream of 500 keys: 1.315 -> 1.216 ms; of a 2B layer-list model: latent 1.394 -> 1.266, with recurrence 1.605 -> 1.538.
+LCC_DEVICE f32x4 shfl4(f32x4 v, int src) {
+  return (f32x4){__shfl(v[0], src, 64), __shfl(v[1], src, 64), __shfl(v[2], src, 64), __shfl(v[3], src, 64)};
+}
+template <int EPI, int NW>
+__global__ __launch_bounds__(NW * 64) void dgemv_rows8_kernel(DgArgs a) {
+  constexpr int UNR = 6, T = NW * 64, XP = 4, STEP = UNR * NW;
+  __shared__ f32x4 red[NW - 1][64];
+  extern __shared__ __attribute__((aligned(16))) bf16_t s_x[];          // [M][K]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, g = lane >> 4, hi = li >> 3;
+  const int M = a.M, N = a.N, K = a.K, n0 = blockIdx.x * 8;
+  const int nchunk = (K + 63) >> 6, K32 = K >> 5, kp = K >> 3, xpieces = M * kp;
+  const bf16_t* wp = a.W + (size_t)(n0 >> 4) * K32 * 512 + g * 128 + ((n0 & 8) + (li & 7)) * 8;
+  const bf16_t* sx = s_x + (size_t)min(li & 7, M - 1) * K + g * 8;
+
+  // the activations ahead of the weight stream (vmcnt retires in issue order), then two stages of weights
+  u32x4 xv[XP];
+#pragma unroll
+  for (int u = 0; u < XP; ++u) {
+    const int p = (int)threadIdx.x + u * T, pc = p < xpieces ? p : 0;
+    xv[u] = ld16(a.X + (size_t)(pc / kp) * a.ldx + (pc % kp) * 8);
+  }
+  u32x2 e_h = {0u, 0u}, e_c = {0u, 0u}, e_s = {0u, 0u};
+  f32x4 e_x = {0.f, 0.f, 0.f, 0.f};
+  float e_alpha = 0.f;
+  const int em = min(li, M - 1), en = n0 + (g & 1) * 4;                  // epilogue: lanes li < M of g 0, 1 own four outputs of row li
+  if (wave == 0) {
+    if (EPI == DG_EPI_RESID_DYT) {
+      e_x = *reinterpret_cast<const f32x4*>(a.X32 + (size_t)em * N + en);
+      e_c = ld8(a.dyt.w + en); e_s = ld8(a.dyt.b + en);
+      e_alpha = bf2f(a.dyt.alpha[0]);
+    }
+    if (EPI == DG_EPI_RESID) e_h = ld8(a.Hres + (size_t)em * N + en);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  u32x4 wa[UNR], wb[UNR];
+  auto load_w = [&](int c0, u32x4 (&w)[UNR]) {
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) w[u] = __builtin_nontemporal_load((const u32x4*)(wp + (size_t)min(2 * (c0 + u * NW) + hi, K32 - 1) * 512));
+  };
+  int c = wave;
+  load_w(c, wa);
+  load_w(c + STEP, wb);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < XP; ++u) {
+    const int p = (int)threadIdx.x + u * T;
+    if (p < xpieces) *reinterpret_cast<u32x4*>(s_x + (size_t)p * 8) = xv[u];
+  }
+  for (int p = (int)threadIdx.x + XP * T; p < xpieces; p += T)           // batches of several streams: the remaining pieces
+    *reinterpret_cast<u32x4*>(s_x + (size_t)p * 8) = ld16(a.X + (size_t)(p / kp) * a.ldx + (p % kp) * 8);
+  __syncthreads();
+  f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
+  auto mma = [&](const u32x4 (&w)[UNR], int c0) {
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) {
+      const int kb = 2 * (c0 + u * NW) + hi;
+      const u32x4 x = kb < K32 ? *reinterpret_cast<const u32x4*>(sx + kb * 32) : (u32x4){0u, 0u, 0u, 0u};
+      acc = mfma16(as_bf16x8(w[u]), as_bf16x8(x), acc);
+    }
+  };
+  for (; c < nchunk; c += 2 * STEP) {
+    mma(wa, c);
+    if (c + 2 * STEP < nchunk) load_w(c + 2 * STEP, wa);                 // wave-uniform
+    if (c + STEP < nchunk) mma(wb, c + STEP);
+    if (c + 3 * STEP < nchunk) load_w(c + 3 * STEP, wb);
+  }
+  if (wave > 0) red[wave - 1][lane] = acc;
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int w = 0; w < NW - 1; ++w) acc += red[w][lane];
+  acc += shfl4(acc, (lane + 40) & 63);                                   // rows i + 8, columns j + 8
+  const bool mine = li < M && g < 2;
+  if (EPI == DG_EPI_F32) {
+    if (mine) *reinterpret_cast<f32x4*>(a.C32 + (size_t)li * a.ldc + en) = acc;
+  } else if (EPI == DG_EPI_RESID_DYT) {
+    if (mine) {
+      const f32x4 v = e_x + acc;
+      *reinterpret_cast<f32x4*>(a.X32 + (size_t)li * N + en) = v;
+      st8(a.C + (size_t)li * N + en, (u32x2){pack2(dyt_value(v[0], e_alpha, lo2f(e_c.x), lo2f(e_s.x)), dyt_value(v[1], e_alpha, hi2f(e_c.x), hi2f(e_s.x))),
+                                             pack2(dyt_value(v[2], e_alpha, lo2f(e_c.y), lo2f(e_s.y)), dyt_value(v[3], e_alpha, hi2f(e_c.y), hi2f(e_s.y)))});
+    }
+  } else {          // DG_EPI_RESID: one sum of squares per 8 outputs (stats_out [M][N / 8])
+    const float v0 = rbf(lo2f(e_h.x) + rbf(acc[0])), v1 = rbf(hi2f(e_h.x) + rbf(acc[1]));
+    const float v2 = rbf(lo2f(e_h.y) + rbf(acc[2])), v3 = rbf(hi2f(e_h.y) + rbf(acc[3]));
+    if (mine) st8(a.Hres + (size_t)li * N + en, (u32x2){pack2(v0, v1), pack2(v2, v3)});
+    float ss = (v0 * v0 + v1 * v1) + (v2 * v2 + v3 * v3);
+    ss += __shfl_xor(ss, 16, 64);
+    if (mine && g == 0) a.stats_out[(size_t)li * (N >> 3) + blockIdx.x] = ss;
+  }
+}
+static int g_resid_waves = [] { const char* v = getenv("LCC_RESID_WAVES16"); return v ? atoi(v) : 1; }();
+// 16-row blocks that fill at most half the chip, whole 64-row groups of statistics, activations that fit LDS; modes 0 and 2
+// ask for blocks of 16 rows
+bool dgemv_rows8_ok(int M, int N, int K, const float* wscale) {
+  return (g_resid_waves == 1 || g_resid_waves == 3) && wscale == nullptr && M >= 1 && M <= 8 && N <= 2048 && (N & 31) == 0 && (K & 31) == 0 && (long)M * K <= 65536;
+}
+template <int EPI>
+static void launch_rows8(const DgArgs& a, hipStream_t st) {
+  if (a.K >= 4096) {
+    static DeviceOnce attr;
+    if (attr.first()) (void)hipFuncSetAttribute((const void*)dgemv_rows8_kernel<EPI, 16>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072);
+    dgemv_rows8_kernel<EPI, 16><<<dim3(a.N / 8), dim3(1024), (size_t)a.M * a.K * 2, st>>>(a);
+  } else {
+    static DeviceOnce attr;
+    if (attr.first()) (void)hipFuncSetAttribute((const void*)dgemv_rows8_kernel<EPI, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072);
+    dgemv_rows8_kernel<EPI, 8><<<dim3(a.N / 8), dim3(512), (size_t)a.M * a.K * 2, st>>>(a);
+  }
+}
+
 // ------------------------------------------------------------------------------------------------------------------------
 // step prologue: one block per stream does what were four launches (seen_set, embed_gather, mrope_table_decode, and the
 // first layer's RMSNorm statistic): marks the consumed token in the stream's seen-id bitmap (repetition penalty), gathers its
@@ -498,7 +615,7 @@ static int dg_check(const DgArgs& a, int pro, int epi) {
   if (a.M < 1 || a.M > 16 || (a.N & 15) || (a.K & 31) || a.W == nullptr) return LCC_ERR_SHAPE;
   if (a.wscale != nullptr && (a.K & 63)) return LCC_ERR_SHAPE;       // fp8 weights: whole 64-k fragments
   if (pro == DG_PRO_PLAIN && (a.X == nullptr || (a.ldx & 7))) return LCC_ERR_ARG;
-  if (pro == DG_PRO_NORM && (a.H == nullptr || a.stats == nullptr || a.norm_w == nullptr || a.n_stat != (a.K >> 4) || (a.n_stat & 3) ||
+  if (pro == DG_PRO_NORM && (a.H == nullptr || a.stats == nullptr || a.norm_w == nullptr || (a.n_stat != (a.K >> 4) && a.n_stat != (a.K >> 3)) || (a.n_stat & 3) ||
                              a.M > 4 || a.M * a.K > 16384 || a.n_stat > 512)) return LCC_ERR_ARG;
   if (epi == DG_EPI_RESID && (a.Hres == nullptr || a.stats_out == nullptr)) return LCC_ERR_ARG;
   if ((epi == DG_EPI_BF16 || epi == DG_EPI_SWIGLU) && a.C == nullptr) return LCC_ERR_ARG;
@@ -524,6 +641,7 @@ static int dg_f32_check(const DgArgs& a) {
 }
 int dgemv_f32(const DgArgs& a, hipStream_t st) {
   if (int rc = dg_f32_check(a)) return rc;
+  if (dgemv_rows8_ok(a.M, a.N, a.K, nullptr)) { launch_rows8<DG_EPI_F32>(a, st); return 0; }
   if (a.K >= 8192) dgemv_kernel<1, DG_PRO_PLAIN, DG_EPI_F32, 16, 3><<<dim3(a.N / 16), dim3(1024), 0, st>>>(a);
   else if (a.N >= 8192) dgemv_kernel<1, DG_PRO_PLAIN, DG_EPI_F32, 4, 2><<<dim3(a.N / 16), dim3(256), 0, st>>>(a);
   else dgemv_kernel<1, DG_PRO_PLAIN, DG_EPI_F32, 8, 4><<<dim3(a.N / 16), dim3(512), 0, st>>>(a);
@@ -556,6 +674,7 @@ int dgemv_resid_dyt(const DgArgs& a, hipStream_t st) {
   g_launch_counts[LC_DGEMV_V2]++;
   if (a.M < 1 || a.M > 16 || (a.N & 15) || (a.K & 31) || (a.ldx & 7)) return LCC_ERR_SHAPE;
   if (!a.W || !a.X || !a.X32 || !a.C || !a.dyt.w || !a.dyt.b || !a.dyt.alpha || a.wscale) return LCC_ERR_ARG;
+  if (dgemv_rows8_ok(a.M, a.N, a.K, nullptr)) { launch_rows8<DG_EPI_RESID_DYT>(a, st); return 0; }
   if (a.K >= 8192) dgemv_kernel<1, DG_PRO_PLAIN, DG_EPI_RESID_DYT, 16, 3><<<dim3(a.N / 16), dim3(1024), 0, st>>>(a);
   else dgemv_kernel<1, DG_PRO_PLAIN, DG_EPI_RESID_DYT, 8, 4><<<dim3(a.N / 16), dim3(512), 0, st>>>(a);
   return 0;
@@ -573,11 +692,15 @@ int dgemv_qkv_rope(const DgArgs& a, hipStream_t st) {
   else dgemv_kernel<1, DG_PRO_NORM, DG_EPI_ROPE, 8, 4, 4><<<dim3(a.N / 16), dim3(512), (size_t)a.M * a.K * 2, st>>>(a);
   return 0;
 }
-static int g_resid_waves = [] { const char* v = getenv("LCC_RESID_WAVES16"); return v ? atoi(v) : 1; }();
-int set_resid_waves(int mode) { const int old = g_resid_waves; g_resid_waves = mode < 0 ? 0 : (mode > 2 ? 2 : mode); return old; }
+int set_resid_waves(int mode) { const int old = g_resid_waves; g_resid_waves = mode < 0 ? 0 : (mode > 3 ? 3 : mode); return old; }
 // o_proj / down_proj: x plain, residual add in place + per-tile sums of squares
 int dgemv_resid(const DgArgs& a, hipStream_t st) {
   if (int rc = dg_check(a, DG_PRO_PLAIN, DG_EPI_RESID)) return rc;
+  if (a.rows8 || g_resid_waves == 3) {
+    if (!dgemv_rows8_ok(a.M, a.N, a.K, a.wscale)) return LCC_ERR_ARG;
+    launch_rows8<DG_EPI_RESID>(a, st);
+    return 0;
+  }
   // A block owns 16 rows x the whole K, so its waves' dependent chain of load stages is K / (64 NW UNR) round trips long: with 8 waves
   // the 7B down_proj (K = 18944) costs 12.7-14.6 us before / after its stream (tools/bench_dgemv_intercept.py: t = fixed + bytes / rate).
   // 1024-thread blocks (16 waves, UNR 3: 120 VGPRs at 4 waves per SIMD) halve that chain: 27.7 -> 25.1 us stand-alone, decode step
@@ -586,6 +709,7 @@ int dgemv_resid(const DgArgs& a, hipStream_t st) {
   // Mode (lcc_debug_set_resid_waves; initial value from LCC_RESID_WAVES16): 0 = 8 waves always, 1 (default) = 16 waves for bf16 weights
   // with K >= 8192, 2 = 16 waves for every call.
   const int w16 = g_resid_waves;
+  // 3 = blocks of 8 output rows (dgemv_rows8_kernel; the engine asks for them by DgArgs::rows8 where they suit).
   const bool wide = w16 == 2 || (w16 == 1 && a.K >= 8192 && a.wscale == nullptr);
   if (a.wscale != nullptr) {
     if (wide) dgemv_kernel<1, DG_PRO_PLAIN, DG_EPI_RESID, 16, 4, 4, true><<<dim3(a.N / 16), dim3(1024), 0, st>>>(a);

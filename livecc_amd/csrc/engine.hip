@@ -61,7 +61,7 @@ size_t lcc_engine::llm_ws_bytes() const {
   t += align_up(S * 64 * 2) * 2;             // cos, sin
   t += align_up(std::max((size_t)MAX_SPLIT * 64 * std::max<size_t>(qkvd, H), (size_t)6 * std::min<size_t>(S, 4096) * H) * 4);  // split-K slabs (up to 6 of S x H floats)
   t += align_up(B * H * 2) * 2;              // last_h, last_xn
-  t += align_up(16 * (H / 16 + 4) * 4);      // decode v2: per-tile sums of squares of the residual rows
+  t += align_up(16 * (H / 8 + 4) * 4);      // decode v2: per-tile sums of squares of the residual rows
   t += align_up(B * V * 2);                  // logits
   t += align_up(std::max<size_t>(B * c.n_kv_heads * 128 * 16, std::min<size_t>(S, 1024) * c.n_q_heads * 8) * 128 * 4) * 2;  // attention split partials (o, ml)
   if (c.llm_fp8) t += align_up(std::max<size_t>((size_t)qkvd * H, 2 * I * H) * 2);   // bf16 dequantisation scratch of the largest LLM weight

@@ -32,7 +32,7 @@ int carve_llm(lcc_engine* e, LlmBuffers* b) {
   b->cos = cv.take<bf16_t>(S * 64); b->sin = cv.take<bf16_t>(S * 64);
   b->partial = cv.take<float>(std::max((size_t)MAX_SPLIT * 64 * std::max<size_t>(e->qkvd, H), (size_t)6 * std::min<size_t>(S, 4096) * H));
   b->last_h = cv.take<bf16_t>(B * H); b->last_xn = cv.take<bf16_t>(B * H);
-  b->stats = cv.take<float>(16 * (H / 16 + 4));
+  b->stats = cv.take<float>(16 * (H / 8 + 4));
   b->logits = cv.take<bf16_t>(B * V);
   const size_t nslot = std::max<size_t>(B * e->c.n_kv_heads * 128 * 16, std::min<size_t>(S, 1024) * e->c.n_q_heads * 8);
   b->ws_o = cv.take<float>(nslot * 128); b->ws_ml = cv.take<float>(nslot * 128);
@@ -197,7 +197,7 @@ bool decode_v2_ok(const lcc_engine* e) {
 // decode_step_begin; on exit b.h is the residual stream after the last layer and b.stats its per-tile sums of squares (the final
 // RMSNorm runs as the prologue of the lm_head GEMV).
 int run_decode_layers_v2(lcc_engine* e, const LlmBuffers& b, int B, const int32_t* d_slots, int nsplit_attn, hipStream_t st,
-                         const AttnDirect* direct = nullptr) {
+                         const AttnDirect* direct, int* n_stat_out) {
   const int H = e->c.hidden_size, I = e->c.intermediate_size;
   const float eps = e->c.rms_eps;
   if (e->llm_over) return fail(LCC_ERR_STATE, "per-layer input overrides are a prefill-only instrument (decode pipeline v2 carries row statistics)");
@@ -207,9 +207,11 @@ int run_decode_layers_v2(lcc_engine* e, const LlmBuffers& b, int B, const int32_
   // chained launches: down_proj of layer l and q/k/v of layer l+1 in ONE launch (the consumer's weights stream under the producer's
   // tail: decode_v2.hip).  Only when both grids fit the chip at once, <= 2 streams, <= 127 layers, and no parity taps are bound
   // (a tap copy between the two halves would have to sit inside the launch).
+  // statistics per row that the last residual product left (8- or 16-row blocks); the step's prologue leaves one per 16 channels
+  int n_stat = H / 16;
   auto qkv_args = [&](int l) {
     const LlmLayerW& L = e->llm[l];
-    DgArgs a; a.W = L.qkv_w_dec; a.wscale = L.qkv_s_dec; a.M = B; a.N = e->qkvd; a.K = H; a.H = b.h; a.stats = b.stats; a.n_stat = H / 16; a.norm_w = L.in_norm;
+    DgArgs a; a.W = L.qkv_w_dec; a.wscale = L.qkv_s_dec; a.M = B; a.N = e->qkvd; a.K = H; a.H = b.h; a.stats = b.stats; a.n_stat = n_stat; a.norm_w = L.in_norm;
     a.eps = eps; a.bias = L.qkv_b; a.cs = b.cos; a.sn = b.sin; a.tok_stream = d_slots; a.kv_len = e->d_kv_len; a.kv_base = e->d_kv_base;
     a.lay = e->lay; a.layer = l; a.q_out = b.q; a.n_q_heads = e->c.n_q_heads;
     return a;
@@ -222,9 +224,11 @@ int run_decode_layers_v2(lcc_engine* e, const LlmBuffers& b, int B, const int32_
     if (l == 0 || !chain) LCC_TRY(dgemv_qkv_rope(qkv_args(l), st));     // otherwise launched together with the previous layer's down_proj
     LCC_TRY(attn_decode_bf16(b.q, b.attn, d_slots, e->d_kv_len, e->d_kv_base, e->lay, l, B, e->c.n_q_heads, nsplit_attn, b.ws_o, b.ws_ml, st, direct));
     a = DgArgs(); a.W = L.o_w; a.wscale = L.o_s; a.M = B; a.N = H; a.K = e->qd; a.X = b.attn; a.ldx = e->qd; a.Hres = b.h; a.stats_out = b.stats;
+    a.rows8 = dgemv_rows8_ok(B, H, e->qd, L.o_s);
     LCC_TRY(dgemv_resid(a, st));
+    n_stat = a.rows8 ? H / 8 : H / 16;
     if (e->llm_taps) HIP_TRY(hipMemcpyAsync(e->llm_taps + (size_t)(2 * l + 1) * tap_stride, b.h, tap_bytes, hipMemcpyDeviceToDevice, st));
-    a = DgArgs(); a.W = L.gate_up_w; a.wscale = L.gate_up_s; a.M = B; a.N = 2 * I; a.K = H; a.H = b.h; a.stats = b.stats; a.n_stat = H / 16; a.norm_w = L.post_norm;
+    a = DgArgs(); a.W = L.gate_up_w; a.wscale = L.gate_up_s; a.M = B; a.N = 2 * I; a.K = H; a.H = b.h; a.stats = b.stats; a.n_stat = n_stat; a.norm_w = L.post_norm;
     a.eps = eps; a.C = b.act; a.ldc = I;
     const bool prof = e->prof_on && l == e->c.n_layers / 2 && 2 * (e->prof_n + 1) <= (int)e->prof_ev.size();   // one sample per step
     // the sampled launch carries its events on the dispatch (kernel begin / end timestamps: kernels.h)
@@ -234,22 +238,26 @@ int run_decode_layers_v2(lcc_engine* e, const LlmBuffers& b, int B, const int32_
     a = DgArgs(); a.W = L.down_w; a.wscale = L.down_s; a.M = B; a.N = H; a.K = I; a.X = b.act; a.ldx = I; a.Hres = b.h; a.stats_out = b.stats;
     if (chain && l + 1 < e->c.n_layers) {
       const unsigned target = ++e->chain_epoch[l] * (unsigned)(H / 16);     // monotonic counter: every launch adds H/16 arrivals
+      n_stat = H / 16;          // the chained launch writes (and its consumer half reads) one per 16
       LCC_TRY(dgemv_down_qkv(a, qkv_args(l + 1), e->d_chain + l, target, e->d_chain + 128, st));
     } else {
+      a.rows8 = dgemv_rows8_ok(B, H, I, L.down_s);
       LCC_TRY(dgemv_resid(a, st));
+      n_stat = a.rows8 ? H / 8 : H / 16;
     }
     if (e->llm_taps) HIP_TRY(hipMemcpyAsync(e->llm_taps + (size_t)(2 * l + 2) * tap_stride, b.h, tap_bytes, hipMemcpyDeviceToDevice, st));
   }
+  *n_stat_out = n_stat;
   return 0;
 }
 
 int head_and_sample(lcc_engine* e, const LlmBuffers& b, const bf16_t* xn_rows, int B, const int32_t* d_slots, const lcc_sampling* sp,
-                    int step_index, hipStream_t st) {
+                    int step_index, hipStream_t st, int n_stat = 0) {
   const int H = e->c.hidden_size, V = e->c.vocab_size;
   bf16_t* logits = b.logits;
   if (sp && sp->logits_out) logits = (bf16_t*)sp->logits_out + (size_t)step_index * B * V;
   if (xn_rows == nullptr) {   // decode v2: final RMSNorm of b.h as the prologue of the lm_head GEMV
-    DgArgs a; a.W = e->lm_head; a.wscale = e->lm_head_s; a.M = B; a.N = V; a.K = H; a.H = b.h; a.stats = b.stats; a.n_stat = H / 16; a.norm_w = e->final_norm;
+    DgArgs a; a.W = e->lm_head; a.wscale = e->lm_head_s; a.M = B; a.N = V; a.K = H; a.H = b.h; a.stats = b.stats; a.n_stat = n_stat; a.norm_w = e->final_norm;
     a.eps = e->c.rms_eps; a.C = logits; a.ldc = V;
     LCC_TRY(dgemv_norm_bf16(a, st));
   } else {
@@ -459,9 +467,14 @@ extern "C" int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots
   }
   LlmBuffers bf; LCC_TRY(carve_llm(e, &bf));
   const int ntile = (max_len + 31) / 32;
-  // key tiles per split of the per-wave decode attention (tuning knob LCC_ATTN_TPS, default 4) and the split cap (LCC_ATTN_MAXSPLIT, 64)
-  static const int tps = [] { const char* v = getenv("LCC_ATTN_TPS"); return v ? std::max(1, atoi(v)) : 4; }();
-  static const int maxsplit = [] { const char* v = getenv("LCC_ATTN_MAXSPLIT"); return v ? std::max(1, std::min(128, atoi(v))) : 64; }();
+  // key tiles per split of the per-wave decode attention: one up to 24 tiles, two beyond -- a wave's first two tiles are requested together,
+  // every further pair is another trip, and the merge fetches up to 64 splits in one (decode step, 1 / 2 / 4 tiles a split: 2B at 500 keys
+  // 1.168 / 1.177 / 1.216 ms, 7B at 2,000 keys 2.792 / 2.787 / 2.825).  64 splits
+  // at most up to 16k keys, 128 beyond: 9,000 keys 2.930 / 2.948 ms with 64 / 128, 24,000 keys 3.136 / 3.067.  Tuning knobs LCC_ATTN_TPS, LCC_ATTN_MAXSPLIT
+  static const int tps_env = [] { const char* v = getenv("LCC_ATTN_TPS"); return v ? std::max(1, atoi(v)) : 0; }();
+  static const int maxsplit_env = [] { const char* v = getenv("LCC_ATTN_MAXSPLIT"); return v ? std::max(1, std::min(128, atoi(v))) : 0; }();
+  const int maxsplit = maxsplit_env ? maxsplit_env : (ntile <= 512 ? 64 : 128);
+  const int tps = tps_env ? tps_env : (ntile <= 24 ? 1 : 2);
   const int nsplit = std::max(1, std::min(maxsplit, (ntile + tps - 1) / tps));
 
   LayerCtx cx{};
@@ -480,6 +493,7 @@ extern "C" int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots
   // two, but 640 vs 655 for four: with more rows the per-block normalisation prologue outweighs the saved launches)
   const bool v2 = decode_v2_ok(e) && n_streams <= 2 && (long)n_streams * e->c.hidden_size <= 16384;
   for (int step = 0; step < n_steps; ++step) {
+    int n_stat = 0;
     const bool prof_step = e->prof_on && (step & 3) == 0 && 2 * (e->step_n + 1) <= (int)e->step_ev.size();   // every 4th step
     if (prof_step) HIP_TRY(hipEventRecord(e->step_ev[2 * e->step_n], st));
     // the token sampled by the previous step (d_cur_tok[slot]) is embedded, appended at kv_len[slot], position pos[slot]
@@ -493,7 +507,7 @@ extern "C" int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots
         for (int bb = 0; bb < n_streams; ++bb) { dir.base[bb] = (const bf16_t*)e->h_kv_base[slots[bb]]; dir.n[bb] = e->h_kv_len[slots[bb]] + step + 1; }
         dir.used = n_streams;
       }
-      LCC_TRY(run_decode_layers_v2(e, bf, n_streams, d_slots, nsplit, st, dir.used ? &dir : nullptr));
+      LCC_TRY(run_decode_layers_v2(e, bf, n_streams, d_slots, nsplit, st, dir.used ? &dir : nullptr, &n_stat));
     } else {
       LCC_TRY(seen_set(e->d_seen, e->words, e->d_cur_tok, d_slots, n_streams, 1, e->d_done, st));
       LCC_TRY(embed_gather_bf16(e->d_cur_tok, d_slots, nullptr, e->embed, nullptr, bf.h, n_streams, e->c.hidden_size, st));
@@ -502,7 +516,7 @@ extern "C" int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots
       if (!cx.skinny) LCC_TRY(rmsnorm_bf16(bf.h, e->final_norm, bf.xn, n_streams, e->c.hidden_size, e->c.rms_eps, st));
     }
     LCC_TRY(advance_lengths(d_slots, e->d_kv_len, e->d_pos, n_streams, e->d_done, st));
-    LCC_TRY(head_and_sample(e, bf, v2 ? nullptr : bf.xn, n_streams, d_slots, sp, first_step_index + step, st));
+    LCC_TRY(head_and_sample(e, bf, v2 ? nullptr : bf.xn, n_streams, d_slots, sp, first_step_index + step, st, n_stat));
     if (prof_step) {
       HIP_TRY(hipEventRecord(e->step_ev[2 * e->step_n + 1], st));
       if (e->step_n < (int)e->step_rel.size()) e->step_rel[e->step_n] = step;

@@ -201,7 +201,7 @@ struct DgArgs {
   const bf16_t* X = nullptr; int ldx = 0;                                      // plain activation rows [M, K]
   const bf16_t* H = nullptr; const float* stats = nullptr; int n_stat = 0; const bf16_t* norm_w = nullptr; float eps = 0.f;  // RMSNorm prologue
   const bf16_t* bias = nullptr; bf16_t* C = nullptr; int ldc = 0;              // bf16 / SwiGLU epilogue
-  bf16_t* Hres = nullptr; float* stats_out = nullptr;                          // residual epilogue
+  bf16_t* Hres = nullptr; float* stats_out = nullptr; bool rows8 = false;      // residual epilogue; rows8: blocks of 8 rows, stats_out [M][N / 8]
   const bf16_t* cs = nullptr; const bf16_t* sn = nullptr; const int32_t* tok_stream = nullptr; const int32_t* kv_len = nullptr;
   bf16_t* const* kv_base = nullptr; KvLayout lay = {0, 0, 0, 0}; int layer = 0; bf16_t* q_out = nullptr; int n_q_heads = 0;   // rope epilogue
   const float* S32 = nullptr; int lds32 = 0, rank = 0;                          // RMS prologue over fp32 rows [M][lds32], K stored and `rank` real channels (norm_w, eps)
@@ -213,6 +213,7 @@ int decode_step_begin(const int32_t* slots, const int32_t* cur_tok, const int32_
                       hipStream_t st);
 int dgemv_qkv_rope(const DgArgs& a, hipStream_t st);      // [RMSNorm] q|k|v Linear (row-permuted decode copy) [bias + M-RoPE + KV append]
 int set_resid_waves(int mode);   // 0: 8-wave blocks, 1: 16 waves for bf16 weights with K >= 8192 (default), 2: 16 waves always; returns the old mode
+bool dgemv_rows8_ok(int M, int N, int K, const float* wscale);      // blocks of 8 output rows serve (and suit) the product
 int dgemv_resid(const DgArgs& a, hipStream_t st);         // o_proj / down_proj [residual add in place + per-tile sums of squares]
 int dgemv_norm_swiglu(const DgArgs& a, hipStream_t st);   // [RMSNorm] gate/up Linear [SwiGLU]
 // Live timing of the dominant kernel (round 6): the NEXT dgemv_norm_swiglu launch of this host thread carries the two events ON THE DISPATCH

@@ -67,6 +67,27 @@ def test_residual_gemv_and_tile_statistics(dev, M, N, K, resid_waves):
     assert torch.allclose(stats, want, rtol=1e-6, atol=1e-6), float((stats - want).abs().max())
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 32, 32), (1, 1536, 8960), (2, 1536, 1536), (3, 96, 96), (4, 2048, 4064), (5, 1536, 10496), (7, 64, 4128), (8, 896, 2464),
+                                   (8, 1536, 8192)])
+def test_residual_gemv_in_blocks_of_eight_rows(dev, M, N, K):
+    """One 32-k block (the operand's other half is absent), odd and even counts of them, fewer chunks than waves, 8- and 16-wave blocks (K from
+    4096 on), activations beyond the staging registers, every row count up to 8; a statistic per 8 outputs of the rows the kernel wrote."""
+    from livecc_amd import _lib, ops
+    lib = _lib.load()
+    x, w, h0 = _rand((M, K), dev, 1.0, 7), _rand((N, K), dev, 0.03, 8), _rand((M, N), dev, 2.0, 9)
+    h, wp, stats = h0.clone(), ops.pack_weight(w), torch.full((M, N // 8), -1.0, device=dev)
+    old = lib.lcc_debug_set_resid_waves(3)
+    try:
+        _lib.check(lib.lcc_dgemv_resid(wp.data_ptr(), None, x.data_ptr(), K, h.data_ptr(), stats.data_ptr(), M, N, K,
+                                       torch.cuda.current_stream(dev).cuda_stream), "lcc_dgemv_resid")
+    finally:
+        lib.lcc_debug_set_resid_waves(old)
+    ref, atol = _ref_linear(x, w, None, 3, h0, with_atol=True)
+    assert_bf16_close(h, ref, f"dgemv_resid8[{M}x{N}x{K}]", max_ulp=1.0, max_frac=1e-2, atol=atol)
+    want = h.float().view(M, N // 8, 8).pow(2).sum(-1)
+    assert torch.allclose(stats, want, rtol=1e-6, atol=1e-6)
+
+
 @pytest.mark.parametrize("Hq,Hkv,K", [(28, 4, 3584), (12, 2, 1536), (2, 1, 256), (7, 1, 896)])
 @pytest.mark.parametrize("M", [1, 2])
 def test_qkv_gemv_with_rope_and_kv_append(dev, Hq, Hkv, K, M):
