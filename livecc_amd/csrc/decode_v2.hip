@@ -36,6 +36,7 @@ namespace lcc {
 __device__ unsigned int lcc_zero_page_v2[64];  // 256 zero bytes: activation operand of absent K chunks
 
 enum { DG_PRO_PLAIN = 0, DG_PRO_NORM = 1, DG_PRO_RMS32 = 2 };      // RMS32: fp32 rows, the wave that normalises a row forms its statistic
+constexpr int X_PAD = 32;                    // elements after each activation row in LDS: rows of whole 256 bytes would all start in one bank
 enum { DG_EPI_BF16 = 0, DG_EPI_SWIGLU = 1, DG_EPI_RESID = 2, DG_EPI_ROPE = 3, DG_EPI_F32 = 4, DG_EPI_RESID_DYT = 5 };
 
 // ---- chained launches (round 3): two dependent GEMVs in ONE launch.  The consumer's blocks (q/k/v of layer l+1) are resident next to
@@ -85,7 +86,15 @@ constexpr int dgemv_min_waves_per_simd() {
   return MR > 2 ? 1 : ((NTILE == 2 && PRO == DG_PRO_NORM && NW == 4) ? 5 : ((EPI == DG_EPI_ROPE && NW == 8) ? 4 : 1));
 }
 
-template <int NTILE, int PRO, int EPI, int NW, int UNR, int MR, int CHAIN, bool W8 = false>
+// US (row-scaled products): the activations are u = bf16(w * h) of the RMSNorm's weight and the residual row, and the row's 1 / rms multiplies the
+// finished fp32 sums.  The producer of h writes u beside it (EPI_RESID with US: norm_w = the next norm's weight, C = u), so there is neither a
+// norm launch nor a normalisation in every block, and one rounding less than bf16(w * bf16(h / rms)).  The n_stat sums of squares of each row
+// go through LDS: every thread fetches a few 16-byte pieces of them ahead of its weights, wave 0 adds them up after it merged the waves.
+// For 3 to 16 streams (engine_llm.hip), whose rows do not fit the normalising prologue; bound by the weight stream.  7B, eight streams of
+// 1,000 keys: gate/up 43.3 us (as before, 5.9 TB/s), down 26.7 and o 7.6 with the residual added where it was 27.2 and 7.4 plus 4.7 each for add + norm; the
+// decode step 3.38 -> 3.25 ms, four streams 3.22 -> 3.02, eight with fp8 weights 2.53 -> 2.30, 2B eight streams 1.43 -> 1.27.  Activations
+// copied to LDS first (up to 64 KB) instead of fetched beside the weights: the same times.
+template <int NTILE, int PRO, int EPI, int NW, int UNR, int MR, int CHAIN, bool W8 = false, bool US = false>
 LCC_DEVICE void dgemv_body(const DgArgs& a, const DgChain& ch, const int bid, f32x4 (*red)[NTILE][64], bf16_t* s_x) {
   static_assert(EPI != DG_EPI_SWIGLU || NTILE == 2, "swiglu needs the gate and the up tile in one block");
   static_assert(EPI == DG_EPI_SWIGLU || NTILE == 1, "one tile per block");
@@ -196,6 +205,15 @@ LCC_DEVICE void dgemv_body(const DgArgs& a, const DgChain& ch, const int bid, f3
   const int kp = K >> 3, xpieces = PRO == DG_PRO_NORM ? M * kp : 0;
   f32x4 pv[PRO == DG_PRO_NORM ? MR : 1][2];
   u32x4 hv[PRO == DG_PRO_NORM ? XP : 1], nv[PRO == DG_PRO_NORM ? XP : 1];
+  constexpr int SU = US && EPI != DG_EPI_RESID ? 4 : 1;
+  constexpr bool RSC = US && EPI != DG_EPI_RESID;                    // 1 / rms in the epilogue
+  float* s_st = reinterpret_cast<float*>(s_x);      // [M][n_stat / 4]
+  const int stp = RSC ? M * n4 : 0;
+  f32x4 stv[SU];
+  if (RSC) {
+#pragma unroll
+    for (int u = 0; u < SU; ++u) stv[u] = *reinterpret_cast<const f32x4*>(a.stats + 4 * (size_t)min((int)threadIdx.x + u * T, stp - 1));
+  }
   // PRO_RMS32: wave m normalises row m (M <= NW, K <= 2048): 4-channel pieces lane, lane + 64, ..
   constexpr int SP = PRO == DG_PRO_RMS32 ? 8 : 1;
   f32x4 sv[SP];
@@ -240,6 +258,7 @@ LCC_DEVICE void dgemv_body(const DgArgs& a, const DgChain& ch, const int bid, f3
     if (EPI == DG_EPI_RESID) {
       const int n = n0 + g * 4;
       if (li < M && n < N) e_h = ld8(a.Hres + (size_t)li * N + n);
+      if (US) e_c = ld8(a.norm_w + min(n, N - 4));
     } else if (EPI == DG_EPI_ROPE) {
       const int tile = n0 >> 4, head = tile >> 3, j = tile & 7;
       const int dc = j * 8 + (g & 1) * 4, d = (g >> 1) * 64 + dc;
@@ -261,6 +280,17 @@ LCC_DEVICE void dgemv_body(const DgArgs& a, const DgChain& ch, const int bid, f3
   load_x(c, sa);
   load_x(c + STEP, sb);
   __builtin_amdgcn_sched_barrier(0);
+  if (RSC) {
+#pragma unroll
+    for (int u = 0; u < SU; ++u) {
+      const int p = (int)threadIdx.x + u * T;
+      if (p < stp) s_st[p] = (stv[u][0] + stv[u][1]) + (stv[u][2] + stv[u][3]);
+    }
+    for (int p = (int)threadIdx.x + SU * T; p < stp; p += T) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(a.stats + 4 * (size_t)p);
+      s_st[p] = (v[0] + v[1]) + (v[2] + v[3]);
+    }
+  }
   if (PRO == DG_PRO_NORM) {
     float rr[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -319,6 +349,15 @@ LCC_DEVICE void dgemv_body(const DgArgs& a, const DgChain& ch, const int bid, f3
     for (int w = 0; w < NW - 1; ++w) acc[t] += red[w][t][lane];
     if (W8) acc[t] *= *reinterpret_cast<const f32x4*>(a.wscale + min(n0 + t * 16 + g * 4, N - 4));   // per-stored-row dequantisation scale
   }
+  if (RSC) {          // this lane's activation row: a quarter of its sums in each lane group, then across the groups
+    float ss = 0.f;
+    for (int i = g; i < n4; i += 4) ss += s_st[xm * n4 + i];
+    ss += __shfl_xor(ss, 16, 64);
+    ss += __shfl_xor(ss, 32, 64);
+    const float r = rsqrtf(ss / (float)K + a.eps);
+#pragma unroll
+    for (int t = 0; t < NTILE; ++t) acc[t] *= r;
+  }
 
   if (EPI == DG_EPI_BF16) {
     if (li >= M) return;
@@ -357,6 +396,7 @@ LCC_DEVICE void dgemv_body(const DgArgs& a, const DgChain& ch, const int bid, f3
       const float v2 = rbf(lo2f(hv.y) + rbf(acc[0][2])), v3 = rbf(hi2f(hv.y) + rbf(acc[0][3]));
       if (CHAIN == DG_CHAIN_SIGNAL) st8_agent(hp, (u32x2){pack2(v0, v1), pack2(v2, v3)});
       else st8(hp, (u32x2){pack2(v0, v1), pack2(v2, v3)});
+      if (US) st8(a.C + (size_t)li * N + n, (u32x2){pack2(v0 * lo2f(e_c.x), v1 * hi2f(e_c.x)), pack2(v2 * lo2f(e_c.y), v3 * hi2f(e_c.y))});
       ss = (v0 * v0 + v1 * v1) + (v2 * v2 + v3 * v3);
     }
     ss += __shfl_xor(ss, 16, 64);
@@ -414,6 +454,13 @@ __global__ __launch_bounds__(NW * 64, (dgemv_min_waves_per_simd<NTILE, PRO, EPI,
   extern __shared__ __attribute__((aligned(16))) bf16_t s_x[];   // PRO_NORM: M * K bf16 (dynamic: 7 KB for one stream at 7B)
   dgemv_body<NTILE, PRO, EPI, NW, UNR, MR, DG_CHAIN_NONE, W8>(a, DgChain{nullptr, 0u, nullptr, 0}, blockIdx.x, red, s_x);
 }
+// row-scaled products (US).  MINW: waves per SIMD the registers must leave room for (the grids of the two-block classes fit one round)
+template <int NTILE, int EPI, int NW, int UNR, int MINW, bool W8>
+__global__ __launch_bounds__(NW * 64, MINW) void dgemv_us_kernel(DgArgs a) {
+  __shared__ f32x4 red[NW - 1][NTILE][64];
+  extern __shared__ __attribute__((aligned(16))) bf16_t s_x[];   // [M][n_stat / 4] floats (no residual product: none)
+  dgemv_body<NTILE, DG_PRO_PLAIN, EPI, NW, UNR, 2, DG_CHAIN_NONE, W8, true>(a, DgChain{nullptr, 0u, nullptr, 0}, blockIdx.x, red, s_x);
+}
 
 // down_proj of layer l (blocks [0, nb_down): producer, publishes the residual stream + its tile statistics) and the q/k/v GEMV of
 // layer l+1 (the remaining blocks: consumer) in ONE launch.  512-thread blocks, <= 128 VGPRs: two blocks per CU, so all
@@ -455,22 +502,25 @@ __global__ __launch_bounds__(512, 2) void dgemv_latent_q_kernel(DgArgs a, Latent
 // Blocks of 16 rows put the 2B o / down projections (N = 1536) on 96 of the 256 compute units, and a unit pulls about 37 GB/s however many
 // waves it runs: down's 27.5 MB took 11.2 us.  Here a block owns 8 rows and the other half of the MFMA's A operand carries the NEXT 32 k of
 // the same rows: operand row i + 8 multiplies columns j + 8 of B, which hold the activations of that k, so D[i][j] + D[i + 8][j + 8] is the
-// product (the other two quarters are not used) and every load still brings 1 KB.  Up to 8 activation rows, kept in LDS (staged while the
-// first twelve loads of a wave are in flight; no registers for them, so that 8,960 k are all requested at once).  Decode step of a 2B
+// product (the other two quarters are not used) and every load still brings 1 KB.  Up to 8 activation rows, kept in LDS (requested ahead of
+// the weights, up to nine 16-byte pieces a thread, and stored while the first twelve weight loads of a wave are in flight).  Decode step of a 2B
 // model, one stream of 500 keys: 1.315 -> 1.216 ms; of a 2B layer-list model: latent 1.394 -> 1.266, with recurrence 1.605 -> 1.538.
+// activations; 15 KB of wave sums beside them.  Eight rows of 8,960 k fit (2B down: 12.8 us in 16-row blocks, 9.5 here)
+constexpr int ROWS8_LDS = 144 * 1024;
 LCC_DEVICE f32x4 shfl4(f32x4 v, int src) {
   return (f32x4){__shfl(v[0], src, 64), __shfl(v[1], src, 64), __shfl(v[2], src, 64), __shfl(v[3], src, 64)};
 }
-template <int EPI, int NW>
+template <int EPI, int NW, int XP>
 __global__ __launch_bounds__(NW * 64) void dgemv_rows8_kernel(DgArgs a) {
-  constexpr int UNR = 6, T = NW * 64, XP = 4, STEP = UNR * NW;
+  constexpr int UNR = 6, T = NW * 64, STEP = UNR * NW;
   __shared__ f32x4 red[NW - 1][64];
-  extern __shared__ __attribute__((aligned(16))) bf16_t s_x[];          // [M][K]
+  extern __shared__ __attribute__((aligned(16))) bf16_t s_x[];          // [M][K + X_PAD]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, g = lane >> 4, hi = li >> 3;
   const int M = a.M, N = a.N, K = a.K, n0 = blockIdx.x * 8;
   const int nchunk = (K + 63) >> 6, K32 = K >> 5, kp = K >> 3, xpieces = M * kp;
   const bf16_t* wp = a.W + (size_t)(n0 >> 4) * K32 * 512 + g * 128 + ((n0 & 8) + (li & 7)) * 8;
-  const bf16_t* sx = s_x + (size_t)min(li & 7, M - 1) * K + g * 8;
+  const int ks = K + X_PAD;
+  const bf16_t* sx = s_x + (size_t)min(li & 7, M - 1) * ks + g * 8;
 
   // the activations ahead of the weight stream (vmcnt retires in issue order), then two stages of weights
   u32x4 xv[XP];
@@ -489,7 +539,10 @@ __global__ __launch_bounds__(NW * 64) void dgemv_rows8_kernel(DgArgs a) {
       e_c = ld8(a.dyt.w + en); e_s = ld8(a.dyt.b + en);
       e_alpha = bf2f(a.dyt.alpha[0]);
     }
-    if (EPI == DG_EPI_RESID) e_h = ld8(a.Hres + (size_t)em * N + en);
+    if (EPI == DG_EPI_RESID) {
+      e_h = ld8(a.Hres + (size_t)em * N + en);
+      if (a.C != nullptr) e_c = ld8(a.norm_w + en);
+    }
   }
   __builtin_amdgcn_sched_barrier(0);
   u32x4 wa[UNR], wb[UNR];
@@ -504,10 +557,10 @@ __global__ __launch_bounds__(NW * 64) void dgemv_rows8_kernel(DgArgs a) {
 #pragma unroll
   for (int u = 0; u < XP; ++u) {
     const int p = (int)threadIdx.x + u * T;
-    if (p < xpieces) *reinterpret_cast<u32x4*>(s_x + (size_t)p * 8) = xv[u];
+    if (p < xpieces) *reinterpret_cast<u32x4*>(s_x + (size_t)(p / kp) * ks + (p % kp) * 8) = xv[u];
   }
   for (int p = (int)threadIdx.x + XP * T; p < xpieces; p += T)           // batches of several streams: the remaining pieces
-    *reinterpret_cast<u32x4*>(s_x + (size_t)p * 8) = ld16(a.X + (size_t)(p / kp) * a.ldx + (p % kp) * 8);
+    *reinterpret_cast<u32x4*>(s_x + (size_t)(p / kp) * ks + (p % kp) * 8) = ld16(a.X + (size_t)(p / kp) * a.ldx + (p % kp) * 8);
   __syncthreads();
   f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
   auto mma = [&](const u32x4 (&w)[UNR], int c0) {
@@ -544,6 +597,8 @@ __global__ __launch_bounds__(NW * 64) void dgemv_rows8_kernel(DgArgs a) {
     const float v0 = rbf(lo2f(e_h.x) + rbf(acc[0])), v1 = rbf(hi2f(e_h.x) + rbf(acc[1]));
     const float v2 = rbf(lo2f(e_h.y) + rbf(acc[2])), v3 = rbf(hi2f(e_h.y) + rbf(acc[3]));
     if (mine) st8(a.Hres + (size_t)li * N + en, (u32x2){pack2(v0, v1), pack2(v2, v3)});
+    if (mine && a.C != nullptr)          // the next product's activations (dgemv_body: US)
+      st8(a.C + (size_t)li * N + en, (u32x2){pack2(v0 * lo2f(e_c.x), v1 * hi2f(e_c.x)), pack2(v2 * lo2f(e_c.y), v3 * hi2f(e_c.y))});
     float ss = (v0 * v0 + v1 * v1) + (v2 * v2 + v3 * v3);
     ss += __shfl_xor(ss, 16, 64);
     if (mine && g == 0) a.stats_out[(size_t)li * (N >> 3) + blockIdx.x] = ss;
@@ -553,18 +608,23 @@ static int g_resid_waves = [] { const char* v = getenv("LCC_RESID_WAVES16"); ret
 // 16-row blocks that fill at most half the chip, whole 64-row groups of statistics, activations that fit LDS; modes 0 and 2
 // ask for blocks of 16 rows
 bool dgemv_rows8_ok(int M, int N, int K, const float* wscale) {
-  return (g_resid_waves == 1 || g_resid_waves == 3) && wscale == nullptr && M >= 1 && M <= 8 && N <= 2048 && (N & 31) == 0 && (K & 31) == 0 && (long)M * K <= 65536;
+  return (g_resid_waves == 1 || g_resid_waves == 3) && wscale == nullptr && M >= 1 && M <= 8 && N <= 2048 && (N & 31) == 0 && (K & 31) == 0 && (long)M * (K + X_PAD) * 2 <= ROWS8_LDS;
+}
+template <int EPI, int NW, int XP>
+static void launch_rows8_as(const DgArgs& a, hipStream_t st) {
+  static DeviceOnce attr;
+  if (attr.first()) (void)hipFuncSetAttribute((const void*)dgemv_rows8_kernel<EPI, NW, XP>, hipFuncAttributeMaxDynamicSharedMemorySize, ROWS8_LDS);
+  dgemv_rows8_kernel<EPI, NW, XP><<<dim3(a.N / 8), dim3(NW * 64), (size_t)a.M * (a.K + X_PAD) * 2, st>>>(a);
 }
 template <int EPI>
 static void launch_rows8(const DgArgs& a, hipStream_t st) {
-  if (a.K >= 4096) {
-    static DeviceOnce attr;
-    if (attr.first()) (void)hipFuncSetAttribute((const void*)dgemv_rows8_kernel<EPI, 16>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072);
-    dgemv_rows8_kernel<EPI, 16><<<dim3(a.N / 8), dim3(1024), (size_t)a.M * a.K * 2, st>>>(a);
+  const int nw = a.K >= 4096 ? 16 : 8, pieces = a.M * (a.K >> 3);
+  if (nw == 16) {
+    if (pieces <= 4 * 1024) launch_rows8_as<EPI, 16, 4>(a, st);
+    else launch_rows8_as<EPI, 16, 9>(a, st);
   } else {
-    static DeviceOnce attr;
-    if (attr.first()) (void)hipFuncSetAttribute((const void*)dgemv_rows8_kernel<EPI, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072);
-    dgemv_rows8_kernel<EPI, 8><<<dim3(a.N / 8), dim3(512), (size_t)a.M * a.K * 2, st>>>(a);
+    if (pieces <= 4 * 512) launch_rows8_as<EPI, 8, 4>(a, st);
+    else launch_rows8_as<EPI, 8, 9>(a, st);
   }
 }
 
@@ -576,7 +636,8 @@ static void launch_rows8(const DgArgs& a, hipStream_t st) {
 __global__ __launch_bounds__(256) void decode_step_begin_kernel(
     const int32_t* __restrict__ slots, const int32_t* __restrict__ cur_tok, const int32_t* __restrict__ done, uint32_t* __restrict__ seen,
     int words, const bf16_t* __restrict__ table, bf16_t* __restrict__ h, float* __restrict__ stats, int dim,
-    const int32_t* __restrict__ pos, const float* __restrict__ inv_freq, bf16_t* __restrict__ cs, bf16_t* __restrict__ sn) {
+    const int32_t* __restrict__ pos, const float* __restrict__ inv_freq, bf16_t* __restrict__ cs, bf16_t* __restrict__ sn,
+    const bf16_t* __restrict__ norm_w, bf16_t* __restrict__ u) {
   const int b = blockIdx.x, t = threadIdx.x;
   const int slot = slots[b];
   const int id = cur_tok[slot];
@@ -590,6 +651,13 @@ __global__ __launch_bounds__(256) void decode_step_begin_kernel(
   for (int c = t; c * 8 < dim; c += 256) {      // 8 channels per thread; a 16-channel tile = 2 neighbouring threads
     const u32x4 q = ld16(src + c * 8);
     st16(h + (size_t)b * dim + c * 8, q);
+    if (u != nullptr) {          // the first product's activations (dgemv_body: US)
+      const u32x4 w = ld16(norm_w + c * 8);
+      u32x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = pack2(lo2f(w[e]) * lo2f(q[e]), hi2f(w[e]) * hi2f(q[e]));
+      st16(u + (size_t)b * dim + c * 8, o);
+    }
     float s = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) { const float lo = lo2f(q[e]), hi = hi2f(q[e]); s += lo * lo + hi * hi; }
@@ -603,10 +671,10 @@ __global__ __launch_bounds__(256) void decode_step_begin_kernel(
 // ------------------------------------------------------------------------------------------------------------------------
 int decode_step_begin(const int32_t* slots, const int32_t* cur_tok, const int32_t* done, uint32_t* seen, int words, const bf16_t* table,
                       bf16_t* h, float* stats, int dim, const int32_t* pos, const float* inv_freq, bf16_t* cs, bf16_t* sn, int B,
-                      hipStream_t st) {
+                      hipStream_t st, const bf16_t* norm_w, bf16_t* u) {
   if (B <= 0) return 0;
   if (dim & 15) return LCC_ERR_SHAPE;
-  decode_step_begin_kernel<<<dim3(B), dim3(256), 0, st>>>(slots, cur_tok, done, seen, words, table, h, stats, dim, pos, inv_freq, cs, sn);
+  decode_step_begin_kernel<<<dim3(B), dim3(256), 0, st>>>(slots, cur_tok, done, seen, words, table, h, stats, dim, pos, inv_freq, cs, sn, norm_w, u);
   return 0;
 }
 
@@ -711,6 +779,15 @@ int dgemv_resid(const DgArgs& a, hipStream_t st) {
   const int w16 = g_resid_waves;
   // 3 = blocks of 8 output rows (dgemv_rows8_kernel; the engine asks for them by DgArgs::rows8 where they suit).
   const bool wide = w16 == 2 || (w16 == 1 && a.K >= 8192 && a.wscale == nullptr);
+  if (a.C != nullptr) {          // u = bf16(norm_w * h) beside h: the activations of the next row-scaled product
+    if (a.norm_w == nullptr) return LCC_ERR_ARG;
+    if (a.wscale != nullptr) {
+      if (wide) dgemv_us_kernel<1, DG_EPI_RESID, 16, 3, 1, true><<<dim3(a.N / 16), dim3(1024), 0, st>>>(a);
+      else dgemv_us_kernel<1, DG_EPI_RESID, 8, 4, 1, true><<<dim3(a.N / 16), dim3(512), 0, st>>>(a);
+    } else if (wide) dgemv_us_kernel<1, DG_EPI_RESID, 16, 3, 1, false><<<dim3(a.N / 16), dim3(1024), 0, st>>>(a);
+    else dgemv_us_kernel<1, DG_EPI_RESID, 8, 4, 1, false><<<dim3(a.N / 16), dim3(512), 0, st>>>(a);
+    return 0;
+  }
   if (a.wscale != nullptr) {
     if (wide) dgemv_kernel<1, DG_PRO_PLAIN, DG_EPI_RESID, 16, 4, 4, true><<<dim3(a.N / 16), dim3(1024), 0, st>>>(a);
     else dgemv_kernel<1, DG_PRO_PLAIN, DG_EPI_RESID, 8, 4, 4, true><<<dim3(a.N / 16), dim3(512), 0, st>>>(a);
@@ -718,6 +795,40 @@ int dgemv_resid(const DgArgs& a, hipStream_t st) {
   }
   if (wide) dgemv_kernel<1, DG_PRO_PLAIN, DG_EPI_RESID, 16, 3><<<dim3(a.N / 16), dim3(1024), 0, st>>>(a);
   else dgemv_kernel<1, DG_PRO_PLAIN, DG_EPI_RESID, 8, 4><<<dim3(a.N / 16), dim3(512), 0, st>>>(a);
+  return 0;
+}
+static thread_local hipEvent_t g_swiglu_ev0 = nullptr, g_swiglu_ev1 = nullptr;
+void dgemv_attach_events_to_next_swiglu(hipEvent_t start, hipEvent_t stop) { g_swiglu_ev0 = start; g_swiglu_ev1 = stop; }
+// row-scaled products of u = bf16(norm weight * h) and h's statistics: X = u, stats / n_stat / eps as for the normalising forms
+static int dg_us_check(const DgArgs& a, int epi) {
+  if (int rc = dg_check(a, DG_PRO_PLAIN, epi)) return rc;
+  if (a.stats == nullptr || (a.n_stat != (a.K >> 4) && a.n_stat != (a.K >> 3)) || (a.n_stat & 3) || a.n_stat > 512) return LCC_ERR_ARG;
+  return 0;
+}
+template <int NTILE, int EPI, int NW, int UNR, int MINW, bool W8>
+static void us_launch(const DgArgs& a, hipStream_t st) {
+  dgemv_us_kernel<NTILE, EPI, NW, UNR, MINW, W8><<<dim3(a.N / (NTILE * 16)), dim3(NW * 64), (size_t)a.M * a.n_stat, st>>>(a);
+}
+int dgemv_us_qkv_rope(const DgArgs& a, hipStream_t st) {
+  if (int rc = dg_us_check(a, DG_EPI_ROPE)) return rc;
+  if (a.wscale != nullptr) us_launch<1, DG_EPI_ROPE, 8, 3, 4, true>(a, st);
+  else us_launch<1, DG_EPI_ROPE, 8, 2, 4, false>(a, st);
+  return 0;
+}
+int dgemv_us_swiglu(const DgArgs& a, hipStream_t st) {
+  if (int rc = dg_us_check(a, DG_EPI_SWIGLU)) return rc;
+  const hipEvent_t ev0 = g_swiglu_ev0, ev1 = g_swiglu_ev1;
+  g_swiglu_ev0 = g_swiglu_ev1 = nullptr;
+  if (ev0 != nullptr) (void)hipEventRecord(ev0, st);
+  if (a.wscale != nullptr) us_launch<2, DG_EPI_SWIGLU, 4, 2, 1, true>(a, st);
+  else us_launch<2, DG_EPI_SWIGLU, 4, 1, 5, false>(a, st);
+  if (ev1 != nullptr) (void)hipEventRecord(ev1, st);
+  return 0;
+}
+int dgemv_us_bf16(const DgArgs& a, hipStream_t st) {
+  if (int rc = dg_us_check(a, DG_EPI_BF16)) return rc;
+  if (a.wscale != nullptr) us_launch<1, DG_EPI_BF16, 4, 2, 1, true>(a, st);
+  else us_launch<1, DG_EPI_BF16, 4, 1, 1, false>(a, st);
   return 0;
 }
 // chained launch: down_proj of one layer + q/k/v of the next (see dgemv_down_qkv_kernel).  `blocks_capacity` = co-resident 512-thread
@@ -748,8 +859,6 @@ int dgemv_down_qkv(const DgArgs& down, const DgArgs& qkv, unsigned* flag, unsign
   dgemv_down_qkv_kernel<2><<<dim3(nb_down + nb_qkv), dim3(512), (size_t)qkv.M * qkv.K * 2, st>>>(down, qkv, ch, nb_down);
   return 0;
 }
-static thread_local hipEvent_t g_swiglu_ev0 = nullptr, g_swiglu_ev1 = nullptr;
-void dgemv_attach_events_to_next_swiglu(hipEvent_t start, hipEvent_t stop) { g_swiglu_ev0 = start; g_swiglu_ev1 = stop; }
 // [RMSNorm] gate/up Linear [SwiGLU]
 int dgemv_norm_swiglu(const DgArgs& a, hipStream_t st) {
   if (int rc = dg_check(a, DG_PRO_NORM, DG_EPI_SWIGLU)) return rc;

@@ -193,11 +193,11 @@ bool decode_v2_ok(const lcc_engine* e) {
   for (const LlmLayerW& L : e->llm) if (L.qkv_w_dec == nullptr || (e->c.llm_fp8 && L.qkv_s_dec == nullptr)) return false;
   return true;
 }
-// the 28 decoder layers of ONE decode step over B rows, v2 launch sequence.  On entry b.h / b.stats / b.cos / b.sin come from
+// the 28 decoder layers of ONE decode step over B rows, v2 launch sequence (us: row-scaled products, b.xn = u).  On entry b.h / b.stats / b.cos / b.sin come from
 // decode_step_begin; on exit b.h is the residual stream after the last layer and b.stats its per-tile sums of squares (the final
 // RMSNorm runs as the prologue of the lm_head GEMV).
 int run_decode_layers_v2(lcc_engine* e, const LlmBuffers& b, int B, const int32_t* d_slots, int nsplit_attn, hipStream_t st,
-                         const AttnDirect* direct, int* n_stat_out) {
+                         const AttnDirect* direct, int* n_stat_out, bool us) {
   const int H = e->c.hidden_size, I = e->c.intermediate_size;
   const float eps = e->c.rms_eps;
   if (e->llm_over) return fail(LCC_ERR_STATE, "per-layer input overrides are a prefill-only instrument (decode pipeline v2 carries row statistics)");
@@ -212,18 +212,20 @@ int run_decode_layers_v2(lcc_engine* e, const LlmBuffers& b, int B, const int32_
   auto qkv_args = [&](int l) {
     const LlmLayerW& L = e->llm[l];
     DgArgs a; a.W = L.qkv_w_dec; a.wscale = L.qkv_s_dec; a.M = B; a.N = e->qkvd; a.K = H; a.H = b.h; a.stats = b.stats; a.n_stat = n_stat; a.norm_w = L.in_norm;
+    if (us) { a.X = b.xn; a.ldx = H; }
     a.eps = eps; a.bias = L.qkv_b; a.cs = b.cos; a.sn = b.sin; a.tok_stream = d_slots; a.kv_len = e->d_kv_len; a.kv_base = e->d_kv_base;
     a.lay = e->lay; a.layer = l; a.q_out = b.q; a.n_q_heads = e->c.n_q_heads;
     return a;
   };
-  const bool chain = g_decode_chain && !e->c.llm_fp8 && B <= 2 && e->c.n_layers <= 127 && !e->llm_taps && (long)B * H * 2 <= 16 * 1024 &&
+  const bool chain = g_decode_chain && !us && !e->c.llm_fp8 && B <= 2 && e->c.n_layers <= 127 && !e->llm_taps && (long)B * H * 2 <= 16 * 1024 &&
                      H / 16 + e->qkvd / 16 <= dgemv_chain_capacity();
   for (int l = 0; l < e->c.n_layers; ++l) {
     const LlmLayerW& L = e->llm[l];
     DgArgs a;
-    if (l == 0 || !chain) LCC_TRY(dgemv_qkv_rope(qkv_args(l), st));     // otherwise launched together with the previous layer's down_proj
+    if (l == 0 || !chain) LCC_TRY(us ? dgemv_us_qkv_rope(qkv_args(l), st) : dgemv_qkv_rope(qkv_args(l), st));     // otherwise launched together with the previous layer's down_proj
     LCC_TRY(attn_decode_bf16(b.q, b.attn, d_slots, e->d_kv_len, e->d_kv_base, e->lay, l, B, e->c.n_q_heads, nsplit_attn, b.ws_o, b.ws_ml, st, direct));
     a = DgArgs(); a.W = L.o_w; a.wscale = L.o_s; a.M = B; a.N = H; a.K = e->qd; a.X = b.attn; a.ldx = e->qd; a.Hres = b.h; a.stats_out = b.stats;
+    if (us) { a.C = b.xn; a.norm_w = L.post_norm; }
     a.rows8 = dgemv_rows8_ok(B, H, e->qd, L.o_s);
     LCC_TRY(dgemv_resid(a, st));
     n_stat = a.rows8 ? H / 8 : H / 16;
@@ -233,7 +235,8 @@ int run_decode_layers_v2(lcc_engine* e, const LlmBuffers& b, int B, const int32_
     const bool prof = e->prof_on && l == e->c.n_layers / 2 && 2 * (e->prof_n + 1) <= (int)e->prof_ev.size();   // one sample per step
     // the sampled launch carries its events on the dispatch (kernel begin / end timestamps: kernels.h)
     if (prof) dgemv_attach_events_to_next_swiglu(e->prof_ev[2 * e->prof_n], e->prof_ev[2 * e->prof_n + 1]);
-    LCC_TRY(dgemv_norm_swiglu(a, st));
+    if (us) { a.X = b.xn; a.ldx = H; LCC_TRY(dgemv_us_swiglu(a, st)); }
+    else LCC_TRY(dgemv_norm_swiglu(a, st));
     if (prof) e->prof_n++;
     a = DgArgs(); a.W = L.down_w; a.wscale = L.down_s; a.M = B; a.N = H; a.K = I; a.X = b.act; a.ldx = I; a.Hres = b.h; a.stats_out = b.stats;
     if (chain && l + 1 < e->c.n_layers) {
@@ -241,6 +244,7 @@ int run_decode_layers_v2(lcc_engine* e, const LlmBuffers& b, int B, const int32_
       n_stat = H / 16;          // the chained launch writes (and its consumer half reads) one per 16
       LCC_TRY(dgemv_down_qkv(a, qkv_args(l + 1), e->d_chain + l, target, e->d_chain + 128, st));
     } else {
+      if (us) { a.C = b.xn; a.norm_w = l + 1 < e->c.n_layers ? e->llm[l + 1].in_norm : e->final_norm; }
       a.rows8 = dgemv_rows8_ok(B, H, I, L.down_s);
       LCC_TRY(dgemv_resid(a, st));
       n_stat = a.rows8 ? H / 8 : H / 16;
@@ -252,14 +256,15 @@ int run_decode_layers_v2(lcc_engine* e, const LlmBuffers& b, int B, const int32_
 }
 
 int head_and_sample(lcc_engine* e, const LlmBuffers& b, const bf16_t* xn_rows, int B, const int32_t* d_slots, const lcc_sampling* sp,
-                    int step_index, hipStream_t st, int n_stat = 0) {
+                    int step_index, hipStream_t st, int n_stat = 0, bool us = false) {
   const int H = e->c.hidden_size, V = e->c.vocab_size;
   bf16_t* logits = b.logits;
   if (sp && sp->logits_out) logits = (bf16_t*)sp->logits_out + (size_t)step_index * B * V;
   if (xn_rows == nullptr) {   // decode v2: final RMSNorm of b.h as the prologue of the lm_head GEMV
     DgArgs a; a.W = e->lm_head; a.wscale = e->lm_head_s; a.M = B; a.N = V; a.K = H; a.H = b.h; a.stats = b.stats; a.n_stat = n_stat; a.norm_w = e->final_norm;
     a.eps = e->c.rms_eps; a.C = logits; a.ldc = V;
-    LCC_TRY(dgemv_norm_bf16(a, st));
+    if (us) { a.X = b.xn; a.ldx = H; LCC_TRY(dgemv_us_bf16(a, st)); }
+    else LCC_TRY(dgemv_norm_bf16(a, st));
   } else {
     GemmArgs g; g.w_packed = 1; g.A = xn_rows; g.lda = H; g.W = e->lm_head; g.ldw = H; g.C = logits; g.ldc = V; g.M = B; g.N = V; g.K = H;
     if (e->lm_head_s != nullptr) { g.w_fp8 = 1; g.wscale = e->lm_head_s; }
@@ -489,9 +494,12 @@ extern "C" int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots
   // fused kernel: 4 waves per block; about one block per CU, never less than one key tile per wave
   static const int fused_blocks = [] { const char* v = getenv("LCC_ATTN_FUSED_BLOCKS"); return v ? std::max(64, atoi(v)) : 256; }();
   cx.nsplit_attn_fused = std::max(1, std::min(std::min(32, (ntile + 3) / 4), std::max(1, fused_blocks / (n_streams * e->c.n_kv_heads))));
-  // v2 serves batches of one or two streams (measured on MI355X at 7B shapes: 246 vs 242 tokens/s for one stream, 414 vs 410 for
-  // two, but 640 vs 655 for four: with more rows the per-block normalisation prologue outweighs the saved launches)
-  const bool v2 = decode_v2_ok(e) && n_streams <= 2 && (long)n_streams * e->c.hidden_size <= 16384;
+  // v2 normalises rows in every block for one or two streams and uses row-scaled products for 3 to 16 (one / two streams: 7B 2.81 / 2.90 ms a
+  // step against 2.81 / 2.93 row-scaled, 2B 1.17 / 1.18 against 1.19 / 1.19; three: 3.02 -> 2.85 against the sequence below, 16: 3.93 -> 3.71).
+  // More than eight rows do not fit the 8-row residual blocks, and 16-row ones leave most of the chip idle at 2,048 hidden channels and
+  // below: 2B, 12 / 16 streams 1.48 / 1.56 ms below against 1.52 / 1.66 (nine: 1.44 against 1.41).
+  const bool us = n_streams >= 3 && n_streams <= (e->c.hidden_size > 2048 ? 16 : 8) && e->llm_over == nullptr;
+  const bool v2 = decode_v2_ok(e) && (us || (n_streams <= 2 && (long)n_streams * e->c.hidden_size <= 16384));
   for (int step = 0; step < n_steps; ++step) {
     int n_stat = 0;
     const bool prof_step = e->prof_on && (step & 3) == 0 && 2 * (e->step_n + 1) <= (int)e->step_ev.size();   // every 4th step
@@ -499,7 +507,7 @@ extern "C" int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots
     // the token sampled by the previous step (d_cur_tok[slot]) is embedded, appended at kv_len[slot], position pos[slot]
     if (v2) {
       LCC_TRY(decode_step_begin(d_slots, e->d_cur_tok, e->d_done, e->d_seen, e->words, e->embed, bf.h, bf.stats, e->c.hidden_size, e->d_pos,
-                                e->inv_freq, bf.cos, bf.sin, n_streams, st));
+                                e->inv_freq, bf.cos, bf.sin, n_streams, st, us ? e->llm[0].in_norm : nullptr, us ? bf.xn : nullptr));
       // the step's key counts and arena pointers travel by value (kernels.h: AttnDirect; LCC_ATTN_DIRECT=0: index loads on the device)
       static const int direct_on = [] { const char* v = getenv("LCC_ATTN_DIRECT"); return v ? atoi(v) : 1; }();
       AttnDirect dir;
@@ -507,7 +515,7 @@ extern "C" int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots
         for (int bb = 0; bb < n_streams; ++bb) { dir.base[bb] = (const bf16_t*)e->h_kv_base[slots[bb]]; dir.n[bb] = e->h_kv_len[slots[bb]] + step + 1; }
         dir.used = n_streams;
       }
-      LCC_TRY(run_decode_layers_v2(e, bf, n_streams, d_slots, nsplit, st, dir.used ? &dir : nullptr, &n_stat));
+      LCC_TRY(run_decode_layers_v2(e, bf, n_streams, d_slots, nsplit, st, dir.used ? &dir : nullptr, &n_stat, us));
     } else {
       LCC_TRY(seen_set(e->d_seen, e->words, e->d_cur_tok, d_slots, n_streams, 1, e->d_done, st));
       LCC_TRY(embed_gather_bf16(e->d_cur_tok, d_slots, nullptr, e->embed, nullptr, bf.h, n_streams, e->c.hidden_size, st));
@@ -516,7 +524,7 @@ extern "C" int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots
       if (!cx.skinny) LCC_TRY(rmsnorm_bf16(bf.h, e->final_norm, bf.xn, n_streams, e->c.hidden_size, e->c.rms_eps, st));
     }
     LCC_TRY(advance_lengths(d_slots, e->d_kv_len, e->d_pos, n_streams, e->d_done, st));
-    LCC_TRY(head_and_sample(e, bf, v2 ? nullptr : bf.xn, n_streams, d_slots, sp, first_step_index + step, st, n_stat));
+    LCC_TRY(head_and_sample(e, bf, v2 ? nullptr : bf.xn, n_streams, d_slots, sp, first_step_index + step, st, n_stat, us));
     if (prof_step) {
       HIP_TRY(hipEventRecord(e->step_ev[2 * e->step_n + 1], st));
       if (e->step_n < (int)e->step_rel.size()) e->step_rel[e->step_n] = step;

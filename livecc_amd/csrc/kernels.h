@@ -210,7 +210,12 @@ struct DgArgs {
 };
 int decode_step_begin(const int32_t* slots, const int32_t* cur_tok, const int32_t* done, uint32_t* seen, int words, const bf16_t* table,
                       bf16_t* h, float* stats, int dim, const int32_t* pos, const float* inv_freq, bf16_t* cs, bf16_t* sn, int B,
-                      hipStream_t st);
+                      hipStream_t st, const bf16_t* norm_w = nullptr, bf16_t* u = nullptr);
+// row-scaled products (decode_v2.hip: US): X = u = bf16(norm weight * h), the row's 1 / rms from `stats` multiplies the fp32 sums; dgemv_resid writes
+// u beside h when C (and norm_w, the next norm's weight) is set
+int dgemv_us_qkv_rope(const DgArgs& a, hipStream_t st);
+int dgemv_us_swiglu(const DgArgs& a, hipStream_t st);
+int dgemv_us_bf16(const DgArgs& a, hipStream_t st);
 int dgemv_qkv_rope(const DgArgs& a, hipStream_t st);      // [RMSNorm] q|k|v Linear (row-permuted decode copy) [bias + M-RoPE + KV append]
 int set_resid_waves(int mode);   // 0: 8-wave blocks, 1: 16 waves for bf16 weights with K >= 8192 (default), 2: 16 waves always; returns the old mode
 bool dgemv_rows8_ok(int M, int N, int K, const float* wscale);      // blocks of 8 output rows serve (and suit) the product

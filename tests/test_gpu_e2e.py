@@ -681,6 +681,54 @@ def test_decode_pipeline_v2_matches_the_round1_launch_sequence(dev, shape):
         assert worst <= 3e-2, f"v2 vs round-1 decode logits differ by {worst:.3g} of the logit scale"
 
 
+@pytest.mark.parametrize("hidden,n_streams,fp8", [(256, 3, False), (896, 8, False), (896, 8, True), (896, 9, False), (2304, 9, False), (2304, 16, False),
+                                                  (2304, 16, True), (2304, 17, False)])
+def test_decode_of_several_streams_matches_the_unfused_sequence(dev, hidden, n_streams, fp8):
+    """3 to 8 streams (16 above 2,048 channels) take the row-scaled products: RMSNorm's weight on the residual row where it is written, 1 / rms on the
+    finished sums; more streams keep the launch sequence with norm kernels.  Each against that sequence on the same weights, prompts of
+    different lengths and the same forced tokens: logits within 3 % of their scale (the bound of the one-stream comparison above: two bf16
+    pipelines that round at different points), and the launch counts say which of them ran."""
+    import dataclasses
+    from livecc_amd import _lib, ops
+    from livecc_amd.config import tiny
+    from livecc_amd.engine import Sampling
+    from livecc_amd.modeling import LiveCCForConditionalGeneration
+    heads = hidden // 128
+    cfg = dataclasses.replace(tiny(), hidden_size=hidden, intermediate_size=2 * hidden + 64, num_attention_heads=heads, num_key_value_heads=2 if heads % 2 == 0 else 1)
+    lens = [5 + 37 * i % 150 for i in range(n_streams)]
+    native = LiveCCForConditionalGeneration.from_config(cfg, dev, seed=5, llm_fp8=fp8, max_streams=n_streams, max_kv_len=256, max_new_rows=sum(lens),
+                                                        max_patches=64, max_history=16)
+    lib, eng, sp = _lib.load(), native.engine, Sampling(suppress_eos=True)
+    rng = np.random.RandomState(7)
+    ids = [rng.randint(0, 1000, size=n) for n in lens]
+    forced = rng.randint(0, 1000, size=(3, n_streams))
+
+    def run(path):
+        _lib.check(lib.lcc_debug_set_decode_path(path), "set_decode_path")
+        try:
+            slots = list(range(n_streams))
+            for i in slots:
+                eng.reset_slot(i)
+            eng.prefill(slots, ids, [np.tile(np.arange(n), (3, 1)) for n in lens], None, sp)
+            out = torch.zeros(4, n_streams, cfg.vocab_size, dtype=torch.bfloat16, device=dev)      # row block = step index (the prefill's is 0)
+            ops.launch_counts(reset=True)
+            for k in range(3):
+                eng.set_tokens(slots, forced[k])
+                eng.decode(slots, 1, 1 + k, sp, None, out)
+            return out[1:].float().cpu(), ops.launch_counts(reset=True)["dgemv_v2"]
+        finally:
+            _lib.check(lib.lcc_debug_set_decode_path(1), "set_decode_path")
+
+    (got, n1), (ref, n0) = run(1), run(0)
+    scaled = n_streams <= (16 if hidden > 2048 else 8)
+    assert n0 == 0 and n1 == (3 * (4 * cfg.num_hidden_layers + 1) if scaled else 0)
+    for k in range(3):
+        for b in range(n_streams):
+            scale = ref[k, b].abs().max().item()
+            err = (got[k, b] - ref[k, b]).abs().max().item()
+            assert 0 < scale and err <= 3e-2 * scale, f"step {k} stream {b}: {err:.3g} of {scale:.3g}"
+
+
 def test_vision_tower_prefetch_on_a_side_stream_is_bit_identical(dev, tiny_models):
     """generate_batch(prefetch=next clips): the next turn's ViT runs on a low-priority side stream under this turn's decode steps
     (own workspace + meta ring in the engine).  Same kernels, same inputs -> bit-identical logits and tokens, for one stream and a
