@@ -193,6 +193,13 @@ def test_latent_decode_attention(dev, lib, rank, heads, vdim, lens, ns):
         assert (out[b].view(heads, vdim).double().cpu() - want).abs().max() < 0.012 * want.abs().max() + 1e-3, (b, lens[s])
 
 
+@pytest.mark.parametrize("rank,heads,vdim,lens,ns", [(512, 12, 128, [200] * 31, 4), (64, 40, 64, [70] * 33, 9), (1024, 3, 192, [65, 1] * 40, 2), (512, 1, 64, [300], 128)])
+def test_latent_merge_of_row_groups_and_channel_groups(dev, lib, rank, heads, vdim, lens, ns):
+    """Blocks of several rows (the last group short) and of fewer value channels than a head has, more splits than a thread fetches ahead, unused
+    splits' memory NaN: the bounds of the test above."""
+    test_latent_decode_attention(dev, lib, rank, heads, vdim, lens, ns)
+
+
 @pytest.mark.parametrize("rows,heads,dim,rank,ns", [(1, 1, 64, 64, 1), (16, 3, 128, 192, 2), (33, 2, 192, 512, 5)])
 def test_absorbed_queries(dev, lib, rows, heads, dim, rank, ns):
     from livecc_amd.weights import pack_weight
