@@ -568,6 +568,8 @@ int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots, int n_ste
 /* blocking: copy the ids generated by the last generate call of a slot to the host (at most max_n), report how many
  * were generated (EOS included) and refresh the host mirror of the slot's KV length / next position. */
 int lcc_slot_read_tokens(lcc_engine* e, int slot, int32_t* out, int max_n, int* n_generated, void* stream);
+/* the same for n_slots slots in one round trip: out [n_slots][max_n], n_generated [n_slots] (or NULL). */
+int lcc_slots_read_tokens(lcc_engine* e, int n_slots, const int32_t* slots, int32_t* out, int max_n, int32_t* n_generated, void* stream);
 
 #ifdef __cplusplus
 }

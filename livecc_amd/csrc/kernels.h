@@ -187,6 +187,9 @@ struct DeviceOnce {
   }
 };
 // cur_tok / prev_tok (both or none): the token just consumed becomes the slot's previous token
+int read_slots(const int32_t* slots, int n, const int32_t* kv_len, const int32_t* pos, const int32_t* hist_col, const int32_t* history, int max_history, int take,
+               const unsigned* err, int32_t* out, hipStream_t st);
+int reset_slot(int slot, int32_t* kv_len, int32_t* pos, int32_t* hist_col, int32_t* done, uint32_t* rng_ctr, uint32_t* seen, int words, hipStream_t st);
 int advance_lengths(const int32_t* slots, int32_t* kv_len, int32_t* pos, int B, const int32_t* done, hipStream_t st, const int32_t* cur_tok = nullptr, int32_t* prev_tok = nullptr);
 // teacher forcing (tests): the token just sampled for stream b becomes forced[b] (current token + last history column); the forced stream
 // also decides where a slot ends (`done`: flags from before this step, updated by a forced EOS)

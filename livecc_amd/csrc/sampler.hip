@@ -581,6 +581,32 @@ int force_tokens(const int32_t* slots, const int32_t* forced, int B, int32_t* cu
   force_tokens_kernel<<<dim3((B + 63) / 64), dim3(64), 0, st>>>(slots, forced, B, cur_tok, history, hist_ld, hist_col, done, eos, eos2);
   return 0;
 }
+// one block per slot: its counters (cached keys, next position, tokens generated) and the first `take` of its tokens, 3 + take words a slot; the
+// hand-off error word behind them
+__global__ __launch_bounds__(64) void read_slots_kernel(const int32_t* __restrict__ slots, const int32_t* __restrict__ kv_len, const int32_t* __restrict__ pos,
+                                                        const int32_t* __restrict__ hist_col, const int32_t* __restrict__ history, int max_history, int take,
+                                                        const unsigned* __restrict__ err, int32_t* __restrict__ out) {
+  const int s = slots[blockIdx.x], t = threadIdx.x, n = hist_col[s];
+  int32_t* o = out + (size_t)blockIdx.x * (3 + take);
+  if (t == 0) { o[0] = kv_len[s]; o[1] = pos[s]; o[2] = n; }
+  for (int i = t; i < min(n, take); i += 64) o[3 + i] = history[(size_t)s * max_history + i];
+  if (blockIdx.x == 0 && t == 0) out[(size_t)gridDim.x * (3 + take)] = (int32_t)*err;
+}
+int read_slots(const int32_t* slots, int n, const int32_t* kv_len, const int32_t* pos, const int32_t* hist_col, const int32_t* history, int max_history, int take,
+               const unsigned* err, int32_t* out, hipStream_t st) {
+  read_slots_kernel<<<dim3(n), dim3(64), 0, st>>>(slots, kv_len, pos, hist_col, history, max_history, take, err, out);
+  return 0;
+}
+// one launch for the counters and the seen-id bitmap of a fresh slot
+__global__ __launch_bounds__(256) void reset_slot_kernel(int slot, int32_t* kv_len, int32_t* pos, int32_t* hist_col, int32_t* done, uint32_t* rng_ctr, uint32_t* seen, int words) {
+  const int t = threadIdx.x;
+  if (t == 0) { kv_len[slot] = 0; pos[slot] = 0; hist_col[slot] = 0; done[slot] = 0; rng_ctr[slot] = 0; }
+  for (int i = t; i < words; i += 256) seen[(size_t)slot * words + i] = 0u;
+}
+int reset_slot(int slot, int32_t* kv_len, int32_t* pos, int32_t* hist_col, int32_t* done, uint32_t* rng_ctr, uint32_t* seen, int words, hipStream_t st) {
+  reset_slot_kernel<<<dim3(1), dim3(256), 0, st>>>(slot, kv_len, pos, hist_col, done, rng_ctr, seen, words);
+  return 0;
+}
 int advance_lengths(const int32_t* slots, int32_t* kv_len, int32_t* pos, int B, const int32_t* done, hipStream_t st, const int32_t* cur_tok, int32_t* prev_tok) {
   if (B <= 0) return 0;
   advance_kernel<<<dim3((B + 63) / 64), dim3(64), 0, st>>>(slots, kv_len, pos, B, done, cur_tok, prev_tok);

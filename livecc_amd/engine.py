@@ -391,16 +391,25 @@ class Engine:
         _lib.check(self.lib.lcc_engine_profile_read_step_index(self.h, buf.ctypes.data, max_n, C.byref(n)), "lcc_engine_profile_read_step_index")
         return buf[:n.value]
 
+    def _read_slots(self, slots: Sequence[int], max_n: int):
+        a = np.asarray(slots, dtype=np.int32)
+        buf, n = np.zeros((len(a), max(max_n, 1)), dtype=np.int32), np.zeros(len(a), dtype=np.int32)
+        if len(a):
+            _lib.check(self.lib.lcc_slots_read_tokens(self.h, len(a), a.ctypes.data, buf.ctypes.data, buf.shape[1] if max_n else 0, n.ctypes.data,
+                                                      self._stream()), "lcc_slots_read_tokens")
+        return buf, n
+
+    def generated_counts(self, slots: Sequence[int]) -> List[int]:
+        """Blocking: number of tokens each slot has generated in the current generate call (stops growing after EOS)."""
+        return self._read_slots(slots, 0)[1].tolist()
+
     def generated_count(self, slot: int) -> int:
-        """Blocking: number of tokens the slot has generated in the current generate call (stops growing after EOS)."""
-        buf = np.zeros(1, dtype=np.int32)
-        n = C.c_int()
-        _lib.check(self.lib.lcc_slot_read_tokens(self.h, slot, buf.ctypes.data, 0, C.byref(n), self._stream()), "lcc_slot_read_tokens")
-        return n.value
+        return self.generated_counts([slot])[0]
+
+    def read_tokens_of(self, slots: Sequence[int], max_n: int) -> List[List[int]]:
+        """Blocking: the tokens (at most max_n) that each slot generated, in one round trip."""
+        buf, n = self._read_slots(slots, max_n)
+        return [buf[i, :min(int(k), max_n)].tolist() for i, k in enumerate(n)]
 
     def read_tokens(self, slot: int, max_n: int) -> List[int]:
-        buf = np.zeros(max(max_n, 1), dtype=np.int32)
-        n = C.c_int()
-        _lib.check(self.lib.lcc_slot_read_tokens(self.h, slot, buf.ctypes.data, max_n, C.byref(n), self._stream()),
-                   "lcc_slot_read_tokens")
-        return buf[:min(n.value, max_n)].tolist()
+        return self.read_tokens_of([slot], max_n)[0]

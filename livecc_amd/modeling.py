@@ -308,14 +308,16 @@ class EngineModel:
                 eng.decode(grp, k, step, sp, scores_out=scores_buf[b0:b0 + G] if scores_buf is not None else None,
                            logits_out=logits_buf if (logits_buf is not None and n <= G) else None)
                 step += k
-                if step < max_new_tokens and all(eng.generated_count(s) < step for s in grp):
+                if step < max_new_tokens and all(c < step for c in eng.generated_counts(grp)):
                     break
         outs = []
-        for b, st in enumerate(states):
-            toks = eng.read_tokens(st.slot, max_new_tokens)
+        read = eng.read_tokens_of(slots, max_new_tokens)
+        ids = [np.concatenate([full_ids[b], np.asarray(t, dtype=np.int64)]) for b, t in enumerate(read)]
+        seqs = torch.from_numpy(np.concatenate(ids)).to(self.device).split([len(i) for i in ids]) if n else []      # one upload for all streams
+        for b, (st, toks) in enumerate(zip(states, read)):
             if thr and logits_processor:
                 logits_processor[0].count += len(toks)        # keep the stateful processor's counter as HF would
-            seq = torch.from_numpy(np.concatenate([full_ids[b], np.asarray(toks, dtype=np.int64)])).view(1, -1).to(self.device)
+            seq = (seqs[b] if n == 1 else seqs[b].clone()).view(1, -1)
             lg = logits_buf[:len(toks), b] if logits_buf is not None and n <= G else None
             outs.append(GenerateOutput(sequences=seq, past_key_values=st, logits=lg,
                                        scores=scores_buf[b, :self.cfg.vocab_size] if scores_buf is not None else None))

@@ -729,6 +729,36 @@ def test_decode_of_several_streams_matches_the_unfused_sequence(dev, hidden, n_s
             assert 0 < scale and err <= 3e-2 * scale, f"step {k} stream {b}: {err:.3g} of {scale:.3g}"
 
 
+@pytest.mark.parametrize("n_streams,max_history,max_new", [(1, 16, 16), (5, 16, 9), (3, 4096, 40)])
+def test_reading_several_slots_equals_reading_each(dev, n_streams, max_history, max_new):
+    """lcc_slots_read_tokens: the counts and tokens of slots in any order, cut at the caller's width, equal one call a slot; 4,096 columns do not fit
+    the metadata ring together.  A slot that is reset afterwards reads empty and starts a stream like a new one."""
+    from livecc_amd.config import tiny
+    from livecc_amd.engine import Sampling
+    from livecc_amd.modeling import LiveCCForConditionalGeneration
+    native = LiveCCForConditionalGeneration.from_config(tiny(), dev, seed=5, max_streams=6, max_kv_len=256 + max_history, max_new_rows=64, max_patches=64, max_history=max_history)
+    eng, sp = native.engine, Sampling(suppress_eos=True)
+    slots = [5, 0, 3, 1, 4][:n_streams]
+
+    def generate(group):
+        for s in group:
+            eng.reset_slot(s)
+        eng.prefill(group, [np.arange(3 + s) for s in group], [np.tile(np.arange(3 + s), (3, 1)) for s in group], None, sp)
+        eng.decode(group, max_new - 1, 1, sp)
+
+    generate(slots)
+    for width in (0, 1, max_new - 1, max_new, max_history, max_history + 5):
+        got = eng.read_tokens_of(slots, width)
+        assert got == [eng.read_tokens(s, width) for s in slots] and all(len(t) == min(width, max_new) for t in got)
+    assert eng.generated_counts(slots) == [max_new] * n_streams == [eng.generated_count(s) for s in slots]
+    assert [eng.slot_length(s)[0] for s in slots] == [3 + s + max_new - 1 for s in slots]
+    before = eng.read_tokens_of(slots, max_new)
+    eng.reset_slot(slots[0])
+    assert eng.read_tokens(slots[0], max_new) == [] and eng.slot_length(slots[0]) == (0, 0)
+    generate(slots)
+    assert eng.read_tokens_of(slots, max_new) == before
+
+
 def test_vision_tower_prefetch_on_a_side_stream_is_bit_identical(dev, tiny_models):
     """generate_batch(prefetch=next clips): the next turn's ViT runs on a low-priority side stream under this turn's decode steps
     (own workspace + meta ring in the engine).  Same kernels, same inputs -> bit-identical logits and tokens, for one stream and a
