@@ -10,7 +10,7 @@
 //  * gemm_mid_kernel     : shapes with few 256-column tiles.  64x128x64 (128x128x64) tile, 8 waves, 6- (4-) stage LDS-DMA ring.
 //  * gemm_glds_kernel /   : row-major W, K % 64 != 0.  64x128x64 (128x128x64) tile, 4 waves,
 //    gemm_tiled_kernel     LDS-DMA 3-stage ring / register-staged double buffer with an XOR swizzle, XCD-aware block remap.
-//  * gemv_skinny_kernel  : M <= 64 (decode, lm_head; MG = ceil(M / 16) activation fragments per weight fragment).  HBM-bound weight streaming.  4 waves per block share 16 (or 32) W rows,
+//  * gemv_skinny_kernel  : M <= 64 (decode, lm_head; MG = ceil(M / 16) activation fragments per weight fragment).  HBM-bound weight streaming.  4 waves per block share 16 (32, 64) W rows,
 //                          each wave a slice of K; W fragments go straight from HBM into the MFMA operand registers (no LDS
 //                          round trip - the operand is used once), split-K partial sums as fp32 slabs that the consumer reduces.
 //  * gemv_w8_kernel      : the same for fp8-e4m3 weights + fp32 row scales (PACKED8 order), e4m3 -> bf16 exactly in registers.
@@ -1774,11 +1774,10 @@ void set_gemv_variant(int v) { g_gemv_variant = v; }
 
 template <int NTILE, int MODE, bool PACKED, int MG>
 static void launch_gemv_mg(dim3 grid, const GemmArgs& a, void* out, int ldo, int cps, hipStream_t st) {
-  if (MG > 1) {     // 17..64 rows: the two-stage pipeline with one chunk per stage (register budget: NTILE x MG accumulators + MG x fragments)
+  if constexpr (MG > 1) {     // 17..64 rows: the two-stage pipeline with one chunk per stage (register budget: NTILE x MG accumulators + MG x fragments)
     gemv_skinny_kernel<NTILE, MODE, PACKED, 1, 1, MG><<<grid, dim3(256), 0, st>>>(a.A, a.lda, a.W, a.ldw, a.bias, out, ldo, a.M, a.N, a.K, cps, a.tail);
     return;
-  }
-  switch (g_gemv_variant) {
+  } else switch (g_gemv_variant) {
     case 1:
       gemv_skinny_kernel<NTILE, MODE, PACKED, 1, 1><<<grid, dim3(256), 0, st>>>(a.A, a.lda, a.W, a.ldw, a.bias, out, ldo, a.M, a.N, a.K, cps, a.tail);
       break;
@@ -1801,6 +1800,34 @@ template <int NTILE, int MODE>
 static void launch_gemv_l(dim3 grid, const GemmArgs& a, void* out, int ldo, int cps, hipStream_t st) {
   if (a.w_packed) launch_gemv<NTILE, MODE, true>(grid, a, out, ldo, cps, st);
   else launch_gemv<NTILE, MODE, false>(grid, a, out, ldo, cps, st);
+}
+
+// 17..64 rows: a block of one 16-row weight tile reads more activations than weights (32 rows: twice as many bytes, and a compute unit pulls about 40
+// GB/s of either), so packed weights go two or four tiles to a block.  What a unit then pulls: rounds of blocks x (tiles + 16-row groups of
+// activations); four tiles only where that is clearly less, since their registers leave two waves a SIMD.  32 rows, [151936, 1536]: 116.5 us with one tile,
+// 80.8 with four (5.8 TB/s); [152064, 3584] 261 -> 182; [1536, 10496] in eight splits 10.7 -> 9.6; 64 rows: 358 -> 239 and 15.1 -> 11.7.  288
+// blocks of four (N = 4608, four splits, 17 rows: 11.2 us against 10.0 with one tile a block) is what the rounds keep away.
+static int gemv_rows_tiles(const GemmArgs& a, int S) {
+  if (!a.w_packed || a.M <= 16) return 1;
+  auto cost = [&](int nt) { return (float)(((long)(a.N / (nt * 16)) * S + 255) / 256) * ((float)nt + (float)a.M / 16.f); };
+  if (a.N % 32 != 0) return 1;
+  const int nt = cost(2) < cost(1) ? 2 : 1;
+  return a.N % 64 == 0 && cost(4) < 0.85f * cost(nt) ? 4 : nt;
+}
+template <int NTILE, int MODE>
+static void launch_gemv_tiles(const GemmArgs& a, int S, void* out, int ldo, int cps, hipStream_t st) {
+  const dim3 grid(a.N / (NTILE * 16), S);
+  if (a.M <= 32) launch_gemv_mg<NTILE, MODE, true, 2>(grid, a, out, ldo, cps, st);
+  else if (a.M <= 48) launch_gemv_mg<NTILE, MODE, true, 3>(grid, a, out, ldo, cps, st);
+  else launch_gemv_mg<NTILE, MODE, true, 4>(grid, a, out, ldo, cps, st);
+}
+template <int MODE>
+static void launch_gemv_rows(const GemmArgs& a, int S, void* out, int ldo, int cps, hipStream_t st) {
+  switch (gemv_rows_tiles(a, S)) {
+    case 4: launch_gemv_tiles<4, MODE>(a, S, out, ldo, cps, st); break;
+    case 2: launch_gemv_tiles<2, MODE>(a, S, out, ldo, cps, st); break;
+    default: launch_gemv_l<1, MODE>(dim3((a.N + 15) / 16, S), a, out, ldo, cps, st);
+  }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -2088,9 +2115,9 @@ int gemm_bf16(const GemmArgs& a, hipStream_t st) {
             a.A, a.lda, a.W, a.ldw, nullptr, a.partial, a.N, a.M, a.N, a.K, (nchunk + S - 1) / S, a.tail);
         return 0;
       }
-      launch_gemv_l<1, 0>(dim3((a.N + 15) / 16, S), a, a.partial, a.N, (nchunk + S - 1) / S, st);
+      launch_gemv_rows<0>(a, S, a.partial, a.N, (nchunk + S - 1) / S, st);
     } else {
-      launch_gemv_l<1, 1>(dim3((a.N + 15) / 16, 1), a, a.C, a.ldc, nchunk, st);
+      launch_gemv_rows<1>(a, 1, a.C, a.ldc, nchunk, st);
     }
     return 0;
   }

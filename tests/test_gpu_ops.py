@@ -456,6 +456,18 @@ def test_gemv_17_to_64_rows_streams_the_weights_once(dev, M, N, K, packed):
     assert part.shape == (S, M, N) and err <= 2e-5 * float(r32.abs().max()) * math.sqrt(K / 256) + 1e-5, f"split-K slabs: {err}"
 
 
+@pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("N,K,S", [(16384, 256, 1), (16416, 192, 1), (16400, 128, 1), (1536, 2624, 8), (4608, 448, 4), (32, 64, 1), (64, 4160, 3)])
+def test_gemv_17_to_64_rows_in_blocks_of_several_tiles(dev, M, N, K, S):
+    """Packed weights take one, two or four 16-row weight tiles to a block (N not a multiple of 64 or of 32 among the shapes), row-major ones
+    always one: each tile adds its products in the same order, so both outputs and every slab are equal bit for bit."""
+    from livecc_amd import ops
+    x, w, b = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.03, 2), _rand((N,), dev, 0.1, 3)
+    wp = ops.pack_weight(w)
+    assert torch.equal(ops.linear(x, wp, b, packed_shape=(N, K)), ops.linear(x, w, b))
+    assert torch.equal(ops.linear_partial(x, wp, S, packed_shape=(N, K)), ops.linear_partial(x, w, S))
+
+
 @pytest.mark.parametrize("M", [17, 40, 64])
 @pytest.mark.parametrize("I,K", [(512, 256), (18944, 3584)])
 def test_gemv_17_to_64_rows_swiglu(dev, M, I, K):
