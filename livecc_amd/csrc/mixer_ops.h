@@ -22,9 +22,10 @@ LCC_DEVICE f32x4 slab_sum4(const float* part, int nsplit, size_t slab, size_t of
   return v;
 }
 
-// Queries (normed, scaled by the position's temperature) to a.q, keys (normed) and values to the slot's cache.  All threads of a block of NW waves.
+// Queries (normed, scaled by the position's temperature) to a.q, keys (normed) and values to the slot's cache.  All threads of `parts` blocks of NW
+// waves; a wave's heads follow one another, each a trip to memory (36 heads of one block of four waves: nine).
 template <int NW>
-LCC_DEVICE void gqa_row(const GqaInArgs& a, int row) {
+LCC_DEVICE void gqa_row(const GqaInArgs& a, int row, int part = 0, int parts = 1) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const size_t slab = (size_t)a.rows * a.ldn, at = (size_t)row * a.ldn;
   int pos;
@@ -32,7 +33,7 @@ LCC_DEVICE void gqa_row(const GqaInArgs& a, int row) {
   if (a.direct.used) { pos = a.direct.n[row & 3] - 1; arena = const_cast<bf16_t*>(a.direct.base[row & 3]); }
   else { const int slot = a.tok_stream[row]; pos = a.tok_pos ? a.tok_pos[row] : a.kv_len[slot]; arena = a.kv_base[slot]; }
   const float temp = 1.f + a.temp_coef * logf((float)((pos + 1) / a.temp_every) + 1.f);
-  for (int h = wave; h < a.heads + a.kv_heads; h += NW) {
+  for (int h = part * NW + wave; h < a.heads + a.kv_heads; h += parts * NW) {
     const bool isq = h < a.heads;
     const int c = lane * 4;                            // dim_pad <= 256
     f32x4 v = {0.f, 0.f, 0.f, 0.f}, w = v;
@@ -48,7 +49,7 @@ LCC_DEVICE void gqa_row(const GqaInArgs& a, int row) {
     }
   }
   const int vcol = (a.heads + a.kv_heads) * a.dim_pad, nv = a.kv_heads * a.vdim_pad;
-  for (int c = tid * 4; c < nv; c += NW * 256) {
+  for (int c = (part * NW * 64 + tid) * 4; c < nv; c += parts * NW * 256) {
     const f32x4 v = slab_sum4(a.part, a.nsplit, slab, at + vcol + c);
     const int g = c / a.vdim_pad, d = c - g * a.vdim_pad;
     bf16_t* dst = arena + a.v_off + (size_t)g * a.lmax * a.vdim_pad + ((size_t)(pos >> 5) * a.vdim_pad + d) * 32 + (pos & 31);
@@ -73,13 +74,15 @@ LCC_DEVICE f32x4 rec_in4(const RecInArgs& a, int row, int r0, int pos, const flo
   }
   return silu4(acc);
 }
-LCC_DEVICE float rec_dt(const RecInArgs& a, int row, int h) {
-  if (a.dt_col < 0) return 1.f;
+// the step size's projection (with its bias) and the step size
+LCC_DEVICE float rec_dt_in(const RecInArgs& a, int row, int h) {
+  if (a.dt_col < 0) return 0.f;
   const float* p = a.part + (size_t)row * a.ldn + a.dt_col + h;
   float z = p[0];
   for (int s = 1; s < a.nsplit; ++s) z += p[(size_t)s * a.rows * a.ldn];
-  return softplus_f(z + a.dt_bias[h]);
+  return z + a.dt_bias[h];
 }
+LCC_DEVICE float rec_dt(const RecInArgs& a, int row, int h) { return a.dt_col < 0 ? 1.f : softplus_f(rec_dt_in(a, row, h)); }
 // one (row, norm group) of the gated norm behind the recurrence, by a block of NW waves; red: NW floats of LDS.  Up to MAXP pieces of 4 channels per
 // thread stay in registers between the statistic and the result.
 template <int NW, int MAXP>

@@ -110,6 +110,9 @@ int mixer_prep(const GqaInArgs* left, const RecInArgs* rec, hipStream_t st) {
 // ------------------------------------------------------------------------------------------------------------------------------
 // Decode: block = (row, head, 64 value channels); thread t owns value channels 4 (t & 15) .. of the state rows t / 16, t / 16 + 16, ..
 // The blocks behind them run the attention beside it (rec_gqa_decode_kernel), or only its rows: queries, keys, values (rec_decode_kernel).
+// HBM-bound over the state when there are many; eight rows of 28 heads (29 MB both ways, ~6 us) waited for the attention's rows, 36 heads one after
+// the other in four waves: 14.2 us, with a wave per head 10.2.  (The convolution's older rows fetched together instead of one by one: eight rows the same, 32 rows 4 us
+// more for the registers.)
 // ------------------------------------------------------------------------------------------------------------------------------
 template <int NT>
 LCC_DEVICE void rec_decode_block(const RecInArgs& a, float* __restrict__ y) {
@@ -120,17 +123,19 @@ LCC_DEVICE void rec_decode_block(const RecInArgs& a, float* __restrict__ y) {
   const int vt = a.ep / 64, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int row = blockIdx.x / (a.heads * vt), rem = blockIdx.x - row * (a.heads * vt), h = rem / vt, v0 = (rem - h * vt) * 64;
   const int slot = a.tok_stream[row], grp = h / (a.heads / a.groups);
+  // the head's scalars with the slot's index, ahead of the state: loads return in the order of their issue
+  const float zdt = rec_dt_in(a, row, h), rate = a.rate[h];
   int pos;
   bf16_t* arena;
   if (a.direct.used) { pos = a.direct.n[row & 3] - 1; arena = const_cast<bf16_t*>(a.direct.base[row & 3]); }
   else { pos = a.kv_len[slot]; arena = a.kv_base[slot]; }
+  const bool frozen = a.done != nullptr && a.done[slot];
   float* S = reinterpret_cast<float*>(arena + a.state_off) + (size_t)h * NP * a.ep + v0 + (tid & 15) * 4;
   const int n0 = tid >> 4;
   f32x4 st[NR];
 #pragma unroll
   for (int i = 0; i < NR; ++i) st[i] = *reinterpret_cast<const f32x4*>(S + (size_t)(n0 + 16 * i) * a.ep);
   float* ring = a.taps ? reinterpret_cast<float*>(arena + a.conv_off) : nullptr;
-  const bool frozen = a.done != nullptr && a.done[slot];
   for (int p = tid * 4; p < 2 * NP + 64; p += 1024) {
     const int col = p < NP ? a.q_col + grp * NP + p : p < 2 * NP ? a.k_col + grp * NP + p - NP : a.v_col + h * a.ep + v0 + p - 2 * NP;
     f32x4 raw;
@@ -141,7 +146,7 @@ LCC_DEVICE void rec_decode_block(const RecInArgs& a, float* __restrict__ y) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) dst[e] = v[e];
   }
-  const float dt = rec_dt(a, row, h), decay = pos > 0 ? exp2f(a.rate[h] * dt) : 0.f;
+  const float dt = a.dt_col < 0 ? 1.f : softplus_f(zdt), decay = pos > 0 ? exp2f(rate * dt) : 0.f;
   __syncthreads();
   const f32x4 v = *reinterpret_cast<const f32x4*>(s_v + (tid & 15) * 4), dv = v * dt;
   f32x4 o = {0.f, 0.f, 0.f, 0.f};
@@ -165,10 +170,14 @@ LCC_DEVICE void rec_decode_block(const RecInArgs& a, float* __restrict__ y) {
     *reinterpret_cast<f32x4*>(y + ((size_t)row * a.heads + h) * a.ep + v0 + tid * 4) = r;
   }
 }
+// 80 registers with NT = 2, six waves a SIMD: many rows hide a block's chain of trips (slot, state, inputs) behind other blocks' states -- 32 rows of 24
+// heads 28-29 us at six, 31.2 at five
 template <int NT>
 __global__ __launch_bounds__(256) void rec_decode_kernel(RecInArgs a, GqaInArgs l, float* __restrict__ y, int n_rec) {
-  if ((int)blockIdx.x >= n_rec) gqa_row<4>(l, (int)blockIdx.x - n_rec);
-  else rec_decode_block<NT>(a, y);
+  if ((int)blockIdx.x >= n_rec) {
+    const int parts = ((int)gridDim.x - n_rec) / l.rows, b = (int)blockIdx.x - n_rec;
+    gqa_row<4>(l, b / parts, b % parts, parts);
+  } else rec_decode_block<NT>(a, y);
 }
 // the attention beside it in the same launch: behind the n_rec blocks, four (split, KV head, head tile, row) items per block, splits fastest
 template <int NT, int DK, int DV>
@@ -209,7 +218,7 @@ int rec_decode(const RecInArgs& rec, const GqaInArgs* left, float* y, hipStream_
   if (!rec_in_ok(rec) || (left && (!gqa_in_ok(*left) || left->rows != rec.rows))) return LCC_ERR_SHAPE;
   if (!rec.kv_len || !y) return LCC_ERR_ARG;
   const int n = rec.rows * rec.heads * (rec.ep / 64);
-  const dim3 grid(n + (left ? rec.rows : 0));
+  const dim3 grid(n + (left ? rec.rows * ((left->heads + left->kv_heads + 3) / 4) : 0));      // a head per wave of the attention's rows
   const GqaInArgs l = left ? *left : GqaInArgs();
   switch (rec.np / 64) {
     case 1: rec_decode_kernel<1><<<grid, dim3(256), 0, st>>>(rec, l, y, n); break;

@@ -377,6 +377,36 @@ def test_state_step_of_linear_attention(dev, lib, n, e, heads, rows):
         assert (end[:, :n, :e] - S1).abs().max() < 1e-5 * S1.abs().max() + 1e-6
 
 
+@pytest.mark.parametrize("heads,kv_heads,rows,dp,ep", [(1, 1, 3, 64, 64), (3, 2, 2, 128, 64), (28, 4, 5, 128, 128), (5, 5, 1, 192, 256)])
+def test_attention_rows_beside_the_state_step(dev, lib, heads, kv_heads, rows, dp, ep):
+    """The decode step gives every wave one head of the attention's rows, the row kernel of the prefill all of them to four waves: bit-identical
+    queries and caches, whatever the number of heads leaves for the last block."""
+    from livecc_amd import _lib
+    ns, L, k_off = 2, 64, 128
+    v_off = k_off + kv_heads * L * dp
+    ldn = (heads + kv_heads) * dp + kv_heads * ep + 3 * 64
+    part = torch.randn(ns, rows, ldn).to(dev)
+    wq, wk = torch.randn(dp).bfloat16().to(dev), torch.randn(dp).bfloat16().to(dev)
+    order, kv = list(range(rows))[::-1], _i32([3 + 17 * i % 40 for i in range(rows)], dev)
+    sd, rate = _i32(order, dev), torch.zeros(1, device=dev)
+    out = []
+    for step in (False, True):
+        arenas, base = _arenas(rows, v_off + kv_heads * L * ep + 2 * 64 * 64, dev, 0.5)
+        q = torch.zeros(rows, heads * dp, dtype=torch.bfloat16, device=dev)
+        left = _lib.GqaInput(partial=_p(part), nsplit=ns, rows=rows, ldn=ldn, heads=heads, kv_heads=kv_heads, dim=dp, dim_pad=dp, vdim_pad=ep, eps=1e-5, q_norm=_p(wq),
+                             k_norm=_p(wk), temp_coef=0.5, temp_every=16, q=_p(q), tok_stream=_p(sd), kv_len=_p(kv), kv_base=_p(base), k_off=k_off, v_off=v_off, lmax=L)
+        if step:
+            c0 = ldn - 192
+            rec = _rec_input(part, rows, ldn, dict(q_col=c0, k_col=c0 + 64, v_col=c0 + 128, dt_col=-1, heads=1, groups=1, key_pad=64, vdim_pad=64, taps=0, conv_col=0,
+                                                   conv_ch=0, state_off=v_off + kv_heads * L * ep, conv_off=0), dict(rate=rate, tok_stream=sd, kv_len=kv, kv_base=base))
+            y = torch.empty(rows, 64, device=dev)
+            _ok(lib.lcc_rec_decode(C.byref(rec), C.byref(left), _p(y), _st()))
+        else:
+            _ok(lib.lcc_mixer_prep(C.byref(left), None, _st()))
+        out.append([q.cpu()] + [t[:v_off + kv_heads * L * ep].cpu() for t in arenas])
+    assert all(torch.equal(x, y) for x, y in zip(*out)) and out[0][0].abs().max() > 0 and not (out[0][1] == 0.5).all()
+
+
 @pytest.mark.parametrize("gate_first", [0, 1])
 @pytest.mark.parametrize("heads,vdim,groups,rows", [(4, 64, 2, 3), (6, 20, 4, 5), (5, 13, 1, 2), (9, 128, 9, 1), (3, 24, 3, 70)])
 def test_gated_group_norm(dev, lib, heads, vdim, groups, rows, gate_first):
