@@ -102,6 +102,14 @@ LCC_DEVICE float block_sum(float v, float* red) {
   return t;
 }
 
+// Lanes of one wave hand values to each other through LDS: nothing that a lane stored before is read, and nothing that it read is overwritten, on
+// the wrong side of this.  LDS serves a wave in order, so no instruction is needed, but alias analysis is per thread: without the fence the compiler
+// may move one lane's load past another lane's store.
+LCC_DEVICE void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // two values after rounding to bf16: one conversion for the pair
 LCC_DEVICE void rbf2(float& a, float& b) {
   const unsigned u = pack2(a, b);

@@ -134,7 +134,7 @@ LCC_DEVICE bool wide_rows(const bf16_t* C, int ldc, const bf16_t* residual, int 
   if (EPI == EPI_PARTIAL || EPI == EPI_SWIGLU) return false;
   return (ldc & 7) == 0 && ((uintptr_t)C & 15) == 0 && (EPI != EPI_RESIDUAL || ((ldr & 7) == 0 && ((uintptr_t)residual & 15) == 0));
 }
-template <int EPI, int MT, int NT, bool AHEAD = true>          // AHEAD: the next group's residual in flight (where the registers are there for it)
+template <int EPI, int MT, int NT>
 LCC_DEVICE void tile_epilogue_wide(const f32x4 (&acc)[MT][NT], int mbase, int nbase, int lane, const bf16_t* __restrict__ bias,
                                    const bf16_t* __restrict__ residual, int ldr, bf16_t* __restrict__ C, int ldc, int M, int N,
                                    const float* __restrict__ wscale, unsigned char* lds) {
@@ -159,15 +159,15 @@ LCC_DEVICE void tile_epilogue_wide(const f32x4 (&acc)[MT][NT], int mbase, int nb
   constexpr int NS = GR * 16 / RPS;                                // stores of a group
   const int sr = lane / RC, schk = lane & (RC - 1), scol = nbase + schk * 8;          // this lane's row and chunk of a store
   const bool cok = scol < N;
-  u32x4 rv[AHEAD ? 2 : 1][NS];
-  auto load_res = [&](int i0, u32x4 (&r)[NS]) {
+  u32x4 rv[NS];                                                    // residual: a piece of the next group is fetched as this group's is used
+  auto load_res = [&](int i0, int q) { return ld16(residual + (size_t)min(mbase + i0 * 16 + q * RPS + sr, M - 1) * ldr + min(scol, N - 8)); };
+  if (EPI == EPI_RESIDUAL) {
 #pragma unroll
-    for (int q = 0; q < NS; ++q) r[q] = ld16(residual + (size_t)min(mbase + i0 * 16 + q * RPS + sr, M - 1) * ldr + min(scol, N - 8));
-  };
-  if (EPI == EPI_RESIDUAL) load_res(0, rv[0]);
+    for (int q = 0; q < NS; ++q) rv[q] = load_res(0, q);
+  }
 #pragma unroll
   for (int i0 = 0; i0 < MT; i0 += GR) {
-    if (EPI == EPI_RESIDUAL && (AHEAD ? i0 + GR < MT : i0 > 0)) load_res(AHEAD ? i0 + GR : i0, rv[AHEAD ? (i0 / GR + 1) & 1 : 0]);
+    wave_lds_order();          // the last group's rows have been read
 #pragma unroll
     for (int ii = 0; ii < GR; ++ii) {
       const int i = i0 + ii, r = ii * 16 + li;
@@ -186,15 +186,17 @@ LCC_DEVICE void tile_epilogue_wide(const f32x4 (&acc)[MT][NT], int mbase, int nb
         st8(lds + r * RB + (((j * 2 + (g >> 1)) ^ swz(r)) * 16) + (g & 1) * 8, (u32x2){pack2(v[0], v[1]), pack2(v[2], v[3])});
       }
     }
+    wave_lds_order();          // rows are read by other lanes than wrote them
 #pragma unroll
     for (int q = 0; q < NS; ++q) {
       if (i0 * 16 + q * RPS >= MT * 16) continue;                    // the last group may be shorter
       const int r = q * RPS + sr, m = mbase + i0 * 16 + r;
       u32x4 v = ld16(lds + r * RB + ((schk ^ swz(r)) * 16));
       if (EPI == EPI_RESIDUAL) {
-        const u32x4 w = rv[AHEAD ? (i0 / GR) & 1 : 0][q];
+        const u32x4 w = rv[q];
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = pack2(lo2f(v[e]) + lo2f(w[e]), hi2f(v[e]) + hi2f(w[e]));
+        if (i0 + GR < MT) rv[q] = load_res(i0 + GR, q);
       }
       if (m < M && cok) st16(C + (size_t)m * ldc + scol, v);
     }
@@ -218,6 +220,7 @@ LCC_DEVICE void tile_slab_wide(const f32x4 (&acc)[MT][NT], int mbase, int nbase,
   float* out = partial + (size_t)blockIdx.y * M * N + scol;
 #pragma unroll
   for (int i0 = 0; i0 < MT; i0 += 2) {
+    wave_lds_order();
 #pragma unroll
     for (int ii = 0; ii < 2; ++ii) {
       if (i0 + ii >= MT) continue;
@@ -225,6 +228,7 @@ LCC_DEVICE void tile_slab_wide(const f32x4 (&acc)[MT][NT], int mbase, int nbase,
 #pragma unroll
       for (int j = 0; j < NT; ++j) *reinterpret_cast<f32x4*>(lds + r * 256 + (((j * 4 + g) ^ (r & 15)) * 16)) = acc[i0 + ii][j] * sc[j];
     }
+    wave_lds_order();
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
       if (i0 * 16 + q * 4 >= MT * 16) continue;
@@ -884,7 +888,7 @@ LCC_DEVICE void gemm_big_body(
     tile_slab_wide<MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, lane, M, N, partial, wscale, reinterpret_cast<unsigned char*>(dsmem) + wave * 8192);
   } else if (wide_rows<EPI>(C, ldc, residual, ldr)) {
     __builtin_amdgcn_s_barrier();          // every wave is done with the stages, and its DMA pieces have landed
-    tile_epilogue_wide<EPI, MT, NT, !(W8 && BM == 256)>(acc, m0 + wm * WM, n0 + wn * 64, lane, bias, residual, ldr, C, ldc, M, N, wscale,
+    tile_epilogue_wide<EPI, MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, lane, bias, residual, ldr, C, ldc, M, N, wscale,
                                     reinterpret_cast<unsigned char*>(dsmem) + wave * 8192);
   } else tile_epilogue<EPI, MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, (n0 + wn * 64) / 2, li, g, bias, residual, ldr, C, ldc, M, N, partial, wscale);
 }
@@ -1100,7 +1104,7 @@ __global__ __launch_bounds__(512) void gemm_vh_kernel(
       tile_slab_wide<MTW, NT>(acc, m0 + my_row0, n0 + wn * 64, lane, M, N, partial, nullptr, reinterpret_cast<unsigned char*>(dsmem) + wave * 8192);
     } else if constexpr (MTW > 0) {
       if (wide)
-        tile_epilogue_wide<EPI, MTW, NT, false>(acc, m0 + my_row0, n0 + wn * 64, lane, bias, residual, ldr, C, ldc, M, N, nullptr,
+        tile_epilogue_wide<EPI, MTW, NT>(acc, m0 + my_row0, n0 + wn * 64, lane, bias, residual, ldr, C, ldc, M, N, nullptr,
                                          reinterpret_cast<unsigned char*>(dsmem) + wave * 8192);
       else tile_epilogue<EPI, MTW, NT>(acc, m0 + my_row0, n0 + wn * 64, (n0 + wn * 64) / 2, li, g, bias, residual, ldr, C, ldc, M, N, partial, nullptr);
     }
@@ -1603,18 +1607,14 @@ __global__ __launch_bounds__(256) void gemv_skinny_kernel(
         xf[1][0] = xv[u][1][0];
       } else {
         // raw lines -> wave-private LDS image [row][8 x 16 B], chunk c of row r at r*8 + (c ^ (r & 7)) -> fragments (row mg*16 + li,
-        // k-block h, lane group g).  One wave and in-order LDS: no s_barrier is needed, but the cross-LANE dependence (lane a's store, lane
-        // b's load of the same address) is invisible in per-thread alias analysis -- a wavefront-scope fence + wave barrier (no
-        // instructions on gfx950) keeps the compiler from reordering the two groups, here and in front of the next stage's stores.
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        // k-block h, lane group g)
+        wave_lds_order();
 #pragma unroll
         for (int i = 0; i < 2 * MG; ++i) {
           const int row = i * 8 + (lane >> 3);
           xs[row * 8 + ((lane & 7) ^ (row & 7))] = xv[u][i / MG][i % MG];
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_order();
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
