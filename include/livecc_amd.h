@@ -122,9 +122,8 @@ int lcc_debug_set_decode_path(int path);
  * CU) and for <= 2 streams; 0 (default) = separate launches.  A hand-off that times out fails the call (lcc_slot_read_tokens) and disables it. */
 int lcc_debug_set_decode_chain(int on);
 /* Block shape of the o_proj / down_proj decode GEMV (lcc_dgemv_resid): 0 = 8 waves per block, 1 (default) = 16 waves for bf16 weights with
- * K >= 8192 (the down projection: half the dependent chain of load stages per wave), 2 = 16 waves for every call, 3 = blocks of 8 output
- * rows (N <= 2048, M <= 8, bf16 weights: what the engine takes by itself under mode 1 where 16-row blocks would leave half the chip idle;
- * lcc_dgemv_resid then writes one statistic per 8 outputs, [M, N/8]).  Returns the old mode.
+ * K >= 8192 (the down projection: half the dependent chain of load stages per wave), 2 = 16 waves for every call; values beyond are 2.  Returns
+ * the old mode.  Under mode 1 the engine takes the blocks of 8 output rows (lcc_dgemv_resid_rows8) by itself where they suit.
  * The K split across the waves of a block -- and so the fp32 summation order -- differs between the two shapes. */
 int lcc_debug_set_resid_waves(int mode);
 /* Largest M (16..64, default 64) served by the weight-streaming GEMV kernels of lcc_gemm_bf16 and by the engine's decode step: with 17..64
@@ -262,6 +261,9 @@ int lcc_dgemv_norm_linear(const void* W_packed, const float* wscale, const void*
  * o_proj and down_proj: no inter-block K split, 8 waves per 16-row block. */
 int lcc_dgemv_resid(const void* W_packed, const float* wscale, const void* x, int ldx, void* h, float* stats_out, int M, int N, int K,
                     void* stream);
+/* the same in blocks of 8 output rows, stats_out [M, N/8] (one statistic per 8 outputs): bf16 weights, M <= 8, N <= 2048, N % 32 == 0 and
+ * K % 32 == 0, M * (K + 32) * 2 bytes of activations at most 144 KB; LCC_ERR_SHAPE otherwise. */
+int lcc_dgemv_resid_rows8(const void* W_packed, const void* x, int ldx, void* h, float* stats_out, int M, int N, int K, void* stream);
 /* q|k|v Linear of RMSNorm(h) + bias + M-RoPE (Q2VL:180-222) + in-place KV append at kv_len[tok_stream[m]] (cache_utils.py:127-146),
  * rotated q -> q_out [M, Hq*128].  W_dec = the q|k|v weight with rows permuted inside every 128-row head so that each 16-row tile
  * holds 8 channels and their rotation partners: stored row j*16 + half*8 + i = logical row half*64 + j*8 + i (weights.py). */

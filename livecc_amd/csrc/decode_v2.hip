@@ -605,11 +605,11 @@ __global__ __launch_bounds__(NW * 64) void dgemv_rows8_kernel(DgArgs a) {
   }
 }
 static int g_resid_waves = [] { const char* v = getenv("LCC_RESID_WAVES16"); return v ? atoi(v) : 1; }();
-// 16-row blocks that fill at most half the chip, whole 64-row groups of statistics, activations that fit LDS; modes 0 and 2
-// ask for blocks of 16 rows
-bool dgemv_rows8_ok(int M, int N, int K, const float* wscale) {
-  return (g_resid_waves == 1 || g_resid_waves == 3) && wscale == nullptr && M >= 1 && M <= 8 && N <= 2048 && (N & 31) == 0 && (K & 31) == 0 && (long)M * (K + X_PAD) * 2 <= ROWS8_LDS;
+// what the kernel takes: 16-row blocks that would fill at most half the chip, whole 32-row groups of statistics, activations that fit LDS
+static bool rows8_fits(int M, int N, int K, const float* wscale) {
+  return wscale == nullptr && M >= 1 && M <= 8 && N <= 2048 && (N & 31) == 0 && (K & 31) == 0 && (long)M * (K + X_PAD) * 2 <= ROWS8_LDS;
 }
+bool dgemv_rows8_ok(int M, int N, int K, const float* wscale) { return g_resid_waves == 1 && rows8_fits(M, N, K, wscale); }      // modes 0 and 2 ask for blocks of 16 rows
 template <int EPI, int NW, int XP>
 static void launch_rows8_as(const DgArgs& a, hipStream_t st) {
   static DeviceOnce attr;
@@ -760,12 +760,12 @@ int dgemv_qkv_rope(const DgArgs& a, hipStream_t st) {
   else dgemv_kernel<1, DG_PRO_NORM, DG_EPI_ROPE, 8, 4, 4><<<dim3(a.N / 16), dim3(512), (size_t)a.M * a.K * 2, st>>>(a);
   return 0;
 }
-int set_resid_waves(int mode) { const int old = g_resid_waves; g_resid_waves = mode < 0 ? 0 : (mode > 3 ? 3 : mode); return old; }
+int set_resid_waves(int mode) { const int old = g_resid_waves; g_resid_waves = mode < 0 ? 0 : (mode > 2 ? 2 : mode); return old; }
 // o_proj / down_proj: x plain, residual add in place + per-tile sums of squares
 int dgemv_resid(const DgArgs& a, hipStream_t st) {
   if (int rc = dg_check(a, DG_PRO_PLAIN, DG_EPI_RESID)) return rc;
-  if (a.rows8 || g_resid_waves == 3) {
-    if (!dgemv_rows8_ok(a.M, a.N, a.K, a.wscale)) return LCC_ERR_ARG;
+  if (a.rows8) {
+    if (!rows8_fits(a.M, a.N, a.K, a.wscale)) return LCC_ERR_SHAPE;
     launch_rows8<DG_EPI_RESID>(a, st);
     return 0;
   }
@@ -777,7 +777,6 @@ int dgemv_resid(const DgArgs& a, hipStream_t st) {
   // Mode (lcc_debug_set_resid_waves; initial value from LCC_RESID_WAVES16): 0 = 8 waves always, 1 (default) = 16 waves for bf16 weights
   // with K >= 8192, 2 = 16 waves for every call.
   const int w16 = g_resid_waves;
-  // 3 = blocks of 8 output rows (dgemv_rows8_kernel; the engine asks for them by DgArgs::rows8 where they suit).
   const bool wide = w16 == 2 || (w16 == 1 && a.K >= 8192 && a.wscale == nullptr);
   if (a.C != nullptr) {          // u = bf16(norm_w * h) beside h: the activations of the next row-scaled product
     if (a.norm_w == nullptr) return LCC_ERR_ARG;

@@ -319,6 +319,11 @@ extern "C" int lcc_dgemv_resid(const void* W_packed, const float* wscale, const 
   DgArgs a; a.W = (const bf16_t*)W_packed; a.wscale = wscale; a.M = M; a.N = N; a.K = K; a.X = (const bf16_t*)x; a.ldx = ldx; a.Hres = (bf16_t*)h; a.stats_out = stats_out;
   OP_RET(dgemv_resid(a, (hipStream_t)stream), "lcc_dgemv_resid");
 }
+extern "C" int lcc_dgemv_resid_rows8(const void* W_packed, const void* x, int ldx, void* h, float* stats_out, int M, int N, int K, void* stream) {
+  if (!W_packed || !x || !h || !stats_out) return fail(LCC_ERR_ARG, "null pointer");
+  DgArgs a; a.W = (const bf16_t*)W_packed; a.M = M; a.N = N; a.K = K; a.X = (const bf16_t*)x; a.ldx = ldx; a.Hres = (bf16_t*)h; a.stats_out = stats_out; a.rows8 = true;
+  OP_RET(dgemv_resid(a, (hipStream_t)stream), "lcc_dgemv_resid_rows8");
+}
 extern "C" int lcc_dgemv_qkv_rope(const void* W_dec_packed, const float* wscale, const void* h, const float* stats, const void* norm_w, float eps,
                                   const void* bias,
                                   const void* cos, const void* sin, const int32_t* tok_stream, const int32_t* kv_len, void* const* kv_base,

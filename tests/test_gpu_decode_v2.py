@@ -76,16 +76,32 @@ def test_residual_gemv_in_blocks_of_eight_rows(dev, M, N, K):
     lib = _lib.load()
     x, w, h0 = _rand((M, K), dev, 1.0, 7), _rand((N, K), dev, 0.03, 8), _rand((M, N), dev, 2.0, 9)
     h, wp, stats = h0.clone(), ops.pack_weight(w), torch.full((M, N // 8), -1.0, device=dev)
-    old = lib.lcc_debug_set_resid_waves(3)
-    try:
-        _lib.check(lib.lcc_dgemv_resid(wp.data_ptr(), None, x.data_ptr(), K, h.data_ptr(), stats.data_ptr(), M, N, K,
-                                       torch.cuda.current_stream(dev).cuda_stream), "lcc_dgemv_resid")
-    finally:
-        lib.lcc_debug_set_resid_waves(old)
+    _lib.check(lib.lcc_dgemv_resid_rows8(wp.data_ptr(), x.data_ptr(), K, h.data_ptr(), stats.data_ptr(), M, N, K,
+                                         torch.cuda.current_stream(dev).cuda_stream), "lcc_dgemv_resid_rows8")
     ref, atol = _ref_linear(x, w, None, 3, h0, with_atol=True)
     assert_bf16_close(h, ref, f"dgemv_resid8[{M}x{N}x{K}]", max_ulp=1.0, max_frac=1e-2, atol=atol)
     want = h.float().view(M, N // 8, 8).pow(2).sum(-1)
     assert torch.allclose(stats, want, rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2, 3, 100])
+@pytest.mark.parametrize("M,N,K,fp8", [(2, 1536, 1536, False), (2, 2112, 512, False), (9, 96, 128, False), (2, 96, 128, True)])
+def test_no_mode_refuses_a_residual_gemv_or_changes_its_statistics(dev, M, N, K, fp8, mode):
+    """The process-wide block shape, whatever it is set to (values beyond the last mean the last): products that blocks of 8 rows serve and products
+    that they do not all run, and write the documented [M, N/16] statistics and nothing behind them."""
+    from livecc_amd import _lib, ops
+    lib = _lib.load()
+    x, w, h = _rand((M, K), dev, 1.0, 7), _rand((N, K), dev, 0.03, 8), _rand((M, N), dev, 2.0, 9)
+    wp, sc = ops.quantize_fp8(w) if fp8 else (ops.pack_weight(w), None)
+    stats = torch.full((2 * M * (N // 16),), -1.0, device=dev)
+    old = lib.lcc_debug_set_resid_waves(mode)
+    try:
+        _lib.check(lib.lcc_dgemv_resid(wp.data_ptr(), sc.data_ptr() if fp8 else None, x.data_ptr(), K, h.data_ptr(), stats.data_ptr(), M, N, K,
+                                       torch.cuda.current_stream(dev).cuda_stream), "lcc_dgemv_resid")
+    finally:
+        assert lib.lcc_debug_set_resid_waves(old) == min(mode, 2)
+    n = M * (N // 16)
+    assert torch.allclose(stats[:n].view(M, -1), ops.tile_stats(h), rtol=1e-6, atol=1e-6) and bool((stats[n:] == -1.0).all())
 
 
 @pytest.mark.parametrize("Hq,Hkv,K", [(28, 4, 3584), (12, 2, 1536), (2, 1, 256), (7, 1, 896)])
