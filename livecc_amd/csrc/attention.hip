@@ -1051,6 +1051,24 @@ int attn_prefill_bf16(const bf16_t* q, bf16_t* out, const int32_t* tile_stream, 
   return 0;
 }
 
+// Key splits of the per-wave decode attention.  One key tile a split up to 24 tiles, two beyond: a wave's first two tiles are requested together, every
+// further pair is another trip, and the merge fetches up to 64 splits in one (decode step of one stream, 1 / 2 / 4 tiles a split: 2B at 500 keys
+// 1.168 / 1.177 / 1.216 ms, 7B at 2,000 keys 2.792 / 2.787 / 2.825).  64 splits at most up to 16k keys, 128 beyond: 9,000 keys 2.930 / 2.948 ms with
+// 64 / 128, 24,000 keys 3.136 / 3.067.
+// At most 768 blocks over all (stream, KV head) pairs: three waves a compute unit already pull what it can, and more only write and merge more partials.
+// Eight layers of a decode step with 512 / 768 / 1,024 blocks / no limit, us: 7B 16 streams of 8,000 keys 1,532 / 1,521 / 1,530 / 1,600, eight of 4,000
+// 1,091 / 1,101 / 1,092 / 1,115; 7B fp8, 32 streams of 4,000 1,720 / 1,714 / 1,718 / 1,846; 72B fp8, 64 streams of 2,000 3,449 / 3,449 / 3,449 / 3,747.
+// Over 120 points of 1 to 64 streams the mean distance from the best split count is 0.30 / 0.26 / 0.45 %.
+// Tuning knobs LCC_ATTN_TPS, LCC_ATTN_MAXSPLIT.
+int attn_decode_splits(int max_keys, int pairs) {
+  static const int tps_env = [] { const char* v = getenv("LCC_ATTN_TPS"); return v ? std::max(1, atoi(v)) : 0; }();
+  static const int maxsplit_env = [] { const char* v = getenv("LCC_ATTN_MAXSPLIT"); return v ? std::max(1, std::min(128, atoi(v))) : 0; }();
+  const int ntile = (max_keys + 31) / 32;
+  const int maxsplit = maxsplit_env ? maxsplit_env : std::min(ntile <= 512 ? 64 : 128, std::max(2, 768 / std::max(1, pairs)));
+  const int tps = tps_env ? tps_env : (ntile <= 24 ? 1 : 2);
+  return std::max(1, std::min(maxsplit, (ntile + tps - 1) / tps));
+}
+
 int attn_decode_bf16(const bf16_t* q, bf16_t* out, const int32_t* slots, const int32_t* kv_len, bf16_t* const* kv_base,
                      KvLayout lay, int layer, int B, int n_q_heads, int nsplit, float* ws_o, float* ws_ml, hipStream_t st,
                      const AttnDirect* direct) {

@@ -472,15 +472,7 @@ extern "C" int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots
   }
   LlmBuffers bf; LCC_TRY(carve_llm(e, &bf));
   const int ntile = (max_len + 31) / 32;
-  // key tiles per split of the per-wave decode attention: one up to 24 tiles, two beyond -- a wave's first two tiles are requested together,
-  // every further pair is another trip, and the merge fetches up to 64 splits in one (decode step, 1 / 2 / 4 tiles a split: 2B at 500 keys
-  // 1.168 / 1.177 / 1.216 ms, 7B at 2,000 keys 2.792 / 2.787 / 2.825).  64 splits
-  // at most up to 16k keys, 128 beyond: 9,000 keys 2.930 / 2.948 ms with 64 / 128, 24,000 keys 3.136 / 3.067.  Tuning knobs LCC_ATTN_TPS, LCC_ATTN_MAXSPLIT
-  static const int tps_env = [] { const char* v = getenv("LCC_ATTN_TPS"); return v ? std::max(1, atoi(v)) : 0; }();
-  static const int maxsplit_env = [] { const char* v = getenv("LCC_ATTN_MAXSPLIT"); return v ? std::max(1, std::min(128, atoi(v))) : 0; }();
-  const int maxsplit = maxsplit_env ? maxsplit_env : (ntile <= 512 ? 64 : 128);
-  const int tps = tps_env ? tps_env : (ntile <= 24 ? 1 : 2);
-  const int nsplit = std::max(1, std::min(maxsplit, (ntile + tps - 1) / tps));
+  const int nsplit = attn_decode_splits(max_len, n_streams * e->c.n_kv_heads);
 
   LayerCtx cx{};
   // weight-streaming ("skinny") layer sequence for up to 64 streams: fp32 split-K slabs consumed by rope / add+norm kernels.  fp8 weights

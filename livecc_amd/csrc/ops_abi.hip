@@ -29,6 +29,10 @@ extern "C" int lcc_debug_attn_tile_rows(int n_q_heads, int n_kv_heads) {   // ho
   const int G = n_q_heads / n_kv_heads;
   return (get_attn_variant() == 3 && G <= 8) ? attn32_tile_rows(G) : 32;
 }
+extern "C" int lcc_debug_attn_decode_splits(int max_keys, int pairs) {
+  if (max_keys < 1 || pairs < 1) return fail(LCC_ERR_ARG, "lcc_debug_attn_decode_splits: invalid arguments");
+  return attn_decode_splits(max_keys, pairs);
+}
 extern "C" int lcc_debug_attn_plan(const int32_t* n_new, int n_streams, int max_kv, int n_q_heads, int n_kv_heads, int cu_count, int32_t* tile_rows,
                                    int32_t* splits) {   // host logic only: no launch
   if (!n_new || n_streams < 1 || max_kv < 1 || n_kv_heads < 1 || n_q_heads < n_kv_heads || n_q_heads % n_kv_heads || cu_count < 1 || !tile_rows || !splits)
