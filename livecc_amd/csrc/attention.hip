@@ -641,12 +641,13 @@ __global__ __launch_bounds__(64, 2) void attn_decode_kernel(
 // need all 204 CUs' worth of one-wave blocks -- and with it the 51 partials.  profiles/r06/decode_attn_multiwave_ab.jsonl.)
 // grid = (Hq, B), 256 threads = 8 split groups x 32 lanes (4 consecutive d each).  Group q merges splits q, q+8, ...; the 8 partial
 // (m, num, den) triples are merged through LDS.  What bounds it is the trip to the partials other XCDs wrote (they come from beyond the
-// L2): all 24 loads of up to 64 splits go out together (one running maximum per split, each iteration's loads behind the last one's use,
-// took two to eight trips).
+// L2): all loads of up to 8 U splits go out together (one running maximum per split, each iteration's loads behind the last one's use,
+// took two to eight trips).  U = 1 / 2 / 4 / 8 for up to 8 / 16 / 32 / more splits: loads that only repeat the last split cost their issue.
+template <int U>
 __global__ __launch_bounds__(256) void attn_decode_combine_kernel(
     const float* __restrict__ ws_o, const float* __restrict__ ws_ml, bf16_t* __restrict__ out, int n_q_heads,
     int n_kv_heads, int nsplit) {
-  constexpr int D = 128, NG = 8, U = 8;
+  constexpr int D = 128, NG = 8;
   __shared__ float sm[NG][32][6];
   const int hq = blockIdx.x, b = blockIdx.y, t = threadIdx.x, dl = t & 31, grp = t >> 5;
   const int G = n_q_heads / n_kv_heads, hk = hq / G, j = hq % G;
@@ -695,6 +696,14 @@ __global__ __launch_bounds__(256) void attn_decode_combine_kernel(
   }
   const float inv = 1.f / dd;
   st8(out + ((size_t)b * n_q_heads + hq) * D + dl * 4, (u32x2){pack2(n0 * inv, n1 * inv), pack2(n2 * inv, n3 * inv)});
+}
+
+static void launch_decode_combine(const float* ws_o, const float* ws_ml, bf16_t* out, int n_q_heads, int n_kv_heads, int B, int nsplit, hipStream_t st) {
+  const dim3 grid(n_q_heads, B), blk(256);
+  if (nsplit <= 8) attn_decode_combine_kernel<1><<<grid, blk, 0, st>>>(ws_o, ws_ml, out, n_q_heads, n_kv_heads, nsplit);
+  else if (nsplit <= 16) attn_decode_combine_kernel<2><<<grid, blk, 0, st>>>(ws_o, ws_ml, out, n_q_heads, n_kv_heads, nsplit);
+  else if (nsplit <= 32) attn_decode_combine_kernel<4><<<grid, blk, 0, st>>>(ws_o, ws_ml, out, n_q_heads, n_kv_heads, nsplit);
+  else attn_decode_combine_kernel<8><<<grid, blk, 0, st>>>(ws_o, ws_ml, out, n_q_heads, n_kv_heads, nsplit);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1081,8 +1090,7 @@ int attn_decode_bf16(const bf16_t* q, bf16_t* out, const int32_t* slots, const i
   else
     attn_decode_kernel<false><<<dim3(nsplit, lay.n_kv_heads, B), dim3(64), 0, st>>>(
         q, slots, kv_len, kv_base, lay, layer, n_q_heads, nsplit, ws_o, ws_ml, scale_l2e(128), AttnDirect{});
-  attn_decode_combine_kernel<<<dim3(n_q_heads, B), dim3(256), 0, st>>>(ws_o, ws_ml, out, n_q_heads,
-                                                                       lay.n_kv_heads, nsplit);
+  launch_decode_combine(ws_o, ws_ml, out, n_q_heads, lay.n_kv_heads, B, nsplit, st);
   return 0;
 }
 
@@ -1124,7 +1132,7 @@ int attn_decode_fused_bf16(const float* qkv_part, int ns_qkv, const bf16_t* bias
   }
 #undef LCC_ADF
   if (tail != 0 && nsplit > 1)
-    attn_decode_combine_kernel<<<dim3(n_q_heads, B), dim3(256), 0, st>>>(ws_o, ws_ml, out, n_q_heads, lay.n_kv_heads, nsplit);
+    launch_decode_combine(ws_o, ws_ml, out, n_q_heads, lay.n_kv_heads, B, nsplit, st);
   return 0;
 }
 

@@ -762,6 +762,21 @@ def test_rope_append_prefill_decode_attention(dev, Hq, Hkv, attn_variant):
         _check_attn(got.view(1, Hq, D), ref, f"attn_decode[Hq{Hq},nsplit{nsplit}]")
 
 
+@pytest.mark.parametrize("nsplit", [1, 8, 9, 16, 17, 32, 33, 64, 65, 128])
+def test_decode_attention_merge_at_every_width(dev, nsplit):
+    """The split merge at both ends of its 8, 16, 32 and 64 splits a trip and beyond, for a long stream and one that leaves most splits without a key."""
+    from livecc_amd import ops
+    Hq, Hkv, D, lens = 14, 2, 128, [4099, 70]
+    kv = ops.KvArena(2, 1, Hkv, 4160, dev)
+    kv.buf.copy_(_rand(tuple(kv.buf.shape), dev, 1.0, 31))
+    q = _rand((2, Hq * D), dev, 1.0, 32)
+    got = ops.attn_decode(q, kv, 0, torch.tensor([0, 1], dtype=torch.int32, device=dev), torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=dev), Hq, nsplit)
+    for b, n in enumerate(lens):
+        K, V = kv.k_view(b, 0)[:, :n].float().transpose(0, 1).cpu(), kv.v_view(b, 0)[:, :n].float().transpose(0, 1).cpu()
+        ref = rb(_ref_attn_causal(q[b].float().view(1, Hq, D).cpu(), K, V, n - 1))
+        _check_attn(got[b].view(1, Hq, D).cpu(), ref, f"attn_decode_merge[{nsplit},{n}]")
+
+
 @pytest.mark.parametrize("Hq,Hkv", [(7, 1), (28, 4), (12, 2), (8, 1), (2, 1)])
 @pytest.mark.parametrize("NS", [1, 3, 4])
 def test_attn_decode_fused_matches_separate_kernels(dev, Hq, Hkv, NS):
