@@ -167,6 +167,7 @@ LCC_DEVICE void tile_epilogue_wide(const f32x4 (&acc)[MT][NT], int mbase, int nb
   }
 #pragma unroll
   for (int i0 = 0; i0 < MT; i0 += GR) {
+    if (mbase + i0 * 16 >= M) break;          // no row of this group exists (wave-uniform)
     wave_lds_order();          // the last group's rows have been read
 #pragma unroll
     for (int ii = 0; ii < GR; ++ii) {
@@ -220,6 +221,7 @@ LCC_DEVICE void tile_slab_wide(const f32x4 (&acc)[MT][NT], int mbase, int nbase,
   float* out = partial + (size_t)blockIdx.y * M * N + scol;
 #pragma unroll
   for (int i0 = 0; i0 < MT; i0 += 2) {
+    if (mbase + i0 * 16 >= M) break;          // 17 rows of a 128-row tile: one group in four (fp8 steps of 17 to 64 streams)
     wave_lds_order();
 #pragma unroll
     for (int ii = 0; ii < 2; ++ii) {
