@@ -1075,7 +1075,8 @@ int attn_decode_splits(int max_keys, int pairs) {
   const int ntile = (max_keys + 31) / 32;
   const int maxsplit = maxsplit_env ? maxsplit_env : std::min(ntile <= 512 ? 64 : 128, std::max(2, 768 / std::max(1, pairs)));
   const int tps = tps_env ? tps_env : (ntile <= 24 ? 1 : 2);
-  return std::max(1, std::min(maxsplit, (ntile + tps - 1) / tps));
+  const int n = std::max(1, std::min(maxsplit, (ntile + tps - 1) / tps)), per = (ntile + n - 1) / n;
+  return (ntile + per - 1) / per;          // without those that would be left without a tile: 10 tiles in 8 splits are 5 of two
 }
 
 int attn_decode_bf16(const bf16_t* q, bf16_t* out, const int32_t* slots, const int32_t* kv_len, bf16_t* const* kv_base,

@@ -86,14 +86,14 @@ def test_prefill_attention_plan_at_the_engines_shapes(built_lib):
 
 def test_decode_attention_splits_over_streams(built_lib):
     """Key splits of the decode attention, as lcc_llm_decode asks for them: one stream as many as its tiles give (one tile up to 24 of them, two
-    beyond, 64 splits, 128 from 16k keys on); batches stop at 768 blocks, two splits at least, so that 64 streams do not write and merge the
+    beyond, up to 64 splits, 128 from 16k keys on, none without a tile); batches stop at 768 blocks, two splits at least, so that 64 streams do not write and merge the
     partials of 64 splits each."""
     f = built_lib.lcc_debug_attn_decode_splits
-    assert [f(k, 4) for k in (1, 32, 33, 500, 768, 769, 2000, 6500, 16384, 16385, 24000)] == [1, 1, 2, 16, 24, 13, 32, 64, 64, 128, 128]
-    assert [f(4000, 4 * n) for n in (1, 2, 3, 4, 8, 12, 16, 17, 32, 48, 64)] == [63, 63, 63, 48, 24, 16, 12, 11, 6, 4, 3]
+    assert [f(k, 4) for k in (1, 32, 33, 500, 768, 769, 2000, 6500, 16384, 16385, 24000)] == [1, 1, 2, 16, 24, 13, 32, 51, 64, 103, 125]
+    assert [f(4000, 4 * n) for n in (1, 2, 3, 4, 8, 12, 16, 17, 32, 48, 64)] == [63, 63, 63, 42, 21, 16, 12, 11, 6, 4, 3]
     assert f(6000, 8 * 64) == 2 and f(40, 8 * 64) == 2 and f(20, 8 * 64) == 1
     for pairs in range(1, 513):
         for keys in (1, 100, 700, 3000, 9000, 30000):
-            n = f(keys, pairs)
-            assert 1 <= n <= 128 and (n <= 2 or n * pairs <= 768) and n <= (keys + 31) // 32
+            n, tiles = f(keys, pairs), (keys + 31) // 32
+            assert 1 <= n <= 128 and (n <= 2 or n * pairs <= 768) and (n - 1) * -(-tiles // n) < tiles          # no split without a tile
     assert f(0, 1) < 0 and f(1, 0) < 0
