@@ -569,6 +569,8 @@ int lcc_llm_prefill(lcc_engine* e, int n_streams, const int32_t* slots, const in
 #define LCC_MAX_DECODE_BATCH 64
 int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots, int n_steps, int first_step_index,
                    const lcc_sampling* sp, void* stream);
+/* 1 if a decode step of that many streams takes the row-scaled products of the fused pipeline (3 to 16 streams: host logic, no GPU), else 0. */
+int lcc_debug_decode_row_scaled(const lcc_engine* e, int n_streams);
 /* blocking: copy the ids generated by the last generate call of a slot to the host (at most max_n), report how many
  * were generated (EOS included) and refresh the host mirror of the slot's KV length / next position. */
 int lcc_slot_read_tokens(lcc_engine* e, int slot, int32_t* out, int max_n, int* n_generated, void* stream);

@@ -193,6 +193,19 @@ bool decode_v2_ok(const lcc_engine* e) {
   for (const LlmLayerW& L : e->llm) if (L.qkv_w_dec == nullptr || (e->c.llm_fp8 && L.qkv_s_dec == nullptr)) return false;
   return true;
 }
+// v2 normalises rows in every block for one or two streams and uses row-scaled products for 3 to 16 (one / two streams: 7B 2.81 / 2.90 ms a
+// step against 2.81 / 2.93 row-scaled, 2B 1.17 / 1.18 against 1.19 / 1.19; three: 3.02 -> 2.85 against the sequence with norm launches).
+// More than eight rows do not fit the 8-row residual blocks, and 16-row ones leave most of the chip idle at 2,048 hidden channels and
+// below: 2B, 12 / 16 streams 1.48 / 1.56 ms with norm launches against 1.52 / 1.66 (nine: 1.44 against 1.41).
+// What it saves is two norm launches and the slabs of a layer, what it costs is slower products, by their bytes and their rows: it serves while a
+// layer's weight bytes x rows stay below 8e9.  Eight layers at 2,000 keys, row-scaled / with norm launches, us: 7B (466 MB a layer) 16 streams
+// 1,271 / 1,284; 72B (1.76 GB) 3 / 4 / 5 / 8 / 16 streams 2,736 / 2,765 / 2,805 / 2,934 / 3,489 against 2,742 / 2,759 / 2,784 / 2,889 / 3,349; 72B in
+// fp8 8 / 9 / 12 / 16 streams 1,876 / 1,944 / 2,197 / 2,525 against 1,891 / 1,940 / 2,175 / 2,468.
+bool decode_row_scaled(const lcc_engine* e, int n_streams) {
+  const double H = e->c.hidden_size, I = e->c.intermediate_size;
+  const double layer_bytes = (H * (e->qkvd + e->qd) + 3.0 * H * I) * (e->c.llm_fp8 ? 1 : 2);
+  return n_streams >= 3 && n_streams <= (H > 2048 ? 16 : 8) && n_streams * layer_bytes <= 8e9;
+}
 // the 28 decoder layers of ONE decode step over B rows, v2 launch sequence (us: row-scaled products, b.xn = u).  On entry b.h / b.stats / b.cos / b.sin come from
 // decode_step_begin; on exit b.h is the residual stream after the last layer and b.stats its per-tile sums of squares (the final
 // RMSNorm runs as the prologue of the lm_head GEMV).
@@ -439,6 +452,10 @@ extern "C" int lcc_llm_prefill(lcc_engine* e, int n_streams, const int32_t* slot
   return check_launch("lcc_llm_prefill");
 }
 
+extern "C" int lcc_debug_decode_row_scaled(const lcc_engine* e, int n_streams) {
+  if (!e || n_streams < 1 || e->family == LCC_FAMILY_DECODER) return fail(LCC_ERR_ARG, "bad argument");
+  return decode_row_scaled(e, n_streams) ? 1 : 0;
+}
 extern "C" int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots, int n_steps, int first_step_index,
                               const lcc_sampling* sp, void* stream) {
   LCC_TRY(ensure_ready(e));
@@ -486,11 +503,7 @@ extern "C" int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots
   // fused kernel: 4 waves per block; about one block per CU, never less than one key tile per wave
   static const int fused_blocks = [] { const char* v = getenv("LCC_ATTN_FUSED_BLOCKS"); return v ? std::max(64, atoi(v)) : 256; }();
   cx.nsplit_attn_fused = std::max(1, std::min(std::min(32, (ntile + 3) / 4), std::max(1, fused_blocks / (n_streams * e->c.n_kv_heads))));
-  // v2 normalises rows in every block for one or two streams and uses row-scaled products for 3 to 16 (one / two streams: 7B 2.81 / 2.90 ms a
-  // step against 2.81 / 2.93 row-scaled, 2B 1.17 / 1.18 against 1.19 / 1.19; three: 3.02 -> 2.85 against the sequence below, 16: 3.93 -> 3.71).
-  // More than eight rows do not fit the 8-row residual blocks, and 16-row ones leave most of the chip idle at 2,048 hidden channels and
-  // below: 2B, 12 / 16 streams 1.48 / 1.56 ms below against 1.52 / 1.66 (nine: 1.44 against 1.41).
-  const bool us = n_streams >= 3 && n_streams <= (e->c.hidden_size > 2048 ? 16 : 8) && e->llm_over == nullptr;
+  const bool us = decode_row_scaled(e, n_streams) && e->llm_over == nullptr;
   const bool v2 = decode_v2_ok(e) && (us || (n_streams <= 2 && (long)n_streams * e->c.hidden_size <= 16384));
   for (int step = 0; step < n_steps; ++step) {
     int n_stat = 0;

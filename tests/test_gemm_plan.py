@@ -97,3 +97,22 @@ def test_decode_attention_splits_over_streams(built_lib):
             n, tiles = f(keys, pairs), (keys + 31) // 32
             assert 1 <= n <= 128 and (n <= 2 or n * pairs <= 768) and (n - 1) * -(-tiles // n) < tiles          # no split without a tile
     assert f(0, 1) < 0 and f(1, 0) < 0
+
+
+@pytest.mark.parametrize("preset,fp8,last", [("livecc-7b", 0, 16), ("livecc-7b", 1, 16), ("qwen2vl-2b", 0, 8), ("qwen2vl-2b", 1, 8), ("qwen2vl-72b", 0, 4), ("qwen2vl-72b", 1, 9)])
+def test_decode_batches_that_take_the_row_scaled_products(built_lib, preset, fp8, last):
+    """From three streams on while a layer's weight bytes x rows are below 8e9, 16 streams at most (8 at 2,048 channels and below)."""
+    import ctypes
+    from livecc_amd import _lib
+    from livecc_amd.config import PRESETS
+    c = PRESETS[preset]()
+    cfg = _lib.ModelConfig(c.vocab_size, c.hidden_size, c.intermediate_size, c.num_hidden_layers, c.num_attention_heads, c.num_key_value_heads, 128, 1e-6, 16, 24, 24,
+                           c.vit_depth, c.vit_embed_dim, c.vit_num_heads, c.vit_mlp_dim, 1176, 2)
+    cfg.llm_fp8 = fp8
+    lim = _lib.EngineLimits(64, 1024, 256, 1024, 16)
+    e = built_lib.lcc_engine_create(ctypes.byref(cfg), ctypes.byref(lim))
+    try:
+        assert [n for n in range(1, 65) if built_lib.lcc_debug_decode_row_scaled(e, n)] == list(range(3, last + 1))
+        assert built_lib.lcc_debug_decode_row_scaled(e, 0) < 0 and built_lib.lcc_debug_decode_row_scaled(None, 3) < 0
+    finally:
+        built_lib.lcc_engine_destroy(e)
