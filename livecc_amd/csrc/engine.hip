@@ -317,7 +317,7 @@ extern "C" int lcc_slot_reset(lcc_engine* e, int slot, void* stream) {
   e->h_kv_len[slot] = 0; e->h_pos[slot] = 0;
   // one launch: six fills of a few bytes cost 17 us a slot
   LCC_TRY(reset_slot(slot, e->d_kv_len, e->d_pos, e->d_hist_col, e->d_done, e->d_rng_ctr, e->d_seen, e->words, st));
-  return 0;
+  return check_launch("lcc_slot_reset");
 }
 extern "C" int lcc_slot_set_length(lcc_engine* e, int slot, int kv_len, int next_pos, void* stream) {
   if (!e || slot < 0 || slot >= e->lim.max_slots) return fail(LCC_ERR_ARG, "bad slot");

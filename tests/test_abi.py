@@ -109,3 +109,23 @@ def test_production_attention_kernels_keep_their_accumulators_in_vgprs():
     flagged = [line for line in p.stdout.splitlines() if line.startswith(("attention.hip", "attn32.hip"))]
     for name in ("attn_decode_kernel<", "attn_decode_fused_kernel<", "attn_gqa32_kernel<", "attn_vit32_kernel<8>"):
         assert not [line for line in flagged if name in line], (name, flagged)
+
+
+def test_a_slot_reset_that_could_not_be_launched_says_so(lib):
+    """Without a GPU no kernel can be launched: the call reports it instead of a slot that was cleared on the host only."""
+    import numpy as np
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("the buffers below are host memory")
+    from livecc_amd.config import tiny
+    c = tiny()
+    cfg = _lib.ModelConfig(c.vocab_size, c.hidden_size, c.intermediate_size, c.num_hidden_layers, c.num_attention_heads, c.num_key_value_heads, 128, 1e-6, 16, 24, 24,
+                           c.vit_depth, c.vit_embed_dim, c.vit_num_heads, c.vit_mlp_dim, 1176, 2)
+    e = lib.lcc_engine_create(ctypes.byref(cfg), ctypes.byref(_lib.EngineLimits(1, 64, 16, 16, 4)))
+    assert e and lib.lcc_slot_reset(e, 0, None) != 0          # nothing bound yet
+    sizes = [lib.lcc_engine_workspace_bytes(e), lib.lcc_engine_state_bytes(e), lib.lcc_engine_meta_bytes(e)]
+    mem = [np.zeros(n + 256, dtype=np.uint8) for n in sizes + sizes[2:]]
+    ptr = [(m.ctypes.data + 255) // 256 * 256 for m in mem]
+    assert lib.lcc_engine_bind_buffers(e, ptr[0], sizes[0], ptr[1], sizes[1], ptr[2], ptr[3], sizes[2]) != 0      # cleared by the device
+    assert lib.lcc_slot_reset(e, 0, None) != 0 and b"lcc_slot_reset" in lib.lcc_last_error()
+    lib.lcc_engine_destroy(e)
