@@ -161,7 +161,9 @@ int lcc_patchify_norm_u8(const uint8_t* frames, int layout, int T, int H, int W,
  * src: uint8 frames, layout 0 = [T,Hin,Win,3], 1 = [T,3,Hin,Win]; dst: uint8 [T,3,Hout,Wout].  Tap tables per output index
  * (first source index, tap count, fp32 weights) are computed by the caller with ATen's arithmetic
  * (livecc_amd/resize.py:aa_bicubic_taps): wx is TAP-MAJOR [kx][Wout] (coalesced across the lanes of the width pass), wy is
- * [Hout][ky]; tmp = T*3*Hin*Wout floats.  Bit-identical to the reference's CPU result. */
+ * [Hout][ky]; tmp = a buffer of at least lcc_resize_bicubic_aa_tmp_floats floats (never NULL): the fp32 rows between the two passes,
+ * T*3*Hin*Wout of them, or none where both passes run in one launch.  Bit-identical to the reference's CPU result. */
+size_t lcc_resize_bicubic_aa_tmp_floats(int layout, int T, int Hin, int Win, int Hout, int Wout, int kx, int ky);
 int lcc_resize_bicubic_aa_u8(const uint8_t* src, int layout, int T, int Hin, int Win, uint8_t* dst, int Hout, int Wout,
                              const int32_t* xmin, const int32_t* xsize, const float* wx, int kx, const int32_t* ymin,
                              const int32_t* ysize, const float* wy, int ky, float* tmp, void* stream);

@@ -782,19 +782,34 @@ static void launch_resize_tile(const uint8_t* src, int layout, int T, int Hin, i
     resize_aa_tile_kernel<K, true><<<grid, dim3(RS_WAVES * 64), lds, st>>>(src, T, Hin, Win, dst, Hout, Wout, xmin, xsize, wx, ymin, ysize, wy, ky, TH, rows_cap, seg_dw);
 }
 
-int resize_bicubic_aa_u8(const uint8_t* src, int layout, int T, int Hin, int Win, uint8_t* dst, int Hout, int Wout,
-                         const int32_t* xmin, const int32_t* xsize, const float* wx, int kx, const int32_t* ymin,
-                         const int32_t* ysize, const float* wy, int ky, float* tmp, hipStream_t st) {
-  if (T <= 0 || Hin <= 0 || Win <= 0 || Hout <= 0 || Wout <= 0 || kx <= 0 || ky <= 0 || (layout != 0 && layout != 1)) return LCC_ERR_SHAPE;
-  // one launch while a tile's window fits RS_LDS_MAX with at least 8 rows: scales up to about 4 (tap tables of 5 to 17 columns); wider filters
-  // take the two passes, whose work does not grow with the overlap of neighbouring tiles
+// one launch while a tile's window fits RS_LDS_MAX with at least 8 rows: scales up to about 4 (tap tables of 5 to 17 columns); wider filters
+// take the two passes, whose work does not grow with the overlap of neighbouring tiles
+struct ResizePlan { int TH = 0, rows_cap = 0, seg_dw = 0; size_t lds = 0; };      // TH 0: two passes
+static ResizePlan resize_plan(int layout, int Hin, int Win, int Hout, int Wout, int kx, int ky) {
+  ResizePlan p;
+  if ((kx & 1) == 0 || kx < 5 || kx > 17) return p;
   const double sx = (double)Win / Wout, sy = (double)Hin / Hout;
   const int seg_dw = (((int)(63 * sx) + 2 + kx) * (layout == 0 ? 3 : 1) + 8 + 3) / 4;
   for (int TH = 16; TH >= 8; TH >>= 1) {
     const int rows_cap = (int)((TH - 1) * sy + 4 * std::max(sy, 1.0)) + 3;
     const size_t lds = ((size_t)rows_cap * (3 * RS_COLS + (layout == 0 ? 1 : 3) * seg_dw) + TH * ((ky + 3) & ~3)) * 4;
-    if ((kx & 1) == 0 || kx < 5 || kx > 17 || lds > RS_LDS_MAX) continue;
-#define LCC_RS(KX) case KX: launch_resize_tile<KX>(src, layout, T, Hin, Win, dst, Hout, Wout, xmin, xsize, wx, ymin, ysize, wy, ky, TH, rows_cap, seg_dw, lds, st); return 0
+    if (lds > RS_LDS_MAX) continue;
+    p.TH = TH; p.rows_cap = rows_cap; p.seg_dw = seg_dw; p.lds = lds;
+    break;
+  }
+  return p;
+}
+size_t resize_tmp_floats(int layout, int T, int Hin, int Win, int Hout, int Wout, int kx, int ky) {
+  if (T <= 0 || Hin <= 0 || Win <= 0 || Hout <= 0 || Wout <= 0 || kx <= 0 || ky <= 0 || resize_plan(layout, Hin, Win, Hout, Wout, kx, ky).TH > 0) return 0;
+  return (size_t)T * 3 * Hin * Wout;
+}
+int resize_bicubic_aa_u8(const uint8_t* src, int layout, int T, int Hin, int Win, uint8_t* dst, int Hout, int Wout,
+                         const int32_t* xmin, const int32_t* xsize, const float* wx, int kx, const int32_t* ymin,
+                         const int32_t* ysize, const float* wy, int ky, float* tmp, hipStream_t st) {
+  if (T <= 0 || Hin <= 0 || Win <= 0 || Hout <= 0 || Wout <= 0 || kx <= 0 || ky <= 0 || (layout != 0 && layout != 1)) return LCC_ERR_SHAPE;
+  const ResizePlan p = resize_plan(layout, Hin, Win, Hout, Wout, kx, ky);
+  if (p.TH > 0) {
+#define LCC_RS(KX) case KX: launch_resize_tile<KX>(src, layout, T, Hin, Win, dst, Hout, Wout, xmin, xsize, wx, ymin, ysize, wy, ky, p.TH, p.rows_cap, p.seg_dw, p.lds, st); return 0
     switch (kx) { LCC_RS(5); LCC_RS(7); LCC_RS(9); LCC_RS(11); LCC_RS(13); LCC_RS(15); LCC_RS(17); }
 #undef LCC_RS
   }

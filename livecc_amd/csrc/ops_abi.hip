@@ -84,6 +84,9 @@ extern "C" int lcc_patchify_norm_u8(const uint8_t* frames, int layout, int T, in
   if (!frames || !out || !mean255 || !std255) return fail(LCC_ERR_ARG, "lcc_patchify_norm_u8: null pointer");
   OP_RET(patchify_norm_u8(frames, layout, T, H, W, mean255, std255, (bf16_t*)out, ld, (hipStream_t)stream), "lcc_patchify_norm_u8");
 }
+extern "C" size_t lcc_resize_bicubic_aa_tmp_floats(int layout, int T, int Hin, int Win, int Hout, int Wout, int kx, int ky) {
+  return resize_tmp_floats(layout, T, Hin, Win, Hout, Wout, kx, ky);
+}
 extern "C" int lcc_resize_bicubic_aa_u8(const uint8_t* src, int layout, int T, int Hin, int Win, uint8_t* dst, int Hout, int Wout,
                                         const int32_t* xmin, const int32_t* xsize, const float* wx, int kx, const int32_t* ymin,
                                         const int32_t* ysize, const float* wy, int ky, float* tmp, void* stream) {

@@ -189,7 +189,8 @@ Tensor resize_bicubic_aa(const Tensor& frames, int64_t layout, int64_t Hout, int
   TORCH_CHECK(xmin.numel() == Wout && xsize.numel() == Wout && wx.numel() == kx * Wout && ymin.numel() == Hout && ysize.numel() == Hout && wy.numel() == ky * Hout,
               "resize_bicubic_aa: tap tables do not match the output size");
   Tensor out = at::empty({T, 3, Hout, Wout}, frames.options());
-  Tensor tmp = at::empty({T * 3 * Hin * Wout}, frames.options().dtype(at::kFloat));
+  const size_t between = lcc_resize_bicubic_aa_tmp_floats((int)layout, (int)T, (int)Hin, (int)Win, (int)Hout, (int)Wout, (int)kx, (int)ky);
+  Tensor tmp = at::empty({(int64_t)std::max<size_t>(between, 1)}, frames.options().dtype(at::kFloat));
   ok(lcc_resize_bicubic_aa_u8((const uint8_t*)frames.data_ptr(), (int)layout, (int)T, (int)Hin, (int)Win, (uint8_t*)out.data_ptr(), (int)Hout, (int)Wout,
                               (const int32_t*)xmin.data_ptr(), (const int32_t*)xsize.data_ptr(), (const float*)wx.data_ptr(), (int)kx,
                               (const int32_t*)ymin.data_ptr(), (const int32_t*)ysize.data_ptr(), (const float*)wy.data_ptr(), (int)ky,

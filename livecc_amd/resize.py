@@ -151,9 +151,10 @@ def resize_bicubic_aa(frames: torch.Tensor, height: int, width: int, layout: str
     if t is not None:
         return t(frames, 0 if layout == "THWC" else 1, int(height), int(width), xmin, xsize, wx, int(kx), ymin, ysize, wy, int(ky))
     out = torch.empty(T, 3, height, width, dtype=torch.uint8, device=dev)
-    tmp = torch.empty(T * 3 * Hin * width, dtype=torch.float32, device=dev)
+    lay = 0 if layout == "THWC" else 1
+    tmp = torch.empty(max(1, _lib.load().lcc_resize_bicubic_aa_tmp_floats(lay, T, Hin, Win, height, width, kx, ky)), dtype=torch.float32, device=dev)
     _lib.check(_lib.load().lcc_resize_bicubic_aa_u8(
-        frames.data_ptr(), 0 if layout == "THWC" else 1, T, Hin, Win, out.data_ptr(), height, width, xmin.data_ptr(), xsize.data_ptr(),
+        frames.data_ptr(), lay, T, Hin, Win, out.data_ptr(), height, width, xmin.data_ptr(), xsize.data_ptr(),
         wx.data_ptr(), kx, ymin.data_ptr(), ysize.data_ptr(), wy.data_ptr(), ky, tmp.data_ptr(),
         torch.cuda.current_stream(dev).cuda_stream), "lcc_resize_bicubic_aa_u8")
     return out

@@ -98,3 +98,18 @@ def test_resize_one_launch_at_tile_edges(dev, T, hi, wi, ho, wo, layout):
     src = tchw.permute(0, 2, 3, 1).contiguous() if layout == "THWC" else tchw
     got = R.resize_bicubic_aa(src.to(dev)[1:], ho, wo, layout).cpu()          # a view: its first byte may lie inside a dword
     assert torch.equal(got, O.resize_ref(tchw[1:].contiguous(), ho, wo))
+
+
+@pytest.mark.parametrize("use_op", [True, False])
+def test_a_resize_in_one_launch_allocates_its_result_only(dev, monkeypatch, use_op):
+    from livecc_amd import resize as R, torch_ops
+    if not use_op:
+        monkeypatch.setattr(torch_ops, "op", lambda name: None)
+    x = torch.zeros(4, 720, 1280, 3, dtype=torch.uint8, device=dev)
+    R.resize_bicubic_aa(x[:1], 392, 728)          # the tap tables
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    out = R.resize_bicubic_aa(x, 392, 728)
+    # torch's allocator hands a cached block out whole where less than 1 MB of it would be left; the fp32 rows between two passes would be 25 MB
+    assert torch.cuda.max_memory_allocated() - before <= out.numel() + (2 << 20)

@@ -86,3 +86,13 @@ def test_golden_fixture_pins_the_oracle():
     z = np.load(os.path.join(os.path.dirname(__file__), "golden", "resize_small.npz"))
     got = O.resize_ref(torch.from_numpy(z["frames"]), int(z["out_hw"][0]), int(z["out_hw"][1])).numpy()
     assert np.array_equal(got, z["resized"])
+
+
+@pytest.mark.parametrize("T,hi,wi,ho,wo,floats", [(2, 720, 1280, 392, 728, 0), (24, 1080, 1920, 280, 504, 0), (1, 1, 1, 1, 1, 0), (1, 97, 65, 33, 65, 0),
+                                                  (2, 101, 1000, 101, 200, 2 * 3 * 101 * 200), (1, 700, 65, 70, 65, 3 * 700 * 65)])
+def test_the_fp32_rows_between_the_passes_are_asked_for_only_where_there_are_two(built_lib, T, hi, wi, ho, wo, floats):
+    """Filters of up to 17 taps run both passes in one launch and need no intermediate; wider ones, or tiles too tall for LDS, need all of it."""
+    kx, ky = R.aa_bicubic_taps(wi, wo)[2].shape[1], R.aa_bicubic_taps(hi, ho)[2].shape[1]
+    for layout in (0, 1):
+        assert built_lib.lcc_resize_bicubic_aa_tmp_floats(layout, T, hi, wi, ho, wo, kx, ky) == floats
+    assert built_lib.lcc_resize_bicubic_aa_tmp_floats(0, 0, hi, wi, ho, wo, kx, ky) == 0
