@@ -117,9 +117,11 @@ LCC_DEVICE void rbf2(float& a, float& b) {
 }
 
 // activations, with HF's bf16 rounding points (inputs are already-rounded bf16 values held in fp32).  exp and the reciprocal are the
-// hardware units (v_exp_f32, v_rcp_f32), as few instructions around them as give the rounded double-precision result on EVERY finite bf16
-// input (all 65,280 were compared): they are what bounds the epilogues of the short products (ViT fc1: 37 us of 205 at 15,840 patches with
-// the error-corrected exponential and reciprocal this replaces, which also gave NaN below -52 / -88).
+// hardware units (v_exp_f32, v_rcp_f32), as few instructions around them as give the rounded double-precision result on every finite bf16
+// input whose result is at least 1e-36 in magnitude (all 65,280 inputs were compared; below, where v_rcp_f32's result is subnormal, nine
+// inputs of each function give zero: -53.5 to -51.5 and -91.5 to -87.5).  They are what bounds the epilogues of the short products (ViT fc1:
+// 37 us of 205 at 15,840 patches with the error-corrected exponential and reciprocal this replaces, which gave NaN below -52 / -88 and
+// above 1.4e38 / 2.3e38).
 constexpr float LOG2E = 1.4426950408889634f;
 // quick_gelu: HF activations.py QuickGELUActivation: input * sigmoid(1.702 * input) on bf16 tensors; two at a time.  The products are left
 // unrounded: the caller packs them.
