@@ -681,20 +681,10 @@ def test_decode_pipeline_v2_matches_the_round1_launch_sequence(dev, shape):
         assert worst <= 3e-2, f"v2 vs round-1 decode logits differ by {worst:.3g} of the logit scale"
 
 
-@pytest.mark.parametrize("hidden,n_streams,fp8", [(256, 3, False), (896, 8, False), (896, 8, True), (896, 9, False), (2304, 9, False), (2304, 16, False),
-                                                  (2304, 16, True), (2304, 17, False)])
-def test_decode_of_several_streams_matches_the_unfused_sequence(dev, hidden, n_streams, fp8):
-    """3 to 8 streams (16 above 2,048 channels) take the row-scaled products: RMSNorm's weight on the residual row where it is written, 1 / rms on the
-    finished sums; more streams keep the launch sequence with norm kernels.  Each against that sequence on the same weights, prompts of
-    different lengths and the same forced tokens: logits within 3 % of their scale (the bound of the one-stream comparison above: two bf16
-    pipelines that round at different points), and the launch counts say which of them ran."""
-    import dataclasses
+def _several_streams_against_the_unfused_sequence(dev, cfg, n_streams, fp8, scaled):
     from livecc_amd import _lib, ops
-    from livecc_amd.config import tiny
     from livecc_amd.engine import Sampling
     from livecc_amd.modeling import LiveCCForConditionalGeneration
-    heads = hidden // 128
-    cfg = dataclasses.replace(tiny(), hidden_size=hidden, intermediate_size=2 * hidden + 64, num_attention_heads=heads, num_key_value_heads=2 if heads % 2 == 0 else 1)
     lens = [5 + 37 * i % 150 for i in range(n_streams)]
     native = LiveCCForConditionalGeneration.from_config(cfg, dev, seed=5, llm_fp8=fp8, max_streams=n_streams, max_kv_len=256, max_new_rows=sum(lens),
                                                         max_patches=64, max_history=16)
@@ -720,13 +710,72 @@ def test_decode_of_several_streams_matches_the_unfused_sequence(dev, hidden, n_s
             _lib.check(lib.lcc_debug_set_decode_path(1), "set_decode_path")
 
     (got, n1), (ref, n0) = run(1), run(0)
-    scaled = n_streams <= (16 if hidden > 2048 else 8)
     assert n0 == 0 and n1 == (3 * (4 * cfg.num_hidden_layers + 1) if scaled else 0)
     for k in range(3):
         for b in range(n_streams):
             scale = ref[k, b].abs().max().item()
             err = (got[k, b] - ref[k, b]).abs().max().item()
             assert 0 < scale and err <= 3e-2 * scale, f"step {k} stream {b}: {err:.3g} of {scale:.3g}"
+
+
+@pytest.mark.parametrize("hidden,n_streams,fp8", [(256, 3, False), (896, 8, False), (896, 8, True), (896, 9, False), (2304, 9, False), (2304, 16, False),
+                                                  (2304, 16, True), (2304, 17, False)])
+def test_decode_of_several_streams_matches_the_unfused_sequence(dev, hidden, n_streams, fp8):
+    """3 to 8 streams (16 above 2,048 channels) of models of these sizes take the row-scaled products: RMSNorm's weight on the residual row where it is
+    written, 1 / rms on the finished sums; more streams keep the launch sequence with norm kernels.  Each against that sequence on the same weights,
+    prompts of different lengths and the same forced tokens: logits within 3 % of their scale (the bound of the one-stream comparison above: two
+    bf16 pipelines that round at different points), and the launch counts say which of them ran.  (Nine streams of 896 channels and 17 of 2,304 only
+    show that: both runs are that sequence, whose logits the oracle checks below.)"""
+    import dataclasses
+    from livecc_amd.config import tiny
+    heads = hidden // 128
+    cfg = dataclasses.replace(tiny(), hidden_size=hidden, intermediate_size=2 * hidden + 64, num_attention_heads=heads, num_key_value_heads=2 if heads % 2 == 0 else 1)
+    _several_streams_against_the_unfused_sequence(dev, cfg, n_streams, fp8, scaled=n_streams <= (16 if hidden > 2048 else 8))
+
+
+def _wide(hidden, inter, kv):
+    import dataclasses
+    from livecc_amd.config import tiny
+    return dataclasses.replace(tiny(), hidden_size=hidden, intermediate_size=inter, num_attention_heads=hidden // 128, num_key_value_heads=kv)
+
+
+# two layers of the 7B's sizes, and of 8,192 channels: 512 statistics a row, at nine rows and more of them than the four waves of a gate/up block fetch ahead
+@pytest.mark.parametrize("hidden,inter,kv,n_streams", [(3584, 18944, 4, 16), (8192, 8256, 8, 16)])
+def test_decode_of_several_streams_at_large_sizes_in_fp8(dev, hidden, inter, kv, n_streams):
+    """The comparison above."""
+    _several_streams_against_the_unfused_sequence(dev, _wide(hidden, inter, kv), n_streams, True, scaled=True)
+
+
+@pytest.mark.parametrize("shape,batches,scaled", [("small", (9, 17, 32), False), ((3584, 18944, 4), (3, 8, 16), True), ((8192, 2048, 8), (4, 16), True)])
+def test_decode_of_many_streams_matches_the_oracle(dev, shape, batches, scaled):
+    """Batches that keep the launch sequence with norm kernels, and the row-scaled products at the sizes of large models (16-wave residual blocks, which
+    are taken from 8,192 k on; 512 statistics a row): the logits of the prefill and three decode steps against HF in bf16 and fp32, teacher-forced
+    along the native tokens, with the bounds of the one-stream comparisons; of the large models the first, the middle and the last stream."""
+    from livecc_amd import ops
+    from livecc_amd.config import small
+    from livecc_amd.modeling import LiveCCForConditionalGeneration
+    from oracle import hf_oracle as O
+    cfg = small() if shape == "small" else _wide(*shape)
+    hf16, hf32 = (O.build_hf_model(cfg, dtype=t, seed=2, init_scale=1.0) for t in (torch.bfloat16, torch.float32))
+    native = LiveCCForConditionalGeneration.from_hf_model(hf16, cfg, dev, max_streams=max(batches), max_kv_len=128, max_new_rows=2048, max_patches=64, max_history=16)
+    rng = np.random.RandomState(11)
+    ids = [rng.randint(0, 2000, size=4 + 7 * i % 29) for i in range(max(batches))]
+    for n in batches:
+        ops.launch_counts(reset=True)
+        outs = native.generate_batch([dict(input_ids=torch.from_numpy(x)) for x in ids[:n]], repetition_penalty=1.05, max_new_tokens=4, force_length=True, output_logits=True)
+        assert ops.launch_counts(reset=True)["dgemv_v2"] == (3 * (4 * cfg.num_hidden_layers + 1) if scaled else 0)
+        for b, o in enumerate(outs):
+            if scaled and b not in (0, n // 2, n - 1):
+                continue
+            toks = o.sequences[0, len(ids[b]):].tolist()
+            r16, r32 = (O.OracleStream(m, cfg).turn(ids[b], None, None, max_new_tokens=4, repetition_penalty=1.05, teacher_tokens=toks) for m in (hf16, hf32))
+            for k in range(4):
+                ln, l16, l32 = o.logits[k].float().cpu().view(-1), r16["logits"][k].float().view(-1), r32["logits"][k].float().view(-1)
+                scale = l32.abs().max().item()
+                assert (ln - l16).abs().max().item() <= 6e-2 * scale, f"{n} streams, stream {b} step {k}"
+                assert (ln - l32).abs().max().item() <= 1.5 * (l16 - l32).abs().max().item() + (1e-3 + 2.0 ** -7) * scale, f"{n} streams, stream {b} step {k}"
+        for o in outs:
+            o.past_key_values.release()
 
 
 @pytest.mark.parametrize("n_streams,max_history,max_new", [(1, 16, 16), (5, 16, 9), (3, 4096, 40)])

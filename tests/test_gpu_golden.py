@@ -386,20 +386,23 @@ def test_livecc7b_oneshot480_against_the_committed_hf_logits(dev):
     assert st["decided_equal"] == st["decided"], st
 
 
-def test_livecc7b_batch_of_8_streams_against_the_committed_hf_logits(dev):
+@pytest.mark.parametrize("route", ["row_scaled", "norm_launches"])
+def test_livecc7b_batch_of_8_streams_against_the_committed_hf_logits(dev, route):
     """ONE GPU's share of BASELINE configs[2] at the REAL shapes (batched parity was at `small` / `tiny` only): 8 streams
     (the benchmark's seeds), the 6-frame turn + a 2-frame turn, ONE `generate_batch` call per turn -- batched vision tower over 34,944 /
     11,648 patches, packed prefill of 9,048 / 3,088 rows (the 256- and 192-row GEMM tiles, `attn_gqa32_kernel`), one weight pass per decode
-    step for the 8 streams (`gemv_skinny_kernel` + `attn_decode_fused_kernel`) -- against tests/golden/livecc7b_batch8.npz: HF run once per
+    step for the 8 streams (the row-scaled products that they take, and the `gemv_skinny_kernel` + `attn_decode_fused_kernel` sequence that
+    batches beyond 16 streams take) -- against tests/golden/livecc7b_batch8.npz: HF run once per
     stream (the reference has no batched path), bf16 free-running + fp32 teacher-forced (oracle/make_golden_7b_batch8.py).  Every stream
     follows its own HF tokens; per stream and step: |native - HF_bf16| at HF's top-64 ids <= 6e-2 x scale, rms(native - fp32) <= 1.25 x
     rms(HF_bf16 - fp32) over the 1,024 sample ids, the native path's own choice equal to HF's wherever HF's processed-score margin exceeds
     8 x its committed rms error."""
-    from livecc_amd import protocol
+    from livecc_amd import _lib, ops, protocol
     from livecc_amd.config import get_config
     from livecc_amd.modeling import LiveCCForConditionalGeneration
     from livecc_amd.weights import WeightArena
     from oracle import make_golden_7b_batch8 as B
+    lib = _lib.load()
     g = dict(np.load(B.PATH))
     seed0, n_streams, n_frames, H, W, n_new, seed_w = (int(x) for x in g["meta"])
     cfg = get_config("livecc-7b")
@@ -423,8 +426,15 @@ def test_livecc7b_batch_of_8_streams_against_the_committed_hf_logits(dev):
             fulls.append(full)
             rows.append([int(x) for x in g[f"s{s}_t{ti}_tokens"]])
             reqs.append(dict(input_ids=torch.from_numpy(full), frames=frames[s][a:b], frames_layout="TCHW", state=states[s]))
-        outs = native.generate_batch(reqs, repetition_penalty=B.PENALTY, max_new_tokens=n_new, force_length=True, output_logits=True,
-                                     teacher_tokens=rows)
+        lib.lcc_debug_set_decode_path(1 if route == "row_scaled" else 0)
+        ops.launch_counts(reset=True)
+        try:
+            outs = native.generate_batch(reqs, repetition_penalty=B.PENALTY, max_new_tokens=n_new, force_length=True, output_logits=True,
+                                         teacher_tokens=rows)
+        finally:
+            lib.lcc_debug_set_decode_path(1)
+        c = ops.launch_counts(reset=True)
+        assert (c["dgemv_v2"] > 0, c["attn_decode_fused"] > 0) == (route == "row_scaled", route != "row_scaled"), c
         for s, o in enumerate(outs):
             states[s] = o.past_key_values
             assert o.sequences[0, len(fulls[s]):].tolist() == rows[s]
@@ -450,7 +460,7 @@ def test_livecc7b_batch_of_8_streams_against_the_committed_hf_logits(dev):
     for x in states:
         x.release()
     ratios = np.asarray(ratios)
-    record("livecc7b_batch8_vs_committed_golden", st | dict(worst_rms_ratio=float(ratios.max()), mean_rms_ratio=float(ratios.mean()),
+    record(f"livecc7b_batch8_vs_committed_golden[{route}]", st | dict(worst_rms_ratio=float(ratios.max()), mean_rms_ratio=float(ratios.mean()),
                                                              rms_ratio_all_steps=float(np.sqrt((ratios ** 2).mean()))))
     assert st["steps"] == n_streams * 2 * n_new
     assert st["worst_rel_dlogit_top"] <= GROSS_MAX, st
