@@ -33,3 +33,10 @@ def test_rows_through_lds_are_ordered_between_lanes(name, store, load):
 def test_the_order_is_a_fence_on_both_sides_of_the_exchange():
     text = body(open(os.path.join(CSRC, "common.h")).read(), "wave_lds_order")
     assert re.search(r'fence\(__ATOMIC_ACQ_REL, "wavefront"\)', text) and "wave_barrier" in text
+
+
+def test_no_requested_residual_piece_is_left_unused():
+    """A row group that is skipped leaves its residual pieces in flight; the compiler then waits for all memory in every k-step of the next tile."""
+    text = body(open(os.path.join(CSRC, "gemm.hip")).read(), "tile_epilogue_wide")
+    skips = re.findall(r"if \((.*?>= M)\) break;", text)
+    assert skips and all(s.startswith("EPI != EPI_RESIDUAL && ") for s in skips)
