@@ -1448,7 +1448,12 @@ static int big_tile_rows(const GemmArgs& a, int S) {
   }
   if (s256 >= s192 && s256 >= s128 && s256 >= s128m && s256 >= s64) return 256;
   if (s192 >= s128 && s192 >= s128m && s192 >= s64) return 192;
-  if (s128 >= s128m && s128 >= s64) return 128;
+  // a last row tile that is half empty saves nothing while all blocks run at once beside full ones, and two 64-row tiles a unit hide each other's ends:
+  // at 129 to 192 rows [17920, 1536] 19.1 us against 23.0 with 128 x 256 tiles, [4608, 3584] in four splits 15.4 / 16.6, [3584, 3584] in six 13.3 / 14.2.
+  // Up to 24 steps a block: [3584, 18944] in six splits (49 steps) 51.7 / 44.4
+  const bool one_round = a.M > 128 && (long)((a.M + 127) / 128) * ((a.N + 255) / 256) * S <= 256 && a.K <= 64 * 24 * S;
+  const float s128_64 = one_round && !a.w_fp8 ? tile_score(a.M, a.N, S, 128, 256, 256, 0.85f, false) : s128;
+  if (s128 >= s128m && s128_64 >= s64) return 128;
   return s128m > s64 ? 129 : 0;
 }
 

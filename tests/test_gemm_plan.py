@@ -84,6 +84,14 @@ def test_prefill_attention_plan_at_the_engines_shapes(built_lib):
         plan([386], 6586, 28, 5)
 
 
+def test_short_products_of_129_to_192_rows_take_the_64_row_tiles(ops):
+    """One round of 128 x 256 tiles whose last row tile is at most half full, with few k-steps a block: two 64-row tiles a compute unit."""
+    assert [ops.gemm_plan(M, 17920, 1536, e)[0] for M in (129, 160, 192) for e in (ops.EPI_NONE, ops.EPI_SWIGLU)] == [64] * 6
+    assert [ops.gemm_plan(M, 17920, 1536, ops.EPI_SWIGLU)[0] for M in (193, 256)] == [128, 128]
+    assert [ops.gemm_plan(M, QKV, H, 0, 4)[0] for M in (150, 192)] == [64, 64]
+    assert ops.gemm_plan(137, H, I, 0, 6)[0] == 128
+
+
 def test_decode_attention_splits_over_streams(built_lib):
     """Key splits of the decode attention, as lcc_llm_decode asks for them: one stream as many as its tiles give (one tile up to 24 of them, two
     beyond, up to 64 splits, 128 from 16k keys on, none without a tile); batches stop at 768 blocks, two splits at least, so that 64 streams do not write and merge the
