@@ -1820,7 +1820,7 @@ static int gemv_rows_tiles(const GemmArgs& a, int S) {
   if (!a.w_packed || a.M <= 16) return 1;
   auto cost = [&](int nt) { return (float)(((long)(a.N / (nt * 16)) * S + 255) / 256) * ((float)nt + (float)a.M / 16.f); };
   if (a.N % 32 != 0) return 1;
-  const int nt = cost(2) < cost(1) ? 2 : 1;
+  const int nt = cost(2) < 0.97f * cost(1) ? 2 : 1;      // a tie (17 and 18 rows, two rounds for three): one tile 8.6 us, two 8.7 at [1536, 8960] in eight splits
   return a.N % 64 == 0 && cost(4) < 0.85f * cost(nt) ? 4 : nt;
 }
 template <int NTILE, int MODE>
