@@ -110,10 +110,10 @@ int lcc_debug_attn_decode_splits(int max_keys, int pairs);
 int lcc_debug_set_fused_tails(int on);
 /* decode launch sequence of the engine: 1 (default) = pipeline v2 where eligible (bf16 weights, the row-permuted decode copy
  * "llm.<i>.qkv_w_dec" of every q|k|v weight set): RMSNorm / bias + M-RoPE + KV append / residual add run inside the weight-streaming
- * GEMVs, 6 launches per layer, for decode batches of ONE or TWO streams (lcc_llm_decode: `n_streams <= 2`; measured: 640 vs 655 tokens/s
- * at four streams, so larger batches keep the round-1 sequence; the MR = 4 forms of the kernels are reachable only through the
- * lcc_dgemv_* operators below); bf16 weights, and since round 3 fp8 weights that carry the permuted decode copy + its scales;
- * 0 = the round-1 sequence of 9 launches per layer.  Merging the attention key splits inside the o_proj GEMV as well (5 launches) was
+ * GEMVs, 6 launches per layer: one or two streams normalise the rows in every block, 3 to 16 take row-scaled products
+ * (lcc_debug_decode_row_scaled; 3 to 8 at 2,048 hidden channels and below, fewer for very wide layers).  bf16 weights, and fp8 weights
+ * that carry the permuted decode copy + its scales; the forms of the kernels for 3 and 4 normalised rows are reachable only through the
+ * lcc_dgemv_* operators below.  0, and larger batches = the sequence of 9 launches per layer with separate norms.  Merging the attention key splits inside the o_proj GEMV as well (5 launches) was
  * measured slower: 4-wave attention blocks 10.0 us + o_proj 9.8 us vs 7.3 + 4.9 + 6.8 us. */
 int lcc_debug_set_decode_path(int path);
 /* 1: pipeline v2 launches down_proj of layer l and the q/k/v GEMV of layer l+1 as ONE chained launch (5 launches per layer; default 0:

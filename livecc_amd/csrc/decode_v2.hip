@@ -505,7 +505,7 @@ __global__ __launch_bounds__(512, 2) void dgemv_latent_q_kernel(DgArgs a, Latent
 // product (the other two quarters are not used) and every load still brings 1 KB.  Up to 8 activation rows, kept in LDS (requested ahead of
 // the weights, up to nine 16-byte pieces a thread, and stored while the first twelve weight loads of a wave are in flight).  Decode step of a 2B
 // model, one stream of 500 keys: 1.315 -> 1.216 ms; of a 2B layer-list model: latent 1.394 -> 1.266, with recurrence 1.605 -> 1.538.
-// activations; 15 KB of wave sums beside them.  Eight rows of 8,960 k fit (2B down: 12.8 us in 16-row blocks, 9.5 here)
+// LDS for the activations, beside 15 KB of wave sums.  Eight rows of 8,960 k fit (2B down: 12.8 us in 16-row blocks, 9.5 here)
 constexpr int ROWS8_LDS = 144 * 1024;
 LCC_DEVICE f32x4 shfl4(f32x4 v, int src) {
   return (f32x4){__shfl(v[0], src, 64), __shfl(v[1], src, 64), __shfl(v[2], src, 64), __shfl(v[3], src, 64)};

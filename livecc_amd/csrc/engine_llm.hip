@@ -1,6 +1,6 @@
 // LLM side of the engine: Qwen2VLTextModel.forward (HF modeling_qwen2_vl.py:762-844) + lm_head (1320-1323) + GenerationMixin._sample
 // (generation/utils.py:2783-2960) as launch sequences: lcc_llm_prefill (packed rows of several streams over their carried KV) and
-// lcc_llm_decode (n steps without a host round trip; decode pipeline v2 for 1-2 streams, the weight-streaming GEMV sequence up to 64).
+// lcc_llm_decode (n steps without a host round trip; decode pipeline v2 for 1 to 16 streams, the weight-streaming GEMV sequence up to 64).
 #include "engine_internal.h"
 
 // 1: decode pipeline v2 launches down_proj(l) + q/k/v(l+1) as ONE chained launch where both grids fit the chip at once (decode_v2.hip).
