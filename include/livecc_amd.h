@@ -103,8 +103,8 @@ int lcc_debug_attn_tile_rows(int n_q_heads, int n_kv_heads);
  * query heads per KV head).  Host logic only (no launch, no GPU). */
 int lcc_debug_attn_plan(const int32_t* n_new, int n_streams, int max_kv, int n_q_heads, int n_kv_heads, int cu_count, int32_t* tile_rows,
                         int32_t* splits);
-/* Key splits of one decode attention launch (lcc_llm_decode's own choice): longest cache incl. the new tokens, (stream, KV head) pairs. */
-int lcc_debug_attn_decode_splits(int max_keys, int pairs);
+/* Key splits of one decode attention launch (lcc_llm_decode's own choice) for streams of n_keys[b] keys incl. the call's new tokens. */
+int lcc_debug_attn_decode_splits(const int32_t* n_keys, int n_streams, int n_kv_heads);
 /* 1: on the batch-1 decode path the consumers of a split-K GEMV (bias + M-RoPE + KV append; residual add + RMSNorm) run as the
  * TAIL of that GEMV in its last-arriving block (agent-scope release/acquire); 0 (default, measured faster): separate kernels */
 int lcc_debug_set_fused_tails(int on);

@@ -1064,18 +1064,34 @@ int attn_prefill_bf16(const bf16_t* q, bf16_t* out, const int32_t* tile_stream, 
 // further pair is another trip, and the merge fetches up to 64 splits in one (decode step of one stream, 1 / 2 / 4 tiles a split: 2B at 500 keys
 // 1.168 / 1.177 / 1.216 ms, 7B at 2,000 keys 2.792 / 2.787 / 2.825).  64 splits at most up to 16k keys, 128 beyond: 9,000 keys 2.930 / 2.948 ms with
 // 64 / 128, 24,000 keys 3.136 / 3.067.
-// At most 768 blocks over all (stream, KV head) pairs: three waves a compute unit already pull what it can, and more only write and merge more partials.
-// Eight layers of a decode step with 512 / 768 / 1,024 blocks / no limit, us: 7B 16 streams of 8,000 keys 1,532 / 1,521 / 1,530 / 1,600, eight of 4,000
-// 1,091 / 1,101 / 1,092 / 1,115; 7B fp8, 32 streams of 4,000 1,720 / 1,714 / 1,718 / 1,846; 72B fp8, 64 streams of 2,000 3,449 / 3,449 / 3,449 / 3,747.
-// Over 120 points of 1 to 64 streams the mean distance from the best split count is 0.30 / 0.26 / 0.45 %.
+// Streams of one length: at most 768 blocks over all (stream, KV head) pairs: three waves a compute unit already pull what it can, and more only write and
+// merge more partials.  Eight layers of a decode step with 512 / 768 / 1,024 blocks / no limit, us: 7B 16 streams of 8,000 keys 1,532 / 1,521 / 1,530 /
+// 1,600, eight of 4,000 1,091 / 1,101 / 1,092 / 1,115; 7B fp8, 32 streams of 4,000 1,720 / 1,714 / 1,718 / 1,846; 72B fp8, 64 streams of 2,000 3,449 /
+// 3,449 / 3,449 / 3,747.  Over 120 points of 1 to 64 streams the mean distance from the best split count is 0.30 / 0.26 / 0.45 %.
+// Streams of unequal length: the split count is one for all, and a long cache beside short ones is a chain of tiles that nothing else hides.  More splits
+// while the longest chain (1.05 us a tile alone, 1.3 beside the other streams) is what the launch waits for and not the key tiles of all streams (16 KB
+// each at 6.5 TB/s), a block written and merged costing 2 ns (the figures without a limit above: 2.3 to 3, the merge's trips among them).
+// Decode step with the rule for one length / with this one / with 64 splits, us: 7B, 16 streams of 300 keys but one of 20,000 4,919 / 3,926 / 3,906;
+// eight of 500 but one of 12,000 3,471 / 3,286 / 3,289; twelve of 2,000 but one of 16,000 - / 3,938 / 3,938; fp8, 16 of 400 but one of 12,000 3,579 /
+// 3,025 / 3,022, 32 of 300 but one of 20,000 - / 4,948 / 4,943; four of 8,000 with twelve of 1,500 - / 4,115 / 4,301.
 // Tuning knobs LCC_ATTN_TPS, LCC_ATTN_MAXSPLIT.
-int attn_decode_splits(int max_keys, int pairs) {
+int attn_decode_splits(const int32_t* n_keys, int n_streams, int n_kv_heads) {
   static const int tps_env = [] { const char* v = getenv("LCC_ATTN_TPS"); return v ? std::max(1, atoi(v)) : 0; }();
   static const int maxsplit_env = [] { const char* v = getenv("LCC_ATTN_MAXSPLIT"); return v ? std::max(1, std::min(128, atoi(v))) : 0; }();
-  const int ntile = (max_keys + 31) / 32;
-  const int maxsplit = maxsplit_env ? maxsplit_env : std::min(ntile <= 512 ? 64 : 128, std::max(2, 768 / std::max(1, pairs)));
+  const int pairs = n_streams * n_kv_heads;
+  int ntile = 1;
+  long total = 0;
+  for (int b = 0; b < n_streams; ++b) { const int t = (n_keys[b] + 31) / 32; ntile = std::max(ntile, t); total += (long)t * n_kv_heads; }
   const int tps = tps_env ? tps_env : (ntile <= 24 ? 1 : 2);
-  const int n = std::max(1, std::min(maxsplit, (ntile + tps - 1) / tps)), per = (ntile + n - 1) / n;
+  const int most = std::min(maxsplit_env ? maxsplit_env : (ntile <= 512 ? 64 : 128), (ntile + tps - 1) / tps);
+  int n = most;
+  if (!maxsplit_env) {
+    n = std::min(most, std::max(2, 768 / pairs));
+    auto cost = [&](int k) { return std::max(1.3f * (float)((ntile + k - 1) / k), 0.0025f * (float)total) + 0.002f * (float)pairs * (float)k; };
+    if (total < (long)ntile * pairs)
+      for (int k = n + 1; k <= most; ++k) if (cost(k) < cost(n)) n = k;
+  }
+  const int per = (ntile + n - 1) / n;
   return (ntile + per - 1) / per;          // without those that would be left without a tile: 10 tiles in 8 splits are 5 of two
 }
 

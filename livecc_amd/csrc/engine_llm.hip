@@ -471,11 +471,13 @@ extern "C" int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots
   if (n_steps == 0) return 0;
   hipStream_t st = (hipStream_t)stream;
   int max_len = 0;
+  int32_t keys[LCC_MAX_DECODE_BATCH];
   for (int b = 0; b < n_streams; ++b) {
     const int s = slots[b];
     if (s < 0 || s >= e->lim.max_slots || !e->h_kv_base[s]) return fail(LCC_ERR_STATE, "slot %d not bound", s);
     if (e->h_kv_len[s] + n_steps > e->lim.max_kv_len) return fail(LCC_ERR_STATE, "slot %d: KV capacity exceeded", s);
-    max_len = std::max(max_len, e->h_kv_len[s] + n_steps);
+    keys[b] = e->h_kv_len[s] + n_steps;
+    max_len = std::max(max_len, keys[b]);
   }
   if (first_step_index + n_steps > e->lim.max_history) return fail(LCC_ERR_STATE, "history capacity %d exceeded", e->lim.max_history);
   MetaWriter mw; LCC_TRY(meta_begin(e, &mw));
@@ -489,7 +491,7 @@ extern "C" int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots
   }
   LlmBuffers bf; LCC_TRY(carve_llm(e, &bf));
   const int ntile = (max_len + 31) / 32;
-  const int nsplit = attn_decode_splits(max_len, n_streams * e->c.n_kv_heads);
+  const int nsplit = attn_decode_splits(keys, n_streams, e->c.n_kv_heads);
 
   LayerCtx cx{};
   // weight-streaming ("skinny") layer sequence for up to 64 streams: fp32 split-K slabs consumed by rope / add+norm kernels.  fp8 weights

@@ -153,7 +153,7 @@ int attn_prefill_bf16(const bf16_t* q, bf16_t* out, const int32_t* tile_stream, 
 // a stream that EOS froze on the device (`done`) has fewer keys than the host's count -- its step output is discarded anyway (the sampler
 // leaves a done slot untouched), and the rows past its length are finite bytes of the same arena.
 struct AttnDirect { const bf16_t* base[4]; int n[4]; int used = 0; };
-int attn_decode_splits(int max_keys, int pairs);      // key splits that attn_decode_bf16 is asked for: longest cache, (stream, KV head) pairs
+int attn_decode_splits(const int32_t* n_keys, int n_streams, int n_kv_heads);      // key splits that attn_decode_bf16 is asked for: cached keys of each stream
 int attn_decode_bf16(const bf16_t* q, bf16_t* out, const int32_t* slots, const int32_t* kv_len, bf16_t* const* kv_base,
                      KvLayout lay, int layer, int B, int n_q_heads, int nsplit, float* ws_o, float* ws_ml, hipStream_t st,
                      const AttnDirect* direct = nullptr);

@@ -29,9 +29,11 @@ extern "C" int lcc_debug_attn_tile_rows(int n_q_heads, int n_kv_heads) {   // ho
   const int G = n_q_heads / n_kv_heads;
   return (get_attn_variant() == 3 && G <= 8) ? attn32_tile_rows(G) : 32;
 }
-extern "C" int lcc_debug_attn_decode_splits(int max_keys, int pairs) {
-  if (max_keys < 1 || pairs < 1) return fail(LCC_ERR_ARG, "lcc_debug_attn_decode_splits: invalid arguments");
-  return attn_decode_splits(max_keys, pairs);
+extern "C" int lcc_debug_attn_decode_splits(const int32_t* n_keys, int n_streams, int n_kv_heads) {
+  if (!n_keys || n_streams < 1 || n_kv_heads < 1) return fail(LCC_ERR_ARG, "lcc_debug_attn_decode_splits: invalid arguments");
+  for (int b = 0; b < n_streams; ++b)
+    if (n_keys[b] < 1) return fail(LCC_ERR_ARG, "lcc_debug_attn_decode_splits: a stream without keys");
+  return attn_decode_splits(n_keys, n_streams, n_kv_heads);
 }
 extern "C" int lcc_debug_attn_plan(const int32_t* n_new, int n_streams, int max_kv, int n_q_heads, int n_kv_heads, int cu_count, int32_t* tile_rows,
                                    int32_t* splits) {   // host logic only: no launch

@@ -94,17 +94,28 @@ def test_short_products_of_129_to_192_rows_take_the_64_row_tiles(ops):
 
 def test_decode_attention_splits_over_streams(built_lib):
     """Key splits of the decode attention, as lcc_llm_decode asks for them: one stream as many as its tiles give (one tile up to 24 of them, two
-    beyond, up to 64 splits, 128 from 16k keys on, none without a tile); batches stop at 768 blocks, two splits at least, so that 64 streams do not write and merge the
-    partials of 64 splits each."""
-    f = built_lib.lcc_debug_attn_decode_splits
-    assert [f(k, 4) for k in (1, 32, 33, 500, 768, 769, 2000, 6500, 16384, 16385, 24000)] == [1, 1, 2, 16, 24, 13, 32, 51, 64, 103, 125]
-    assert [f(4000, 4 * n) for n in (1, 2, 3, 4, 8, 12, 16, 17, 32, 48, 64)] == [63, 63, 63, 42, 21, 16, 12, 11, 6, 4, 3]
-    assert f(6000, 8 * 64) == 2 and f(40, 8 * 64) == 2 and f(20, 8 * 64) == 1
-    for pairs in range(1, 513):
-        for keys in (1, 100, 700, 3000, 9000, 30000):
-            n, tiles = f(keys, pairs), (keys + 31) // 32
-            assert 1 <= n <= 128 and (n <= 2 or n * pairs <= 768) and (n - 1) * -(-tiles // n) < tiles          # no split without a tile
-    assert f(0, 1) < 0 and f(1, 0) < 0
+    beyond, up to 64 splits, 128 from 16k keys on, none without a tile); batches of one length stop at 768 blocks, two splits at least, so that 64 streams do
+    not write and merge the partials of 64 splits each; a long cache beside short ones keeps more, so that the launch does not wait for its chain of tiles."""
+    import numpy as np
+
+    def f(keys, heads=4):
+        a = np.asarray(keys, dtype=np.int32)
+        return built_lib.lcc_debug_attn_decode_splits(a.ctypes.data, len(a), heads)
+
+    assert [f([k]) for k in (1, 32, 33, 500, 768, 769, 2000, 6500, 16384, 16385, 24000)] == [1, 1, 2, 16, 24, 13, 32, 51, 64, 103, 125]
+    assert [f([4000] * n) for n in (1, 2, 3, 4, 8, 12, 16, 17, 32, 48, 64)] == [63, 63, 63, 42, 21, 16, 12, 11, 6, 4, 3]
+    assert f([6000] * 64, 8) == 2 and f([40] * 64, 8) == 2 and f([20] * 64, 8) == 1
+    for heads in (2, 4, 8):
+        for streams in range(1, 65):
+            for k in (1, 100, 700, 3000, 9000, 30000):
+                n, tiles = f([k] * streams, heads), (k + 31) // 32
+                assert 1 <= n <= 128 and (n <= 2 or n * streams * heads <= 768) and (n - 1) * -(-tiles // n) < tiles          # no split without a tile
+    # one long cache: its chain is a few tiles a split, whatever its place; more short ones beside it make a split dearer, never fewer splits than one length has
+    for streams, most in ((8, 12), (16, 16), (64, 32)):
+        mixed = [f(([500] * i + [20000] + [500] * (streams - 1 - i))) for i in (0, streams // 2, streams - 1)]
+        assert len(set(mixed)) == 1 and f([20000] * streams) <= mixed[0] <= 128 and -(-625 // mixed[0]) <= most
+    assert f([6000] * 7 + [5000]) == f([6000] * 8) < f([6000, 6000] + [1000] * 6)
+    assert f([]) < 0 and f([0]) < 0 and f([5, 0]) < 0 and f([5], 0) < 0 and built_lib.lcc_debug_attn_decode_splits(None, 1, 4) < 0
 
 
 @pytest.mark.parametrize("preset,fp8,last", [("livecc-7b", 0, 16), ("livecc-7b", 1, 16), ("qwen2vl-2b", 0, 8), ("qwen2vl-2b", 1, 8), ("qwen2vl-72b", 0, 4), ("qwen2vl-72b", 1, 9)])
