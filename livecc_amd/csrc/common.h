@@ -57,6 +57,12 @@ LCC_DEVICE void glds16(const void* gsrc, unsigned lds_dst) {
   asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" LCC_GLDS_POLICY "\n\ts_mov_b32 m0, %0"
                : "=&s"(keep) : "v"(gsrc), "s"(__builtin_amdgcn_readfirstlane(lds_dst)) : "memory");   // readfirstlane: free when provably uniform
 }
+// the same from a base that is uniform in the wave and a byte offset per lane
+LCC_DEVICE void glds16_base(const void* base, unsigned off, unsigned lds_dst) {
+  unsigned keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" LCC_GLDS_POLICY "\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "v"(off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(lds_dst)) : "memory");
+}
 // Make the compiler wait HERE for a plain global load it is tracking (it must insert its own s_waitcnt in front of a statement that reads
 // the registers).  Needed wherever plain loads are followed by glds16() pieces: a vmcnt(N) the compiler places later -- at the first use
 // of the value, possibly inside the ring loop -- would also drain the LDS-DMAs it cannot see (vmcnt retires in order).

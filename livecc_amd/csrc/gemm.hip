@@ -3,9 +3,11 @@
 // W keeps the nn.Linear layout [N,K] (K contiguous) so that both MFMA operands are read as 8 contiguous
 // bf16 (16 bytes) per lane.  fp32 accumulation, one rounding to bf16 at the points where HF rounds.
 //
-//  * gemm_big_kernel     : M >= 17, packed W, K % 64 == 0 (LLM prefill, ViT).  MFMA-bound.  8 waves, BM x 256 x 64 tile
-//                          (BM 256 / 192 / 128), LDS-DMA for both operands, optional fp8-e4m3 W converted after the LDS read.
-//  * gemm_vh_kernel      : the same pipeline over row tiles of 256 / 272 / 288 rows (no ragged last row tile; round 5).
+//  * gemm_walk_kernel    : M >= 17, packed W, K % 64 == 0 (LLM prefill, ViT).  MFMA-bound.  8 waves, BM x 256 x 64 tile
+//                          (BM 256 / 192 / 128), LDS-DMA for both operands; one block a compute unit, the DMA ring runs on from tile to tile.
+//  * gemm_big_kernel     : the same tiles one a block: fp8-e4m3 W converted after the LDS read, and the vision q|k|v epilogues.
+//  * gemm_walk_vh_kernel : the walk over row tiles of 256 / 272 / 288 rows (no ragged last row tile).
+//  * gemm_vh_kernel      : row tiles of 128 / 144 rows, split-K slabs of one streaming chunk.
 //  * gemm_tall_kernel    : one block row covers all of M (256 < M <= 448: one streaming chunk's gate/up).
 //  * gemm_mid_kernel     : shapes with few 256-column tiles.  64x128x64 (128x128x64) tile, 8 waves, 6- (4-) stage LDS-DMA ring.
 //  * gemm_glds_kernel /   : row-major W, K % 64 != 0.  64x128x64 (128x128x64) tile, 4 waves,
@@ -128,18 +130,27 @@ LCC_DEVICE void tile_epilogue(const f32x4 (&acc)[AM][AN], int mbase, int nbase, 
 // The epilogue is a large part of a short product.  15840 x 5120 with K = 64, plain -> here: bias 55 -> 38 us, quick GELU 71 -> 57 (with the
 // shorter activation), residual 130 -> 77; 15840 x 1280 with residual 29 -> 20.  SwiGLU (half the bytes, bound by its arithmetic) measured
 // 44.4 / 44.8 and keeps the plain form.
-// Needs C and the residual in rows of 16-byte pieces (wide_rows).
+// Needs C and the residual in rows of 16-byte pieces, and a bias that scalar loads can read (wide_rows).
 template <int EPI>
-LCC_DEVICE bool wide_rows(const bf16_t* C, int ldc, const bf16_t* residual, int ldr) {
+LCC_DEVICE bool wide_rows(const bf16_t* C, int ldc, const bf16_t* bias, const bf16_t* residual, int ldr) {
   if (EPI == EPI_PARTIAL || EPI == EPI_SWIGLU) return false;
-  return (ldc & 7) == 0 && ((uintptr_t)C & 15) == 0 && (EPI != EPI_RESIDUAL || ((ldr & 7) == 0 && ((uintptr_t)residual & 15) == 0));
+  return (ldc & 7) == 0 && ((uintptr_t)bias & 3) == 0 && ((uintptr_t)C & 15) == 0 && (EPI != EPI_RESIDUAL || ((ldr & 7) == 0 && ((uintptr_t)residual & 15) == 0));
 }
-template <int EPI, int MT, int NT>
+// Four bf16 bias values of columns n .. n + 15 a lane group g owns (n uniform in the wave): through the scalar unit, which has a counter of its own --
+// a vector load here would also wait for the LDS-DMA pieces of a walking kernel's next tile.
+LCC_DEVICE u32x2 bias_of_group(const bf16_t* bias, int n, int g) {
+  typedef const __attribute__((address_space(4))) unsigned* sptr;
+  const sptr p = (sptr)(uintptr_t)(bias + __builtin_amdgcn_readfirstlane(n));
+  const unsigned x0 = p[0], y0 = p[1], x1 = p[2], y1 = p[3], x2 = p[4], y2 = p[5], x3 = p[6], y3 = p[7];
+  const bool odd = (g & 1) != 0, high = (g & 2) != 0;
+  return (u32x2){high ? (odd ? x3 : x2) : (odd ? x1 : x0), high ? (odd ? y3 : y2) : (odd ? y1 : y0)};
+}
+template <int EPI, int MT, int NT, int GRT = 4>                    // GRT: row tiles of a group (lds: GRT x 16 x NT x 32 bytes)
 LCC_DEVICE void tile_epilogue_wide(const f32x4 (&acc)[MT][NT], int mbase, int nbase, int lane, const bf16_t* __restrict__ bias,
                                    const bf16_t* __restrict__ residual, int ldr, bf16_t* __restrict__ C, int ldc, int M, int N,
                                    const float* __restrict__ wscale, unsigned char* lds) {
   constexpr int RC = NT * 2, RPS = 64 / RC, RB = RC * 16;          // 16-byte chunks of a row; rows of a store; row bytes
-  constexpr int GR = MT < 4 ? MT : 4;                              // row tiles of a group
+  constexpr int GR = MT < GRT ? MT : GRT;                          // row tiles of a group
   const int li = lane & 15, g = lane >> 4;
   auto swz = [](int r) { return NT == 4 ? (r >> 1) & 7 : (r >> 2) & 3; };
   f32x4 sc[NT];
@@ -154,7 +165,7 @@ LCC_DEVICE void tile_epilogue_wide(const f32x4 (&acc)[MT][NT], int mbase, int nb
   for (int j = 0; j < NT; ++j) bv[j] = (u32x2){0u, 0u};
   if (bias != nullptr) {
 #pragma unroll
-    for (int j = 0; j < NT; ++j) bv[j] = ld8(bias + min(nbase + j * 16 + g * 4, N - 4));
+    for (int j = 0; j < NT; ++j) bv[j] = bias_of_group(bias, min(nbase + j * 16, N - 16), g);
   }
   constexpr int NS = GR * 16 / RPS;                                // stores of a group
   const int sr = lane / RC, schk = lane & (RC - 1), scol = nbase + schk * 8;          // this lane's row and chunk of a store
@@ -206,11 +217,12 @@ LCC_DEVICE void tile_epilogue_wide(const f32x4 (&acc)[MT][NT], int mbase, int nb
   }
 }
 
-// fp32 slabs the same way: 32 rows of 256 bytes at a time (lds: 8 KB, wave-private)
-template <int MT, int NT>
+// fp32 slabs the same way: GRT x 16 rows of NTG x 64 bytes at a time (lds: GRT x NTG KB, wave-private)
+template <int MT, int NT, int GRT = 2, int NTG = NT>
 LCC_DEVICE void tile_slab_wide(const f32x4 (&acc)[MT][NT], int mbase, int nbase, int lane, int M, int N, float* __restrict__ partial,
                                const float* __restrict__ wscale, unsigned char* lds) {
-  static_assert(NT == 4, "64 columns a wave");
+  static_assert(NT == 4 && (NTG == 4 || NTG == 2), "64 columns a wave");
+  constexpr int RC = NTG * 4, RPS = 64 / RC, RB = RC * 16;         // 16-byte chunks of a row; rows of a store; row bytes
   const int li = lane & 15, g = lane >> 4;
   f32x4 sc[NT];
 #pragma unroll
@@ -219,26 +231,31 @@ LCC_DEVICE void tile_slab_wide(const f32x4 (&acc)[MT][NT], int mbase, int nbase,
 #pragma unroll
     for (int j = 0; j < NT; ++j) sc[j] = *reinterpret_cast<const f32x4*>(wscale + min(nbase + j * 16 + g * 4, N - 4));
   }
-  const int sr = lane >> 4, schk = lane & 15, scol = nbase + schk * 4;
-  float* out = partial + (size_t)blockIdx.y * M * N + scol;
+  auto swz = [](int r) { return NTG == 4 ? r & 15 : (r >> 1) & 7; };
+  const int sr = lane / RC, schk = lane & (RC - 1);
 #pragma unroll
-  for (int i0 = 0; i0 < MT; i0 += 2) {
+  for (int i0 = 0; i0 < MT; i0 += GRT) {
     if (mbase + i0 * 16 >= M) break;          // 17 rows of a 128-row tile: one group in four (fp8 steps of 17 to 64 streams)
-    wave_lds_order();
 #pragma unroll
-    for (int ii = 0; ii < 2; ++ii) {
-      if (i0 + ii >= MT) continue;
-      const int r = ii * 16 + li;
+    for (int j0 = 0; j0 < NT; j0 += NTG) {
+      const int scol = nbase + j0 * 16 + schk * 4;
+      float* out = partial + (size_t)blockIdx.y * M * N + scol;
+      wave_lds_order();
 #pragma unroll
-      for (int j = 0; j < NT; ++j) *reinterpret_cast<f32x4*>(lds + r * 256 + (((j * 4 + g) ^ (r & 15)) * 16)) = acc[i0 + ii][j] * sc[j];
-    }
-    wave_lds_order();
+      for (int ii = 0; ii < GRT; ++ii) {
+        if (i0 + ii >= MT) continue;
+        const int r = ii * 16 + li;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      if (i0 * 16 + q * 4 >= MT * 16) continue;
-      const int r = q * 4 + sr, m = mbase + i0 * 16 + r;
-      const f32x4 v = *reinterpret_cast<const f32x4*>(lds + r * 256 + ((schk ^ (r & 15)) * 16));
-      if (m < M && scol < N) *reinterpret_cast<f32x4*>(out + (size_t)m * N) = v;
+        for (int j = 0; j < NTG; ++j) *reinterpret_cast<f32x4*>(lds + r * RB + (((j * 4 + g) ^ swz(r)) * 16)) = acc[i0 + ii][j0 + j] * sc[j0 + j];
+      }
+      wave_lds_order();
+#pragma unroll
+      for (int q = 0; q < GRT * 16 / RPS; ++q) {
+        if (i0 * 16 + q * RPS >= MT * 16) continue;
+        const int r = q * RPS + sr, m = mbase + i0 * 16 + r;
+        const f32x4 v = *reinterpret_cast<const f32x4*>(lds + r * RB + ((schk ^ swz(r)) * 16));
+        if (m < M && scol < N) *reinterpret_cast<f32x4*>(out + (size_t)m * N) = v;
+      }
     }
   }
 }
@@ -687,7 +704,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(
   }
   if (kt < nkt) mul(f0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the clamped copies
-  if (wide_rows<EPI>(C, ldc, residual, ldr)) {
+  if (wide_rows<EPI>(C, ldc, bias, residual, ldr)) {
     __builtin_amdgcn_s_barrier();          // every wave is done with the stages, and its DMA pieces have landed
     tile_epilogue_wide<EPI, MT, NT>(acc, m0 + wm * (BM / 2), n0 + wn * 32, lane, bias, residual, ldr, C, ldc, M, N, wscale,
                                     reinterpret_cast<unsigned char*>(dsmem) + wave * 4096);
@@ -890,7 +907,7 @@ LCC_DEVICE void gemm_big_body(
   } else if constexpr (EPI == EPI_PARTIAL) {
     __builtin_amdgcn_s_barrier();          // every wave is done with the stages, and its DMA pieces have landed
     tile_slab_wide<MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, lane, M, N, partial, wscale, reinterpret_cast<unsigned char*>(dsmem) + wave * 8192);
-  } else if (wide_rows<EPI>(C, ldc, residual, ldr)) {
+  } else if (wide_rows<EPI>(C, ldc, bias, residual, ldr)) {
     __builtin_amdgcn_s_barrier();          // every wave is done with the stages, and its DMA pieces have landed
     tile_epilogue_wide<EPI, MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, lane, bias, residual, ldr, C, ldc, M, N, wscale,
                                     reinterpret_cast<unsigned char*>(dsmem) + wave * 8192);
@@ -941,7 +958,158 @@ __global__ __launch_bounds__(512) void gemm_big_kernel(
 }
 
 // ------------------------------------------------------------------------------------------------
-// tiled GEMM v6 (round 5): the pipeline of gemm_big_kernel<256> over row tiles of VARIABLE height (16, 17 or 18 row fragments = 256 /
+// the same tiles, walked: one block a compute unit goes through its tiles with the DMA ring running on from tile to tile
+// ------------------------------------------------------------------------------------------------
+// What bounds a short product (the vision tower's K = 1280 is 20 k-steps of 1.3 us) beside the MFMAs and the ring is what lies between two
+// tiles of a compute unit: the last block's stores, a dispatch, addresses, and the first DMA's round trip, with nothing else resident (the
+// ring takes the LDS).  Here the pieces that gemm_big_body issues behind its last k-steps for nobody are the next tile's first ones, the epilogue
+// runs in LDS of its own behind the stages while they land, and its stores drain under the next tile's first step (vmcnt retires in order: the
+// step waits for the pieces and lets the younger stores be, if all of them were issued -- inner tiles).
+// Measured (us, gemm_big_kernel -> here): vision fc1 of 15,840 rows 200 -> 194, fc2 and proj with residual 284 -> 274 together; 4096 x 37888, K 3584
+// with SwiGLU 903 -> 862; 4096 x 18944 fp32, K 3584 473 -> 454.  What is left is the matrix pipe at the clock that the chip holds under it.
+// Bits as gemm_big_kernel (same k order per output).  bf16 weights; every epilogue but the vision q|k|v ones, whose rotation tables need
+// the stages.  Grid: at most 256 blocks over all splits (one a compute unit), or the cap.
+template <int BM, int EPI>
+__global__ __launch_bounds__(512) void gemm_walk_kernel(
+    const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
+    const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
+    bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n,
+    float* __restrict__ partial, int kt_per_split, const float* __restrict__ wscale, int raster) {
+  constexpr int BN = 256, BK = 64, NSTAGE = BM >= 192 ? 2 : 3;
+  constexpr int WM = BM / 2, MT = WM / 16, NT = 4;
+  constexpr int A_UNITS = BM * 8, STAGE = A_UNITS + 2048;        // 16-byte units: activations, then 32 weight sub-tiles
+  constexpr int APW = BM / 64, BPW = 4, G = APW + BPW;           // DMA pieces of a wave per k-tile
+  constexpr int EGR = BM >= 192 && EPI != EPI_GELU_ERF ? 2 : 1;  // row tiles of an epilogue group: 4 / 2 KB of LDS a wave (the erf: registers)
+  constexpr int NSTORE = EPI == EPI_PARTIAL ? MT * 4 : MT * 2;   // stores of a wave in the epilogue of an inner tile
+  extern __shared__ __attribute__((aligned(16))) u32x4 dsmem[];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 2, wn = wave & 3;
+  const int li = lane & 15, g = lane >> 4;
+  const int K32 = K >> 5, nfrag = N >> 4;
+  const int nblk = tiles_m * tiles_n, step = gridDim.x;
+  const int nkt_all = K / BK;
+  const int kt0 = (EPI == EPI_PARTIAL) ? blockIdx.y * kt_per_split : 0;
+  const int nkt = (EPI == EPI_PARTIAL) ? min(nkt_all, kt0 + kt_per_split) : nkt_all;
+
+  auto tile_of = [&](int bid, int& m0, int& n0) {     // tile order: see gemm_big_kernel
+    const int q = nblk >> 3, r = nblk & 7, xcd = bid & 7, idx = bid >> 3;
+    bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
+    int tn, tm;
+    if (raster > 0) {
+      const int band = bid / (raster * tiles_m), rem = bid - band * raster * tiles_m;
+      const int bw = min(raster, tiles_n - band * raster);
+      tm = rem / bw;
+      tn = band * raster + (rem - tm * bw);
+    } else {
+      tn = bid / tiles_m;
+      tm = bid - tn * tiles_m;
+    }
+    m0 = tm * BM; n0 = tn * BN;
+  };
+  // the DMA's tile: the one being multiplied, or the next one already.  Scalar bases, a 32-bit offset per lane and piece inside the tile.
+  unsigned aoffs[APW];
+  const bf16_t *abase, *bbase[BPW / 2];
+  int dvb = blockIdx.x, dkt = kt0;
+  auto point = [&] {
+    int m0, n0;
+    tile_of(dvb, m0, n0);
+    m0 = __builtin_amdgcn_readfirstlane(m0); n0 = __builtin_amdgcn_readfirstlane(n0);
+    abase = A + (size_t)m0 * lda;
+#pragma unroll
+    for (int q = 0; q < BPW / 2; ++q) bbase[q] = W + (size_t)min((n0 >> 4) + wave * (BPW / 2) + q, nfrag - 1) * K32 * 512;
+#pragma unroll
+    for (int q = 0; q < APW; ++q)
+      aoffs[q] = (unsigned)min((wave * APW + q) * 8 + (lane >> 3), M - 1 - m0) * (unsigned)(lda * 2) + (((lane & 7) ^ (lane >> 3)) << 4);
+  };
+  auto piece = [&](int t, unsigned base) {            // base: LDS byte address of the stage
+    if (t < APW) glds16_base(abase + dkt * BK, aoffs[t < APW ? t : 0], base + (wave * APW + t) * 1024u);
+    else glds16_base(bbase[t >= APW ? (t - APW) >> 1 : 0] + (size_t)dkt * 1024 + ((t - APW) & 1) * 512, lane * 16u, base + (A_UNITS + (wave * BPW + (t - APW)) * 64) * 16u);
+  };
+  auto advance = [&] {                                // behind the last tile: the last k-tile again, into a stage that nobody reads any more
+    if (++dkt < nkt) return;
+    if (dvb + step < nblk) { dvb += step; dkt = kt0; point(); }
+    else dkt = nkt - 1;
+  };
+  const unsigned lds0 = lds_addr(dsmem);
+  unsigned char* const elds = reinterpret_cast<unsigned char*>(dsmem + NSTAGE * STAGE) + wave * (EGR * 2048);
+  static_assert(NSTAGE * STAGE * 16 + 8 * EGR * 2048 <= 163840, "LDS of a compute unit");
+
+  point();
+  if (kt0 < nkt) {
+#pragma unroll
+    for (int p = 0; p < NSTAGE - 1; ++p) {
+#pragma unroll
+      for (int t = 0; t < G; ++t) piece(t, lds0 + (unsigned)(p * STAGE) * 16u);
+      advance();
+    }
+  }
+  int aoff[2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) aoff[kk] = (wm * WM + li) * 8 + ((kk * 4 + g) ^ (li & 7));
+  const int boff = A_UNITS + (wn * NT * 2) * 64 + lane;
+  int st = 0;                      // stage of the k-tile that is multiplied
+  bool all_stored = false;         // the last epilogue issued NSTORE stores in this wave
+  for (int vb = blockIdx.x; vb < nblk; vb += step) {
+    int m0, n0;
+    tile_of(vb, m0, n0);
+    const bool wave_has_rows = m0 + wm * WM < M;
+    f32x4 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    for (int kt = kt0; kt < nkt; ++kt) {
+      // this wave's pieces of tile kt have landed; younger: the pieces of NSTAGE - 2 tiles, and behind a tile's end its stores
+      if (all_stored && kt - kt0 < NSTAGE - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G * (NSTAGE - 2) + NSTORE) : "memory");
+      else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G * (NSTAGE - 2)) : "memory");
+      __builtin_amdgcn_s_barrier();   // tile kt complete in LDS; every wave is done reading the stage that is filled now
+      const u32x4* s = dsmem + st * STAGE;
+      const unsigned dma_base = lds0 + (unsigned)((st == 0 ? NSTAGE - 1 : st - 1) * STAGE) * 16u;
+      st = st == NSTAGE - 1 ? 0 : st + 1;
+      if (!wave_has_rows) {           // ragged last row tile: feed the ring only
+#pragma unroll
+        for (int t = 0; t < G; ++t) piece(t, dma_base);
+      } else {                        // fragment reads ahead of the MFMAs, a piece between two row tiles: gemm_big_body's order
+        bf16x8 fb[2][NT], fa[3];
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+          for (int j = 0; j < NT; ++j) fb[kk][j] = as_bf16x8(s[boff + (j * 2 + kk) * 64]);
+        fa[0] = as_bf16x8(s[aoff[0]]);
+        fa[1] = as_bf16x8(s[aoff[0] + 128]);
+#pragma unroll
+        for (int t = 0; t < 2 * MT; ++t) {
+          if (t + 2 < 2 * MT) fa[(t + 2) % 3] = as_bf16x8(s[aoff[(t + 2) / MT] + ((t + 2) % MT) * 128]);
+#pragma unroll
+          for (int j = 0; j < NT; ++j) acc[t % MT][j] = mfma16(fb[t / MT][j], fa[t % 3], acc[t % MT][j]);
+          if (t < G) piece(t, dma_base);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x100, 2 * NT + 2, 0);
+#pragma unroll
+        for (int t = 0; t < 2 * MT; ++t) {
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, NT, 0);
+          if (t < G) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+        }
+      }
+      advance();
+    }
+    int l = lane;          // opaque: the epilogue's addresses are formed here and not kept in registers through the k-loop
+    asm volatile("" : "+v"(l));
+    if constexpr (EPI == EPI_PARTIAL) {
+      tile_slab_wide<MT, NT, 1, EGR * 2>(acc, m0 + wm * WM, n0 + wn * 64, l, M, N, partial, wscale, elds);
+    } else if (wide_rows<EPI>(C, ldc, bias, residual, ldr)) {
+      tile_epilogue_wide<EPI, MT, NT, EGR>(acc, m0 + wm * WM, n0 + wn * 64, l, bias, residual, ldr, C, ldc, M, N, wscale, elds);
+    } else tile_epilogue<EPI, MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, (n0 + wn * 64) / 2, l & 15, l >> 4, bias, residual, ldr, C, ldc, M, N, partial, wscale);
+    all_stored = m0 + BM <= M && n0 + BN <= N;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the copies behind the last tile: this block's LDS until they have landed
+}
+
+// ------------------------------------------------------------------------------------------------
+// tiled GEMM v6: the pipeline of gemm_big_kernel<256> over row tiles of VARIABLE height (16, 17 or 18 row fragments = 256 /
 // 272 / 288 rows x 256 columns)
 // ------------------------------------------------------------------------------------------------
 // Why.  M is whatever the turn packs: 8 co-scheduled streaming chunks are 8 x 386 = 3088 rows = 12 x 256 + 16, so the 13th row tile of
@@ -960,25 +1128,172 @@ __global__ __launch_bounds__(512) void gemm_big_kernel(
 //     spread one per row-tile step behind the barrier (gemm_big_kernel's SCHED 6).
 // Accumulation order per output element = gemm_big_kernel's (k-step 0, then 1, tile after tile): bit-identical outputs.
 // Requires packed bf16 W, K % 64 == 0, F >= 16, F <= 18 * floor(F / 16).
-// SMALL = 1 (round 5): the same kernel over row tiles of 8 or 9 fragments (128 / 144 rows) for the split-K projections of ONE streaming
+// The small class (gemm_vh_kernel): the same pipeline over row tiles of 8 or 9 fragments (128 / 144 rows) for the split-K projections of ONE streaming
 // chunk (M = 386 = 25 fragments: 3 row tiles of 9 + 8 + 8 instead of gemm_big_kernel<128>'s 4, whose fourth holds 2 rows): an M-wave
 // multiplies 4 or 5 row fragments, 2 activation pieces per wave + the extra slot (rows 128-143, waves 0-1), a ring of THREE 51,200-B stages
 // (one more tile in flight: at 32-40 MFMAs per wave and k-tile a single stage of look-ahead left the DMA round trip exposed: 104 vs 72 us).
-template <int EPI, int SMALL>
+// One kernel for the big class, walked (gemm_walk_kernel: the ring runs on from tile to tile, the epilogue has LDS of its own), one tile a block for
+// the small one (its three stages leave no room for an epilogue, and its launches are one round).
+template <int EPI>
+__global__ __launch_bounds__(512) void gemm_walk_vh_kernel(
+    const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
+    const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
+    bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n,
+    float* __restrict__ partial, int kt_per_split, int raster) {
+  constexpr int BN = 256, BK = 64, NT = 4, MTX = 9, MTL = 8;     // row fragments of an M-wave: MTL or MTX
+  constexpr int APW = 4, NSLOT = APW + 5, AROWS = 288;           // 8-row activation pieces per wave below row 256, the slot above, weights
+  constexpr int A_UNITS = AROWS * 8, STAGE = A_UNITS + 2048;     // 69,632 B
+  constexpr unsigned SCRATCH = 2u * STAGE * 16u;                 // 1 KB: where a slot without rows lands
+  constexpr int NSTORE = EPI == EPI_PARTIAL ? MTL * 4 : MTL * 2;
+  static_assert(SCRATCH + 1024 + 8 * 2048 <= 163840, "LDS of a compute unit");
+  extern __shared__ __attribute__((aligned(16))) u32x4 dsmem[];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 2, wn = wave & 3;
+  const int li = lane & 15, g = lane >> 4;
+  const int K32 = K >> 5, nfrag = N >> 4;
+  const int nblk = tiles_m * tiles_n, step = gridDim.x;
+  const int F = (M + 15) >> 4, fbase = F / tiles_m, frem = F - fbase * tiles_m;
+  const int nkt_all = K / BK;
+  const int kt0 = (EPI == EPI_PARTIAL) ? blockIdx.y * kt_per_split : 0;
+  const int nkt = (EPI == EPI_PARTIAL) ? min(nkt_all, kt0 + kt_per_split) : nkt_all;
+
+  auto tile_of = [&](int bid, int& m0, int& n0, int& f) {     // tile order: see gemm_big_kernel; f: row fragments, 16..18
+    const int q = nblk >> 3, r = nblk & 7, xcd = bid & 7, idx = bid >> 3;
+    bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
+    int tn, tm;
+    if (raster > 0) {
+      const int band = bid / (raster * tiles_m), rem = bid - band * raster * tiles_m;
+      const int bw = min(raster, tiles_n - band * raster);
+      tm = rem / bw;
+      tn = band * raster + (rem - tm * bw);
+    } else {
+      tn = bid / tiles_m;
+      tm = bid - tn * tiles_m;
+    }
+    f = __builtin_amdgcn_readfirstlane(fbase + (tm < frem ? 1 : 0));
+    m0 = __builtin_amdgcn_readfirstlane((tm * fbase + min(tm, frem)) << 4);
+    n0 = __builtin_amdgcn_readfirstlane(tn * BN);
+  };
+  unsigned aoffs[APW + 1], xdst;                              // as gemm_walk_kernel; xdst: where the slot above row 256 goes
+  const bf16_t *abase, *bbase[2];
+  int dvb = blockIdx.x, dkt = kt0;
+  auto point = [&] {
+    int m0, n0, f;
+    tile_of(dvb, m0, n0, f);
+    abase = A + (size_t)m0 * lda;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) bbase[q] = W + (size_t)min((n0 >> 4) + wave * 2 + q, nfrag - 1) * K32 * 512;
+    const unsigned swz = ((lane & 7) ^ (lane >> 3)) << 4, row_bytes = (unsigned)(lda * 2);
+#pragma unroll
+    for (int q = 0; q < APW; ++q) aoffs[q] = (unsigned)min((wave * APW + q) * 8 + (lane >> 3), M - 1 - m0) * row_bytes + swz;
+    const bool have = wave < 4 && 256 + wave * 8 < f * 16;
+    aoffs[APW] = have ? (unsigned)min(256 + wave * 8 + (lane >> 3), M - 1 - m0) * row_bytes + swz : 0u;
+    xdst = have ? (unsigned)(32 + wave) * 1024u : SCRATCH;
+  };
+  const unsigned lds0 = lds_addr(dsmem);
+  auto piece = [&](int t, unsigned stage) {                   // stage: byte offset
+    if (t < APW) glds16_base(abase + dkt * BK, aoffs[t < APW ? t : 0], lds0 + stage + (wave * APW + t) * 1024u);
+    else if (t == APW) glds16_base(abase + dkt * BK, aoffs[APW], lds0 + (xdst == SCRATCH ? SCRATCH : stage + xdst));
+    else glds16_base(bbase[t > APW ? (t - APW - 1) >> 1 : 0] + (size_t)dkt * 1024 + ((t - APW - 1) & 1) * 512, lane * 16u, lds0 + stage + (A_UNITS + (wave * 4 + (t - APW - 1)) * 64) * 16u);
+  };
+  auto advance = [&] {
+    if (++dkt < nkt) return;
+    if (dvb + step < nblk) { dvb += step; dkt = kt0; point(); }
+    else dkt = nkt - 1;
+  };
+  unsigned char* const elds = reinterpret_cast<unsigned char*>(dsmem) + SCRATCH + 1024 + wave * 2048;
+
+  point();
+  if (kt0 < nkt) {
+#pragma unroll
+    for (int t = 0; t < NSLOT; ++t) piece(t, 0u);
+    advance();
+  }
+  const int boff = A_UNITS + (wn * NT * 2) * 64 + lane;
+  int st = 0;
+  bool all_stored = false;
+  auto run = [&](auto mt_c, int m0, int n0, int my_row0) {      // one tile
+    constexpr int MTW = decltype(mt_c)::value;
+    int aoff[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) aoff[kk] = (my_row0 + li) * 8 + ((kk * 4 + g) ^ (li & 7));
+    f32x4 acc[MTW > 0 ? MTW : 1][NT];
+#pragma unroll
+    for (int i = 0; i < (MTW > 0 ? MTW : 1); ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int kt = kt0; kt < nkt; ++kt) {
+      if (all_stored && kt == kt0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NSTORE) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();   // tile kt complete in LDS; every wave is done reading the other stage
+      const u32x4* s = dsmem + st * STAGE;
+      st ^= 1;
+      const unsigned dma = (unsigned)(st * STAGE) * 16u;
+      if constexpr (MTW == 0) {
+#pragma unroll
+        for (int t = 0; t < NSLOT; ++t) piece(t, dma);
+      } else {
+        bf16x8 fb[2][NT], fa[3];
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+          for (int j = 0; j < NT; ++j) fb[kk][j] = as_bf16x8(s[boff + (j * 2 + kk) * 64]);
+        fa[0] = as_bf16x8(s[aoff[0]]);
+        fa[1] = as_bf16x8(s[aoff[0] + 128]);
+#pragma unroll
+        for (int t = 0; t < 2 * MTW; ++t) {
+          if (t + 2 < 2 * MTW) fa[(t + 2) % 3] = as_bf16x8(s[aoff[(t + 2) / MTW] + ((t + 2) % MTW) * 128]);
+#pragma unroll
+          for (int j = 0; j < NT; ++j) acc[t % MTW][j] = mfma16(fb[t / MTW][j], fa[t % 3], acc[t % MTW][j]);
+          if (t < NSLOT) piece(t, dma);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x100, 2 * NT + 2, 0);
+#pragma unroll
+        for (int t = 0; t < 2 * MTW; ++t) {
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, NT, 0);
+        }
+      }
+      advance();
+    }
+    int l = lane;          // opaque: see gemm_walk_kernel
+    asm volatile("" : "+v"(l));
+    if constexpr (MTW > 0 && EPI == EPI_PARTIAL) {
+      tile_slab_wide<MTW, NT, 1, 2>(acc, m0 + my_row0, n0 + wn * 64, l, M, N, partial, nullptr, elds);
+    } else if constexpr (MTW > 0) {
+      if (wide_rows<EPI>(C, ldc, bias, residual, ldr))
+        tile_epilogue_wide<EPI, MTW, NT, 1>(acc, m0 + my_row0, n0 + wn * 64, l, bias, residual, ldr, C, ldc, M, N, nullptr, elds);
+      else tile_epilogue<EPI, MTW, NT>(acc, m0 + my_row0, n0 + wn * 64, (n0 + wn * 64) / 2, l & 15, l >> 4, bias, residual, ldr, C, ldc, M, N, partial, nullptr);
+    }
+  };
+  for (int vb = blockIdx.x; vb < nblk; vb += step) {
+    int m0, n0, f;
+    tile_of(vb, m0, n0, f);
+    const int f0 = f >> 1, my_mt = wm ? f - f0 : f0, my_row0 = wm ? f0 * 16 : 0;      // M-wave 0: f0 fragments, M-wave 1: the rest
+    if (m0 + my_row0 >= M) run(std::integral_constant<int, 0>{}, m0, n0, my_row0);
+    else if (my_mt == MTX) run(std::integral_constant<int, MTX>{}, m0, n0, my_row0);
+    else run(std::integral_constant<int, MTL>{}, m0, n0, my_row0);
+    all_stored = m0 + f * 16 <= M && n0 + BN <= N;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the copies behind the last tile
+}
+
+template <int EPI>
 __global__ __launch_bounds__(512) void gemm_vh_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
     const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
     bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n,
     float* __restrict__ partial, int kt_per_split, int raster) {
   constexpr int BN = 256, BK = 64, NT = 4;
-  constexpr int MTX = SMALL ? 5 : 9, MTL = MTX - 1;          // row fragments of an M-wave: MTL or MTX
-  constexpr int APW = SMALL ? 2 : 4;                         // 8-row activation pieces per wave below XBASE
-  constexpr int XBASE = APW * 64;                            // 128 / 256: the rows above ride on the extra slot
-  constexpr int AROWS = XBASE + (SMALL ? 16 : 32);           // 144 / 288
+  constexpr int MTX = 5, MTL = 4;                            // row fragments of an M-wave: MTL or MTX
+  constexpr int APW = 2;                                     // 8-row activation pieces per wave below XBASE
+  constexpr int XBASE = APW * 64;                            // the rows above ride on the extra slot
+  constexpr int AROWS = XBASE + 16;
   constexpr int NSLOT = APW + 5;
   constexpr int A_UNITS = AROWS * 8;              // 16-byte units of the activation image
-  constexpr int STAGE = A_UNITS + 32 * 64;        // + 32 W sub-tiles of 1 KB: 4352 units = 69,632 B (SMALL: 3200 units = 51,200 B)
-  constexpr int NST = SMALL ? 3 : 2;              // ring depth: the small tile's k-step is too short to hide a DMA round trip behind one stage
+  constexpr int STAGE = A_UNITS + 32 * 64;        // + 32 W sub-tiles of 1 KB: 51,200 B
+  constexpr int NST = 3;                          // ring depth: the k-step is too short to hide a DMA round trip behind one stage
   constexpr unsigned SCRATCH = (unsigned)NST * STAGE * 16u;  // byte offset of the 1-KB scratch behind the stages
   extern __shared__ __attribute__((aligned(16))) u32x4 dsmem[];
 
@@ -1000,7 +1315,7 @@ __global__ __launch_bounds__(512) void gemm_vh_kernel(
     tm = bid - tn * tiles_m;
   }
   const int F = (M + 15) >> 4, fbase = F / tiles_m, frem = F - fbase * tiles_m;
-  const int f = fbase + (tm < frem ? 1 : 0);                       // row fragments of this tile: 16..18 (SMALL: 8..9)
+  const int f = fbase + (tm < frem ? 1 : 0);                       // row fragments of this tile: 8..9
   const int m0 = (tm * fbase + min(tm, frem)) << 4, n0 = tn * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 2, wn = wave & 3;
@@ -1010,8 +1325,8 @@ __global__ __launch_bounds__(512) void gemm_vh_kernel(
   const int my_mt = wm ? f - f0 : f0, my_row0 = wm ? f0 * 16 : 0;
   const bool wave_has_rows = m0 + my_row0 < M;
 
-  // DMA piece table of this wave: slots 0-3 activation rows (wave*4 + q)*8 .. +7, slot 4 rows 256 + wave*8 .. (waves 0-3, if the tile
-  // has them), slots 5-8 W sub-tiles wave*4 + q (n-fragment row st >> 1, 32-k block st & 1)
+  // DMA piece table of this wave: slots 0-1 activation rows (wave*2 + q)*8 .. +7, slot 2 rows 128 + wave*8 .. (waves 0-1, if the tile
+  // has them), slots 3-6 W sub-tiles wave*4 + q (n-fragment row st >> 1, 32-k block st & 1)
   const bf16_t* psrc[NSLOT];
   unsigned pdst[NSLOT];
   const int swz = ((lane & 7) ^ (lane >> 3)) << 3;
@@ -1061,10 +1376,9 @@ __global__ __launch_bounds__(512) void gemm_vh_kernel(
       for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
     int st_cur = 0;                   // stage of tile kt = (kt - kt0) % NST
     for (int kt = kt0; kt < nkt; ++kt) {
-      // every wave issues exactly NSLOT pieces per tile, so with NST = 3 the newest tile's pieces may stay in flight across the barrier
-      static_assert(NST == 2 || NSLOT == 7, "the counted wait below is written for 7 pieces per tile");
-      if constexpr (NST == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(7)" ::: "memory");
+      // every wave issues exactly NSLOT pieces per tile, so the newest tile's pieces may stay in flight across the barrier
+      static_assert(NSLOT == 7, "the counted wait below is written for 7 pieces per tile");
+      asm volatile("s_waitcnt vmcnt(7)" ::: "memory");
       __builtin_amdgcn_s_barrier();   // tile kt complete in LDS; every wave is done reading tile kt-1
       const u32x4* s = dsmem + st_cur * STAGE;
       // the pieces of tile kt+NST-1 go out unconditionally (a branch would cut the scheduling region): past the last tile the source is
@@ -1102,7 +1416,7 @@ __global__ __launch_bounds__(512) void gemm_vh_kernel(
       }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the clamped copies of the last iteration
-    const bool wide = EPI == EPI_PARTIAL || wide_rows<EPI>(C, ldc, residual, ldr);          // block-uniform
+    const bool wide = EPI == EPI_PARTIAL || wide_rows<EPI>(C, ldc, bias, residual, ldr);          // block-uniform
     if (wide) __builtin_amdgcn_s_barrier();          // every wave is done with the stages, and its DMA pieces have landed
     if constexpr (MTW > 0 && EPI == EPI_PARTIAL) {
       tile_slab_wide<MTW, NT>(acc, m0 + my_row0, n0 + wn * 64, lane, M, N, partial, nullptr, reinterpret_cast<unsigned char*>(dsmem) + wave * 8192);
@@ -1344,22 +1658,46 @@ static void launch_big_s(const GemmArgs& a, hipStream_t st) {
       a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.partial, (nkt + S - 1) / S, a.wscale, a.vq,
       raster_for(tiles_m));
 }
+// the walking kernels' offsets inside a tile are 32-bit (288 activation rows)
+static bool walk_offsets_fit(const GemmArgs& a) { return (size_t)a.lda * 576 <= 0xffffffffu; }
+template <int BM, int EPI>
+static void launch_walk(const GemmArgs& a, hipStream_t st) {
+  const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + 255) / 256;
+  const int nkt = a.K / 64, S = (EPI == EPI_PARTIAL) ? a.nsplit : 1;
+  constexpr size_t lds = (size_t)(BM >= 192 ? 2 : 3) * (BM * 8 + 2048) * 16 + 8 * (BM >= 192 && EPI != EPI_GELU_ERF ? 4096 : 2048);      // 160 / 144 / 160 KB
+  static DeviceOnce attr_set;   // per instantiation
+  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_walk_kernel<BM, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  const unsigned grid = std::min(capped_grid((long)tiles_m * tiles_n), (unsigned)std::max(8, (256 / S) & ~7));
+  gemm_walk_kernel<BM, EPI><<<dim3(grid, S), dim3(512), lds, st>>>(a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m,
+                                                                   tiles_n, a.partial, (nkt + S - 1) / S, a.wscale, raster_for(tiles_m));
+}
 // variable-height row tiles (gemm_vh_kernel): tiles_m = floor(F / 16) row tiles for F = ceil(M / 16) row fragments (small class: F / 8)
 static bool vh_legal(const GemmArgs& a, bool small = false) {
   const int F = (a.M + 15) >> 4, t = F >> (small ? 3 : 4);
   // wscale == nullptr: gemm_w8's dequantisation fallback re-enters with w_fp8 = 0 and a LIVE row scale for the epilogue, which
   // this kernel does not carry
-  return a.w_packed && !a.w_fp8 && a.wscale == nullptr && (a.K % 64) == 0 && t >= 1 && F <= (small ? 9 : 18) * t && (a.N & 15) == 0;
+  return a.w_packed && !a.w_fp8 && a.wscale == nullptr && (a.K % 64) == 0 && t >= 1 && F <= (small ? 9 : 18) * t && (a.N & 15) == 0 && walk_offsets_fit(a);
 }
-template <int EPI, int SMALL = 0>
+template <int EPI>
 static void launch_vh(const GemmArgs& a, hipStream_t st) {
-  const int F = (a.M + 15) >> 4, tiles_m = F >> (SMALL ? 3 : 4), tiles_n = (a.N + 255) / 256;
+  const int F = (a.M + 15) >> 4, tiles_m = F >> 4, tiles_n = (a.N + 255) / 256;
   const int nkt = a.K / 64, S = (EPI == EPI_PARTIAL) ? a.nsplit : 1;
-  constexpr size_t lds = (size_t)(SMALL ? 3 : 2) * ((SMALL ? 144 : 288) * 8 + 2048) * 16 + 1024;      // 2 x 69,632 B / 3 x 51,200 B + the scratch
+  constexpr size_t lds = (size_t)2 * (288 * 8 + 2048) * 16 + 1024 + 8 * 2048;      // stages, scratch, epilogue: 156,672 B
   static DeviceOnce attr_set;   // per instantiation
-  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_vh_kernel<EPI, SMALL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_walk_vh_kernel<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   g_launch_counts[LC_GEMM_VH]++;
-  gemm_vh_kernel<EPI, SMALL><<<dim3(capped_grid((long)tiles_m * tiles_n), S), dim3(512), lds, st>>>(
+  const unsigned grid = std::min(capped_grid((long)tiles_m * tiles_n), (unsigned)std::max(8, (256 / S) & ~7));
+  gemm_walk_vh_kernel<EPI><<<dim3(grid, S), dim3(512), lds, st>>>(
+      a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.partial, (nkt + S - 1) / S, raster_for(tiles_m));
+}
+static void launch_vh_small(const GemmArgs& a, hipStream_t st) {      // split-K slabs
+  const int F = (a.M + 15) >> 4, tiles_m = F >> 3, tiles_n = (a.N + 255) / 256;
+  const int nkt = a.K / 64, S = a.nsplit;
+  constexpr size_t lds = (size_t)3 * (144 * 8 + 2048) * 16 + 1024;      // 3 x 51,200 B + the scratch
+  static DeviceOnce attr_set;
+  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_vh_kernel<EPI_PARTIAL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  g_launch_counts[LC_GEMM_VH]++;
+  gemm_vh_kernel<EPI_PARTIAL><<<dim3(capped_grid((long)tiles_m * tiles_n), S), dim3(512), lds, st>>>(
       a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.partial, (nkt + S - 1) / S, raster_for(tiles_m));
 }
 template <int BM, int EPI>
@@ -1369,7 +1707,10 @@ static void launch_big(const GemmArgs& a, hipStream_t st) {
   // GEMMs, +0.6 / +0.8 % tokens/s at 1 / 8 streams, profiles/r03/gemm_sched_spread_dma.txt); LCC_GEMM_SCHED=1 restores SCHED 1
   static const int spread = [] { const char* v = getenv("LCC_GEMM_SCHED"); return (v && atoi(v) == 1) ? 0 : 1; }();
   if (a.w_fp8) launch_big_s<(BM == 192 ? 256 : BM), EPI, 1, true>(a, st);     // the 192-row tile is a bf16-weight shape (big_tile_rows never picks it for fp8)
-  else if (g_gemm_sched && spread) launch_big_s<BM, EPI, 6, false>(a, st);
+  else if (g_gemm_sched && spread) {
+    if (!walk_offsets_fit(a)) launch_big_s<BM, EPI, 1, false>(a, st);
+    else launch_walk<BM, EPI>(a, st);
+  }
   else if (g_gemm_sched) launch_big_s<BM, EPI, 1, false>(a, st);
   else launch_big_s<BM, EPI, 0, false>(a, st);
 }
@@ -2134,7 +2475,7 @@ int gemm_bf16(const GemmArgs& a, hipStream_t st) {
     if (a.epilogue != EPI_NONE || a.nsplit < 1 || a.nsplit > 8 || a.nsplit > (a.K + 63) / 64) return LCC_ERR_ARG;
     const int big = big_tile_rows(a, a.nsplit);
     if (big == 272) launch_vh<EPI_PARTIAL>(a, st);
-    else if (big == 144) launch_vh<EPI_PARTIAL, 1>(a, st);
+    else if (big == 144) launch_vh_small(a, st);
     else if (big == 256) launch_big<256, EPI_PARTIAL>(a, st);
     else if (big == 192) launch_big<192, EPI_PARTIAL>(a, st);
     else if (big == 128) launch_big<128, EPI_PARTIAL>(a, st);

@@ -203,6 +203,28 @@ def test_gemm_epilogue_rows_of_16_byte_pieces_and_others_give_the_same_bits(dev,
     assert_bf16_close(outs[0], ref, f"gemm rows[{variant},epi{epi}]", max_ulp=1.0, max_frac=5e-3, atol=atol)
 
 
+@pytest.mark.parametrize("variant,M,K,S", [(3, 2100, 64, 0), (3, 2100, 192, 3), (13, 1600, 128, 1), (13, 1600, 64, 0), (4, 1100, 64, 0), (4, 1100, 128, 0),
+                                           (4, 1100, 320, 0), (14, 2130, 64, 0), (14, 2130, 192, 3)])
+def test_gemm_blocks_that_walk_several_tiles_are_bit_identical_to_one_tile_a_block(dev, variant, M, K, S):
+    """More tiles than compute units (9 x 34 and 8 x 34, ragged rows and columns), one k-tile up to more than the ring holds: every epilogue and the
+    fp32 slabs, three splits with the chip's blocks shared among them."""
+    from livecc_amd import ops
+    N = 8480
+    x, w, b, r = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.05, 2), _rand((N,), dev, 0.1, 3), _rand((M, N), dev, 1.0, 4)
+    wp = ops.pack_weight(w)
+
+    def outputs(v):
+        ops.set_gemm_variant(v)
+        try:
+            y = [ops.linear(x, wp, None if epi == 4 else b, epi, r if epi == 3 else None, packed_shape=(N, K)) for epi in range(5)]
+            return y + ([ops.linear_partial(x, wp, S, packed_shape=(N, K))] if S else [])
+        finally:
+            ops.set_gemm_variant(ops.GEMM_DEFAULT_VARIANT)
+
+    for i, (got, ref) in enumerate(zip(outputs(variant), outputs(5))):
+        assert torch.equal(got, ref), f"output {i}: {int((got != ref).sum())} of {got.numel()} values differ"
+
+
 def test_activations_round_like_double_precision_on_every_finite_bf16_input(dev):
     """quick_gelu (the rounding points of its three bf16 operations) and silu over all 65,280 finite inputs: the rounded double-precision value
     wherever it is at least 1e-36 in magnitude.  Smaller normal values may come out as zero, their reciprocal's subnormal result being flushed
