@@ -42,12 +42,6 @@ LCC_DEVICE float xor32_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-__device__ unsigned int lcc_attn32_zero_page[256];
-__device__ unsigned int lcc_attn32_ones_page[256] = {[0 ... 255] = 0x3F803F80u};      // 1 KB of bf16 1.0: the V^T rows 80..95 of the tower kernel (LM)
-
-// (Round 6, measured null and removed: a static `s_setprio 1` for the younger or for the older half of the waves -- MI355X_MICROARCH "Two
-// waves per SIMD" item 4 -- 416-421 us either way at 8 x 386 rows x 6.2k keys, tower 20.8 ms either way: profiles/r06/attn_static_prio_ab.jsonl.)
-
 // ------------------------------------------------------------------------------------------------------------------------------
 // The key loop shared by the LLM prefill kernel (D = 128) and the ViT kernel (D = 80): software pipeline, one key tile per REGION.
 // The softmax of tile t (vector pipe: ~70 VALU instructions) is issued next to the MFMAs that do not depend on it -- the P . V of tile
@@ -56,150 +50,281 @@ __device__ unsigned int lcc_attn32_ones_page[256] = {[0 ... 255] = 0x3F803F80u};
 // ran the same phase in lock step behind the block barrier: the first version of the D = 128 kernel, 0.57 PF at 8 x 386 rows x 6k
 // keys against 0.54 for the 16x16x32 kernel; pipelined: 0.76 PF, 1.36 vs 1.93 ms for a 4,096-row piece against 20k keys.)
 //
-// Ring of NSTAGE = 10 tile stages = five pair-stages (the register budget allows one block per CU anyway).  At the top of the
-// iteration of pair P = (t, t+1): pairs P-1 (its second tile still owes its P.V), P and P+1 have landed (counted vmcnt: only pair P+2,
-// issued one iteration ago, may still be in flight; barrier: every wave's pieces), every wave is done with pair P-2, whose stages
-// receive pair P+3.  The iteration enters with sc_a = K.Q^T of tile t and leaves with sc_a = K.Q^T of tile t+2.
-// LDS image of a stage: KP = D/16 K pieces (32 keys x 16 d each, rows in swap23 order) then VP = 2 * ceil(D/32) V^T pieces
-// (32 d rows x 16 keys each), every piece 1 KB in MFMA fragment (lane) order.
+// Ring of three pair-stages.  Slot t holds what region t multiplies -- K of tile t + 1 and V^T of tile t - 1 -- so a pair needs its own two slots only:
+// at the top of the iteration of pair (t, t + 1) its slots have landed (counted vmcnt: only the next pair's, issued one iteration ago, may still
+// be in flight; barrier: every wave's pieces) and the slots of the pair before receive pair t + 4.  (Whole tiles a slot needed five pair-stages: one
+// block a compute unit.)  The iteration enters with sc_a = K.Q^T of tile t and leaves with sc_a = K.Q^T of tile t + 2.
+//
+// An iteration is ONE basic block -- 2 x NP MFMAs, every fragment read FRAG_LEAD MFMAs ahead of its use, the DMA pieces of pair P+3 spread between
+// them -- because the softmax has no branch: probabilities are taken against a reference that is only moved between two pairs.
+//   * Reference: the ceiling of the row's maximum over its first key tile (log2 units); moved to the ceiling of the maximum so far when a
+//     pair held a score more than `slack` above it.  Until then probabilities are up to 2^slack (fp32 and bf16 hold the exponent; numerator and denominator carry
+//     the same factor), and moving by a whole number of powers of two is exact on O, l and the pending P.  The running maximum itself moves in nearly
+//     every tile of a short key range (32 rows, each with chance 1 / t in tile t): a rescale of O behind the MFMAs, a maximum that every exponential
+//     waits for, and a branch in every region that cut the schedule in two.
+//   * A score more than REF_JUMP above the reference within one pair could overflow: the block then goes through its keys a second time (`again`),
+//     those rows with the final reference of the first time, which no score exceeds.
+//   * Each row decides by its own scores (both lanes of its column), so its bits do not depend on its neighbours in the wave.
+// Measured (us; one region of 16 / 11 MFMAs a block, running maximum, fragment-order gathers -> here): 4,096 rows on 8k keys 700 -> 597 (1.01 PF), 386 rows on
+// 2k keys in five splits 40.7 -> 36.8, 8 x 386 rows on 1.1k 103 -> 84; with a bias, 4,096 rows on 4k 577 -> 503; tower, 18 slices of 880 patches 173 -> 138 with 256
+// rows a block and 113 with 128, one slice of 1,456 35.7 -> 29.5.  What bounds it now: the vector pipe beside the matrix pipe (with neither DMA nor fragment
+// reads the loop ran 4,096 rows on 8k keys in 489).
+//
+// LDS image of a slot: rows as they lie in memory, so that a DMA instruction copies whole runs of lines (K: 32 keys x 2 D bytes; V^T: DV rows x 64 bytes)
+// instead of 64 separate 16-byte chunks, each a line of its own for the address path (a 4-wave block of the tower kernel spent 15 of its 42 us on that).  A row's
+// 16-byte chunks are permuted (kx, vx) so that the fragment reads -- one chunk of 16 rows at a time -- touch every bank once; K rows of 256 bytes
+// also shift by a chunk every four rows (their DMA instruction).
 //   mlim: tiles reaching past it need the mask (causal diagonal / end of the key range); lim: this lane's effective key limit.
 //
-// (Round 5, measured null and removed: reading the next region's first three V^T fragments at the end of the region before it -- no LDS
-// round trip in front of a region's first MFMAs -- 377-382 us either way at 8 x 386 rows x 6.2k keys, profiles/r05/attn_pipe_ab.txt.)
-// (Round 6, measured and removed -- the first two were tests of "the kernel is bound by the staging of its K / V tiles":
-//   * ROW-MAJOR stage images (every LDS-DMA instruction copies one contiguous KB of the cache -- 4 K rows / 16 V^T rows -- into an XOR-swizzled
-//     [32][256 B] / [D][64 B] image, conflict-free fragment reads, same bits) instead of the fragment-order pieces below, whose DMA gathers 64
-//     separate 16-byte chunks: 8 x 386 rows 427.8 / 429.0 us vs 431.3 / 420.4, one-shot piece 690 / 692 vs 687 / 685, tower 20.80-20.88 ms vs
-//     20.52 (8 K pieces instead of 5 there): a null; profiles/r06/attn_rowmajor_staging_ab.jsonl, tower_rowmajor_staging_ab.jsonl.
-//   * one wave per SIMD (the 7 heads of a KV head as two 4-wave blocks with a ring each): 675 vs 420 us,
-//     profiles/r06/attn_one_wave_per_simd_ab.jsonl.  NOT a clean test, found afterwards: the 4-wave instantiation was compiled in the AGPR form
-//     (see attn_gqa32_kernel) and issued 329 instructions per region against the 8-wave kernel's 185 (of which 32 v_pk_mul sit in the skipped
-//     rescale branch: 16 MFMAs, 16 fragment reads, 83 vector and ~38 scalar instructions per region and wave).  A 4-wave block with 1.8 x the
-//     instructions took 0.8 of the 8-wave block's time, so a wave alone on its SIMD runs its stream ~2.2 x faster than one that shares it:
-//     the two waves of a SIMD do not overlap their matrix and vector work, they mostly take turns.
-//   * PING-PONG phases ("two waves of a SIMD in the same phase"): a region issued as a matrix phase (its 16 / 11 MFMAs with
-//     their fragment reads) and a vector phase (the softmax), in OPPOSITE order on the two waves that share a SIMD (w and w + 4; both phases
-//     of region t depend only on region t - 1; two copies of the key loop under a wave-uniform branch, 235 VGPRs, same bits) instead of the
-//     instruction-by-instruction interleave below: 8 x 386 rows 429-432 vs 382-387 us (+11 %), a 4,096-row piece 708 vs 655 (+8 %), one
-//     chunk 81.5 vs 74.0, tower 20.59 vs 20.38 ms; profiles/r06/attn_pingpong_phases_ab.jsonl.  The interleave already overlaps a wave's own
-//     MFMAs with its own vector instructions; separating them loses that and the other wave does not make up for it.  Removed.)
-// LM (round 6, the tower kernel only): the softmax denominator comes out of the P . V MFMAs -- the V^T rows 80..95 of the third d-tile do not
-// exist at d = 80 and are fed with ONES, so O^T rows 80..95 accumulate sum_k bf16(P) under the same lazy rescale as O -- instead of 16 v_add +
-// the l_run update per region.  l then sums the ROUNDED probabilities the numerator uses (fp32 accumulation either way).
-// D = channels of q / k, DV = channels of v.  BIAS: slope (pos - key) is taken off the scaled scores (slope in units of log2), pos = this lane's query.
-template <int D, int DV, int PW, bool LM, bool BIAS = false, class Issue>
-LCC_DEVICE void attn32_key_loop(const u32x4* alds, Issue issue, const u32x4 (&qf)[D / 16], int tb, int te, int mlim, int lim, float scale_raw,
-                                bool active, int lane, int hh, f32x16 (&o)[(DV + 31) / 32], float& m_run, float& l_run, float slope = 0.f, int pos = 0) {
-  const float scale_log2e = BIAS ? 1.f : scale_raw;     // with a bias the scores are brought to log2 units before the maximum
-  constexpr int KP = D / 16, DT = (DV + 31) / 32, VP = 2 * DT, NP = KP + VP, NSTAGE = 10;
-  auto stage_of = [&](int t) { return alds + ((t - tb) % NSTAGE) * (NP * 64); };
-  bf16x8 p_prev[2];                                     // P of the previous tile, its P . V still pending
-  p_prev[0] = as_bf16x8((u32x4){0u, 0u, 0u, 0u});
-  p_prev[1] = p_prev[0];
-  const u32x4* v_prev = alds;                           // V stage of that tile (while nothing is pending P = 0: any landed stage will do)
-  f32x16 sc_a, sc_b;
+// Measured and not taken: the two waves of a SIMD in opposite phases (matrix work of one beside the softmax of the other): 11 % slower than the
+// instruction-by-instruction interleave; all fragments of a region read a region ahead: 64 registers, spills.
+// LM (the tower kernel): the softmax denominator comes out of the P . V MFMAs -- the V^T rows 80..95 of the third d-tile do not exist at d = 80 and
+// are ONES, so O^T rows 80..95 accumulate sum_k bf16(P) under the same rescale as O -- instead of 16 additions per region.  l then sums the ROUNDED
+// probabilities the numerator uses (fp32 accumulation either way).
+// D = channels of q / k, DV = channels of v.  BIAS: slope (pos - key) is taken off the scaled scores (slope in units of log2), pos = this lane's query:
+// K.Q^T is added to it instead of to zero.
+struct Kv32 {                   // keys and values of one (stream, head); all wave-uniform
+  const bf16_t *k, *v;          // tile 0
+  unsigned k_row, v_row;        // bytes between keys of K, between channels of V^T
+  size_t k_tile, v_tile;        // bytes between 32-key tiles
+  int ntile, nkeys;             // tiles; CLAMP: keys that exist (the last tile's rows beyond them are not read)
+};
+template <int D, int DV>
+struct Attn32Image {
+  static constexpr int CR = D / 8, DT = (DV + 31) / 32, KPD = D / 16, VPD = DV / 16, NPD = KPD + VPD;      // chunks of a K row; DMA instructions of K, V
+  static constexpr int KB = D == 128 ? 8 * 1040 : 64 * D, VB = DT * 2048, SLOT = KB + VB, BYTES = 6 * SLOT;
+  LCC_DEVICE static int kx(int row) { return D == 128 ? (row & 3) * 4 : D == 64 ? (row >> 1) & 7 : (row >> 3) & 1; }
+  LCC_DEVICE static int vx(int d) { return (d >> 2) & 3; }
+};
 
-  auto region = [&](auto masked_tag, int t, f32x16& sc_cur, f32x16& sc_nxt) {
-    constexpr bool MASKED = decltype(masked_tag)::value;
-    const u32x4* vs = v_prev;
-    const u32x4* kn = stage_of(t + 1);
-    // matrix pipe: P.V of tile t-1 ...
+template <int D, int DV, int NWAVE, bool LM, bool BIAS = false, bool CLAMP = false>
+LCC_DEVICE void attn32_key_loop(unsigned char* alds, const Kv32& kv, const u32x4 (&qf)[D / 16], int tb, int te, int mlim, int lim, float scale_log2e,
+                                bool active, int lane, int wave, int hh, f32x16 (&o)[(DV + 31) / 32], float& m_run, float& l_run, float slope = 0.f, int pos = 0) {
+  using Im = Attn32Image<D, DV>;
+  constexpr int KP = D / 16, DT = Im::DT, VP = 2 * DT, NP = KP + VP, FRAG_LEAD = 4;
+  constexpr int NPD = Im::NPD, PWP = (2 * NPD + NWAVE - 1) / NWAVE, PK = (Im::KPD + NWAVE - 1) / NWAVE;     // DMA pieces of a wave: a pair; K of one tile
+  constexpr float REF_JUMP = 100.f;
+  m_run = -INFINITY;
+  if (te <= tb) return;                                 // (block-uniform: a key split without a tile)
+  // a bias of `slope` a key lifts a row's scores by 64 slope from pair to pair: the slack leaves room for that below the jump
+  const float slack = BIAS ? fmaxf(0.f, fminf(40.f, 88.f - 64.f * slope)) : 16.f;
+  const unsigned lds0 = lds_addr(alds);
+  float m_ref = 0.f, m_limit = -INFINITY;               // m_limit = -inf: the row has seen no key
+  const float bias_raw = BIAS ? slope / scale_log2e : 0.f, bias_pos = BIAS ? bias_raw * (float)(8 * hh - pos) : 0.f;
+  const int col = lane & 31;
+
+  // DMA: this wave's pieces of a pair.  Surplus slots copy the last piece again (same bytes, same place).
+  unsigned off[PWP], prow[CLAMP ? PWP : 1];
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int ss = 0; ss < 2; ++ss) o[dt] = mfma32(as_bf16x8(vs[(KP + dt * 2 + ss) * 64 + lane]), p_prev[ss], o[dt]);
-    // ... and K.Q^T of tile t+1
-#pragma unroll
-    for (int r = 0; r < 16; ++r) sc_nxt[r] = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < KP; ++ks) sc_nxt = mfma32(as_bf16x8(kn[ks * 64 + lane]), as_bf16x8(qf[ks]), sc_nxt);
-    // vector pipe: softmax of tile t
-    const int kb = t * 32;
-    if (BIAS) {
-      const float base = slope * (float)(kb + 8 * hh - pos);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) sc_cur[r] = fmaf(sc_cur[r], scale_raw, fmaf(slope, (float)(16 * (r >> 3) + (r & 7)), base));
+  for (int j = 0; j < PWP; ++j) {
+    const int u = min(j * NWAVE + wave, 2 * NPD - 1), p = u >= NPD ? u - NPD : u;
+    if (p < Im::KPD) {
+      const int row = (p * 64 + lane) / Im::CR, c = (p * 64 + lane) % Im::CR;
+      off[j] = (CLAMP ? 0u : (unsigned)row * kv.k_row) + (unsigned)((c ^ Im::kx(row)) * 16);
+      if (CLAMP) prow[j] = row;
+    } else {
+      const int d = (p - Im::KPD) * 16 + (lane >> 2);
+      off[j] = (unsigned)d * kv.v_row + (unsigned)(((lane & 3) ^ Im::vx(d)) * 16);
+      if (CLAMP) prow[j] = 0u;
     }
-    if (MASKED) {
+  }
+  auto piece = [&](int p, int tile, bool is_k, unsigned o_lane, unsigned row, unsigned slot) {      // p: of the slot; tile: in range
+    if (CLAMP) o_lane += __umul24(min(row, (unsigned)(kv.nkeys - 1 - tile * 32)), is_k ? kv.k_row : 0u);      // no branch: this is inside the pair's basic block
+    const char* base = is_k ? reinterpret_cast<const char*>(kv.k) + (size_t)tile * kv.k_tile : reinterpret_cast<const char*>(kv.v) + (size_t)tile * kv.v_tile;
+    glds16_base(base, o_lane, slot + (unsigned)(is_k ? p * (D == 128 ? 1040 : 1024) : Im::KB + (p - Im::KPD) * 1024));
+  };
+  auto issue = [&](int j, int t, int ps) {              // piece j of the pair (t, t + 1) into pair-stage ps
+    const int u = min(j * NWAVE + wave, 2 * NPD - 1), r = u >= NPD ? 1 : 0, p = u - r * NPD;
+    const bool is_k = p < Im::KPD;
+    const int tile = min(is_k ? t + r + 1 : max(t + r - 1, tb), kv.ntile - 1);
+    piece(p, tile, is_k, off[j], CLAMP ? prow[CLAMP ? j : 0] : 0u, lds0 + (unsigned)((2 * ps + r) * Im::SLOT));
+  };
+  // fragment addresses inside a slot: K row swap23(col), chunk 2 ks + hh; V^T row 32 dt + col, chunk 2 s + hh
+  constexpr int NKA = D == 80 ? 1 : 4;
+  int ka[NKA], va[2];
+  {
+    const int row = swap23(col), r0 = D == 128 ? (row >> 2) * 1040 + (row & 3) * 256 : row * D * 2, x = Im::kx(row);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) sc_cur[r] = (kb + 16 * (r >> 3) + 8 * hh + (r & 7)) < lim ? sc_cur[r] : -INFINITY;
+    for (int i = 0; i < NKA; ++i) ka[i] = r0 + (((D == 128 ? 4 * i + hh : 2 * i + hh) ^ x) * 16);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) va[s] = Im::KB + col * 64 + (((2 * s + hh) ^ Im::vx(col)) * 16);
+  }
+  auto kfrag = [&](const unsigned char* slot, int ks) {
+    return *reinterpret_cast<const u32x4*>(slot + ka[D == 128 ? ks >> 1 : D == 80 ? 0 : ks] + (D == 128 ? (ks & 1) * 32 : D == 80 ? ks * 32 : 0));
+  };
+  auto vfrag = [&](const unsigned char* slot, int i) { return *reinterpret_cast<const u32x4*>(slot + va[i & 1] + (i >> 1) * 2048); };
+
+  auto clear = [&](int t, f32x16& sc) {                           // what K.Q^T of tile t is added to: the bias, in units of unscaled scores
+    const float base = BIAS ? fmaf(bias_raw, (float)(t * 32), bias_pos) : 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sc[r] = BIAS ? fmaf(bias_raw, (float)(16 * (r >> 3) + (r & 7)), base) : 0.f;
+  };
+  auto mask = [&](auto masked_tag, int t, f32x16& sc) {
+    if (decltype(masked_tag)::value) {
+      const int kb = t * 32;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) sc[r] = (kb + 16 * (r >> 3) + 8 * hh + (r & 7)) < lim ? sc[r] : -INFINITY;
     }
-    float mx = vmax3(sc_cur[0], sc_cur[1], sc_cur[2]);
+  };
+  auto lane_max = [&](const f32x16& sc) {                         // of this lane's 16 keys
+    float mx = vmax3(sc[0], sc[1], sc[2]);
 #pragma unroll
-    for (int r = 3; r < 15; r += 2) mx = vmax3(mx, sc_cur[r], sc_cur[r + 1]);
-    mx = vmax(mx, sc_cur[15]);
-    mx = xor32_max(mx);
-    const float m_new = vmax(m_run, mx * scale_log2e);
-    const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);       // m_run = -inf -> 0
-    m_run = m_new;
-    float p[16], psum = 0.f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      p[r] = __builtin_amdgcn_exp2f(fmaf(sc_cur[r], scale_log2e, -m_use));   // masked scores are -inf -> 0
-      if (!LM) psum += p[r];
-    }
-    if (!LM) l_run = l_run * alpha + psum;
-    bf16x8 pn[2];
-#pragma unroll
-    for (int ss = 0; ss < 2; ++ss)
-      pn[ss] = as_bf16x8((u32x4){pack2(p[8 * ss + 0], p[8 * ss + 1]), pack2(p[8 * ss + 2], p[8 * ss + 3]),
-                                 pack2(p[8 * ss + 4], p[8 * ss + 5]), pack2(p[8 * ss + 6], p[8 * ss + 7])});
-    // keep the exponentials and the packing of P INSIDE this region: P is only consumed by the next region's MFMAs, and LLVM otherwise
-    // sinks its computation behind the rescale branch below, where no matrix work is left to hide it
-    {
-      u32x4 w0 = as_u32x4(pn[0]), w1 = as_u32x4(pn[1]);
-      asm volatile("" : "+v"(w0[0]), "+v"(w0[1]), "+v"(w0[2]), "+v"(w0[3]), "+v"(w1[0]), "+v"(w1[1]), "+v"(w1[2]), "+v"(w1[3]), "+v"(l_run));
-      pn[0] = as_bf16x8(w0); pn[1] = as_bf16x8(w1);
-    }
-    // issue order: a few fragment reads ahead, then per MFMA one more read and a handful of vector instructions
-    __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
-#pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if (i < NP - 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, ((MASKED ? 7 : 5) - (LM ? 1 : 0) + (BIAS ? 2 : 0)) * 16 / NP, 0);
-    }
-    // region boundary: the accumulators now hold tiles <= t-1 at the OLD maximum; bring them to the new one before tile t's P.V.
-    // Lazy: once the running maximum has settled alpha is exactly 1.0 in every lane and the multiplies are skipped (x * 1.0f is
-    // exact: bit-identical to always rescaling)
-    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
-    }
-    p_prev[0] = pn[0]; p_prev[1] = pn[1];
-    v_prev = stage_of(t);
+    for (int r = 3; r < 15; r += 2) mx = vmax3(mx, sc[r], sc[r + 1]);
+    return vmax(mx, sc[15]) * scale_log2e;
   };
 
-  issue(tb); issue(tb + 1); issue(tb + 2); issue(tb + 3); issue(tb + 4); issue(tb + 5);
-  for (int t = tb; t < te; t += 2) {
-    if (PW == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
-    else if (PW == 2) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-    else if (PW == 3) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-    else if (PW == 4) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    issue(t + 6); issue(t + 7);
-    if (!active) continue;
-    if (t == tb) {
-      const u32x4* k0 = stage_of(tb);
+  bool bad = false;
+  for (int pass = 0;; ++pass) {
+    bf16x8 p_prev[2];                                   // P of the previous tile, its P . V still pending
+    p_prev[0] = as_bf16x8((u32x4){0u, 0u, 0u, 0u});
+    p_prev[1] = p_prev[0];
+    f32x16 sc_a, sc_b;
+    float mx_pair = -INFINITY;                          // of the last pair, this lane's keys
+    int st = 0;                                         // pair-stage of the pair
+    // one pair: softmax of tiles t and t + 1 (vector pipe) beside P.V of t - 1 and t, K.Q^T of t + 1 and t + 2 (matrix pipe)
+    auto pair = [&](auto masked_tag, int t) {
+      constexpr bool MASKED = decltype(masked_tag)::value;
+      // the two copies of the pair keep their fragment reads: shared, they would all sit in front of the branch between them
+      if (MASKED) asm volatile("; masked pair" ::: "memory"); else asm volatile("; whole pair" ::: "memory");
+      const unsigned char* slot[2] = {alds + 2 * st * Im::SLOT, alds + (2 * st + 1) * Im::SLOT};
+      const int ps = st == 0 ? 2 : st - 1;
+      u32x4 f[FRAG_LEAD + 1];
+      auto read = [&](int i) { const int r = i / NP, w = i % NP; return w < VP ? vfrag(slot[r], w) : kfrag(slot[r], w - VP); };
 #pragma unroll
-      for (int r = 0; r < 16; ++r) sc_a[r] = 0.f;
+      for (int i = 0; i < FRAG_LEAD; ++i) f[i] = read(i);
+      mx_pair = -INFINITY;
 #pragma unroll
-      for (int ks = 0; ks < KP; ++ks) sc_a = mfma32(as_bf16x8(k0[ks * 64 + lane]), as_bf16x8(qf[ks]), sc_a);
+      for (int r = 0; r < 2; ++r) {
+        f32x16& cur = r == 0 ? sc_a : sc_b;
+        f32x16& nxt = r == 0 ? sc_b : sc_a;
+        // vector pipe
+        f32x16 x = cur;
+        mask(masked_tag, t + r, x);
+        mx_pair = vmax(mx_pair, lane_max(x));
+        float p[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) p[e] = __builtin_amdgcn_exp2f(fmaf(x[e], scale_log2e, -m_ref));   // masked scores are -inf -> 0
+        if (!LM) {
+#pragma unroll
+          for (int e = 0; e < 16; ++e) l_run += p[e];
+        }
+        u32x4 w0 = {pack2(p[0], p[1]), pack2(p[2], p[3]), pack2(p[4], p[5]), pack2(p[6], p[7])};
+        u32x4 w1 = {pack2(p[8], p[9]), pack2(p[10], p[11]), pack2(p[12], p[13]), pack2(p[14], p[15])};
+        // matrix pipe
+#pragma unroll
+        for (int w = 0; w < NP; ++w) {
+          const int i = r * NP + w;
+          if (w < VP) o[w >> 1] = mfma32(as_bf16x8(f[i % (FRAG_LEAD + 1)]), p_prev[w & 1], o[w >> 1]);
+          else {
+            if (w == VP) clear(t + r + 1, nxt);
+            nxt = mfma32(as_bf16x8(f[i % (FRAG_LEAD + 1)]), as_bf16x8(qf[w >= VP ? w - VP : 0]), nxt);
+          }
+          if (i + FRAG_LEAD < 2 * NP) f[(i + FRAG_LEAD) % (FRAG_LEAD + 1)] = read(i + FRAG_LEAD);
+#pragma unroll
+          for (int j = 0; j < PWP; ++j)
+            if (i == (2 * j + 1) * NP / PWP) issue(j, t + 4, ps);
+        }
+        if (r == 1) {     // P of the pair's second tile is consumed by the next iteration: formed here, under this one's MFMAs
+          asm volatile("" : "+v"(w0[0]), "+v"(w0[1]), "+v"(w0[2]), "+v"(w0[3]), "+v"(w1[0]), "+v"(w1[1]), "+v"(w1[2]), "+v"(w1[3]), "+v"(l_run), "+v"(mx_pair));
+        }
+        p_prev[0] = as_bf16x8(w0); p_prev[1] = as_bf16x8(w1);
+      }
+      // issue order: fragment reads ahead, then per MFMA one more read and a handful of vector instructions
+      __builtin_amdgcn_sched_group_barrier(0x100, FRAG_LEAD, 0);
+#pragma unroll
+      for (int i = 0; i < 2 * NP; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (i + FRAG_LEAD < 2 * NP) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, ((MASKED ? 6 : 4) - (LM ? 1 : 0) + (BIAS ? 1 : 0)) * 16 / NP, 0);
+      }
+    };
+
+    // K of tile tb (the first slot of the third pair-stage, free until the loop's first iteration is past its barrier), then two pairs
+#pragma unroll
+    for (int j = 0; j < PK; ++j) {
+      const int p = min(j * NWAVE + wave, Im::KPD - 1), row = (p * 64 + lane) / Im::CR, c = (p * 64 + lane) % Im::CR;
+      piece(p, tb, true, (CLAMP ? 0u : (unsigned)row * kv.k_row) + (unsigned)((c ^ Im::kx(row)) * 16), row, lds0 + 4u * Im::SLOT);
     }
-    if ((t + 1) * 32 > mlim) region(std::true_type{}, t, sc_a, sc_b); else region(std::false_type{}, t, sc_a, sc_b);
-    if ((t + 2) * 32 > mlim) region(std::true_type{}, t + 1, sc_b, sc_a); else region(std::false_type{}, t + 1, sc_b, sc_a);
-  }
-  if (active && te > tb) {     // the last tile's P.V (an empty key range never filled the ring: nothing to flush, and 0 x garbage = NaN)
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int j = 0; j < PWP; ++j) issue(j, tb + 2 * k, k);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PWP) : "memory");
+    __builtin_amdgcn_s_barrier();
+    if (active) {
+      asm volatile("" ::: "memory");
+      clear(tb, sc_a);
+#pragma unroll
+      for (int ks = 0; ks < KP; ++ks) sc_a = mfma32(as_bf16x8(kfrag(alds + 4 * Im::SLOT, ks)), as_bf16x8(qf[ks]), sc_a);
+      if (!bad) {
+        f32x16 x = sc_a;
+        mask(std::true_type{}, tb, x);
+        const float mx = xor32_max(lane_max(x));
+        m_ref = mx > -INFINITY ? ceilf(mx) : 0.f;
+        m_limit = mx > -INFINITY ? m_ref + slack : -INFINITY;
+      }
+    }
+    for (int t = tb; t < te; t += 2) {
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PWP) : "memory");
+      __builtin_amdgcn_s_barrier();
+      if (active) {
+        if (__builtin_amdgcn_ballot_w64(mx_pair > m_limit) != 0) {
+          const float mx = xor32_max(mx_pair);
+          const bool move = mx > m_limit;
+          bad = bad || (move && mx - m_ref > REF_JUMP);
+          const float to = move ? ceilf(mx) : m_ref, alpha = __builtin_amdgcn_exp2f(m_ref - to);      // a whole power of two: exact
+          m_ref = to; m_limit = move ? to + slack : m_limit;
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+          l_run *= alpha;
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            u32x4 w = as_u32x4(p_prev[i]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = pack2(lo2f(w[e]) * alpha, hi2f(w[e]) * alpha);
+            p_prev[i] = as_bf16x8(w);
+          }
+        }
+        if ((t + 2) * 32 > mlim) pair(std::true_type{}, t); else pair(std::false_type{}, t);
+      } else {
+#pragma unroll
+        for (int j = 0; j < PWP; ++j) issue(j, t + 4, st == 0 ? 2 : st - 1);
+      }
+      st = st == 2 ? 0 : st + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");     // all pieces: no LDS-DMA of this block may land after it has left the CU
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (active) {                // the last tile's P.V: its V^T is in the next pair's first slot
+      const unsigned char* slot = alds + 2 * st * Im::SLOT;
+#pragma unroll
+      for (int i = 0; i < VP; ++i) o[i >> 1] = mfma32(as_bf16x8(vfrag(slot, i)), p_prev[i & 1], o[i >> 1]);
+      const float mx = xor32_max(mx_pair);
+      bad = bad || mx - m_ref > REF_JUMP;
+      if (mx > m_limit && bad) { m_ref = ceilf(mx); m_limit = m_ref + slack; }
+    }
+    if (pass == 1) break;
+    const unsigned mine = __builtin_amdgcn_ballot_w64(active && bad) != 0 ? 1u : 0u;
+    unsigned* vote = reinterpret_cast<unsigned*>(alds + (2 * st + 1) * Im::SLOT);       // a K image that nobody reads any more
+    if (lane == 0) vote[wave] = mine;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    unsigned again = 0;
+#pragma unroll
+    for (int w = 0; w < NWAVE; ++w) again |= vote[w];
+    if (__builtin_amdgcn_readfirstlane(again) == 0u) break;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();                        // the ring is filled anew
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int ss = 0; ss < 2; ++ss) o[dt] = mfma32(as_bf16x8(v_prev[(KP + dt * 2 + ss) * 64 + lane]), p_prev[ss], o[dt]);
+      for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
+    l_run = 0.f;
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // no LDS-DMA of this block may land after it has left the CU
+  m_run = m_limit > -INFINITY ? m_ref : -INFINITY;
 }
 
 // ------------------------------------------------------------------------------------------------------------------------------
@@ -224,8 +349,8 @@ __global__ __launch_bounds__(NWAVE * 64, 2) void attn_gqa32_kernel(
     const int32_t* __restrict__ tile_q0, const int32_t* __restrict__ tile_nq, const int32_t* __restrict__ tile_pos0,
     bf16_t* const* __restrict__ kv_base, KvLayout lay, int layer, int heads, float scale_log2e, int nsplit,
     float* __restrict__ ws_o, float* __restrict__ ws_ml, int n_tiles, int xcd_chunks, int pack) {
-  constexpr int D = 128, KP = 8, VP = 8, NP = KP + VP, NSTAGE = 10, PW = (NP + NWAVE - 1) / NWAVE;
-  extern __shared__ __attribute__((aligned(16))) u32x4 alds[];      // NSTAGE x NP pieces of 1 KB in MFMA fragment (lane) order
+  constexpr int D = 128, KP = 8;
+  extern __shared__ __attribute__((aligned(16))) unsigned char alds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 31, hh = lane >> 5;
   const int n_items = n_tiles * lay.n_kv_heads * nsplit;
@@ -263,31 +388,8 @@ __global__ __launch_bounds__(NWAVE * 64, 2) void attn_gqa32_kernel(
     for (int ks = 0; ks < KP; ++ks) settle_load(qf[ks]);     // before the first LDS-DMA piece (common.h: glds16)
   }
 
-  // DMA sources of this wave's pieces for key tile 0 + per-tile strides (computed once: a DMA issue is one multiply-add per piece).
   // The KV cache is allocated in whole 32-key tiles, so the rows of the last (partial) tile exist and are masked.
-  const bf16_t* pbase[PW];
-  size_t pstride[PW];
-#pragma unroll
-  for (int j = 0; j < PW; ++j) {
-    const int p = min(j * NWAVE + wave, NP - 1);         // surplus slots re-fetch the last piece (same bytes, same place)
-    if (p < KP) {                                        // K piece ks = p: rows in swap23 order, 16 d per lane-half pair
-      pbase[j] = kbase + (size_t)swap23(col) * D + p * 16 + hh * 8;
-      pstride[j] = (size_t)32 * D;
-    } else {                                             // V^T piece (dt, s): V^T[d = dt * 32 + col][keys s * 16 + hh * 8 .. + 8]
-      const int dt = (p - KP) >> 1, s = (p - KP) & 1;
-      pbase[j] = vbase + (size_t)(dt * 32 + col) * 32 + s * 16 + hh * 8;
-      pstride[j] = (size_t)D * 32;
-    }
-  }
-  auto issue = [&](int t) {
-    const int tc = min(t, ntile - 1);
-    u32x4* sbase = alds + ((t - tb) % NSTAGE) * (NP * 64);
-#pragma unroll
-    for (int j = 0; j < PW; ++j) {
-      const int p = min(j * NWAVE + wave, NP - 1);
-      glds16((pbase[j] + (size_t)tc * pstride[j]), lds_addr(sbase + p * 64));
-    }
-  };
+  Kv32 kv; kv.k = kbase; kv.v = vbase; kv.k_row = D * 2; kv.v_row = 64; kv.k_tile = 32 * D * 2; kv.v_tile = D * 64; kv.ntile = ntile; kv.nkeys = nkeys;
 
   f32x16 o[4];
 #pragma unroll
@@ -298,7 +400,7 @@ __global__ __launch_bounds__(NWAVE * 64, 2) void attn_gqa32_kernel(
   int min_limit = key_limit;                             // wave-wide minimum of the key limits: tiles entirely below it need no mask
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) min_limit = min(min_limit, __shfl_xor(min_limit, off, 64));
-  attn32_key_loop<D, D, PW, false>(alds, issue, qf, tb, te, min(min_limit, te * 32), min(key_limit, te * 32), scale_log2e, active, lane, hh, o, m_run, l_run);
+  attn32_key_loop<D, D, NWAVE, false>(alds, kv, qf, tb, te, min(min_limit, te * 32), min(key_limit, te * 32), scale_log2e, active, lane, wave, hh, o, m_run, l_run);
   if (!active) return;
 
   float l = xor32_sum(l_run);
@@ -332,20 +434,25 @@ __global__ __launch_bounds__(NWAVE * 64, 2) void attn_gqa32_kernel(
 // ViT attention (Q2VL:375-417: non-causal inside each temporal slice, d = 80) on the same key loop.  grid = (groups of NWAVE x 32
 // query rows of ONE segment, heads): wave w owns the 32 rows q0 + 32 w of the group, all waves share the segment's K / V^T tiles of
 // this head through the ring.  d = 80 is 5 k-steps of the 32x32x16 MFMA for K.Q^T (no padding; the 16x16x32 kernel pads 80 -> 96)
-// and 3 d-tiles for O^T (the third half empty: its V^T rows 80..95 come from a zero page).  qkv = [P, 3E] with q, k rotated in place,
+// and 3 d-tiles for O^T (the third half empty: ones, see LM).  qkv = [P, 3E] with q, k rotated in place,
 // vt = V blocked-transposed [head][32-key block][80][32] (vit_rope_vt_kernel); keys past the segment end are masked, and the K rows of
 // the last (partial) tile are clamped into the segment (the next segment's rows are NOT part of this attention).
-// (the 4-wave instantiation keeps one wave per SIMD and the AGPR form: capped at 256 registers it spills 52 bytes; it is an opt-in variant,
-// LCC_VIT32_MIN_BLOCKS4, and its 118 accumulator copies per region are what made it lose to the 8-wave form in rounds 3 and 6)
-template <int NWAVE, bool LM>
+// NWAVE 4: two blocks share a compute unit (67,584 bytes of LDS each), so one's ends hide behind the other, and 880 rows are 7 groups of 128 instead of 4 of 256:
+// 18 slices of 880 113 us against 138, 40 of 400 83 / 92, 8 of 1,456 119 / 122.  NWAVE 8 serves calls under a grid cap (one block a unit).
+template <int NWAVE>
 __global__ __launch_bounds__(NWAVE * 64, 2) void attn_vit32_kernel(
     const bf16_t* __restrict__ qkv, const bf16_t* __restrict__ vt, bf16_t* __restrict__ out, const int32_t* __restrict__ grp_seg,
     const int32_t* __restrict__ grp_q0, const int32_t* __restrict__ seg_start, const int32_t* __restrict__ seg_len,
     const int32_t* __restrict__ seg_blk_start, int heads, int total_blocks, float scale_log2e, int n_groups, int xcd_chunks) {
-  constexpr int D = 80, KP = 5, DT = 3, VP = 6, NP = KP + VP, NSTAGE = 10, PW = (NP + NWAVE - 1) / NWAVE;
-  extern __shared__ __attribute__((aligned(16))) u32x4 alds[];
+  constexpr int D = 80, KP = 5, DT = 3;
+  using Im = Attn32Image<D, D>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char alds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 31, hh = lane >> 5;
+  // V^T rows 80..95 of the third d-tile do not exist: ones in every slot (the DMA copies rows 0..79), so O^T rows 80..95 = sum of P
+  for (int i = threadIdx.x; i < 6 * 64; i += NWAVE * 64)
+    *reinterpret_cast<u32x4*>(alds + (i >> 6) * Im::SLOT + Im::KB + 80 * 64 + (i & 63) * 16) = (u32x4){0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // before the key loop's first barrier
   // one (group, head) per block, or a persistent walk under the grid cap (gemm.hip: g_grid_cap): virtual block vb = head * n_groups + group.
   // xcd_chunks (round 6): the virtual blocks are dealt to the 8 XCDs in contiguous chunks (block b runs on XCD b % 8: speed only), so the
   // ~6 row groups that read the same segment's K / V of one head share ONE L2 instead of landing on six
@@ -371,45 +478,15 @@ __global__ __launch_bounds__(NWAVE * 64, 2) void attn_vit32_kernel(
 #pragma unroll
     for (int ks = 0; ks < KP; ++ks) settle_load(qf[ks]);     // before the first LDS-DMA piece (common.h: glds16)
   }
-  // DMA sources: ONE 32-bit element offset per piece and lane from the wave-uniform base of the piece (K: kbase, V^T: vbase) -- the piece
-  // index is wave-uniform, so base and per-tile stride stay in SGPRs (round 6: the 64-bit pointer + stride + row per piece of the first
-  // version cost 5 VGPRs per piece in a kernel that sits at the 256-register limit).  V^T rows 80..95 of the third d-tile do not exist:
-  // their lanes fetch row 79 again (finite values; the output rows >= 80 are never stored).
-  const int krow = swap23(col);
-  unsigned poff[PW];
-#pragma unroll
-  for (int j = 0; j < PW; ++j) {
-    const int p = min(j * NWAVE + wave, NP - 1);
-    if (p < KP) {
-      poff[j] = (unsigned)(krow * ld + p * 16 + hh * 8);
-    } else {
-      const int dt = (p - KP) >> 1, s = (p - KP) & 1, d = min(dt * 32 + col, D - 1);
-      poff[j] = (unsigned)(d * 32 + s * 16 + hh * 8);
-    }
-  }
-  auto issue = [&](int t) {
-    const int tc = min(t, ntile - 1);
-    u32x4* sbase = alds + (t % NSTAGE) * (NP * 64);
-#pragma unroll
-    for (int j = 0; j < PW; ++j) {
-      const int p = min(j * NWAVE + wave, NP - 1);
-      const bool isk = p < KP;                           // wave-uniform
-      const bf16_t* src = (isk ? kbase + (size_t)tc * (32 * ld) : vbase + (size_t)tc * (D * 32)) + poff[j];
-      if (isk && tc == ntile - 1)                        // last tile: rows past the segment end are clamped (and masked)
-        src = kbase + (size_t)min(tc * 32 + krow, nkeys - 1) * ld + p * 16 + hh * 8;
-      if (LM && p >= KP + 4 && col >= 16)                // V^T rows 80..95 (third d-tile, upper half): ones -> O^T rows 80..95 = sum of P
-        src = reinterpret_cast<const bf16_t*>(lcc_attn32_ones_page) + lane * 8;
-      glds16(src, lds_addr(sbase + p * 64));
-    }
-  };
+  Kv32 kv; kv.k = kbase; kv.v = vbase; kv.k_row = (unsigned)ld * 2; kv.v_row = 64; kv.k_tile = (size_t)64 * ld; kv.v_tile = D * 64; kv.ntile = ntile; kv.nkeys = nkeys;
   f32x16 o[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;
-  attn32_key_loop<D, D, PW, LM>(alds, issue, qf, 0, ntile, sl, sl, scale_log2e, active, lane, hh, o, m_run, l_run);
-  const float l = LM ? o[2][8] : xor32_sum(l_run);       // LM: row 80 + 4 hh of O^T, every one of rows 80..95 holds the sum over ALL keys
+  attn32_key_loop<D, D, NWAVE, true, false, true>(alds, kv, qf, 0, ntile, sl, sl, scale_log2e, active, lane, wave, hh, o, m_run, l_run);
+  const float l = o[2][8];                               // row 80 + 4 hh of O^T, every one of rows 80..95 holds the sum over ALL keys
   if (active && col < nq) {
     const float inv = 1.f / l;
     bf16_t* op = out + (size_t)(s0 + q0 + col) * E + h * D;
@@ -426,23 +503,17 @@ __global__ __launch_bounds__(NWAVE * 64, 2) void attn_vit32_kernel(
   }
 }
 
-// LCC_VIT32_LSUM_MFMA (A/B, read once): 1 = the tower kernel takes its softmax denominator from the P . V MFMAs (LM above), 0 = vector adds
-static int vit32_lsum_mfma() {
-  static const int v = [] { const char* e = getenv("LCC_VIT32_LSUM_MFMA"); return e ? atoi(e) : 1; }();
-  return v;
-}
-
-template <int NWAVE, bool LM>
+template <int NWAVE>
 static void vit32_launch_t(const bf16_t* qkv, const bf16_t* vt, bf16_t* out, const int32_t* grp_seg, const int32_t* grp_q0, const int32_t* seg_start,
                            const int32_t* seg_len, const int32_t* seg_blk_start, int n_groups, int heads, int total_blocks, float scale_log2e, hipStream_t st) {
-  constexpr size_t lds = (size_t)10 * 11 * 1024;
+  constexpr size_t lds = Attn32Image<80, 80>::BYTES;
   static DeviceOnce once;   // per instantiation
-  if (once.first()) (void)hipFuncSetAttribute((const void*)attn_vit32_kernel<NWAVE, LM>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (once.first()) (void)hipFuncSetAttribute((const void*)attn_vit32_kernel<NWAVE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   const long nvb = (long)n_groups * heads;
   const int cap = get_grid_cap();
   static const int xcd = [] { const char* v = getenv("LCC_ATTN32_XCD"); return v ? atoi(v) : 1; }();      // A/B: 0 = virtual block = physical block
   const long nb = (cap > 0 && nvb > cap) ? cap : (xcd ? (nvb + 7) / 8 * 8 : nvb);      // (the cap is a multiple of 8: gemm.hip set_grid_cap)
-  attn_vit32_kernel<NWAVE, LM><<<dim3((unsigned)nb), dim3(NWAVE * 64), lds, st>>>(
+  attn_vit32_kernel<NWAVE><<<dim3((unsigned)nb), dim3(NWAVE * 64), lds, st>>>(
       qkv, vt, out, grp_seg, grp_q0, seg_start, seg_len, seg_blk_start, heads, total_blocks, scale_log2e, n_groups, xcd);
 }
 int attn_vit32_launch(const bf16_t* qkv, const bf16_t* vt, bf16_t* out, const int32_t* grp_seg, const int32_t* grp_q0,
@@ -450,11 +521,9 @@ int attn_vit32_launch(const bf16_t* qkv, const bf16_t* vt, bf16_t* out, const in
                       int total_blocks, float scale_log2e, hipStream_t st, int group_rows) {
   if (n_groups <= 0) return 0;
   if (group_rows != 256 && group_rows != 128) return LCC_ERR_ARG;
-  // group_rows 256: 8 waves x 32 rows per block; 128: 4 waves (one per SIMD) -- twice the blocks for a grid that does not fill the chip
-#define LCC_VIT32_GO(NW, LMV) vit32_launch_t<NW, LMV>(qkv, vt, out, grp_seg, grp_q0, seg_start, seg_len, seg_blk_start, n_groups, heads, total_blocks, scale_log2e, st)
-  if (vit32_lsum_mfma()) { if (group_rows == 256) LCC_VIT32_GO(8, true); else LCC_VIT32_GO(4, true); }
-  else { if (group_rows == 256) LCC_VIT32_GO(8, false); else LCC_VIT32_GO(4, false); }
-#undef LCC_VIT32_GO
+  // group_rows 256: 8 waves x 32 rows per block; 128: 4 waves, two blocks a compute unit
+  auto go = [&](auto nw) { vit32_launch_t<decltype(nw)::value>(qkv, vt, out, grp_seg, grp_q0, seg_start, seg_len, seg_blk_start, n_groups, heads, total_blocks, scale_log2e, st); };
+  if (group_rows == 256) go(std::integral_constant<int, 8>{}); else go(std::integral_constant<int, 4>{});
   g_launch_counts[LC_ATTN_VIT32] += 1;
   return 0;
 }
@@ -515,7 +584,7 @@ int attn_prefill32_launch(const bf16_t* q, bf16_t* out, const int32_t* tile_stre
                           int nsplit, float* ws_o, float* ws_ml, float scale_log2e, hipStream_t st) {
   const int G = n_q_heads / lay.n_kv_heads;
   if (G < 1 || G > 8 || lay.head_dim != 128) return LCC_ERR_SHAPE;
-  constexpr size_t lds = (size_t)10 * 16 * 1024;
+  constexpr size_t lds = Attn32Image<128, 128>::BYTES;
   static DeviceOnce once;
   if (once.first()) {
     (void)hipFuncSetAttribute((const void*)attn_gqa32_kernel<8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -546,8 +615,8 @@ int attn_prefill32_launch(const bf16_t* q, bf16_t* out, const int32_t* tile_stre
 // SLOTS: keys and values out of the slots' arenas, shared by the query heads of a KV head, and a distance bias per head (kernels.h: MhaArgs).
 template <int DK, int DV, bool SLOTS>
 __global__ __launch_bounds__(512, 2) void attn_mha32_kernel(MhaArgs a) {
-  constexpr int NWAVE = 8, KP = DK / 16, DT = DV / 32, VP = 2 * DT, NP = KP + VP, NSTAGE = 10, PW = (NP + NWAVE - 1) / NWAVE;
-  extern __shared__ __attribute__((aligned(16))) u32x4 alds[];
+  constexpr int NWAVE = 8, KP = DK / 16, DT = DV / 32;
+  extern __shared__ __attribute__((aligned(16))) unsigned char alds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 31, hh = lane >> 5;
   const int n_items = a.n_groups * a.heads;
@@ -580,28 +649,17 @@ __global__ __launch_bounds__(512, 2) void attn_mha32_kernel(MhaArgs a) {
 #pragma unroll
     for (int ks = 0; ks < KP; ++ks) settle_load(qf[ks]);     // before the first LDS-DMA piece (common.h: glds16)
   }
-  const bf16_t* pbase[PW];
-  size_t pstride[PW];
+  // the key loop takes a positive scale: a negative one turns the sign of q, none at all leaves the bias alone
+  float scale = a.scale_log2e;
+  if (scale <= 0.f) {
 #pragma unroll
-  for (int j = 0; j < PW; ++j) {
-    const int p = min(j * NWAVE + wave, NP - 1);         // surplus slots re-fetch the last piece (same bytes, same place)
-    if (p < KP) {
-      pbase[j] = kbase + (size_t)swap23(col) * ldk + p * 16 + hh * 8;
-      pstride[j] = (size_t)32 * ldk;
-    } else {
-      const int dt = (p - KP) >> 1, s = (p - KP) & 1;
-      pbase[j] = vbase + (size_t)(dt * 32 + col) * ldv + s * 16 + hh * 8;
-      pstride[j] = SLOTS ? (size_t)DV * 32 : 32;
-    }
+    for (int ks = 0; ks < KP; ++ks)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) qf[ks][e] = scale < 0.f ? qf[ks][e] ^ 0x80008000u : 0u;
+    scale = scale < 0.f ? -scale : 1.f;
   }
-  int tb = 0;
-  asm volatile("" : "+s"(tb));      // opaque: with a known first tile hipcc splits the ring's index arithmetic into registers it then spills
-  auto issue = [&](int t) {
-    const int tc = min(t, ntile - 1);
-    u32x4* sbase = alds + ((t - tb) % NSTAGE) * (NP * 64);
-#pragma unroll
-    for (int j = 0; j < PW; ++j) glds16(pbase[j] + (size_t)tc * pstride[j], lds_addr(sbase + min(j * NWAVE + wave, NP - 1) * 64));
-  };
+  Kv32 kv; kv.k = kbase; kv.v = vbase; kv.k_row = (unsigned)ldk * 2; kv.v_row = (unsigned)ldv * 2; kv.k_tile = (size_t)64 * ldk; kv.v_tile = SLOTS ? (size_t)DV * 64 : 64;
+  kv.ntile = ntile; kv.nkeys = pos0 + nq;
   f32x16 o[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -612,7 +670,7 @@ __global__ __launch_bounds__(512, 2) void attn_mha32_kernel(MhaArgs a) {
   int min_limit = pos0 + min(wave * 32, nq - 1) + 1;            // of the wave's first row
   asm volatile("" : "+v"(min_limit));
   const float slope = SLOTS && a.slope ? a.slope[h] : 0.f;
-  attn32_key_loop<DK, DV, PW, false, SLOTS>(alds, issue, qf, tb, ntile, min_limit, key_limit, a.scale_log2e, active, lane, hh, o, m_run, l_run, slope, pos0 + qr);
+  attn32_key_loop<DK, DV, NWAVE, false, SLOTS>(alds, kv, qf, 0, ntile, min_limit, key_limit, scale, active, lane, wave, hh, o, m_run, l_run, slope, pos0 + qr);
   if (!active) return;
   const float l = xor32_sum(l_run);
   if (valid) {
@@ -627,7 +685,7 @@ __global__ __launch_bounds__(512, 2) void attn_mha32_kernel(MhaArgs a) {
 }
 template <int DK, int DV, bool SLOTS>
 static void mha32_go(const MhaArgs& a, hipStream_t st) {
-  constexpr size_t lds = (size_t)10 * (DK / 16 + 2 * (DV / 32)) * 1024;
+  constexpr size_t lds = Attn32Image<DK, DV>::BYTES;
   static DeviceOnce once;   // per instantiation
   if (once.first()) (void)hipFuncSetAttribute((const void*)attn_mha32_kernel<DK, DV, SLOTS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   const long n_items = (long)a.n_groups * a.heads;

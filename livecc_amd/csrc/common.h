@@ -57,10 +57,14 @@ LCC_DEVICE void glds16(const void* gsrc, unsigned lds_dst) {
   asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" LCC_GLDS_POLICY "\n\ts_mov_b32 m0, %0"
                : "=&s"(keep) : "v"(gsrc), "s"(__builtin_amdgcn_readfirstlane(lds_dst)) : "memory");   // readfirstlane: free when provably uniform
 }
-// the same from a base that is uniform in the wave and a byte offset per lane
-LCC_DEVICE void glds16_base(const void* base, unsigned off, unsigned lds_dst) {
+// the same from a base that is uniform in the wave and a byte offset per lane (s_nop 2: five wait states between a vector instruction that wrote
+// the base's registers -- readfirstlane -- and the load that reads them)
+LCC_DEVICE void glds16_base(const void* uniform_base, unsigned off, unsigned lds_dst) {
   unsigned keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" LCC_GLDS_POLICY "\n\ts_mov_b32 m0, %0"
+  const unsigned long long b = reinterpret_cast<unsigned long long>(uniform_base);
+  const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32)), lo = __builtin_amdgcn_readfirstlane((unsigned)b);      // the builtin is signed: through 32 unsigned bits
+  const unsigned long long base = (unsigned long long)hi << 32 | lo;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 2\n\tglobal_load_lds_dwordx4 %1, %2" LCC_GLDS_POLICY "\n\ts_mov_b32 m0, %0"
                : "=&s"(keep) : "v"(off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(lds_dst)) : "memory");
 }
 // Make the compiler wait HERE for a plain global load it is tracking (it must insert its own s_waitcnt in front of a statement that reads

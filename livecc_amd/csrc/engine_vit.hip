@@ -48,7 +48,7 @@ extern "C" int lcc_vit_encode(lcc_engine* e, int n_clips, const lcc_clip* clips,
       seg_start.push_back(P); seg_len.push_back(n); seg_blk.push_back(blocks);
       for (int q = 0; q < n; q += 32) { tile_seg.push_back(sg); tile_q0.push_back(q); }
       for (int q = 0; q < n; q += 128) { grp_seg.push_back(sg); grp_q0.push_back(q); }
-      for (int q = 0; q < n; q += 256) { g8_seg.push_back(sg); g8_q0.push_back(q); }     // attention variant 3: 8 waves x 32 rows
+      for (int q = 0; q < n; q += 256) { g8_seg.push_back(sg); g8_q0.push_back(q); }     // attention variant 3 under a grid cap: 8 waves x 32 rows
       seg_of_patch.insert(seg_of_patch.end(), n, sg);
       P += n; blocks += (n + 31) / 32;
     }
@@ -141,21 +141,13 @@ extern "C" int lcc_vit_encode(lcc_engine* e, int n_clips, const lcc_clip* clips,
       LCC_TRY(gemm_bf16(g, st));
       LCC_TRY(vit_rope_vt_bf16(qkv, rope_cos, rope_sin, d_seg_of_patch, d_seg_start, d_seg_blk, vt, P, heads, blocks, st));
     }
-    // 32x32x16 kernel (8 waves x 32 rows per block) once its grid fills the chip: 8 streams' chunks = 768 blocks, 170 vs 359 us per
-    // block of the tower; ONE 2-frame chunk is only 6 groups x 16 heads = 96 blocks (49 us) -- there the 16-row-per-wave LDS-shared
-    // kernel with twice the blocks stays (41 us)
-    // (the 4-wave form of the 32x32x16 kernel -- 128-row groups, 192 blocks for one chunk -- measured the same as the 16-row kernel:
-    // 261.6 vs 262.1 tokens/s without prefetch, profiles/r03/knob_sweeps_call11_13.txt; off unless LCC_VIT32_MIN_BLOCKS4 says otherwise)
-    // Round 6: that instantiation had been compiled in the AGPR form (118 accumulator copies per region, tools/audit_agpr_copies.py); in the
-    // VGPR form it beats the 16-row kernel on one chunk (192 blocks): tower 5.20 -> 5.02 ms (profiles/r06/tower_4wave_vgprform_ab.jsonl), so
-    // grids of >= 128 four-wave blocks that are too small for the 8-wave form now take it.
-    static const int vit32_min4 = [] { const char* v = getenv("LCC_VIT32_MIN_BLOCKS4"); return v ? atoi(v) : 128; }();
-    if (get_attn_variant() == 3 && e->vit_hd == 80 && (long)n_groups8 * heads >= 224)
-      LCC_TRY(attn_vit32_launch(qkv, vt, attn, d_g8_seg, d_g8_q0, d_seg_start, d_seg_len, d_seg_blk, n_groups8, heads, blocks,
-                                1.4426950408889634f / sqrtf(80.f), st, 256));
-    else if (get_attn_variant() == 3 && e->vit_hd == 80 && (long)n_groups * heads >= vit32_min4)   // 128-row groups: 4 waves, one per SIMD
-      LCC_TRY(attn_vit32_launch(qkv, vt, attn, d_grp_seg, d_grp_q0, d_seg_start, d_seg_len, d_seg_blk, n_groups, heads, blocks,
-                                1.4426950408889634f / sqrtf(80.f), st, 128));
+    // 32x32x16 kernel, 128 rows a block and two blocks a compute unit (256 rows under a grid cap, where a unit has one block).  The 16-row kernel keeps
+    // the few short slices a launch of which is nearly all latency: one slice of 140 / 280 / 420 / 720 patches 8.9 / 11.6 / 15.1 / 22.7 us there, 9.4 / 11.2 / 13.1 / 18.0 here.
+    const bool vit32 = get_attn_variant() == 3 && e->vit_hd == 80 && ((long)n_groups * heads >= 128 || P >= 256 * n_seg);
+    const bool wide = vit32 && get_grid_cap() > 0 && (long)n_groups8 * heads >= 224;
+    if (vit32)
+      LCC_TRY(attn_vit32_launch(qkv, vt, attn, wide ? d_g8_seg : d_grp_seg, wide ? d_g8_q0 : d_grp_q0, d_seg_start, d_seg_len, d_seg_blk, wide ? n_groups8 : n_groups,
+                                heads, blocks, 1.4426950408889634f / sqrtf(80.f), st, wide ? 256 : 128));
     else
       LCC_TRY(attn_vit_bf16(qkv, vt, attn, d_tile_seg, d_tile_q0, d_seg_start, d_seg_len, d_seg_blk, n_tiles, heads, blocks, d_grp_seg, d_grp_q0,
                             n_groups, st));

@@ -196,6 +196,29 @@ def test_biased_attention_of_packed_streams(dev, lib, dim, vdim, heads, kv, new,
         row += n
 
 
+@pytest.mark.parametrize("dim,vdim", [(128, 128), (64, 128)])
+@pytest.mark.parametrize("scale,slopes", [(-0.06, True), (0.0, True), (0.06, False), (0.02, True)])
+def test_biased_attention_with_any_scale(dev, lib, dim, vdim, scale, slopes):
+    """A negative scale, none at all (the bias alone), no bias; steep slopes over 400 keys."""
+    g = torch.Generator().manual_seed(7)
+    n, p, heads = 130, 270, 2
+    kvs, arenas, base, k_off, v_off = _kv_slots([n], 1, dim, vdim, 416, dev, g)
+    q = torch.randn(n, heads, dim, generator=g).bfloat16()
+    slope = torch.tensor([0.9, 0.01]) if slopes else torch.zeros(2)
+    qd, sl = q.to(dev), (slope * SLOPES_LOG2).float().to(dev)
+    out = torch.full((n, heads * vdim), 7.0, dtype=torch.bfloat16, device=dev)
+    tabs = [_i32([x], dev) for x in (0, n, p, 0)]
+    _ok(lib.lcc_gqa_attn_prefill(_p(qd), _p(out), *[_p(t) for t in tabs], 1, n, heads, 1, dim, vdim, scale, _p(sl) if slopes else None, _p(base), k_off, v_off,
+                                 416, _st()))
+    k, v = (t[0, :p + n].double() for t in kvs[0])
+    at = torch.arange(p + n)
+    for h in range(heads):
+        dist = (at[p:, None] - at[None]).double()
+        s = q[:, h].double() @ k.T * scale - float(slope[h]) * dist
+        want = torch.softmax(s.masked_fill(dist < 0, -torch.inf), -1) @ v
+        assert (out.view(n, heads, vdim)[:, h].double().cpu() - want).abs().max() < 0.03, h
+
+
 @pytest.mark.parametrize("dim,vdim,heads,kv,lens,ns", [(64, 64, 6, 1, [1, 2, 31, 32, 33, 64, 65], 2), (128, 128, 12, 2, [700], 11), (128, 64, 34, 2, [64] * 18, 1),
                                                        (192, 256, 3, 3, [200, 10], 4), (256, 128, 2, 1, [65], 64), (256, 256, 4, 2, [500, 1, 63], 3), (64, 192, 5, 5, [97], 3)])
 def test_biased_decode_attention(dev, lib, dim, vdim, heads, kv, lens, ns):

@@ -674,6 +674,51 @@ def test_vit_rope_attention(dev, grids, attn_variant):
         assert torch.equal(got4, got), "a query row's arithmetic does not depend on the group size"
 
 
+@pytest.mark.parametrize("Hq,Hkv,S,past,nsplit", [(28, 4, 70, 200, 1), (28, 4, 70, 330, 2), (8, 2, 33, 95, 1)])
+def test_prefill_attention_of_rows_whose_scores_jump(dev, Hq, Hkv, S, past, nsplit):
+    """Rows whose score jumps by far more than a power of 2^100 behind the first key tiles (the 32x32x16 kernel goes through its keys a second
+    time), rises from pair to pair, or falls from the first key on; the rows beside them keep their bits."""
+    from livecc_amd import ops
+    D, L = 128, S + past
+    kv = ops.KvArena(1, 1, Hkv, (L + 31) // 32 * 32, dev)
+    kv.buf.copy_(_rand(tuple(kv.buf.shape), dev, 0.7, 5))
+    K, V = kv.k_view(0, 0)[:, :L].float().transpose(0, 1), kv.v_view(0, 0)[:, :L].float().transpose(0, 1)
+    q = _rand((S, Hq * D), dev, 1.0, 6)
+    plain = ops.attn_prefill(q, kv, 0, [(0, S, past)], Hq, tile_rows=32, nsplit=nsplit)
+    q2 = q.clone().view(S, Hq, D)
+    loud = {3: 90, 17: 0, S - 1: L - 1, S - 2: past // 2}
+    for i, j in loud.items():
+        for h in range(Hq):
+            q2[i, h] = (K[j, h * Hkv // Hq] * 40).bfloat16()          # about 220 / 0.69 in powers of two
+    q2 = q2.view(S, Hq * D)
+    got = ops.attn_prefill(q2, kv, 0, [(0, S, past)], Hq, tile_rows=32, nsplit=nsplit)
+    _check_attn(got.view(S, Hq, D), rb(_ref_attn_causal(q2.float().view(S, Hq, D), K, V, past)), f"jump[{Hq},{S},{past},{nsplit}]")
+    same = [i for i in range(S) if i not in loud]
+    assert torch.equal(got[same], plain[same])
+
+
+@pytest.mark.parametrize("rows", [128, 256])
+def test_vit_attention_of_rows_whose_scores_jump(dev, rows):
+    from livecc_amd import ops
+    heads, D, grids = 2, 80, [(1, 10, 14), (1, 14, 20)]
+    P, E = 420, 160
+    one, zero = torch.ones(P, 40, device=dev), torch.zeros(P, 40, device=dev)
+    qkv = _rand((P, 3 * E), dev, 1.0, 7)
+    plain = ops.vit_attention(qkv.clone(), one, zero, grids, heads, group_rows=rows)
+    loud = {5: 100, 139: 0, 150: 419, 300: 141}
+    for i, j in loud.items():
+        qkv[i, :E] = qkv[j, E:2 * E] * 30
+    got = ops.vit_attention(qkv.clone(), one, zero, grids, heads, group_rows=rows)
+    q, k, v = (x.reshape(P, heads, D).float() for x in qkv.float().split(E, dim=1))
+    ref = torch.zeros(P, heads, D, device=dev)
+    for a, b in ((0, 140), (140, 420)):
+        for h in range(heads):
+            ref[a:b, h] = torch.softmax(q[a:b, h] @ k[a:b, h].T.contiguous() / math.sqrt(D), -1) @ v[a:b, h]
+    _check_attn(got.view(P, heads, D), rb(ref), f"vit jump[{rows}]")
+    same = [i for i in range(P) if i not in loud]
+    assert torch.equal(got[same], plain[same])
+
+
 def _hf_mrope_ref(pos3, theta=1e6):
     inv = 1.0 / (theta ** (torch.arange(0, 128, 2, dtype=torch.float) / 128))
     freqs = pos3.float()[:, :, None] * inv[None, None, :]          # [3,S,64]
