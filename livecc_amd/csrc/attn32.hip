@@ -57,7 +57,7 @@ LCC_DEVICE float xor32_sum(float x) {
 //
 // An iteration is ONE basic block -- 2 x NP MFMAs, every fragment read FRAG_LEAD MFMAs ahead of its use, the DMA pieces of pair P+3 spread between
 // them -- because the softmax has no branch: probabilities are taken against a reference that is only moved between two pairs.
-//   * Reference: the ceiling of the row's maximum over its first key tile (log2 units); moved to the ceiling of the maximum so far when a
+//   * Reference: the row's maximum over its first key tile (log2 units); moved up by the whole number that reaches the maximum so far when a
 //     pair held a score more than `slack` above it.  Until then probabilities are up to 2^slack (fp32 and bf16 hold the exponent; numerator and denominator carry
 //     the same factor), and moving by a whole number of powers of two is exact on O, l and the pending P.  The running maximum itself moves in nearly
 //     every tile of a short key range (32 rows, each with chance 1 / t in tile t): a rescale of O behind the MFMAs, a maximum that every exponential
@@ -83,6 +83,11 @@ LCC_DEVICE float xor32_sum(float x) {
 // probabilities the numerator uses (fp32 accumulation either way).
 // D = channels of q / k, DV = channels of v.  BIAS: slope (pos - key) is taken off the scaled scores (slope in units of log2), pos = this lane's query:
 // K.Q^T is added to it instead of to zero.
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
+LCC_DEVICE float dot_ones(unsigned pair, float c) {          // c + both bf16 halves of `pair`
+  const unsigned ones = 0x3F803F80u;
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, pair), __builtin_bit_cast(bf16x2_t, ones), c, false);
+}
 struct Kv32 {                   // keys and values of one (stream, head); all wave-uniform
   const bf16_t *k, *v;          // tile 0
   unsigned k_row, v_row;        // bytes between keys of K, between channels of V^T
@@ -204,12 +209,12 @@ LCC_DEVICE void attn32_key_loop(unsigned char* alds, const Kv32& kv, const u32x4
         float p[16];
 #pragma unroll
         for (int e = 0; e < 16; ++e) p[e] = __builtin_amdgcn_exp2f(fmaf(x[e], scale_log2e, -m_ref));   // masked scores are -inf -> 0
-        if (!LM) {
-#pragma unroll
-          for (int e = 0; e < 16; ++e) l_run += p[e];
-        }
         u32x4 w0 = {pack2(p[0], p[1]), pack2(p[2], p[3]), pack2(p[4], p[5]), pack2(p[6], p[7])};
         u32x4 w1 = {pack2(p[8], p[9]), pack2(p[10], p[11]), pack2(p[12], p[13]), pack2(p[14], p[15])};
+        if (!LM) {          // the denominator takes the probabilities as the numerator does, rounded
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { l_run = dot_ones(w0[e], l_run); l_run = dot_ones(w1[e], l_run); }
+        }
         // matrix pipe
 #pragma unroll
         for (int w = 0; w < NP; ++w) {
@@ -260,7 +265,7 @@ LCC_DEVICE void attn32_key_loop(unsigned char* alds, const Kv32& kv, const u32x4
         f32x16 x = sc_a;
         mask(std::true_type{}, tb, x);
         const float mx = xor32_max(lane_max(x));
-        m_ref = mx > -INFINITY ? ceilf(mx) : 0.f;
+        m_ref = mx > -INFINITY ? mx : 0.f;
         m_limit = mx > -INFINITY ? m_ref + slack : -INFINITY;
       }
     }
@@ -272,7 +277,7 @@ LCC_DEVICE void attn32_key_loop(unsigned char* alds, const Kv32& kv, const u32x4
           const float mx = xor32_max(mx_pair);
           const bool move = mx > m_limit;
           bad = bad || (move && mx - m_ref > REF_JUMP);
-          const float to = move ? ceilf(mx) : m_ref, alpha = __builtin_amdgcn_exp2f(m_ref - to);      // a whole power of two: exact
+          const float to = move ? m_ref + ceilf(mx - m_ref) : m_ref, alpha = __builtin_amdgcn_exp2f(m_ref - to);      // a whole power of two: exact
           m_ref = to; m_limit = move ? to + slack : m_limit;
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt)
@@ -303,7 +308,7 @@ LCC_DEVICE void attn32_key_loop(unsigned char* alds, const Kv32& kv, const u32x4
       for (int i = 0; i < VP; ++i) o[i >> 1] = mfma32(as_bf16x8(vfrag(slot, i)), p_prev[i & 1], o[i >> 1]);
       const float mx = xor32_max(mx_pair);
       bad = bad || mx - m_ref > REF_JUMP;
-      if (mx > m_limit && bad) { m_ref = ceilf(mx); m_limit = m_ref + slack; }
+      if (mx > m_limit && bad) { m_ref = mx; m_limit = m_ref + slack; }
     }
     if (pass == 1) break;
     const unsigned mine = __builtin_amdgcn_ballot_w64(active && bad) != 0 ? 1u : 0u;
