@@ -969,17 +969,22 @@ __global__ __launch_bounds__(512) void gemm_big_kernel(
 // with SwiGLU 903 -> 862; 4096 x 18944 fp32, K 3584 473 -> 454.  What is left is the matrix pipe at the clock that the chip holds under it.
 // Bits as gemm_big_kernel (same k order per output).  bf16 weights; every epilogue but the vision q|k|v ones, whose rotation tables need
 // the stages.  Grid: at most 256 blocks over all splits (one a compute unit), or the cap.
+constexpr int walk_stages(int bm) { return bm >= 192 ? 2 : 3; }
+constexpr bool walk_epilogue_own(int bm) { return bm != 160; }                   // three stages of 160 rows leave no room
+constexpr int walk_epilogue_rows(int bm, int epi) { return bm >= 160 && epi != EPI_GELU_ERF ? 2 : 1; }      // (the erf: registers)
+constexpr size_t walk_lds(int bm, int epi) { return (size_t)walk_stages(bm) * (bm * 8 + 2048) * 16 + (walk_epilogue_own(bm) ? 8 * walk_epilogue_rows(bm, epi) * 2048 : 0); }
 template <int BM, int EPI>
 __global__ __launch_bounds__(512) void gemm_walk_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
     const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
     bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n,
     float* __restrict__ partial, int kt_per_split, const float* __restrict__ wscale, int raster) {
-  constexpr int BN = 256, BK = 64, NSTAGE = BM >= 192 ? 2 : 3;
+  constexpr int BN = 256, BK = 64, NSTAGE = walk_stages(BM);
   constexpr int WM = BM / 2, MT = WM / 16, NT = 4;
   constexpr int A_UNITS = BM * 8, STAGE = A_UNITS + 2048;        // 16-byte units: activations, then 32 weight sub-tiles
-  constexpr int APW = BM / 64, BPW = 4, G = APW + BPW;           // DMA pieces of a wave per k-tile
-  constexpr int EGR = BM >= 192 && EPI != EPI_GELU_ERF ? 2 : 1;  // row tiles of an epilogue group: 4 / 2 KB of LDS a wave (the erf: registers)
+  constexpr int APW = (BM + 63) / 64, BPW = 4, G = APW + BPW;    // DMA pieces of a wave per k-tile (surplus ones copy the last rows again)
+  constexpr int EGR = walk_epilogue_rows(BM, EPI);               // row tiles of an epilogue group: 4 / 2 KB of LDS a wave
+  constexpr bool OWN = walk_epilogue_own(BM);                    // ... behind the stages, or the stage that was multiplied last, behind a barrier
   constexpr int NSTORE = EPI == EPI_PARTIAL ? MT * 4 : MT * 2;   // stores of a wave in the epilogue of an inner tile
   extern __shared__ __attribute__((aligned(16))) u32x4 dsmem[];
 
@@ -1020,10 +1025,10 @@ __global__ __launch_bounds__(512) void gemm_walk_kernel(
     for (int q = 0; q < BPW / 2; ++q) bbase[q] = W + (size_t)min((n0 >> 4) + wave * (BPW / 2) + q, nfrag - 1) * K32 * 512;
 #pragma unroll
     for (int q = 0; q < APW; ++q)
-      aoffs[q] = (unsigned)min((wave * APW + q) * 8 + (lane >> 3), M - 1 - m0) * (unsigned)(lda * 2) + (((lane & 7) ^ (lane >> 3)) << 4);
+      aoffs[q] = (unsigned)min(min(wave * APW + q, BM / 8 - 1) * 8 + (lane >> 3), M - 1 - m0) * (unsigned)(lda * 2) + (((lane & 7) ^ (lane >> 3)) << 4);
   };
   auto piece = [&](int t, unsigned base) {            // base: LDS byte address of the stage
-    if (t < APW) glds16_base(abase + dkt * BK, aoffs[t < APW ? t : 0], base + (wave * APW + t) * 1024u);
+    if (t < APW) glds16_base(abase + dkt * BK, aoffs[t < APW ? t : 0], base + min(wave * APW + t, BM / 8 - 1) * 1024u);
     else glds16_base(bbase[t >= APW ? (t - APW) >> 1 : 0] + (size_t)dkt * 1024 + ((t - APW) & 1) * 512, lane * 16u, base + (A_UNITS + (wave * BPW + (t - APW)) * 64) * 16u);
   };
   auto advance = [&] {                                // behind the last tile: the last k-tile again, into a stage that nobody reads any more
@@ -1032,8 +1037,7 @@ __global__ __launch_bounds__(512) void gemm_walk_kernel(
     else dkt = nkt - 1;
   };
   const unsigned lds0 = lds_addr(dsmem);
-  unsigned char* const elds = reinterpret_cast<unsigned char*>(dsmem + NSTAGE * STAGE) + wave * (EGR * 2048);
-  static_assert(NSTAGE * STAGE * 16 + 8 * EGR * 2048 <= 163840, "LDS of a compute unit");
+  static_assert(NSTAGE * STAGE * 16 + (OWN ? 8 * EGR * 2048 : 0) <= 163840, "LDS of a compute unit");
 
   point();
   if (kt0 < nkt) {
@@ -1096,6 +1100,8 @@ __global__ __launch_bounds__(512) void gemm_walk_kernel(
       }
       advance();
     }
+    if (!OWN) __builtin_amdgcn_s_barrier();          // every wave is done with that stage; the ring fills it behind its next barrier
+    unsigned char* const elds = reinterpret_cast<unsigned char*>(dsmem + (OWN ? NSTAGE : st == 0 ? NSTAGE - 1 : st - 1) * STAGE) + wave * (EGR * 2048);
     int l = lane;          // opaque: the epilogue's addresses are formed here and not kept in registers through the k-loop
     asm volatile("" : "+v"(l));
     if constexpr (EPI == EPI_PARTIAL) {
@@ -1660,14 +1666,16 @@ static void launch_big_s(const GemmArgs& a, hipStream_t st) {
 }
 // the walking kernels' offsets inside a tile are 32-bit (288 activation rows)
 static bool walk_offsets_fit(const GemmArgs& a) { return (size_t)a.lda * 576 <= 0xffffffffu; }
+// blocks of one split: one a tile while all splits' tiles fit the chip at once, else as many as it has units for
+static unsigned walk_grid(long tiles, int S) { return tiles * S <= 256 ? capped_grid(tiles) : std::min(capped_grid(tiles), (unsigned)std::max(8, (256 / S) & ~7)); }
 template <int BM, int EPI>
 static void launch_walk(const GemmArgs& a, hipStream_t st) {
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + 255) / 256;
   const int nkt = a.K / 64, S = (EPI == EPI_PARTIAL) ? a.nsplit : 1;
-  constexpr size_t lds = (size_t)(BM >= 192 ? 2 : 3) * (BM * 8 + 2048) * 16 + 8 * (BM >= 192 && EPI != EPI_GELU_ERF ? 4096 : 2048);      // 160 / 144 / 160 KB
+  constexpr size_t lds = walk_lds(BM, EPI);      // 256 / 192 / 160 / 128 rows: 160 / 144 / 156 / 160 KB
   static DeviceOnce attr_set;   // per instantiation
   if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_walk_kernel<BM, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  const unsigned grid = std::min(capped_grid((long)tiles_m * tiles_n), (unsigned)std::max(8, (256 / S) & ~7));
+  const unsigned grid = walk_grid((long)tiles_m * tiles_n, S);
   gemm_walk_kernel<BM, EPI><<<dim3(grid, S), dim3(512), lds, st>>>(a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m,
                                                                    tiles_n, a.partial, (nkt + S - 1) / S, a.wscale, raster_for(tiles_m));
 }
@@ -1686,7 +1694,7 @@ static void launch_vh(const GemmArgs& a, hipStream_t st) {
   static DeviceOnce attr_set;   // per instantiation
   if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_walk_vh_kernel<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   g_launch_counts[LC_GEMM_VH]++;
-  const unsigned grid = std::min(capped_grid((long)tiles_m * tiles_n), (unsigned)std::max(8, (256 / S) & ~7));
+  const unsigned grid = walk_grid((long)tiles_m * tiles_n, S);
   gemm_walk_vh_kernel<EPI><<<dim3(grid, S), dim3(512), lds, st>>>(
       a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.partial, (nkt + S - 1) / S, raster_for(tiles_m));
 }
@@ -1706,15 +1714,19 @@ static void launch_big(const GemmArgs& a, hipStream_t st) {
   // bit-identical to the burst-behind-the-barrier order SCHED 1 -- tools/gemm_checksum.py -- and 1.6-3.3 % faster on the prefill
   // GEMMs, +0.6 / +0.8 % tokens/s at 1 / 8 streams, profiles/r03/gemm_sched_spread_dma.txt); LCC_GEMM_SCHED=1 restores SCHED 1
   static const int spread = [] { const char* v = getenv("LCC_GEMM_SCHED"); return (v && atoi(v) == 1) ? 0 : 1; }();
-  if (a.w_fp8) launch_big_s<(BM == 192 ? 256 : BM), EPI, 1, true>(a, st);     // the 192-row tile is a bf16-weight shape (big_tile_rows never picks it for fp8)
+  if (a.w_fp8) launch_big_s<(BM == 192 || BM == 160 ? 256 : BM), EPI, 1, true>(a, st);     // 192 and 160 rows are bf16-weight shapes (big_tile_rows never picks them for fp8)
   else if (g_gemm_sched && spread) {
-    if (!walk_offsets_fit(a)) launch_big_s<BM, EPI, 1, false>(a, st);
+    // 128-row tiles that fill one round at most have nothing to walk, and the walk's longer prologue shows: 4,006 x 1536, K 768 17.6 us there, 19.1 walked;
+    // vision fc1 of one chunk 27.7 / 28.6.  (192 and 256 rows gain from the scalar addresses: 4096 x 3584, K 3584 fp32 105.9 -> 102.5.)
+    const long tiles = (long)((a.M + BM - 1) / BM) * ((a.N + 255) / 256) * (EPI == EPI_PARTIAL ? a.nsplit : 1);
+    if (!walk_offsets_fit(a)) launch_big_s<(BM == 160 ? 192 : BM), EPI, 1, false>(a, st);
+    else if (BM == 128 && tiles <= 256) launch_big_s<128, EPI, 6, false>(a, st);
     else launch_walk<BM, EPI>(a, st);
   }
-  else if (g_gemm_sched) launch_big_s<BM, EPI, 1, false>(a, st);
-  else launch_big_s<BM, EPI, 0, false>(a, st);
+  else if (g_gemm_sched) launch_big_s<(BM == 160 ? 192 : BM), EPI, 1, false>(a, st);
+  else launch_big_s<(BM == 160 ? 192 : BM), EPI, 0, false>(a, st);
 }
-// 13: the 192-row tile wherever eligible (bf16 weights); 14: variable-height row tiles (gemm_vh_kernel) wherever legal, else as 3;
+// 13 / 17: the 192- / 160-row tile wherever eligible (bf16 weights); 14: variable-height row tiles (gemm_vh_kernel) wherever legal, else as 3;
 // 16: 128 x 128 tiles (gemm_mid_kernel) wherever eligible, bf16 weights
 // 15: the small variable-height class (8 / 9 fragments) for split-K slabs wherever legal, else as 4
 void set_gemm_variant(int v) {
@@ -1753,18 +1765,23 @@ static float tile_score(int M, int N, int S, int BM, int BN, int slots, float ef
 // Variable-height tiles (round 5; returned as 272): floor(F / 16) row tiles of 16-18 fragments -- scored with every tile as tall as the
 // tallest (a 17-fragment tile costs 17/16 of a 256-row tile on every SIMD), no ragged tile, the 256-row tile's efficiency.
 // LCC_GEMM_VH=0: rounds 2-4 tile choice.
-static int big_tile_rows(const GemmArgs& a, int S) {
+static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr) {      // score: of the chosen tile, automatic choice only
   if (!big_eligible(a)) return 0;
   if (g_gemm_variant == 14) return vh_legal(a) ? 272 : 256;
   if (g_gemm_variant == 3 || g_gemm_variant == 5) return 256;
   if (g_gemm_variant == 4 || g_gemm_variant == 6) return 128;
   if (g_gemm_variant == 13) return a.w_fp8 ? 256 : 192;
+  if (g_gemm_variant == 17) return a.w_fp8 ? 256 : 160;
   if (g_gemm_variant == 15) return (a.partial != nullptr && vh_small_shape(a.M, a.K) && vh_legal(a, true)) ? 144 : 128;
   if (g_gemm_variant == 16) return a.w_fp8 ? 128 : 129;
   if (g_gemm_variant != 2) return 0;
   const float s256 = tile_score(a.M, a.N, S, 256, 256, 256, 1.0f, true);
   static const int allow192 = [] { const char* v = getenv("LCC_GEMM_192"); return v ? atoi(v) : 1; }();     // A/B: 0 = round-3 tile choice
   const float s192 = (a.w_fp8 || !allow192) ? 0.f : tile_score(a.M, a.N, S, 192, 256, 256, 0.93f, true);
+  // BM 160 (bf16 weights): where 192 rows start a last round that is mostly empty.  The vision proj / fc2 of 15,840 rows are 83 x 5 tiles of 192 rows =
+  // 1.62 rounds; 99 x 5 of 160 fill 1.93 at 5/6 of the time each: proj 55.7 -> 52.1 us, fc2 201 -> 178.
+  // 1000 / 2100 x 17920, K 1536 with SwiGLU 63.6 -> 58.4 / 117.5 -> 111.3.
+  const float s160 = (a.w_fp8 || !allow192 || a.wscale != nullptr) ? 0.f : tile_score(a.M, a.N, S, 160, 256, 256, 0.90f, false);
   const float s128 = tile_score(a.M, a.N, S, 128, 256, 256, 0.85f, true);
   // gemm_mid_kernel: 0.38 / 0.52 us a step of 64 x 128 / 128 x 128 against 0.85 of 128 x 256, one tile a compute unit at a time (two 64-row
   // tiles side by side take twice as long).  Returned as 0 / 129.  The 128-row form wins where its blocks fill one round and the 64-row
@@ -1773,22 +1790,27 @@ static int big_tile_rows(const GemmArgs& a, int S) {
   // dequantises first, scored as measured with it.
   const float s64 = a.w_fp8 ? tile_score(a.M, a.N, S, 64, 128, 512, 0.55f, false) : tile_score(a.M, a.N, S, 64, 128, 256, 0.48f, false);
   const float s128m = a.w_fp8 ? 0.f : tile_score(a.M, a.N, S, 128, 128, 256, 0.70f, false);
+  if (score) *score = std::max(std::max(std::max(s256, s192), std::max(s160, s128)), std::max(s128m, s64));
   static const int allow_vh = [] { const char* v = getenv("LCC_GEMM_VH"); return v ? atoi(v) : 1; }();
   if (allow_vh && vh_legal(a) && (((a.M + 15) >> 4) & 15) != 0) {      // F % 16 == 0: the 256-row tiles are the same thing
     const int F = (a.M + 15) >> 4, t = F >> 4, maxf = (F + t - 1) / t;
     const long blocks = (long)t * ((a.N + 255) / 256) * S;
     const float svh = (float)a.M / (float)(t * maxf * 16) * (float)blocks / (float)((blocks + 255) / 256 * 256);
-    if (svh > s256 && svh > s192 && svh > s128 && svh > s128m && svh > s64) return 272;
+    if (svh > s256 && svh > s192 && svh > s160 && svh > s128 && svh > s128m && svh > s64) {
+      if (score) *score = svh;
+      return 272;
+    }
   }
   // small class (returned as 144): split-K slabs of one streaming chunk's projections, where the 128-row tiles leave a nearly empty last row tile
   if (vh_small_on() && a.partial != nullptr && vh_small_shape(a.M, a.K) && vh_legal(a, true)) {
     const int F = (a.M + 15) >> 4, t = F >> 3, maxf = (F + t - 1) / t;
     const long blocks = (long)t * ((a.N + 255) / 256) * S;
     const float svs = 0.85f * (float)a.M / (float)(t * maxf * 16) * (float)blocks / (float)((blocks + 255) / 256 * 256);
-    if (svs > s256 && svs > s192 && svs > s128 && svs > s128m && svs > s64) return 144;
+    if (svs > s256 && svs > s192 && svs > s160 && svs > s128 && svs > s128m && svs > s64) return 144;
   }
-  if (s256 >= s192 && s256 >= s128 && s256 >= s128m && s256 >= s64) return 256;
-  if (s192 >= s128 && s192 >= s128m && s192 >= s64) return 192;
+  if (s256 >= s192 && s256 >= s160 && s256 >= s128 && s256 >= s128m && s256 >= s64) return 256;
+  if (s192 >= s160 && s192 >= s128 && s192 >= s128m && s192 >= s64) return 192;
+  if (s160 > s128 && s160 > s128m && s160 > s64) return 160;
   // a last row tile that is half empty saves nothing while all blocks run at once beside full ones, and two 64-row tiles a unit hide each other's ends:
   // at 129 to 192 rows [17920, 1536] 19.1 us against 23.0 with 128 x 256 tiles, [4608, 3584] in four splits 15.4 / 16.6, [3584, 3584] in six 13.3 / 14.2.
   // Up to 24 steps a block: [3584, 18944] in six splits (49 steps) 51.7 / 44.4
@@ -1841,6 +1863,7 @@ static void launch_tiled_bm(const GemmArgs& a, hipStream_t st) {
   if (big == 272) return launch_vh<EPI>(a, st);
   if (big == 256) return launch_big<256, EPI>(a, st);
   if (big == 192) return launch_big<192, EPI>(a, st);
+  if (big == 160) return launch_big<160, EPI>(a, st);
   if (big == 128) return launch_big<128, EPI>(a, st);
   // 128-row tiles only for large M with a grid that fills the chip; otherwise 64-row tiles (less waste on a ragged M such as
   // 386 rows, more blocks, and the faster LDS-DMA kernel)
@@ -1850,7 +1873,7 @@ static void launch_tiled_bm(const GemmArgs& a, hipStream_t st) {
 }
 
 // Which kernel family serves a packed-weight GEMM of this shape under the current variant (host logic only: no launch, no GPU needed):
-// 16 = weight-streaming GEMV, 448 = tall, 272 / 144 = variable-height tiles (big / small class), 256 / 192 / 128 = the 8-wave tile of
+// 16 = weight-streaming GEMV, 448 = tall, 272 / 144 = variable-height tiles (big / small class), 256 / 192 / 160 / 128 = the 8-wave tile of
 // that height x 256 columns, 129 = 128 x 128, 64 = 64 x 128.  `nsplit` > 0: the split-K slab form with that many splits (as the engine asks: gemm_tiled_num_splits).
 int gemm_plan(int M, int N, int K, int epilogue, int nsplit, bool w_fp8) {
   GemmArgs a; a.M = M; a.N = N; a.K = K; a.w_packed = 1; a.w_fp8 = w_fp8 ? 1 : 0; a.epilogue = epilogue; a.nsplit = nsplit;
@@ -2347,6 +2370,23 @@ int gemv_num_splits(int N, int K) {
 // split-K factor for a tiled GEMM whose output grid alone cannot fill 256 CUs (e.g. M = 386, N = 3584: 196 tiles)
 int gemm_tiled_num_splits(int M, int N, int K, bool packed_bf16) {
   const long tiles = (long)((M + 63) / 64) * ((N + 127) / 128);
+  // More than one chunk's rows on a long K (bf16 weights): the split count whose best tile (big_tile_rows' scores against 1.25 PFLOP/s) plus the slabs' way
+  // to memory and back is shortest, and only if that saves a tenth.  Product and consumer together, us, without / with: 1000 x 3584, K 22528 240 / 170
+  // (four splits of 256 x 256 tiles instead of 128 x 128); 600 x 3584, K 18944 107 (three) / 94; 2104 x 1536, K 10496 86 / 73; 1000 x 1536, K 8960 52 / 40.
+  if (packed_bf16 && M > 448 && M <= 4096 && K >= 6144 && (K & 63) == 0 && (N & 15) == 0 && g_gemm_variant == 2) {
+    static float dummy;
+    GemmArgs a; a.M = M; a.N = N; a.K = K; a.w_packed = 1; a.lda = K;
+    int best = 1;
+    float best_us = 0.f;
+    for (int S = 1; S <= 6; ++S) {
+      if (S > 1) { a.partial = &dummy; a.nsplit = S; }          // never dereferenced: the slab form is asked for
+      float score = 0.f;
+      big_tile_rows(a, S, &score);
+      const float us = 2e-9f * (float)M * (float)N * (float)K / (1.25f * score) + (S > 1 ? (float)S * (float)M * (float)N * 8e-6f / 4.5f : 0.f);
+      if (S == 1 || us < (best == 1 ? 0.9f : 1.f) * best_us) { best = S; best_us = us; }
+    }
+    return best;
+  }
   if (tiles >= 400 || M > 4096) return 1;
   int s = (int)((640 + tiles - 1) / tiles);
   s = std::min(s, std::max(1, ((K + 63) / 64) / 8));
@@ -2431,6 +2471,7 @@ int gemm_bf16(const GemmArgs& a, hipStream_t st) {
     if ((v && ((uintptr_t)q.vt & 7) != 0) || (a.bias != nullptr && ((uintptr_t)a.bias & 7) != 0)) return LCC_ERR_ALIGN;
     g_launch_counts[LC_GEMM_VIT_QKV]++;
     int big = big_tile_rows(a, 1);
+    if (big == 160) big = 192;
     if (big == 272) big = 256;      // the rotation / transposed-V epilogues live on the fixed-height 256-column tiles (129: the 128-row one)
     if (a.epilogue == EPI_VIT_QKV) {
       if (big == 256) launch_big_s<256, EPI_VIT_QKV, 6, false>(a, st);
@@ -2478,6 +2519,7 @@ int gemm_bf16(const GemmArgs& a, hipStream_t st) {
     else if (big == 144) launch_vh_small(a, st);
     else if (big == 256) launch_big<256, EPI_PARTIAL>(a, st);
     else if (big == 192) launch_big<192, EPI_PARTIAL>(a, st);
+    else if (big == 160) launch_big<160, EPI_PARTIAL>(a, st);
     else if (big == 128) launch_big<128, EPI_PARTIAL>(a, st);
     else if (big == 129) launch_mid<128, EPI_PARTIAL, 4>(a, st);
     else launch_tiled<64, EPI_PARTIAL>(a, st);

@@ -135,3 +135,16 @@ def test_decode_batches_that_take_the_row_scaled_products(built_lib, preset, fp8
         assert built_lib.lcc_debug_decode_row_scaled(e, 0) < 0 and built_lib.lcc_debug_decode_row_scaled(None, 3) < 0
     finally:
         built_lib.lcc_engine_destroy(e)
+
+
+def test_long_contractions_of_a_few_hundred_to_a_few_thousand_rows_are_split(built_lib):
+    """Between one chunk's rows and a piece of 4,096: two to six splits where a tenth is saved, never more than the slab buffer holds (six), each split
+    of several k-tiles; one where the tiles fill the chip, on a short K, for fp8 weights."""
+    from livecc_amd import ops
+    plan = lambda M, N, K, **kw: ops.gemm_plan(M, N, K, ops.EPI_NONE, **kw)[1]
+    assert all(2 <= plan(M, N, K) <= 6 for M, N, K in ((449, 3584, 18944), (600, 3584, 18944), (1000, 3584, 22528), (1131, 3584, 18944), (1000, 1536, 8960), (2104, 1536, 10496)))
+    assert plan(4096, 3584, 18944) == plan(3088, 3584, 18944) == plan(2000, 3584, 18944) == plan(5000, 3584, 18944) == 1
+    assert plan(1000, 3584, 18944, w_fp8=True) == 1 and plan(1000, 3584, 6080) == 1
+    for M in range(449, 4097, 37):
+        for N, K in ((3584, 18944), (1536, 8960), (272, 6144)):
+            assert 1 <= plan(M, N, K) <= 6

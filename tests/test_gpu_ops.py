@@ -204,9 +204,10 @@ def test_gemm_epilogue_rows_of_16_byte_pieces_and_others_give_the_same_bits(dev,
 
 
 @pytest.mark.parametrize("variant,M,K,S", [(3, 2100, 64, 0), (3, 2100, 192, 3), (13, 1600, 128, 1), (13, 1600, 64, 0), (4, 1100, 64, 0), (4, 1100, 128, 0),
-                                           (4, 1100, 320, 0), (14, 2130, 64, 0), (14, 2130, 192, 3)])
+                                           (4, 1100, 320, 0), (14, 2130, 64, 0), (14, 2130, 192, 3), (17, 1290, 64, 0),
+                                           (17, 1290, 128, 1), (17, 1441, 320, 3)])
 def test_gemm_blocks_that_walk_several_tiles_are_bit_identical_to_one_tile_a_block(dev, variant, M, K, S):
-    """More tiles than compute units (9 x 34 and 8 x 34, ragged rows and columns), one k-tile up to more than the ring holds: every epilogue and the
+    """More tiles than compute units (9 or 10 x 34 and 8 x 34, ragged rows and columns), one k-tile up to more than the ring holds: every epilogue and the
     fp32 slabs, three splits with the chip's blocks shared among them."""
     from livecc_amd import ops
     N = 8480
