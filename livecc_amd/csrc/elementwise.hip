@@ -605,10 +605,13 @@ __global__ __launch_bounds__(256) void resize_aa_v_kernel(const float* __restric
 // pass over an fp32 tensor of 12.6 MB that nothing else reads.  Here a lane owns a column and keeps its K weights (zero behind its own count)
 // in registers for all rows of the tile, its 3 K source bytes are K dword reads shifted into place, and the height pass takes four columns a
 // lane.  Two 720p frames to 392 x 728: 33.3 -> 11.6 us (rows x channels one column a lane: 15.9); two of 300 x 500: 15 -> 9.6; 24 of
-// 1080p to 280 x 504 (17 taps, half of a tile's rows are its neighbour's too): 391 -> 138.
+// 1080p to 280 x 504 (17 taps, half of a tile's rows are its neighbour's too): 391 -> 138.  With the window from scalar loads, so that the source
+// is asked for at once and not behind the tables' round trip and six reductions, and the tile's rows chosen for the launch (resize_plan), 16 or 8
+// rows before: in a row of launches 10.5 -> 9.6, 8.8 -> 7.7 and 124 -> 112 us; 64 frames of 360p to 280 x 504: 83 -> 56; planar 480p pair: 10.2 -> 8.0.
 // The tables are the caller's: a tile whose window does not fit what the host sized from the scale is computed tap by tap (same values).
 constexpr int RS_COLS = 64;
 constexpr int RS_WAVES = 8;
+constexpr int RS_ROWS = 32;                     // output rows of a tile at most
 constexpr int RS_LDS_MAX = 80 * 1024;          // two blocks on a compute unit
 template <int K, bool PLANAR>
 __global__ __launch_bounds__(RS_WAVES * 64) void resize_aa_tile_kernel(const uint8_t* __restrict__ src, int T, int Hin, int Win, uint8_t* __restrict__ dst,
@@ -618,7 +621,7 @@ __global__ __launch_bounds__(RS_WAVES * 64) void resize_aa_tile_kernel(const uin
                                                              const float* __restrict__ wy, int ky, int TH, int rows_cap, int seg_dw) {
   constexpr int PX = PLANAR ? 1 : 3, NSEG = PLANAR ? 3 : 1;       // bytes from a pixel to the next; staged pieces of a source row
   extern __shared__ __attribute__((aligned(16))) float wrow[];    // [TH][ky up to 4s], then mid [rows_cap][3][64], then the pieces [rows_cap * NSEG][seg_dw]
-  __shared__ int tap0[16], taps[16];
+  __shared__ int tap0[RS_ROWS], taps[RS_ROWS];
   float* mid = wrow + TH * ((ky + 3) & ~3);
   unsigned* raw = reinterpret_cast<unsigned*>(mid + (size_t)rows_cap * 3 * RS_COLS);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -626,20 +629,19 @@ __global__ __launch_bounds__(RS_WAVES * 64) void resize_aa_tile_kernel(const uin
   const int tx = blockIdx.x % tiles_x, ty = (blockIdx.x / tiles_x) % tiles_y, t = blockIdx.x / (tiles_x * tiles_y);
   const int y0t = ty * TH, nrow = min(TH, Hout - y0t);
   const int xo = min(tx * RS_COLS + lane, Wout - 1), yl = y0t + min(lane, nrow - 1);
+  // The window is that of the tile's first and last column and row (scalar loads: the staging below does not wait for the tables); a table in
+  // which another one reaches beyond them takes the tap-by-tap form, as one whose window does not fit.
+  typedef const __attribute__((address_space(4))) int* sptr;
+  const sptr sx = (sptr)(uintptr_t)xmin, sy = (sptr)(uintptr_t)ymin, sn = (sptr)(uintptr_t)ysize;
+  const int y_last = y0t + nrow - 1;
+  const int lo = sx[tx * RS_COLS], hi = sx[min(tx * RS_COLS + RS_COLS, Wout) - 1], rlo = sy[y0t], rhi = sy[y_last] + max(sn[y_last], 1);
   const int x0 = xmin[xo], n = xsize[xo], yy = ymin[yl], yn = ysize[yl];
-  int lo = x0, hi = x0, nmax = n, nymax = yn, rlo = yy, rhi = yy + max(yn, 1);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    lo = min(lo, __shfl_xor(lo, o, 64)); hi = max(hi, __shfl_xor(hi, o, 64)); nmax = max(nmax, __shfl_xor(nmax, o, 64)); nymax = max(nymax, __shfl_xor(nymax, o, 64));
-    rlo = min(rlo, __shfl_xor(rlo, o, 64)); rhi = max(rhi, __shfl_xor(rhi, o, 64));
-  }
-  lo = __builtin_amdgcn_readfirstlane(lo); hi = __builtin_amdgcn_readfirstlane(hi); nmax = __builtin_amdgcn_readfirstlane(nmax); nymax = __builtin_amdgcn_readfirstlane(nymax);
-  rlo = __builtin_amdgcn_readfirstlane(rlo); rhi = __builtin_amdgcn_readfirstlane(rhi);
+  const bool out = x0 < lo || x0 > hi || n > K || yy < rlo || yy + max(yn, 1) > rhi || yn > ky || yn < 1;          // every wave asks for all rows and columns
   const int cols = hi - lo + K, rows = rhi - rlo;
   const uint8_t* frame = src + (size_t)t * 3 * Hin * Win;
   const size_t plane = (size_t)Hin * Win;
   const bool live = tx * RS_COLS + lane < Wout;
-  if (rows > rows_cap || nymax > ky || nymax < 1 || cols * PX + 8 > seg_dw * 4 || nmax > K) {      // block-uniform: every wave reduced the same values
+  auto tap_by_tap = [&] {
     for (int it = wave; it < nrow * 3; it += RS_WAVES) {
       const int yo = y0t + it / 3, c = it - it / 3 * 3, ys = ymin[yo], ny = ysize[yo];
       float acc = 0.f;
@@ -652,8 +654,9 @@ __global__ __launch_bounds__(RS_WAVES * 64) void resize_aa_tile_kernel(const uin
       }
       if (live) dst[(((size_t)t * 3 + c) * Hout + yo) * Wout + xo] = (uint8_t)rintf(fminf(fmaxf(acc, 0.f), 255.f));
     }
-    return;
-  }
+  };
+  // block-uniform, and before anything is read through the tables: the window is inside the picture and what the host sized
+  if (rows < 1 || rows > rows_cap || hi < lo || cols * PX + 8 > seg_dw * 4 || lo < 0 || lo >= Win || rlo < 0 || rhi > Hin) return tap_by_tap();
   float w[K];
 #pragma unroll
   for (int j = 0; j < K; ++j) {
@@ -694,6 +697,7 @@ __global__ __launch_bounds__(RS_WAVES * 64) void resize_aa_tile_kernel(const uin
   if (wave == 0 && lane < nrow) { tap0[lane] = yy - rlo; taps[lane] = max(yn, 1); }
 #pragma unroll
   for (int j = 0; j < K; ++j) asm volatile("" ::"v"(w[j]));          // the weights arrive under the staging, not behind it
+  if (__builtin_amdgcn_ballot_w64(out) != 0) return tap_by_tap();      // block-uniform: every wave compared the same values
   __syncthreads();
   for (int r = wave; r < rows; r += RS_WAVES) {
     float a[3];
@@ -741,7 +745,7 @@ __global__ __launch_bounds__(RS_WAVES * 64) void resize_aa_tile_kernel(const uin
     const float* wr = wrow + r * kyp;
     const float* p = mid + (tap0[r] * 3 + c) * RS_COLS + col;
     f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
-    for (int j0 = 0; j0 < nymax; j0 += 4) {
+    for (int j0 = 0; j0 < ny; j0 += 4) {
       const f32x4 w4 = *reinterpret_cast<const f32x4*>(wr + j0);
       f32x4 m[4];
 #pragma unroll
@@ -785,29 +789,35 @@ static void launch_resize_tile(const uint8_t* src, int layout, int T, int Hin, i
 // one launch while a tile's window fits RS_LDS_MAX with at least 8 rows: scales up to about 4 (tap tables of 5 to 17 columns); wider filters
 // take the two passes, whose work does not grow with the overlap of neighbouring tiles
 struct ResizePlan { int TH = 0, rows_cap = 0, seg_dw = 0; size_t lds = 0; };      // TH 0: two passes
-static ResizePlan resize_plan(int layout, int Hin, int Win, int Hout, int Wout, int kx, int ky) {
+static ResizePlan resize_plan(int layout, int T, int Hin, int Win, int Hout, int Wout, int kx, int ky) {
   ResizePlan p;
   if ((kx & 1) == 0 || kx < 5 || kx > 17) return p;
   const double sx = (double)Win / Wout, sy = (double)Hin / Hout;
   const int seg_dw = (((int)(63 * sx) + 2 + kx) * (layout == 0 ? 3 : 1) + 8 + 3) / 4;
-  for (int TH = 16; TH >= 8; TH >>= 1) {
+  // rows a compute unit walks: tiles dealt to it x source rows of a tile.  More rows a tile: fewer source rows twice; fewer: an even share for all units
+  // (two 720p frames to 392 x 728: 600 tiles of 16 rows put three on some units, 504 of 19 two on each: 10.5 -> 9.6 us; 64 of 360p to 280 x 504: 83 -> 56).
+  long best = 0;
+  for (int TH = 8; TH <= RS_ROWS; ++TH) {
     const int rows_cap = (int)((TH - 1) * sy + 4 * std::max(sy, 1.0)) + 3;
     const size_t lds = ((size_t)rows_cap * (3 * RS_COLS + (layout == 0 ? 1 : 3) * seg_dw) + TH * ((ky + 3) & ~3)) * 4;
-    if (lds > RS_LDS_MAX) continue;
-    p.TH = TH; p.rows_cap = rows_cap; p.seg_dw = seg_dw; p.lds = lds;
-    break;
+    if (lds > RS_LDS_MAX) break;
+    const long tiles = (long)T * ((Hout + TH - 1) / TH) * ((Wout + RS_COLS - 1) / RS_COLS), per = (tiles + 255) / 256;
+    // a unit holds 160 KB and four blocks of eight waves: what is beyond runs behind
+    const long fit = std::max<long>(1, std::min<long>(4, (long)(163840 / (lds + 512))));
+    const long cost = (per + fit - 1) / fit * 12 + per * rows_cap;      // a round's latency: as long as some 12 source rows
+    if (p.TH == 0 || cost < best) { p.TH = TH; p.rows_cap = rows_cap; p.seg_dw = seg_dw; p.lds = lds; best = cost; }
   }
   return p;
 }
 size_t resize_tmp_floats(int layout, int T, int Hin, int Win, int Hout, int Wout, int kx, int ky) {
-  if (T <= 0 || Hin <= 0 || Win <= 0 || Hout <= 0 || Wout <= 0 || kx <= 0 || ky <= 0 || resize_plan(layout, Hin, Win, Hout, Wout, kx, ky).TH > 0) return 0;
+  if (T <= 0 || Hin <= 0 || Win <= 0 || Hout <= 0 || Wout <= 0 || kx <= 0 || ky <= 0 || resize_plan(layout, T, Hin, Win, Hout, Wout, kx, ky).TH > 0) return 0;
   return (size_t)T * 3 * Hin * Wout;
 }
 int resize_bicubic_aa_u8(const uint8_t* src, int layout, int T, int Hin, int Win, uint8_t* dst, int Hout, int Wout,
                          const int32_t* xmin, const int32_t* xsize, const float* wx, int kx, const int32_t* ymin,
                          const int32_t* ysize, const float* wy, int ky, float* tmp, hipStream_t st) {
   if (T <= 0 || Hin <= 0 || Win <= 0 || Hout <= 0 || Wout <= 0 || kx <= 0 || ky <= 0 || (layout != 0 && layout != 1)) return LCC_ERR_SHAPE;
-  const ResizePlan p = resize_plan(layout, Hin, Win, Hout, Wout, kx, ky);
+  const ResizePlan p = resize_plan(layout, T, Hin, Win, Hout, Wout, kx, ky);
   if (p.TH > 0) {
 #define LCC_RS(KX) case KX: launch_resize_tile<KX>(src, layout, T, Hin, Win, dst, Hout, Wout, xmin, xsize, wx, ymin, ysize, wy, ky, p.TH, p.rows_cap, p.seg_dw, p.lds, st); return 0
     switch (kx) { LCC_RS(5); LCC_RS(7); LCC_RS(9); LCC_RS(11); LCC_RS(13); LCC_RS(15); LCC_RS(17); }

@@ -113,3 +113,34 @@ def test_a_resize_in_one_launch_allocates_its_result_only(dev, monkeypatch, use_
     out = R.resize_bicubic_aa(x, 392, 728)
     # torch's allocator hands a cached block out whole where less than 1 MB of it would be left; the fp32 rows between two passes would be 25 MB
     assert torch.cuda.max_memory_allocated() - before <= out.numel() + (2 << 20)
+
+
+@pytest.mark.parametrize("swap", ["reversed", "ends", "inside"])
+@pytest.mark.parametrize("axis", ["columns", "rows"])
+def test_resize_with_tables_in_another_order(dev, swap, axis):
+    """The window of a tile is taken from its first and last column and row: tables in which others reach beyond them (reversed; the first
+    swapped with a middle one) give the same bytes in their order, as those that stay inside (two middle ones swapped)."""
+    from livecc_amd import resize as R, torch_ops
+    T, hi, wi, ho, wo = 2, 97, 255, 49, 129
+    x = torch.randint(0, 256, (T, hi, wi, 3), dtype=torch.uint8, generator=torch.Generator().manual_seed(3)).to(dev)
+    xmin, xsize, wx, kx = R._taps_on(x.device, wi, wo, tap_major=True)
+    ymin, ysize, wy, ky = R._taps_on(x.device, hi, ho)
+    n = wo if axis == "columns" else ho
+    order = torch.arange(n)
+    if swap == "reversed":
+        order = order.flip(0)
+    else:
+        a, b = (0, 5) if swap == "ends" else (3, 6)
+        order[a], order[b] = b, a
+    order = order.to(dev)
+    op = torch_ops.op("resize_bicubic_aa")
+    plain = op(x, 0, ho, wo, xmin, xsize, wx, kx, ymin, ysize, wy, ky)
+    wx2 = wx.reshape(kx, wo)
+    wy2 = wy.reshape(ho, ky)
+    if axis == "columns":
+        got = op(x, 0, ho, wo, xmin[order].contiguous(), xsize[order].contiguous(), wx2[:, order].contiguous().reshape(wx.shape), kx, ymin, ysize, wy, ky)
+        want = plain[..., order]
+    else:
+        got = op(x, 0, ho, wo, xmin, xsize, wx, kx, ymin[order].contiguous(), ysize[order].contiguous(), wy2[order].contiguous().reshape(wy.shape), ky)
+        want = plain[:, :, order]
+    assert torch.equal(got, want)
