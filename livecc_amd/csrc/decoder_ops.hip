@@ -19,6 +19,22 @@ LCC_DEVICE u32x4 dyt8(const float (&x)[8], float alpha, const bf16_t* w, const b
   return o;
 }
 
+LCC_DEVICE f32x4 bf4(u32x2 q) { return (f32x4){lo2f(q.x), hi2f(q.x), lo2f(q.y), hi2f(q.y)}; }
+LCC_DEVICE float sq4(f32x4 v) { return (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]); }
+// sum of the slabs, four of them in flight
+LCC_DEVICE f32x4 slabs4(const float* part, int nsplit, size_t slab, size_t at) {
+  f32x4 v = *reinterpret_cast<const f32x4*>(part + at);
+  for (int k = 1; k < nsplit; k += 4) {
+    f32x4 u[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) u[j] = *reinterpret_cast<const f32x4*>(part + (size_t)min(k + j, nsplit - 1) * slab + at);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (k + j < nsplit) v += u[j];
+  }
+  return v;
+}
+
 // x = embedding row (fp32), h = norm(x).  ids[i], or -- decode -- the slot's current token ids[indirect[i]].
 __global__ __launch_bounds__(256) void embed_dyt_kernel(const int32_t* __restrict__ ids, const int32_t* __restrict__ indirect,
                                                         const bf16_t* __restrict__ table, DytNorm nm, float* __restrict__ x,
@@ -39,26 +55,39 @@ __global__ __launch_bounds__(256) void embed_dyt_kernel(const int32_t* __restric
   }
 }
 
-// x += sum of the nsplit fp32 slabs of the layer's output product, h = norm(x) of the NEXT norm
+// x += sum of the nsplit fp32 slabs of the layer's output product, h = norm(x) of the NEXT norm.  A decode step's launch is a chain of memory trips:
+// 4 channels a thread in blocks of 64 threads, so that the slabs of 32 rows of 1,536 come in over 192 compute units and not 24, the loads of a piece in
+// flight together: 4.9 -> 4.1 us (eight slabs).  Launches that fill the chip anyway are bound by bytes: 8 channels a thread, whole 16-byte stores
+// of bf16 (4,000 rows of 1,536: 17.9 us, with 4 channels 20.6).
+template <int V>
 __global__ __launch_bounds__(256) void resid_dyt_kernel(float* __restrict__ x, const float* __restrict__ part, int nsplit, DytNorm nm,
                                                         bf16_t* __restrict__ h, int rows, int dim) {
-  const int cpr = dim >> 3;
+  const int cpr = dim / V;
   const float alpha = bf2f(nm.alpha[0]);
   const size_t slab = (size_t)rows * dim;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < (int64_t)rows * cpr; i += (int64_t)gridDim.x * 256) {
-    const int c = (int)(i % cpr) * 8;
-    const size_t off = (size_t)i * 8;
-    f32x4 a = *reinterpret_cast<const f32x4*>(x + off), b = *reinterpret_cast<const f32x4*>(x + off + 4);
-    f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < nsplit; ++s) {
-      sa += *reinterpret_cast<const f32x4*>(part + s * slab + off);
-      sb += *reinterpret_cast<const f32x4*>(part + s * slab + off + 4);
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < (int64_t)rows * cpr; i += (int64_t)gridDim.x * blockDim.x) {
+    const int c = (int)(i % cpr) * V;
+    const size_t off = (size_t)i * V;
+    f32x4 a = *reinterpret_cast<const f32x4*>(x + off);
+    if constexpr (V == 4) {
+      const f32x4 w = bf4(ld8(nm.w + c)), b = bf4(ld8(nm.b + c));
+      if (nsplit > 0) a += slabs4(part, nsplit, slab, off);
+      *reinterpret_cast<f32x4*>(x + off) = a;
+      st8(h + off, (u32x2){pack2(dyt_value(a[0], alpha, w[0], b[0]), dyt_value(a[1], alpha, w[1], b[1])),
+                           pack2(dyt_value(a[2], alpha, w[2], b[2]), dyt_value(a[3], alpha, w[3], b[3]))});
+    } else {
+      f32x4 b = *reinterpret_cast<const f32x4*>(x + off + 4);
+      f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+      for (int s = 0; s < nsplit; ++s) {
+        sa += *reinterpret_cast<const f32x4*>(part + s * slab + off);
+        sb += *reinterpret_cast<const f32x4*>(part + s * slab + off + 4);
+      }
+      a += sa; b += sb;
+      *reinterpret_cast<f32x4*>(x + off) = a;
+      *reinterpret_cast<f32x4*>(x + off + 4) = b;
+      const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+      st16(h + off, dyt8(v, alpha, nm.w + c, nm.b + c));
     }
-    a += sa; b += sb;
-    *reinterpret_cast<f32x4*>(x + off) = a;
-    *reinterpret_cast<f32x4*>(x + off + 4) = b;
-    const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-    st16(h + off, dyt8(v, alpha, nm.w + c, nm.b + c));
   }
 }
 
@@ -80,21 +109,6 @@ __global__ __launch_bounds__(256) void logits_cap_kernel(const float* __restrict
 }
 
 // ---- RMS norms with weights stored around zero: one block of NW waves per row, two 4-channel pieces per thread ----
-LCC_DEVICE f32x4 bf4(u32x2 q) { return (f32x4){lo2f(q.x), hi2f(q.x), lo2f(q.y), hi2f(q.y)}; }
-LCC_DEVICE float sq4(f32x4 v) { return (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]); }
-// sum of the slabs, four of them in flight
-LCC_DEVICE f32x4 slabs4(const float* part, int nsplit, size_t slab, size_t at) {
-  f32x4 v = *reinterpret_cast<const f32x4*>(part + at);
-  for (int k = 1; k < nsplit; k += 4) {
-    f32x4 u[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) u[j] = *reinterpret_cast<const f32x4*>(part + (size_t)min(k + j, nsplit - 1) * slab + at);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (k + j < nsplit) v += u[j];
-  }
-  return v;
-}
 LCC_DEVICE float inv_rms(float sum, int n, float eps) { return 1.f / sqrtf(sum / (float)n + eps); }
 
 template <int NW>
@@ -217,7 +231,9 @@ int resid_dyt(float* x, const float* part, int nsplit, const DytNorm& nm, bf16_t
   if (rows <= 0) return 0;
   if (dim <= 0 || (dim & 7) || nsplit < 0) return LCC_ERR_SHAPE;
   if (!x || !h || (nsplit > 0 && !part) || !dyt_ok(nm)) return LCC_ERR_ARG;
-  resid_dyt_kernel<<<dim3(grid_for((int64_t)rows * (dim >> 3))), dim3(256), 0, st>>>(x, part, nsplit, nm, h, rows, dim);
+  const int64_t quads = (int64_t)rows * (dim >> 2);
+  if (quads <= 64 * 1024) resid_dyt_kernel<4><<<dim3((unsigned)((quads + 63) / 64)), dim3(64), 0, st>>>(x, part, nsplit, nm, h, rows, dim);
+  else resid_dyt_kernel<8><<<dim3(grid_for(quads >> 1)), dim3(256), 0, st>>>(x, part, nsplit, nm, h, rows, dim);
   return 0;
 }
 int logits_cap(const float* part, int nsplit, int rows, int ld, int vocab, float scale, float cap, float* out, float* dense, hipStream_t st) {

@@ -1938,7 +1938,7 @@ __global__ __launch_bounds__(256) void gemv_skinny_kernel(
   const bf16_t* wp[NTILE];
 #pragma unroll
   for (int t = 0; t < NTILE; ++t)
-    wp[t] = PACKED ? W + (size_t)((n0 >> 4) + t) * K32 * 512 + lane * 8
+    wp[t] = PACKED ? W + (size_t)min((n0 >> 4) + t, ((N + 15) >> 4) - 1) * K32 * 512 + lane * 8      // a last block's absent tiles: the last one again, not stored
                    : W + (size_t)min(n0 + t * 16 + li, N - 1) * ldw + g * 8;
 
   f32x4 acc[NTILE][MG];
@@ -2119,15 +2119,16 @@ __global__ __launch_bounds__(256) void gemv_skinny_kernel(
         }
         st8(o + n, (u32x2){pack2(v[0], v[1]), pack2(v[2], v[3])});
       }
-    } else {  // swiglu: tile 0 = 16 gate rows, tile 1 = the 16 matching up rows
-      static_assert(MODE != 2 || NTILE == 2, "swiglu needs the gate and up tile in one block");
+    } else {  // swiglu: even tiles = 16 gate rows, the next one = the 16 matching up rows
+      static_assert(MODE != 2 || NTILE % 2 == 0, "swiglu needs the gate and up tile in one block");
       bf16_t* o = (bf16_t*)out + (size_t)m * ldo;
-      const int oc = n0 / 2 + g * 4;
-      if (n0 < N) {
+#pragma unroll
+      for (int t = 0; t + 1 < NTILE; t += 2) {
+        if (n0 + t * 16 >= N) continue;
         float r[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) r[q] = silu_bf16(rbf(acc[0][mg][q])) * rbf(acc[NTILE - 1][mg][q]);
-        st8(o + oc, (u32x2){pack2(r[0], r[1]), pack2(r[2], r[3])});
+        for (int q = 0; q < 4; ++q) r[q] = silu_bf16(rbf(acc[t][mg][q])) * rbf(acc[t + 1][mg][q]);
+        st8(o + n0 / 2 + t * 8 + g * 4, (u32x2){pack2(r[0], r[1]), pack2(r[2], r[3])});
       }
     }
   }
@@ -2176,30 +2177,39 @@ static void launch_gemv_l(dim3 grid, const GemmArgs& a, void* out, int ldo, int 
 }
 
 // 17..64 rows: a block of one 16-row weight tile reads more activations than weights (32 rows: twice as many bytes, and a compute unit pulls about 40
-// GB/s of either), so packed weights go two or four tiles to a block.  What a unit then pulls: rounds of blocks x (tiles + 16-row groups of
-// activations); four tiles only where that is clearly less, since their registers leave two waves a SIMD.  32 rows, [151936, 1536]: 116.5 us with one tile,
-// 80.8 with four (5.8 TB/s); [152064, 3584] 261 -> 182; [1536, 10496] in eight splits 10.7 -> 9.6; 64 rows: 358 -> 239 and 15.1 -> 11.7.  288
-// blocks of four (N = 4608, four splits, 17 rows: 11.2 us against 10.0 with one tile a block) is what the rounds keep away.
+// GB/s of either), so packed weights go up to six tiles to a block.  What a unit then pulls: rounds of blocks x (tiles + 16-row groups of
+// activations); more tiles only where that is clearly less, since their registers leave one or two waves a SIMD.  32 rows, [151936, 1536]: 116.5 us with
+// one tile, 80.8 with four (5.8 TB/s); [152064, 3584] 261 -> 182; 64 rows: 358 -> 239.  Three tiles against one, two, four at 32 rows (a row of launches
+// on weights from memory): [1536, 10496] in eight splits 9.7 / 11.7, 11.7, 10.3; [1536, 8960] in eight 9.0 / 12.0, 10.5, 9.6.  Six: [3584, 18944] in five
+// 30.3 against 35.6 with two and 37.4 with four, [4608, 3584] in four 10.7 / 12.4 with one, gate/up with SwiGLU [17920, 1536] 14.1 / 16.2 with two,
+// 64 rows of [37888, 3584] 68.6 / 76.0.  Where one tile's blocks fill a round at most it stays: [2048, 1536] in two splits 4.7 / 5.1.
 static int gemv_rows_tiles(const GemmArgs& a, int S) {
-  if (!a.w_packed || a.M <= 16) return 1;
-  auto cost = [&](int nt) { return (float)(((long)(a.N / (nt * 16)) * S + 255) / 256) * ((float)nt + (float)a.M / 16.f); };
-  if (a.N % 32 != 0) return 1;
-  const int nt = cost(2) < 0.97f * cost(1) ? 2 : 1;      // a tie (17 and 18 rows, two rounds for three): one tile 8.6 us, two 8.7 at [1536, 8960] in eight splits
-  return a.N % 64 == 0 && cost(4) < 0.85f * cost(nt) ? 4 : nt;
+  const bool pairs = a.epilogue == EPI_SWIGLU;
+  const int least = pairs ? 2 : 1;
+  if (!a.w_packed || a.M <= 16) return least;
+  const int tiles = (a.N + 15) / 16;
+  auto cost = [&](int nt) { return (float)(((long)((tiles + nt - 1) / nt) * S + 255) / 256) * ((float)nt + (float)a.M / 16.f); };
+  int nt = least;
+  for (int c : {2, 3, 4, 6})
+    if (c > least && !(pairs && (c & 1)) && cost(c) < (c == 2 ? 0.97f : 0.85f) * cost(nt)) nt = c;
+  return nt;
 }
 template <int NTILE, int MODE>
 static void launch_gemv_tiles(const GemmArgs& a, int S, void* out, int ldo, int cps, hipStream_t st) {
-  const dim3 grid(a.N / (NTILE * 16), S);
+  const dim3 grid((a.N + NTILE * 16 - 1) / (NTILE * 16), S);
   if (a.M <= 32) launch_gemv_mg<NTILE, MODE, true, 2>(grid, a, out, ldo, cps, st);
   else if (a.M <= 48) launch_gemv_mg<NTILE, MODE, true, 3>(grid, a, out, ldo, cps, st);
   else launch_gemv_mg<NTILE, MODE, true, 4>(grid, a, out, ldo, cps, st);
 }
 template <int MODE>
 static void launch_gemv_rows(const GemmArgs& a, int S, void* out, int ldo, int cps, hipStream_t st) {
+  constexpr int LEAST = MODE == 2 ? 2 : 1;
   switch (gemv_rows_tiles(a, S)) {
+    case 6: launch_gemv_tiles<6, MODE>(a, S, out, ldo, cps, st); break;
     case 4: launch_gemv_tiles<4, MODE>(a, S, out, ldo, cps, st); break;
-    case 2: launch_gemv_tiles<2, MODE>(a, S, out, ldo, cps, st); break;
-    default: launch_gemv_l<1, MODE>(dim3((a.N + 15) / 16, S), a, out, ldo, cps, st);
+    case 3: if constexpr (MODE != 2) launch_gemv_tiles<3, MODE>(a, S, out, ldo, cps, st); break;
+    case 2: if constexpr (MODE != 2) { launch_gemv_tiles<2, MODE>(a, S, out, ldo, cps, st); break; } [[fallthrough]];
+    default: launch_gemv_l<LEAST, MODE>(dim3((a.N + 16 * LEAST - 1) / (16 * LEAST), S), a, out, ldo, cps, st);
   }
 }
 
@@ -2495,7 +2505,7 @@ int gemm_bf16(const GemmArgs& a, hipStream_t st) {
   if (skinny) {
     const int nchunk = (a.K + 63) / 64;
     if (a.epilogue == EPI_SWIGLU) {
-      launch_gemv_l<2, 2>(dim3((a.N + 31) / 32, 1), a, a.C, a.ldc, nchunk, st);
+      launch_gemv_rows<2>(a, 1, a.C, a.ldc, nchunk, st);
     } else if (a.partial != nullptr) {
       const int S = a.nsplit > 0 ? a.nsplit : 1;
       if (S > nchunk) return LCC_ERR_SHAPE;

@@ -497,6 +497,20 @@ def test_gemv_17_to_64_rows_in_blocks_of_several_tiles(dev, M, N, K, S):
     assert torch.equal(ops.linear_partial(x, wp, S, packed_shape=(N, K)), ops.linear_partial(x, w, S))
 
 
+@pytest.mark.parametrize("M", [17, 32, 33, 49, 64])
+@pytest.mark.parametrize("N,K,S,epi", [(8320, 320, 1, 0), (8336, 64, 1, 0), (1568, 1088, 8, 0), (20800, 192, 1, 0), (3584, 448, 5, 0), (17888, 128, 1, 4),
+                                       (17920, 192, 1, 4), (17952, 64, 1, 4), (10240, 128, 1, 4), (8256, 320, 1, 4)])
+def test_gemv_17_to_64_rows_in_blocks_of_three_and_six_tiles(dev, M, N, K, S, epi):
+    """Three and six weight tiles (for SwiGLU two, four and six) to a block, with one to five tiles in the last block: as the row-major form, bit for bit."""
+    from livecc_amd import ops
+    x, w = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.03, 2)
+    b = None if epi == 4 else _rand((N,), dev, 0.1, 3)
+    wp = ops.pack_weight(w)
+    assert torch.equal(ops.linear(x, wp, b, epi, packed_shape=(N, K)), ops.linear(x, w, b, epi))
+    if epi == 0:
+        assert torch.equal(ops.linear_partial(x, wp, S, packed_shape=(N, K)), ops.linear_partial(x, w, S))
+
+
 @pytest.mark.parametrize("M", [17, 40, 64])
 @pytest.mark.parametrize("I,K", [(512, 256), (18944, 3584)])
 def test_gemv_17_to_64_rows_swiglu(dev, M, I, K):
