@@ -1459,15 +1459,16 @@ __global__ __launch_bounds__(512) void gemm_vh_kernel(
 //     takes the 4-row-tile code path; a wave without rows only feeds the DMA ring.
 //   * LDS: A image 448 rows x 128 B (XOR-swizzled 16-byte chunks, as gemm_big_kernel) + W tile 20 fragment sub-tiles of 1 KB =
 //     77,824 B per stage, two stages = 155,648 B; per k-step 76 KB of DMA (1216 clk at 64 B/clk) under 2240 clk of MFMA issue.
-// Requires packed bf16 W, K % 64 == 0.
-template <int EPI, int SCHED>
+// Requires packed W, K % 64 == 0.  W8: fp8 weights in their packed order, converted after the LDS read (each of the four M-waves converts the columns
+// it multiplies: 96 conversions of 16 bytes beside 84 MFMAs), their scale in the epilogue.
+template <int EPI, int SCHED, bool W8>
 __global__ __launch_bounds__(512) void gemm_tall_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
     const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
-    bf16_t* __restrict__ C, int ldc, int M, int N, int K) {
+    bf16_t* __restrict__ C, int ldc, int M, int N, int K, const float* __restrict__ wscale) {
   constexpr int BM = 448, BN = 160, BK = 64, WM = 112, MT = 7, NT0 = 6;
   constexpr int A_UNITS = BM * 8;                 // 16-byte units of the A image
-  constexpr int B_SUB = (BN / 16) * 2;            // 20 fragment sub-tiles of 1 KB
+  constexpr int B_SUB = (BN / 16) * (W8 ? 1 : 2); // 20 fragment sub-tiles of 1 KB (W8: 10, each a fragment's 64 k)
   constexpr int STAGE = A_UNITS + B_SUB * 64;
   constexpr int A_PER_WAVE = BM / 64;             // 7 pieces of 8 rows x 128 B per wave
   extern __shared__ __attribute__((aligned(16))) u32x4 dsmem[];
@@ -1487,14 +1488,16 @@ __global__ __launch_bounds__(512) void gemm_tall_kernel(
     aoffs[q] = min(row, M - 1) * lda + (((lane & 7) ^ (lane >> 3)) << 3);
   }
   // W sub-tiles: waves 0-3 copy three each (0..11), waves 4-7 two each (12..19); sub-tile st = fragment row st >> 1, 32-k block st & 1
-  const int nb = wave < 4 ? 3 : 2;
-  const int st0 = wave < 4 ? wave * 3 : 12 + (wave - 4) * 2;
-  const bf16_t* bsrc[3];
+  // (W8: waves 0 and 1 two, the others one)
+  constexpr int NB = W8 ? 2 : 3, WK = W8 ? 512 : 1024;       // pieces of a wave at most; elements of W (2 bytes) from k-tile to k-tile
+  const int nb = W8 ? (wave < 2 ? 2 : 1) : (wave < 4 ? 3 : 2);
+  const int st0 = W8 ? (wave < 2 ? wave * 2 : wave + 2) : (wave < 4 ? wave * 3 : 12 + (wave - 4) * 2);
+  const bf16_t* bsrc[NB];
 #pragma unroll
-  for (int q = 0; q < 3; ++q) {
+  for (int q = 0; q < NB; ++q) {
     const int st = min(st0 + q, B_SUB - 1);
-    const int fr = min((n0 >> 4) + (st >> 1), nfrag - 1);
-    bsrc[q] = W + ((size_t)fr * K32 + (st & 1)) * 512 + lane * 8;
+    const int fr = min((n0 >> 4) + (W8 ? st : st >> 1), nfrag - 1);
+    bsrc[q] = W8 ? W + (size_t)fr * (K >> 6) * 512 + lane * 8 : W + ((size_t)fr * K32 + (st & 1)) * 512 + lane * 8;
   }
   // Round 6: activation pieces (8 rows each) that lie entirely beyond the last 16-row MFMA tile are not fetched at all -- at M = 386 the rows
   // 400..447 of the 448-row image (6 of 56 pieces: 11 % of the activation DMA, which is 70 % of this kernel's L2 -> LDS traffic) were copies
@@ -1507,9 +1510,9 @@ __global__ __launch_bounds__(512) void gemm_tall_kernel(
       if ((wave * A_PER_WAVE + q) * 8 < m_rows)
         glds16((A + aoffs[q] + kt * BK), lds_addr(sbase + (wave * A_PER_WAVE + q) * 64));
 #pragma unroll
-    for (int q = 0; q < 3; ++q)
+    for (int q = 0; q < NB; ++q)
       if (q < nb)
-        glds16((bsrc[q] + (size_t)kt * 1024), lds_addr(sbase + A_UNITS + (st0 + q) * 64));
+        glds16((bsrc[q] + (size_t)kt * WK), lds_addr(sbase + A_UNITS + (st0 + q) * 64));
   };
 
   // SCHED 2: the 10 pieces of a wave (7 activation + 3 W; waves 4-7 repeat their second W sub-tile as the third) go out ONE at a time
@@ -1522,10 +1525,10 @@ __global__ __launch_bounds__(512) void gemm_tall_kernel(
         glds16((A + aoffs[q < A_PER_WAVE ? q : 0] + kt * BK), lds_addr(sbase + (wave * A_PER_WAVE + q) * 64));
     } else {
       const int qq = min(q - A_PER_WAVE, nb - 1);
-      glds16((bsrc[qq] + (size_t)kt * 1024), lds_addr(sbase + A_UNITS + (st0 + qq) * 64));
+      glds16((bsrc[qq] + (size_t)kt * WK), lds_addr(sbase + A_UNITS + (st0 + qq) * 64));
     }
   };
-  constexpr int NPIECE = A_PER_WAVE + 3;
+  constexpr int NPIECE = A_PER_WAVE + NB;
 
   f32x4 acc[MT][NT0];
 #pragma unroll
@@ -1537,8 +1540,8 @@ __global__ __launch_bounds__(512) void gemm_tall_kernel(
   issue(0, 0);
   int aoff[2];
 #pragma unroll
-  for (int kk = 0; kk < 2; ++kk) aoff[kk] = (wm * WM + li) * 8 + ((kk * 4 + g) ^ (li & 7));
-  const int boff = A_UNITS + (wn * NT0 * 2) * 64 + lane;
+  for (int kk = 0; kk < 2; ++kk) aoff[kk] = (wm * WM + li) * 8 + ((W8 ? g * 2 + kk : kk * 4 + g) ^ (li & 7));
+  const int boff = A_UNITS + (wn * NT0 * (W8 ? 1 : 2)) * 64 + lane;
 
   // one k-tile of this wave: MTW live row tiles x NTW column tiles.  Per 32-k half: the NTW W fragments are read up front, the
   // activation fragments stream through a 3-register ring two row tiles ahead of their MFMAs.
@@ -1548,7 +1551,12 @@ __global__ __launch_bounds__(512) void gemm_tall_kernel(
     for (int kk = 0; kk < 2; ++kk) {
       bf16x8 fb[NTW], fa[3];
 #pragma unroll
-      for (int j = 0; j < NTW; ++j) fb[j] = as_bf16x8(s[boff + (j * 2 + kk) * 64]);
+      for (int j = 0; j < NTW; ++j) {
+        if constexpr (W8) {          // this half's 8 of the lane's 16 k: half a fragment slot
+          const u32x2 raw = *reinterpret_cast<const u32x2*>(reinterpret_cast<const unsigned char*>(s + boff + j * 64) + kk * 8);
+          fb[j] = fp8x8_to_bf16x8(raw[0], raw[1]);
+        } else fb[j] = as_bf16x8(s[boff + (j * 2 + kk) * 64]);
+      }
       fa[0] = as_bf16x8(s[aoff[kk]]);
       if (MTW > 1) fa[1] = as_bf16x8(s[aoff[kk] + 128]);
 #pragma unroll
@@ -1594,7 +1602,7 @@ __global__ __launch_bounds__(512) void gemm_tall_kernel(
     if (SCHED == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if constexpr (MTW > 0)
       tile_epilogue<EPI, (MTW > 0 ? MTW : 1), (MTW > 0 ? NTW : 2), MT, NT0>(acc, wm * WM, nbase, nbase / 2, li, g, bias, residual, ldr, C, ldc, M, N,
-                                                                        nullptr, nullptr);
+                                                                        nullptr, wscale);
   };
   if (mt_live == 0) run(I0{}, I4{});                 // no rows: DMA + barriers only
   else if (wn == 0) { if (mt_live <= 4) run(I4{}, I6{}); else run(I7{}, I6{}); }
@@ -1714,7 +1722,8 @@ static void launch_big(const GemmArgs& a, hipStream_t st) {
   // bit-identical to the burst-behind-the-barrier order SCHED 1 -- tools/gemm_checksum.py -- and 1.6-3.3 % faster on the prefill
   // GEMMs, +0.6 / +0.8 % tokens/s at 1 / 8 streams, profiles/r03/gemm_sched_spread_dma.txt); LCC_GEMM_SCHED=1 restores SCHED 1
   static const int spread = [] { const char* v = getenv("LCC_GEMM_SCHED"); return (v && atoi(v) == 1) ? 0 : 1; }();
-  if (a.w_fp8) launch_big_s<(BM == 192 || BM == 160 ? 256 : BM), EPI, 1, true>(a, st);     // 192 and 160 rows are bf16-weight shapes (big_tile_rows never picks them for fp8)
+  // fp8 weights: spread pieces on 256 rows (4096 x 3584, K 18944 415 -> 405 us, x 4608, K 3584 161 -> 156), a burst on 128 (386 x 37888 149 against 155)
+  if (a.w_fp8) launch_big_s<(BM == 192 || BM == 160 ? 256 : BM), EPI, (BM == 128 ? 1 : 6), true>(a, st);     // 192 and 160 rows are bf16-weight shapes (big_tile_rows never picks them for fp8)
   else if (g_gemm_sched && spread) {
     // 128-row tiles that fill one round at most have nothing to walk, and the walk's longer prologue shows: 4,006 x 1536, K 768 17.6 us there, 19.1 walked;
     // vision fc1 of one chunk 27.7 / 28.6.  (192 and 256 rows gain from the scalar addresses: 4096 x 3584, K 3584 fp32 105.9 -> 102.5.)
@@ -1822,35 +1831,35 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr) {    
 
 // The tall kernel serves one-block-row problems whose column tiles fill most of ONE round of the chip (7B gate/up at a streaming
 // chunk: 237 blocks).  Variant 8 forces it wherever it is legal (tests).
-static bool tall_legal(const GemmArgs& a) { return big_eligible(a) && !a.w_fp8 && a.M <= 448 && (a.N & 15) == 0; }
+static bool tall_legal(const GemmArgs& a) { return big_eligible(a) && a.M <= 448 && (a.N & 15) == 0; }
 static bool tall_wanted(const GemmArgs& a) {
   if (!tall_legal(a)) return false;
   if (g_gemm_variant == 8) return true;
   if (g_gemm_variant != 2) return false;
   const int blocks = (a.N + 159) / 160;
-  return a.M > 256 && blocks >= 192 && blocks <= 256;
+  // fp8 weights: where 128-row tiles would need a fourth row of blocks (386 x 37888, K 3584 with SwiGLU 149 -> 107 us; 300 rows 101 / 103, 272 rows 107 / 105)
+  return a.M > (a.w_fp8 ? 384 : 256) && blocks >= 192 && blocks <= 256;
 }
 // (a 4-stage ring of 32-k half tiles in the same LDS was measured equal-to-slower -- 122.5 vs 125.2 us at M = 386, profiles/r03/gemm_tall_ring.txt:
 // the L2 -> LDS DMA is throughput-bound, a deeper ring has nothing to hide -- and was retired in round 5)
+template <int EPI, int SCHED, bool W8>
+static void launch_tall_s(const GemmArgs& a, hipStream_t st) {
+  constexpr size_t lds = (size_t)2 * (448 * 8 + (W8 ? 10 : 20) * 64) * 16;   // 155,648 B; fp8 weights 135,168 B
+  static DeviceOnce attr_set;   // per instantiation
+  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_tall_kernel<EPI, SCHED, W8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  gemm_tall_kernel<EPI, SCHED, W8><<<dim3((a.N + 159) / 160), dim3(512), lds, st>>>(a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K,
+                                                                                   a.wscale);
+}
 template <int EPI>
 static void launch_tall(const GemmArgs& a, hipStream_t st) {
   g_launch_counts[LC_GEMM_TALL]++;
-  constexpr size_t lds = (size_t)2 * (448 * 8 + 20 * 64) * 16;   // 155,648 B
-  static DeviceOnce attr_set;   // per instantiation
-  if (attr_set.first()) {
-    (void)hipFuncSetAttribute((const void*)gemm_tall_kernel<EPI, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    (void)hipFuncSetAttribute((const void*)gemm_tall_kernel<EPI, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    (void)hipFuncSetAttribute((const void*)gemm_tall_kernel<EPI, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  }
   // 0 compiler order, 1 pinned (default since round 6: 127.6 vs 131.6-132.6 us at M = 386 on N(0,1) activations, A/B/A/B, bit-identical --
   // profiles/r06/m386_gemms_tall_sched_ab.jsonl; before the LDS-DMA went into inline asm the compiler's order had been the faster one), 2 pinned + spread DMA
   static const int sched = [] { const char* v = getenv("LCC_TALL_SCHED"); return v ? atoi(v) : 1; }();
-  if (sched == 2)
-    gemm_tall_kernel<EPI, 2><<<dim3((a.N + 159) / 160), dim3(512), lds, st>>>(a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K);
-  else if (sched == 1)
-    gemm_tall_kernel<EPI, 1><<<dim3((a.N + 159) / 160), dim3(512), lds, st>>>(a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K);
-  else
-    gemm_tall_kernel<EPI, 0><<<dim3((a.N + 159) / 160), dim3(512), lds, st>>>(a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K);
+  if (a.w_fp8) { if (sched == 2) launch_tall_s<EPI, 2, true>(a, st); else if (sched == 0) launch_tall_s<EPI, 0, true>(a, st); else launch_tall_s<EPI, 1, true>(a, st); }
+  else if (sched == 2) launch_tall_s<EPI, 2, false>(a, st);
+  else if (sched == 1) launch_tall_s<EPI, 1, false>(a, st);
+  else launch_tall_s<EPI, 0, false>(a, st);
 }
 
 template <int EPI>
@@ -1881,7 +1890,7 @@ int gemm_plan(int M, int N, int K, int epilogue, int nsplit, bool w_fp8) {
   if (nsplit > 0) a.partial = &dummy;      // never dereferenced here: only "is this the slab form?"
   const bool skinny = gemm_routes_skinny(M, K, w_fp8) && epilogue != EPI_QUICK_GELU && epilogue != EPI_GELU_ERF && epilogue != EPI_RESIDUAL;
   if (skinny) return 16;
-  if (nsplit <= 0 && !w_fp8 && tall_wanted(a)) return 448;
+  if (nsplit <= 0 && tall_wanted(a)) return 448;
   const int big = big_tile_rows(a, nsplit > 0 ? nsplit : 1);
   return big != 0 ? big : 64;
 }
@@ -2438,10 +2447,11 @@ static int gemm_w8(const GemmArgs& a, hipStream_t st) {
     const bool part = a.partial != nullptr;
     if (part && (a.epilogue != EPI_NONE || a.nsplit < 1 || a.nsplit > 8 || a.nsplit > a.K / 64)) return LCC_ERR_ARG;
     if (a.epilogue == EPI_RESIDUAL && a.residual == nullptr) return LCC_ERR_ARG;
+    const bool tall = !part && tall_wanted(c);
     const int big = (g_gemm_variant == 7) ? 0 : big_tile_rows(c, part ? a.nsplit : 1);
-    if (big != 0) {
-#define LCC_BIG8(EPI) (big == 256 ? launch_big<256, EPI>(c, st) : launch_big<128, EPI>(c, st))
-      if (part) { LCC_BIG8(EPI_PARTIAL); return 0; }
+    if (big != 0 || tall) {
+#define LCC_BIG8(EPI) (tall ? launch_tall<EPI>(c, st) : big == 256 ? launch_big<256, EPI>(c, st) : launch_big<128, EPI>(c, st))
+      if (part) { big == 256 ? launch_big<256, EPI_PARTIAL>(c, st) : launch_big<128, EPI_PARTIAL>(c, st); return 0; }
       switch (a.epilogue) {
         case EPI_NONE: LCC_BIG8(EPI_NONE); return 0;
         case EPI_QUICK_GELU: LCC_BIG8(EPI_QUICK_GELU); return 0;

@@ -420,6 +420,26 @@ def test_gemm_w8_tiled(dev, M, N, K, epi, variant):
     assert (part.sum(0) - r32).abs().max().item() <= 2e-5 * float(r32.abs().max()) * math.sqrt(K / 256) + 1e-5
 
 
+@pytest.mark.parametrize("M", [17, 113, 225, 337, 385, 386, 448])
+@pytest.mark.parametrize("N,K,epi", [(352, 192, 0), (160, 64, 1), (480, 320, 3), (352, 128, 4)])
+def test_gemm_w8_tall(dev, M, N, K, epi):
+    """fp8 weights in the tile that holds all rows (variant 8): a last block of 32 columns, waves with all, some and none of their rows."""
+    from livecc_amd import ops
+    from livecc_amd.weights import dequantize_fp8_rows, quantize_fp8_rows
+    x, w = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.05, 2).float()
+    b = None if epi == 4 else _rand((N,), dev, 0.1, 3)
+    res = _rand((M, N), dev, 1.0, 4) if epi == 3 else None
+    q, sc = quantize_fp8_rows(w)
+    w8, _ = ops.quantize_fp8(w)
+    ops.set_gemm_variant(8)
+    try:
+        got = ops.linear_w8(x, w8, sc, b, epi, res)
+    finally:
+        ops.set_gemm_variant(ops.GEMM_DEFAULT_VARIANT)
+    ref, atol = _ref_linear(x, dequantize_fp8_rows(q, sc), b, epi, res, with_atol=True)
+    assert_bf16_close(got, ref, f"gemm_w8_tall[{M}x{N}x{K},epi{epi}]", max_ulp=1.0, max_frac=5e-3, atol=atol)
+
+
 def test_gemm_no_bias_identity_layout(dev):
     """A = I with an asymmetric W catches a transposed C write (symmetric inputs would not)."""
     from livecc_amd import ops
