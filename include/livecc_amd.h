@@ -142,9 +142,9 @@ int lcc_gemv_num_splits(int N, int K);
 /* nn.Linear with fp8 (OCP e4m3) weights, the 72B single-GPU path: W8 = bytes in the PACKED8 order
  * [N/16][K/64][4 g][16 rows][16 k] (lane (g,row) owns 16 consecutive k), wscale = fp32 [N] per-output-row scale:
  * y[m][n] = epilogue(wscale[n] * sum_k x[m][k] * q[n][k] (+ bias[n])).  M <= 16: weight-streaming GEMV (e4m3 -> bf16 exactly
- * in registers, bf16 MFMA, fp32 accumulate).  M > 16: the 8-wave GEMM stages the fp8 fragments themselves (half the L2 -> LDS bytes) and
- * expands them to bf16 after the LDS read, the row scale in its epilogue; only shapes with too few 256-column tiles for that kernel fall
- * back to an exact dequantisation into dq_scratch (N*K bf16, caller-provided) + the bf16 GEMM.  K % 64 == 0, N % 16 == 0.  partial /
+ * in registers, bf16 MFMA, fp32 accumulate).  M > 16: the GEMM tiles stage the fp8 fragments themselves (half the L2 -> LDS bytes) and
+ * expand them to bf16 after the LDS read, the row scale in their epilogue.  dq_scratch (N*K bf16, caller-provided) holds the exactly dequantised
+ * weight where a forced tile variant has no such form.  K % 64 == 0, N % 16 == 0.  partial /
  * nsplit as in lcc_gemm_bf16. */
 int lcc_gemm_w8_bf16(const void* A, int lda, const void* W8, const float* wscale, const void* bias, const void* residual, int ldr,
                      void* C, int ldc, int M, int N, int K, int epilogue, float* partial, int nsplit, void* dq_scratch, void* stream);

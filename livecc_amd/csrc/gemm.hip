@@ -597,15 +597,18 @@ __global__ __launch_bounds__(256) void gemm_glds_kernel(
 // 128-row tile: 1000 x 3584, K 22528 285 -> 196; 2000 x 1280, K 5120 55 -> 41.
 // NST 6 / 4 stages (64- / 128-row tile): one block on a compute unit.  NST 3 (72 KB, two blocks): more than 256 blocks of the 64-row tile
 // (2912 x 1280, K 5120: 57 us, gemm_glds_kernel 77).
-// Requires packed bf16 W, K % 64 == 0.
-template <int BM, int EPI, int NST>
+// Requires packed W, K % 64 == 0.  W8: fp8 weights in their packed order, 1 KB a fragment's 64 k, converted in registers in front of the
+// MFMAs (the form before wrote the whole weight as bf16 first): 386 x 4608, K 3584 34.5 -> 25; 64 rows in four splits, [3584, 18944] 58 -> 29,
+// [3584, 3584] 20 -> 9.3; 128-row tile: 600 x 4608, K 3584 50 -> 34.
+template <int BM, int EPI, int NST, bool W8>
 __global__ __launch_bounds__(512) void gemm_mid_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual,
     int ldr, bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n, float* __restrict__ partial, int kt_per_split,
     const float* __restrict__ wscale, int raster) {
   constexpr int BN = 128, BK = 64, MT = BM / 32, NT = 2;
-  constexpr int A_UNITS = BM * 8, STAGE = A_UNITS + 16 * 64;      // 16-byte units: [BM rows][8 chunks] (XOR-swizzled) + 16 weight sub-tiles = 24 / 32 KB
-  constexpr int APW = BM / 64, P = APW + 2;                       // DMA pieces of a wave per k-tile: 8 activation rows each, then the weights
+  constexpr int WF = W8 ? 1 : 2;                                  // 1-KB weight sub-tiles of a fragment row
+  constexpr int A_UNITS = BM * 8, STAGE = A_UNITS + 8 * WF * 64;  // 16-byte units: [BM rows][8 chunks] (XOR-swizzled) + 16 weight sub-tiles = 24 / 32 KB
+  constexpr int APW = BM / 64, P = APW + WF;                      // DMA pieces of a wave per k-tile: 8 activation rows each, then the weights
   extern __shared__ __attribute__((aligned(16))) u32x4 dsmem[];
 
   const int nblk = tiles_m * tiles_n;
@@ -635,7 +638,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(
   const bf16_t* asrc[APW];
 #pragma unroll
   for (int q = 0; q < APW; ++q) asrc[q] = A + (size_t)min(m0 + (wave + 8 * q) * 8 + (lane >> 3), M - 1) * lda + (((lane & 7) ^ (lane >> 3)) << 3);
-  const bf16_t* bsrc = W + (size_t)min((n0 >> 4) + wave, nfrag - 1) * K32 * 512 + lane * 8;
+  const bf16_t* bsrc = W + (size_t)min((n0 >> 4) + wave, nfrag - 1) * (W8 ? K32 >> 1 : K32) * 512 + lane * 8;
   const unsigned lds0 = lds_addr(dsmem);
   const int nkt_all = K / BK;
   const int kt0 = (EPI == EPI_PARTIAL) ? blockIdx.y * kt_per_split : 0;
@@ -645,8 +648,8 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(
     const unsigned base = lds0 + (unsigned)(stage * STAGE) * 16u;
 #pragma unroll
     for (int q = 0; q < APW; ++q) glds16(asrc[q] + (size_t)k * BK, base + (wave + 8 * q) * 1024u);
-    glds16(bsrc + (size_t)k * 1024, base + (A_UNITS + wave * 128) * 16u);
-    glds16(bsrc + (size_t)k * 1024 + 512, base + (A_UNITS + wave * 128 + 64) * 16u);
+#pragma unroll
+    for (int h = 0; h < WF; ++h) glds16(bsrc + (size_t)k * (WF * 512) + h * 512, base + (A_UNITS + (wave * WF + h) * 64) * 16u);
   };
 
   f32x4 acc[MT][NT];
@@ -656,9 +659,9 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(
     for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
   int aoff[2];
 #pragma unroll
-  for (int kk = 0; kk < 2; ++kk) aoff[kk] = (wm * (BM / 2) + li) * 8 + ((kk * 4 + g) ^ (li & 7));
-  const int boff = A_UNITS + wn * 4 * 64 + lane;
-  struct Frag { bf16x8 a[2][MT], b[2][NT]; };
+  for (int kk = 0; kk < 2; ++kk) aoff[kk] = (wm * (BM / 2) + li) * 8 + ((W8 ? g * 2 + kk : kk * 4 + g) ^ (li & 7));
+  const int boff = A_UNITS + wn * NT * WF * 64 + lane;
+  struct Frag { bf16x8 a[2][MT]; u32x4 b[WF][NT]; };
   auto read = [&](Frag& f, int stage) {
     const u32x4* s = dsmem + stage * STAGE;
 #pragma unroll
@@ -666,16 +669,21 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(
 #pragma unroll
       for (int i = 0; i < MT; ++i) f.a[kk][i] = as_bf16x8(s[aoff[kk] + i * 128]);
 #pragma unroll
-      for (int j = 0; j < NT; ++j) f.b[kk][j] = as_bf16x8(s[boff + (j * 2 + kk) * 64]);
+      for (int j = 0; j < NT; ++j)
+        if (kk < WF) f.b[kk % WF][j] = s[boff + (j * WF + kk) * 64];
     }
   };
   auto mul = [&](const Frag& f) {
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
+    for (int kk = 0; kk < 2; ++kk) {
+      bf16x8 b[NT];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) b[j] = W8 ? fp8x8_to_bf16x8(f.b[0][j][2 * kk], f.b[0][j][2 * kk + 1]) : as_bf16x8(f.b[kk % WF][j]);
 #pragma unroll
       for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) acc[i][j] = mfma16(f.b[kk][j], f.a[kk][i], acc[i][j]);
+        for (int j = 0; j < NT; ++j) acc[i][j] = mfma16(b[j], f.a[kk][i], acc[i][j]);
+    }
   };
   // tile kt + 1 has landed (this wave's pieces; NST - 3 newer tiles may stay in flight) -> barrier -> DMA of tile kt + NST - 1 into the stage
   // of tile kt - 1 (its fragments were in registers before the barrier) -> fragment reads of tile kt + 1 -> MFMAs of tile kt
@@ -1617,22 +1625,27 @@ static int g_gemm_sched = 1;   // fragment-read schedule of gemm_big_kernel: 0 c
 void set_gemm_variant(int v);
 
 static inline int raster_for(int tiles_m);
-template <int BM, int EPI, int NST>
-static void launch_mid(const GemmArgs& a, hipStream_t st) {
+template <int BM, int EPI, int NST, bool W8>
+static void launch_mid_w(const GemmArgs& a, hipStream_t st) {
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + 127) / 128, nkt = a.K / 64, S = (EPI == EPI_PARTIAL) ? a.nsplit : 1;
-  constexpr size_t lds = (size_t)NST * (BM * 128 + 16384);
+  constexpr size_t lds = (size_t)NST * (BM * 128 + (W8 ? 8192 : 16384));
   static DeviceOnce attr_set;   // per instantiation
-  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_mid_kernel<BM, EPI, NST>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  gemm_mid_kernel<BM, EPI, NST><<<dim3(capped_grid((long)tiles_m * tiles_n), S), dim3(512), lds, st>>>(
+  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_mid_kernel<BM, EPI, NST, W8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  gemm_mid_kernel<BM, EPI, NST, W8><<<dim3(capped_grid((long)tiles_m * tiles_n), S), dim3(512), lds, st>>>(
       a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.partial, (nkt + S - 1) / S, a.wscale, raster_for(tiles_m));
+}
+template <int BM, int EPI, int NST>
+static void launch_mid(const GemmArgs& a, hipStream_t st) { a.w_fp8 ? launch_mid_w<BM, EPI, NST, true>(a, st) : launch_mid_w<BM, EPI, NST, false>(a, st); }
+// the 64 x 128 tile
+template <int EPI>
+static void launch_mid64(const GemmArgs& a, hipStream_t st) {
+  const long blocks = (long)capped_grid((long)((a.M + 63) / 64) * ((a.N + 127) / 128)) * (EPI == EPI_PARTIAL ? a.nsplit : 1);
+  return blocks <= 256 ? launch_mid<64, EPI, 6>(a, st) : launch_mid<64, EPI, 3>(a, st);
 }
 template <int BM, int EPI>
 static void launch_tiled(const GemmArgs& a, hipStream_t st) {
   if constexpr (BM == 64) {
-    if ((g_gemm_variant == 2 || g_gemm_variant == 7) && a.w_packed && (a.K & 63) == 0) {
-      const long blocks = (long)capped_grid((long)((a.M + 63) / 64) * ((a.N + 127) / 128)) * (EPI == EPI_PARTIAL ? a.nsplit : 1);
-      return blocks <= 256 ? launch_mid<64, EPI, 6>(a, st) : launch_mid<64, EPI, 3>(a, st);
-    }
+    if ((g_gemm_variant == 2 || g_gemm_variant == 7) && a.w_packed && (a.K & 63) == 0) return launch_mid64<EPI>(a, st);
   }
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + 127) / 128;
   const int nkt = (a.K + 63) / 64, S = (EPI == EPI_PARTIAL) ? a.nsplit : 1;
@@ -1736,7 +1749,7 @@ static void launch_big(const GemmArgs& a, hipStream_t st) {
   else launch_big_s<(BM == 160 ? 192 : BM), EPI, 0, false>(a, st);
 }
 // 13 / 17: the 192- / 160-row tile wherever eligible (bf16 weights); 14: variable-height row tiles (gemm_vh_kernel) wherever legal, else as 3;
-// 16: 128 x 128 tiles (gemm_mid_kernel) wherever eligible, bf16 weights
+// 16: 128 x 128 tiles (gemm_mid_kernel) wherever eligible
 // 15: the small variable-height class (8 / 9 fragments) for split-K slabs wherever legal, else as 4
 void set_gemm_variant(int v) {
   g_gemm_variant = v;
@@ -1782,7 +1795,7 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr) {    
   if (g_gemm_variant == 13) return a.w_fp8 ? 256 : 192;
   if (g_gemm_variant == 17) return a.w_fp8 ? 256 : 160;
   if (g_gemm_variant == 15) return (a.partial != nullptr && vh_small_shape(a.M, a.K) && vh_legal(a, true)) ? 144 : 128;
-  if (g_gemm_variant == 16) return a.w_fp8 ? 128 : 129;
+  if (g_gemm_variant == 16) return 129;
   if (g_gemm_variant != 2) return 0;
   const float s256 = tile_score(a.M, a.N, S, 256, 256, 256, 1.0f, true);
   static const int allow192 = [] { const char* v = getenv("LCC_GEMM_192"); return v ? atoi(v) : 1; }();     // A/B: 0 = round-3 tile choice
@@ -1795,10 +1808,10 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr) {    
   // gemm_mid_kernel: 0.38 / 0.52 us a step of 64 x 128 / 128 x 128 against 0.85 of 128 x 256, one tile a compute unit at a time (two 64-row
   // tiles side by side take twice as long).  Returned as 0 / 129.  The 128-row form wins where its blocks fill one round and the 64-row
   // form's need two; beyond a round the 256-column tiles do (shapes around the lines: 1000 x 3584, K 3584: 43 / 34 / 52 us for 64 x 128 /
-  // 128 x 128 / 128 x 256; 1456 x 3584: 73 / 61 / 52; 520 x 3584: 25 / 33 / 50).  fp8 weights: the 64-row tile means a pass that
-  // dequantises first, scored as measured with it.
-  const float s64 = a.w_fp8 ? tile_score(a.M, a.N, S, 64, 128, 512, 0.55f, false) : tile_score(a.M, a.N, S, 64, 128, 256, 0.48f, false);
-  const float s128m = a.w_fp8 ? 0.f : tile_score(a.M, a.N, S, 128, 128, 256, 0.70f, false);
+  // 128 x 128 / 128 x 256; 1456 x 3584: 73 / 61 / 52; 520 x 3584: 25 / 33 / 50).  With fp8 weights the steps stand alike (4608, K 3584: 386 rows
+  // 25 / 33 / 49, 600 rows 42 / 34 / 50, 1000 rows 73 / 61 / 49; 200 x 3584, K 18944 in four splits 68 / 48 / 66).
+  const float s64 = tile_score(a.M, a.N, S, 64, 128, 256, 0.48f, false);
+  const float s128m = tile_score(a.M, a.N, S, 128, 128, 256, 0.70f, false);
   if (score) *score = std::max(std::max(std::max(s256, s192), std::max(s160, s128)), std::max(s128m, s64));
   static const int allow_vh = [] { const char* v = getenv("LCC_GEMM_VH"); return v ? atoi(v) : 1; }();
   if (allow_vh && vh_legal(a) && (((a.M + 15) >> 4) & 15) != 0) {      // F % 16 == 0: the 256-row tiles are the same thing
@@ -2441,7 +2454,7 @@ static int gemm_w8(const GemmArgs& a, hipStream_t st) {
     }
     return 0;
   }
-  // M > 16: the 8-wave kernel consumes the fp8 fragments directly (e4m3 -> bf16 after the LDS read) ...
+  // M > 16: the tile kernels consume the fp8 fragments directly (e4m3 -> bf16 after the LDS read) ...
   {
     GemmArgs c = a; c.w_packed = 1;
     const bool part = a.partial != nullptr;
@@ -2449,21 +2462,23 @@ static int gemm_w8(const GemmArgs& a, hipStream_t st) {
     if (a.epilogue == EPI_RESIDUAL && a.residual == nullptr) return LCC_ERR_ARG;
     const bool tall = !part && tall_wanted(c);
     const int big = (g_gemm_variant == 7) ? 0 : big_tile_rows(c, part ? a.nsplit : 1);
-    if (big != 0 || tall) {
-#define LCC_BIG8(EPI) (tall ? launch_tall<EPI>(c, st) : big == 256 ? launch_big<256, EPI>(c, st) : launch_big<128, EPI>(c, st))
-      if (part) { big == 256 ? launch_big<256, EPI_PARTIAL>(c, st) : launch_big<128, EPI_PARTIAL>(c, st); return 0; }
+    if (big != 0 || tall || g_gemm_variant == 2) {
+#define LCC_W8_TILE(EPI) (big == 256 ? launch_big<256, EPI>(c, st) : big == 128 ? launch_big<128, EPI>(c, st) : big == 129 ? launch_mid<128, EPI, 4>(c, st) : launch_mid64<EPI>(c, st))
+#define LCC_W8(EPI) (tall ? launch_tall<EPI>(c, st) : LCC_W8_TILE(EPI))
+      if (part) { LCC_W8_TILE(EPI_PARTIAL); return 0; }
       switch (a.epilogue) {
-        case EPI_NONE: LCC_BIG8(EPI_NONE); return 0;
-        case EPI_QUICK_GELU: LCC_BIG8(EPI_QUICK_GELU); return 0;
-        case EPI_GELU_ERF: LCC_BIG8(EPI_GELU_ERF); return 0;
-        case EPI_RESIDUAL: LCC_BIG8(EPI_RESIDUAL); return 0;
-        case EPI_SWIGLU: LCC_BIG8(EPI_SWIGLU); return 0;
+        case EPI_NONE: LCC_W8(EPI_NONE); return 0;
+        case EPI_QUICK_GELU: LCC_W8(EPI_QUICK_GELU); return 0;
+        case EPI_GELU_ERF: LCC_W8(EPI_GELU_ERF); return 0;
+        case EPI_RESIDUAL: LCC_W8(EPI_RESIDUAL); return 0;
+        case EPI_SWIGLU: LCC_W8(EPI_SWIGLU); return 0;
         default: return LCC_ERR_ARG;
       }
-#undef LCC_BIG8
+#undef LCC_W8
+#undef LCC_W8_TILE
     }
   }
-  // ... shapes with too few 256-column tiles: exact dequantisation into the bf16 packed order, then the 4-wave bf16 GEMM with
+  // ... forced variants without such a kernel: exact dequantisation into the bf16 packed order, then the 4-wave bf16 GEMM with
   // the row scale in its epilogue
   if (a.dq_scratch == nullptr) return LCC_ERR_ARG;
   const size_t pieces = (size_t)a.N * a.K / 16;

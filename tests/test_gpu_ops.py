@@ -420,6 +420,33 @@ def test_gemm_w8_tiled(dev, M, N, K, epi, variant):
     assert (part.sum(0) - r32).abs().max().item() <= 2e-5 * float(r32.abs().max()) * math.sqrt(K / 256) + 1e-5
 
 
+@pytest.mark.parametrize("M", [17, 64, 65, 127, 200])
+@pytest.mark.parametrize("N,K,epi,S", [(272, 64, 0, 1), (128, 128, 1, 2), (400, 832, 3, 5), (288, 192, 4, 0), (16, 448, 2, 7), (16640, 128, 0, 2)])
+@pytest.mark.parametrize("variant", [2, 16])
+def test_gemm_w8_narrow_tiles(dev, M, N, K, epi, S, variant):
+    """fp8 weights in the 64 x 128 tile (the shipped choice here; with one and with two blocks to a compute unit) and the 128 x 128 one (16): one to
+    thirteen k-tiles, columns and rows that end inside a tile, splits of one k-tile."""
+    from livecc_amd import ops
+    from livecc_amd.weights import dequantize_fp8_rows, quantize_fp8_rows
+    x, w = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.05, 2).float()
+    b = None if epi == 4 else _rand((N,), dev, 0.1, 3)
+    res = _rand((M, N), dev, 1.0, 4) if epi == 3 else None
+    q, sc = quantize_fp8_rows(w)
+    w8, _ = ops.quantize_fp8(w)
+    ops.set_gemm_variant(variant)
+    try:
+        got = ops.linear_w8(x, w8, sc, b, epi, res)
+        part = ops.linear_w8(x, w8, sc, nsplit=S) if S else None
+    finally:
+        ops.set_gemm_variant(ops.GEMM_DEFAULT_VARIANT)
+    wd = dequantize_fp8_rows(q, sc)
+    ref, atol = _ref_linear(x, wd, b, epi, res, with_atol=True)
+    assert_bf16_close(got, ref, f"gemm_w8_mid[{M}x{N}x{K},epi{epi},v{variant}]", max_ulp=1.0, max_frac=5e-3, atol=atol)
+    if part is not None:
+        r32 = x.float() @ wd.t()
+        assert (part.sum(0) - r32).abs().max().item() <= 2e-5 * float(r32.abs().max()) * math.sqrt(K / 256) + 1e-5
+
+
 @pytest.mark.parametrize("M", [17, 113, 225, 337, 385, 386, 448])
 @pytest.mark.parametrize("N,K,epi", [(352, 192, 0), (160, 64, 1), (480, 320, 3), (352, 128, 4)])
 def test_gemm_w8_tall(dev, M, N, K, epi):
