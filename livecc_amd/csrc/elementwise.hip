@@ -85,15 +85,23 @@ __global__ __launch_bounds__(NW * 64) void layernorm_kernel(const bf16_t* __rest
   __shared__ float red[NW];
   const int row = blockIdx.x, tid = threadIdx.x, nchunk = dim / 8;
   const bf16_t* xr = x + (size_t)row * dim;
+  // the row, the weights and the biases are asked for at once, at clamped addresses: behind branches a row of 1,280 was three trips to memory in a row and the
+  // weights a fourth (in a row of launches: 1,456 rows 4.1 -> 3.6 us, 15,840 rows 15.6 -> 14.0)
+  u32x4 xq[MAXC], wq[MAXC], bq[MAXC];
+#pragma unroll
+  for (int c = 0; c < MAXC; ++c) xq[c] = ld16(xr + min(tid + c * NW * 64, nchunk - 1) * 8);
+#pragma unroll
+  for (int c = 0; c < MAXC; ++c) {
+    const int at = min(tid + c * NW * 64, nchunk - 1) * 8;
+    wq[c] = ld16(w + at); bq[c] = ld16(b + at);
+  }
   float v[MAXC][8];
   float s = 0.f;
 #pragma unroll
   for (int c = 0; c < MAXC; ++c) {
-    const int ch = tid + c * NW * 64;
-    if (ch < nchunk) {
-      const u32x4 q = ld16(xr + ch * 8);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) { v[c][2 * e] = lo2f(q[e]); v[c][2 * e + 1] = hi2f(q[e]); }
+    for (int e = 0; e < 4; ++e) { v[c][2 * e] = lo2f(xq[c][e]); v[c][2 * e + 1] = hi2f(xq[c][e]); }
+    if (tid + c * NW * 64 < nchunk) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) s += v[c][e];
     }
@@ -114,12 +122,11 @@ __global__ __launch_bounds__(NW * 64) void layernorm_kernel(const bf16_t* __rest
   for (int c = 0; c < MAXC; ++c) {
     const int ch = tid + c * NW * 64;
     if (ch < nchunk) {
-      const u32x4 wq = ld16(w + ch * 8), bq = ld16(b + ch * 8);
       float o[8];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        o[2 * e] = (v[c][2 * e] - mean) * rstd * lo2f(wq[e]) + lo2f(bq[e]);
-        o[2 * e + 1] = (v[c][2 * e + 1] - mean) * rstd * hi2f(wq[e]) + hi2f(bq[e]);
+        o[2 * e] = (v[c][2 * e] - mean) * rstd * lo2f(wq[c][e]) + lo2f(bq[c][e]);
+        o[2 * e + 1] = (v[c][2 * e + 1] - mean) * rstd * hi2f(wq[c][e]) + hi2f(bq[c][e]);
       }
       st16(y + (size_t)row * dim + ch * 8,
            (u32x4){pack2(o[0], o[1]), pack2(o[2], o[3]), pack2(o[4], o[5]), pack2(o[6], o[7])});
@@ -131,7 +138,9 @@ int layernorm_bf16(const bf16_t* x, const bf16_t* w, const bf16_t* b, bf16_t* y,
                    hipStream_t st) {
   if (rows <= 0) return 0;
   if ((dim & 7) || dim > 4 * 64 * 8 * 4) return LCC_ERR_SHAPE;
-  if (dim <= 64 * 8 * 4) layernorm_kernel<1, 4><<<dim3(rows), dim3(64), 0, st>>>(x, w, b, y, dim, eps);
+  if (dim <= 64 * 8 * 2) layernorm_kernel<1, 2><<<dim3(rows), dim3(64), 0, st>>>(x, w, b, y, dim, eps);
+  else if (dim <= 64 * 8 * 3) layernorm_kernel<1, 3><<<dim3(rows), dim3(64), 0, st>>>(x, w, b, y, dim, eps);
+  else if (dim <= 64 * 8 * 4) layernorm_kernel<1, 4><<<dim3(rows), dim3(64), 0, st>>>(x, w, b, y, dim, eps);
   else layernorm_kernel<4, 4><<<dim3(rows), dim3(256), 0, st>>>(x, w, b, y, dim, eps);
   return 0;
 }
