@@ -81,7 +81,7 @@ __global__ __launch_bounds__(NT) void sample_greedy_kernel(
       if (so) so[id] = v[e];
       // online max / exp-sum over ALL scores (softmax denominator of the threshold processor)
       if (v[e] > mx) { sum = sum * __expf(mx - v[e]) + 1.f; mx = v[e]; }
-      else sum += __expf(v[e] - mx);
+      else if (mx > -INFINITY) sum += __expf(v[e] - mx);          // masked scores in front of a thread's first finite one add nothing
       if (id == thr_token) thr_score = v[e];
       else best = better(best, Best{v[e], id});
     }
@@ -129,40 +129,60 @@ __global__ __launch_bounds__(NT) void sample_greedy_kernel(
   }
 }
 
-// ---- two-stage variant: stage 1 spreads the V-wide pass over SAMPLE_NB blocks per stream, stage 2 merges the partials
-constexpr int SAMPLE_NB = 32;
+// ---- two-stage variant: stage 1 spreads the V-wide pass over SAMPLE_NB blocks per stream, stage 2 merges the partials.  A block's 600 chunks of 8 scores
+// are one trip to memory (three chunks a thread, asked for together and before the slot's flags are known), and a chunk moves the running maximum once
+// instead of score by score behind a branch.  Both stages and the fill of the result, one row of 151,936 ids 10.8 -> 9.8 us, 32 rows 12.5 -> 12.1 (two
+// chunks each for 512 threads: 9.1 and 13.5)
+constexpr int SAMPLE_NB = 32, SAMPLE_NT = 256;
 
 template <class LT>
-__global__ __launch_bounds__(256) void sample_partial_kernel(
+__global__ __launch_bounds__(SAMPLE_NT) void sample_partial_kernel(
     const LT* __restrict__ logits, int ld, int V, const uint32_t* __restrict__ seen, int words,
     const int32_t* __restrict__ stream_slot, float penalty, int thr_token, int eos_token, int eos_token2, int suppress_eos,
     const int32_t* __restrict__ done, float* __restrict__ part, float* __restrict__ scores_out) {
-  __shared__ float s_max[4], s_sum[4], s_bv[4], s_thr[4];
-  __shared__ int s_bi[4];
+  constexpr int NW = SAMPLE_NT / 64, U = 3;
+  __shared__ float s_max[NW], s_sum[NW], s_bv[NW], s_thr[NW];
+  __shared__ int s_bi[NW];
   const int b = blockIdx.y, blk = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int slot = stream_slot[b];
-  if (done != nullptr && done[slot]) return;
+  const bool frozen = done != nullptr && done[slot];          // writes nothing
   const LT* lg = logits + (size_t)b * ld;
   const uint32_t* sb = seen + (size_t)slot * words;
-  float* so = scores_out ? scores_out + (size_t)b * V : nullptr;
+  float* so = scores_out && !frozen ? scores_out + (size_t)b * V : nullptr;
   const int nch = V / 8, per = (nch + SAMPLE_NB - 1) / SAMPLE_NB;
   const int c0 = blk * per, c1 = min(nch, c0 + per);
   Best best = {-INFINITY, 0x7fffffff};
   float mx = -INFINITY, sum = 0.f, thr_score = -INFINITY;
-  for (int c = c0 + tid; c < c1; c += 256) {
-    const uint32_t bits = (sb[c >> 2] >> ((c & 3) * 8)) & 0xffu;
-    float v[8];
-    load8_logits(lg, c, v);
+  for (int cb = c0 + tid; cb < c1; cb += SAMPLE_NT * U) {
+    float v[U][8];
+    uint32_t word[U];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      if (penalty != 1.0f && ((bits >> e) & 1u)) v[e] = v[e] < 0.f ? v[e] * penalty : v[e] / penalty;
-      const int id = c * 8 + e;
-      if ((suppress_eos & 1) && (id == eos_token || id == eos_token2)) v[e] = -INFINITY;
-      if (so) so[id] = v[e];
-      if (v[e] > mx) { sum = sum * __expf(mx - v[e]) + 1.f; mx = v[e]; }
-      else sum += __expf(v[e] - mx);
-      if (id == thr_token) thr_score = v[e];
-      else best = better(best, Best{v[e], id});
+    for (int u = 0; u < U; ++u) load8_logits(lg, min(cb + u * SAMPLE_NT, c1 - 1), v[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u) word[u] = sb[min(cb + u * SAMPLE_NT, c1 - 1) >> 2];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int c = cb + u * SAMPLE_NT;
+      if (c >= c1) continue;
+      const uint32_t bits = (word[u] >> ((c & 3) * 8)) & 0xffu;
+      float cm = -INFINITY;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float& x = v[u][e];
+        if (penalty != 1.0f && ((bits >> e) & 1u)) x = x < 0.f ? x * penalty : x / penalty;
+        const int id = c * 8 + e;
+        if ((suppress_eos & 1) && (id == eos_token || id == eos_token2)) x = -INFINITY;
+        if (so) so[id] = x;
+        cm = fmaxf(cm, x);
+        if (id == thr_token) thr_score = x;
+        else best = better(best, Best{x, id});
+      }
+      // exp-sum over ALL scores (softmax denominator of the threshold processor)
+      if (cm > mx) { sum *= __expf(mx - cm); mx = cm; }
+      if (mx > -INFINITY) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum += v[u][e] == mx ? 1.f : __expf(v[u][e] - mx);
+      }
     }
   }
   float wmx = wave_max(mx);
@@ -176,11 +196,13 @@ __global__ __launch_bounds__(256) void sample_partial_kernel(
   thr_score = wave_max(thr_score);
   if (lane == 0) { s_max[wave] = wmx; s_sum[wave] = sum; s_bv[wave] = best.v; s_bi[wave] = best.i; s_thr[wave] = thr_score; }
   __syncthreads();
-  if (tid == 0) {
+  if (tid == 0 && !frozen) {
     float M = -INFINITY, tot = 0.f, ts = -INFINITY;
     Best bb = {-INFINITY, 0x7fffffff};
-    for (int w = 0; w < 4; ++w) M = fmaxf(M, s_max[w]);
-    for (int w = 0; w < 4; ++w) {
+#pragma unroll
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, s_max[w]);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
       tot += (s_max[w] == -INFINITY) ? 0.f : s_sum[w] * __expf(s_max[w] - M);
       bb = better(bb, Best{s_bv[w], s_bi[w]});
       ts = fmaxf(ts, s_thr[w]);
@@ -236,7 +258,7 @@ static int sample_greedy_t(const LT* logits, int ld, int B, int V, uint32_t* see
   if (B <= 0) return 0;
   if ((V & 31) || (ld & 7) || words_per_stream * 32 < V) return LCC_ERR_SHAPE;
   if (ws != nullptr && V >= 8192) {   // ws: B * 32 * 8 floats of scratch
-    sample_partial_kernel<LT><<<dim3(SAMPLE_NB, B), dim3(256), 0, st>>>(logits, ld, V, seen, words_per_stream, stream_slot, repetition_penalty,
+    sample_partial_kernel<LT><<<dim3(SAMPLE_NB, B), dim3(SAMPLE_NT), 0, st>>>(logits, ld, V, seen, words_per_stream, stream_slot, repetition_penalty,
                                                                    thr_token, eos_token, eos_token2, suppress_eos, done, ws, scores_out);
     sample_final_kernel<<<dim3(B), dim3(64), 0, st>>>(ws, V, stream_slot, thr_token, use_thr, thr_value, eos_token, eos_token2, suppress_eos & 2, done, out_tokens,
                                                       history, hist_ld, hist_col, scores_out);

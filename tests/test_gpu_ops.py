@@ -1122,3 +1122,26 @@ def test_embed_gather_with_video_row_scatter_is_bit_exact(dev):
     slots = torch.tensor([9, 2, 14], dtype=torch.int32)
     got = ops.embed_gather(cur_tok.to(dev), table, indirect=slots.to(dev))
     assert torch.equal(got, table[cur_tok[slots.long()].long().to(dev)])
+
+
+@pytest.mark.parametrize("V", [8192, 8224, 151936, 262144])
+def test_two_stage_sampler_gives_the_single_launch_tokens(dev, V):
+    """The spread pass against the one-block pass: short and long shares of a block (32 to 1,024 chunks for 256 threads), equal scores (the lower id wins), masked
+    ids at the start of a share, penalised ids, and a row that is done, which keeps its token and its scores."""
+    from livecc_amd import ops
+    g = torch.Generator().manual_seed(V)
+    lg = (torch.randn(4, V, generator=g) * 4).bfloat16()
+    lg[0, V - 1] = lg[0, 5] = 60.0
+    lg[1, :4096] = float("-inf")
+    lg[2, V // 2] = 50.0
+    lg = lg.to(dev)
+    seen = torch.randint(-2 ** 31, 2 ** 31 - 1, (4, V // 32), dtype=torch.int32, generator=g).to(dev)
+    slots = torch.arange(4, dtype=torch.int32, device=dev)
+    for kw in (dict(), dict(repetition_penalty=1.15), dict(repetition_penalty=1.15, thr_token=V // 2, thr_value=0.5, eos_token=0, suppress_eos=True)):
+        a, sa = ops.sample_greedy(lg, seen, slots, want_scores=True, **kw)
+        b, sb = ops.sample_greedy(lg, seen, slots, want_scores=True, two_stage=True, **kw)
+        assert torch.equal(a, b) and torch.equal(sa, sb)
+    done = torch.tensor([0, 1, 0, 0], dtype=torch.int32, device=dev)
+    c, _ = ops.sample_greedy(lg, seen, slots, two_stage=True, done=done)
+    a, _ = ops.sample_greedy(lg, seen, slots)
+    assert c[1] == 0 and torch.equal(c[[0, 2, 3]], a[[0, 2, 3]])
