@@ -58,6 +58,55 @@ LCC_DEVICE void gqa_row(const GqaInArgs& a, int row, int part = 0, int parts = 1
   }
 }
 
+// The same by one block of a prefill launch: a head takes dim_pad / 4 lanes, so a wave has two heads of 128 channels side by side, and U groups of heads are
+// asked for together (one head a wave and trip: 32 heads were eight trips).  The sums of squares add in the same order.
+template <int NW, int U>
+LCC_DEVICE void gqa_row_batch(const GqaInArgs& a, int row) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const size_t slab = (size_t)a.rows * a.ldn, at = (size_t)row * a.ldn;
+  const int slot = a.tok_stream[row], nh = a.heads + a.kv_heads;
+  const int vcol = nh * a.dim_pad, nv = a.kv_heads * a.vdim_pad;
+  f32x4 v0 = *reinterpret_cast<const f32x4*>(a.part + at + vcol + min(tid * 4, nv - 4));
+  const int pos = a.tok_pos ? a.tok_pos[row] : a.kv_len[slot];
+  bf16_t* arena = a.kv_base[slot];
+  const int L = (a.dim_pad & (a.dim_pad - 1)) == 0 ? a.dim_pad >> 2 : 64, per = 64 / L, sub = lane / L, c = (lane - sub * L) * 4, cc = min(c, a.dim_pad - 4);
+  const float temp = 1.f + a.temp_coef * logf((float)((pos + 1) / a.temp_every) + 1.f);
+  for (int h0 = wave * per + sub; h0 - sub < nh; h0 += NW * per * U) {
+    f32x4 v[U];
+    u32x2 w[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int h = min(h0 + u * NW * per, nh - 1);
+      v[u] = *reinterpret_cast<const f32x4*>(a.part + at + (size_t)h * a.dim_pad + cc);
+      w[u] = ld8((h < a.heads ? a.q_norm : a.k_norm) + cc);
+    }
+    for (int s = 1; s < a.nsplit; ++s)
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] += *reinterpret_cast<const f32x4*>(a.part + s * slab + at + (size_t)min(h0 + u * NW * per, nh - 1) * a.dim_pad + cc);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int h = h0 + u * NW * per;
+      const bool isq = h < a.heads;
+      float ss = c < a.dim_pad ? (v[u][0] * v[u][0] + v[u][1] * v[u][1]) + (v[u][2] * v[u][2] + v[u][3] * v[u][3]) : 0.f;
+      for (int o = L >> 1; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+      const float r = (isq ? temp : 1.f) / sqrtf(ss / (float)a.dim + a.eps);
+      if (h < nh && c < a.dim_pad) {
+        bf16_t* dst = isq ? a.q + ((size_t)row * a.heads + h) * a.dim_pad : arena + a.k_off + ((size_t)(h - a.heads) * a.lmax + pos) * a.dim_pad;
+        st8(dst + c, pack4(v[u] * r * unpack4(w[u])));
+      }
+    }
+  }
+  for (int p = tid * 4; p < nv; p += NW * 256) {
+    f32x4 v = v0;
+    if (p != tid * 4) v = *reinterpret_cast<const f32x4*>(a.part + at + vcol + p);
+    for (int s = 1; s < a.nsplit; ++s) v += *reinterpret_cast<const f32x4*>(a.part + s * slab + at + vcol + p);
+    const int g = p / a.vdim_pad, d = p - g * a.vdim_pad;
+    bf16_t* dst = arena + a.v_off + (size_t)g * a.lmax * a.vdim_pad + ((size_t)(pos >> 5) * a.vdim_pad + d) * 32 + (pos & 31);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) dst[e * 32] = f2bf(v[e]);
+  }
+}
+
 // Four channels of a recurrent mixer's activated input at `col` of the projection: silu of the value, or of the short causal convolution over the
 // projection's rows (rows of this call from r0 on, older ones out of the slot's ring: position p at row p % taps, zeros before the start).
 LCC_DEVICE f32x4 rec_in4(const RecInArgs& a, int row, int r0, int pos, const float* ring, int col, f32x4* raw) {

@@ -150,6 +150,36 @@ def test_attention_inputs_norms_temperature_and_cache(dev, lib):
         assert (K[s][:, keep] == 9).all() and (V[s][:, keep] == 9).all() and (arenas[s][:k_off] == 9).all()
 
 
+@pytest.mark.parametrize("H,G,d,dp,ep", [(28, 4, 128, 128, 128), (1, 1, 40, 64, 64), (33, 3, 64, 64, 128), (17, 1, 128, 128, 64), (7, 2, 180, 192, 192), (16, 16, 250, 256, 256)])
+@pytest.mark.parametrize("ns", [1, 3])
+def test_attention_inputs_of_every_head_width(dev, lib, H, G, d, dp, ep, ns):
+    """Heads of 16, 32 and 64 lanes (192: 48 of them), head counts that end inside a batch of a wave, more value channels than one pass of the block."""
+    from livecc_amd import _lib
+    S, L, eps = 5, 64, 3e-2
+    q, k, v = torch.randn(ns, S, H, d), torch.randn(ns, S, G, d), torch.randn(ns, S, G, ep)
+    part = torch.cat([_heads(q, dp), _heads(k, dp), _heads(v, ep), torch.randn(ns, S, 64)], -1)
+    wq, wk = torch.zeros(dp).bfloat16(), torch.zeros(dp).bfloat16()
+    wq[:d], wk[:d] = 1 + 0.2 * torch.randn(d), 1 + 0.2 * torch.randn(d)
+    slot, pos = [1, 0, 0, 1, 1], [3, 31, 32, 63, 0]
+    k_off, v_off = 128, 128 + G * L * dp
+    arenas, base = _arenas(2, v_off + G * L * ep, dev, 9.0)
+    dv, sd, pd = [t.to(dev) for t in (part, wq, wk)], _i32(slot, dev), _i32(pos, dev)
+    qo = torch.empty(S, H * dp, dtype=torch.bfloat16, device=dev)
+    a = _lib.GqaInput(partial=_p(dv[0]), nsplit=ns, rows=S, ldn=part.shape[-1], heads=H, kv_heads=G, dim=d, dim_pad=dp, vdim_pad=ep, eps=eps, q_norm=_p(dv[1]),
+                      k_norm=_p(dv[2]), temp_coef=0.0, temp_every=16, q=_p(qo), tok_stream=_p(sd), tok_pos=_p(pd), kv_base=_p(base), k_off=k_off, v_off=v_off, lmax=L)
+    _ok(lib.lcc_mixer_prep(C.byref(a), None, _st()))
+    qs, ks, vs = q.double().sum(0), k.double().sum(0), v.double().sum(0)
+    assert _near(qo.view(S, H, dp)[:, :, :d], R.over_rms(qs, eps) * wq[:d].double(), absolute=1e-5) and qo.view(S, H, dp)[:, :, d:].abs().sum() == 0
+    K = [t[k_off:k_off + G * L * dp].view(G, L, dp).cpu() for t in arenas]
+    V = [t[v_off:].view(G, L // 32, ep, 32).permute(0, 1, 3, 2).reshape(G, L, ep).cpu() for t in arenas]
+    kw = R.over_rms(ks, eps) * wk[:d].double()
+    for i, (s, p) in enumerate(zip(slot, pos)):
+        assert _near(K[s][:, p, :d], kw[i], absolute=1e-5) and K[s][:, p, d:].abs().sum() == 0 and _near(V[s][:, p], vs[i])
+    for s in range(2):
+        keep = [p for p in range(L) if (s, p) not in set(zip(slot, pos))]
+        assert (K[s][:, keep] == 9).all() and (V[s][:, keep] == 9).all() and (arenas[s][:k_off] == 9).all()
+
+
 def _kv_slots(lens, G, d, e, L, dev, g):
     """Random keys and values of every slot, in the arena's layout; returns (k [G, L, d], v [G, L, e]) per slot, arenas, base, offsets."""
     k_off, v_off = 64, 64 + G * L * d
