@@ -70,16 +70,17 @@ int lcc_debug_set_gemv_variant(int variant);
  * shape (default: 8-wave 256x256 / 128x256 LDS-DMA kernel where its grid fills the chip, else the 4-wave kernels), 3 / 4 = force the
  * 8-wave kernel with 256 / 128 rows where eligible, 5 / 6 = the same with the compiler's fragment-read schedule, 7 = 2 without the
  * 8-wave kernel, 8 = force the "tall" kernel (one block row covers all of M <= 448, 448x160 tiles) wherever it is legal; the default
- * takes it when 256 < M <= 448 and ceil(N/160) fills 75-100 % of one round of the chip (LiveCC-7B gate/up of a streaming chunk);
+ * takes it when 256 < M <= 448 (fp8 weights: 384 < M) and ceil(N/160) fills 75-100 % of one round of the chip (LiveCC-7B gate/up of a streaming chunk);
  * 13 = the 192-row 8-wave tile wherever eligible; 14 = row tiles of variable height (256 / 272 / 288 rows: ceil(M/16) row fragments dealt
  * out over floor(ceil(M/16)/16) tiles, no ragged last tile; round 5) wherever legal, else as 3 -- the default picks them by score (e.g. the
  * gate/up GEMM of 8 co-scheduled chunks: 12 x 148 tiles instead of 13 x 148); 15 = the SMALL variable-height class (row tiles of 128 / 144
  * rows) for split-K slabs of 64 < M <= 448 wherever legal, else as 4 -- the default picks it by score for the o / down / q|k|v projections
  * of one streaming chunk (M = 386: 3 row tiles instead of 4, 6 / 6 / 4 splits; LCC_GEMM_VH_SMALL=0 restores the 128-row tiles and their
- * 4 / 4 / 3 splits); 16 = 128 x 128 tiles (bf16 weights).  Every tile shape produces the same bits for the same split count. */
+ * 4 / 4 / 3 splits); 16 = 128 x 128 tiles; 17 = the 160-row 8-wave tile wherever
+ * eligible (bf16 weights).  Every tile shape of bf16 weights produces the same bits for the same split count. */
 int lcc_debug_set_gemm_variant(int variant);
 /* Host logic only (no launch; works without a GPU): which kernel family serves a packed-weight GEMM of this shape under the current
- * variant -- *tile_rows = 16 weight-streaming GEMV, 448 tall, 272 / 144 variable-height tiles (big / small class), 256 / 192 / 128 the
+ * variant -- *tile_rows = 16 weight-streaming GEMV, 448 tall, 272 / 144 variable-height tiles (big / small class), 256 / 192 / 160 / 128 the
  * 8-wave tile of that height x 256 columns, 129 the 128 x 128 tile, 64 the 64 x 128 tile; nsplit > 0 asks for the split-K slab form -- and *engine_splits = the split count
  * the engine's prefill asks for at this shape (what csrc/engine_llm.hip passes as nsplit for the o / down / q|k|v projections).
  * w_fp8 != 0: *tile_rows = 0 (fp8 weights route inside their own entry point), *engine_splits as for fp8 weights. */
@@ -240,7 +241,7 @@ int lcc_debug_bench_grid_barrier(int mode, int blocks, int iters, void* scratch,
  * the in-launch merge, 4 split-K GEMV with a fused consumer tail, 5 decode-pipeline-v2 GEMVs, 6 prefill attention on 32x32x16 MFMAs
  * (attn32.hip), 7 LDS-shared prefill attention, 8 per-wave prefill attention, 9 prefill split-merge launches, 10 / 11 = key splits of the
  * most recent decode / prefill attention launch (values, not counts), 12 tall-tile GEMM, 13 32x32x16 vision attention, 14 variable-height
- * GEMM tiles (gemm_vh_kernel), 15 vision q|k|v projection with the RoPE / V-transpose epilogue. */
+ * GEMM tiles (gemm_walk_vh_kernel; small class: gemm_vh_kernel), 15 vision q|k|v projection with the RoPE / V-transpose epilogue. */
 int lcc_debug_launch_counts(int64_t* out, int n, int reset);
 int lcc_debug_set_fused_attn(int mode); /* bit 0 (default on): engine decode uses the fused kernel for batches of >= 16 (stream,
                                           KV head) pairs; bit 2: for every batch; bit 1: key splits merged in the same launch by the

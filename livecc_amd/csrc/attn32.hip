@@ -83,11 +83,6 @@ LCC_DEVICE float xor32_sum(float x) {
 // probabilities the numerator uses (fp32 accumulation either way).
 // D = channels of q / k, DV = channels of v.  BIAS: slope (pos - key) is taken off the scaled scores (slope in units of log2), pos = this lane's query:
 // K.Q^T is added to it instead of to zero.
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
-LCC_DEVICE float dot_ones(unsigned pair, float c) {          // c + both bf16 halves of `pair`
-  const unsigned ones = 0x3F803F80u;
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, pair), __builtin_bit_cast(bf16x2_t, ones), c, false);
-}
 struct Kv32 {                   // keys and values of one (stream, head); all wave-uniform
   const bf16_t *k, *v;          // tile 0
   unsigned k_row, v_row;        // bytes between keys of K, between channels of V^T
@@ -211,9 +206,9 @@ LCC_DEVICE void attn32_key_loop(unsigned char* alds, const Kv32& kv, const u32x4
         for (int e = 0; e < 16; ++e) p[e] = __builtin_amdgcn_exp2f(fmaf(x[e], scale_log2e, -m_ref));   // masked scores are -inf -> 0
         u32x4 w0 = {pack2(p[0], p[1]), pack2(p[2], p[3]), pack2(p[4], p[5]), pack2(p[6], p[7])};
         u32x4 w1 = {pack2(p[8], p[9]), pack2(p[10], p[11]), pack2(p[12], p[13]), pack2(p[14], p[15])};
-        if (!LM) {          // the denominator takes the probabilities as the numerator does, rounded
+        if (!LM) {          // the denominator sums the probabilities unrounded
 #pragma unroll
-          for (int e = 0; e < 4; ++e) { l_run = dot_ones(w0[e], l_run); l_run = dot_ones(w1[e], l_run); }
+          for (int e = 0; e < 16; ++e) l_run += p[e];
         }
         // matrix pipe
 #pragma unroll

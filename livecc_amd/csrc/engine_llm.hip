@@ -357,13 +357,19 @@ extern "C" int lcc_llm_prefill(lcc_engine* e, int n_streams, const int32_t* slot
   // 386 rows against 6k keys): 674 us with 16-row tiles vs 747 us with 32-row tiles, so the wide tile is kept for very large
   // prefills only (e.g. the 8 x 1114-row first turn), where the grid is several waves of blocks either way.
   // attention variant 3 (attn32.hip: 32x32x16 MFMAs, one wave = 32 rows of one head) always takes 32-row tiles.
-  const bool mfma32 = get_attn_variant() == 3 && e->c.n_q_heads / e->c.n_kv_heads <= 8;
+  int max_kv = 0;
+  long tiles16 = 0;
+  for (int b = 0; b < n_streams; ++b) { max_kv = std::max(max_kv, e->h_kv_len[slots[b]] + n_new[b]); tiles16 += (n_new[b] + 15) / 16; }
+  // Short prompts: up to 384 keys a block of the 32x32x16 kernel is mostly prologue and the last tiles' chain.  While 16-row blocks fill the chip once at most,
+  // attn_shared_kernel's are sooner done (28 heads on 4: 64 keys 11.1 -> 6.6 us, 128 12.5 -> 8.1, 384 18.6 -> 15.2, 8 x 128 14.0 -> 10.0; 8 x 192 rows, 384
+  // blocks: 17 against 18.4; beyond 384 keys the other one splits them).
+  const int gq = e->c.n_q_heads / e->c.n_kv_heads;
+  const bool brief = max_kv <= 384 && tiles16 * e->c.n_kv_heads <= e->cu_count && gq >= 2;
+  const bool mfma32 = get_attn_variant() == 3 && gq <= 8 && !brief;
   // Round 6: a block of that kernel can hold 8 x 32 / G rows -- 36 at 7 heads per KV head, all eight waves busy instead of seven -- and a
   // block's time does not depend on that (it is set by its busiest SIMD).  Tile height and key-split count are planned TOGETHER
   // (attn32.hip: attn32_plan, pinned on the CPU through lcc_debug_attn_plan).
   int tile_rows = mfma32 ? 32 : ((long)((S + 31) / 32) * e->c.n_q_heads >= 6144 ? 32 : 16);
-  int max_kv = 0;
-  for (int b = 0; b < n_streams; ++b) max_kv = std::max(max_kv, e->h_kv_len[slots[b]] + n_new[b]);
   const int ks_cap = std::max(1, std::min(8, (max_kv / 32) / 8));      // >= 8 key tiles per split
   int ks32 = 1;
   if (mfma32) attn32_plan(n_new, n_streams, max_kv, e->c.n_q_heads / e->c.n_kv_heads, e->c.n_kv_heads, e->cu_count, &tile_rows, &ks32);

@@ -26,7 +26,7 @@ enum LaunchCounter {
   LC_LAST_PREFILL_NSPLIT = 11, // key splits of the most recent prefill attention launch
   LC_GEMM_TALL = 12,
   LC_ATTN_VIT32 = 13,          // attn_vit32_kernel (vision attention on 32x32x16 MFMAs)
-  LC_GEMM_VH = 14,             // gemm_vh_kernel (row tiles of 256 / 272 / 288 rows, small class 128 / 144; round 5 -- the slot of the retired gemm_pp_kernel)
+  LC_GEMM_VH = 14,             // gemm_walk_vh_kernel (row tiles of 256 / 272 / 288 rows), gemm_vh_kernel (small class 128 / 144; round 5 -- the slot of the retired gemm_pp_kernel)
   LC_GEMM_VIT_QKV = 15,        // gemm_big_kernel with the EPI_VIT_QK / EPI_VIT_V epilogues (RoPE / V transpose fused into the q|k|v projection; one EPI_VIT_QKV launch per tower block when E % 128 == 0, else a q|k launch + a V launch)
   LC_COUNT = 16
 };
@@ -74,8 +74,8 @@ struct GemmArgs {
   int epilogue = 0;
   GemvTail tail;
   // fp8 (OCP e4m3) weights: W points at bytes in the PACKED8 order [N/16][K/64][4 g][16 rows][16 k], wscale = fp32 [N]
-  // (y[n] = wscale[n] * sum_k x[k] q[n][k]); M > 16 needs dq_scratch = N*K bf16 (exact dequantisation into the bf16 packed
-  // order, then the bf16 GEMM with the scale in its epilogue)
+  // (y[n] = wscale[n] * sum_k x[k] q[n][k]); M > 16: tiles that convert the bytes behind their LDS read; forced variants
+  // without one go through dq_scratch = N*K bf16 (exact dequantisation into the bf16 packed order, then the bf16 GEMM)
   int w_fp8 = 0; const float* wscale = nullptr; bf16_t* dq_scratch = nullptr;
   VitQkvEpi vq;                                 // epilogue == GEMM_EPI_VIT_QK / GEMM_EPI_VIT_V only
 };

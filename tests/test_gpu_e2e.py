@@ -681,6 +681,34 @@ def test_decode_pipeline_v2_matches_the_round1_launch_sequence(dev, shape):
         assert worst <= 3e-2, f"v2 vs round-1 decode logits differ by {worst:.3g} of the logit scale"
 
 
+@pytest.mark.parametrize("rows,kernel", [((1,), "attn_prefill_shared"), ((17, 384), "attn_prefill_shared"), ((385,), "attn_prefill_mfma32"), ((32, 512), "attn_prefill_mfma32")])
+def test_short_prompts_take_the_16_row_attention_blocks(dev, rows, kernel):
+    """Up to 384 keys and one round of blocks; the logits of a prompt are those of the other kernel family up to rounding (the same bound as the two decode
+    pipelines above)."""
+    from livecc_amd import ops
+    from livecc_amd.config import tiny
+    from livecc_amd.modeling import LiveCCForConditionalGeneration
+    cfg = tiny()
+    native = LiveCCForConditionalGeneration.from_config(cfg, dev, seed=3, max_streams=2, max_kv_len=1024, max_new_rows=1024, max_patches=64, max_history=16)
+    g = torch.Generator().manual_seed(sum(rows))
+    ids = [torch.randint(0, min(cfg.vocab_size, 500), (n,), generator=g) for n in rows]
+    got = {}
+    for variant in (3, 0):
+        ops.set_attn_variant(variant)
+        try:
+            before = ops.launch_counts()[kernel]
+            res = native.generate_batch([dict(input_ids=x) for x in ids], max_new_tokens=1, force_length=True, output_logits=True)
+            got[variant] = [r.logits[0].float().cpu() for r in res]
+            if variant == 3:
+                assert ops.launch_counts()[kernel] > before
+            for r in res:
+                r.past_key_values.release()
+        finally:
+            ops.set_attn_variant(3)
+    for a, b in zip(got[3], got[0]):
+        assert (a - b).abs().max() <= 3e-2 * b.abs().max()
+
+
 def _several_streams_against_the_unfused_sequence(dev, cfg, n_streams, fp8, scaled):
     from livecc_amd import _lib, ops
     from livecc_amd.engine import Sampling
