@@ -1516,11 +1516,18 @@ __global__ __launch_bounds__(512) void gemm_tall_kernel(
 #pragma unroll
     for (int q = 0; q < A_PER_WAVE; ++q)
       if ((wave * A_PER_WAVE + q) * 8 < m_rows)
-        glds16((A + aoffs[q] + kt * BK), lds_addr(sbase + (wave * A_PER_WAVE + q) * 64));
+{
+        if constexpr (W8) glds16_base(A + kt * BK, (unsigned)aoffs[q] * 2u, lds_addr(sbase + (wave * A_PER_WAVE + q) * 64));
+        else glds16((A + aoffs[q] + kt * BK), lds_addr(sbase + (wave * A_PER_WAVE + q) * 64));
+      }
 #pragma unroll
     for (int q = 0; q < NB; ++q)
-      if (q < nb)
-        glds16((bsrc[q] + (size_t)kt * WK), lds_addr(sbase + A_UNITS + (st0 + q) * 64));
+      if (q < nb) {
+        if constexpr (W8) {      // scalar bases: the converted fragments need the registers
+          const int fr = min((n0 >> 4) + st0 + q, nfrag - 1);
+          glds16_base(W + (size_t)fr * (K >> 6) * 512 + (size_t)kt * WK, (unsigned)lane * 16u, lds_addr(sbase + A_UNITS + (st0 + q) * 64));
+        } else glds16((bsrc[q] + (size_t)kt * WK), lds_addr(sbase + A_UNITS + (st0 + q) * 64));
+      }
   };
 
   // SCHED 2: the 10 pieces of a wave (7 activation + 3 W; waves 4-7 repeat their second W sub-tile as the third) go out ONE at a time
@@ -1608,9 +1615,22 @@ __global__ __launch_bounds__(512) void gemm_tall_kernel(
       if constexpr (MTW > 0) ktile(dsmem + (kt & 1) * STAGE, mtw_c, ntw_c, min(kt + 1, nkt - 1), (kt + 1) & 1);
     }
     if (SCHED == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if constexpr (MTW > 0)
-      tile_epilogue<EPI, (MTW > 0 ? MTW : 1), (MTW > 0 ? NTW : 2), MT, NT0>(acc, wm * WM, nbase, nbase / 2, li, g, bias, residual, ldr, C, ldc, M, N,
-                                                                        nullptr, wscale);
+    if constexpr (MTW > 0) {
+      int le = lane;
+      asm volatile("" : "+v"(le));          // the epilogue's addresses are formed here, not carried through the loop
+      const int lie = le & 15, ge = le >> 4;
+      if constexpr (W8) {                   // the rows' scales, one column tile at a time
+#pragma unroll
+        for (int j = 0; j < NTW; ++j) {
+          asm volatile("" ::: "memory");
+          const f32x4 sc = *reinterpret_cast<const f32x4*>(wscale + min(nbase + j * 16 + ge * 4, N - 4));
+#pragma unroll
+          for (int i = 0; i < MTW; ++i) acc[i][j] *= sc;
+        }
+      }
+      tile_epilogue<EPI, (MTW > 0 ? MTW : 1), (MTW > 0 ? NTW : 2), MT, NT0>(acc, wm * WM, nbase, nbase / 2, lie, ge, bias, residual, ldr, C, ldc, M, N,
+                                                                        nullptr, nullptr);
+    }
   };
   if (mt_live == 0) run(I0{}, I4{});                 // no rows: DMA + barriers only
   else if (wn == 0) { if (mt_live <= 4) run(I4{}, I6{}); else run(I7{}, I6{}); }
@@ -1844,7 +1864,8 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr) {    
 
 // The tall kernel serves one-block-row problems whose column tiles fill most of ONE round of the chip (7B gate/up at a streaming
 // chunk: 237 blocks).  Variant 8 forces it wherever it is legal (tests).
-static bool tall_legal(const GemmArgs& a) { return big_eligible(a) && a.M <= 448 && (a.N & 15) == 0; }
+// (fp8 weights with a residual would need more registers than a wave has)
+static bool tall_legal(const GemmArgs& a) { return big_eligible(a) && (a.w_fp8 ? a.epilogue != EPI_RESIDUAL : a.wscale == nullptr) && a.M <= 448 && (a.N & 15) == 0; }
 static bool tall_wanted(const GemmArgs& a) {
   if (!tall_legal(a)) return false;
   if (g_gemm_variant == 8) return true;
@@ -1869,8 +1890,10 @@ static void launch_tall(const GemmArgs& a, hipStream_t st) {
   // 0 compiler order, 1 pinned (default since round 6: 127.6 vs 131.6-132.6 us at M = 386 on N(0,1) activations, A/B/A/B, bit-identical --
   // profiles/r06/m386_gemms_tall_sched_ab.jsonl; before the LDS-DMA went into inline asm the compiler's order had been the faster one), 2 pinned + spread DMA
   static const int sched = [] { const char* v = getenv("LCC_TALL_SCHED"); return v ? atoi(v) : 1; }();
-  if (a.w_fp8) { if (sched == 2) launch_tall_s<EPI, 2, true>(a, st); else if (sched == 0) launch_tall_s<EPI, 0, true>(a, st); else launch_tall_s<EPI, 1, true>(a, st); }
-  else if (sched == 2) launch_tall_s<EPI, 2, false>(a, st);
+  if constexpr (EPI != EPI_RESIDUAL) {
+    if (a.w_fp8) return launch_tall_s<EPI, 1, true>(a, st);
+  }
+  if (sched == 2) launch_tall_s<EPI, 2, false>(a, st);
   else if (sched == 1) launch_tall_s<EPI, 1, false>(a, st);
   else launch_tall_s<EPI, 0, false>(a, st);
 }

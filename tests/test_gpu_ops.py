@@ -450,7 +450,8 @@ def test_gemm_w8_narrow_tiles(dev, M, N, K, epi, S, variant):
 @pytest.mark.parametrize("M", [17, 113, 225, 337, 385, 386, 448])
 @pytest.mark.parametrize("N,K,epi", [(352, 192, 0), (160, 64, 1), (480, 320, 3), (352, 128, 4)])
 def test_gemm_w8_tall(dev, M, N, K, epi):
-    """fp8 weights in the tile that holds all rows (variant 8): a last block of 32 columns, waves with all, some and none of their rows."""
+    """fp8 weights in the tile that holds all rows (variant 8; with a residual, which that tile has no registers for, in the forced variant's other
+    form): a last block of 32 columns, waves with all, some and none of their rows."""
     from livecc_amd import ops
     from livecc_amd.weights import dequantize_fp8_rows, quantize_fp8_rows
     x, w = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.05, 2).float()
