@@ -20,6 +20,7 @@
 #include <type_traits>
 
 #include <algorithm>
+#include <utility>
 
 #include "common.h"
 #include "kernels.h"
@@ -42,33 +43,33 @@ LCC_DEVICE float xor32_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+template <class F, int... I>
+LCC_DEVICE void unrolled_of(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, class F>
+LCC_DEVICE void unrolled(F&& f) { unrolled_of(f, std::make_integer_sequence<int, N>{}); }      // f(0) .. f(N - 1), the index a constant
+
 // ------------------------------------------------------------------------------------------------------------------------------
-// The key loop shared by the LLM prefill kernel (D = 128) and the ViT kernel (D = 80): software pipeline, one key tile per REGION.
-// The softmax of tile t (vector pipe: ~70 VALU instructions) is issued next to the MFMAs that do not depend on it -- the P . V of tile
-// t-1 and the K . Q^T of tile t+1 (matrix pipe: 16 x 32 cycles at D = 128) -- in ONE scheduling region, interleaved by
-// sched_group_barrier: a wave always has matrix AND vector work in flight.  (With one tile at a time per wave the two waves of a SIMD
-// ran the same phase in lock step behind the block barrier: the first version of the D = 128 kernel, 0.57 PF at 8 x 386 rows x 6k
-// keys against 0.54 for the 16x16x32 kernel; pipelined: 0.76 PF, 1.36 vs 1.93 ms for a 4,096-row piece against 20k keys.)
+// The key loop shared by the LLM prefill kernel (D = 128), the causal multi-head kernel and the ViT kernel (D = 80): software pipeline, a pair of key
+// tiles an iteration.  The softmax of pair P (vector pipe) is issued next to the MFMAs that do not depend on it -- the P . V of pair P - 1 and the K . Q^T of
+// pair P + 1 (matrix pipe: 32 x 32 cycles at D = 128) -- in ONE basic block: every fragment read FRAG_LEAD MFMAs ahead of its use, the vector work dealt out in
+// steps (Attn32Steps), the DMA pieces of pair P + 2 spread between them: a wave always has matrix AND vector work in flight.
 //
-// Ring of three pair-stages.  Slot t holds what region t multiplies -- K of tile t + 1 and V^T of tile t - 1 -- so a pair needs its own two slots only:
-// at the top of the iteration of pair (t, t + 1) its slots have landed (counted vmcnt: only the next pair's, issued one iteration ago, may still
-// be in flight; barrier: every wave's pieces) and the slots of the pair before receive pair t + 4.  (Whole tiles a slot needed five pair-stages: one
-// block a compute unit.)  The iteration enters with sc_a = K.Q^T of tile t and leaves with sc_a = K.Q^T of tile t + 2.
+// Ring of three pair-stages.  Slot t holds what the iteration of tile t multiplies -- K of tile t + 2 and V^T of tile t - 2 -- so a pair needs its own two slots
+// only: at the top of the iteration of pair (t, t + 1) its slots have landed (counted vmcnt: only the next pair's, issued one iteration ago, may still
+// be in flight; barrier: every wave's pieces) and the slots of the pair before receive pair t + 4.  The iteration enters with the scores of tiles t and t + 1 and leaves with
+// those of t + 2 and t + 3.
 //
-// An iteration is ONE basic block -- 2 x NP MFMAs, every fragment read FRAG_LEAD MFMAs ahead of its use, the DMA pieces of pair P+3 spread between
-// them -- because the softmax has no branch: probabilities are taken against a reference that is only moved between two pairs.
-//   * Reference: the row's maximum over its first key tile (log2 units); moved up by the whole number that reaches the maximum so far when a
-//     pair held a score more than `slack` above it.  Until then probabilities are up to 2^slack (fp32 and bf16 hold the exponent; numerator and denominator carry
-//     the same factor), and moving by a whole number of powers of two is exact on O, l and the pending P.  The running maximum itself moves in nearly
-//     every tile of a short key range (32 rows, each with chance 1 / t in tile t): a rescale of O behind the MFMAs, a maximum that every exponential
-//     waits for, and a branch in every region that cut the schedule in two.
-//   * A score more than REF_JUMP above the reference within one pair could overflow: the block then goes through its keys a second time (`again`),
-//     those rows with the final reference of the first time, which no score exceeds.
+// Reference of the softmax: the row's running maximum, that of the pair included.  All scores of the pair are there when the iteration begins, so every
+// probability is at most one, the row's largest IS one and no rounding touches it.  O, which is one pair behind, is brought to the maximum by the factor alpha at
+// the top of the next iteration, if any row of the wave needs it.
+//   * A reference that moves rarely (a first tile's maximum plus whole powers of two: no rescale in most iterations) was taken back: the row's largest probability is
+//     then rounded to bf16 like any other.  Error against 64 bits (2-norm, 1e-3), 386 rows on 386 keys / 64 on 8,000 with a bias, normal keys and values of 1 / 2 / 4:
+//     2.02 / 2.09 / 2.14 and 2.34 / 2.34 / 2.34 there, 1.96 / 1.82 / 1.72 and 1.89 / 1.80 / 1.72 here (a maximum per tile: 1.94 / 1.81 / 1.72 and 1.89 / 1.79 / 1.71).
+//   * Scores of one tile alone at the top (the second tile's maximum a region later): two places to rescale O, and a branch in each.
 //   * Each row decides by its own scores (both lanes of its column), so its bits do not depend on its neighbours in the wave.
-// Measured (us; one region of 16 / 11 MFMAs a block, running maximum, fragment-order gathers -> here): 4,096 rows on 8k keys 700 -> 597 (1.01 PF), 386 rows on
-// 2k keys in five splits 40.7 -> 36.8, 8 x 386 rows on 1.1k 103 -> 84; with a bias, 4,096 rows on 4k 577 -> 503; tower, 18 slices of 880 patches 173 -> 138 with 256
-// rows a block and 113 with 128, one slice of 1,456 35.7 -> 29.5.  What bounds it now: the vector pipe beside the matrix pipe (with neither DMA nor fragment
-// reads the loop ran 4,096 rows on 8k keys in 489).
+// Measured (us; one region of 16 / 11 MFMAs a tile with fragment-order gathers -> rare moves -> here): 4,096 rows on 8k keys 667 -> 589 -> 598 (1.01 PF), 386 rows
+// on 2k keys in five splits 38.1 -> 34.2 -> 34.9, 8 x 386 rows on 1.1k 102 -> 84.0 -> 87.0; with a bias, 4,096 rows on 4k 577 -> 516 -> 420; tower, 18 slices of 880
+// patches 174 -> 117 -> 122, one of 1,456 32.8 -> 29.4 -> 30.0.  What bounds it: the vector pipe beside the matrix pipe.
 //
 // LDS image of a slot: rows as they lie in memory, so that a DMA instruction copies whole runs of lines (K: 32 keys x 2 D bytes; V^T: DV rows x 64 bytes)
 // instead of 64 separate 16-byte chunks, each a line of its own for the address path (a 4-wave block of the tower kernel spent 15 of its 42 us on that).  A row's
@@ -97,19 +98,28 @@ struct Attn32Image {
   LCC_DEVICE static int vx(int d) { return (d >> 2) & 3; }
 };
 
+// The 32 probabilities of a pair are formed two at a time beside its MFMAs: how many twos up to behind MFMA i (17: the last one summed, too).  Evenly, or with
+// wide values (whose P.V leaves the time) each tile's before the MFMAs that overwrite its scores: the new scores then take the old ones' registers.
+template <int VP, int KP>
+struct Attn32Steps {
+  static constexpr int formed(int i) {
+    constexpr int N = 2 * (VP + KP), A = 2 * VP - 1, B = 2 * VP + KP - 1;
+    if (i < 5) return 0;
+    if (VP < 8) return i == N - 1 ? 17 : (i - 4) * 16 / (N - 6);
+    if (i < A) return (i - 4) * 8 / (A - 5);
+    return i >= B ? 17 : i == B - 1 ? 16 : 8 + (i - A + 1) * 8 / (B - A);
+  }
+};
 template <int D, int DV, int NWAVE, bool LM, bool BIAS = false, bool CLAMP = false>
 LCC_DEVICE void attn32_key_loop(unsigned char* alds, const Kv32& kv, const u32x4 (&qf)[D / 16], int tb, int te, int mlim, int lim, float scale_log2e,
                                 bool active, int lane, int wave, int hh, f32x16 (&o)[(DV + 31) / 32], float& m_run, float& l_run, float slope = 0.f, int pos = 0) {
   using Im = Attn32Image<D, DV>;
   constexpr int KP = D / 16, DT = Im::DT, VP = 2 * DT, NP = KP + VP, FRAG_LEAD = 4;
+  using Steps = Attn32Steps<VP, KP>;
   constexpr int NPD = Im::NPD, PWP = (2 * NPD + NWAVE - 1) / NWAVE, PK = (Im::KPD + NWAVE - 1) / NWAVE;     // DMA pieces of a wave: a pair; K of one tile
-  constexpr float REF_JUMP = 100.f;
   m_run = -INFINITY;
   if (te <= tb) return;                                 // (block-uniform: a key split without a tile)
-  // a bias of `slope` a key lifts a row's scores by 64 slope from pair to pair: the slack leaves room for that below the jump
-  const float slack = BIAS ? fmaxf(0.f, fminf(40.f, 88.f - 64.f * slope)) : 16.f;
   const unsigned lds0 = lds_addr(alds);
-  float m_ref = 0.f, m_limit = -INFINITY;               // m_limit = -inf: the row has seen no key
   const float bias_raw = BIAS ? slope / scale_log2e : 0.f, bias_pos = BIAS ? bias_raw * (float)(8 * hh - pos) : 0.f;
   const int col = lane & 31;
 
@@ -136,7 +146,7 @@ LCC_DEVICE void attn32_key_loop(unsigned char* alds, const Kv32& kv, const u32x4
   auto issue = [&](int j, int t, int ps) {              // piece j of the pair (t, t + 1) into pair-stage ps
     const int u = min(j * NWAVE + wave, 2 * NPD - 1), r = u >= NPD ? 1 : 0, p = u - r * NPD;
     const bool is_k = p < Im::KPD;
-    const int tile = min(is_k ? t + r + 1 : max(t + r - 1, tb), kv.ntile - 1);
+    const int tile = min(is_k ? t + r + 2 : max(t + r - 2, tb), kv.ntile - 1);
     piece(p, tile, is_k, off[j], CLAMP ? prow[CLAMP ? j : 0] : 0u, lds0 + (unsigned)((2 * ps + r) * Im::SLOT));
   };
   // fragment addresses inside a slot: K row swap23(col), chunk 2 ks + hh; V^T row 32 dt + col, chunk 2 s + hh
@@ -159,172 +169,140 @@ LCC_DEVICE void attn32_key_loop(unsigned char* alds, const Kv32& kv, const u32x4
 #pragma unroll
     for (int r = 0; r < 16; ++r) sc[r] = BIAS ? fmaf(bias_raw, (float)(16 * (r >> 3) + (r & 7)), base) : 0.f;
   };
-  auto mask = [&](auto masked_tag, int t, f32x16& sc) {
-    if (decltype(masked_tag)::value) {
-      const int kb = t * 32;
+  bf16x8 p_prev[4];                                     // P of the previous pair, its P . V still pending
 #pragma unroll
-      for (int r = 0; r < 16; ++r) sc[r] = (kb + 16 * (r >> 3) + 8 * hh + (r & 7)) < lim ? sc[r] : -INFINITY;
-    }
-  };
-  auto lane_max = [&](const f32x16& sc) {                         // of this lane's 16 keys
-    float mx = vmax3(sc[0], sc[1], sc[2]);
+  for (int i = 0; i < 4; ++i) p_prev[i] = as_bf16x8((u32x4){0u, 0u, 0u, 0u});
+  f32x16 sc[2];
+  float alpha = 1.f;                                    // what brings O (pairs before the previous one) to the maximum that p_prev was taken against
+  int st = 0;                                           // pair-stage of the pair
+  // one pair: softmax of tiles t and t + 1 (vector pipe) beside P.V of t - 2 and t - 1, K.Q^T of t + 2 and t + 3 (matrix pipe)
+  auto pair = [&](auto masked_tag, int t) {
+    constexpr bool MASKED = decltype(masked_tag)::value;
+    // the two copies of the pair keep their fragment reads: shared, they would all sit in front of the branch between them
+    if (MASKED) asm volatile("; masked pair" ::: "memory"); else asm volatile("; whole pair" ::: "memory");
+    const unsigned char* slot[2] = {alds + 2 * st * Im::SLOT, alds + (2 * st + 1) * Im::SLOT};
+    const int ps = st == 0 ? 2 : st - 1;
+    u32x4 f[FRAG_LEAD + 1];
+    auto read = [&](int i) { return i < 2 * VP ? vfrag(slot[i / VP], i % VP) : kfrag(slot[(i - 2 * VP) / KP], (i - 2 * VP) % KP); };
 #pragma unroll
-    for (int r = 3; r < 15; r += 2) mx = vmax3(mx, sc[r], sc[r + 1]);
-    return vmax(mx, sc[15]) * scale_log2e;
-  };
-
-  bool bad = false;
-  for (int pass = 0;; ++pass) {
-    bf16x8 p_prev[2];                                   // P of the previous tile, its P . V still pending
-    p_prev[0] = as_bf16x8((u32x4){0u, 0u, 0u, 0u});
-    p_prev[1] = p_prev[0];
-    f32x16 sc_a, sc_b;
-    float mx_pair = -INFINITY;                          // of the last pair, this lane's keys
-    int st = 0;                                         // pair-stage of the pair
-    // one pair: softmax of tiles t and t + 1 (vector pipe) beside P.V of t - 1 and t, K.Q^T of t + 1 and t + 2 (matrix pipe)
-    auto pair = [&](auto masked_tag, int t) {
-      constexpr bool MASKED = decltype(masked_tag)::value;
-      // the two copies of the pair keep their fragment reads: shared, they would all sit in front of the branch between them
-      if (MASKED) asm volatile("; masked pair" ::: "memory"); else asm volatile("; whole pair" ::: "memory");
-      const unsigned char* slot[2] = {alds + 2 * st * Im::SLOT, alds + (2 * st + 1) * Im::SLOT};
-      const int ps = st == 0 ? 2 : st - 1;
-      u32x4 f[FRAG_LEAD + 1];
-      auto read = [&](int i) { const int r = i / NP, w = i % NP; return w < VP ? vfrag(slot[r], w) : kfrag(slot[r], w - VP); };
-#pragma unroll
-      for (int i = 0; i < FRAG_LEAD; ++i) f[i] = read(i);
-      mx_pair = -INFINITY;
-#pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        f32x16& cur = r == 0 ? sc_a : sc_b;
-        f32x16& nxt = r == 0 ? sc_b : sc_a;
-        // vector pipe
-        f32x16 x = cur;
-        mask(masked_tag, t + r, x);
-        mx_pair = vmax(mx_pair, lane_max(x));
-        float p[16];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) p[e] = __builtin_amdgcn_exp2f(fmaf(x[e], scale_log2e, -m_ref));   // masked scores are -inf -> 0
-        u32x4 w0 = {pack2(p[0], p[1]), pack2(p[2], p[3]), pack2(p[4], p[5]), pack2(p[6], p[7])};
-        u32x4 w1 = {pack2(p[8], p[9]), pack2(p[10], p[11]), pack2(p[12], p[13]), pack2(p[14], p[15])};
-        if (!LM) {          // the denominator sums the probabilities unrounded
-#pragma unroll
-          for (int e = 0; e < 16; ++e) l_run += p[e];
-        }
-        // matrix pipe
-#pragma unroll
-        for (int w = 0; w < NP; ++w) {
-          const int i = r * NP + w;
-          if (w < VP) o[w >> 1] = mfma32(as_bf16x8(f[i % (FRAG_LEAD + 1)]), p_prev[w & 1], o[w >> 1]);
-          else {
-            if (w == VP) clear(t + r + 1, nxt);
-            nxt = mfma32(as_bf16x8(f[i % (FRAG_LEAD + 1)]), as_bf16x8(qf[w >= VP ? w - VP : 0]), nxt);
-          }
-          if (i + FRAG_LEAD < 2 * NP) f[(i + FRAG_LEAD) % (FRAG_LEAD + 1)] = read(i + FRAG_LEAD);
-#pragma unroll
-          for (int j = 0; j < PWP; ++j)
-            if (i == (2 * j + 1) * NP / PWP) issue(j, t + 4, ps);
-        }
-        if (r == 1) {     // P of the pair's second tile is consumed by the next iteration: formed here, under this one's MFMAs
-          asm volatile("" : "+v"(w0[0]), "+v"(w0[1]), "+v"(w0[2]), "+v"(w0[3]), "+v"(w1[0]), "+v"(w1[1]), "+v"(w1[2]), "+v"(w1[3]), "+v"(l_run), "+v"(mx_pair));
-        }
-        p_prev[0] = as_bf16x8(w0); p_prev[1] = as_bf16x8(w1);
+    for (int i = 0; i < FRAG_LEAD; ++i) f[i] = read(i);
+    // the vector work in steps: the maximum of eight scores (four of them), the new reference, then two probabilities at a time
+    f32x16 x[2] = {sc[0], sc[1]};
+    float mx[2] = {-INFINITY, -INFINITY}, psum[2] = {0.f, 0.f}, m_use = 0.f, al = 1.f;
+    u32x4 w[4];
+    auto settle = [&](auto kc) {              // they are there by now: without this the compiler moves pure arithmetic behind the MFMAs, in front of its use
+      constexpr int r = decltype(kc)::value >> 3, e = (decltype(kc)::value & 7) * 2;
+      float a = x[r][e], b = x[r][e + 1];
+      if constexpr (LM) asm volatile("" : "+v"(a), "+v"(b));
+      else {
+        psum[0] += a; psum[1] += b;           // the denominator sums the probabilities unrounded
+        asm volatile("" : "+v"(a), "+v"(b), "+v"(psum[0]), "+v"(psum[1]));
       }
-      // issue order: fragment reads ahead, then per MFMA one more read and a handful of vector instructions
-      __builtin_amdgcn_sched_group_barrier(0x100, FRAG_LEAD, 0);
+      x[r][e] = a; x[r][e + 1] = b;
+    };
+    auto step = [&](auto nc) {
+      constexpr int n = decltype(nc)::value;
+      if constexpr (n < 4) {
+        constexpr int r = n >> 1, e0 = (n & 1) * 8;
 #pragma unroll
-      for (int i = 0; i < 2 * NP; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if (i + FRAG_LEAD < 2 * NP) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, ((MASKED ? 6 : 4) - (LM ? 1 : 0) + (BIAS ? 1 : 0)) * 16 / NP, 0);
+        for (int e = e0; e < e0 + 8; ++e)
+          if (MASKED) x[r][e] = ((t + r) * 32 + 16 * (e >> 3) + 8 * hh + (e & 7)) < lim ? x[r][e] : -INFINITY;
+#pragma unroll
+        for (int e = e0; e < e0 + 8; e += 2) mx[(e >> 1) & 1] = vmax3(mx[(e >> 1) & 1], x[r][e], x[r][e + 1]);
+      } else if constexpr (n == 4) {
+        const float m_new = vmax(m_run, xor32_max(vmax(mx[0], mx[1])) * scale_log2e);
+        m_use = m_new == -INFINITY ? 0.f : m_new;
+        al = __builtin_amdgcn_exp2f(m_run - m_use);       // m_run = -inf -> 0
+        m_run = m_new;
+      } else {
+        constexpr int r = (n - 5) >> 3, e = ((n - 5) & 7) * 2;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) x[r][e + k] = __builtin_amdgcn_exp2f(fmaf(x[r][e + k], scale_log2e, -m_use));   // masked scores are -inf -> 0
+        if constexpr (n > 5) settle(std::integral_constant<int, n - 6>{});
       }
     };
-
-    // K of tile tb (the first slot of the third pair-stage, free until the loop's first iteration is past its barrier), then two pairs
-#pragma unroll
-    for (int j = 0; j < PK; ++j) {
-      const int p = min(j * NWAVE + wave, Im::KPD - 1), row = (p * 64 + lane) / Im::CR, c = (p * 64 + lane) % Im::CR;
-      piece(p, tb, true, (CLAMP ? 0u : (unsigned)row * kv.k_row) + (unsigned)((c ^ Im::kx(row)) * 16), row, lds0 + 4u * Im::SLOT);
-    }
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-#pragma unroll
-      for (int j = 0; j < PWP; ++j) issue(j, tb + 2 * k, k);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PWP) : "memory");
-    __builtin_amdgcn_s_barrier();
-    if (active) {
-      asm volatile("" ::: "memory");
-      clear(tb, sc_a);
-#pragma unroll
-      for (int ks = 0; ks < KP; ++ks) sc_a = mfma32(as_bf16x8(kfrag(alds + 4 * Im::SLOT, ks)), as_bf16x8(qf[ks]), sc_a);
-      if (!bad) {
-        f32x16 x = sc_a;
-        mask(std::true_type{}, tb, x);
-        const float mx = xor32_max(lane_max(x));
-        m_ref = mx > -INFINITY ? mx : 0.f;
-        m_limit = mx > -INFINITY ? m_ref + slack : -INFINITY;
-      }
-    }
-    for (int t = tb; t < te; t += 2) {
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PWP) : "memory");
-      __builtin_amdgcn_s_barrier();
-      if (active) {
-        if (__builtin_amdgcn_ballot_w64(mx_pair > m_limit) != 0) {
-          const float mx = xor32_max(mx_pair);
-          const bool move = mx > m_limit;
-          bad = bad || (move && mx - m_ref > REF_JUMP);
-          const float to = move ? m_ref + ceilf(mx - m_ref) : m_ref, alpha = __builtin_amdgcn_exp2f(m_ref - to);      // a whole power of two: exact
-          m_ref = to; m_limit = move ? to + slack : m_limit;
-#pragma unroll
-          for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
-          l_run *= alpha;
-#pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            u32x4 w = as_u32x4(p_prev[i]);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) w[e] = pack2(lo2f(w[e]) * alpha, hi2f(w[e]) * alpha);
-            p_prev[i] = as_bf16x8(w);
-          }
+    unrolled<2 * NP>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      if constexpr (i >= 2 * VP && (i - 2 * VP) % KP == 0) clear(t + (i - 2 * VP) / KP + 2, sc[(i - 2 * VP) / KP]);
+      const bf16x8 fi = as_bf16x8(f[i % (FRAG_LEAD + 1)]);
+      if constexpr (i + FRAG_LEAD < 2 * NP) f[(i + FRAG_LEAD) % (FRAG_LEAD + 1)] = read(i + FRAG_LEAD);
+      if constexpr (i < 2 * VP) o[(i % VP) >> 1] = mfma32(fi, p_prev[2 * (i / VP) + (i & 1)], o[(i % VP) >> 1]);
+      else sc[(i - 2 * VP) / KP] = mfma32(fi, as_bf16x8(qf[(i - 2 * VP) % KP]), sc[(i - 2 * VP) / KP]);
+      constexpr int before = Steps::formed(i - 1), formed = Steps::formed(i);
+      if constexpr (i < 5) step(ic);
+      unrolled<formed - before>([&](auto k) {
+        constexpr int n = before + decltype(k)::value;
+        if constexpr (n < 16) step(std::integral_constant<int, 5 + n>{}); else settle(std::integral_constant<int, 15>{});
+      });
+      unrolled<16>([&](auto kc) {             // rounded, into the registers of the pending P whose last MFMA has been issued
+        constexpr int k = decltype(kc)::value, last = ((k >> 3) + 1) * VP - 1;
+        if constexpr (k + 1 < formed && (i == last || (i > last && k + 1 >= before))) {
+          unsigned v = pack2(x[k >> 3][(k & 7) * 2], x[k >> 3][(k & 7) * 2 + 1]);
+          asm volatile("" : "+v"(v));
+          w[k >> 2][k & 3] = v;
         }
-        if ((t + 2) * 32 > mlim) pair(std::true_type{}, t); else pair(std::false_type{}, t);
-      } else {
+      });
 #pragma unroll
-        for (int j = 0; j < PWP; ++j) issue(j, t + 4, st == 0 ? 2 : st - 1);
-      }
-      st = st == 2 ? 0 : st + 1;
-    }
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");     // all pieces: no LDS-DMA of this block may land after it has left the CU
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (active) {                // the last tile's P.V: its V^T is in the next pair's first slot
-      const unsigned char* slot = alds + 2 * st * Im::SLOT;
+      for (int j = 0; j < PWP; ++j)
+        if (i == (2 * j + 1) * NP / PWP) issue(j, t + 4, ps);
+      if (LM) __builtin_amdgcn_sched_barrier(0);      // this order is the order of issue (tower: 18 slices of 880 121 us, 123 without; D = 128: 1.5 % slower with it)
+    });
+    if (!LM) l_run = l_run * al + (psum[0] + psum[1]);
 #pragma unroll
-      for (int i = 0; i < VP; ++i) o[i >> 1] = mfma32(as_bf16x8(vfrag(slot, i)), p_prev[i & 1], o[i >> 1]);
-      const float mx = xor32_max(mx_pair);
-      bad = bad || mx - m_ref > REF_JUMP;
-      if (mx > m_limit && bad) { m_ref = mx; m_limit = m_ref + slack; }
-    }
-    if (pass == 1) break;
-    const unsigned mine = __builtin_amdgcn_ballot_w64(active && bad) != 0 ? 1u : 0u;
-    unsigned* vote = reinterpret_cast<unsigned*>(alds + (2 * st + 1) * Im::SLOT);       // a K image that nobody reads any more
-    if (lane == 0) vote[wave] = mine;
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    unsigned again = 0;
-#pragma unroll
-    for (int w = 0; w < NWAVE; ++w) again |= vote[w];
-    if (__builtin_amdgcn_readfirstlane(again) == 0u) break;
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();                        // the ring is filled anew
+    for (int i = 0; i < 4; ++i) p_prev[i] = as_bf16x8(w[i]);
+    alpha = al;
+  };
+  auto rescale = [&] {                                  // alpha is one while a row's maximum stands (x * 1.0f is exact: its bits do not depend on its neighbours)
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.f) == 0) return;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
-    l_run = 0.f;
+      for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+  };
+
+  // K of tiles tb and tb + 1 (the slots of the third pair-stage, free until the loop's first iteration is past its barrier), then two pairs
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int j = 0; j < PK; ++j) {
+      const int p = min(j * NWAVE + wave, Im::KPD - 1), row = (p * 64 + lane) / Im::CR, c = (p * 64 + lane) % Im::CR;
+      piece(p, min(tb + r, kv.ntile - 1), true, (CLAMP ? 0u : (unsigned)row * kv.k_row) + (unsigned)((c ^ Im::kx(row)) * 16), row, lds0 + (unsigned)(4 + r) * Im::SLOT);
+    }
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+#pragma unroll
+    for (int j = 0; j < PWP; ++j) issue(j, tb + 2 * k, k);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PWP) : "memory");
+  __builtin_amdgcn_s_barrier();
+  if (active) {
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      clear(tb + r, sc[r]);
+#pragma unroll
+      for (int ks = 0; ks < KP; ++ks) sc[r] = mfma32(as_bf16x8(kfrag(alds + (4 + r) * Im::SLOT, ks)), as_bf16x8(qf[ks]), sc[r]);
+    }
   }
-  m_run = m_limit > -INFINITY ? m_ref : -INFINITY;
+  for (int t = tb; t < te; t += 2) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PWP) : "memory");
+    __builtin_amdgcn_s_barrier();
+    if (active) {
+      if (t > tb + 2) rescale();                        // O is zero until then
+      if ((t + 2) * 32 > mlim) pair(std::true_type{}, t); else pair(std::false_type{}, t);
+    } else {
+#pragma unroll
+      for (int j = 0; j < PWP; ++j) issue(j, t + 4, st == 0 ? 2 : st - 1);
+    }
+    st = st == 2 ? 0 : st + 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");     // all pieces: no LDS-DMA of this block may land after it has left the CU
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  if (active) {                // the last pair's P.V: its V^T is in the next pair's slots
+    rescale();
+#pragma unroll
+    for (int i = 0; i < 2 * VP; ++i) o[(i % VP) >> 1] = mfma32(as_bf16x8(vfrag(alds + (2 * st + i / VP) * Im::SLOT, i % VP)), p_prev[2 * (i / VP) + (i & 1)], o[(i % VP) >> 1]);
+  }
 }
 
 // ------------------------------------------------------------------------------------------------------------------------------
@@ -472,7 +450,9 @@ __global__ __launch_bounds__(NWAVE * 64, 2) void attn_vit32_kernel(
 
   u32x4 qf[KP];
   {
-    const bf16_t* qp = qkv + (size_t)(s0 + qrow) * ld + h * D + hh * 8;
+    int hq = hh;          // opaque: formed for every (group, head), not kept in registers through the key loop
+    asm volatile("" : "+v"(hq));
+    const bf16_t* qp = qkv + (size_t)(s0 + qrow) * ld + h * D + hq * 8;
 #pragma unroll
     for (int ks = 0; ks < KP; ++ks) qf[ks] = ld16(qp + ks * 16);
 #pragma unroll

@@ -2,6 +2,7 @@
 whole model: prompts, decoding, portions, batches, slots that are used again, and greedy generation through the model's entry points."""
 import ctypes as C
 import json
+import math
 import os
 import subprocess
 import sys
@@ -247,6 +248,27 @@ def test_biased_attention_with_any_scale(dev, lib, dim, vdim, scale, slopes):
         s = q[:, h].double() @ k.T * scale - float(slope[h]) * dist
         want = torch.softmax(s.masked_fill(dist < 0, -torch.inf), -1) @ v
         assert (out.view(n, heads, vdim)[:, h].double().cpu() - want).abs().max() < 0.03, h
+
+
+@pytest.mark.parametrize("dim,vdim", [(128, 128), (64, 128)])
+def test_biased_attention_rounds_against_the_rows_maximum(dev, lib, dim, vdim):
+    """The bias alone, a factor of 3/4 a key, values on a row's last six keys: bf16 holds those weights (243 / 1024 is the smallest) against the row's
+    largest, so the result's rounding is the only one.  Against any other reference each would be off by up to 2^-8."""
+    past, L = [64, 101, 333, 518, 1000], 1024
+    n = len(past)
+    kvs, arenas, base, k_off, v_off = _kv_slots([1] * n, 1, dim, vdim, L, dev, torch.Generator().manual_seed(dim))
+    for (k, v), a, p in zip(kvs, arenas, past):
+        v[:, :p - 5] = 0
+        view = a[v_off:v_off + L * vdim].view(L // 32, vdim, 32)
+        view.copy_(v[0].view(L // 32, 32, vdim).permute(0, 2, 1).to(dev))
+    q = torch.zeros(n, dim, dtype=torch.bfloat16, device=dev)
+    out = torch.full((n, vdim), 7.0, dtype=torch.bfloat16, device=dev)
+    tabs = [_i32(x, dev) for x in (range(n), [1] * n, past, range(n))]
+    sl = torch.full((1,), math.log2(4 / 3), device=dev)
+    _ok(lib.lcc_gqa_attn_prefill(_p(q), _p(out), *[_p(t) for t in tabs], n, n, 1, 1, dim, vdim, 0.125, _p(sl), _p(base), k_off, v_off, L, _st()))
+    w = 0.75 ** torch.arange(6).double()
+    want = torch.stack([(w[:, None] * v[0, p - 5:p + 1].flip(0).double()).sum(0) / (4 * (1 - 0.75 ** (p + 1))) for (k, v), p in zip(kvs, past)])
+    assert ((out.double().cpu() - want).abs() <= want.abs() * 2.0 ** -8 + 2e-5).all()
 
 
 @pytest.mark.parametrize("dim,vdim,heads,kv,lens,ns", [(64, 64, 6, 1, [1, 2, 31, 32, 33, 64, 65], 2), (128, 128, 12, 2, [700], 11), (128, 64, 34, 2, [64] * 18, 1),

@@ -739,8 +739,8 @@ def test_vit_rope_attention(dev, grids, attn_variant):
 
 @pytest.mark.parametrize("Hq,Hkv,S,past,nsplit", [(28, 4, 70, 200, 1), (28, 4, 70, 330, 2), (8, 2, 33, 95, 1)])
 def test_prefill_attention_of_rows_whose_scores_jump(dev, Hq, Hkv, S, past, nsplit):
-    """Rows whose score jumps by far more than a power of 2^100 behind the first key tiles (the 32x32x16 kernel goes through its keys a second
-    time), rises from pair to pair, or falls from the first key on; the rows beside them keep their bits."""
+    """Rows whose score jumps by far more than a power of 2^100 behind the first key tiles, rises from pair to pair, or falls from the first key on; the
+    rows beside them keep their bits."""
     from livecc_amd import ops
     D, L = 128, S + past
     kv = ops.KvArena(1, 1, Hkv, (L + 31) // 32 * 32, dev)
@@ -758,6 +758,29 @@ def test_prefill_attention_of_rows_whose_scores_jump(dev, Hq, Hkv, S, past, nspl
     _check_attn(got.view(S, Hq, D), rb(_ref_attn_causal(q2.float().view(S, Hq, D), K, V, past)), f"jump[{Hq},{S},{past},{nsplit}]")
     same = [i for i in range(S) if i not in loud]
     assert torch.equal(got[same], plain[same])
+
+
+@pytest.mark.parametrize("Hq,Hkv,S,past,tile", [(28, 4, 70, 330, 36), (8, 2, 33, 415, 32)])
+def test_prefill_attention_of_rows_that_one_key_decides(dev, Hq, Hkv, S, past, tile):
+    """Rows whose probability lies on one key behind the first tiles (some 2^40 above the others): the fp32 partial of its split is that key's value, because the
+    row's largest probability is one and no rounding touches it; a reference other than the maximum would leave up to 2^-8."""
+    from livecc_amd import _lib, ops
+    D, L, ns = 128, S + past, 2
+    kv = ops.KvArena(1, 1, Hkv, (L + 31) // 32 * 32, dev)
+    kv.buf.copy_(_rand(tuple(kv.buf.shape), dev, 0.7, 5))
+    K, V = kv.k_view(0, 0)[:, :L].float(), kv.v_view(0, 0)[:, :L].float()
+    j = torch.randint(40, past + 1, (S, Hq), generator=torch.Generator().manual_seed(Hq))
+    g = torch.arange(Hq) * Hkv // Hq
+    q = (K[g[None].expand(S, Hq), j] * 6).bfloat16().view(S, Hq * D)
+    t = [torch.tensor(x, dtype=torch.int32, device=dev) for x in zip(*[(0, o, min(tile, S - o), past + o) for o in range(0, S, tile)])]
+    out, wo, wm = torch.empty_like(q), torch.empty(S, Hq, ns, D, device=dev), torch.empty(S, Hq, ns, 2, device=dev)
+    _lib.check(_lib.load().lcc_attn_prefill_bf16(q.data_ptr(), out.data_ptr(), *[x.data_ptr() for x in t], kv.ptrs.data_ptr(), kv.lay, 0, t[0].numel(), Hq, tile, ns, S,
+                                                 wo.data_ptr(), wm.data_ptr(), torch.cuda.current_stream().cuda_stream), "lcc_attn_prefill_bf16")
+    pick = wm[..., 0].argmax(-1).view(S, Hq, 1)                       # the split that holds the key
+    part = wo.gather(2, pick[..., None].expand(S, Hq, 1, D))[:, :, 0] / wm[..., 1].gather(2, pick)
+    want = V[g[None].expand(S, Hq), j]
+    # the other keys: at most 2^-20 of the row (measured 1e-9); fp32 sums
+    assert ((part - want).abs() <= want.abs() * 2.0 ** -20 + 2.0 ** -18).all()
 
 
 @pytest.mark.parametrize("rows", [128, 256])
