@@ -120,7 +120,7 @@ LCC_DEVICE void attn32_key_loop(unsigned char* alds, const Kv32& kv, const u32x4
   m_run = -INFINITY;
   if (te <= tb) return;                                 // (block-uniform: a key split without a tile)
   const unsigned lds0 = lds_addr(alds);
-  const float bias_raw = BIAS ? slope / scale_log2e : 0.f, bias_pos = BIAS ? bias_raw * (float)(8 * hh - pos) : 0.f;
+  const float bias_raw = BIAS ? slope / scale_log2e : 0.f;
   const int col = lane & 31;
 
   // DMA: this wave's pieces of a pair.  Surplus slots copy the last piece again (same bytes, same place).
@@ -165,7 +165,9 @@ LCC_DEVICE void attn32_key_loop(unsigned char* alds, const Kv32& kv, const u32x4
   auto vfrag = [&](const unsigned char* slot, int i) { return *reinterpret_cast<const u32x4*>(slot + va[i & 1] + (i >> 1) * 2048); };
 
   auto clear = [&](int t, f32x16& sc) {                           // what K.Q^T of tile t is added to: the bias, in units of unscaled scores
-    const float base = BIAS ? fmaf(bias_raw, (float)(t * 32), bias_pos) : 0.f;
+    // the distance as a whole number, so that near keys keep theirs at any position (slope times position, cancelled against slope times key, is off by
+    // up to 8e-3 in log2 units at 131,000)
+    const float base = BIAS ? bias_raw * (float)(t * 32 + 8 * hh - pos) : 0.f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) sc[r] = BIAS ? fmaf(bias_raw, (float)(16 * (r >> 3) + (r & 7)), base) : 0.f;
   };

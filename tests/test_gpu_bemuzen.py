@@ -250,6 +250,25 @@ def test_biased_attention_with_any_scale(dev, lib, dim, vdim, scale, slopes):
         assert (out.view(n, heads, vdim)[:, h].double().cpu() - want).abs().max() < 0.03, h
 
 
+@pytest.mark.parametrize("dim,vdim", [(128, 128), (64, 64)])
+@pytest.mark.parametrize("past", [70, 8000, 131000])
+def test_biased_attention_keeps_its_distances_at_any_position(dev, lib, dim, vdim, past):
+    """The bias alone, a factor of two a key: every weight is a power of two, so bf16 holds the probabilities and nothing but the result is rounded -- if the
+    distances are.  (Slope times position in fp32, cancelled against slope times key, is off by up to 8e-3 in log2 units at 131,000.)"""
+    n, L, scale = 40, -(-(past + 40) // 64) * 64, 0.125
+    kvs, arenas, base, k_off, v_off = _kv_slots([n], 1, dim, vdim, L, dev, torch.Generator().manual_seed(past))
+    q = torch.zeros(n, dim, dtype=torch.bfloat16, device=dev)
+    out = torch.full((n, vdim), 7.0, dtype=torch.bfloat16, device=dev)
+    tabs = [_i32([x], dev) for x in (0, n, past, 0)]
+    sl = torch.ones(1, device=dev)
+    _ok(lib.lcc_gqa_attn_prefill(_p(q), _p(out), *[_p(t) for t in tabs], 1, n, 1, 1, dim, vdim, scale, _p(sl), _p(base), k_off, v_off, L, _st()))
+    v = kvs[0][1][0].double()
+    w = 2.0 ** -torch.arange(64).double()
+    want = torch.stack([(w[:, None] * v[past + i - 63:past + i + 1].flip(0)).sum(0) / w.sum() for i in range(n)])
+    # 2^-8: one rounding of the result; 2e-5: the scale's fp32 rounding over the nearest keys, values below 6
+    assert ((out.double().cpu() - want).abs() <= want.abs() * 2.0 ** -8 + 2e-5).all()
+
+
 @pytest.mark.parametrize("dim,vdim", [(128, 128), (64, 128)])
 def test_biased_attention_rounds_against_the_rows_maximum(dev, lib, dim, vdim):
     """The bias alone, a factor of 3/4 a key, values on a row's last six keys: bf16 holds those weights (243 / 1024 is the smallest) against the row's
