@@ -1807,7 +1807,8 @@ static float tile_score(int M, int N, int S, int BM, int BN, int slots, float ef
 // Variable-height tiles (round 5; returned as 272): floor(F / 16) row tiles of 16-18 fragments -- scored with every tile as tall as the
 // tallest (a 17-fragment tile costs 17/16 of a 256-row tile on every SIMD), no ragged tile, the 256-row tile's efficiency.
 // LCC_GEMM_VH=0: rounds 2-4 tile choice.
-static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr) {      // score: of the chosen tile, automatic choice only
+// score: of the chosen tile, automatic choice only.  wide_only: 256-column tiles as they stand against a 64 x 128 one that dequantises fp8 weights first (gemm_w8)
+static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr, bool wide_only = false) {
   if (!big_eligible(a)) return 0;
   if (g_gemm_variant == 14) return vh_legal(a) ? 272 : 256;
   if (g_gemm_variant == 3 || g_gemm_variant == 5) return 256;
@@ -1815,7 +1816,7 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr) {    
   if (g_gemm_variant == 13) return a.w_fp8 ? 256 : 192;
   if (g_gemm_variant == 17) return a.w_fp8 ? 256 : 160;
   if (g_gemm_variant == 15) return (a.partial != nullptr && vh_small_shape(a.M, a.K) && vh_legal(a, true)) ? 144 : 128;
-  if (g_gemm_variant == 16) return 129;
+  if (g_gemm_variant == 16) return wide_only ? 128 : 129;
   if (g_gemm_variant != 2) return 0;
   const float s256 = tile_score(a.M, a.N, S, 256, 256, 256, 1.0f, true);
   static const int allow192 = [] { const char* v = getenv("LCC_GEMM_192"); return v ? atoi(v) : 1; }();     // A/B: 0 = round-3 tile choice
@@ -1830,8 +1831,8 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr) {    
   // form's need two; beyond a round the 256-column tiles do (shapes around the lines: 1000 x 3584, K 3584: 43 / 34 / 52 us for 64 x 128 /
   // 128 x 128 / 128 x 256; 1456 x 3584: 73 / 61 / 52; 520 x 3584: 25 / 33 / 50).  With fp8 weights the steps stand alike (4608, K 3584: 386 rows
   // 25 / 33 / 49, 600 rows 42 / 34 / 50, 1000 rows 73 / 61 / 49; 200 x 3584, K 18944 in four splits 68 / 48 / 66).
-  const float s64 = tile_score(a.M, a.N, S, 64, 128, 256, 0.48f, false);
-  const float s128m = tile_score(a.M, a.N, S, 128, 128, 256, 0.70f, false);
+  const float s64 = wide_only ? tile_score(a.M, a.N, S, 64, 128, 512, 0.55f, false) : tile_score(a.M, a.N, S, 64, 128, 256, 0.48f, false);
+  const float s128m = wide_only ? 0.f : tile_score(a.M, a.N, S, 128, 128, 256, 0.70f, false);
   if (score) *score = std::max(std::max(std::max(s256, s192), std::max(s160, s128)), std::max(s128m, s64));
   static const int allow_vh = [] { const char* v = getenv("LCC_GEMM_VH"); return v ? atoi(v) : 1; }();
   if (allow_vh && vh_legal(a) && (((a.M + 15) >> 4) & 15) != 0) {      // F % 16 == 0: the 256-row tiles are the same thing
@@ -2483,8 +2484,12 @@ static int gemm_w8(const GemmArgs& a, hipStream_t st) {
     const bool part = a.partial != nullptr;
     if (part && (a.epilogue != EPI_NONE || a.nsplit < 1 || a.nsplit > 8 || a.nsplit > a.K / 64)) return LCC_ERR_ARG;
     if (a.epilogue == EPI_RESIDUAL && a.residual == nullptr) return LCC_ERR_ARG;
-    const bool tall = !part && tall_wanted(c);
-    const int big = (g_gemm_variant == 7) ? 0 : big_tile_rows(c, part ? a.nsplit : 1);
+    // A C that gemm_bf16 refuses (8-byte stores would not be aligned) only ever went to the 256-column tiles, where they scored above a narrow tile
+    // behind a dequantising pass: they take it by the same lines, and the other shapes refuse it.
+    const bool odd = (a.ldc & 3) != 0 || ((uintptr_t)a.C & 15) != 0;
+    const bool tall = !part && !odd && tall_wanted(c);
+    const int big = (g_gemm_variant == 7) ? 0 : big_tile_rows(c, part ? a.nsplit : 1, nullptr, odd);
+    if (odd && big != 256 && big != 128) return (a.ldc & 3) != 0 ? LCC_ERR_SHAPE : LCC_ERR_ALIGN;
     if (big != 0 || tall || g_gemm_variant == 2) {
 #define LCC_W8_TILE(EPI) (big == 256 ? launch_big<256, EPI>(c, st) : big == 128 ? launch_big<128, EPI>(c, st) : big == 129 ? launch_mid<128, EPI, 4>(c, st) : launch_mid64<EPI>(c, st))
 #define LCC_W8(EPI) (tall ? launch_tall<EPI>(c, st) : LCC_W8_TILE(EPI))

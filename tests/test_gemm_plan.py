@@ -148,3 +148,15 @@ def test_long_contractions_of_a_few_hundred_to_a_few_thousand_rows_are_split(bui
     for M in range(449, 4097, 37):
         for N, K in ((3584, 18944), (1536, 8960), (272, 6144)):
             assert 1 <= plan(M, N, K) <= 6
+
+
+@pytest.mark.parametrize("M,N", [(90, 256), (100, 1024), (386, 3584), (600, 4608)])
+def test_narrow_fp8_products_refuse_a_result_they_cannot_store_aligned(built_lib, M, N):
+    """Shapes of the 64 x 128 and 128 x 128 tiles: rows of C at an odd multiple of four bytes, or C itself at 8 bytes, are refused before anything is launched (host
+    memory stands in for the device's)."""
+    import ctypes as C
+    from livecc_amd import _lib
+    buf = C.create_string_buffer(4096)
+    p = (C.addressof(buf) + 15) // 16 * 16
+    call = lambda c, ldc: built_lib.lcc_gemm_w8_bf16(p, 256, p, C.cast(p, C.POINTER(C.c_float)), None, None, 0, c, ldc, M, N, 256, 0, None, 0, p, None)
+    assert call(p, N + 2) == call(p, N + 1) == -2 and call(p + 8, N) == -3
