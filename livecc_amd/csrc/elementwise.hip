@@ -138,6 +138,7 @@ int layernorm_bf16(const bf16_t* x, const bf16_t* w, const bf16_t* b, bf16_t* y,
                    hipStream_t st) {
   if (rows <= 0) return 0;
   if ((dim & 7) || dim > 4 * 64 * 8 * 4) return LCC_ERR_SHAPE;
+  if (dim <= 0) return 0;          // the kernel's loads are clamped to a row's last piece
   if (dim <= 64 * 8 * 2) layernorm_kernel<1, 2><<<dim3(rows), dim3(64), 0, st>>>(x, w, b, y, dim, eps);
   else if (dim <= 64 * 8 * 3) layernorm_kernel<1, 3><<<dim3(rows), dim3(64), 0, st>>>(x, w, b, y, dim, eps);
   else if (dim <= 64 * 8 * 4) layernorm_kernel<1, 4><<<dim3(rows), dim3(64), 0, st>>>(x, w, b, y, dim, eps);

@@ -27,7 +27,7 @@ LCC_DEVICE void latent_row(const LatentInArgs& a, int row, float* red) {
   // Bound by trips to memory: the first piece of either part (two slabs of it), its norm weights, the gates and the cache address are asked for at once,
   // at clamped addresses instead of behind branches, and the pieces stay in registers across the sums: 32 rows of 768 + 512
   // channels in two slabs, a launch of a decode step, 4.5 -> 3.6 us
-  const int slot = a.rp > 0 ? a.tok_stream[row] : 0, c0 = tid * 4, zc = a.qp + a.rp + min(tid, a.heads - 1);
+  const int slot = a.rp > 0 ? a.tok_stream[row] : 0, c0 = tid * 4, zc = a.qp + a.rp + max(min(tid, a.heads - 1), -1);
   const int cq = QUERY ? min(c0, a.qp - 4) : 0, ck = a.rp > 0 ? a.qp + min(c0, a.rp - 4) : 0;
   const size_t second = a.nsplit > 1 ? slab : 0;
   auto first = [&](int c) { return *reinterpret_cast<const f32x4*>(src + c); };

@@ -66,7 +66,7 @@ LCC_DEVICE void gqa_row_batch(const GqaInArgs& a, int row) {
   const size_t slab = (size_t)a.rows * a.ldn, at = (size_t)row * a.ldn;
   const int slot = a.tok_stream[row], nh = a.heads + a.kv_heads;
   const int vcol = nh * a.dim_pad, nv = a.kv_heads * a.vdim_pad;
-  f32x4 v0 = *reinterpret_cast<const f32x4*>(a.part + at + vcol + min(tid * 4, nv - 4));
+  f32x4 v0 = *reinterpret_cast<const f32x4*>(a.part + at + vcol + max(min(tid * 4, nv - 4), -4));
   const int pos = a.tok_pos ? a.tok_pos[row] : a.kv_len[slot];
   bf16_t* arena = a.kv_base[slot];
   const int L = (a.dim_pad & (a.dim_pad - 1)) == 0 ? a.dim_pad >> 2 : 64, per = 64 / L, sub = lane / L, c = (lane - sub * L) * 4, cc = min(c, a.dim_pad - 4);

@@ -1148,6 +1148,15 @@ def test_embed_gather_with_video_row_scatter_is_bit_exact(dev):
     assert torch.equal(got, table[cur_tok[slots.long()].long().to(dev)])
 
 
+def test_layernorm_without_columns_leaves_everything(dev):
+    """dim 0: the kernel's loads are clamped to a row's last piece, which would lie in front of the buffers -- nothing is launched."""
+    from livecc_amd import _lib
+    lib, t = _lib.load(), torch.full((4, 8), 3.0, dtype=torch.bfloat16, device=dev)
+    assert lib.lcc_layernorm_bf16(*[t.data_ptr()] * 4, 4, 0, 1e-6, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert (t == 3).all()
+
+
 @pytest.mark.parametrize("V", [8192, 8224, 151936, 262144])
 def test_two_stage_sampler_gives_the_single_launch_tokens(dev, V):
     """The spread pass against the one-block pass: short and long shares of a block (32 to 1,024 chunks for 256 threads), equal scores (the lower id wins), masked
