@@ -131,8 +131,9 @@ __global__ __launch_bounds__(NT) void sample_greedy_kernel(
 
 // ---- two-stage variant: stage 1 spreads the V-wide pass over SAMPLE_NB blocks per stream, stage 2 merges the partials.  A block's 600 chunks of 8 scores
 // are one trip to memory (three chunks a thread, asked for together and before the slot's flags are known), and a chunk moves the running maximum once
-// instead of score by score behind a branch.  Both stages and the fill of the result, one row of 151,936 ids 10.8 -> 9.8 us, 32 rows 12.5 -> 12.1 (two
-// chunks each for 512 threads: 9.1 and 13.5)
+// instead of score by score behind a branch.  Both stages and the fill of the result, one row of 151,936 ids 10.8 -> 9.8 us, 32 rows 12.5 -> 12.2 (two
+// chunks each for 512 threads: 9.1 and 13.5).  Rows that are done leave with their first loads on the way: 31 of 32 rows 11.0 -> 10.3, all of them 5.2 -> 5.3 (10.2
+// when they went through their scores to write nothing)
 constexpr int SAMPLE_NB = 32, SAMPLE_NT = 256;
 
 template <class LT>
@@ -148,7 +149,7 @@ __global__ __launch_bounds__(SAMPLE_NT) void sample_partial_kernel(
   const bool frozen = done != nullptr && done[slot];          // writes nothing
   const LT* lg = logits + (size_t)b * ld;
   const uint32_t* sb = seen + (size_t)slot * words;
-  float* so = scores_out && !frozen ? scores_out + (size_t)b * V : nullptr;
+  float* so = scores_out ? scores_out + (size_t)b * V : nullptr;
   const int nch = V / 8, per = (nch + SAMPLE_NB - 1) / SAMPLE_NB;
   const int c0 = blk * per, c1 = min(nch, c0 + per);
   Best best = {-INFINITY, 0x7fffffff};
@@ -160,6 +161,8 @@ __global__ __launch_bounds__(SAMPLE_NT) void sample_partial_kernel(
     for (int u = 0; u < U; ++u) load8_logits(lg, min(cb + u * SAMPLE_NT, c1 - 1), v[u]);
 #pragma unroll
     for (int u = 0; u < U; ++u) word[u] = sb[min(cb + u * SAMPLE_NT, c1 - 1) >> 2];
+    asm volatile("" ::: "memory");      // asked for before the flag is known, and not behind it
+    if (frozen) return;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int c = cb + u * SAMPLE_NT;
@@ -185,6 +188,7 @@ __global__ __launch_bounds__(SAMPLE_NT) void sample_partial_kernel(
       }
     }
   }
+  if (frozen) return;          // (the whole block)
   float wmx = wave_max(mx);
   sum *= (mx == -INFINITY) ? 0.f : __expf(mx - wmx);
   sum = wave_sum(sum);
@@ -196,7 +200,7 @@ __global__ __launch_bounds__(SAMPLE_NT) void sample_partial_kernel(
   thr_score = wave_max(thr_score);
   if (lane == 0) { s_max[wave] = wmx; s_sum[wave] = sum; s_bv[wave] = best.v; s_bi[wave] = best.i; s_thr[wave] = thr_score; }
   __syncthreads();
-  if (tid == 0 && !frozen) {
+  if (tid == 0) {
     float M = -INFINITY, tot = 0.f, ts = -INFINITY;
     Best bb = {-INFINITY, 0x7fffffff};
 #pragma unroll

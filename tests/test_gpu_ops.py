@@ -1176,5 +1176,11 @@ def test_two_stage_sampler_gives_the_single_launch_tokens(dev, V):
         assert torch.equal(a, b) and torch.equal(sa, sb)
     done = torch.tensor([0, 1, 0, 0], dtype=torch.int32, device=dev)
     c, _ = ops.sample_greedy(lg, seen, slots, two_stage=True, done=done)
-    a, _ = ops.sample_greedy(lg, seen, slots)
+    a, sa = ops.sample_greedy(lg, seen, slots, want_scores=True)
     assert c[1] == 0 and torch.equal(c[[0, 2, 3]], a[[0, 2, 3]])
+    from livecc_amd import _lib
+    tok, sc, ws = torch.full((4,), 9, dtype=torch.int32, device=dev), torch.full((4, V), 7.0, device=dev), torch.empty(4 * 256, device=dev)
+    for flags in (done, torch.ones_like(done)):
+        _lib.check(_lib.load().lcc_sample_greedy(lg.data_ptr(), V, 4, V, seen.data_ptr(), V // 32, slots.data_ptr(), 1.0, -1, 0, 0.0, -1, -1, 0, flags.data_ptr(), tok.data_ptr(),
+                                                 None, 0, None, sc.data_ptr(), ws.data_ptr(), torch.cuda.current_stream().cuda_stream), "lcc_sample_greedy")
+        assert tok[1] == 9 and (sc[1] == 7).all() and torch.equal(tok[[0, 2, 3]], a[[0, 2, 3]]) and torch.equal(sc[[0, 2, 3]], sa[[0, 2, 3]])
