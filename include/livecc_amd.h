@@ -140,12 +140,12 @@ int lcc_debug_set_skinny_rows(int rows);
  * 342-368).  Returns the old value. */
 int lcc_debug_set_vit_fused_qkv(int on);
 int lcc_gemv_num_splits(int N, int K);
-/* nn.Linear with fp8 (OCP e4m3) weights, the 72B single-GPU path (BASELINE.json configs[4]): W8 = bytes in the PACKED8 order
+/* nn.Linear with fp8 (OCP e4m3) weights, the 72B single-GPU path: W8 = bytes in the PACKED8 order
  * [N/16][K/64][4 g][16 rows][16 k] (lane (g,row) owns 16 consecutive k), wscale = fp32 [N] per-output-row scale:
  * y[m][n] = epilogue(wscale[n] * sum_k x[m][k] * q[n][k] (+ bias[n])).  M <= 16: weight-streaming GEMV (e4m3 -> bf16 exactly
  * in registers, bf16 MFMA, fp32 accumulate).  M > 16: the GEMM tiles stage the fp8 fragments themselves (half the L2 -> LDS bytes) and
- * expand them to bf16 after the LDS read, the row scale in their epilogue.  dq_scratch (N*K bf16, caller-provided) holds the exactly dequantised
- * weight where a forced tile variant has no such form.  K % 64 == 0, N % 16 == 0.  partial /
+ * expand them to bf16 after the LDS read, the row scale in their epilogue.  dq_scratch: not used, may be NULL (it
+ * held the dequantised weight of the tiles that took bf16 alone).  K % 64 == 0, N % 16 == 0.  partial /
  * nsplit as in lcc_gemm_bf16. */
 int lcc_gemm_w8_bf16(const void* A, int lda, const void* W8, const float* wscale, const void* bias, const void* residual, int ldr,
                      void* C, int ldc, int M, int N, int K, int epilogue, float* partial, int nsplit, void* dq_scratch, void* stream);
@@ -413,7 +413,7 @@ typedef struct {
   int mrope_sec_t, mrope_sec_h, mrope_sec_w;
   int vit_depth, vit_embed, vit_heads, vit_mlp, patch_dim, merge;
   int llm_fp8;   /* 1: the LLM Linear weights (q/k/v, o, gate/up, down, lm_head) are fp8 e4m3 (PACKED8 order) + fp32 row scales
-                    set as "<name>.scale"; the workspace then includes a bf16 dequantisation scratch for prefill */
+                    set as "<name>.scale" */
 } lcc_model_config;
 
 typedef struct {

@@ -64,7 +64,6 @@ size_t lcc_engine::llm_ws_bytes() const {
   t += align_up(16 * (H / 8 + 4) * 4);      // decode v2: per-tile sums of squares of the residual rows
   t += align_up(B * V * 2);                  // logits
   t += align_up(std::max<size_t>(B * c.n_kv_heads * 128 * 16, std::min<size_t>(S, 1024) * c.n_q_heads * 8) * 128 * 4) * 2;  // attention split partials (o, ml)
-  if (c.llm_fp8) t += align_up(std::max<size_t>((size_t)qkvd * H, 2 * I * H) * 2);   // bf16 dequantisation scratch of the largest LLM weight
   return t + 4096;
 }
 size_t lcc_engine::vit_ws_bytes() const {

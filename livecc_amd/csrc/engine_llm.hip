@@ -21,7 +21,7 @@ int g_fuse_tails = 0;   // 1: batch-1 decode runs rope/KV-append and residual+RM
                         // block, ticket counter).  Measured on MI355X at 7B shapes: 184 tok/s fused vs 215 tok/s with separate
                         // kernels (the slab write-through + ticket serialises the GEMV's tail), so it stays an opt-in variant.
 struct LlmBuffers {
-  bf16_t *h, *xn, *qkv, *q, *attn, *act, *cos, *sin, *last_h, *last_xn, *logits, *dq;
+  bf16_t *h, *xn, *qkv, *q, *attn, *act, *cos, *sin, *last_h, *last_xn, *logits;
   float *partial, *ws_o, *ws_ml, *stats;
 };
 int carve_llm(lcc_engine* e, LlmBuffers* b) {
@@ -36,7 +36,6 @@ int carve_llm(lcc_engine* e, LlmBuffers* b) {
   b->logits = cv.take<bf16_t>(B * V);
   const size_t nslot = std::max<size_t>(B * e->c.n_kv_heads * 128 * 16, std::min<size_t>(S, 1024) * e->c.n_q_heads * 8);
   b->ws_o = cv.take<float>(nslot * 128); b->ws_ml = cv.take<float>(nslot * 128);
-  b->dq = e->c.llm_fp8 ? cv.take<bf16_t>(std::max<size_t>((size_t)e->qkvd * H, 2 * I * H)) : nullptr;
   if (cv.off > e->ws_bytes) return fail(LCC_ERR_STATE, "workspace too small");
   return 0;
 }
@@ -65,10 +64,10 @@ int run_layers(lcc_engine* e, const LlmBuffers& b, const LayerCtx& cx, hipStream
   static const int qkv_split_on = [] { const char* v = getenv("LCC_PREFILL_QKV_SPLIT"); return v ? atoi(v) : 1; }();
   const int tp_qkv = (cx.skinny || !qkv_split_on || e->c.llm_fp8 || (size_t)6 * std::min<size_t>(e->lim.max_new_rows, 4096) * H <
                       (size_t)8 * S * e->qkvd) ? 1 : gemm_tiled_num_splits(S, e->qkvd, H, true);
-  // fp8 weights: the same GemmArgs with the byte pointer, the row scales and the dequantisation scratch of the tiled path
+  // fp8 weights: the same GemmArgs with the byte pointer and the row scales
   auto set_w = [&](GemmArgs& g, const bf16_t* w, const float* scale) {
     g.w_packed = 1; g.W = w;
-    if (scale != nullptr) { g.w_fp8 = 1; g.wscale = scale; g.dq_scratch = b.dq; }
+    if (scale != nullptr) { g.w_fp8 = 1; g.wscale = scale; }
   };
   LCC_TRY(rmsnorm_bf16(b.h, e->llm[0].in_norm, b.xn, S, H, eps, st));
   // parity instrumentation: tap 0 = embeddings, 2l+1 = residual stream after the attention block of layer l, 2l+2 = after its MLP;

@@ -356,7 +356,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, int ldw,
     const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
     bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n, int w_packed,
-    float* __restrict__ partial, int kt_per_split, const float* __restrict__ wscale) {
+    float* __restrict__ partial, int kt_per_split) {
   constexpr int BN = 128, BK = 64;
   constexpr int WM = BM / 2;       // wave tile rows (of A)
   constexpr int MT = WM / 16;      // 16-row MFMA tiles per wave in M
@@ -462,7 +462,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(
     __syncthreads();
   }
 
-  tile_epilogue<EPI, MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, (n0 + wn * 64) / 2, li, g, bias, residual, ldr, C, ldc, M, N, partial, wscale);
+  tile_epilogue<EPI, MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, (n0 + wn * 64) / 2, li, g, bias, residual, ldr, C, ldc, M, N, partial, nullptr);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -480,7 +480,7 @@ __global__ __launch_bounds__(256) void gemm_glds_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, int ldw,
     const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
     bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n, int w_packed,
-    float* __restrict__ partial, int kt_per_split, const float* __restrict__ wscale) {
+    float* __restrict__ partial, int kt_per_split) {
   constexpr int BN = 128, BK = 64, NSTAGE = 3;
   constexpr int WM = BM / 2, MT = WM / 16, NT = 4;
   constexpr int A_SUB = (BM / 16) * 2;          // 1-KB sub-tiles of the A tile (row tiles x 2 k-blocks)
@@ -576,7 +576,7 @@ __global__ __launch_bounds__(256) void gemm_glds_kernel(
         for (int j = 0; j < NT; ++j) acc[i][j] = mfma16(fb[j], fa[i], acc[i][j]);
     }
   }
-  tile_epilogue<EPI, MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, (n0 + wn * 64) / 2, li, g, bias, residual, ldr, C, ldc, M, N, partial, wscale);
+  tile_epilogue<EPI, MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, (n0 + wn * 64) / 2, li, g, bias, residual, ldr, C, ldc, M, N, partial, nullptr);
   if (vb + (int)gridDim.x < nblk) __syncthreads();     // the next tile's DMA reuses the stages
   }
 }
@@ -986,7 +986,7 @@ __global__ __launch_bounds__(512) void gemm_walk_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
     const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
     bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n,
-    float* __restrict__ partial, int kt_per_split, const float* __restrict__ wscale, int raster) {
+    float* __restrict__ partial, int kt_per_split, int raster) {
   constexpr int BN = 256, BK = 64, NSTAGE = walk_stages(BM);
   constexpr int WM = BM / 2, MT = WM / 16, NT = 4;
   constexpr int A_UNITS = BM * 8, STAGE = A_UNITS + 2048;        // 16-byte units: activations, then 32 weight sub-tiles
@@ -1113,10 +1113,10 @@ __global__ __launch_bounds__(512) void gemm_walk_kernel(
     int l = lane;          // opaque: the epilogue's addresses are formed here and not kept in registers through the k-loop
     asm volatile("" : "+v"(l));
     if constexpr (EPI == EPI_PARTIAL) {
-      tile_slab_wide<MT, NT, 1, EGR * 2>(acc, m0 + wm * WM, n0 + wn * 64, l, M, N, partial, wscale, elds);
+      tile_slab_wide<MT, NT, 1, EGR * 2>(acc, m0 + wm * WM, n0 + wn * 64, l, M, N, partial, nullptr, elds);
     } else if (wide_rows<EPI>(C, ldc, bias, residual, ldr)) {
-      tile_epilogue_wide<EPI, MT, NT, EGR>(acc, m0 + wm * WM, n0 + wn * 64, l, bias, residual, ldr, C, ldc, M, N, wscale, elds);
-    } else tile_epilogue<EPI, MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, (n0 + wn * 64) / 2, l & 15, l >> 4, bias, residual, ldr, C, ldc, M, N, partial, wscale);
+      tile_epilogue_wide<EPI, MT, NT, EGR>(acc, m0 + wm * WM, n0 + wn * 64, l, bias, residual, ldr, C, ldc, M, N, nullptr, elds);
+    } else tile_epilogue<EPI, MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, (n0 + wn * 64) / 2, l & 15, l >> 4, bias, residual, ldr, C, ldc, M, N, partial, nullptr);
     all_stored = m0 + BM <= M && n0 + BN <= N;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the copies behind the last tile: this block's LDS until they have landed
@@ -1677,12 +1677,12 @@ static void launch_tiled(const GemmArgs& a, hipStream_t st) {
     }
     gemm_glds_kernel<BM, EPI><<<dim3(capped_grid((long)tiles_m * tiles_n), S), dim3(256), lds, st>>>(
         a.A, a.lda, a.W, a.ldw, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.w_packed, a.partial,
-        (nkt + S - 1) / S, a.wscale);
+        (nkt + S - 1) / S);
     return;
   }
   gemm_tiled_kernel<BM, EPI><<<dim3(tiles_m * tiles_n, S), dim3(256), 0, st>>>(
       a.A, a.lda, a.W, a.ldw, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.w_packed, a.partial,
-      (nkt + S - 1) / S, a.wscale);
+      (nkt + S - 1) / S);
 }
 
 // LCC_GEMM_RASTER (A/B, read once): band width of the tile order of the 8-wave kernels (bands of G column tiles walked row-major: the ~32
@@ -1718,14 +1718,12 @@ static void launch_walk(const GemmArgs& a, hipStream_t st) {
   if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_walk_kernel<BM, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   const unsigned grid = walk_grid((long)tiles_m * tiles_n, S);
   gemm_walk_kernel<BM, EPI><<<dim3(grid, S), dim3(512), lds, st>>>(a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m,
-                                                                   tiles_n, a.partial, (nkt + S - 1) / S, a.wscale, raster_for(tiles_m));
+                                                                   tiles_n, a.partial, (nkt + S - 1) / S, raster_for(tiles_m));
 }
 // variable-height row tiles (gemm_vh_kernel): tiles_m = floor(F / 16) row tiles for F = ceil(M / 16) row fragments (small class: F / 8)
 static bool vh_legal(const GemmArgs& a, bool small = false) {
   const int F = (a.M + 15) >> 4, t = F >> (small ? 3 : 4);
-  // wscale == nullptr: gemm_w8's dequantisation fallback re-enters with w_fp8 = 0 and a LIVE row scale for the epilogue, which
-  // this kernel does not carry
-  return a.w_packed && !a.w_fp8 && a.wscale == nullptr && (a.K % 64) == 0 && t >= 1 && F <= (small ? 9 : 18) * t && (a.N & 15) == 0 && walk_offsets_fit(a);
+  return a.w_packed && !a.w_fp8 && (a.K % 64) == 0 && t >= 1 && F <= (small ? 9 : 18) * t && (a.N & 15) == 0 && walk_offsets_fit(a);
 }
 template <int EPI>
 static void launch_vh(const GemmArgs& a, hipStream_t st) {
@@ -1824,7 +1822,7 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr, bool 
   // BM 160 (bf16 weights): where 192 rows start a last round that is mostly empty.  The vision proj / fc2 of 15,840 rows are 83 x 5 tiles of 192 rows =
   // 1.62 rounds; 99 x 5 of 160 fill 1.93 at 5/6 of the time each: proj 55.7 -> 52.1 us, fc2 201 -> 178.
   // 1000 / 2100 x 17920, K 1536 with SwiGLU 63.6 -> 58.4 / 117.5 -> 111.3.
-  const float s160 = (a.w_fp8 || !allow192 || a.wscale != nullptr) ? 0.f : tile_score(a.M, a.N, S, 160, 256, 256, 0.90f, false);
+  const float s160 = (a.w_fp8 || !allow192) ? 0.f : tile_score(a.M, a.N, S, 160, 256, 256, 0.90f, false);
   const float s128 = tile_score(a.M, a.N, S, 128, 256, 256, 0.85f, true);
   // gemm_mid_kernel: 0.38 / 0.52 us a step of 64 x 128 / 128 x 128 against 0.85 of 128 x 256, one tile a compute unit at a time (two 64-row
   // tiles side by side take twice as long).  Returned as 0 / 129.  The 128-row form wins where its blocks fill one round and the 64-row
@@ -1866,7 +1864,7 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr, bool 
 // The tall kernel serves one-block-row problems whose column tiles fill most of ONE round of the chip (7B gate/up at a streaming
 // chunk: 237 blocks).  Variant 8 forces it wherever it is legal (tests).
 // (fp8 weights with a residual would need more registers than a wave has)
-static bool tall_legal(const GemmArgs& a) { return big_eligible(a) && (a.w_fp8 ? a.epilogue != EPI_RESIDUAL : a.wscale == nullptr) && a.M <= 448 && (a.N & 15) == 0; }
+static bool tall_legal(const GemmArgs& a) { return big_eligible(a) && !(a.w_fp8 && a.epilogue == EPI_RESIDUAL) && a.M <= 448 && (a.N & 15) == 0; }
 static bool tall_wanted(const GemmArgs& a) {
   if (!tall_legal(a)) return false;
   if (g_gemm_variant == 8) return true;
@@ -2260,7 +2258,7 @@ static void launch_gemv_rows(const GemmArgs& a, int S, void* out, int ldo, int c
 }
 
 // ------------------------------------------------------------------------------------------------
-// fp8 weights (OCP e4m3, per-output-row fp32 scale): decode GEMV + exact dequantisation for the tiled GEMMs
+// fp8 weights (OCP e4m3, per-output-row fp32 scale): decode GEMV, and the routes of every product
 // ------------------------------------------------------------------------------------------------
 // PACKED8 layout [N/16][K/64][4 g][16 rows][16 k] bytes: lane (g, row) of a 16-row x 64-k fragment owns the 16 consecutive
 // k = kb*64 + g*16 .. +15 of its row, i.e. ONE 16-byte load per lane per fragment and 1 KB contiguous per wave load -- the same
@@ -2372,21 +2370,6 @@ __global__ __launch_bounds__(256) void gemv_w8_kernel(
   }
 }
 
-// PACKED8 fp8 -> bf16 packed fragments (exact; no scale): thread = one 16-byte piece (row, 16 k) of a 16 x 64 fragment ->
-// the two 16-byte pieces (g' = 2*(g&1), 2*(g&1)+1) of the bf16 fragment of 32-k block 2*kb + (g >> 1)
-__global__ __launch_bounds__(256) void dequant_w8_kernel(const uint8_t* __restrict__ W8, bf16_t* __restrict__ out, size_t n_pieces) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n_pieces) return;
-  const size_t frag = i >> 6;                    // (row tile, 64-k block)
-  const int lane = (int)(i & 63), g = lane >> 4, row = lane & 15;
-  const u32x4 q = ld16(W8 + i * 16);
-  const bf16x8 lo = fp8x8_to_bf16x8(q[0], q[1]), hi = fp8x8_to_bf16x8(q[2], q[3]);
-  // bf16 packed: [row tile][32-k block][4 g'][16 rows][8 k]; 32-k block index = 2*kb64 + (g >> 1); frag already = rt*nchunk + kb64
-  bf16_t* dst = out + (frag * 2 + (size_t)(g >> 1)) * 512 + ((g & 1) * 2 * 16 + row) * 8;
-  st16(dst, as_u32x4(lo));
-  st16(dst + 16 * 8, as_u32x4(hi));
-}
-
 // layout probe (tests/test_gpu_ops.py::test_mfma_layout_probe): D[16x16] = A[16x32] * B[32x16] with the fragment maps of
 // common.h, one wave.  Verifies the operand/result lane maps every kernel in this library relies on.
 __global__ __launch_bounds__(64) void mfma_probe_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
@@ -2478,42 +2461,30 @@ static int gemm_w8(const GemmArgs& a, hipStream_t st) {
     }
     return 0;
   }
-  // M > 16: the tile kernels consume the fp8 fragments directly (e4m3 -> bf16 after the LDS read) ...
-  {
-    GemmArgs c = a; c.w_packed = 1;
-    const bool part = a.partial != nullptr;
-    if (part && (a.epilogue != EPI_NONE || a.nsplit < 1 || a.nsplit > 8 || a.nsplit > a.K / 64)) return LCC_ERR_ARG;
-    if (a.epilogue == EPI_RESIDUAL && a.residual == nullptr) return LCC_ERR_ARG;
-    // A C that gemm_bf16 refuses (8-byte stores would not be aligned) only ever went to the 256-column tiles, where they scored above a narrow tile
-    // behind a dequantising pass: they take it by the same lines, and the other shapes refuse it.
-    const bool odd = (a.ldc & 3) != 0 || ((uintptr_t)a.C & 15) != 0;
-    const bool tall = !part && !odd && tall_wanted(c);
-    const int big = (g_gemm_variant == 7) ? 0 : big_tile_rows(c, part ? a.nsplit : 1, nullptr, odd);
-    if (odd && big != 256 && big != 128) return (a.ldc & 3) != 0 ? LCC_ERR_SHAPE : LCC_ERR_ALIGN;
-    if (big != 0 || tall || g_gemm_variant == 2) {
+  // the tile kernels consume the fp8 fragments directly (e4m3 -> bf16 after the LDS read); forced variants without such a kernel take the 64 x 128 tile
+  GemmArgs c = a; c.w_packed = 1;
+  const bool part = a.partial != nullptr;
+  if (part && (a.epilogue != EPI_NONE || a.nsplit < 1 || a.nsplit > 8 || a.nsplit > a.K / 64)) return LCC_ERR_ARG;
+  if (a.epilogue == EPI_RESIDUAL && a.residual == nullptr) return LCC_ERR_ARG;
+  // A C that gemm_bf16 refuses (8-byte stores would not be aligned) only ever went to the 256-column tiles, where they scored above a narrow tile
+  // behind a dequantising pass: they take it by the same lines, and the other shapes refuse it.
+  const bool odd = (a.ldc & 3) != 0 || ((uintptr_t)a.C & 15) != 0;
+  const bool tall = !part && !odd && tall_wanted(c);
+  const int big = (g_gemm_variant == 7) ? 0 : big_tile_rows(c, part ? a.nsplit : 1, nullptr, odd);
+  if (odd && big != 256 && big != 128) return (a.ldc & 3) != 0 ? LCC_ERR_SHAPE : LCC_ERR_ALIGN;
 #define LCC_W8_TILE(EPI) (big == 256 ? launch_big<256, EPI>(c, st) : big == 128 ? launch_big<128, EPI>(c, st) : big == 129 ? launch_mid<128, EPI, 4>(c, st) : launch_mid64<EPI>(c, st))
 #define LCC_W8(EPI) (tall ? launch_tall<EPI>(c, st) : LCC_W8_TILE(EPI))
-      if (part) { LCC_W8_TILE(EPI_PARTIAL); return 0; }
-      switch (a.epilogue) {
-        case EPI_NONE: LCC_W8(EPI_NONE); return 0;
-        case EPI_QUICK_GELU: LCC_W8(EPI_QUICK_GELU); return 0;
-        case EPI_GELU_ERF: LCC_W8(EPI_GELU_ERF); return 0;
-        case EPI_RESIDUAL: LCC_W8(EPI_RESIDUAL); return 0;
-        case EPI_SWIGLU: LCC_W8(EPI_SWIGLU); return 0;
-        default: return LCC_ERR_ARG;
-      }
+  if (part) { LCC_W8_TILE(EPI_PARTIAL); return 0; }
+  switch (a.epilogue) {
+    case EPI_NONE: LCC_W8(EPI_NONE); return 0;
+    case EPI_QUICK_GELU: LCC_W8(EPI_QUICK_GELU); return 0;
+    case EPI_GELU_ERF: LCC_W8(EPI_GELU_ERF); return 0;
+    case EPI_RESIDUAL: LCC_W8(EPI_RESIDUAL); return 0;
+    case EPI_SWIGLU: LCC_W8(EPI_SWIGLU); return 0;
+    default: return LCC_ERR_ARG;
+  }
 #undef LCC_W8
 #undef LCC_W8_TILE
-    }
-  }
-  // ... forced variants without such a kernel: exact dequantisation into the bf16 packed order, then the 4-wave bf16 GEMM with
-  // the row scale in its epilogue
-  if (a.dq_scratch == nullptr) return LCC_ERR_ARG;
-  const size_t pieces = (size_t)a.N * a.K / 16;
-  dequant_w8_kernel<<<dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, st>>>(W8, a.dq_scratch, pieces);
-  GemmArgs b = a;
-  b.w_fp8 = 0; b.W = a.dq_scratch; b.w_packed = 1; b.ldw = a.K;
-  return gemm_bf16(b, st);
 }
 
 int gemm_bf16(const GemmArgs& a, hipStream_t st) {

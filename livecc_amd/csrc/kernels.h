@@ -74,9 +74,8 @@ struct GemmArgs {
   int epilogue = 0;
   GemvTail tail;
   // fp8 (OCP e4m3) weights: W points at bytes in the PACKED8 order [N/16][K/64][4 g][16 rows][16 k], wscale = fp32 [N]
-  // (y[n] = wscale[n] * sum_k x[k] q[n][k]); M > 16: tiles that convert the bytes behind their LDS read; forced variants
-  // without one go through dq_scratch = N*K bf16 (exact dequantisation into the bf16 packed order, then the bf16 GEMM)
-  int w_fp8 = 0; const float* wscale = nullptr; bf16_t* dq_scratch = nullptr;
+  // (y[n] = wscale[n] * sum_k x[k] q[n][k]); M > 16: tiles that convert the bytes behind their LDS read
+  int w_fp8 = 0; const float* wscale = nullptr;
   VitQkvEpi vq;                                 // epilogue == GEMM_EPI_VIT_QK / GEMM_EPI_VIT_V only
 };
 int gemm_bf16(const GemmArgs& a, hipStream_t st);

@@ -70,10 +70,10 @@ extern "C" int lcc_gemm_w8_bf16(const void* A, int lda, const void* W8, const fl
                                 int ldr, void* C, int ldc, int M, int N, int K, int epilogue, float* partial, int nsplit,
                                 void* dq_scratch, void* stream) {
   if (!A || !W8 || !wscale || (!C && !partial)) return fail(LCC_ERR_ARG, "lcc_gemm_w8_bf16: null pointer");
-  if (M > 16 && !dq_scratch) return fail(LCC_ERR_ARG, "lcc_gemm_w8_bf16: M > 16 needs dq_scratch (N*K bf16)");
+  (void)dq_scratch;
   GemmArgs g; g.A = (const bf16_t*)A; g.lda = lda; g.W = (const bf16_t*)W8; g.ldw = K; g.w_packed = 1; g.bias = (const bf16_t*)bias;
   g.residual = (const bf16_t*)residual; g.ldr = ldr; g.C = (bf16_t*)C; g.ldc = ldc; g.M = M; g.N = N; g.K = K; g.epilogue = epilogue;
-  g.partial = partial; g.nsplit = nsplit; g.w_fp8 = 1; g.wscale = wscale; g.dq_scratch = (bf16_t*)dq_scratch;
+  g.partial = partial; g.nsplit = nsplit; g.w_fp8 = 1; g.wscale = wscale;
   if (partial && C == nullptr) g.C = (bf16_t*)partial;
   OP_RET(gemm_bf16(g, (hipStream_t)stream), "lcc_gemm_w8_bf16");
 }

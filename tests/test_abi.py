@@ -59,6 +59,10 @@ def test_engine_sizing_queries_work_without_gpu(lib):
     # 57,344 B per token x 32768 tokens
     assert lib.lcc_engine_kv_bytes_per_slot(e) == 57344 * 32768 == c.kv_bytes_per_token * 32768
     assert lib.lcc_engine_workspace_bytes(e) > 0 and lib.lcc_engine_meta_bytes(e) > 0
+    cfg.llm_fp8 = 1          # every tile takes the bytes as they are: nothing is set aside for a bf16 copy of a weight
+    e8 = lib.lcc_engine_create(ctypes.byref(cfg), ctypes.byref(lim))
+    assert lib.lcc_engine_workspace_bytes(e8) == lib.lcc_engine_workspace_bytes(e)
+    lib.lcc_engine_destroy(e8)
     lib.lcc_engine_destroy(e)
 
 

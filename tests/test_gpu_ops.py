@@ -379,7 +379,7 @@ def test_gemv_w8_fp8_weights(dev, M, N, K):
 @pytest.mark.parametrize("M,I,K", [(1, 512, 256), (8, 2432, 896), (300, 2432, 896), (40, 512, 256), (530, 400, 128)])
 @pytest.mark.parametrize("variant", [2, 3, 4])
 def test_gemm_w8_swiglu(dev, M, I, K, variant):
-    """gate/up with fp8 weights: skinny GEMV (M <= 16) and the dequantise-then-GEMM path (M > 16), SwiGLU epilogue with the
+    """gate/up with fp8 weights: skinny GEMV (M <= 16) and the tiles (M > 16), SwiGLU epilogue with the
     row scales applied before the activation."""
     from livecc_amd import ops
     from livecc_amd.weights import dequantize_fp8_rows, quantize_fp8_rows
@@ -400,8 +400,7 @@ def test_gemm_w8_swiglu(dev, M, I, K, variant):
 @pytest.mark.parametrize("variant", [2, 3, 4, 7])
 def test_gemm_w8_tiled(dev, M, N, K, epi, variant):
     """M > 16 with fp8 weights.  variant 3 / 4: the 8-wave 256x256 / 128x256 kernel reads the fp8 fragments directly (e4m3 ->
-    bf16 after the LDS read, three 48-KB stages); 7: exact dequantisation into the bf16 fragment order + the 4-wave bf16 GEMM;
-    2: the shipped choice.  The row scale is applied in the epilogue in every case."""
+    bf16 after the LDS read, three 48-KB stages); 7: the 64 x 128 tile; 2: the shipped choice.  The row scale is applied in the epilogue in every case."""
     from livecc_amd import ops
     from livecc_amd.weights import dequantize_fp8_rows, quantize_fp8_rows
     x, w, b = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.05, 2).float(), _rand((N,), dev, 0.1, 3)
