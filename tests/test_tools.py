@@ -1,6 +1,9 @@
-"""Host-side tools: the kernel-trace breakdown (tools/trace_breakdown.py) on a synthetic rocprofv3 CSV."""
+"""Host-side tools on synthetic rocprofv3 CSVs: the kernel-trace breakdown (tools/trace_breakdown.py), the counter summary (tools/summarize_pmc.py)."""
 import importlib.util
+import json
 import os
+import subprocess
+import sys
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -35,3 +38,18 @@ def test_trace_breakdown_finds_decode_steps_and_gaps(tmp_path):
     assert out["avg_gap_per_step_us"] == 0.6                       # 6 gaps of 100 ns inside a step
     assert out["kernels"]["dgemv_kernel<2, 1, 1, 4, 1, 2>"] == dict(calls_per_step=2.0, avg_us=40.0, us_per_step=80.0)
     assert "gemm_big_kernel<128, 4, 1, false>" not in out["kernels"]
+
+
+def test_summarize_pmc_files_every_product_kernel_under_its_own_name(tmp_path):
+    d = tmp_path / "pmc_gemm_a"
+    d.mkdir()
+    rows = ["Kernel_Name,Counter_Name,Counter_Value,Grid_Size,Start_Timestamp,End_Timestamp"]
+    for name, grid, us in (("void lcc::gemm_walk_vh_kernel<4>(unsigned short const*)", 131072, 900), ("void lcc::gemm_walk_kernel<256, 3>(unsigned short const*)", 131072, 400),
+                           ("void lcc::gemm_big_kernel<128, 4, 1, true>(unsigned short const*)", 131072, 90), ("lcc::gemm_vh_kernel(unsigned short const*)", 216 * 512, 20),
+                           ("lcc::gemm_vh_kernel(unsigned short const*)", 252 * 512, 40), ("void lcc::gemm_tall_kernel<4, 1, false>(unsigned short const*)", 121344, 110),
+                           ("void lcc::attn_vit32_kernel<4>(unsigned short const*)", 1, 1)):
+        rows.append(f'"{name}",MfmaUtil,30,{grid},1000,{1000 + us * 1000}')
+    (d / "x_counter_collection.csv").write_text("\n".join(rows) + "\n")
+    r = subprocess.run([sys.executable, os.path.join(ROOT, "tools", "summarize_pmc.py"), str(tmp_path)], capture_output=True, text=True, check=True)
+    assert set(json.loads(r.stdout)["gemm_counters_mean_per_dispatch"]) == {
+        "M3088_gemm_walk_vh_kernel", "M3088_gemm_walk_kernel_256", "M386_gemm_big_kernel_128", "M386_qkv_splitk4_vh_small", "M386_down_splitk6_vh_small", "M386_gemm_tall_kernel"}

@@ -34,12 +34,13 @@ gemm = {}
 for f in glob.glob(os.path.join(out, "pmc_gemm_*", "**", "*counter_collection.csv"), recursive=True):
     for r in csv.DictReader(open(f)):
         kn = r.get("Kernel_Name", "")
-        if "gemm_big_kernel" not in kn and "gemm_tall_kernel" not in kn and "gemm_vh_kernel" not in kn:
+        kind = next((k for k in ("gemm_walk_vh_kernel", "gemm_walk_kernel", "gemm_big_kernel", "gemm_tall_kernel", "gemm_vh_kernel") if k in kn), None)
+        if kind is None:
             continue
-        # round 5: the gate/up GEMM at M = 3088 runs on the variable-height tiles (gemm_vh_kernel: 12 x 148 tiles of 256 / 272 rows)
-        key = ("M386_gemm_tall_kernel" if "gemm_tall_kernel" in kn else "M3088_gemm_vh_kernel" if "gemm_vh_kernel" in kn else
-               "M3088_gemm_big_kernel_256" if "<256" in kn else "M386_gemm_big_kernel_128")
-        if "gemm_vh_kernel<5, 1>" in kn:      # the small variable-height class (split-K slabs of one chunk): 54 tiles x 4 splits = q/k/v, 42 x 6 = o / down
+        # the gate/up GEMM at M = 3088 runs on the variable-height tiles (gemm_walk_vh_kernel: 12 x 148 tiles of 256 / 272 rows)
+        key = ("M386_" if kind == "gemm_tall_kernel" else "M3088_") + kind if kind in ("gemm_tall_kernel", "gemm_walk_vh_kernel") else (
+            f"M3088_{kind}_256" if "<256" in kn else f"M386_{kind}_128")
+        if kind == "gemm_vh_kernel":      # the small variable-height class (split-K slabs of one chunk): 54 tiles x 4 splits = q/k/v, 42 x 6 = o / down
             grid = int(r.get("Grid_Size", 0)) // 512
             dur = (float(r["End_Timestamp"]) - float(r["Start_Timestamp"])) / 1e3
             key = "M386_qkv_splitk4_vh_small" if grid == 216 else ("M386_down_splitk6_vh_small" if dur > 35.0 else "M386_o_splitk6_vh_small")
