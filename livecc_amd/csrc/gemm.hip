@@ -4,7 +4,7 @@
 // bf16 (16 bytes) per lane.  fp32 accumulation, one rounding to bf16 at the points where HF rounds.
 //
 //  * gemm_walk_kernel    : M >= 17, packed W, K % 64 == 0 (LLM prefill, ViT).  MFMA-bound.  8 waves, BM x 256 x 64 tile
-//                          (BM 256 / 192 / 128), LDS-DMA for both operands; one block a compute unit, the DMA ring runs on from tile to tile.
+//                          (BM 256 / 192 / 160 / 128), LDS-DMA for both operands; one block a compute unit, the DMA ring runs on from tile to tile.
 //  * gemm_big_kernel     : the same tiles one a block: fp8-e4m3 W converted after the LDS read, and the vision q|k|v epilogues.
 //  * gemm_walk_vh_kernel : the walk over row tiles of 256 / 272 / 288 rows (no ragged last row tile).
 //  * gemm_vh_kernel      : row tiles of 128 / 144 rows, split-K slabs of one streaming chunk.
@@ -1293,12 +1293,8 @@ __global__ __launch_bounds__(512) void gemm_walk_vh_kernel(
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the copies behind the last tile
 }
 
-template <int EPI>
-__global__ __launch_bounds__(512) void gemm_vh_kernel(
-    const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
-    const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
-    bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n,
-    float* __restrict__ partial, int kt_per_split, int raster) {
+__global__ __launch_bounds__(512) void gemm_vh_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, int M, int N, int K, int tiles_m,
+                                                      int tiles_n, float* __restrict__ partial, int kt_per_split, int raster) {
   constexpr int BN = 256, BK = 64, NT = 4;
   constexpr int MTX = 5, MTL = 4;                            // row fragments of an M-wave: MTL or MTX
   constexpr int APW = 2;                                     // 8-row activation pieces per wave below XBASE
@@ -1368,8 +1364,7 @@ __global__ __launch_bounds__(512) void gemm_vh_kernel(
   };
 
   const int nkt_all = K / BK;
-  const int kt0 = (EPI == EPI_PARTIAL) ? blockIdx.y * kt_per_split : 0;
-  const int nkt = (EPI == EPI_PARTIAL) ? min(nkt_all, kt0 + kt_per_split) : nkt_all;
+  const int kt0 = blockIdx.y * kt_per_split, nkt = min(nkt_all, kt0 + kt_per_split);
   if (kt0 < nkt) {      // tiles kt0 .. kt0 + NST - 2 (clamped) into stages 0 .. NST - 2
 #pragma unroll
     for (int p = 0; p < NST - 1; ++p)
@@ -1430,16 +1425,9 @@ __global__ __launch_bounds__(512) void gemm_vh_kernel(
       }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the clamped copies of the last iteration
-    const bool wide = EPI == EPI_PARTIAL || wide_rows<EPI>(C, ldc, bias, residual, ldr);          // block-uniform
-    if (wide) __builtin_amdgcn_s_barrier();          // every wave is done with the stages, and its DMA pieces have landed
-    if constexpr (MTW > 0 && EPI == EPI_PARTIAL) {
+    __builtin_amdgcn_s_barrier();          // every wave is done with the stages, and its DMA pieces have landed
+    if constexpr (MTW > 0)
       tile_slab_wide<MTW, NT>(acc, m0 + my_row0, n0 + wn * 64, lane, M, N, partial, nullptr, reinterpret_cast<unsigned char*>(dsmem) + wave * 8192);
-    } else if constexpr (MTW > 0) {
-      if (wide)
-        tile_epilogue_wide<EPI, MTW, NT>(acc, m0 + my_row0, n0 + wn * 64, lane, bias, residual, ldr, C, ldc, M, N, nullptr,
-                                         reinterpret_cast<unsigned char*>(dsmem) + wave * 8192);
-      else tile_epilogue<EPI, MTW, NT>(acc, m0 + my_row0, n0 + wn * 64, (n0 + wn * 64) / 2, li, g, bias, residual, ldr, C, ldc, M, N, partial, nullptr);
-    }
   };
   using I0 = std::integral_constant<int, 0>;
   using IL = std::integral_constant<int, MTL>;
@@ -1474,6 +1462,7 @@ __global__ __launch_bounds__(512) void gemm_tall_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
     const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
     bf16_t* __restrict__ C, int ldc, int M, int N, int K, const float* __restrict__ wscale) {
+  static_assert(!W8 || SCHED == 1, "fp8 weights: one issue order is built");
   constexpr int BM = 448, BN = 160, BK = 64, WM = 112, MT = 7, NT0 = 6;
   constexpr int A_UNITS = BM * 8;                 // 16-byte units of the A image
   constexpr int B_SUB = (BN / 16) * (W8 ? 1 : 2); // 20 fragment sub-tiles of 1 KB (W8: 10, each a fragment's 64 k)
@@ -1500,12 +1489,14 @@ __global__ __launch_bounds__(512) void gemm_tall_kernel(
   constexpr int NB = W8 ? 2 : 3, WK = W8 ? 512 : 1024;       // pieces of a wave at most; elements of W (2 bytes) from k-tile to k-tile
   const int nb = W8 ? (wave < 2 ? 2 : 1) : (wave < 4 ? 3 : 2);
   const int st0 = W8 ? (wave < 2 ? wave * 2 : wave + 2) : (wave < 4 ? wave * 3 : 12 + (wave - 4) * 2);
-  const bf16_t* bsrc[NB];
+  const bf16_t* bsrc[NB];                        // bf16 weights
+  if constexpr (!W8) {
 #pragma unroll
-  for (int q = 0; q < NB; ++q) {
-    const int st = min(st0 + q, B_SUB - 1);
-    const int fr = min((n0 >> 4) + (W8 ? st : st >> 1), nfrag - 1);
-    bsrc[q] = W8 ? W + (size_t)fr * (K >> 6) * 512 + lane * 8 : W + ((size_t)fr * K32 + (st & 1)) * 512 + lane * 8;
+    for (int q = 0; q < NB; ++q) {
+      const int st = min(st0 + q, B_SUB - 1);
+      const int fr = min((n0 >> 4) + (st >> 1), nfrag - 1);
+      bsrc[q] = W + ((size_t)fr * K32 + (st & 1)) * 512 + lane * 8;
+    }
   }
   // Round 6: activation pieces (8 rows each) that lie entirely beyond the last 16-row MFMA tile are not fetched at all -- at M = 386 the rows
   // 400..447 of the 448-row image (6 of 56 pieces: 11 % of the activation DMA, which is 70 % of this kernel's L2 -> LDS traffic) were copies
@@ -1515,8 +1506,7 @@ __global__ __launch_bounds__(512) void gemm_tall_kernel(
     u32x4* sbase = dsmem + stage * STAGE;
 #pragma unroll
     for (int q = 0; q < A_PER_WAVE; ++q)
-      if ((wave * A_PER_WAVE + q) * 8 < m_rows)
-{
+      if ((wave * A_PER_WAVE + q) * 8 < m_rows) {
         if constexpr (W8) glds16_base(A + kt * BK, (unsigned)aoffs[q] * 2u, lds_addr(sbase + (wave * A_PER_WAVE + q) * 64));
         else glds16((A + aoffs[q] + kt * BK), lds_addr(sbase + (wave * A_PER_WAVE + q) * 64));
       }
@@ -1742,10 +1732,10 @@ static void launch_vh_small(const GemmArgs& a, hipStream_t st) {      // split-K
   const int nkt = a.K / 64, S = a.nsplit;
   constexpr size_t lds = (size_t)3 * (144 * 8 + 2048) * 16 + 1024;      // 3 x 51,200 B + the scratch
   static DeviceOnce attr_set;
-  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_vh_kernel<EPI_PARTIAL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_vh_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   g_launch_counts[LC_GEMM_VH]++;
-  gemm_vh_kernel<EPI_PARTIAL><<<dim3(capped_grid((long)tiles_m * tiles_n), S), dim3(512), lds, st>>>(
-      a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.partial, (nkt + S - 1) / S, raster_for(tiles_m));
+  gemm_vh_kernel<<<dim3(capped_grid((long)tiles_m * tiles_n), S), dim3(512), lds, st>>>(a.A, a.lda, a.W, a.M, a.N, a.K, tiles_m, tiles_n, a.partial, (nkt + S - 1) / S,
+                                                                                        raster_for(tiles_m));
 }
 template <int BM, int EPI>
 static void launch_big(const GemmArgs& a, hipStream_t st) {
