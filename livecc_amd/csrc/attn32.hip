@@ -418,7 +418,7 @@ __global__ __launch_bounds__(NWAVE * 64, 2) void attn_gqa32_kernel(
 // vt = V blocked-transposed [head][32-key block][80][32] (vit_rope_vt_kernel); keys past the segment end are masked, and the K rows of
 // the last (partial) tile are clamped into the segment (the next segment's rows are NOT part of this attention).
 // NWAVE 4: two blocks share a compute unit (67,584 bytes of LDS each), so one's ends hide behind the other, and 880 rows are 7 groups of 128 instead of 4 of 256:
-// 18 slices of 880 113 us against 138, 40 of 400 83 / 92, 8 of 1,456 119 / 122.  NWAVE 8 serves calls under a grid cap (one block a unit).
+// 18 slices of 880 132 us against 151, 40 of 400 87 / 93, 8 of 1,456 132 / 128 (one card, in turn).  NWAVE 8 serves calls under a grid cap (one block a unit).
 template <int NWAVE>
 __global__ __launch_bounds__(NWAVE * 64, 2) void attn_vit32_kernel(
     const bf16_t* __restrict__ qkv, const bf16_t* __restrict__ vt, bf16_t* __restrict__ out, const int32_t* __restrict__ grp_seg,

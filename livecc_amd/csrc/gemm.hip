@@ -593,7 +593,7 @@ __global__ __launch_bounds__(256) void gemm_glds_kernel(
 // What bounds it now: LDS.  A step of the 64-row tile reads 64 KB of fragments and takes 24 KB from the DMA = 704 clocks at 128 B/clk against
 // 256 clocks of MFMA per SIMD; measured 0.33 us a step with 120 blocks, 0.40 with 230.  The 128-row tile reads 96 KB for twice the work.
 // Same summation order as every other tile kernel of this file.  Measured (us, gemm_glds_kernel or the tile chosen before -> here):
-// 1456 x 1280, K 5120 73 -> 31; K 1280 22 -> 12; 720 x 1280, K 5120 72 -> 28; 390 x 3584, K 3584 without a split 23 (128 x 256 tiles: 50);
+// 1456 x 1280, K 5120 73 -> 31 (36 between the other launches of a tower); K 1280 22 -> 12; 720 x 1280, K 5120 72 -> 28; 390 x 3584, K 3584 without a split 23 (128 x 256 tiles: 50);
 // 128-row tile: 1000 x 3584, K 22528 285 -> 196; 2000 x 1280, K 5120 55 -> 41.
 // NST 6 / 4 stages (64- / 128-row tile): one block on a compute unit.  NST 3 (72 KB, two blocks): more than 256 blocks of the 64-row tile
 // (2912 x 1280, K 5120: 57 us, gemm_glds_kernel 77).
