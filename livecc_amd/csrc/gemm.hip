@@ -966,34 +966,56 @@ __global__ __launch_bounds__(512) void gemm_big_kernel(
 }
 
 // ------------------------------------------------------------------------------------------------
-// the same tiles, walked: one block a compute unit goes through its tiles with the DMA ring running on from tile to tile
+// the same tiles, walked: one block a compute unit goes through its tiles with the DMA ring running on from tile to tile, and the two waves of a SIMD
+// take turns at its matrix pipe
 // ------------------------------------------------------------------------------------------------
-// What bounds a short product (the vision tower's K = 1280 is 20 k-steps of 1.3 us) beside the MFMAs and the ring is what lies between two
-// tiles of a compute unit: the last block's stores, a dispatch, addresses, and the first DMA's round trip, with nothing else resident (the
-// ring takes the LDS).  Here the pieces that gemm_big_body issues behind its last k-steps for nobody are the next tile's first ones, the epilogue
-// runs in LDS of its own behind the stages while they land, and its stores drain under the next tile's first step (vmcnt retires in order: the
-// step waits for the pieces and lets the younger stores be, if all of them were issued -- inner tiles).
-// Measured (us, gemm_big_kernel -> here): vision fc1 of 15,840 rows 200 -> 194, fc2 and proj with residual 284 -> 274 together; 4096 x 37888, K 3584
-// with SwiGLU 903 -> 862; 4096 x 18944 fp32, K 3584 473 -> 454.  What is left is the matrix pipe at the clock that the chip holds under it.
+// Turns.  Waves w and w + 4 share a SIMD.  A k-tile of a wave is two phases -- the first half of its row fragments, then the second -- and a phase two slots
+// with a barrier behind each: in the first the wave reads the phase's fragments and issues DMA pieces, in the second it multiplies.  Waves 4..7 are one slot
+// behind, so that one wave of a SIMD multiplies (32 MFMAs back to back at 256 rows, operands all in registers) while the other reads: with both in step
+// (before: reads between the MFMAs of either, one barrier a k-tile) the matrix pipe waited for LDS and barriers a quarter of the time.
+// A row of launches on weights from memory, us, in step -> here: 4096 x 3584, K 18944 460 -> 390; 4096 x 18944, K 3584 460 -> 420; 8192-cube 800 -> 728
+// (1.51 PF; the MFMAs alone, on such data, hold 1.755 GHz = 1.85 PF).  Tried there: s_setprio around the MFMAs 1-4 % slower; the pieces between the MFMAs
+// instead of behind the reads 437 (K 18944); phases by k halves, which balance the reads but free a stage late, 460.
+//
+// Ring.  Stage = [rows][8 x 16 B] activations (XOR-swizzled) + 32 weight sub-tiles.  What phase 0 reads (first halves of the rows, all weights) is filled
+// again in the next phase 1, what phase 1 reads (second halves) in the next phase 0: two slots later, when either wave's reads are back.  Pieces leave in the order
+// in which they are needed, so "all but the last (NSTAGE - 1) k-tiles' worth have landed" is the wait of every phase.  They run on into the
+// next tile, whose first stages land while this one's results leave through LDS of their own; stores drain under the next tile's first phases (vmcnt retires
+// in order: a wait counts the pieces and lets the younger stores be, if all of them were issued -- inner tiles).
+// The first wave of a SIMD stores its results while the second is still multiplying, and the second in the slot in which the first begins the next tile.
+//
+// Rows: 256, 192, 160 or 128 (BM), or VARIABLE (BM 272): 16, 17 or 18 row fragments a tile.  M is whatever the turn packs: 8 co-scheduled streaming chunks are 8 x 386 =
+// 3088 rows = 12 x 256 + 16, so a 13th row tile of 256 would multiply 16 live rows and 13 x 148 = 1924 blocks be 7.5 rounds of the 256 CUs.  The F = ceil(M / 16)
+// fragments are dealt out over floor(F / 16) tiles, the first F % tiles of them one fragment taller (3088 rows: 11 tiles of 256 + one of 272 = 6.94 rounds; 1131
+// rows: 4 tiles of 288 / 272; 9048: 35 tiles instead of 36); the two wave rows split f fragments f / 2 : f - f / 2, one copy of the k loop per count.
+// A slot without rows (192, 160 and variable rows) copies one 16-byte piece into a scratch: the stream of pieces is the same in every wave.
 // Bits as gemm_big_kernel (same k order per output).  bf16 weights; every epilogue but the vision q|k|v ones, whose rotation tables need
 // the stages.  Grid: at most 256 blocks over all splits (one a compute unit), or the cap.
-constexpr int walk_stages(int bm) { return bm >= 192 ? 2 : 3; }
-constexpr bool walk_epilogue_own(int bm) { return bm != 160; }                   // three stages of 160 rows leave no room
-constexpr int walk_epilogue_rows(int bm, int epi) { return bm >= 160 && epi != EPI_GELU_ERF ? 2 : 1; }      // (the erf: registers)
-constexpr size_t walk_lds(int bm, int epi) { return (size_t)walk_stages(bm) * (bm * 8 + 2048) * 16 + (walk_epilogue_own(bm) ? 8 * walk_epilogue_rows(bm, epi) * 2048 : 0); }
 template <int BM, int EPI>
-__global__ __launch_bounds__(512) void gemm_walk_kernel(
+struct Walk {
+  static constexpr bool VH = BM == 272;
+  static constexpr int ROWS = VH ? 288 : BM, MT = VH ? 8 : BM / 32, MTX = VH ? 9 : MT;             // row fragments of a wave (variable rows: 8 or 9)
+  static constexpr int H0 = VH ? 4 : (MT + 1) / 2, H1 = MTX - H0;                                  // of phase 0, at most of phase 1
+  static constexpr int P0 = (4 * H0 + 7) / 8, P1 = (4 * H1 + 7) / 8, PB = 4, G = P0 + PB + P1;     // a wave's pieces of a k-tile: rows of phase 0, weights; rows of phase 1
+  static constexpr bool SPARE = VH || (4 * H0) % 8 != 0 || (4 * H1) % 8 != 0;                      // slots without rows
+  static constexpr int NSTAGE = BM == 128 ? 3 : 2;
+  static constexpr int A_UNITS = ROWS * 8, STAGE = A_UNITS + 2048;                                 // 16-byte units
+  static constexpr int EGR = BM >= 160 && !VH && EPI != EPI_GELU_ERF ? 2 : 1;                      // row tiles of an epilogue group: 2 KB of LDS a wave each (the erf: registers)
+  static constexpr unsigned SCRATCH = (unsigned)NSTAGE * STAGE * 16u, EPILOGUE = SCRATCH + (SPARE ? 1024u : 0u);
+  static constexpr size_t LDS = EPILOGUE + 8 * EGR * 2048;
+  static constexpr int LATER = G * (NSTAGE - 1);                                                   // pieces that may be on their way behind those that are read next
+  static constexpr int NSTORE = EPI == EPI_PARTIAL ? MT * 4 : MT * 2;                              // stores of a wave in the epilogue of an inner tile
+  static_assert(LDS <= 163840, "LDS of a compute unit");
+  static_assert(LATER + NSTORE <= 63, "vmcnt");
+};
+template <int BM, int EPI>
+LCC_DEVICE void gemm_walk_body(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
     const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
     bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n,
     float* __restrict__ partial, int kt_per_split, int raster) {
-  constexpr int BN = 256, BK = 64, NSTAGE = walk_stages(BM);
-  constexpr int WM = BM / 2, MT = WM / 16, NT = 4;
-  constexpr int A_UNITS = BM * 8, STAGE = A_UNITS + 2048;        // 16-byte units: activations, then 32 weight sub-tiles
-  constexpr int APW = (BM + 63) / 64, BPW = 4, G = APW + BPW;    // DMA pieces of a wave per k-tile (surplus ones copy the last rows again)
-  constexpr int EGR = walk_epilogue_rows(BM, EPI);               // row tiles of an epilogue group: 4 / 2 KB of LDS a wave
-  constexpr bool OWN = walk_epilogue_own(BM);                    // ... behind the stages, or the stage that was multiplied last, behind a barrier
-  constexpr int NSTORE = EPI == EPI_PARTIAL ? MT * 4 : MT * 2;   // stores of a wave in the epilogue of an inner tile
+  using S = Walk<BM, EPI>;
+  constexpr int BN = 256, BK = 64, NT = 4, NSTAGE = S::NSTAGE, STAGE = S::STAGE, H0 = S::H0, P0 = S::P0, P1 = S::P1, PB = S::PB, LATER = S::LATER;
   extern __shared__ __attribute__((aligned(16))) u32x4 dsmem[];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1001,11 +1023,12 @@ __global__ __launch_bounds__(512) void gemm_walk_kernel(
   const int li = lane & 15, g = lane >> 4;
   const int K32 = K >> 5, nfrag = N >> 4;
   const int nblk = tiles_m * tiles_n, step = gridDim.x;
+  const int F = (M + 15) >> 4, fbase = S::VH ? F / tiles_m : 0, frem = S::VH ? F - fbase * tiles_m : 0;
   const int nkt_all = K / BK;
   const int kt0 = (EPI == EPI_PARTIAL) ? blockIdx.y * kt_per_split : 0;
   const int nkt = (EPI == EPI_PARTIAL) ? min(nkt_all, kt0 + kt_per_split) : nkt_all;
 
-  auto tile_of = [&](int bid, int& m0, int& n0) {     // tile order: see gemm_big_kernel
+  auto tile_of = [&](int bid, int& m0, int& n0, int& row1, int& rows) {     // tile order: see gemm_big_kernel; row1: the second wave row's first; rows: of the tile
     const int q = nblk >> 3, r = nblk & 7, xcd = bid & 7, idx = bid >> 3;
     bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
     int tn, tm;
@@ -1018,281 +1041,178 @@ __global__ __launch_bounds__(512) void gemm_walk_kernel(
       tn = bid / tiles_m;
       tm = bid - tn * tiles_m;
     }
-    m0 = tm * BM; n0 = tn * BN;
+    const int f = S::VH ? __builtin_amdgcn_readfirstlane(fbase + (tm < frem ? 1 : 0)) : BM / 16;
+    m0 = __builtin_amdgcn_readfirstlane(S::VH ? (tm * fbase + min(tm, frem)) << 4 : tm * BM);
+    n0 = __builtin_amdgcn_readfirstlane(tn * BN);
+    row1 = (f >> 1) * 16;
+    rows = f * 16;
   };
-  // the DMA's tile: the one being multiplied, or the next one already.  Scalar bases, a 32-bit offset per lane and piece inside the tile.
-  unsigned aoffs[APW];
-  const bf16_t *abase, *bbase[BPW / 2];
-  int dvb = blockIdx.x, dkt = kt0;
-  auto point = [&] {
-    int m0, n0;
-    tile_of(dvb, m0, n0);
-    m0 = __builtin_amdgcn_readfirstlane(m0); n0 = __builtin_amdgcn_readfirstlane(n0);
-    abase = A + (size_t)m0 * lda;
+  // The pieces of phase 0 and of phase 1 each go their own way through (tile, k-tile).  Scalar bases, a 32-bit offset per lane and piece inside the tile.
+  // A slot's rows: 8 of the first wave row's part, behind them the second's; none: one 16-byte piece into the scratch
+  struct Way { int vb, kt; const bf16_t* a; };
+  Way w0 = {(int)blockIdx.x, kt0, nullptr}, w1 = w0;
+  const bf16_t* bbase[PB / 2];
+  unsigned off0[P0], off1[P1], dst0[P0], dst1[P1];
+  const unsigned swz = ((lane & 7) ^ (lane >> 3)) << 4, row_bytes = (unsigned)(lda * 2);
+  auto slot_row = [&](int p, int from, int n_first, int n_second, int row1) { return p < n_first ? from + p * 8 : p < n_first + n_second ? row1 + from + (p - n_first) * 8 : -1; };
+  auto slot = [&](int row, int m0, unsigned& off, unsigned& dst) {
+    off = row >= 0 ? (unsigned)min(row + (lane >> 3), M - 1 - m0) * row_bytes + swz : 0u;
+    dst = row >= 0 ? (unsigned)row * 128u : S::SCRATCH;
+  };
+  auto point0 = [&] {
+    int m0, n0, row1, rows;
+    tile_of(w0.vb, m0, n0, row1, rows);
+    w0.a = A + (size_t)m0 * lda;
 #pragma unroll
-    for (int q = 0; q < BPW / 2; ++q) bbase[q] = W + (size_t)min((n0 >> 4) + wave * (BPW / 2) + q, nfrag - 1) * K32 * 512;
+    for (int q = 0; q < PB / 2; ++q) bbase[q] = W + (size_t)min((n0 >> 4) + wave * (PB / 2) + q, nfrag - 1) * K32 * 512;
 #pragma unroll
-    for (int q = 0; q < APW; ++q)
-      aoffs[q] = (unsigned)min(min(wave * APW + q, BM / 8 - 1) * 8 + (lane >> 3), M - 1 - m0) * (unsigned)(lda * 2) + (((lane & 7) ^ (lane >> 3)) << 4);
+    for (int q = 0; q < P0; ++q) slot(slot_row(wave * P0 + q, 0, 2 * H0, 2 * H0, row1), m0, off0[q], dst0[q]);
   };
-  auto piece = [&](int t, unsigned base) {            // base: LDS byte address of the stage
-    if (t < APW) glds16_base(abase + dkt * BK, aoffs[t < APW ? t : 0], base + min(wave * APW + t, BM / 8 - 1) * 1024u);
-    else glds16_base(bbase[t >= APW ? (t - APW) >> 1 : 0] + (size_t)dkt * 1024 + ((t - APW) & 1) * 512, lane * 16u, base + (A_UNITS + (wave * BPW + (t - APW)) * 64) * 16u);
-  };
-  auto advance = [&] {                                // behind the last tile: the last k-tile again, into a stage that nobody reads any more
-    if (++dkt < nkt) return;
-    if (dvb + step < nblk) { dvb += step; dkt = kt0; point(); }
-    else dkt = nkt - 1;
+  auto point1 = [&] {
+    int m0, n0, row1, rows;
+    tile_of(w1.vb, m0, n0, row1, rows);
+    w1.a = A + (size_t)m0 * lda;
+#pragma unroll
+    for (int q = 0; q < P1; ++q) slot(slot_row(wave * P1 + q, H0 * 16, (row1 >> 3) - 2 * H0, ((rows - row1) >> 3) - 2 * H0, row1), m0, off1[q], dst1[q]);
   };
   const unsigned lds0 = lds_addr(dsmem);
-  static_assert(NSTAGE * STAGE * 16 + (OWN ? 8 * EGR * 2048 : 0) <= 163840, "LDS of a compute unit");
-
-  point();
+  auto to = [&](unsigned stage, unsigned dst) { return lds0 + (S::SPARE && dst == S::SCRATCH ? dst : stage + dst); };
+  auto advance = [&](Way& w, auto&& point) {
+    if (++w.kt < nkt) return;
+    if (w.vb + step < nblk) { w.vb += step; w.kt = kt0; point(); }
+    else w.kt = nkt - 1;          // behind the last tile: copies that nobody reads
+  };
+  auto issue0 = [&](unsigned stage) {                 // stage: its byte offset
+#pragma unroll
+    for (int q = 0; q < P0; ++q) glds16_base(w0.a + (size_t)w0.kt * BK, off0[q], to(stage, dst0[q]));
+#pragma unroll
+    for (int q = 0; q < PB; ++q) glds16_base(bbase[q >> 1] + (size_t)w0.kt * 1024 + (q & 1) * 512, lane * 16u, lds0 + stage + (S::A_UNITS + (wave * PB + q) * 64) * 16u);
+    advance(w0, point0);
+  };
+  auto issue1 = [&](unsigned stage) {
+#pragma unroll
+    for (int q = 0; q < P1; ++q) glds16_base(w1.a + (size_t)w1.kt * BK, off1[q], to(stage, dst1[q]));
+    advance(w1, point1);
+  };
+  point0();
+  point1();
   if (kt0 < nkt) {
 #pragma unroll
-    for (int p = 0; p < NSTAGE - 1; ++p) {
-#pragma unroll
-      for (int t = 0; t < G; ++t) piece(t, lds0 + (unsigned)(p * STAGE) * 16u);
-      advance();
+    for (int p = 0; p < NSTAGE; ++p) {
+      issue0((unsigned)(p * STAGE) * 16u);
+      if (p + 1 < NSTAGE) issue1((unsigned)(p * STAGE) * 16u);
     }
   }
-  int aoff[2];
-#pragma unroll
-  for (int kk = 0; kk < 2; ++kk) aoff[kk] = (wm * WM + li) * 8 + ((kk * 4 + g) ^ (li & 7));
-  const int boff = A_UNITS + (wn * NT * 2) * 64 + lane;
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LATER) : "memory");
+  __builtin_amdgcn_s_barrier();
+  if (wm) __builtin_amdgcn_s_barrier();               // the second wave of a SIMD: one slot behind
+  const int boff = S::A_UNITS + (wn * NT * 2) * 64 + lane;
   int st = 0;                      // stage of the k-tile that is multiplied
   bool all_stored = false;         // the last epilogue issued NSTORE stores in this wave
-  for (int vb = blockIdx.x; vb < nblk; vb += step) {
-    int m0, n0;
-    tile_of(vb, m0, n0);
-    const bool wave_has_rows = m0 + wm * WM < M;
-    f32x4 acc[MT][NT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-    for (int kt = kt0; kt < nkt; ++kt) {
-      // this wave's pieces of tile kt have landed; younger: the pieces of NSTAGE - 2 tiles, and behind a tile's end its stores
-      if (all_stored && kt - kt0 < NSTAGE - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G * (NSTAGE - 2) + NSTORE) : "memory");
-      else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G * (NSTAGE - 2)) : "memory");
-      __builtin_amdgcn_s_barrier();   // tile kt complete in LDS; every wave is done reading the stage that is filled now
-      const u32x4* s = dsmem + st * STAGE;
-      const unsigned dma_base = lds0 + (unsigned)((st == 0 ? NSTAGE - 1 : st - 1) * STAGE) * 16u;
-      st = st == NSTAGE - 1 ? 0 : st + 1;
-      if (!wave_has_rows) {           // ragged last row tile: feed the ring only
-#pragma unroll
-        for (int t = 0; t < G; ++t) piece(t, dma_base);
-      } else {                        // fragment reads ahead of the MFMAs, a piece between two row tiles: gemm_big_body's order
-        bf16x8 fb[2][NT], fa[3];
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-          for (int j = 0; j < NT; ++j) fb[kk][j] = as_bf16x8(s[boff + (j * 2 + kk) * 64]);
-        fa[0] = as_bf16x8(s[aoff[0]]);
-        fa[1] = as_bf16x8(s[aoff[0] + 128]);
-#pragma unroll
-        for (int t = 0; t < 2 * MT; ++t) {
-          if (t + 2 < 2 * MT) fa[(t + 2) % 3] = as_bf16x8(s[aoff[(t + 2) / MT] + ((t + 2) % MT) * 128]);
-#pragma unroll
-          for (int j = 0; j < NT; ++j) acc[t % MT][j] = mfma16(fb[t / MT][j], fa[t % 3], acc[t % MT][j]);
-          if (t < G) piece(t, dma_base);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x100, 2 * NT + 2, 0);
-#pragma unroll
-        for (int t = 0; t < 2 * MT; ++t) {
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x008, NT, 0);
-          if (t < G) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
-        }
-      }
-      advance();
-    }
-    if (!OWN) __builtin_amdgcn_s_barrier();          // every wave is done with that stage; the ring fills it behind its next barrier
-    unsigned char* const elds = reinterpret_cast<unsigned char*>(dsmem + (OWN ? NSTAGE : st == 0 ? NSTAGE - 1 : st - 1) * STAGE) + wave * (EGR * 2048);
-    int l = lane;          // opaque: the epilogue's addresses are formed here and not kept in registers through the k-loop
-    asm volatile("" : "+v"(l));
-    if constexpr (EPI == EPI_PARTIAL) {
-      tile_slab_wide<MT, NT, 1, EGR * 2>(acc, m0 + wm * WM, n0 + wn * 64, l, M, N, partial, nullptr, elds);
-    } else if (wide_rows<EPI>(C, ldc, bias, residual, ldr)) {
-      tile_epilogue_wide<EPI, MT, NT, EGR>(acc, m0 + wm * WM, n0 + wn * 64, l, bias, residual, ldr, C, ldc, M, N, nullptr, elds);
-    } else tile_epilogue<EPI, MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, (n0 + wn * 64) / 2, l & 15, l >> 4, bias, residual, ldr, C, ldc, M, N, partial, nullptr);
-    all_stored = m0 + BM <= M && n0 + BN <= N;
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the copies behind the last tile: this block's LDS until they have landed
-}
-
-// ------------------------------------------------------------------------------------------------
-// tiled GEMM v6: the pipeline of gemm_big_kernel<256> over row tiles of VARIABLE height (16, 17 or 18 row fragments = 256 /
-// 272 / 288 rows x 256 columns)
-// ------------------------------------------------------------------------------------------------
-// Why.  M is whatever the turn packs: 8 co-scheduled streaming chunks are 8 x 386 = 3088 rows = 12 x 256 + 16, so the 13th row tile of
-// gemm_big_kernel<256> multiplies 16 live rows (and moves a whole W panel for them), and 13 x 148 = 1924 blocks are 7.5 rounds of the
-// 256 CUs: the gate/up GEMM pays 8 rounds for 7.0 rounds of work (1.01 PF algorithmic against 1.18 PF inside full tiles).  Here the
-// F = ceil(M / 16) row fragments are dealt out over floor(F / 16) row tiles, the first F % tiles of them one fragment taller: no ragged
-// last tile wherever the leftover is at most two fragments per tile (3088 rows: 11 tiles of 256 + one of 272 -> 12 x 148 = 1776 blocks
-// = 6.94 rounds; the first turn's 1131 rows: 4 tiles of 288 / 272 instead of 5; 9048 rows: 35 tiles instead of 36).
-//   * waves: 2 (M) x 4 (N) as gemm_big_kernel; the M-wave pair splits the f fragments f/2 : f - f/2, i.e. a wave multiplies 8 or 9 row
-//     fragments x 4 column fragments -- one copy of the k loop per count (the accumulator array must have a compile-time shape), same
-//     barrier sequence in both.  Waves w and w + 4 share a SIMD, so a SIMD issues 4 f MFMAs per 32-k step: a 272-row tile costs 17/16 of
-//     a 256-row tile, not two tiles.
-//   * LDS image of a stage: [288 rows][8 x 16 B] activations (XOR-swizzled chunks, as gemm_big_kernel) + 32 W fragment sub-tiles = 69,632
-//     B, two stages + a 1-KB scratch.  DMA pieces per wave and k-tile: 4 activation pieces (rows 0-255), ONE more for waves 0-3 when the
-//     tile has the rows 256 + 8 w .. (else the slot copies one 16-byte piece into the scratch: uniform instruction stream), 4 W sub-tiles,
-//     spread one per row-tile step behind the barrier (gemm_big_kernel's SCHED 6).
-// Accumulation order per output element = gemm_big_kernel's (k-step 0, then 1, tile after tile): bit-identical outputs.
-// Requires packed bf16 W, K % 64 == 0, F >= 16, F <= 18 * floor(F / 16).
-// The small class (gemm_vh_kernel): the same pipeline over row tiles of 8 or 9 fragments (128 / 144 rows) for the split-K projections of ONE streaming
-// chunk (M = 386 = 25 fragments: 3 row tiles of 9 + 8 + 8 instead of gemm_big_kernel<128>'s 4, whose fourth holds 2 rows): an M-wave
-// multiplies 4 or 5 row fragments, 2 activation pieces per wave + the extra slot (rows 128-143, waves 0-1), a ring of THREE 51,200-B stages
-// (one more tile in flight: at 32-40 MFMAs per wave and k-tile a single stage of look-ahead left the DMA round trip exposed: 104 vs 72 us).
-// One kernel for the big class, walked (gemm_walk_kernel: the ring runs on from tile to tile, the epilogue has LDS of its own), one tile a block for
-// the small one (its three stages leave no room for an epilogue, and its launches are one round).
-template <int EPI>
-__global__ __launch_bounds__(512) void gemm_walk_vh_kernel(
-    const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
-    const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
-    bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n,
-    float* __restrict__ partial, int kt_per_split, int raster) {
-  constexpr int BN = 256, BK = 64, NT = 4, MTX = 9, MTL = 8;     // row fragments of an M-wave: MTL or MTX
-  constexpr int APW = 4, NSLOT = APW + 5, AROWS = 288;           // 8-row activation pieces per wave below row 256, the slot above, weights
-  constexpr int A_UNITS = AROWS * 8, STAGE = A_UNITS + 2048;     // 69,632 B
-  constexpr unsigned SCRATCH = 2u * STAGE * 16u;                 // 1 KB: where a slot without rows lands
-  constexpr int NSTORE = EPI == EPI_PARTIAL ? MTL * 4 : MTL * 2;
-  static_assert(SCRATCH + 1024 + 8 * 2048 <= 163840, "LDS of a compute unit");
-  extern __shared__ __attribute__((aligned(16))) u32x4 dsmem[];
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 2, wn = wave & 3;
-  const int li = lane & 15, g = lane >> 4;
-  const int K32 = K >> 5, nfrag = N >> 4;
-  const int nblk = tiles_m * tiles_n, step = gridDim.x;
-  const int F = (M + 15) >> 4, fbase = F / tiles_m, frem = F - fbase * tiles_m;
-  const int nkt_all = K / BK;
-  const int kt0 = (EPI == EPI_PARTIAL) ? blockIdx.y * kt_per_split : 0;
-  const int nkt = (EPI == EPI_PARTIAL) ? min(nkt_all, kt0 + kt_per_split) : nkt_all;
-
-  auto tile_of = [&](int bid, int& m0, int& n0, int& f) {     // tile order: see gemm_big_kernel; f: row fragments, 16..18
-    const int q = nblk >> 3, r = nblk & 7, xcd = bid & 7, idx = bid >> 3;
-    bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
-    int tn, tm;
-    if (raster > 0) {
-      const int band = bid / (raster * tiles_m), rem = bid - band * raster * tiles_m;
-      const int bw = min(raster, tiles_n - band * raster);
-      tm = rem / bw;
-      tn = band * raster + (rem - tm * bw);
-    } else {
-      tn = bid / tiles_m;
-      tm = bid - tn * tiles_m;
-    }
-    f = __builtin_amdgcn_readfirstlane(fbase + (tm < frem ? 1 : 0));
-    m0 = __builtin_amdgcn_readfirstlane((tm * fbase + min(tm, frem)) << 4);
-    n0 = __builtin_amdgcn_readfirstlane(tn * BN);
-  };
-  unsigned aoffs[APW + 1], xdst;                              // as gemm_walk_kernel; xdst: where the slot above row 256 goes
-  const bf16_t *abase, *bbase[2];
-  int dvb = blockIdx.x, dkt = kt0;
-  auto point = [&] {
-    int m0, n0, f;
-    tile_of(dvb, m0, n0, f);
-    abase = A + (size_t)m0 * lda;
-#pragma unroll
-    for (int q = 0; q < 2; ++q) bbase[q] = W + (size_t)min((n0 >> 4) + wave * 2 + q, nfrag - 1) * K32 * 512;
-    const unsigned swz = ((lane & 7) ^ (lane >> 3)) << 4, row_bytes = (unsigned)(lda * 2);
-#pragma unroll
-    for (int q = 0; q < APW; ++q) aoffs[q] = (unsigned)min((wave * APW + q) * 8 + (lane >> 3), M - 1 - m0) * row_bytes + swz;
-    const bool have = wave < 4 && 256 + wave * 8 < f * 16;
-    aoffs[APW] = have ? (unsigned)min(256 + wave * 8 + (lane >> 3), M - 1 - m0) * row_bytes + swz : 0u;
-    xdst = have ? (unsigned)(32 + wave) * 1024u : SCRATCH;
-  };
-  const unsigned lds0 = lds_addr(dsmem);
-  auto piece = [&](int t, unsigned stage) {                   // stage: byte offset
-    if (t < APW) glds16_base(abase + dkt * BK, aoffs[t < APW ? t : 0], lds0 + stage + (wave * APW + t) * 1024u);
-    else if (t == APW) glds16_base(abase + dkt * BK, aoffs[APW], lds0 + (xdst == SCRATCH ? SCRATCH : stage + xdst));
-    else glds16_base(bbase[t > APW ? (t - APW - 1) >> 1 : 0] + (size_t)dkt * 1024 + ((t - APW - 1) & 1) * 512, lane * 16u, lds0 + stage + (A_UNITS + (wave * 4 + (t - APW - 1)) * 64) * 16u);
-  };
-  auto advance = [&] {
-    if (++dkt < nkt) return;
-    if (dvb + step < nblk) { dvb += step; dkt = kt0; point(); }
-    else dkt = nkt - 1;
-  };
-  unsigned char* const elds = reinterpret_cast<unsigned char*>(dsmem) + SCRATCH + 1024 + wave * 2048;
-
-  point();
-  if (kt0 < nkt) {
-#pragma unroll
-    for (int t = 0; t < NSLOT; ++t) piece(t, 0u);
-    advance();
-  }
-  const int boff = A_UNITS + (wn * NT * 2) * 64 + lane;
-  int st = 0;
-  bool all_stored = false;
   auto run = [&](auto mt_c, int m0, int n0, int my_row0) {      // one tile
-    constexpr int MTW = decltype(mt_c)::value;
+    constexpr int MTW = decltype(mt_c)::value, MA = MTW > 0 ? MTW : 1, R0 = MTW > 0 ? H0 : 0, R1 = MTW - R0, RF = R0 > R1 ? R0 : R1;
     int aoff[2];
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) aoff[kk] = (my_row0 + li) * 8 + ((kk * 4 + g) ^ (li & 7));
-    f32x4 acc[MTW > 0 ? MTW : 1][NT];
+    f32x4 acc[MA][NT];
 #pragma unroll
-    for (int i = 0; i < (MTW > 0 ? MTW : 1); ++i)
+    for (int i = 0; i < MA; ++i)
 #pragma unroll
       for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    for (int kt = kt0; kt < nkt; ++kt) {
-      if (all_stored && kt == kt0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NSTORE) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();   // tile kt complete in LDS; every wave is done reading the other stage
-      const u32x4* s = dsmem + st * STAGE;
-      st ^= 1;
-      const unsigned dma = (unsigned)(st * STAGE) * 16u;
-      if constexpr (MTW == 0) {
+    bf16x8 fa[2][RF > 0 ? RF : 1], fb[2][NT];
+    auto slot_end = [] {
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto landed = [&](int kt) {     // what the next phase reads has landed and this one's fragments are in registers
+      if (all_stored && kt - kt0 < NSTAGE - 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LATER + S::NSTORE) : "memory");
+      else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LATER) : "memory");
+    };
+    auto multiply = [&](auto from_c, auto n_c) {
+      constexpr int from = decltype(from_c)::value, n = decltype(n_c)::value;
 #pragma unroll
-        for (int t = 0; t < NSLOT; ++t) piece(t, dma);
-      } else {
-        bf16x8 fb[2][NT], fa[3];
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int i = 0; i < n; ++i)
+#pragma unroll
+          for (int j = 0; j < NT; ++j) acc[from + i][j] = mfma16(fb[kk][j], fa[kk][i], acc[from + i][j]);
+    };
+    for (int kt = kt0; kt < nkt; ++kt) {
+      const u32x4* s = dsmem + st * STAGE;
+      const unsigned cur = (unsigned)(st * STAGE) * 16u, before = (unsigned)((st == 0 ? NSTAGE - 1 : st - 1) * STAGE) * 16u;
+      st = st == NSTAGE - 1 ? 0 : st + 1;
+      if constexpr (MTW > 0) {
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+          for (int j = 0; j < NT; ++j) fb[kk][j] = as_bf16x8(s[boff + (j * 2 + kk) * 64]);
+#pragma unroll
+          for (int i = 0; i < R0; ++i) fa[kk][i] = as_bf16x8(s[aoff[kk] + i * 128]);
+        }
+      }
+      issue1(before);
+      landed(kt);
+      slot_end();
+      if constexpr (MTW > 0) multiply(std::integral_constant<int, 0>{}, std::integral_constant<int, R0>{});
+      slot_end();
+      if constexpr (MTW > 0) {
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-          for (int j = 0; j < NT; ++j) fb[kk][j] = as_bf16x8(s[boff + (j * 2 + kk) * 64]);
-        fa[0] = as_bf16x8(s[aoff[0]]);
-        fa[1] = as_bf16x8(s[aoff[0] + 128]);
-#pragma unroll
-        for (int t = 0; t < 2 * MTW; ++t) {
-          if (t + 2 < 2 * MTW) fa[(t + 2) % 3] = as_bf16x8(s[aoff[(t + 2) / MTW] + ((t + 2) % MTW) * 128]);
-#pragma unroll
-          for (int j = 0; j < NT; ++j) acc[t % MTW][j] = mfma16(fb[t / MTW][j], fa[t % 3], acc[t % MTW][j]);
-          if (t < NSLOT) piece(t, dma);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x100, 2 * NT + 2, 0);
-#pragma unroll
-        for (int t = 0; t < 2 * MTW; ++t) {
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x008, NT, 0);
-        }
+          for (int i = 0; i < R1; ++i) fa[kk][i] = as_bf16x8(s[aoff[kk] + (R0 + i) * 128]);
       }
-      advance();
+      issue0(cur);
+      landed(kt);
+      slot_end();
+      if constexpr (MTW > 0) multiply(std::integral_constant<int, R0>{}, std::integral_constant<int, R1>{});
+      if (kt + 1 < nkt) slot_end();
     }
-    int l = lane;          // opaque: see gemm_walk_kernel
+    if (kt0 < nkt && wm == 0) slot_end();
+    unsigned char* const elds = reinterpret_cast<unsigned char*>(dsmem) + S::EPILOGUE + wave * (S::EGR * 2048);
+    int l = lane;          // opaque: the epilogue's addresses are formed here and not kept in registers through the k-loop
     asm volatile("" : "+v"(l));
     if constexpr (MTW > 0 && EPI == EPI_PARTIAL) {
-      tile_slab_wide<MTW, NT, 1, 2>(acc, m0 + my_row0, n0 + wn * 64, l, M, N, partial, nullptr, elds);
+      tile_slab_wide<MTW, NT, 1, S::EGR * 2>(acc, m0 + my_row0, n0 + wn * 64, l, M, N, partial, nullptr, elds);
     } else if constexpr (MTW > 0) {
       if (wide_rows<EPI>(C, ldc, bias, residual, ldr))
-        tile_epilogue_wide<EPI, MTW, NT, 1>(acc, m0 + my_row0, n0 + wn * 64, l, bias, residual, ldr, C, ldc, M, N, nullptr, elds);
+        tile_epilogue_wide<EPI, MTW, NT, S::EGR>(acc, m0 + my_row0, n0 + wn * 64, l, bias, residual, ldr, C, ldc, M, N, nullptr, elds);
       else tile_epilogue<EPI, MTW, NT>(acc, m0 + my_row0, n0 + wn * 64, (n0 + wn * 64) / 2, l & 15, l >> 4, bias, residual, ldr, C, ldc, M, N, partial, nullptr);
     }
+    if (kt0 < nkt && wm == 1) slot_end();
   };
   for (int vb = blockIdx.x; vb < nblk; vb += step) {
-    int m0, n0, f;
-    tile_of(vb, m0, n0, f);
-    const int f0 = f >> 1, my_mt = wm ? f - f0 : f0, my_row0 = wm ? f0 * 16 : 0;      // M-wave 0: f0 fragments, M-wave 1: the rest
-    if (m0 + my_row0 >= M) run(std::integral_constant<int, 0>{}, m0, n0, my_row0);
-    else if (my_mt == MTX) run(std::integral_constant<int, MTX>{}, m0, n0, my_row0);
-    else run(std::integral_constant<int, MTL>{}, m0, n0, my_row0);
-    all_stored = m0 + f * 16 <= M && n0 + BN <= N;
+    int m0, n0, row1, rows;
+    tile_of(vb, m0, n0, row1, rows);
+    const int my_row0 = wm ? row1 : 0;
+    if (m0 + my_row0 >= M) run(std::integral_constant<int, 0>{}, m0, n0, my_row0);          // ragged last row tile: feed the ring only
+    else if (S::VH && (wm ? rows - row1 : row1) == S::MTX * 16) run(std::integral_constant<int, S::MTX>{}, m0, n0, my_row0);
+    else run(std::integral_constant<int, S::MT>{}, m0, n0, my_row0);
+    all_stored = m0 + rows <= M && n0 + BN <= N;
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the copies behind the last tile
+  if (!wm) __builtin_amdgcn_s_barrier();
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the copies behind the last tile: this block's LDS until they have landed
+}
+template <int BM, int EPI>
+__global__ __launch_bounds__(512) void gemm_walk_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias,
+                                                        const bf16_t* __restrict__ residual, int ldr, bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m,
+                                                        int tiles_n, float* __restrict__ partial, int kt_per_split, int raster) {
+  gemm_walk_body<BM, EPI>(A, lda, W, bias, residual, ldr, C, ldc, M, N, K, tiles_m, tiles_n, partial, kt_per_split, raster);
+}
+template <int EPI>          // variable rows
+__global__ __launch_bounds__(512) void gemm_walk_vh_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias,
+                                                           const bf16_t* __restrict__ residual, int ldr, bf16_t* __restrict__ C, int ldc, int M, int N, int K,
+                                                           int tiles_m, int tiles_n, float* __restrict__ partial, int kt_per_split, int raster) {
+  gemm_walk_body<272, EPI>(A, lda, W, bias, residual, ldr, C, ldc, M, N, K, tiles_m, tiles_n, partial, kt_per_split, raster);
 }
 
+// ------------------------------------------------------------------------------------------------
+// row tiles of 8 or 9 fragments (128 / 144 rows) for the split-K projections of ONE streaming chunk
+// ------------------------------------------------------------------------------------------------
+// M = 386 = 25 fragments: 3 row tiles of 9 + 8 + 8 instead of gemm_big_kernel<128>'s 4, whose fourth holds 2 rows.  A wave multiplies 4 or 5 row fragments x 4
+// column fragments, 2 activation pieces per wave + an extra slot (rows 128-143, waves 0-1), a ring of THREE 51,200-B stages (one more tile in flight: at
+// 32-40 MFMAs per wave and k-tile a single stage of look-ahead left the DMA round trip exposed: 104 vs 72 us).  One tile a block: its launches are one round.
+// Accumulation order per output element = gemm_big_kernel's.  Requires packed bf16 W, K % 64 == 0, F >= 8, F <= 9 * floor(F / 8).
 __global__ __launch_bounds__(512) void gemm_vh_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, int M, int N, int K, int tiles_m,
                                                       int tiles_n, float* __restrict__ partial, int kt_per_split, int raster) {
   constexpr int BN = 256, BK = 64, NT = 4;
@@ -1703,7 +1623,7 @@ template <int BM, int EPI>
 static void launch_walk(const GemmArgs& a, hipStream_t st) {
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + 255) / 256;
   const int nkt = a.K / 64, S = (EPI == EPI_PARTIAL) ? a.nsplit : 1;
-  constexpr size_t lds = walk_lds(BM, EPI);      // 256 / 192 / 160 / 128 rows: 160 / 144 / 156 / 160 KB
+  constexpr size_t lds = Walk<BM, EPI>::LDS;      // 256 / 192 / 160 / 128 rows: 160 / 145 / 137 / 160 KB
   static DeviceOnce attr_set;   // per instantiation
   if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_walk_kernel<BM, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   const unsigned grid = walk_grid((long)tiles_m * tiles_n, S);
@@ -1719,7 +1639,7 @@ template <int EPI>
 static void launch_vh(const GemmArgs& a, hipStream_t st) {
   const int F = (a.M + 15) >> 4, tiles_m = F >> 4, tiles_n = (a.N + 255) / 256;
   const int nkt = a.K / 64, S = (EPI == EPI_PARTIAL) ? a.nsplit : 1;
-  constexpr size_t lds = (size_t)2 * (288 * 8 + 2048) * 16 + 1024 + 8 * 2048;      // stages, scratch, epilogue: 156,672 B
+  constexpr size_t lds = Walk<272, EPI>::LDS;      // stages, scratch, epilogue: 156,672 B
   static DeviceOnce attr_set;   // per instantiation
   if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_walk_vh_kernel<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   g_launch_counts[LC_GEMM_VH]++;
@@ -1813,7 +1733,7 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr, bool 
   // 1.62 rounds; 99 x 5 of 160 fill 1.93 at 5/6 of the time each: proj 55.7 -> 52.1 us, fc2 201 -> 178.
   // 1000 / 2100 x 17920, K 1536 with SwiGLU 63.6 -> 58.4 / 117.5 -> 111.3.
   const float s160 = (a.w_fp8 || !allow192) ? 0.f : tile_score(a.M, a.N, S, 160, 256, 256, 0.90f, false);
-  const float s128 = tile_score(a.M, a.N, S, 128, 256, 256, 0.85f, true);
+  const float s128 = tile_score(a.M, a.N, S, 128, 256, 256, a.w_fp8 ? 0.85f : 0.82f, true);
   // gemm_mid_kernel: 0.38 / 0.52 us a step of 64 x 128 / 128 x 128 against 0.85 of 128 x 256, one tile a compute unit at a time (two 64-row
   // tiles side by side take twice as long).  Returned as 0 / 129.  The 128-row form wins where its blocks fill one round and the 64-row
   // form's need two; beyond a round the 256-column tiles do (shapes around the lines: 1000 x 3584, K 3584: 43 / 34 / 52 us for 64 x 128 /
@@ -2411,7 +2331,7 @@ int gemm_tiled_num_splits(int M, int N, int K, bool packed_bf16) {
       if (S > 1) { a.partial = &dummy; a.nsplit = S; }          // never dereferenced: the slab form is asked for
       float score = 0.f;
       big_tile_rows(a, S, &score);
-      const float us = 2e-9f * (float)M * (float)N * (float)K / (1.25f * score) + (S > 1 ? (float)S * (float)M * (float)N * 8e-6f / 4.5f : 0.f);
+      const float us = 2e-9f * (float)M * (float)N * (float)K / (1.45f * score) + (S > 1 ? (float)S * (float)M * (float)N * 8e-6f / 4.5f : 0.f);
       if (S == 1 || us < (best == 1 ? 0.9f : 1.f) * best_us) { best = S; best_us = us; }
     }
     return best;
