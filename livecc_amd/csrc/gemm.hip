@@ -5,7 +5,8 @@
 //
 //  * gemm_walk_kernel    : M >= 17, packed W, K % 64 == 0 (LLM prefill, ViT).  MFMA-bound.  8 waves, BM x 256 x 64 tile
 //                          (BM 256 / 192 / 160 / 128), LDS-DMA for both operands; one block a compute unit, the DMA ring runs on from tile to tile.
-//  * gemm_big_kernel     : the same tiles one a block: fp8-e4m3 W converted after the LDS read, and the vision q|k|v epilogues.
+//  * gemm_vit_kernel     : the same pipeline, a tile a block, with the vision q|k|v epilogues.
+//  * gemm_big_kernel     : the same tiles one a block, both waves of a SIMD in step: fp8-e4m3 W converted after the LDS read; 128-row tiles of one round.
 //  * gemm_walk_vh_kernel : the walk over row tiles of 256 / 272 / 288 rows (no ragged last row tile).
 //  * gemm_vh_kernel      : row tiles of 128 / 144 rows, split-K slabs of one streaming chunk.
 //  * gemm_tall_kernel    : one block row covers all of M (256 < M <= 448: one streaming chunk's gate/up).
@@ -264,7 +265,7 @@ LCC_DEVICE void tile_slab_wide(const f32x4 (&acc)[MT][NT], int mbase, int nbase,
 // EPI_VIT_QK / EPI_VIT_V (round 4): the vision tower's q|k|v projection writes what its attention kernels read -- q and k rotated (2-D
 // RoPE, HF modeling_qwen2_vl.py:225-248) at their natural columns of C, V blocked-transposed into vt[head][32-key block][80][32] -- instead
 // of a plain [P, 3E] tensor that vit_rope_vt_kernel re-reads and re-writes (52 us per tower block at 8 streams, 179 MB of traffic).
-// Two launches of gemm_big_kernel over the `qkv_w_rope` copy of the weight (weights.py: vit_qkv_rope_row_permutation):
+// One launch of gemm_vit_kernel (two, q|k and V apart, where a column tile would hold both) over the `qkv_w_rope` copy of the weight (weights.py: vit_qkv_rope_row_permutation):
 //
 //  * q|k (N = 2E, EPI_VIT_QK): inside q and inside k every 32 stored rows are [16 first-half channels | their 16 rotation partners],
 //    first-half channels enumerated head-major (f = head * 40 + c, c < 40), so a lane's accumulators acc[i][j] / acc[i][j + 1] hold
@@ -740,17 +741,15 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(
 // fragment read is one ds_read_b128 per 16 rows whose halves are converted to bf16 in registers, and the activation chunk
 // order follows PACKED8's k assignment (MFMA h of lane group g takes k = g*16 + h*8 ..).  Half the W bytes in L2 and LDS;
 // the stage shrinks to 48 KB (BM 256) so that three stages fit and one tile stays in flight across the barrier.
-// (the kernel proper is gemm_big_kernel below: it maps blockIdx to a tile (tm, tn) and runs this body -- once for every epilogue but
-// EPI_VIT_QKV, whose column tiles take the q|k body or the V body)
+// (the kernel proper is gemm_big_kernel below: it maps blockIdx to a tile (tm, tn) and runs this body)
 template <int BM, int EPI, int SCHED, bool W8>
 LCC_DEVICE void gemm_big_body(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
     const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
     bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tm, int tn,
-    float* __restrict__ partial, int kt_per_split, const float* __restrict__ wscale, const VitQkvEpi& vq) {
+    float* __restrict__ partial, int kt_per_split, const float* __restrict__ wscale) {
   constexpr int BN = 256, BK = 64, NSTAGE = (BM >= 192 && !W8) ? 2 : 3;     // BM 192 (round 4): 56-KB stages, two of them
   constexpr int WM = BM / 2, MT = WM / 16, NT = 4;
-  constexpr bool SWAP = EPI == EPI_VIT_V;         // activations as the MFMA A operand: a lane ends with 4 consecutive rows of one column
   constexpr int A_UNITS = BM * 8;                 // 16-byte units of the A image
   constexpr int B_SUB = (BN / 16) * (W8 ? 1 : 2); // 1-KB fragment sub-tiles of the W tile
   constexpr int STAGE = A_UNITS + B_SUB * 64;     // 16-byte units per stage
@@ -847,7 +846,7 @@ LCC_DEVICE void gemm_big_body(
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-          for (int j = 0; j < NT; ++j) acc[i][j] = SWAP ? mfma16(fa[i], fb[j], acc[i][j]) : mfma16(fb[j], fa[i], acc[i][j]);
+          for (int j = 0; j < NT; ++j) acc[i][j] = mfma16(fb[j], fa[i], acc[i][j]);
       }
     } else {
       // explicit software pipeline of the fragment reads: the 8 W fragments of the k-tile are read up front, the activation
@@ -877,7 +876,7 @@ LCC_DEVICE void gemm_big_body(
       for (int t = 0; t < 2 * MT; ++t) {
         if (t + 2 < 2 * MT) fa[(t + 2) % 3] = as_bf16x8(s[aoff[(t + 2) / MT] + ((t + 2) % MT) * 128]);
 #pragma unroll
-        for (int j = 0; j < NT; ++j) acc[t % MT][j] = SWAP ? mfma16(fa[t % 3], fb[t / MT][j], acc[t % MT][j]) : mfma16(fb[t / MT][j], fa[t % 3], acc[t % MT][j]);
+        for (int j = 0; j < NT; ++j) acc[t % MT][j] = mfma16(fb[t / MT][j], fa[t % 3], acc[t % MT][j]);
         if (SCHED == 6 && t < G) {
           if (t < A_PER_WAVE)
             glds16((asrc[t < A_PER_WAVE ? t : 0] + kt_dma * BK), lds_addr(dma_base + (wave * A_PER_WAVE + t) * 64));
@@ -895,24 +894,7 @@ LCC_DEVICE void gemm_big_body(
     }
   }
   if (SCHED == 6) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the clamped copies of the last iterations
-  if constexpr (EPI == EPI_VIT_QK) {
-    // cos / sin rows of this block -> LDS (the fragment stages are dead): rows m0 .. m0 + BM - 1 of the [P, 40] fp32 tables are one
-    // contiguous piece of BM * 10 16-byte units each; reads past the last row are clamped (those rows are never stored)
-    __builtin_amdgcn_s_barrier();
-    constexpr int UNITS = BM * 10;
-    const long first = (long)m0 * 10, last = (long)M * 10 - 1;
-    for (int t = wave; t * 64 < UNITS; t += 8) {
-      const long u = min(first + t * 64 + lane, last);
-      glds16((vq.cs + u * 4), lds_addr(dsmem + t * 64));
-      glds16((vq.sn + u * 4), lds_addr(dsmem + UNITS + t * 64));
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    const float* lcs = reinterpret_cast<const float*>(dsmem);
-    vit_qk_epilogue<MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, wm * WM, li, g, bias, C, ldc, M, N, vq.E, lcs, lcs + UNITS * 4);
-  } else if constexpr (EPI == EPI_VIT_V) {
-    vit_v_epilogue<MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, li, g, bias, M, N, vq);
-  } else if constexpr (EPI == EPI_PARTIAL) {
+  if constexpr (EPI == EPI_PARTIAL) {
     __builtin_amdgcn_s_barrier();          // every wave is done with the stages, and its DMA pieces have landed
     tile_slab_wide<MT, NT>(acc, m0 + wm * WM, n0 + wn * 64, lane, M, N, partial, wscale, reinterpret_cast<unsigned char*>(dsmem) + wave * 8192);
   } else if (wide_rows<EPI>(C, ldc, bias, residual, ldr)) {
@@ -927,7 +909,7 @@ __global__ __launch_bounds__(512) void gemm_big_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
     const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
     bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n,
-    float* __restrict__ partial, int kt_per_split, const float* __restrict__ wscale, VitQkvEpi vq, int raster) {
+    float* __restrict__ partial, int kt_per_split, const float* __restrict__ wscale, int raster) {
   const int nblk = tiles_m * tiles_n;
   for (int vb = blockIdx.x; vb < nblk; vb += gridDim.x) {     // one tile per block, or a persistent walk under the grid cap
   int bid = vb;
@@ -949,19 +931,8 @@ __global__ __launch_bounds__(512) void gemm_big_kernel(
     tn = bid / tiles_m;
     tm = bid - tn * tiles_m;
   }
-  if constexpr (EPI == EPI_VIT_QKV) {
-    // one launch for q|k|v (N = 3E, 2E % 256 == 0): the column tiles of q and k run the rotation body, those of V the swapped-operand
-    // body on rows 2E.. of the packed weight -- a block-uniform choice made once, outside the k-loop
-    const int qk_tiles = (2 * vq.E) >> 8;
-    if (tn >= qk_tiles)
-      gemm_big_body<BM, EPI_VIT_V, SCHED, W8>(A, lda, W + (size_t)2 * vq.E * K, bias != nullptr ? bias + 2 * vq.E : nullptr, nullptr, 0, nullptr, 0, M,
-                                                  vq.E, K, tm, tn - qk_tiles, nullptr, 0, nullptr, vq);
-    else
-      gemm_big_body<BM, EPI_VIT_QK, SCHED, W8>(A, lda, W, bias, nullptr, 0, C, ldc, M, 2 * vq.E, K, tm, tn, nullptr, 0, nullptr, vq);
-  } else {
-    gemm_big_body<BM, EPI, SCHED, W8>(A, lda, W, bias, residual, ldr, C, ldc, M, N, K, tm, tn, partial, kt_per_split, wscale, vq);
-  }
-  if (vb + (int)gridDim.x < nblk) __syncthreads();     // the next tile's DMA reuses the stages (and the rotation epilogue's tables)
+  gemm_big_body<BM, EPI, SCHED, W8>(A, lda, W, bias, residual, ldr, C, ldc, M, N, K, tm, tn, partial, kt_per_split, wscale);
+  if (vb + (int)gridDim.x < nblk) __syncthreads();     // the next tile's DMA reuses the stages
   }
 }
 
@@ -989,8 +960,8 @@ __global__ __launch_bounds__(512) void gemm_big_kernel(
 // fragments are dealt out over floor(F / 16) tiles, the first F % tiles of them one fragment taller (3088 rows: 11 tiles of 256 + one of 272 = 6.94 rounds; 1131
 // rows: 4 tiles of 288 / 272; 9048: 35 tiles instead of 36); the two wave rows split f fragments f / 2 : f - f / 2, one copy of the k loop per count.
 // A slot without rows (192, 160 and variable rows) copies one 16-byte piece into a scratch: the stream of pieces is the same in every wave.
-// Bits as gemm_big_kernel (same k order per output).  bf16 weights; every epilogue but the vision q|k|v ones, whose rotation tables need
-// the stages.  Grid: at most 256 blocks over all splits (one a compute unit), or the cap.
+// Bits as gemm_big_kernel (same k order per output).  bf16 weights.  The vision q|k|v epilogues (gemm_vit_kernel) run a tile a block: their rotation tables need
+// the stages (15,840 x 3840, K 1280: 182 -> 172 us).  Grid: at most 256 blocks over all splits (one a compute unit), or the cap.
 template <int BM, int EPI>
 struct Walk {
   static constexpr bool VH = BM == 272;
@@ -1013,8 +984,9 @@ LCC_DEVICE void gemm_walk_body(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
     const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
     bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n,
-    float* __restrict__ partial, int kt_per_split, int raster) {
+    float* __restrict__ partial, int kt_per_split, int raster, const VitQkvEpi& vq = VitQkvEpi(), int one_m = 0, int one_n = 0) {
   using S = Walk<BM, EPI>;
+  constexpr bool VIT = EPI == EPI_VIT_QK || EPI == EPI_VIT_V;      // the tile (one_m, one_n) alone: the rotation's tables take the stages
   constexpr int BN = 256, BK = 64, NT = 4, NSTAGE = S::NSTAGE, STAGE = S::STAGE, H0 = S::H0, P0 = S::P0, P1 = S::P1, PB = S::PB, LATER = S::LATER;
   extern __shared__ __attribute__((aligned(16))) u32x4 dsmem[];
 
@@ -1022,7 +994,7 @@ LCC_DEVICE void gemm_walk_body(
   const int wm = wave >> 2, wn = wave & 3;
   const int li = lane & 15, g = lane >> 4;
   const int K32 = K >> 5, nfrag = N >> 4;
-  const int nblk = tiles_m * tiles_n, step = gridDim.x;
+  const int nblk = VIT ? 1 : tiles_m * tiles_n, step = VIT ? 1 : gridDim.x, vb0 = VIT ? 0 : blockIdx.x;
   const int F = (M + 15) >> 4, fbase = S::VH ? F / tiles_m : 0, frem = S::VH ? F - fbase * tiles_m : 0;
   const int nkt_all = K / BK;
   const int kt0 = (EPI == EPI_PARTIAL) ? blockIdx.y * kt_per_split : 0;
@@ -1032,7 +1004,10 @@ LCC_DEVICE void gemm_walk_body(
     const int q = nblk >> 3, r = nblk & 7, xcd = bid & 7, idx = bid >> 3;
     bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
     int tn, tm;
-    if (raster > 0) {
+    if (VIT) {
+      tm = one_m;
+      tn = one_n;
+    } else if (raster > 0) {
       const int band = bid / (raster * tiles_m), rem = bid - band * raster * tiles_m;
       const int bw = min(raster, tiles_n - band * raster);
       tm = rem / bw;
@@ -1050,7 +1025,7 @@ LCC_DEVICE void gemm_walk_body(
   // The pieces of phase 0 and of phase 1 each go their own way through (tile, k-tile).  Scalar bases, a 32-bit offset per lane and piece inside the tile.
   // A slot's rows: 8 of the first wave row's part, behind them the second's; none: one 16-byte piece into the scratch
   struct Way { int vb, kt; const bf16_t* a; };
-  Way w0 = {(int)blockIdx.x, kt0, nullptr}, w1 = w0;
+  Way w0 = {vb0, kt0, nullptr}, w1 = w0;
   const bf16_t* bbase[PB / 2];
   unsigned off0[P0], off1[P1], dst0[P0], dst1[P1];
   const unsigned swz = ((lane & 7) ^ (lane >> 3)) << 4, row_bytes = (unsigned)(lda * 2);
@@ -1136,7 +1111,7 @@ LCC_DEVICE void gemm_walk_body(
 #pragma unroll
         for (int i = 0; i < n; ++i)
 #pragma unroll
-          for (int j = 0; j < NT; ++j) acc[from + i][j] = mfma16(fb[kk][j], fa[kk][i], acc[from + i][j]);
+          for (int j = 0; j < NT; ++j) acc[from + i][j] = EPI == EPI_VIT_V ? mfma16(fa[kk][i], fb[kk][j], acc[from + i][j]) : mfma16(fb[kk][j], fa[kk][i], acc[from + i][j]);
     };
     for (int kt = kt0; kt < nkt; ++kt) {
       const u32x4* s = dsmem + st * STAGE;
@@ -1172,7 +1147,29 @@ LCC_DEVICE void gemm_walk_body(
     unsigned char* const elds = reinterpret_cast<unsigned char*>(dsmem) + S::EPILOGUE + wave * (S::EGR * 2048);
     int l = lane;          // opaque: the epilogue's addresses are formed here and not kept in registers through the k-loop
     asm volatile("" : "+v"(l));
-    if constexpr (MTW > 0 && EPI == EPI_PARTIAL) {
+    if constexpr (VIT) {
+      slot_end();                             // the slot in which the second wave of a SIMD multiplies for the last time
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();          // every wave is done with the stages, and its DMA pieces have landed
+      if constexpr (EPI == EPI_VIT_V) {
+        if constexpr (MTW > 0) vit_v_epilogue<MA, NT>(acc, m0 + my_row0, n0 + wn * 64, li, g, bias, M, N, vq);
+      } else {
+        // cos / sin rows of this tile: rows m0 .. m0 + BM - 1 of the [P, 40] fp32 tables are one contiguous piece of BM * 10 16-byte units each; reads
+        // past the last row are clamped (those rows are never stored)
+        constexpr int UNITS = BM * 10;
+        const long first = (long)m0 * 10, last = (long)M * 10 - 1;
+        for (int t = wave; t * 64 < UNITS; t += 8) {
+          const long u = min(first + t * 64 + lane, last);
+          glds16((vq.cs + u * 4), lds_addr(dsmem + t * 64));
+          glds16((vq.sn + u * 4), lds_addr(dsmem + UNITS + t * 64));
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        const float* lcs = reinterpret_cast<const float*>(dsmem);
+        if constexpr (MTW > 0) vit_qk_epilogue<MA, NT>(acc, m0 + my_row0, n0 + wn * 64, my_row0, li, g, bias, C, ldc, M, N, vq.E, lcs, lcs + UNITS * 4);
+      }
+      return;
+    } else if constexpr (MTW > 0 && EPI == EPI_PARTIAL) {
       tile_slab_wide<MTW, NT, 1, S::EGR * 2>(acc, m0 + my_row0, n0 + wn * 64, l, M, N, partial, nullptr, elds);
     } else if constexpr (MTW > 0) {
       if (wide_rows<EPI>(C, ldc, bias, residual, ldr))
@@ -1181,7 +1178,7 @@ LCC_DEVICE void gemm_walk_body(
     }
     if (kt0 < nkt && wm == 1) slot_end();
   };
-  for (int vb = blockIdx.x; vb < nblk; vb += step) {
+  for (int vb = vb0; vb < nblk; vb += step) {
     int m0, n0, row1, rows;
     tile_of(vb, m0, n0, row1, rows);
     const int my_row0 = wm ? row1 : 0;
@@ -1190,6 +1187,7 @@ LCC_DEVICE void gemm_walk_body(
     else run(std::integral_constant<int, S::MT>{}, m0, n0, my_row0);
     all_stored = m0 + rows <= M && n0 + BN <= N;
   }
+  if constexpr (VIT) return;
   if (!wm) __builtin_amdgcn_s_barrier();
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the copies behind the last tile: this block's LDS until they have landed
 }
@@ -1198,6 +1196,37 @@ __global__ __launch_bounds__(512) void gemm_walk_kernel(const bf16_t* __restrict
                                                         const bf16_t* __restrict__ residual, int ldr, bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m,
                                                         int tiles_n, float* __restrict__ partial, int kt_per_split, int raster) {
   gemm_walk_body<BM, EPI>(A, lda, W, bias, residual, ldr, C, ldc, M, N, K, tiles_m, tiles_n, partial, kt_per_split, raster);
+}
+// the vision tower's q|k|v projection (EPI_VIT_QK, EPI_VIT_V; EPI_VIT_QKV: both, N = 3E and 2E % 256 == 0): a tile a block
+template <int BM, int EPI>
+__global__ __launch_bounds__(512) void gemm_vit_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias,
+                                                       bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n, VitQkvEpi vq, int raster) {
+  const int nblk = tiles_m * tiles_n;
+  for (int vb = blockIdx.x; vb < nblk; vb += gridDim.x) {     // one tile per block, or a persistent walk under the grid cap
+    const int q = nblk >> 3, r = nblk & 7, xcd = vb & 7, bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (vb >> 3);
+    int tn, tm;                                               // tile order: see gemm_big_kernel
+    if (raster > 0) {
+      const int band = bid / (raster * tiles_m), rem = bid - band * raster * tiles_m;
+      const int bw = min(raster, tiles_n - band * raster);
+      tm = rem / bw;
+      tn = band * raster + (rem - tm * bw);
+    } else {
+      tn = bid / tiles_m;
+      tm = bid - tn * tiles_m;
+    }
+    if constexpr (EPI == EPI_VIT_QKV) {
+      // the column tiles of q and k run the rotation body, those of V the swapped-operand body on rows 2E.. of the packed weight
+      const int qk_tiles = (2 * vq.E) >> 8;
+      if (tn >= qk_tiles)
+        gemm_walk_body<BM, EPI_VIT_V>(A, lda, W + (size_t)2 * vq.E * K, bias != nullptr ? bias + 2 * vq.E : nullptr, nullptr, 0, nullptr, 0, M, vq.E, K, 1, 1, nullptr, 0, 0,
+                                      vq, tm, tn - qk_tiles);
+      else
+        gemm_walk_body<BM, EPI_VIT_QK>(A, lda, W, bias, nullptr, 0, C, ldc, M, 2 * vq.E, K, 1, 1, nullptr, 0, 0, vq, tm, tn);
+    } else {
+      gemm_walk_body<BM, EPI>(A, lda, W, bias, nullptr, 0, C, ldc, M, N, K, 1, 1, nullptr, 0, 0, vq, tm, tn);
+    }
+    if (vb + (int)gridDim.x < nblk) __syncthreads();          // the next tile's DMA reuses the stages (and the rotation's tables)
+  }
 }
 template <int EPI>          // variable rows
 __global__ __launch_bounds__(512) void gemm_walk_vh_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias,
@@ -1612,7 +1641,7 @@ static void launch_big_s(const GemmArgs& a, hipStream_t st) {
     (void)hipFuncSetAttribute((const void*)gemm_big_kernel<BM, EPI, SCHED, W8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   }
   gemm_big_kernel<BM, EPI, SCHED, W8><<<dim3(capped_grid((long)tiles_m * tiles_n), S), dim3(512), lds, st>>>(
-      a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.partial, (nkt + S - 1) / S, a.wscale, a.vq,
+      a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.partial, (nkt + S - 1) / S, a.wscale,
       raster_for(tiles_m));
 }
 // the walking kernels' offsets inside a tile are 32-bit (288 activation rows)
@@ -1629,6 +1658,22 @@ static void launch_walk(const GemmArgs& a, hipStream_t st) {
   const unsigned grid = walk_grid((long)tiles_m * tiles_n, S);
   gemm_walk_kernel<BM, EPI><<<dim3(grid, S), dim3(512), lds, st>>>(a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m,
                                                                    tiles_n, a.partial, (nkt + S - 1) / S, raster_for(tiles_m));
+}
+template <int BM, int EPI>
+static void launch_vit_rows(const GemmArgs& a, hipStream_t st) {
+  const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + 255) / 256;
+  constexpr size_t lds = Walk<BM, EPI == EPI_VIT_QKV ? EPI_VIT_QK : EPI>::LDS;
+  static_assert(BM * 320 <= Walk<BM, EPI_VIT_QK>::SCRATCH, "the rotation's tables in the stages");
+  static DeviceOnce attr_set;   // per instantiation
+  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_vit_kernel<BM, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  gemm_vit_kernel<BM, EPI><<<dim3(capped_grid((long)tiles_m * tiles_n)), dim3(512), lds, st>>>(a.A, a.lda, a.W, a.bias, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.vq,
+                                                                                              raster_for(tiles_m));
+}
+template <int EPI>
+static void launch_vit(const GemmArgs& a, int rows, hipStream_t st) {
+  if (rows == 256) launch_vit_rows<256, EPI>(a, st);
+  else if (rows == 192) launch_vit_rows<192, EPI>(a, st);
+  else launch_vit_rows<128, EPI>(a, st);
 }
 // variable-height row tiles (gemm_vh_kernel): tiles_m = floor(F / 16) row tiles for F = ceil(M / 16) row fragments (small class: F / 8)
 static bool vh_legal(const GemmArgs& a, bool small = false) {
@@ -2413,23 +2458,14 @@ int gemm_bf16(const GemmArgs& a, hipStream_t st) {
     if (v && (q.grp_off == nullptr || q.vt == nullptr || q.total_blocks <= 0)) return LCC_ERR_ARG;
     if (qk && (((uintptr_t)q.cs | (uintptr_t)q.sn) & 15) != 0) return LCC_ERR_ALIGN;
     if ((v && ((uintptr_t)q.vt & 7) != 0) || (a.bias != nullptr && ((uintptr_t)a.bias & 7) != 0)) return LCC_ERR_ALIGN;
+    if (!walk_offsets_fit(a)) return LCC_ERR_SHAPE;      // lda is E, whose square of weights is in memory
     g_launch_counts[LC_GEMM_VIT_QKV]++;
     int big = big_tile_rows(a, 1);
     if (big == 160) big = 192;
     if (big == 272) big = 256;      // the rotation / transposed-V epilogues live on the fixed-height 256-column tiles (129: the 128-row one)
-    if (a.epilogue == EPI_VIT_QKV) {
-      if (big == 256) launch_big_s<256, EPI_VIT_QKV, 6, false>(a, st);
-      else if (big == 192) launch_big_s<192, EPI_VIT_QKV, 6, false>(a, st);
-      else launch_big_s<128, EPI_VIT_QKV, 6, false>(a, st);
-    } else if (qk) {
-      if (big == 256) launch_big_s<256, EPI_VIT_QK, 6, false>(a, st);
-      else if (big == 192) launch_big_s<192, EPI_VIT_QK, 6, false>(a, st);
-      else launch_big_s<128, EPI_VIT_QK, 6, false>(a, st);
-    } else {
-      if (big == 256) launch_big_s<256, EPI_VIT_V, 6, false>(a, st);
-      else if (big == 192) launch_big_s<192, EPI_VIT_V, 6, false>(a, st);
-      else launch_big_s<128, EPI_VIT_V, 6, false>(a, st);
-    }
+    if (a.epilogue == EPI_VIT_QKV) launch_vit<EPI_VIT_QKV>(a, big, st);
+    else if (qk) launch_vit<EPI_VIT_QK>(a, big, st);
+    else launch_vit<EPI_VIT_V>(a, big, st);
     return 0;
   }
   // weight-streaming path: up to g_skinny_rows rows (64: decode batches of 17-64 streams multiply every weight fragment with 2-4 activation
