@@ -101,13 +101,14 @@ int run_decoder_layers(lcc_engine* e, const DecBuffers& b, int S, const PrefillT
     const size_t kv_off = e->dec_off[owner].kv;
     const float scale_log2e = L.scale * 1.4426950408889634f;
     int ns = 1;
+    bool paired = false;          // the feed-forward's first product went with the input projection
     if (fused) {
       DgArgs gi, gs;
       gi.W = w.in_w; gi.M = S; gi.N = in_n; gi.K = W; gi.X = b.h; gi.ldx = W; gi.C32 = b.part; gi.ldc = in_n;
       gs.W = w.gate_up_w; gs.M = S; gs.N = 2 * L.ff_pad; gs.K = W; gs.X = b.h; gs.ldx = W; gs.C = b.cat + L.heads * L.vdim_pad; gs.ldc = ldcat;
       LCC_TRY(dgemv_in_swiglu(gi, gs, st));
     } else {
-      LCC_TRY(slab_gemm(b, b.h, W, w.in_w, S, in_n, W, &ns, st));
+      LCC_TRY(slab_swiglu_gemm(b, b.h, W, w.in_w, S, in_n, W, L.ff_pad > 0 ? w.gate_up_w : nullptr, 2 * L.ff_pad, b.cat + L.heads * L.vdim_pad, ldcat, &ns, &paired, st));
     }
     LatentInArgs in; in.part = b.part; in.nsplit = ns; in.rows = S; in.ldn = in_n; in.qp = L.q_rank_pad; in.rp = own ? rp : 0; in.q_rank = L.q_rank;
     in.kv_rank = L.kv_rank; in.heads = L.heads; in.eps = e->dc.norm_eps; in.q_norm = w.q_norm; in.kv_norm = w.kv_norm; in.cq = b.cq; in.gate = b.gate;
@@ -144,7 +145,7 @@ int run_decoder_layers(lcc_engine* e, const DecBuffers& b, int S, const PrefillT
       LCC_TRY(latent_attn_decode(a, st));
       LCC_TRY(latent_merge_uv(a, w.uv_w, L.vdim_pad, b.gate, b.cat, ldcat, st));
     }
-    if (!fused && L.ff_pad > 0) LCC_TRY(plain_gemm(b.h, W, w.gate_up_w, b.cat + L.heads * L.vdim_pad, ldcat, S, 2 * L.ff_pad, W, LCC_EPI_SWIGLU, st));
+    if (!fused && !paired && L.ff_pad > 0) LCC_TRY(plain_gemm(b.h, W, w.gate_up_w, b.cat + L.heads * L.vdim_pad, ldcat, S, 2 * L.ff_pad, W, LCC_EPI_SWIGLU, st));
     const DytNorm& next = l + 1 < NL ? e->dw[l + 1].norm : e->dec_final_norm;
     if (fused) {
       DgArgs go; go.W = w.out_w; go.M = S; go.N = W; go.K = ldcat; go.X = b.cat; go.ldx = ldcat; go.X32 = b.x; go.C = b.h; go.dyt = next;

@@ -1905,21 +1905,20 @@ __device__ unsigned int lcc_zero_page_g[64];  // 256 zero bytes: x operand of ab
 // MG = 16-row groups of activations (M <= 16 * MG): the weight fragment of a k-block is loaded ONCE and multiplied with MG activation
 // fragments (rows mg*16 + li), so 17..64 decode streams still read every weight byte once per step (round 4: before, they went through the
 // 64-row GEMM tiles: 8.5-11.9 ms per 32-stream step where the weight stream alone costs ~2.6 ms).
-template <int NTILE, int MODE, bool PACKED, int UNR, int PIPE, int MG = 1>
-__global__ __launch_bounds__(256) void gemv_skinny_kernel(
+// bx, split, nsplit: the block's weight tiles and its share of K.  red: the waves' sums; xs_all: the activations of MG > 1
+template <int NTILE, int MODE, bool PACKED, int UNR, int PIPE, int MG>
+LCC_DEVICE void gemv_skinny_body(
     const bf16_t* __restrict__ X, int ldx, const bf16_t* __restrict__ W, int ldw,
-    const bf16_t* __restrict__ bias, void* __restrict__ out, int ldo, int M, int N, int K, int chunks_per_split, GemvTail tail) {
+    const bf16_t* __restrict__ bias, void* __restrict__ out, int ldo, int M, int N, int K, int chunks_per_split, const GemvTail& tail, int bx, int split, int nsplit,
+    f32x4 (*red)[NTILE * MG][64], u32x4* xs_all) {
   constexpr int NW = 4;
   static_assert(MODE != 3 || MG == 1, "the fused tail serves M <= 2");
-  __shared__ f32x4 red[NW - 1][NTILE * MG][64];
   // MG > 1: the activation rows of a 64-k chunk are fetched in FULL 128-byte lines (one load instruction = 8 rows x 128 B; the
   // fragment-shaped load -- 16 rows x 64 B per instruction -- was 2.3x slower at M = 32: 99 vs 43 us for the gate/up GEMV,
   // profiles/r04/bench_32streams_mg_gemv_first_version.json) and turned into MFMA fragments through a wave-private LDS scratch with the
   // (chunk ^ row & 7) swizzle of gemm_big_kernel's activation image: ds_write_b128 of the raw lines, ds_read_b128 of the fragments.
-  __shared__ u32x4 xs_all[MG > 1 ? NW * MG * 128 : 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * (NTILE * 16);
-  const int split = blockIdx.y;
+  const int n0 = bx * (NTILE * 16);
   const int nchunk = (K + 63) >> 6, K32 = (K + 31) >> 5;
   const int cb = split * chunks_per_split, ce = min(nchunk, cb + chunks_per_split);
 
@@ -2073,7 +2072,6 @@ __global__ __launch_bounds__(256) void gemv_skinny_kernel(
     if (flag[0] == 0.f) return;
     if (threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     __syncthreads();
-    const int nsplit = gridDim.y;
     if (tail.kind == 1) {
       for (int m = 0; m < M; ++m)
         tail_add_rmsnorm_row(tail.h + (size_t)m * N, (const float*)out, nsplit, (size_t)M * ldo, (size_t)m * ldo, tail.norm_w,
@@ -2131,6 +2129,34 @@ __global__ __launch_bounds__(256) void gemv_skinny_kernel(
       }
     }
   }
+}
+constexpr int gemv_sums(int ntile, int mg) { return 3 * ntile * mg * 64; }      // 16-byte pieces of LDS
+constexpr int gemv_rows_lds(int mg) { return mg > 1 ? 4 * mg * 128 : 1; }
+template <int NTILE, int MODE, bool PACKED, int UNR, int PIPE, int MG = 1>
+__global__ __launch_bounds__(256) void gemv_skinny_kernel(
+    const bf16_t* __restrict__ X, int ldx, const bf16_t* __restrict__ W, int ldw,
+    const bf16_t* __restrict__ bias, void* __restrict__ out, int ldo, int M, int N, int K, int chunks_per_split, GemvTail tail) {
+  __shared__ f32x4 red[3][NTILE * MG][64];
+  __shared__ u32x4 xs_all[gemv_rows_lds(MG)];
+  gemv_skinny_body<NTILE, MODE, PACKED, UNR, PIPE, MG>(X, ldx, W, ldw, bias, out, ldo, M, N, K, chunks_per_split, tail, blockIdx.x, blockIdx.y, gridDim.y, red, xs_all);
+}
+// Two products of the same 17..64 rows in ONE launch: a gate/up projection (SwiGLU, NTILE tiles a block) and, behind its blocks, another one into fp32 slabs (a tile
+// a block).  Alone, neither fills the chip (32 rows of the 2B layer-list decoder: 187 blocks of gate/up, 13.6 us; 162 of the input projection, 4.6 us): the
+// small one runs on the units that the large one leaves, and a launch of the step is gone.  Same sums, same bits.
+struct GemvPart { const bf16_t *X, *W; void* out; int ldx, ldo, N, K, cps; };
+template <int NTILE, int MG>
+__global__ __launch_bounds__(256) void gemv_rows_pair_kernel(GemvPart sw, GemvPart in, int M, int nb_sw, int nb_in) {
+  constexpr int S1 = gemv_sums(NTILE, MG), S2 = gemv_sums(1, MG);
+  __shared__ f32x4 red[S1 > S2 ? S1 : S2];
+  __shared__ u32x4 xs_all[gemv_rows_lds(MG)];
+  const int b = blockIdx.x;
+  const GemvTail none{};
+  if (b < nb_sw)
+    gemv_skinny_body<NTILE, 2, true, 1, 1, MG>(sw.X, sw.ldx, sw.W, sw.K, nullptr, sw.out, sw.ldo, M, sw.N, sw.K, sw.cps, none, b, 0, 1,
+                                               reinterpret_cast<f32x4(*)[NTILE * MG][64]>(red), xs_all);
+  else
+    gemv_skinny_body<1, 0, true, 1, 1, MG>(in.X, in.ldx, in.W, in.K, nullptr, in.out, in.ldo, M, in.N, in.K, in.cps, none, (b - nb_sw) % nb_in, (b - nb_sw) / nb_in, 1,
+                                           reinterpret_cast<f32x4(*)[MG][64]>(red), xs_all);
 }
 
 static int g_skinny_rows = 64;
@@ -2210,6 +2236,34 @@ static void launch_gemv_rows(const GemmArgs& a, int S, void* out, int ldo, int c
     case 2: if constexpr (MODE != 2) { launch_gemv_tiles<2, MODE>(a, S, out, ldo, cps, st); break; } [[fallthrough]];
     default: launch_gemv_l<LEAST, MODE>(dim3((a.N + 16 * LEAST - 1) / (16 * LEAST), S), a, out, ldo, cps, st);
   }
+}
+
+// in: fp32 slabs (partial, nsplit); sw: SwiGLU.  Takes what the two calls of gemm_bf16 would take on the weight-streaming path with 17 to 64 rows
+bool gemv_rows_pair_ok(const GemmArgs& in, const GemmArgs& sw) {
+  auto one = [](const GemmArgs& a) {
+    return a.w_packed && !a.w_fp8 && a.M > 16 && a.M <= 64 && a.N > 0 && gemm_routes_skinny(a.M, a.K, false) && (a.N & 15) == 0 && (a.lda & 7) == 0 &&
+           (((uintptr_t)a.A | (uintptr_t)a.W) & 15) == 0 && a.bias == nullptr && a.tail.kind == 0;
+  };
+  return one(in) && one(sw) && in.M == sw.M && in.partial != nullptr && in.nsplit >= 1 && in.nsplit <= 8 && in.nsplit <= (in.K + 63) / 64 && in.epilogue == EPI_NONE &&
+         sw.partial == nullptr && sw.epilogue == EPI_SWIGLU && (sw.N & 31) == 0 && (sw.ldc & 3) == 0 && ((uintptr_t)sw.C & 15) == 0;
+}
+template <int NTILE>
+static void launch_rows_pair(const GemmArgs& in, const GemmArgs& sw, hipStream_t st) {
+  const int nin = (in.K + 63) / 64, nb_sw = (sw.N + NTILE * 16 - 1) / (NTILE * 16), nb_in = in.N / 16;
+  const GemvPart a{sw.A, sw.W, sw.C, sw.lda, sw.ldc, sw.N, sw.K, (sw.K + 63) / 64}, b{in.A, in.W, in.partial, in.lda, in.N, in.N, in.K, (nin + in.nsplit - 1) / in.nsplit};
+  const dim3 grid(nb_sw + nb_in * in.nsplit);
+  if (in.M <= 32) gemv_rows_pair_kernel<NTILE, 2><<<grid, dim3(256), 0, st>>>(a, b, in.M, nb_sw, nb_in);
+  else if (in.M <= 48) gemv_rows_pair_kernel<NTILE, 3><<<grid, dim3(256), 0, st>>>(a, b, in.M, nb_sw, nb_in);
+  else gemv_rows_pair_kernel<NTILE, 4><<<grid, dim3(256), 0, st>>>(a, b, in.M, nb_sw, nb_in);
+}
+int gemv_rows_pair(const GemmArgs& in, const GemmArgs& sw, hipStream_t st) {
+  if (!gemv_rows_pair_ok(in, sw)) return LCC_ERR_ARG;
+  switch (gemv_rows_tiles(sw, 1)) {
+    case 6: launch_rows_pair<6>(in, sw, st); break;
+    case 4: launch_rows_pair<4>(in, sw, st); break;
+    default: launch_rows_pair<2>(in, sw, st);
+  }
+  return 0;
 }
 
 // ------------------------------------------------------------------------------------------------

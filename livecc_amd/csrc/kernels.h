@@ -79,6 +79,8 @@ struct GemmArgs {
   VitQkvEpi vq;                                 // epilogue == GEMM_EPI_VIT_QK / GEMM_EPI_VIT_V only
 };
 int gemm_bf16(const GemmArgs& a, hipStream_t st);
+bool gemv_rows_pair_ok(const GemmArgs& in, const GemmArgs& sw);                      // two products of the same 17..64 rows in one launch:
+int gemv_rows_pair(const GemmArgs& in, const GemmArgs& sw, hipStream_t st);          //   fp32 slabs and SwiGLU
 bool gemm_vit_qkv_eligible(int M, int E, int K);   // shapes the EPI_VIT_QK / EPI_VIT_V epilogues serve (8-wave kernel: K % 64 == 0; M > 64, M % 4 == 0, E % 32 == 0)
 int gemv_num_splits(int N, int K);
 int gemm_plan(int M, int N, int K, int epilogue, int nsplit, bool w_fp8);     // host logic: which kernel family would serve this GEMM

@@ -482,6 +482,21 @@ def test_many_streams_decode_in_groups(dev):
             assert U.error(g, U.oracle_logits(cfg, T, seqs[k])[[-1]]) < U.LIMIT
 
 
+@pytest.mark.parametrize("ff,n", [(8300, 17), (8300, 32), (8300, 64), (7900, 33), (7900, 48), (100, 64)])
+def test_wide_feed_forward_beside_the_input_projection(dev, ff, n):
+    """17 to 64 rows: both products of the normed rows are one launch, the wide one in four or six weight tiles a block (8300: two in the last block)."""
+    from livecc_amd.config import DebunexConfig
+    cfg = DebunexConfig(200, 100, [U.L(U.M(3, 40, 48, 72, 90, 0.2), ff), U.L(U.M(2, 64, 64, 64, 90, 0.2, 0), 0)], 1e-5, 20.0, name="wide-ff")
+    T = U.make_weights(cfg, 8)
+    m = _model(cfg, T, dev, max_streams=n, max_kv_len=64, max_new_rows=512)
+    seqs = [U.ids_of(cfg, 3 + i % 5, 50 + i) for i in range(n)]
+    st = [m.new_stream() for _ in seqs]
+    m.forward_step([(s, x[:-1], []) for s, x in zip(st, seqs)])
+    got = m.forward_step([(s, [x[-1]], [0]) for s, x in zip(st, seqs)])
+    for i in sorted({0, 1, 15, 16, n // 2, n - 2, n - 1}):
+        assert U.error(got[i], U.oracle_logits(cfg, T, seqs[i])[[-1]]) < U.LIMIT
+
+
 def test_fused_and_separate_decode_launches_agree(dev, lib):
     cfg = U.configs()["full-heads"]
     T = U.make_weights(cfg, 4)
