@@ -9,7 +9,7 @@
 //  * gemm_big_kernel     : the same tiles one a block, both waves of a SIMD in step: fp8-e4m3 W converted after the LDS read; 128-row tiles of one round.
 //  * gemm_walk_vh_kernel : the walk over row tiles of 256 / 272 / 288 rows (no ragged last row tile).
 //  * gemm_vh_kernel      : row tiles of 128 / 144 rows, split-K slabs of one streaming chunk.
-//  * gemm_tall_kernel    : one block row covers all of M (256 < M <= 448: one streaming chunk's gate/up).
+//  * gemm_tall_kernel    : one block row covers all of M (up to 448 rows: gate/up of one streaming chunk or of a few short ones).
 //  * gemm_mid_kernel     : shapes with few 256-column tiles.  64x128x64 (128x128x64) tile, 8 waves, 6- (4-) stage LDS-DMA ring.
 //  * gemm_glds_kernel /   : row-major W, K % 64 != 0.  64x128x64 (128x128x64) tile, 4 waves,
 //    gemm_tiled_kernel     LDS-DMA 3-stage ring / register-staged double buffer with an XOR swizzle, XCD-aware block remap.
@@ -1390,190 +1390,182 @@ __global__ __launch_bounds__(512) void gemm_vh_kernel(const bf16_t* __restrict__
 }
 
 // ------------------------------------------------------------------------------------------------
-// tiled GEMM v4 ("tall"): ONE block row covers all of M (256 < M <= 448: a single-stream streaming chunk is 386 rows), 8 waves,
-// 448 x 160 x 64 block tile, LDS-DMA for both operands
+// tiled GEMM v4 ("tall"): ONE block row covers all of M (up to 448: a single-stream streaming chunk is 386 rows), 8 waves,
+// (4 MT x 16) x 160 x 64 block tile, LDS-DMA for both operands, the two waves of a SIMD taking turns (gemm_walk_kernel)
 // ------------------------------------------------------------------------------------------------
-// Why: M = 386 on the 128 x 256 tiles of gemm_big_kernel is 4 row tiles (the fourth holds 2 rows) x 148 = 592 blocks = 2.3 rounds
-// of the 256 CUs at one block per CU: the gate/up GEMM of a chunk ran at 0.65 PF / 29.8 % MfmaUtil against 50.7 % at M = 3088
-// (profiles/r02).  Split-K or stream-K on those tiles buys <= 13 % (1.75 instead of 2 rounds).  Here every block owns ALL rows and
-// 160 columns, so N = 37888 is 237 blocks = ONE round on 92.5 % of the CUs, the W panel of a block is read once from L2, and the
-// activation tile (448 x 64 per k-step, the same for every block) comes out of L2.
-//   * waves: 4 (M) x 2 (N).  M-wave wm owns rows wm*112 .. +111 = 7 MFMA row tiles; N-wave 0 owns column tiles 0-5, N-wave 1
-//     tiles 6-9 (gate/up pairs stay inside a wave: SwiGLU epilogue).  Waves w and w + 4 share a SIMD, so every SIMD issues
-//     7 x (6 + 4) x 2 = 140 MFMAs per k-step.  A wave whose rows end early (M = 386: the last M-wave has 4 live row tiles)
-//     takes the 4-row-tile code path; a wave without rows only feeds the DMA ring.
-//   * LDS: A image 448 rows x 128 B (XOR-swizzled 16-byte chunks, as gemm_big_kernel) + W tile 20 fragment sub-tiles of 1 KB =
-//     77,824 B per stage, two stages = 155,648 B; per k-step 76 KB of DMA (1216 clk at 64 B/clk) under 2240 clk of MFMA issue.
-// Requires packed W, K % 64 == 0.  W8: fp8 weights in their packed order, converted after the LDS read (each of the four M-waves converts the columns
-// it multiplies: 96 conversions of 16 bytes beside 84 MFMAs), their scale in the epilogue.
-template <int EPI, int SCHED, bool W8>
+// Why: M = 386 on 128 x 256 tiles is 4 row tiles (the fourth holds 2 rows) x 148 = 592 blocks = 2.3 rounds of the 256 CUs.  Here every block owns ALL
+// rows and 160 columns, so N = 37888 is 237 blocks = ONE round on 92.5 % of the CUs, and the W panel of a block is read once.
+//   * waves: 4 (M) x 2 (N).  M-wave wm owns MT = ceil(fragments / 4) row fragments from wm * MT on; N-wave 0 owns column tiles 0-5, N-wave 1 tiles 6-9
+//     (gate/up pairs stay inside a wave: SwiGLU epilogue).  Waves w and w + 4 share a SIMD: 6 + 4 column tiles of the same rows.
+//   * a k-tile is two phases of row fragments (MT 7: three, 3 + 2 + 2 -- the weight fragments of a k-tile, 48 registers, stay for all of them); what a phase
+//     reads is filled again behind it, in the order in which it is needed, as in gemm_walk_kernel.  (Phases for the two 32-k halves, 13 fragments each, with the
+//     activations asked for one k-tile ahead: 103 us at 386 rows, but 108 / 103 at 448 and 73 / 67 at 192.)
+//   * LDS: A image rows x 128 B (XOR-swizzled 16-byte chunks) + W tile 20 fragment sub-tiles of 1 KB = 77,824 B per stage (MT 7); two stages, with few rows up to four:
+//     there the weights' way from HBM is what a launch takes.
+// [37888, 3584] with SwiGLU, us, both waves in step (and always seven fragments) -> here: 100 rows 86 -> 57, 192 90 -> 67, 256 101 -> 74, 300 108 -> 84, 386 114 -> 106, 448 119 -> 107.
+// Rows beyond M hold copies of the last ones: their products go into rows that are not stored.
+// Requires packed W, K % 64 == 0.  W8: fp8 weights in their packed order, converted behind the LDS read, beside the other wave's MFMAs; their scale in the epilogue.
+template <int MT, bool W8>
+struct Tall {
+  static constexpr int NP = MT > 6 ? 3 : 2, ROWS = 4 * MT * 16, A_UNITS = ROWS * 8;
+  static constexpr int B_SUB = W8 ? 10 : 20, PB = (B_SUB + 7) / 8, STAGE = A_UNITS + B_SUB * 64;      // fragment sub-tiles of 1 KB (W8: a fragment's 64 k); 16-byte units
+  static constexpr int frags(int p) { return NP == 3 ? (p == 0 ? 3 : 2) : (p == 0 ? (MT + 1) / 2 : MT / 2); }      // row fragments of phase p, = a wave's pieces of 8 rows
+  static constexpr int from(int p) { return p == 0 ? 0 : p == 1 ? frags(0) : frags(0) + frags(1); }
+  static constexpr int pieces(int p) { return frags(p) + (p == 0 ? PB : 0); }
+  static constexpr int NSTAGE = 163840 / (STAGE * 16) > 4 ? 4 : 163840 / (STAGE * 16);
+  // pieces that may be on their way when phase p ends: those of the NP NSTAGE - 2 parts asked for behind what the next phase reads
+  static constexpr int later(int p) { int n = 0; for (int e = 0; e < NP * NSTAGE - 2; ++e) n += pieces((p + 2 + e) % NP); return n; }
+  static constexpr size_t LDS = (size_t)NSTAGE * STAGE * 16;
+  static_assert(NSTAGE >= 2 && (NP == 2 || MT == 7) && later(0) <= 63 && later(1) <= 63 && later(NP - 1) <= 63, "");
+};
+template <int EPI, int MT, bool W8>
 __global__ __launch_bounds__(512) void gemm_tall_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
     const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
     bf16_t* __restrict__ C, int ldc, int M, int N, int K, const float* __restrict__ wscale) {
-  static_assert(!W8 || SCHED == 1, "fp8 weights: one issue order is built");
-  constexpr int BM = 448, BN = 160, BK = 64, WM = 112, MT = 7, NT0 = 6;
-  constexpr int A_UNITS = BM * 8;                 // 16-byte units of the A image
-  constexpr int B_SUB = (BN / 16) * (W8 ? 1 : 2); // 20 fragment sub-tiles of 1 KB (W8: 10, each a fragment's 64 k)
-  constexpr int STAGE = A_UNITS + B_SUB * 64;
-  constexpr int A_PER_WAVE = BM / 64;             // 7 pieces of 8 rows x 128 B per wave
+  using T = Tall<MT, W8>;
+  constexpr int BN = 160, BK = 64, NT0 = 6, NP = T::NP;
   extern __shared__ __attribute__((aligned(16))) u32x4 dsmem[];
 
   const int n0 = blockIdx.x * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 3, wn = wave >> 2;
   const int li = lane & 15, g = lane >> 4;
-  const int K32 = K >> 5, nfrag = N >> 4;
-  const int rows_left = M - wm * WM;                                     // wave-uniform
-  const int mt_live = rows_left <= 0 ? 0 : min(MT, (rows_left + 15) >> 4);
+  const int K32 = K >> 5, nfrag = N >> 4, nkt = K / BK;
+  const unsigned lds0 = lds_addr(dsmem), row_bytes = (unsigned)lda * 2u;
 
-  int aoffs[A_PER_WAVE];                         // element offsets from A (the row is clamped into the matrix)
+  // A wave's pieces of 8 rows: an offset per lane, the same for all of them but the one that ends at row M - 1, and a scalar one.  Pieces behind that one copy it
+  // again, each to its own place: another phase's rows may still be read.
+  const unsigned swz = ((lane & 7) ^ (lane >> 3)) << 4, whole = (unsigned)(lane >> 3) * row_bytes + swz;
+  const int last = (M - 1) & ~7;
+  const unsigned ends = (unsigned)min(lane >> 3, M - 1 - last) * row_bytes + swz;
+  auto rows_part = [&](auto pc, int kt, int stage) {          // of phase p
+    constexpr int p = decltype(pc)::value, n = T::frags(p);
+    const bf16_t* base = A + (size_t)min(kt, nkt - 1) * BK;
 #pragma unroll
-  for (int q = 0; q < A_PER_WAVE; ++q) {
-    const int row = (wave * A_PER_WAVE + q) * 8 + (lane >> 3);
-    aoffs[q] = min(row, M - 1) * lda + (((lane & 7) ^ (lane >> 3)) << 3);
-  }
-  // W sub-tiles: waves 0-3 copy three each (0..11), waves 4-7 two each (12..19); sub-tile st = fragment row st >> 1, 32-k block st & 1
-  // (W8: waves 0 and 1 two, the others one)
-  constexpr int NB = W8 ? 2 : 3, WK = W8 ? 512 : 1024;       // pieces of a wave at most; elements of W (2 bytes) from k-tile to k-tile
-  const int nb = W8 ? (wave < 2 ? 2 : 1) : (wave < 4 ? 3 : 2);
-  const int st0 = W8 ? (wave < 2 ? wave * 2 : wave + 2) : (wave < 4 ? wave * 3 : 12 + (wave - 4) * 2);
-  const bf16_t* bsrc[NB];                        // bf16 weights
-  if constexpr (!W8) {
-#pragma unroll
-    for (int q = 0; q < NB; ++q) {
-      const int st = min(st0 + q, B_SUB - 1);
-      const int fr = min((n0 >> 4) + (st >> 1), nfrag - 1);
-      bsrc[q] = W + ((size_t)fr * K32 + (st & 1)) * 512 + lane * 8;
-    }
-  }
-  // Round 6: activation pieces (8 rows each) that lie entirely beyond the last 16-row MFMA tile are not fetched at all -- at M = 386 the rows
-  // 400..447 of the 448-row image (6 of 56 pieces: 11 % of the activation DMA, which is 70 % of this kernel's L2 -> LDS traffic) were copies
-  // of row 385 that no MFMA reads.  Wave-uniform; the ring's waits are vmcnt(0), so the piece count per wave need not be uniform.
-  const int m_rows = (M + 15) & ~15;
-  auto issue = [&](int kt, int stage) {
-    u32x4* sbase = dsmem + stage * STAGE;
-#pragma unroll
-    for (int q = 0; q < A_PER_WAVE; ++q)
-      if ((wave * A_PER_WAVE + q) * 8 < m_rows) {
-        if constexpr (W8) glds16_base(A + kt * BK, (unsigned)aoffs[q] * 2u, lds_addr(sbase + (wave * A_PER_WAVE + q) * 64));
-        else glds16((A + aoffs[q] + kt * BK), lds_addr(sbase + (wave * A_PER_WAVE + q) * 64));
-      }
-#pragma unroll
-    for (int q = 0; q < NB; ++q)
-      if (q < nb) {
-        if constexpr (W8) {      // scalar bases: the converted fragments need the registers
-          const int fr = min((n0 >> 4) + st0 + q, nfrag - 1);
-          glds16_base(W + (size_t)fr * (K >> 6) * 512 + (size_t)kt * WK, (unsigned)lane * 16u, lds_addr(sbase + A_UNITS + (st0 + q) * 64));
-        } else glds16((bsrc[q] + (size_t)kt * WK), lds_addr(sbase + A_UNITS + (st0 + q) * 64));
-      }
-  };
-
-  // SCHED 2: the 10 pieces of a wave (7 activation + 3 W; waves 4-7 repeat their second W sub-tile as the third) go out ONE at a time
-  // between the row-tile steps of the MFMA stream instead of as a burst behind the barrier (every LDS-DMA instruction holds the wave's
-  // issue port for ~60-100 cycles, and right after the barrier both waves of a SIMD are at the same point)
-  auto issue_piece = [&](int kt, int stage, int q) {
-    u32x4* sbase = dsmem + stage * STAGE;
-    if (q < A_PER_WAVE) {
-      if ((wave * A_PER_WAVE + q) * 8 < m_rows)
-        glds16((A + aoffs[q < A_PER_WAVE ? q : 0] + kt * BK), lds_addr(sbase + (wave * A_PER_WAVE + q) * 64));
-    } else {
-      const int qq = min(q - A_PER_WAVE, nb - 1);
-      glds16((bsrc[qq] + (size_t)kt * WK), lds_addr(sbase + A_UNITS + (st0 + qq) * 64));
+    for (int q = 0; q < n; ++q) {
+      const int x = wave * n + q, wr = x / (2 * n), to = wr * (MT * 16) + T::from(p) * 16 + (x - wr * 2 * n) * 8, row = min(to, last);
+      glds16_base(base, (row == last ? ends : whole) + (unsigned)row * row_bytes, lds0 + (unsigned)(stage * T::STAGE) * 16u + to * 128u);
     }
   };
-  constexpr int NPIECE = A_PER_WAVE + NB;
-
-  f32x4 acc[MT][NT0];
+  auto weights = [&](int kt, int stage) {
+    const int k = min(kt, nkt - 1);
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < NT0; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-  const int nkt = K / BK;
-  issue(0, 0);
-  int aoff[2];
-#pragma unroll
-  for (int kk = 0; kk < 2; ++kk) aoff[kk] = (wm * WM + li) * 8 + ((W8 ? g * 2 + kk : kk * 4 + g) ^ (li & 7));
-  const int boff = A_UNITS + (wn * NT0 * (W8 ? 1 : 2)) * 64 + lane;
-
-  // one k-tile of this wave: MTW live row tiles x NTW column tiles.  Per 32-k half: the NTW W fragments are read up front, the
-  // activation fragments stream through a 3-register ring two row tiles ahead of their MFMAs.
-  auto ktile = [&](const u32x4* s, auto mtw_c, auto ntw_c, int kt_dma, int st_dma) {
-    constexpr int MTW = decltype(mtw_c)::value, NTW = decltype(ntw_c)::value;
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      bf16x8 fb[NTW], fa[3];
-#pragma unroll
-      for (int j = 0; j < NTW; ++j) {
-        if constexpr (W8) {          // this half's 8 of the lane's 16 k: half a fragment slot
-          const u32x2 raw = *reinterpret_cast<const u32x2*>(reinterpret_cast<const unsigned char*>(s + boff + j * 64) + kk * 8);
-          fb[j] = fp8x8_to_bf16x8(raw[0], raw[1]);
-        } else fb[j] = as_bf16x8(s[boff + (j * 2 + kk) * 64]);
-      }
-      fa[0] = as_bf16x8(s[aoff[kk]]);
-      if (MTW > 1) fa[1] = as_bf16x8(s[aoff[kk] + 128]);
-#pragma unroll
-      for (int i = 0; i < MTW; ++i) {
-        if (i + 2 < MTW) fa[(i + 2) % 3] = as_bf16x8(s[aoff[kk] + (i + 2) * 128]);
-#pragma unroll
-        for (int j = 0; j < NTW; ++j) acc[i][j] = mfma16(fb[j], fa[i % 3], acc[i][j]);
-        if (SCHED == 2 && kk * MTW + i < NPIECE) issue_piece(kt_dma, st_dma, kk * MTW + i);
-      }
-      if (SCHED >= 1) {   // pin the issue order: the fragment reads up front, then one activation read per row tile of MFMAs
-        __builtin_amdgcn_sched_group_barrier(0x100, NTW + (MTW > 1 ? 2 : 1), 0);
-#pragma unroll
-        for (int i = 0; i < MTW; ++i) {
-          if (i + 2 < MTW) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x008, NTW, 0);
-          if (SCHED == 2 && kk * MTW + i < NPIECE) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
-        }
-      }
+    for (int q = 0; q < T::PB; ++q) {
+      const int st = min(wave + 8 * q, T::B_SUB - 1);         // bf16: fragment row st >> 1, 32-k block st & 1
+      const int fr = min((n0 >> 4) + (W8 ? st : st >> 1), nfrag - 1);
+      const bf16_t* src = W8 ? W + (size_t)fr * (K >> 6) * 512 : W + ((size_t)fr * K32 + (st & 1)) * 512;
+      glds16_base(src + (size_t)k * (W8 ? 512 : 1024), (unsigned)lane * 16u, lds0 + (unsigned)(stage * T::STAGE + T::A_UNITS + st * 64) * 16u);
     }
-    if (SCHED == 2) {     // fewer row-tile steps than pieces (the 4-row-tile wave: 8 steps): the rest behind the last MFMAs
-#pragma unroll
-      for (int q = 2 * MTW; q < NPIECE; ++q) issue_piece(kt_dma, st_dma, q);
-    }
+  };
+  auto part = [&](auto pc, int kt, int stage) {
+    if constexpr (decltype(pc)::value == 0) weights(kt, stage);
+    rows_part(pc, kt, stage);
   };
   using I0 = std::integral_constant<int, 0>;
-  using I4 = std::integral_constant<int, 4>;
-  using I6 = std::integral_constant<int, 6>;
-  using I7 = std::integral_constant<int, 7>;
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, NP - 1>;
+#pragma unroll
+  for (int k = 0; k < T::NSTAGE; ++k) {
+    part(I0{}, k, k);
+    if (NP == 3 || k + 1 < T::NSTAGE) part(I1{}, k, k);
+    if constexpr (NP == 3) { if (k + 1 < T::NSTAGE) part(I2{}, k, k); }
+  }
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(T::later(NP - 1)) : "memory");
+  __builtin_amdgcn_s_barrier();
+  if (wn) __builtin_amdgcn_s_barrier();          // the second wave of a SIMD: one slot behind
+
+  int aoff[2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) aoff[kk] = (wm * (MT * 16) + li) * 8 + ((W8 ? g * 2 + kk : kk * 4 + g) ^ (li & 7));
+  const int boff = T::A_UNITS + (wn * NT0 * (W8 ? 1 : 2)) * 64 + lane;
   const int nbase = n0 + wn * NT0 * 16;
-  // The live tile shape of a wave is loop-invariant, so every shape gets its OWN copy of the k loop (same barrier sequence in all
-  // of them): one loop with a switch inside made hipcc keep the accumulators of all shapes alive across the paths and spill 190
-  // registers; a single-shape loop needs 252.
-  auto run = [&](auto mtw_c, auto ntw_c) {
-    constexpr int MTW = decltype(mtw_c)::value, NTW = decltype(ntw_c)::value;
-    for (int kt = 0; kt < nkt; ++kt) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();   // tile kt complete in LDS; every wave is done reading tile kt-1
-      // SCHED 2 (waves with rows): the pieces go out inside ktile, unconditionally -- past the last tile the source is clamped and the
-      // copy lands in the stage nobody reads any more
-      if ((SCHED != 2 || MTW == 0) && kt + 1 < nkt) issue(kt + 1, (kt + 1) & 1);
-      if constexpr (MTW > 0) ktile(dsmem + (kt & 1) * STAGE, mtw_c, ntw_c, min(kt + 1, nkt - 1), (kt + 1) & 1);
-    }
-    if (SCHED == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if constexpr (MTW > 0) {
-      int le = lane;
-      asm volatile("" : "+v"(le));          // the epilogue's addresses are formed here, not carried through the loop
-      const int lie = le & 15, ge = le >> 4;
-      if constexpr (W8) {                   // the rows' scales, one column tile at a time
+  auto run = [&](auto ntw_c) {
+    constexpr int NTW = decltype(ntw_c)::value;
+    f32x4 acc[MT][NTW];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NTW; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    bf16x8 fb[2][NTW], fa[2][T::frags(0)];
+    auto slot_end = [] {
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto read = [&](auto pc, const u32x4* s) {
+      constexpr int p = decltype(pc)::value;
+      if constexpr (p == 0) {
 #pragma unroll
         for (int j = 0; j < NTW; ++j) {
-          asm volatile("" ::: "memory");
-          const f32x4 sc = *reinterpret_cast<const f32x4*>(wscale + min(nbase + j * 16 + ge * 4, N - 4));
-#pragma unroll
-          for (int i = 0; i < MTW; ++i) acc[i][j] *= sc;
+          if constexpr (W8) {
+            const u32x4 raw = s[boff + j * 64];
+            fb[0][j] = fp8x8_to_bf16x8(raw[0], raw[1]);
+            fb[1][j] = fp8x8_to_bf16x8(raw[2], raw[3]);
+          } else {
+            fb[0][j] = as_bf16x8(s[boff + (j * 2) * 64]);
+            fb[1][j] = as_bf16x8(s[boff + (j * 2 + 1) * 64]);
+          }
         }
       }
-      tile_epilogue<EPI, (MTW > 0 ? MTW : 1), (MTW > 0 ? NTW : 2), MT, NT0>(acc, wm * WM, nbase, nbase / 2, lie, ge, bias, residual, ldr, C, ldc, M, N,
-                                                                        nullptr, nullptr);
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int i = 0; i < T::frags(p); ++i) fa[kk][i] = as_bf16x8(s[aoff[kk] + (T::from(p) + i) * 128]);
+    };
+    auto landed = [&](auto pc) {                 // what the next phase reads has landed and this one's fragments are in registers
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(T::later(decltype(pc)::value)) : "memory");
+      slot_end();
+    };
+    auto multiply = [&](auto pc) {
+      constexpr int p = decltype(pc)::value;
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int i = 0; i < T::frags(p); ++i)
+#pragma unroll
+          for (int j = 0; j < NTW; ++j) acc[T::from(p) + i][j] = mfma16(fb[kk][j], fa[kk][i], acc[T::from(p) + i][j]);
+    };
+    int st = 0;                                  // stage of the k-tile
+    for (int kt = 0; kt < nkt; ++kt) {
+      const int before = st == 0 ? T::NSTAGE - 1 : st - 1;
+      const u32x4* s = dsmem + st * T::STAGE;
+      read(I0{}, s);
+      part(I2{}, kt + T::NSTAGE - 1, before);    // into what the last phase of the k-tile before has read
+      landed(I0{});
+      multiply(I0{});
+      slot_end();
+      read(I1{}, s);
+      part(I0{}, kt + T::NSTAGE, st);
+      landed(I1{});
+      multiply(I1{});
+      if constexpr (NP == 3) {
+        slot_end();
+        read(I2{}, s);
+        part(I1{}, kt + T::NSTAGE, st);
+        landed(I2{});
+        multiply(I2{});
+      }
+      st = st == T::NSTAGE - 1 ? 0 : st + 1;
+      if (wn == 0 || kt + 1 < nkt) slot_end();
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the copies behind the last k-tile: this block's LDS until they have landed
+    int le = lane;
+    asm volatile("" : "+v"(le));          // the epilogue's addresses are formed here, not carried through the loop
+    const int lie = le & 15, ge = le >> 4;
+    if constexpr (W8) {                   // the rows' scales, one column tile at a time
+#pragma unroll
+      for (int j = 0; j < NTW; ++j) {
+        asm volatile("" ::: "memory");
+        const f32x4 sc = *reinterpret_cast<const f32x4*>(wscale + min(nbase + j * 16 + ge * 4, N - 4));
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[i][j] *= sc;
+      }
+    }
+    tile_epilogue<EPI, MT, NTW>(acc, wm * (MT * 16), nbase, nbase / 2, lie, ge, bias, residual, ldr, C, ldc, M, N, nullptr, nullptr);
   };
-  if (mt_live == 0) run(I0{}, I4{});                 // no rows: DMA + barriers only
-  else if (wn == 0) { if (mt_live <= 4) run(I4{}, I6{}); else run(I7{}, I6{}); }
-  else { if (mt_live <= 4) run(I4{}, I4{}); else run(I7{}, I4{}); }
+  if (wn == 0) run(std::integral_constant<int, NT0>{});
+  else run(std::integral_constant<int, 10 - NT0>{});
 }
 
 // 0: register-staged 2-stage kernel; 1: LDS-DMA 3-stage kernel; 2 (default): measured best per tile shape --
@@ -1825,31 +1817,39 @@ static bool tall_wanted(const GemmArgs& a) {
   if (g_gemm_variant == 8) return true;
   if (g_gemm_variant != 2) return false;
   const int blocks = (a.N + 159) / 160;
-  // fp8 weights: where 128-row tiles would need a fourth row of blocks (386 x 37888, K 3584 with SwiGLU 149 -> 107 us; 300 rows 101 / 103, 272 rows 107 / 105)
-  return a.M > (a.w_fp8 ? 384 : 256) && blocks >= 192 && blocks <= 256;
+  if (blocks < 192 || blocks > 256) return false;
+  // Up to 256 rows where the other tiles (128 x 128, or two rows of 128 x 256) are more than one round.  K 3584 with SwiGLU, us, other tiles / these:
+  //   bf16, N 37888: 65 rows 67 / 55, 128 71 / 59, 192 80 / 67, 256 89 / 74, 272 and more 84 / 84 (walking tiles; 300 rows 101 before them);  N 30720: 100 rows 48 / 52, 256 67 / 67
+  //   fp8,  N 37888: 65 to 128 rows 56 / 57, 129 105 / 68, 256 90 / 75, 272 110 / 87, 330 114 / 96;  N 30720: 100 rows 44 / 56, 256 61 / 73
+  return a.M > 256 || (a.N > 32768 && a.M > (a.w_fp8 ? 128 : 64));
 }
-// (a 4-stage ring of 32-k half tiles in the same LDS was measured equal-to-slower -- 122.5 vs 125.2 us at M = 386, profiles/r03/gemm_tall_ring.txt:
-// the L2 -> LDS DMA is throughput-bound, a deeper ring has nothing to hide -- and was retired in round 5)
-template <int EPI, int SCHED, bool W8>
-static void launch_tall_s(const GemmArgs& a, hipStream_t st) {
-  constexpr size_t lds = (size_t)2 * (448 * 8 + (W8 ? 10 : 20) * 64) * 16;   // 155,648 B; fp8 weights 135,168 B
+template <int EPI, int MT, bool W8>
+static void launch_tall_rows(const GemmArgs& a, hipStream_t st) {
+  constexpr size_t lds = Tall<MT, W8>::LDS;
   static DeviceOnce attr_set;   // per instantiation
-  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_tall_kernel<EPI, SCHED, W8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  gemm_tall_kernel<EPI, SCHED, W8><<<dim3((a.N + 159) / 160), dim3(512), lds, st>>>(a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K,
-                                                                                   a.wscale);
+  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_tall_kernel<EPI, MT, W8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  gemm_tall_kernel<EPI, MT, W8><<<dim3((a.N + 159) / 160), dim3(512), lds, st>>>(a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, a.wscale);
+}
+template <int EPI, bool W8>
+static void launch_tall_w(const GemmArgs& a, hipStream_t st) {
+  if constexpr (EPI == EPI_SWIGLU) {          // the one product that comes here unforced (tall_wanted): fragments for each quarter of the rows
+    switch (((a.M + 15) / 16 + 3) / 4) {
+      case 1: case 2: return launch_tall_rows<EPI, 2, W8>(a, st);
+      case 3: return launch_tall_rows<EPI, 3, W8>(a, st);
+      case 4: return launch_tall_rows<EPI, 4, W8>(a, st);
+      case 5: return launch_tall_rows<EPI, 5, W8>(a, st);
+      case 6: return launch_tall_rows<EPI, 6, W8>(a, st);
+    }
+  }
+  launch_tall_rows<EPI, 7, W8>(a, st);
 }
 template <int EPI>
 static void launch_tall(const GemmArgs& a, hipStream_t st) {
   g_launch_counts[LC_GEMM_TALL]++;
-  // 0 compiler order, 1 pinned (default since round 6: 127.6 vs 131.6-132.6 us at M = 386 on N(0,1) activations, A/B/A/B, bit-identical --
-  // profiles/r06/m386_gemms_tall_sched_ab.jsonl; before the LDS-DMA went into inline asm the compiler's order had been the faster one), 2 pinned + spread DMA
-  static const int sched = [] { const char* v = getenv("LCC_TALL_SCHED"); return v ? atoi(v) : 1; }();
   if constexpr (EPI != EPI_RESIDUAL) {
-    if (a.w_fp8) return launch_tall_s<EPI, 1, true>(a, st);
+    if (a.w_fp8) return launch_tall_w<EPI, true>(a, st);
   }
-  if (sched == 2) launch_tall_s<EPI, 2, false>(a, st);
-  else if (sched == 1) launch_tall_s<EPI, 1, false>(a, st);
-  else launch_tall_s<EPI, 0, false>(a, st);
+  launch_tall_w<EPI, false>(a, st);
 }
 
 template <int EPI>

@@ -125,6 +125,36 @@ def test_gemm_tall_kernel(dev, M, N, K, epi, variant):
     assert_bf16_close(got, ref, f"gemm_tall[{M}x{N}x{K},epi{epi},v{variant}]", max_ulp=1.0, max_frac=5e-3, atol=atol)
 
 
+@pytest.mark.parametrize("M", [65, 96, 128, 129, 176, 192, 193, 248, 256, 257, 320, 321, 384])
+@pytest.mark.parametrize("K", [64, 128, 576])
+@pytest.mark.parametrize("fp8", [False, True], ids=["bf16", "fp8"])
+def test_gemm_tall_rows_in_quarters(dev, M, K, fp8):
+    """Every height of the tall tile's SwiGLU form (2 to 6 row fragments a quarter) at its edges: the last rows in each phase's part of a quarter, quarters
+    without rows, fewer k-tiles than the ring holds and more; the height the default variant takes at 33,280 columns is the forced one."""
+    from livecc_amd import ops
+    from livecc_amd.weights import dequantize_fp8_rows, quantize_fp8_rows
+    N = 352
+    x, w = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.05, 2)
+    ops.set_gemm_variant(8)
+    try:
+        if fp8:
+            q, sc = quantize_fp8_rows(w.float())
+            got = ops.linear_w8(x, ops.quantize_fp8(w.float())[0], sc, None, ops.EPI_SWIGLU)
+            w = dequantize_fp8_rows(q, sc)
+        else:
+            got = ops.linear(x, ops.pack_weight(w), None, ops.EPI_SWIGLU, packed_shape=(N, K))
+    finally:
+        ops.set_gemm_variant(ops.GEMM_DEFAULT_VARIANT)
+    ref, atol = _ref_linear(x, w, None, ops.EPI_SWIGLU, with_atol=True)
+    assert_bf16_close(got, ref, f"gemm_tall_quarters[{M}x{K},fp8={fp8}]", max_ulp=1.0, max_frac=5e-3, atol=atol)
+    if not fp8:
+        assert ops.gemm_plan(M, 33280, K, ops.EPI_SWIGLU)[0] == 448
+    elif K == 64:
+        before = ops.launch_counts()["gemm_tall"]
+        ops.linear_w8(x, torch.zeros(33280, K, dtype=torch.uint8, device=dev), torch.ones(33280, device=dev), None, ops.EPI_SWIGLU)
+        assert ops.launch_counts()["gemm_tall"] - before == (M > 128)
+
+
 @pytest.mark.parametrize("M", [256 + 16, 272 + 7, 288, 2 * 256 + 1, 2 * 288 - 16, 3088, 1131])
 @pytest.mark.parametrize("N,K,epi", [(512, 256, 0), (768, 192, 3), (3584, 1024, 4)])
 def test_gemm_variable_height_tiles_are_bit_identical_to_the_256_row_tiles(dev, M, N, K, epi):

@@ -1,6 +1,6 @@
 #!/usr/bin/env python
 """Times the LLM prefill gate/up GEMM of ONE streaming chunk (M = 386, N = 2 x 18944, K = 3584, SwiGLU epilogue) with the tall kernel
-(default choice) and the 128 x 256 tiles (variant 4), hipEvents over rotating weight buffers.  LCC_TALL_SCHED=1: pinned schedule."""
+(default choice) and the 128 x 256 tiles (variant 4), hipEvents over rotating weight buffers."""
 import json
 import os
 import sys
@@ -28,6 +28,6 @@ for M in (386, 300, 448):
         e1.record()
         torch.cuda.synchronize()
         us = e0.elapsed_time(e1) * 1e3 / n
-        print(json.dumps(dict(M=M, kernel=name, sched=os.environ.get("LCC_TALL_SCHED", "0"), us=round(us, 2),
+        print(json.dumps(dict(M=M, kernel=name, us=round(us, 2),
                               pflops=round(2.0 * M * 2 * I * H / us / 1e9, 4))))
 ops.set_gemm_variant(ops.GEMM_DEFAULT_VARIANT)

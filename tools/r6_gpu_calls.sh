@@ -80,8 +80,8 @@ attn_tps)      # key tiles per split of the decode attention with the split cap 
   for cfg in "4 64" "2 128" "3 128" "4 64" "2 128" "3 128"; do set -- $cfg
     LCC_ATTN_TPS=$1 LCC_ATTN_MAXSPLIT=$2 python bench.py --steps 3 --warmup 1 --no-prefetch $QUIET 2>/dev/null | step "tps=$1, maxsplit=$2" >> $O/attn_tps_maxsplit_ab.jsonl; done
   cat $O/attn_tps_maxsplit_ab.jsonl ;;
-tall)          # one-chunk GEMMs: tall kernel schedule A/B
-  for s in 0 1 2 0 1 2; do LCC_TALL_SCHED=$s python tools/r6_tall_sched.py "tall_sched$s" 2>/dev/null >> $O/m386_gemms_ab.jsonl; done; cat $O/m386_gemms_ab.jsonl ;;
+tall)          # one-chunk GEMMs
+  python tools/r6_tall_sched.py 2>/dev/null >> $O/m386_gemms_ab.jsonl; cat $O/m386_gemms_ab.jsonl ;;
 rccl)          # can RCCL run two ranks on the box's one GPU?
   timeout 150 python tools/r6_rccl_same_device_probe.py | tee $O/rccl_probe.json ;;
 *) echo "recipes: tier bench pmc pmc_gemv attn_map attn_rowmajor attn_vgprform attn_tall tower_prof pingpong pmc_attn attn_direct attn_tps tall rccl" ;;

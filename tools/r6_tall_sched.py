@@ -1,7 +1,6 @@
 #!/usr/bin/env python
-"""Round-6 A/B target: the one-chunk (M = 386) LLM GEMMs timed back to back with hipEvents over rotating weights -- gate/up on the tall kernel under
-LCC_TALL_SCHED = 0 / 1 / 2 (the pinned schedules were last measured BEFORE the LDS-DMA went into inline asm: round 5 changed what hipcc's waitcnt
-pass sees), and the three split-K projections.  argv[1] = tag; one JSON line per GEMM."""
+"""Round-6 A/B target: the one-chunk (M = 386) LLM GEMMs timed back to back with hipEvents over rotating weights -- gate/up on the tall kernel and
+the three split-K projections.  argv[1] = tag; one JSON line per GEMM."""
 import json
 import os
 import sys
