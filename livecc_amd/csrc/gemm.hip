@@ -957,8 +957,8 @@ __global__ __launch_bounds__(512) void gemm_big_kernel(
 //
 // Rows: 256, 192, 160 or 128 (BM), or VARIABLE (BM 272): 16, 17 or 18 row fragments a tile.  M is whatever the turn packs: 8 co-scheduled streaming chunks are 8 x 386 =
 // 3088 rows = 12 x 256 + 16, so a 13th row tile of 256 would multiply 16 live rows and 13 x 148 = 1924 blocks be 7.5 rounds of the 256 CUs.  The F = ceil(M / 16)
-// fragments are dealt out over floor(F / 16) tiles, the first F % tiles of them one fragment taller (3088 rows: 11 tiles of 256 + one of 272 = 6.94 rounds; 1131
-// rows: 4 tiles of 288 / 272; 9048: 35 tiles instead of 36); the two wave rows split f fragments f / 2 : f - f / 2, one copy of the k loop per count.
+// fragments are dealt out over F / 18 to F / 16 tiles (vh_tiles), the first F % tiles of them one fragment taller (3088 rows: 11 tiles of 256 + one of 272 = 6.94 rounds;
+// 3436: 12 of 288 / 272); the two wave rows split f fragments f / 2 : f - f / 2, one copy of the k loop per count.
 // A slot without rows (192, 160 and variable rows) copies one 16-byte piece into a scratch: the stream of pieces is the same in every wave.
 // Bits as gemm_big_kernel (same k order per output).  bf16 weights.  The vision q|k|v epilogues (gemm_vit_kernel) run a tile a block: their rotation tables need
 // the stages (15,840 x 3840, K 1280: 182 -> 172 us).  Grid: at most 256 blocks over all splits (one a compute unit), or the cap.
@@ -1667,15 +1667,30 @@ static void launch_vit(const GemmArgs& a, int rows, hipStream_t st) {
   else if (rows == 192) launch_vit_rows<192, EPI>(a, st);
   else launch_vit_rows<128, EPI>(a, st);
 }
-// variable-height row tiles (gemm_vh_kernel): tiles_m = floor(F / 16) row tiles for F = ceil(M / 16) row fragments (small class: F / 8)
+// variable-height row tiles: floor(F / 16) row tiles or fewer for F = ceil(M / 16) row fragments (small class: F / 8)
 static bool vh_legal(const GemmArgs& a, bool small = false) {
   const int F = (a.M + 15) >> 4, t = F >> (small ? 3 : 4);
   return a.w_packed && !a.w_fp8 && (a.K % 64) == 0 && t >= 1 && F <= (small ? 9 : 18) * t && (a.N & 15) == 0 && walk_offsets_fit(a);
 }
+// Row tiles of an automatic choice: F / 18 to F / 16.  A tile of 17 / 18 fragments takes 1.08 / 1.17 of a 256-row tile's time (gate/up of 3,436 rows: 12 tiles of
+// 17.9 fragments are 6.94 rounds, 642 us; 13 of 16.5 are 7.52, 663)
+struct VhTiles { int tiles_m; float score; };
+static VhTiles vh_tiles(int M, int N, int S) {
+  const int F = (M + 15) >> 4;
+  VhTiles best{F >> 4, 0.f};
+  if (g_gemm_variant == 14) return best;
+  for (int t = (F + 17) / 18; t <= F >> 4; ++t) {
+    const int top = (F + t - 1) / t;
+    const long blocks = (long)t * ((N + 255) / 256) * S;
+    const float score = (top == 16 ? 1.f : top == 17 ? 0.985f : 0.96f) * (float)M / (float)(t * top * 16) * (float)blocks / (float)((blocks + 255) / 256 * 256);
+    if (score > best.score) best = {t, score};
+  }
+  return best;
+}
 template <int EPI>
 static void launch_vh(const GemmArgs& a, hipStream_t st) {
-  const int F = (a.M + 15) >> 4, tiles_m = F >> 4, tiles_n = (a.N + 255) / 256;
   const int nkt = a.K / 64, S = (EPI == EPI_PARTIAL) ? a.nsplit : 1;
+  const int tiles_m = vh_tiles(a.M, a.N, S).tiles_m, tiles_n = (a.N + 255) / 256;
   constexpr size_t lds = Walk<272, EPI>::LDS;      // stages, scratch, epilogue: 156,672 B
   static DeviceOnce attr_set;   // per instantiation
   if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_walk_vh_kernel<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -1748,9 +1763,14 @@ static float tile_score(int M, int N, int S, int BM, int BN, int slots, float ef
 }
 // BM 192 (round 4, bf16 weights): a 256-row tile leaves the chip partly idle whenever (M / 256) x (N / 256) falls just short of a round --
 // the o / down projections of 8 co-scheduled chunks are M = 3088 x N = 3584 = 13 x 14 = 182 blocks on 256 CUs (29 % idle); 17 x 14 = 238
-// blocks of 192 rows fill 93 % of one round at 3/4 of the tile time.  The tile moves 17 % more L2 -> LDS bytes per flop (efficiency 0.93).
-// Variable-height tiles (round 5; returned as 272): floor(F / 16) row tiles of 16-18 fragments -- scored with every tile as tall as the
-// tallest (a 17-fragment tile costs 17/16 of a 256-row tile on every SIMD), no ragged tile, the 256-row tile's efficiency.
+// blocks of 192 rows fill 93 % of one round at 3/4 of the tile time.
+// Variable-height tiles (returned as 272): F / 18 to floor(F / 16) row tiles of 16-18 fragments (vh_tiles) -- scored with every tile as tall as the
+// tallest, no ragged tile.
+// Efficiencies against 256 rows: a round of [37888, 3584] takes 52 / 58 / 67 / 77.5 us with 128 / 160 / 192 / 256 rows and 82-85 / 91 with 17 / 18 fragments: 0.75, 0.84,
+// 0.87, 1, 0.985, 0.96 (short tiles move more bytes from the L2 per product, and from 0.85 of the chip on power is the limit).  192 rows at 0.93 and 160 at 0.90 had
+// been measured on tiles whose waves kept in step, us there / here: 3580 x 37888 722 / 701, 5000 x 3584, K 18944 590 / 464, 3994 x 17920, K 1536 181 / 169, 11648 x 1536,
+// K 8960 278 / 225, 3994 x 4608 113 / 96, 1600 x 37888 372 / 341, 4096 x 14336 326 / 309; the worst of 28 shapes whose tile changed 1950 / 1973.
+// Slabs and their count (gemm_tiled_num_splits) keep the older figures: one round at most, the ends of the tiles as long as their loops.
 // LCC_GEMM_VH=0: rounds 2-4 tile choice.
 // score: of the chosen tile, automatic choice only.  wide_only: 256-column tiles as they stand against a 64 x 128 one that dequantises fp8 weights first (gemm_w8)
 static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr, bool wide_only = false) {
@@ -1763,13 +1783,13 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr, bool 
   if (g_gemm_variant == 15) return (a.partial != nullptr && vh_small_shape(a.M, a.K) && vh_legal(a, true)) ? 144 : 128;
   if (g_gemm_variant == 16) return wide_only ? 128 : 129;
   if (g_gemm_variant != 2) return 0;
+  const bool slabs = a.partial != nullptr || score != nullptr;
   const float s256 = tile_score(a.M, a.N, S, 256, 256, 256, 1.0f, true);
   static const int allow192 = [] { const char* v = getenv("LCC_GEMM_192"); return v ? atoi(v) : 1; }();     // A/B: 0 = round-3 tile choice
-  const float s192 = (a.w_fp8 || !allow192) ? 0.f : tile_score(a.M, a.N, S, 192, 256, 256, 0.93f, true);
+  const float s192 = (a.w_fp8 || !allow192) ? 0.f : tile_score(a.M, a.N, S, 192, 256, 256, slabs ? 0.93f : 0.88f, true);
   // BM 160 (bf16 weights): where 192 rows start a last round that is mostly empty.  The vision proj / fc2 of 15,840 rows are 83 x 5 tiles of 192 rows =
   // 1.62 rounds; 99 x 5 of 160 fill 1.93 at 5/6 of the time each: proj 55.7 -> 52.1 us, fc2 201 -> 178.
-  // 1000 / 2100 x 17920, K 1536 with SwiGLU 63.6 -> 58.4 / 117.5 -> 111.3.
-  const float s160 = (a.w_fp8 || !allow192) ? 0.f : tile_score(a.M, a.N, S, 160, 256, 256, 0.90f, false);
+  const float s160 = (a.w_fp8 || !allow192) ? 0.f : tile_score(a.M, a.N, S, 160, 256, 256, slabs ? 0.90f : 0.86f, false);
   const float s128 = tile_score(a.M, a.N, S, 128, 256, 256, a.w_fp8 ? 0.85f : 0.82f, true);
   // gemm_mid_kernel: 0.38 / 0.52 us a step of 64 x 128 / 128 x 128 against 0.85 of 128 x 256, one tile a compute unit at a time (two 64-row
   // tiles side by side take twice as long).  Returned as 0 / 129.  The 128-row form wins where its blocks fill one round and the 64-row
@@ -1781,9 +1801,7 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr, bool 
   if (score) *score = std::max(std::max(std::max(s256, s192), std::max(s160, s128)), std::max(s128m, s64));
   static const int allow_vh = [] { const char* v = getenv("LCC_GEMM_VH"); return v ? atoi(v) : 1; }();
   if (allow_vh && vh_legal(a) && (((a.M + 15) >> 4) & 15) != 0) {      // F % 16 == 0: the 256-row tiles are the same thing
-    const int F = (a.M + 15) >> 4, t = F >> 4, maxf = (F + t - 1) / t;
-    const long blocks = (long)t * ((a.N + 255) / 256) * S;
-    const float svh = (float)a.M / (float)(t * maxf * 16) * (float)blocks / (float)((blocks + 255) / 256 * 256);
+    const float svh = vh_tiles(a.M, a.N, S).score;
     if (svh > s256 && svh > s192 && svh > s160 && svh > s128 && svh > s128m && svh > s64) {
       if (score) *score = svh;
       return 272;

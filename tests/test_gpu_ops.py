@@ -297,6 +297,24 @@ def test_gemm_128_column_tiles_give_the_slabs_of_the_128_row_tiles(dev, M, N, K,
     assert torch.equal(got, ref)
 
 
+@pytest.mark.parametrize("M,N,K,epi", [(3436, 5120, 128, 0), (3425, 5104, 64, 3), (3441, 10240, 128, 4), (2577, 7136, 192, 1)])
+def test_gemm_fewer_and_taller_variable_height_tiles_give_the_same_bits(dev, M, N, K, epi):
+    """Where the row tiles of 16 fragments start another round, F / 18 of them are taken: 215, 216 and 162 fragments in 12, 12 and 9 tiles of 17 and 18
+    where floor(F / 16) is 13 / 13 / 10; a partial last fragment, a ragged last column tile."""
+    from livecc_amd import ops
+    x, w, b = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.05, 2), _rand((N,), dev, 0.1, 3)
+    res = _rand((M, N), dev, 1.0, 4) if epi == 3 else None
+    wp = ops.pack_weight(w)
+    assert ops.gemm_plan(M, N, K, epi)[0] == 272
+    got = ops.linear(x, wp, None if epi == 4 else b, epi, res, packed_shape=(N, K))
+    try:
+        ops.set_gemm_variant(3)
+        ref = ops.linear(x, wp, None if epi == 4 else b, epi, res, packed_shape=(N, K))
+    finally:
+        ops.set_gemm_variant(ops.GEMM_DEFAULT_VARIANT)
+    assert torch.equal(got, ref), f"{int((got != ref).sum())} of {got.numel()} outputs differ from the 256-row tiles"
+
+
 @pytest.mark.parametrize("M,N,K,S", [(386, 3584, 18944, 6), (386, 4608, 3584, 4), (386, 3584, 3584, 6), (400, 3600, 1024, 2), (130, 512, 512, 2),
                                      (272, 1024, 1024, 4), (144, 256, 4096, 8), (391, 1536, 8960, 5)])
 def test_gemm_small_variable_height_tiles_give_the_slabs_of_the_128_row_tiles(dev, M, N, K, S):
