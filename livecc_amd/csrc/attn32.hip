@@ -77,6 +77,8 @@ LCC_DEVICE void unrolled(F&& f) { unrolled_of(f, std::make_integer_sequence<int,
 // also shift by a chunk every four rows (their DMA instruction).
 //   mlim: tiles reaching past it need the mask (causal diagonal / end of the key range); lim: this lane's effective key limit.
 //
+// Fragments are read four MFMAs ahead, at 128 channels five, as many as there are registers for: 4,096 rows on 8k keys 631 -> 626 us, 8 x 386 on 1.1k 90.6 -> 88.9,
+// 1,131 rows 36.2 -> 35.3; six 629, 89.0 and 35.3, three 638, 90.2 and 36.0.  At 80 channels five and six are no faster (18 slices of 880 123 / 124 / 127).
 // Measured and not taken: the two waves of a SIMD in opposite phases (matrix work of one beside the softmax of the other): 11 % slower than the
 // instruction-by-instruction interleave; all fragments of a region read a region ahead: 64 registers, spills.
 // LM (the tower kernel): the softmax denominator comes out of the P . V MFMAs -- the V^T rows 80..95 of the third d-tile do not exist at d = 80 and
@@ -114,7 +116,7 @@ template <int D, int DV, int NWAVE, bool LM, bool BIAS = false, bool CLAMP = fal
 LCC_DEVICE void attn32_key_loop(unsigned char* alds, const Kv32& kv, const u32x4 (&qf)[D / 16], int tb, int te, int mlim, int lim, float scale_log2e,
                                 bool active, int lane, int wave, int hh, f32x16 (&o)[(DV + 31) / 32], float& m_run, float& l_run, float slope = 0.f, int pos = 0) {
   using Im = Attn32Image<D, DV>;
-  constexpr int KP = D / 16, DT = Im::DT, VP = 2 * DT, NP = KP + VP, FRAG_LEAD = 4;
+  constexpr int KP = D / 16, DT = Im::DT, VP = 2 * DT, NP = KP + VP, FRAG_LEAD = D == 128 ? 5 : 4;
   using Steps = Attn32Steps<VP, KP>;
   constexpr int NPD = Im::NPD, PWP = (2 * NPD + NWAVE - 1) / NWAVE, PK = (Im::KPD + NWAVE - 1) / NWAVE;     // DMA pieces of a wave: a pair; K of one tile
   m_run = -INFINITY;
