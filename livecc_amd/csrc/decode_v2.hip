@@ -79,11 +79,11 @@ LCC_DEVICE u32x4 norm_frag(u32x4 hv, u32x4 wv, float r) {
 
 // Occupancy decides whether the whole grid is resident at once (one round) or a few blocks start a second round that pays the
 // prologue latency again behind an almost idle memory system (7B shapes): gate/up = 1184 blocks of 4 waves need 5 blocks per CU
-// (<= 96 VGPRs; at 97 the kernel ran 1024 + 160); q/k/v = 288 blocks of 8 waves need 2 per CU (<= 128 VGPRs; at 140: 256 + 32).
+// (<= 96 VGPRs) with one chunk a stage; with two, four blocks and a short second round are faster (dgemv_norm_swiglu); q/k/v = 288 blocks of 8 waves need 2 per CU (<= 128 VGPRs; at 140: 256 + 32).
 // MR = activation rows (streams) whose RMSNorm statistic every wave reduces in the prologue: 2 (the engine's v2 batches) or 4.
-template <int NTILE, int PRO, int EPI, int NW, int MR>
+template <int NTILE, int PRO, int EPI, int NW, int UNR, int MR>
 constexpr int dgemv_min_waves_per_simd() {
-  return MR > 2 ? 1 : ((NTILE == 2 && PRO == DG_PRO_NORM && NW == 4) ? 5 : ((EPI == DG_EPI_ROPE && NW == 8) ? 4 : 1));
+  return MR > 2 ? 1 : ((NTILE == 2 && PRO == DG_PRO_NORM && NW == 4) ? (UNR == 1 ? 5 : 4) : ((EPI == DG_EPI_ROPE && NW == 8) ? 4 : 1));
 }
 
 // US (row-scaled products): the activations are u = bf16(w * h) of the RMSNorm's weight and the residual row, and the row's 1 / rms multiplies the
@@ -449,7 +449,7 @@ LCC_DEVICE void dgemv_body(const DgArgs& a, const DgChain& ch, const int bid, f3
 }
 
 template <int NTILE, int PRO, int EPI, int NW, int UNR, int MR = 4, bool W8 = false>
-__global__ __launch_bounds__(NW * 64, (dgemv_min_waves_per_simd<NTILE, PRO, EPI, NW, MR>())) void dgemv_kernel(DgArgs a) {
+__global__ __launch_bounds__(NW * 64, (dgemv_min_waves_per_simd<NTILE, PRO, EPI, NW, UNR, MR>())) void dgemv_kernel(DgArgs a) {
   __shared__ f32x4 red[NW - 1][NTILE][64];
   extern __shared__ __attribute__((aligned(16))) bf16_t s_x[];   // PRO_NORM: M * K bf16 (dynamic: 7 KB for one stream at 7B)
   dgemv_body<NTILE, PRO, EPI, NW, UNR, MR, DG_CHAIN_NONE, W8>(a, DgChain{nullptr, 0u, nullptr, 0}, blockIdx.x, red, s_x);
@@ -861,10 +861,15 @@ int dgemv_down_qkv(const DgArgs& down, const DgArgs& qkv, unsigned* flag, unsign
 // [RMSNorm] gate/up Linear [SwiGLU]
 int dgemv_norm_swiglu(const DgArgs& a, hipStream_t st) {
   if (int rc = dg_check(a, DG_PRO_NORM, DG_EPI_SWIGLU)) return rc;
+  // Weight chunks a stage: two where a unit's blocks are one at most, or more than three, and a wave has eight or more of them (the norm goes on under the
+  // first two stages); between, their bytes only wait for one another.  us, one / two: [37888, 3584] 48.7 / 47.3, [59136, 8192] 157 / 155, [28672, 2048] 23.5 / 23.2, [4736, 3584]
+  // 13.0 / 10.7;  [9472, 3584] 16.5 / 16.8, [9472, 8192] 32.7 / 34.4, [18944, 3584] 28.0 / 28.2, [17920, 1536] 13.2 / 13.4, [8960, 1536] 8.2 / 9.1
+  const bool two = a.K >= 2048 && (a.N > 768 * 32 || a.N <= 256 * 32);
   hipEvent_t ev0 = g_swiglu_ev0, ev1 = g_swiglu_ev1;
   g_swiglu_ev0 = g_swiglu_ev1 = nullptr;
   if (ev0 != nullptr && ev1 != nullptr && a.wscale == nullptr && a.M <= 2) {      // the profiled launch of the bf16 one-/two-stream kernel
-    hipExtLaunchKernelGGL((dgemv_kernel<2, DG_PRO_NORM, DG_EPI_SWIGLU, 4, 1, 2>), dim3(a.N / 32), dim3(256), (uint32_t)((size_t)a.M * a.K * 2), st, ev0, ev1, 0u, a);
+    if (two) hipExtLaunchKernelGGL((dgemv_kernel<2, DG_PRO_NORM, DG_EPI_SWIGLU, 4, 2, 2>), dim3(a.N / 32), dim3(256), (uint32_t)((size_t)a.M * a.K * 2), st, ev0, ev1, 0u, a);
+    else hipExtLaunchKernelGGL((dgemv_kernel<2, DG_PRO_NORM, DG_EPI_SWIGLU, 4, 1, 2>), dim3(a.N / 32), dim3(256), (uint32_t)((size_t)a.M * a.K * 2), st, ev0, ev1, 0u, a);
     return 0;
   }
   if (ev0 != nullptr && ev1 != nullptr) {      // other instantiations: bracket with plain records (the events must be recorded either way)
@@ -878,7 +883,8 @@ int dgemv_norm_swiglu(const DgArgs& a, hipStream_t st) {
     else dgemv_kernel<2, DG_PRO_NORM, DG_EPI_SWIGLU, 4, 2, 4, true><<<dim3(a.N / 32), dim3(256), (size_t)a.M * a.K * 2, st>>>(a);
     return 0;
   }
-  if (a.M <= 2) dgemv_kernel<2, DG_PRO_NORM, DG_EPI_SWIGLU, 4, 1, 2><<<dim3(a.N / 32), dim3(256), (size_t)a.M * a.K * 2, st>>>(a);
+  if (a.M <= 2 && two) dgemv_kernel<2, DG_PRO_NORM, DG_EPI_SWIGLU, 4, 2, 2><<<dim3(a.N / 32), dim3(256), (size_t)a.M * a.K * 2, st>>>(a);
+  else if (a.M <= 2) dgemv_kernel<2, DG_PRO_NORM, DG_EPI_SWIGLU, 4, 1, 2><<<dim3(a.N / 32), dim3(256), (size_t)a.M * a.K * 2, st>>>(a);
   else dgemv_kernel<2, DG_PRO_NORM, DG_EPI_SWIGLU, 4, 1, 4><<<dim3(a.N / 32), dim3(256), (size_t)a.M * a.K * 2, st>>>(a);
   return 0;
 }

@@ -34,6 +34,16 @@ def test_norm_swiglu_gemv(dev, M, N, K):
     assert_bf16_close(got, ref, f"dgemv_norm_swiglu[{M}x{N}x{K}]", max_ulp=1.0, max_frac=1e-2, atol=atol)
 
 
+@pytest.mark.parametrize("M,K", [(1, 2048), (2, 2112), (1, 2240), (2, 3584), (1, 8192)])
+def test_norm_swiglu_gemv_chunks_a_stage_give_the_same_bits(dev, M, K):
+    """Two weight chunks a stage (at most 8,192 rows, or more than 24,576) and one (between): the first rows of all three are the same weights, each wave adds
+    its chunks up in the same order, so the outputs agree bit for bit; odd counts of chunks."""
+    from livecc_amd import ops
+    h, w, nw = _rand((M, K), dev, 2.0, 1), _rand((24608, K), dev, 0.03, 2), _rand((K,), dev, 1.0, 3)
+    out = [ops.dgemv_norm_linear(ops.pack_weight(w[:n].contiguous()), h, ops.tile_stats(h), nw, 1e-6, (n, K), swiglu=True) for n in (96, 8224, 24608)]
+    assert torch.equal(out[0], out[1][:, :48]) and torch.equal(out[1], out[2][:, :4112])
+
+
 @pytest.mark.parametrize("M", [1, 3])
 @pytest.mark.parametrize("N,K", [(152064, 3584), (2048, 256), (8192, 896)])
 def test_norm_linear_gemv_lm_head(dev, M, N, K):
