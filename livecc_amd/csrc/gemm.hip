@@ -6,7 +6,7 @@
 //  * gemm_walk_kernel    : M >= 17, packed W, K % 64 == 0 (LLM prefill, ViT).  MFMA-bound.  8 waves, BM x 256 x 64 tile
 //                          (BM 256 / 192 / 160 / 128), LDS-DMA for both operands; one block a compute unit, the DMA ring runs on from tile to tile.
 //  * gemm_vit_kernel     : the same pipeline, a tile a block, with the vision q|k|v epilogues.
-//  * gemm_big_kernel     : the same tiles one a block, both waves of a SIMD in step: fp8-e4m3 W converted after the LDS read; 128-row tiles of one round.
+//  * gemm_big_kernel     : the same tiles one a block, both waves of a SIMD in step: 128-row tiles of one round.
 //  * gemm_walk_vh_kernel : the walk over row tiles of 256 / 272 / 288 rows (no ragged last row tile).
 //  * gemm_vh_kernel      : row tiles of 128 / 144 rows, split-K slabs of one streaming chunk.
 //  * gemm_tall_kernel    : one block row covers all of M (up to 448 rows: gate/up of one streaming chunk or of a few short ones).
@@ -960,17 +960,18 @@ __global__ __launch_bounds__(512) void gemm_big_kernel(
 // fragments are dealt out over F / 18 to F / 16 tiles (vh_tiles), the first F % tiles of them one fragment taller (3088 rows: 11 tiles of 256 + one of 272 = 6.94 rounds;
 // 3436: 12 of 288 / 272); the two wave rows split f fragments f / 2 : f - f / 2, one copy of the k loop per count.
 // A slot without rows (192, 160 and variable rows) copies one 16-byte piece into a scratch: the stream of pieces is the same in every wave.
-// Bits as gemm_big_kernel (same k order per output).  bf16 weights.  The vision q|k|v epilogues (gemm_vit_kernel) run a tile a block: their rotation tables need
+// Bits as gemm_big_kernel (same k order per output).  fp8 weights (W8) are converted behind the LDS read, beside the other wave's MFMAs; [37888, 3584] with SwiGLU,
+// us, in step and 128 or 256 rows -> here: 514 rows 175 -> 145, 772 274 -> 196, 1158 293 -> 265, 1544 447 -> 378, 3088 696 -> 628; [3584, 18944], 2316 rows 384 -> 286.  The vision q|k|v epilogues (gemm_vit_kernel) run a tile a block: their rotation tables need
 // the stages (15,840 x 3840, K 1280: 182 -> 172 us).  Grid: at most 256 blocks over all splits (one a compute unit), or the cap.
-template <int BM, int EPI>
+template <int BM, int EPI, bool W8 = false>
 struct Walk {
   static constexpr bool VH = BM == 272;
   static constexpr int ROWS = VH ? 288 : BM, MT = VH ? 8 : BM / 32, MTX = VH ? 9 : MT;             // row fragments of a wave (variable rows: 8 or 9)
   static constexpr int H0 = VH ? 4 : (MT + 1) / 2, H1 = MTX - H0;                                  // of phase 0, at most of phase 1
-  static constexpr int P0 = (4 * H0 + 7) / 8, P1 = (4 * H1 + 7) / 8, PB = 4, G = P0 + PB + P1;     // a wave's pieces of a k-tile: rows of phase 0, weights; rows of phase 1
+  static constexpr int P0 = (4 * H0 + 7) / 8, P1 = (4 * H1 + 7) / 8, PB = W8 ? 2 : 4, G = P0 + PB + P1;     // a wave's pieces of a k-tile: rows of phase 0, weights; rows of phase 1
   static constexpr bool SPARE = VH || (4 * H0) % 8 != 0 || (4 * H1) % 8 != 0;                      // slots without rows
   static constexpr int NSTAGE = BM == 128 ? 3 : 2;
-  static constexpr int A_UNITS = ROWS * 8, STAGE = A_UNITS + 2048;                                 // 16-byte units
+  static constexpr int A_UNITS = ROWS * 8, STAGE = A_UNITS + PB * 512;                             // 16-byte units
   static constexpr int EGR = BM >= 160 && !VH && EPI != EPI_GELU_ERF ? 2 : 1;                      // row tiles of an epilogue group: 2 KB of LDS a wave each (the erf: registers)
   static constexpr unsigned SCRATCH = (unsigned)NSTAGE * STAGE * 16u, EPILOGUE = SCRATCH + (SPARE ? 1024u : 0u);
   static constexpr size_t LDS = EPILOGUE + 8 * EGR * 2048;
@@ -979,13 +980,14 @@ struct Walk {
   static_assert(LDS <= 163840, "LDS of a compute unit");
   static_assert(LATER + NSTORE <= 63, "vmcnt");
 };
-template <int BM, int EPI>
+template <int BM, int EPI, bool W8 = false>
 LCC_DEVICE void gemm_walk_body(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
     const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual, int ldr,
     bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n,
-    float* __restrict__ partial, int kt_per_split, int raster, const VitQkvEpi& vq = VitQkvEpi(), int one_m = 0, int one_n = 0) {
-  using S = Walk<BM, EPI>;
+    float* __restrict__ partial, int kt_per_split, int raster, const VitQkvEpi& vq = VitQkvEpi(), int one_m = 0, int one_n = 0,
+    const float* __restrict__ wscale = nullptr) {
+  using S = Walk<BM, EPI, W8>;
   constexpr bool VIT = EPI == EPI_VIT_QK || EPI == EPI_VIT_V;      // the tile (one_m, one_n) alone: the rotation's tables take the stages
   constexpr int BN = 256, BK = 64, NT = 4, NSTAGE = S::NSTAGE, STAGE = S::STAGE, H0 = S::H0, P0 = S::P0, P1 = S::P1, PB = S::PB, LATER = S::LATER;
   extern __shared__ __attribute__((aligned(16))) u32x4 dsmem[];
@@ -1026,7 +1028,7 @@ LCC_DEVICE void gemm_walk_body(
   // A slot's rows: 8 of the first wave row's part, behind them the second's; none: one 16-byte piece into the scratch
   struct Way { int vb, kt; const bf16_t* a; };
   Way w0 = {vb0, kt0, nullptr}, w1 = w0;
-  const bf16_t* bbase[PB / 2];
+  const bf16_t* bbase[2];
   unsigned off0[P0], off1[P1], dst0[P0], dst1[P1];
   const unsigned swz = ((lane & 7) ^ (lane >> 3)) << 4, row_bytes = (unsigned)(lda * 2);
   auto slot_row = [&](int p, int from, int n_first, int n_second, int row1) { return p < n_first ? from + p * 8 : p < n_first + n_second ? row1 + from + (p - n_first) * 8 : -1; };
@@ -1039,7 +1041,7 @@ LCC_DEVICE void gemm_walk_body(
     tile_of(w0.vb, m0, n0, row1, rows);
     w0.a = A + (size_t)m0 * lda;
 #pragma unroll
-    for (int q = 0; q < PB / 2; ++q) bbase[q] = W + (size_t)min((n0 >> 4) + wave * (PB / 2) + q, nfrag - 1) * K32 * 512;
+    for (int q = 0; q < 2; ++q) bbase[q] = W + (size_t)min((n0 >> 4) + wave * 2 + q, nfrag - 1) * (W8 ? K >> 6 : K32) * 512;
 #pragma unroll
     for (int q = 0; q < P0; ++q) slot(slot_row(wave * P0 + q, 0, 2 * H0, 2 * H0, row1), m0, off0[q], dst0[q]);
   };
@@ -1061,7 +1063,7 @@ LCC_DEVICE void gemm_walk_body(
 #pragma unroll
     for (int q = 0; q < P0; ++q) glds16_base(w0.a + (size_t)w0.kt * BK, off0[q], to(stage, dst0[q]));
 #pragma unroll
-    for (int q = 0; q < PB; ++q) glds16_base(bbase[q >> 1] + (size_t)w0.kt * 1024 + (q & 1) * 512, lane * 16u, lds0 + stage + (S::A_UNITS + (wave * PB + q) * 64) * 16u);
+    for (int q = 0; q < PB; ++q) glds16_base(W8 ? bbase[q] + (size_t)w0.kt * 512 : bbase[q >> 1] + (size_t)w0.kt * 1024 + (q & 1) * 512, lane * 16u, lds0 + stage + (S::A_UNITS + (wave * PB + q) * 64) * 16u);
     advance(w0, point0);
   };
   auto issue1 = [&](unsigned stage) {
@@ -1081,14 +1083,14 @@ LCC_DEVICE void gemm_walk_body(
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LATER) : "memory");
   __builtin_amdgcn_s_barrier();
   if (wm) __builtin_amdgcn_s_barrier();               // the second wave of a SIMD: one slot behind
-  const int boff = S::A_UNITS + (wn * NT * 2) * 64 + lane;
+  const int boff = S::A_UNITS + (wn * NT * (W8 ? 1 : 2)) * 64 + lane;
   int st = 0;                      // stage of the k-tile that is multiplied
   bool all_stored = false;         // the last epilogue issued NSTORE stores in this wave
   auto run = [&](auto mt_c, int m0, int n0, int my_row0) {      // one tile
     constexpr int MTW = decltype(mt_c)::value, MA = MTW > 0 ? MTW : 1, R0 = MTW > 0 ? H0 : 0, R1 = MTW - R0, RF = R0 > R1 ? R0 : R1;
     int aoff[2];
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) aoff[kk] = (my_row0 + li) * 8 + ((kk * 4 + g) ^ (li & 7));
+    for (int kk = 0; kk < 2; ++kk) aoff[kk] = (my_row0 + li) * 8 + ((W8 ? g * 2 + kk : kk * 4 + g) ^ (li & 7));
     f32x4 acc[MA][NT];
 #pragma unroll
     for (int i = 0; i < MA; ++i)
@@ -1118,10 +1120,20 @@ LCC_DEVICE void gemm_walk_body(
       const unsigned cur = (unsigned)(st * STAGE) * 16u, before = (unsigned)((st == 0 ? NSTAGE - 1 : st - 1) * STAGE) * 16u;
       st = st == NSTAGE - 1 ? 0 : st + 1;
       if constexpr (MTW > 0) {
+        if constexpr (W8) {
+#pragma unroll
+          for (int j = 0; j < NT; ++j) {
+            const u32x4 raw = s[boff + j * 64];
+            fb[0][j] = fp8x8_to_bf16x8(raw[0], raw[1]);
+            fb[1][j] = fp8x8_to_bf16x8(raw[2], raw[3]);
+          }
+        }
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
+          if constexpr (!W8) {
 #pragma unroll
-          for (int j = 0; j < NT; ++j) fb[kk][j] = as_bf16x8(s[boff + (j * 2 + kk) * 64]);
+            for (int j = 0; j < NT; ++j) fb[kk][j] = as_bf16x8(s[boff + (j * 2 + kk) * 64]);
+          }
 #pragma unroll
           for (int i = 0; i < R0; ++i) fa[kk][i] = as_bf16x8(s[aoff[kk] + i * 128]);
         }
@@ -1170,11 +1182,11 @@ LCC_DEVICE void gemm_walk_body(
       }
       return;
     } else if constexpr (MTW > 0 && EPI == EPI_PARTIAL) {
-      tile_slab_wide<MTW, NT, 1, S::EGR * 2>(acc, m0 + my_row0, n0 + wn * 64, l, M, N, partial, nullptr, elds);
+      tile_slab_wide<MTW, NT, 1, S::EGR * 2>(acc, m0 + my_row0, n0 + wn * 64, l, M, N, partial, W8 ? wscale : nullptr, elds);
     } else if constexpr (MTW > 0) {
       if (wide_rows<EPI>(C, ldc, bias, residual, ldr))
-        tile_epilogue_wide<EPI, MTW, NT, S::EGR>(acc, m0 + my_row0, n0 + wn * 64, l, bias, residual, ldr, C, ldc, M, N, nullptr, elds);
-      else tile_epilogue<EPI, MTW, NT>(acc, m0 + my_row0, n0 + wn * 64, (n0 + wn * 64) / 2, l & 15, l >> 4, bias, residual, ldr, C, ldc, M, N, partial, nullptr);
+        tile_epilogue_wide<EPI, MTW, NT, S::EGR>(acc, m0 + my_row0, n0 + wn * 64, l, bias, residual, ldr, C, ldc, M, N, W8 ? wscale : nullptr, elds);
+      else tile_epilogue<EPI, MTW, NT>(acc, m0 + my_row0, n0 + wn * 64, (n0 + wn * 64) / 2, l & 15, l >> 4, bias, residual, ldr, C, ldc, M, N, partial, W8 ? wscale : nullptr);
     }
     if (kt0 < nkt && wm == 1) slot_end();
   };
@@ -1191,11 +1203,11 @@ LCC_DEVICE void gemm_walk_body(
   if (!wm) __builtin_amdgcn_s_barrier();
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the copies behind the last tile: this block's LDS until they have landed
 }
-template <int BM, int EPI>
+template <int BM, int EPI, bool W8>
 __global__ __launch_bounds__(512) void gemm_walk_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias,
                                                         const bf16_t* __restrict__ residual, int ldr, bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m,
-                                                        int tiles_n, float* __restrict__ partial, int kt_per_split, int raster) {
-  gemm_walk_body<BM, EPI>(A, lda, W, bias, residual, ldr, C, ldc, M, N, K, tiles_m, tiles_n, partial, kt_per_split, raster);
+                                                        int tiles_n, float* __restrict__ partial, int kt_per_split, int raster, const float* __restrict__ wscale) {
+  gemm_walk_body<BM, EPI, W8>(A, lda, W, bias, residual, ldr, C, ldc, M, N, K, tiles_m, tiles_n, partial, kt_per_split, raster, VitQkvEpi(), 0, 0, wscale);
 }
 // the vision tower's q|k|v projection (EPI_VIT_QK, EPI_VIT_V; EPI_VIT_QKV: both, N = 3E and 2E % 256 == 0): a tile a block
 template <int BM, int EPI>
@@ -1640,16 +1652,16 @@ static void launch_big_s(const GemmArgs& a, hipStream_t st) {
 static bool walk_offsets_fit(const GemmArgs& a) { return (size_t)a.lda * 576 <= 0xffffffffu; }
 // blocks of one split: one a tile while all splits' tiles fit the chip at once, else as many as it has units for
 static unsigned walk_grid(long tiles, int S) { return tiles * S <= 256 ? capped_grid(tiles) : std::min(capped_grid(tiles), (unsigned)std::max(8, (256 / S) & ~7)); }
-template <int BM, int EPI>
+template <int BM, int EPI, bool W8>
 static void launch_walk(const GemmArgs& a, hipStream_t st) {
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + 255) / 256;
   const int nkt = a.K / 64, S = (EPI == EPI_PARTIAL) ? a.nsplit : 1;
-  constexpr size_t lds = Walk<BM, EPI>::LDS;      // 256 / 192 / 160 / 128 rows: 160 / 145 / 137 / 160 KB
+  constexpr size_t lds = Walk<BM, EPI, W8>::LDS;      // 256 / 192 / 160 / 128 rows: 160 / 145 / 137 / 160 KB; fp8 weights 128 / 113 / 105 / 112 KB
   static DeviceOnce attr_set;   // per instantiation
-  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_walk_kernel<BM, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_walk_kernel<BM, EPI, W8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   const unsigned grid = walk_grid((long)tiles_m * tiles_n, S);
-  gemm_walk_kernel<BM, EPI><<<dim3(grid, S), dim3(512), lds, st>>>(a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m,
-                                                                   tiles_n, a.partial, (nkt + S - 1) / S, raster_for(tiles_m));
+  gemm_walk_kernel<BM, EPI, W8><<<dim3(grid, S), dim3(512), lds, st>>>(a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m,
+                                                                       tiles_n, a.partial, (nkt + S - 1) / S, raster_for(tiles_m), a.wscale);
 }
 template <int BM, int EPI>
 static void launch_vit_rows(const GemmArgs& a, hipStream_t st) {
@@ -1715,16 +1727,16 @@ static void launch_big(const GemmArgs& a, hipStream_t st) {
   // bit-identical to the burst-behind-the-barrier order SCHED 1 -- tools/gemm_checksum.py -- and 1.6-3.3 % faster on the prefill
   // GEMMs, +0.6 / +0.8 % tokens/s at 1 / 8 streams, profiles/r03/gemm_sched_spread_dma.txt); LCC_GEMM_SCHED=1 restores SCHED 1
   static const int spread = [] { const char* v = getenv("LCC_GEMM_SCHED"); return (v && atoi(v) == 1) ? 0 : 1; }();
-  // fp8 weights: spread pieces on 256 rows (4096 x 3584, K 18944 415 -> 405 us, x 4608, K 3584 161 -> 156), a burst on 128 (386 x 37888 149 against 155)
-  if (a.w_fp8) launch_big_s<(BM == 192 || BM == 160 ? 256 : BM), EPI, (BM == 128 ? 1 : 6), true>(a, st);     // 192 and 160 rows are bf16-weight shapes (big_tile_rows never picks them for fp8)
-  else if (g_gemm_sched && spread) {
+  if (g_gemm_sched && spread) {
     // 128-row tiles that fill one round at most have nothing to walk, and the walk's longer prologue shows: 4,006 x 1536, K 768 17.6 us there, 19.1 walked;
     // vision fc1 of one chunk 27.7 / 28.6.  (192 and 256 rows gain from the scalar addresses: 4096 x 3584, K 3584 fp32 105.9 -> 102.5.)
     const long tiles = (long)((a.M + BM - 1) / BM) * ((a.N + 255) / 256) * (EPI == EPI_PARTIAL ? a.nsplit : 1);
-    if (!walk_offsets_fit(a)) launch_big_s<(BM == 160 ? 192 : BM), EPI, 1, false>(a, st);
-    else if (BM == 128 && tiles <= 256) launch_big_s<128, EPI, 6, false>(a, st);
-    else launch_walk<BM, EPI>(a, st);
+    // fp8 weights on 128 rows: a burst instead of pieces spread over the steps (386 x 37888 149 us against 155)
+    if (!walk_offsets_fit(a)) a.w_fp8 ? launch_big_s<(BM == 128 ? 128 : 256), EPI, 1, true>(a, st) : launch_big_s<(BM == 160 ? 192 : BM), EPI, 1, false>(a, st);
+    else if (BM == 128 && tiles <= 256) a.w_fp8 ? launch_big_s<128, EPI, 1, true>(a, st) : launch_big_s<128, EPI, 6, false>(a, st);
+    else a.w_fp8 ? launch_walk<BM, EPI, true>(a, st) : launch_walk<BM, EPI, false>(a, st);
   }
+  else if (a.w_fp8) launch_big_s<(BM == 128 ? 128 : 256), EPI, 1, true>(a, st);
   else if (g_gemm_sched) launch_big_s<(BM == 160 ? 192 : BM), EPI, 1, false>(a, st);
   else launch_big_s<(BM == 160 ? 192 : BM), EPI, 0, false>(a, st);
 }
@@ -1778,19 +1790,22 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr, bool 
   if (g_gemm_variant == 14) return vh_legal(a) ? 272 : 256;
   if (g_gemm_variant == 3 || g_gemm_variant == 5) return 256;
   if (g_gemm_variant == 4 || g_gemm_variant == 6) return 128;
-  if (g_gemm_variant == 13) return a.w_fp8 ? 256 : 192;
-  if (g_gemm_variant == 17) return a.w_fp8 ? 256 : 160;
+  if (g_gemm_variant == 13) return wide_only ? 256 : 192;
+  if (g_gemm_variant == 17) return wide_only ? 256 : 160;
   if (g_gemm_variant == 15) return (a.partial != nullptr && vh_small_shape(a.M, a.K) && vh_legal(a, true)) ? 144 : 128;
   if (g_gemm_variant == 16) return wide_only ? 128 : 129;
   if (g_gemm_variant != 2) return 0;
   const bool slabs = a.partial != nullptr || score != nullptr;
   const float s256 = tile_score(a.M, a.N, S, 256, 256, 256, 1.0f, true);
   static const int allow192 = [] { const char* v = getenv("LCC_GEMM_192"); return v ? atoi(v) : 1; }();     // A/B: 0 = round-3 tile choice
-  const float s192 = (a.w_fp8 || !allow192) ? 0.f : tile_score(a.M, a.N, S, 192, 256, 256, slabs ? 0.93f : 0.88f, true);
+  const bool short_tiles = allow192 && !(a.w_fp8 && (slabs || wide_only));
+  const float s192 = !short_tiles ? 0.f : tile_score(a.M, a.N, S, 192, 256, 256, slabs ? 0.93f : 0.88f, true);
   // BM 160 (bf16 weights): where 192 rows start a last round that is mostly empty.  The vision proj / fc2 of 15,840 rows are 83 x 5 tiles of 192 rows =
   // 1.62 rounds; 99 x 5 of 160 fill 1.93 at 5/6 of the time each: proj 55.7 -> 52.1 us, fc2 201 -> 178.
-  const float s160 = (a.w_fp8 || !allow192) ? 0.f : tile_score(a.M, a.N, S, 160, 256, 256, slabs ? 0.90f : 0.86f, false);
-  const float s128 = tile_score(a.M, a.N, S, 128, 256, 256, a.w_fp8 ? 0.85f : 0.82f, true);
+  const float s160 = !short_tiles ? 0.f : tile_score(a.M, a.N, S, 160, 256, 256, slabs ? 0.90f : 0.86f, false);
+  // 128 rows: 0.85 us a step while all tiles run at once, 0.93 in several rounds (514 rows of [37888, 3584]: 192-row tiles 141 us, these 156; fp8 weights 136 / 160)
+  const bool second_round = (long)((a.M + 127) / 128) * ((a.N + 255) / 256) * S > 256;
+  const float s128 = tile_score(a.M, a.N, S, 128, 256, 256, second_round && !slabs && !wide_only ? 0.76f : a.w_fp8 ? 0.85f : 0.82f, true);
   // gemm_mid_kernel: 0.38 / 0.52 us a step of 64 x 128 / 128 x 128 against 0.85 of 128 x 256, one tile a compute unit at a time (two 64-row
   // tiles side by side take twice as long).  Returned as 0 / 129.  The 128-row form wins where its blocks fill one round and the 64-row
   // form's need two; beyond a round the 256-column tiles do (shapes around the lines: 1000 x 3584, K 3584: 43 / 34 / 52 us for 64 x 128 /
@@ -2499,7 +2514,7 @@ static int gemm_w8(const GemmArgs& a, hipStream_t st) {
   const bool tall = !part && !odd && tall_wanted(c);
   const int big = (g_gemm_variant == 7) ? 0 : big_tile_rows(c, part ? a.nsplit : 1, nullptr, odd);
   if (odd && big != 256 && big != 128) return (a.ldc & 3) != 0 ? LCC_ERR_SHAPE : LCC_ERR_ALIGN;
-#define LCC_W8_TILE(EPI) (big == 256 ? launch_big<256, EPI>(c, st) : big == 128 ? launch_big<128, EPI>(c, st) : big == 129 ? launch_mid<128, EPI, 4>(c, st) : launch_mid64<EPI>(c, st))
+#define LCC_W8_TILE(EPI) (big == 256 ? launch_big<256, EPI>(c, st) : big == 192 ? launch_big<192, EPI>(c, st) : big == 160 ? launch_big<160, EPI>(c, st) : big == 128 ? launch_big<128, EPI>(c, st) : big == 129 ? launch_mid<128, EPI, 4>(c, st) : launch_mid64<EPI>(c, st))
 #define LCC_W8(EPI) (tall ? launch_tall<EPI>(c, st) : LCC_W8_TILE(EPI))
   if (part) { LCC_W8_TILE(EPI_PARTIAL); return 0; }
   switch (a.epilogue) {

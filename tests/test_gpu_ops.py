@@ -494,6 +494,33 @@ def test_gemm_w8_narrow_tiles(dev, M, N, K, epi, S, variant):
         assert (part.sum(0) - r32).abs().max().item() <= 2e-5 * float(r32.abs().max()) * math.sqrt(K / 256) + 1e-5
 
 
+@pytest.mark.parametrize("M,N,K,epi,S", [(300, 528, 192, 0, 0), (129, 272, 64, 1, 0), (1030, 16640, 64, 3, 0), (1030, 16640, 320, 4, 0), (577, 528, 704, 0, 3)])
+def test_gemm_w8_walking_tiles_give_the_same_bits(dev, M, N, K, epi, S):
+    """fp8 weights in row tiles of 256, 192, 160 and 128: one tile a block and several, fewer k-tiles than stages, a ragged last row and column tile, slabs;
+    the sums of the 128 x 128 tiles, which the reference bounds."""
+    from livecc_amd import ops
+    from livecc_amd.weights import dequantize_fp8_rows, quantize_fp8_rows
+    x, w = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.05, 2).float()
+    b = None if epi == 4 or S else _rand((N,), dev, 0.1, 3)
+    res = _rand((M, N), dev, 1.0, 4) if epi == 3 else None
+    w8, sc = ops.quantize_fp8(w)
+    out = {}
+    for variant in (16, 3, 13, 17, 4):
+        ops.set_gemm_variant(variant)
+        try:
+            out[variant] = ops.linear_w8(x, w8, sc, b, epi, res, nsplit=S) if S else ops.linear_w8(x, w8, sc, b, epi, res)
+        finally:
+            ops.set_gemm_variant(ops.GEMM_DEFAULT_VARIANT)
+    for variant in (3, 13, 17, 4):
+        assert torch.equal(out[variant], out[16]), variant
+    wd = dequantize_fp8_rows(*quantize_fp8_rows(w))
+    if S:
+        assert (out[3].sum(0) - x.float() @ wd.float().t()).abs().max().item() <= 2e-5 * float((x.float() @ wd.float().t()).abs().max()) * math.sqrt(K / 256) + 1e-5
+    else:
+        ref, atol = _ref_linear(x, wd, b, epi, res, with_atol=True)
+        assert_bf16_close(out[3], ref, f"gemm_w8_walk[{M}x{N}x{K},epi{epi}]", max_ulp=1.0, max_frac=5e-3, atol=atol)
+
+
 @pytest.mark.parametrize("M", [17, 113, 225, 337, 385, 386, 448])
 @pytest.mark.parametrize("N,K,epi", [(352, 192, 0), (160, 64, 1), (480, 320, 3), (352, 128, 4)])
 def test_gemm_w8_tall(dev, M, N, K, epi):
