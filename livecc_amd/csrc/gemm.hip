@@ -1782,7 +1782,8 @@ static float tile_score(int M, int N, int S, int BM, int BN, int slots, float ef
 // 0.87, 1, 0.985, 0.96 (short tiles move more bytes from the L2 per product, and from 0.85 of the chip on power is the limit).  192 rows at 0.93 and 160 at 0.90 had
 // been measured on tiles whose waves kept in step, us there / here: 3580 x 37888 722 / 701, 5000 x 3584, K 18944 590 / 464, 3994 x 17920, K 1536 181 / 169, 11648 x 1536,
 // K 8960 278 / 225, 3994 x 4608 113 / 96, 1600 x 37888 372 / 341, 4096 x 14336 326 / 309; the worst of 28 shapes whose tile changed 1950 / 1973.
-// Slabs and their count (gemm_tiled_num_splits) keep the older figures: one round at most, the ends of the tiles as long as their loops.
+// (fp32 output, one slab: 4096 x 25088 672 / 603, 4096 x 14336 372 / 342, 5992 x 14336 531 / 477, 7920 x 7168 363 / 331.)
+// Two slabs and more, and their count (gemm_tiled_num_splits), keep the older figures: one round at most, the ends of the tiles as long as their loops.
 // LCC_GEMM_VH=0: rounds 2-4 tile choice.
 // score: of the chosen tile, automatic choice only.  wide_only: 256-column tiles as they stand against a 64 x 128 one that dequantises fp8 weights first (gemm_w8)
 static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr, bool wide_only = false) {
@@ -1795,7 +1796,7 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr, bool 
   if (g_gemm_variant == 15) return (a.partial != nullptr && vh_small_shape(a.M, a.K) && vh_legal(a, true)) ? 144 : 128;
   if (g_gemm_variant == 16) return wide_only ? 128 : 129;
   if (g_gemm_variant != 2) return 0;
-  const bool slabs = a.partial != nullptr || score != nullptr;
+  const bool slabs = (a.partial != nullptr && S > 1) || score != nullptr;
   const float s256 = tile_score(a.M, a.N, S, 256, 256, 256, 1.0f, true);
   static const int allow192 = [] { const char* v = getenv("LCC_GEMM_192"); return v ? atoi(v) : 1; }();     // A/B: 0 = round-3 tile choice
   const bool short_tiles = allow192 && !(a.w_fp8 && (slabs || wide_only));
