@@ -1783,7 +1783,6 @@ static float tile_score(int M, int N, int S, int BM, int BN, int slots, float ef
 // been measured on tiles whose waves kept in step, us there / here: 3580 x 37888 722 / 701, 5000 x 3584, K 18944 590 / 464, 3994 x 17920, K 1536 181 / 169, 11648 x 1536,
 // K 8960 278 / 225, 3994 x 4608 113 / 96, 1600 x 37888 372 / 341, 4096 x 14336 326 / 309; the worst of 28 shapes whose tile changed 1950 / 1973.
 // (fp32 output, one slab: 4096 x 25088 672 / 603, 4096 x 14336 372 / 342, 5992 x 14336 531 / 477, 7920 x 7168 363 / 331.)
-// Two slabs and more, and their count (gemm_tiled_num_splits), keep the older figures: one round at most, the ends of the tiles as long as their loops.
 // LCC_GEMM_VH=0: rounds 2-4 tile choice.
 // score: of the chosen tile, automatic choice only.  wide_only: 256-column tiles as they stand against a 64 x 128 one that dequantises fp8 weights first (gemm_w8)
 static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr, bool wide_only = false) {
@@ -1800,10 +1799,10 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr, bool 
   const float s256 = tile_score(a.M, a.N, S, 256, 256, 256, 1.0f, true);
   static const int allow192 = [] { const char* v = getenv("LCC_GEMM_192"); return v ? atoi(v) : 1; }();     // A/B: 0 = round-3 tile choice
   const bool short_tiles = allow192 && !(a.w_fp8 && (slabs || wide_only));
-  const float s192 = !short_tiles ? 0.f : tile_score(a.M, a.N, S, 192, 256, 256, slabs ? 0.93f : 0.88f, true);
+  const float s192 = !short_tiles ? 0.f : tile_score(a.M, a.N, S, 192, 256, 256, 0.88f, true);
   // BM 160 (bf16 weights): where 192 rows start a last round that is mostly empty.  The vision proj / fc2 of 15,840 rows are 83 x 5 tiles of 192 rows =
   // 1.62 rounds; 99 x 5 of 160 fill 1.93 at 5/6 of the time each: proj 55.7 -> 52.1 us, fc2 201 -> 178.
-  const float s160 = !short_tiles ? 0.f : tile_score(a.M, a.N, S, 160, 256, 256, slabs ? 0.90f : 0.86f, false);
+  const float s160 = !short_tiles ? 0.f : tile_score(a.M, a.N, S, 160, 256, 256, 0.86f, false);
   // 128 rows: 0.85 us a step while all tiles run at once, 0.93 in several rounds (514 rows of [37888, 3584]: 192-row tiles 141 us, these 156; fp8 weights 136 / 160)
   const bool second_round = (long)((a.M + 127) / 128) * ((a.N + 255) / 256) * S > 256;
   const float s128 = tile_score(a.M, a.N, S, 128, 256, 256, second_round && !slabs && !wide_only ? 0.76f : a.w_fp8 ? 0.85f : 0.82f, true);
@@ -1813,7 +1812,9 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr, bool 
   // 128 x 128 / 128 x 256; 1456 x 3584: 73 / 61 / 52; 520 x 3584: 25 / 33 / 50).  With fp8 weights the steps stand alike (4608, K 3584: 386 rows
   // 25 / 33 / 49, 600 rows 42 / 34 / 50, 1000 rows 73 / 61 / 49; 200 x 3584, K 18944 in four splits 68 / 48 / 66).
   const float s64 = wide_only ? tile_score(a.M, a.N, S, 64, 128, 512, 0.55f, false) : tile_score(a.M, a.N, S, 64, 128, 256, 0.48f, false);
-  const float s128m = wide_only ? 0.f : tile_score(a.M, a.N, S, 128, 128, 256, 0.70f, false);
+  // (a long contraction, all of it in one split, on most of the chip: 0.65 -- 1131 x 3584, K 18944 170 us)
+  const bool crowded = score && S == 1 && (long)((a.M + 127) / 128) * ((a.N + 127) / 128) > 192;
+  const float s128m = wide_only ? 0.f : tile_score(a.M, a.N, S, 128, 128, 256, crowded ? 0.65f : 0.70f, false);
   if (score) *score = std::max(std::max(std::max(s256, s192), std::max(s160, s128)), std::max(s128m, s64));
   static const int allow_vh = [] { const char* v = getenv("LCC_GEMM_VH"); return v ? atoi(v) : 1; }();
   if (allow_vh && vh_legal(a) && (((a.M + 15) >> 4) & 15) != 0) {      // F % 16 == 0: the 256-row tiles are the same thing
@@ -2453,7 +2454,8 @@ int gemv_num_splits(int N, int K) {
 int gemm_tiled_num_splits(int M, int N, int K, bool packed_bf16) {
   const long tiles = (long)((M + 63) / 64) * ((N + 127) / 128);
   // More than one chunk's rows on a long K (bf16 weights): the split count whose best tile (big_tile_rows' scores against 1.25 PFLOP/s) plus the slabs' way
-  // to memory and back is shortest, and only if that saves a tenth.  Product and consumer together, us, without / with: 1000 x 3584, K 22528 240 / 170
+  // to memory and back is shortest, and only if that saves a tenth.  Product and slabs, us, with the heights' older weights / today's: 1000 x 3584, K 22528 three splits
+  // 171 / four 154, K 18944 146 / 135; 500 x 3584, K 18944 six 99 / four 91; 1200 x 3584, K 22528 two 191 / three 177; 2500 x 3584, K 22528 one 340 / two 327.  Product and consumer together, us, without / with: 1000 x 3584, K 22528 240 / 170
   // (four splits of 256 x 256 tiles instead of 128 x 128); 600 x 3584, K 18944 107 (three) / 94; 2104 x 1536, K 10496 86 / 73; 1000 x 1536, K 8960 52 / 40.
   if (packed_bf16 && M > 448 && M <= 4096 && K >= 6144 && (K & 63) == 0 && (N & 15) == 0 && g_gemm_variant == 2) {
     static float dummy;
