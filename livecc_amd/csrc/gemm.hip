@@ -1773,6 +1773,22 @@ static float tile_score(int M, int N, int S, int BM, int BN, int slots, float ef
   const float quant = (float)blocks / (float)((blocks + slots - 1) / slots * slots);
   return util * quant * eff;
 }
+static bool tiles_192_on() { static const int on = [] { const char* v = getenv("LCC_GEMM_192"); return v ? atoi(v) : 1; }(); return on != 0; }      // A/B: 0 = 256 / 128 rows
+static bool vh_on() { static const int on = [] { const char* v = getenv("LCC_GEMM_VH"); return v ? atoi(v) : 1; }(); return on != 0; }
+// Score of the best tile of S splits, for the search of a split count alone (gemm_tiled_num_splits).  Which tile runs leaves a result's bits as they are; into how
+// many fp32 sums a contraction is cut does not, so the count has weights of its own, which stay when the tiles' are measured anew.
+static float split_score(const GemmArgs& a, int S) {
+  const float on192 = tiles_192_on() ? 1.f : 0.f;
+  float best = std::max(std::max(std::max(tile_score(a.M, a.N, S, 256, 256, 256, 1.0f, true), tile_score(a.M, a.N, S, 192, 256, 256, on192 * 0.93f, true)),
+                                 std::max(tile_score(a.M, a.N, S, 160, 256, 256, on192 * 0.90f, false), tile_score(a.M, a.N, S, 128, 256, 256, 0.85f, true))),
+                        std::max(tile_score(a.M, a.N, S, 128, 128, 256, 0.70f, false), tile_score(a.M, a.N, S, 64, 128, 256, 0.48f, false)));
+  const int F = (a.M + 15) >> 4, t = F >> 4;
+  if (vh_on() && vh_legal(a) && (F & 15) != 0) {
+    const long blocks = (long)t * ((a.N + 255) / 256) * S;
+    best = std::max(best, (float)a.M / (float)(t * ((F + t - 1) / t) * 16) * (float)blocks / (float)((blocks + 255) / 256 * 256));
+  }
+  return best;
+}
 // BM 192 (round 4, bf16 weights): a 256-row tile leaves the chip partly idle whenever (M / 256) x (N / 256) falls just short of a round --
 // the o / down projections of 8 co-scheduled chunks are M = 3088 x N = 3584 = 13 x 14 = 182 blocks on 256 CUs (29 % idle); 17 x 14 = 238
 // blocks of 192 rows fill 93 % of one round at 3/4 of the tile time.
@@ -1784,8 +1800,8 @@ static float tile_score(int M, int N, int S, int BM, int BN, int slots, float ef
 // K 8960 278 / 225, 3994 x 4608 113 / 96, 1600 x 37888 372 / 341, 4096 x 14336 326 / 309; the worst of 28 shapes whose tile changed 1950 / 1973.
 // (fp32 output, one slab: 4096 x 25088 672 / 603, 4096 x 14336 372 / 342, 5992 x 14336 531 / 477, 7920 x 7168 363 / 331.)
 // LCC_GEMM_VH=0: rounds 2-4 tile choice.
-// score: of the chosen tile, automatic choice only.  wide_only: 256-column tiles as they stand against a 64 x 128 one that dequantises fp8 weights first (gemm_w8)
-static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr, bool wide_only = false) {
+// wide_only: 256-column tiles as they stand against a 64 x 128 one that dequantises fp8 weights first (gemm_w8)
+static int big_tile_rows(const GemmArgs& a, int S, bool wide_only = false) {
   if (!big_eligible(a)) return 0;
   if (g_gemm_variant == 14) return vh_legal(a) ? 272 : 256;
   if (g_gemm_variant == 3 || g_gemm_variant == 5) return 256;
@@ -1795,10 +1811,9 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr, bool 
   if (g_gemm_variant == 15) return (a.partial != nullptr && vh_small_shape(a.M, a.K) && vh_legal(a, true)) ? 144 : 128;
   if (g_gemm_variant == 16) return wide_only ? 128 : 129;
   if (g_gemm_variant != 2) return 0;
-  const bool slabs = (a.partial != nullptr && S > 1) || score != nullptr;
+  const bool slabs = a.partial != nullptr && S > 1;
   const float s256 = tile_score(a.M, a.N, S, 256, 256, 256, 1.0f, true);
-  static const int allow192 = [] { const char* v = getenv("LCC_GEMM_192"); return v ? atoi(v) : 1; }();     // A/B: 0 = round-3 tile choice
-  const bool short_tiles = allow192 && !(a.w_fp8 && (slabs || wide_only));
+  const bool short_tiles = tiles_192_on() && !(a.w_fp8 && (slabs || wide_only));
   const float s192 = !short_tiles ? 0.f : tile_score(a.M, a.N, S, 192, 256, 256, 0.88f, true);
   // BM 160 (bf16 weights): where 192 rows start a last round that is mostly empty.  The vision proj / fc2 of 15,840 rows are 83 x 5 tiles of 192 rows =
   // 1.62 rounds; 99 x 5 of 160 fill 1.93 at 5/6 of the time each: proj 55.7 -> 52.1 us, fc2 201 -> 178.
@@ -1812,17 +1827,10 @@ static int big_tile_rows(const GemmArgs& a, int S, float* score = nullptr, bool 
   // 128 x 128 / 128 x 256; 1456 x 3584: 73 / 61 / 52; 520 x 3584: 25 / 33 / 50).  With fp8 weights the steps stand alike (4608, K 3584: 386 rows
   // 25 / 33 / 49, 600 rows 42 / 34 / 50, 1000 rows 73 / 61 / 49; 200 x 3584, K 18944 in four splits 68 / 48 / 66).
   const float s64 = wide_only ? tile_score(a.M, a.N, S, 64, 128, 512, 0.55f, false) : tile_score(a.M, a.N, S, 64, 128, 256, 0.48f, false);
-  // (a long contraction, all of it in one split, on most of the chip: 0.65 -- 1131 x 3584, K 18944 170 us)
-  const bool crowded = score && S == 1 && (long)((a.M + 127) / 128) * ((a.N + 127) / 128) > 192;
-  const float s128m = wide_only ? 0.f : tile_score(a.M, a.N, S, 128, 128, 256, crowded ? 0.65f : 0.70f, false);
-  if (score) *score = std::max(std::max(std::max(s256, s192), std::max(s160, s128)), std::max(s128m, s64));
-  static const int allow_vh = [] { const char* v = getenv("LCC_GEMM_VH"); return v ? atoi(v) : 1; }();
-  if (allow_vh && vh_legal(a) && (((a.M + 15) >> 4) & 15) != 0) {      // F % 16 == 0: the 256-row tiles are the same thing
+  const float s128m = wide_only ? 0.f : tile_score(a.M, a.N, S, 128, 128, 256, 0.70f, false);
+  if (vh_on() && vh_legal(a) && (((a.M + 15) >> 4) & 15) != 0) {      // F % 16 == 0: the 256-row tiles are the same thing
     const float svh = vh_tiles(a.M, a.N, S).score;
-    if (svh > s256 && svh > s192 && svh > s160 && svh > s128 && svh > s128m && svh > s64) {
-      if (score) *score = svh;
-      return 272;
-    }
+    if (svh > s256 && svh > s192 && svh > s160 && svh > s128 && svh > s128m && svh > s64) return 272;
   }
   // small class (returned as 144): split-K slabs of one streaming chunk's projections, where the 128-row tiles leave a nearly empty last row tile
   if (vh_small_on() && a.partial != nullptr && vh_small_shape(a.M, a.K) && vh_legal(a, true)) {
@@ -2453,20 +2461,15 @@ int gemv_num_splits(int N, int K) {
 // split-K factor for a tiled GEMM whose output grid alone cannot fill 256 CUs (e.g. M = 386, N = 3584: 196 tiles)
 int gemm_tiled_num_splits(int M, int N, int K, bool packed_bf16) {
   const long tiles = (long)((M + 63) / 64) * ((N + 127) / 128);
-  // More than one chunk's rows on a long K (bf16 weights): the split count whose best tile (big_tile_rows' scores against 1.25 PFLOP/s) plus the slabs' way
-  // to memory and back is shortest, and only if that saves a tenth.  Product and slabs, us, with the heights' older weights / today's: 1000 x 3584, K 22528 three splits
-  // 171 / four 154, K 18944 146 / 135; 500 x 3584, K 18944 six 99 / four 91; 1200 x 3584, K 22528 two 191 / three 177; 2500 x 3584, K 22528 one 340 / two 327.  Product and consumer together, us, without / with: 1000 x 3584, K 22528 240 / 170
-  // (four splits of 256 x 256 tiles instead of 128 x 128); 600 x 3584, K 18944 107 (three) / 94; 2104 x 1536, K 10496 86 / 73; 1000 x 1536, K 8960 52 / 40.
+  // More than one chunk's rows on a long K (bf16 weights): the split count whose best tile (split_score against 1.25 PFLOP/s) plus the slabs' way
+  // to memory and back is shortest, and only if that saves a tenth.  Product and consumer together, us, without / with: 1000 x 3584, K 22528 240 / 170
+  // (three splits instead of 128 x 128 tiles); 600 x 3584, K 18944 107 (three) / 94; 2104 x 1536, K 10496 86 / 73; 1000 x 1536, K 8960 52 / 40.
   if (packed_bf16 && M > 448 && M <= 4096 && K >= 6144 && (K & 63) == 0 && (N & 15) == 0 && g_gemm_variant == 2) {
-    static float dummy;
     GemmArgs a; a.M = M; a.N = N; a.K = K; a.w_packed = 1; a.lda = K;
     int best = 1;
     float best_us = 0.f;
     for (int S = 1; S <= 6; ++S) {
-      if (S > 1) { a.partial = &dummy; a.nsplit = S; }          // never dereferenced: the slab form is asked for
-      float score = 0.f;
-      big_tile_rows(a, S, &score);
-      const float us = 2e-9f * (float)M * (float)N * (float)K / (1.45f * score) + (S > 1 ? (float)S * (float)M * (float)N * 8e-6f / 4.5f : 0.f);
+      const float us = 2e-9f * (float)M * (float)N * (float)K / (1.25f * split_score(a, S)) + (S > 1 ? (float)S * (float)M * (float)N * 8e-6f / 4.5f : 0.f);
       if (S == 1 || us < (best == 1 ? 0.9f : 1.f) * best_us) { best = S; best_us = us; }
     }
     return best;
@@ -2515,7 +2518,7 @@ static int gemm_w8(const GemmArgs& a, hipStream_t st) {
   // behind a dequantising pass: they take it by the same lines, and the other shapes refuse it.
   const bool odd = (a.ldc & 3) != 0 || ((uintptr_t)a.C & 15) != 0;
   const bool tall = !part && !odd && tall_wanted(c);
-  const int big = (g_gemm_variant == 7) ? 0 : big_tile_rows(c, part ? a.nsplit : 1, nullptr, odd);
+  const int big = (g_gemm_variant == 7) ? 0 : big_tile_rows(c, part ? a.nsplit : 1, odd);
   if (odd && big != 256 && big != 128) return (a.ldc & 3) != 0 ? LCC_ERR_SHAPE : LCC_ERR_ALIGN;
 #define LCC_W8_TILE(EPI) (big == 256 ? launch_big<256, EPI>(c, st) : big == 192 ? launch_big<192, EPI>(c, st) : big == 160 ? launch_big<160, EPI>(c, st) : big == 128 ? launch_big<128, EPI>(c, st) : big == 129 ? launch_mid<128, EPI, 4>(c, st) : launch_mid64<EPI>(c, st))
 #define LCC_W8(EPI) (tall ? launch_tall<EPI>(c, st) : LCC_W8_TILE(EPI))

@@ -160,3 +160,10 @@ def test_narrow_fp8_products_refuse_a_result_they_cannot_store_aligned(built_lib
     p = (C.addressof(buf) + 15) // 16 * 16
     call = lambda c, ldc: built_lib.lcc_gemm_w8_bf16(p, 256, p, C.cast(p, C.POINTER(C.c_float)), None, None, 0, c, ldc, M, N, 256, 0, None, 0, p, None)
     assert call(p, N + 2) == call(p, N + 1) == -2 and call(p + 8, N) == -3
+
+
+@pytest.mark.parametrize("m,n,k,splits", [(1000, 3584, 22528, 3), (1000, 3584, 18944, 3), (500, 3584, 18944, 6), (1200, 3584, 22528, 5), (2500, 3584, 22528, 2),
+                                          (514, 4608, 6144, 4), (1227, 1280, 6144, 5), (496, 37888, 22528, 1), (1000, 1536, 8960, 5), (2104, 1536, 10496, 3)])
+def test_split_counts_of_long_contractions_do_not_follow_the_tiles_weights(ops, m, n, k, splits):
+    """The count decides into how many fp32 sums a contraction is cut, and so a result's bits; which tile runs a product does not."""
+    assert ops.gemm_plan(m, n, k, ops.EPI_NONE)[1] == splits
