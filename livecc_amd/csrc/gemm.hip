@@ -1853,8 +1853,10 @@ static int big_tile_rows(const GemmArgs& a, int S, bool wide_only = false) {
 
 // The tall kernel serves one-block-row problems whose column tiles fill most of ONE round of the chip (7B gate/up at a streaming
 // chunk: 237 blocks).  Variant 8 forces it wherever it is legal (tests).
-// (fp8 weights with a residual would need more registers than a wave has)
-static bool tall_legal(const GemmArgs& a) { return big_eligible(a) && !(a.w_fp8 && a.epilogue == EPI_RESIDUAL) && a.M <= 448 && (a.N & 15) == 0; }
+// (fp8 weights with a residual would need more registers than a wave has; a row's offset, up to 448 rows from A, is 32-bit)
+static bool tall_legal(const GemmArgs& a) {
+  return big_eligible(a) && !(a.w_fp8 && a.epilogue == EPI_RESIDUAL) && a.M <= 448 && (a.N & 15) == 0 && (size_t)a.lda * 896 <= 0xffffffffu;
+}
 static bool tall_wanted(const GemmArgs& a) {
   if (!tall_legal(a)) return false;
   if (g_gemm_variant == 8) return true;

@@ -155,6 +155,40 @@ def test_gemm_tall_rows_in_quarters(dev, M, K, fp8):
         assert ops.launch_counts()["gemm_tall"] - before == (M > 128)
 
 
+@pytest.mark.parametrize("M,lda", [(256, 8500000), (300, 7500000), (448, 4800000), (448, 4793488)])
+@pytest.mark.parametrize("fp8", [False, True], ids=["bf16", "fp8"])
+@pytest.mark.parametrize("variant", [2, 8], ids=["default", "tall_where_legal"])
+def test_gemm_rows_far_apart(dev, M, lda, fp8, variant):
+    """Rows of a larger tensor whose last ones start more than 4 GiB behind the first: the tall tile's offsets are 32-bit and it leaves them to the
+    others (4,793,488 elements of 448 rows are the last it takes).  The same bits as for the rows side by side."""
+    from livecc_amd import _lib, ops
+    N, K = 33280, 64
+    far = torch.empty((M - 1) * lda + K, dtype=torch.bfloat16, device=dev).as_strided((M, K), (lda, 1))
+    x, w = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.05, 2)
+    far.copy_(x)
+    w8, sc = ops.quantize_fp8(w.float())
+    wp = ops.pack_weight(w)
+
+    def product(a, stride):
+        out = torch.empty(M, N // 2, dtype=torch.bfloat16, device=dev)
+        st = torch.cuda.current_stream().cuda_stream
+        if fp8:
+            rc = _lib.load().lcc_gemm_w8_bf16(a.data_ptr(), stride, w8.data_ptr(), sc.data_ptr(), None, None, 0, out.data_ptr(), N // 2, M, N, K, ops.EPI_SWIGLU, None, 0, None, st)
+        else:
+            rc = _lib.load().lcc_gemm_bf16(a.data_ptr(), stride, wp.data_ptr(), K, 1, None, None, 0, out.data_ptr(), N // 2, M, N, K, ops.EPI_SWIGLU, None, 0, st)
+        _lib.check(rc, "product")
+        return out
+    ops.set_gemm_variant(variant)
+    try:
+        want = product(x, K)
+        before = ops.launch_counts()["gemm_tall"]
+        got = product(far, lda)
+        assert ops.launch_counts()["gemm_tall"] - before == (lda * 896 < 2 ** 32)
+    finally:
+        ops.set_gemm_variant(ops.GEMM_DEFAULT_VARIANT)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("M", [256 + 16, 272 + 7, 288, 2 * 256 + 1, 2 * 288 - 16, 3088, 1131])
 @pytest.mark.parametrize("N,K,epi", [(512, 256, 0), (768, 192, 3), (3584, 1024, 4)])
 def test_gemm_variable_height_tiles_are_bit_identical_to_the_256_row_tiles(dev, M, N, K, epi):
