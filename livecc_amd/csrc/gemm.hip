@@ -9,7 +9,7 @@
 //  * gemm_big_kernel     : the same tiles one a block, both waves of a SIMD in step: 128-row tiles of one round.
 //  * gemm_walk_vh_kernel : the walk over row tiles of 256 / 272 / 288 rows (no ragged last row tile).
 //  * gemm_vh_kernel      : row tiles of 128 / 144 rows, split-K slabs of one streaming chunk.
-//  * gemm_tall_kernel    : one block row covers all of M (up to 448 rows: gate/up of one streaming chunk or of a few short ones).
+//  * gemm_tall_kernel    : one block row covers all of M (up to 448 rows: gate/up of one streaming chunk or of a few short ones; wide products of 257 rows and more).
 //  * gemm_mid_kernel     : shapes with few 256-column tiles.  64x128x64 (128x128x64) tile, 8 waves, 6- (4-) stage LDS-DMA ring.
 //  * gemm_glds_kernel /   : row-major W, K % 64 != 0.  64x128x64 (128x128x64) tile, 4 waves,
 //    gemm_tiled_kernel     LDS-DMA 3-stage ring / register-staged double buffer with an XOR swizzle, XCD-aware block remap.
@@ -1863,6 +1863,9 @@ static bool tall_wanted(const GemmArgs& a) {
   if (g_gemm_variant != 2) return false;
   const int blocks = (a.N + 159) / 160;
   if (blocks < 192 || blocks > 256) return false;
+  // without SwiGLU: [37888, 3584] with bias, us, other tiles / these: 256 rows 82 / 102, 288 100 / 86, 340 110 / 95, 448 123 / 108; fp8 weights, which have one height there (launch_tall_w):
+  // 256 72 / 102, 300 98 / 104, 386 113 / 107
+  if (a.epilogue != EPI_SWIGLU) return a.M > (a.w_fp8 ? 384 : 256);
   // Up to 256 rows where the other tiles (128 x 128, or two rows of 128 x 256) are more than one round.  K 3584 with SwiGLU, us, other tiles / these:
   //   bf16, N 37888: 65 rows 67 / 55, 128 71 / 59, 192 80 / 67, 256 89 / 74, 272 and more 84 / 84 (walking tiles; 300 rows 101 before them);  N 30720: 100 rows 48 / 52, 256 67 / 67
   //   fp8,  N 37888: 65 to 128 rows 56 / 57, 129 105 / 68, 256 90 / 75, 272 110 / 87, 330 114 / 96;  N 30720: 100 rows 44 / 56, 256 61 / 73
@@ -1877,14 +1880,17 @@ static void launch_tall_rows(const GemmArgs& a, hipStream_t st) {
 }
 template <int EPI, bool W8>
 static void launch_tall_w(const GemmArgs& a, hipStream_t st) {
-  if constexpr (EPI == EPI_SWIGLU) {          // the one product that comes here unforced (tall_wanted): fragments for each quarter of the rows
-    switch (((a.M + 15) / 16 + 3) / 4) {
-      case 1: case 2: return launch_tall_rows<EPI, 2, W8>(a, st);
-      case 3: return launch_tall_rows<EPI, 3, W8>(a, st);
-      case 4: return launch_tall_rows<EPI, 4, W8>(a, st);
-      case 5: return launch_tall_rows<EPI, 5, W8>(a, st);
-      case 6: return launch_tall_rows<EPI, 6, W8>(a, st);
-    }
+  // fragments for each quarter of the rows, where such rows come here unforced (tall_wanted); [37888, 3584] with bias, us, always seven / these: 272 rows 102 / 86, 300 103 / 87, 340 105 / 95
+  constexpr bool few = EPI == EPI_SWIGLU;
+  const int mt = ((a.M + 15) / 16 + 3) / 4;
+  if constexpr (few) {
+    if (mt <= 2) return launch_tall_rows<EPI, 2, W8>(a, st);
+    if (mt == 3) return launch_tall_rows<EPI, 3, W8>(a, st);
+    if (mt == 4) return launch_tall_rows<EPI, 4, W8>(a, st);
+  }
+  if constexpr (few || !W8) {
+    if (mt == 5) return launch_tall_rows<EPI, 5, W8>(a, st);
+    if (mt == 6) return launch_tall_rows<EPI, 6, W8>(a, st);
   }
   launch_tall_rows<EPI, 7, W8>(a, st);
 }

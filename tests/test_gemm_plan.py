@@ -167,3 +167,12 @@ def test_narrow_fp8_products_refuse_a_result_they_cannot_store_aligned(built_lib
 def test_split_counts_of_long_contractions_do_not_follow_the_tiles_weights(ops, m, n, k, splits):
     """The count decides into how many fp32 sums a contraction is cut, and so a result's bits; which tile runs a product does not."""
     assert ops.gemm_plan(m, n, k, ops.EPI_NONE)[1] == splits
+
+
+@pytest.mark.parametrize("m", [65, 128, 129, 192, 193, 256, 257, 320, 385, 448])
+@pytest.mark.parametrize("n", [32800, 37888, 40960])
+def test_the_tall_tile_of_few_rows_is_swiglu_alone(ops, m, n):
+    """Its heights of 2 to 4 fragments a quarter exist for that epilogue; another product of up to 256 rows would multiply 448."""
+    for epi in (ops.EPI_NONE, ops.EPI_QUICK_GELU, ops.EPI_GELU_ERF, ops.EPI_RESIDUAL):
+        assert (ops.gemm_plan(m, n, H, epi)[0] == 448) == (m > 256), epi
+    assert ops.gemm_plan(m, n, H, ops.EPI_SWIGLU)[0] == 448

@@ -155,6 +155,30 @@ def test_gemm_tall_rows_in_quarters(dev, M, K, fp8):
         assert ops.launch_counts()["gemm_tall"] - before == (M > 128)
 
 
+@pytest.mark.parametrize("M", [240, 257, 320, 321, 384, 385, 448])
+@pytest.mark.parametrize("epi", [0, 1, 2, 3])
+@pytest.mark.parametrize("fp8", [False, True], ids=["bf16", "fp8"])
+def test_gemm_tall_rows_of_other_epilogues(dev, M, epi, fp8):
+    """Bias, GELU and residual: at 33,280 columns the default takes the tall tile from 257 rows on (fp8 weights 385, none with a residual), in five, six or
+    seven fragments a quarter; the bits of the 128-row tiles (fp8 without a bias: the tall tile rounds the scaled sum before it is added)."""
+    from livecc_amd import ops
+    N, K = 33280, 192
+    x, w, b = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.05, 2), _rand((N,), dev, 0.1, 3)
+    res = _rand((M, N), dev, 1.0, 4) if epi == 3 else None
+    w8, sc = ops.quantize_fp8(w.float())
+    wp = ops.pack_weight(w)
+    product = lambda: ops.linear_w8(x, w8, sc, None, epi, res) if fp8 else ops.linear(x, wp, b, epi, res, packed_shape=(N, K))
+    before = ops.launch_counts()["gemm_tall"]
+    got = product()
+    assert ops.launch_counts()["gemm_tall"] - before == (M > 384 and epi != 3 if fp8 else M > 256)
+    try:
+        ops.set_gemm_variant(4)
+        want = product()
+    finally:
+        ops.set_gemm_variant(ops.GEMM_DEFAULT_VARIANT)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("M,lda", [(256, 8500000), (300, 7500000), (448, 4800000), (448, 4793488)])
 @pytest.mark.parametrize("fp8", [False, True], ids=["bf16", "fp8"])
 @pytest.mark.parametrize("variant", [2, 8], ids=["default", "tall_where_legal"])
