@@ -949,7 +949,8 @@ __global__ __launch_bounds__(512) void gemm_big_kernel(
 // instead of behind the reads 437 (K 18944); phases by k halves, which balance the reads but free a stage late, 460.
 //
 // Ring.  Stage = [rows][8 x 16 B] activations (XOR-swizzled) + 32 weight sub-tiles.  What phase 0 reads (first halves of the rows, all weights) is filled
-// again in the next phase 1, what phase 1 reads (second halves) in the next phase 0: two slots later, when either wave's reads are back.  Pieces leave in the order
+// again in the next phase 1, what phase 1 reads (second halves) in the next phase 0: two slots later, when either wave's reads are back.  A phase's rows of a
+// stage are the same for tiles of every height (ROW1), so that this holds from a tile to a taller one too.  Pieces leave in the order
 // in which they are needed, so "all but the last (NSTAGE - 1) k-tiles' worth have landed" is the wait of every phase.  They run on into the
 // next tile, whose first stages land while this one's results leave through LDS of their own; stores drain under the next tile's first phases (vmcnt retires
 // in order: a wait counts the pieces and lets the younger stores be, if all of them were issued -- inner tiles).
@@ -970,6 +971,7 @@ struct Walk {
   static constexpr int H0 = VH ? 4 : (MT + 1) / 2, H1 = MTX - H0;                                  // of phase 0, at most of phase 1
   static constexpr int P0 = (4 * H0 + 7) / 8, P1 = (4 * H1 + 7) / 8, PB = W8 ? 2 : 4, G = P0 + PB + P1;     // a wave's pieces of a k-tile: rows of phase 0, weights; rows of phase 1
   static constexpr bool SPARE = VH || (4 * H0) % 8 != 0 || (4 * H1) % 8 != 0;                      // slots without rows
+  static constexpr int ROW1 = VH ? 16 * MTX : BM / 2;                                              // of the stage: the second wave row's first, whatever a tile's height
   static constexpr int NSTAGE = BM == 128 ? 3 : 2;
   static constexpr int A_UNITS = ROWS * 8, STAGE = A_UNITS + PB * 512;                             // 16-byte units
   static constexpr int EGR = BM >= 160 && !VH && EPI != EPI_GELU_ERF ? 2 : 1;                      // row tiles of an epilogue group: 2 KB of LDS a wave each (the erf: registers)
@@ -1031,9 +1033,9 @@ LCC_DEVICE void gemm_walk_body(
   const bf16_t* bbase[2];
   unsigned off0[P0], off1[P1], dst0[P0], dst1[P1];
   const unsigned swz = ((lane & 7) ^ (lane >> 3)) << 4, row_bytes = (unsigned)(lda * 2);
-  auto slot_row = [&](int p, int from, int n_first, int n_second, int row1) { return p < n_first ? from + p * 8 : p < n_first + n_second ? row1 + from + (p - n_first) * 8 : -1; };
-  auto slot = [&](int row, int m0, unsigned& off, unsigned& dst) {
-    off = row >= 0 ? (unsigned)min(row + (lane >> 3), M - 1 - m0) * row_bytes + swz : 0u;
+  auto slot = [&](int p, int from, int n_first, int n_second, int row1, int m0, unsigned& off, unsigned& dst) {
+    const int row = p < n_first ? from + p * 8 : p < n_first + n_second ? S::ROW1 + from + (p - n_first) * 8 : -1;          // of the stage
+    off = row >= 0 ? (unsigned)min((S::VH && p >= n_first ? row - (S::ROW1 - row1) : row) + (lane >> 3), M - 1 - m0) * row_bytes + swz : 0u;
     dst = row >= 0 ? (unsigned)row * 128u : S::SCRATCH;
   };
   auto point0 = [&] {
@@ -1043,14 +1045,14 @@ LCC_DEVICE void gemm_walk_body(
 #pragma unroll
     for (int q = 0; q < 2; ++q) bbase[q] = W + (size_t)min((n0 >> 4) + wave * 2 + q, nfrag - 1) * (W8 ? K >> 6 : K32) * 512;
 #pragma unroll
-    for (int q = 0; q < P0; ++q) slot(slot_row(wave * P0 + q, 0, 2 * H0, 2 * H0, row1), m0, off0[q], dst0[q]);
+    for (int q = 0; q < P0; ++q) slot(wave * P0 + q, 0, 2 * H0, 2 * H0, row1, m0, off0[q], dst0[q]);
   };
   auto point1 = [&] {
     int m0, n0, row1, rows;
     tile_of(w1.vb, m0, n0, row1, rows);
     w1.a = A + (size_t)m0 * lda;
 #pragma unroll
-    for (int q = 0; q < P1; ++q) slot(slot_row(wave * P1 + q, H0 * 16, (row1 >> 3) - 2 * H0, ((rows - row1) >> 3) - 2 * H0, row1), m0, off1[q], dst1[q]);
+    for (int q = 0; q < P1; ++q) slot(wave * P1 + q, H0 * 16, (row1 >> 3) - 2 * H0, ((rows - row1) >> 3) - 2 * H0, row1, m0, off1[q], dst1[q]);
   };
   const unsigned lds0 = lds_addr(dsmem);
   auto to = [&](unsigned stage, unsigned dst) { return lds0 + (S::SPARE && dst == S::SCRATCH ? dst : stage + dst); };
@@ -1090,7 +1092,7 @@ LCC_DEVICE void gemm_walk_body(
     constexpr int MTW = decltype(mt_c)::value, MA = MTW > 0 ? MTW : 1, R0 = MTW > 0 ? H0 : 0, R1 = MTW - R0, RF = R0 > R1 ? R0 : R1;
     int aoff[2];
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) aoff[kk] = (my_row0 + li) * 8 + ((W8 ? g * 2 + kk : kk * 4 + g) ^ (li & 7));
+    for (int kk = 0; kk < 2; ++kk) aoff[kk] = ((wm ? S::ROW1 : 0) + li) * 8 + ((W8 ? g * 2 + kk : kk * 4 + g) ^ (li & 7));
     f32x4 acc[MA][NT];
 #pragma unroll
     for (int i = 0; i < MA; ++i)

@@ -373,6 +373,47 @@ def test_gemm_fewer_and_taller_variable_height_tiles_give_the_same_bits(dev, M, 
     assert torch.equal(got, ref), f"{int((got != ref).sum())} of {got.numel()} outputs differ from the 256-row tiles"
 
 
+def _heights_of_walking_blocks(M, N, S):
+    """Row fragments of the tiles that each block of the forced variable-height walk goes through (one split), in its order."""
+    F, tn = (M + 15) // 16, (N + 255) // 256
+    tm = F // 16
+    n, raster = tm * tn, 4 if tm > 6 else 0
+    step = n if n * S <= 256 else min(n, max(8, 256 // S & ~7))
+
+    def height(vb):
+        q, r, xcd, idx = n >> 3, n & 7, vb & 7, vb >> 3
+        t = (xcd * (q + 1) if xcd < r else r * (q + 1) + (xcd - r) * q) + idx
+        if raster:
+            band = t // (raster * tm)
+            row = (t - band * raster * tm) // min(raster, tn - band * raster)
+        else:
+            row = t % tm
+        return F // tm + (row < F % tm)
+    return [[height(vb) for vb in range(b, n, step)] for b in range(step)]
+
+
+@pytest.mark.parametrize("M,N,K,epi,S", [(843, 24640, 64, 0, 0), (1403, 16416, 320, 4, 0), (1403, 13840, 128, 3, 0), (3300, 6672, 64, 1, 0), (1403, 13600, 576, 0, 2)])
+def test_gemm_walk_between_tiles_of_17_and_18_fragments(dev, M, N, K, epi, S):
+    """Blocks that go from a tile of one height to one of the other, both ways, with fewer k-tiles than stages and more; the 256-row tiles' bits."""
+    from livecc_amd import ops
+    steps = {p for seq in _heights_of_walking_blocks(M, N, max(S, 1)) for p in zip(seq, seq[1:])}
+    assert {(17, 18), (18, 17)} <= steps, steps
+    x, w = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.05, 2)
+    b = None if epi == 4 or S else _rand((N,), dev, 0.1, 3)
+    res = _rand((M, N), dev, 1.0, 4) if epi == 3 else None
+    wp = ops.pack_weight(w)
+    out = {}
+    for variant in (14, 3):
+        ops.set_gemm_variant(variant)
+        try:
+            before = ops.launch_counts()["gemm_vh"]
+            out[variant] = ops.linear_partial(x, wp, S, packed_shape=(N, K)) if S else ops.linear(x, wp, b, epi, res, packed_shape=(N, K))
+            assert ops.launch_counts()["gemm_vh"] - before == (variant == 14)
+        finally:
+            ops.set_gemm_variant(ops.GEMM_DEFAULT_VARIANT)
+    assert torch.equal(out[14], out[3])
+
+
 @pytest.mark.parametrize("M,N,K,S", [(386, 3584, 18944, 6), (386, 4608, 3584, 4), (386, 3584, 3584, 6), (400, 3600, 1024, 2), (130, 512, 512, 2),
                                      (272, 1024, 1024, 4), (144, 256, 4096, 8), (391, 1536, 8960, 5)])
 def test_gemm_small_variable_height_tiles_give_the_slabs_of_the_128_row_tiles(dev, M, N, K, S):

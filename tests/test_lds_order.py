@@ -40,3 +40,23 @@ def test_no_requested_residual_piece_is_left_unused():
     text = body(open(os.path.join(CSRC, "gemm.hip")).read(), "tile_epilogue_wide")
     skips = re.findall(r"if \((.*?>= M)\) break;", text)
     assert skips and all(s.startswith("EPI != EPI_RESIDUAL && ") for s in skips)
+
+
+def test_a_stage_row_of_the_walking_tiles_belongs_to_one_phase_whatever_the_height():
+    """A block that goes from a tile of 17 row fragments to one of 18 copies the next tile's first phase into the stage whose second phase is being read: no row
+    of the stage may be in the first phase of one height and in the second of another."""
+    text = body(open(os.path.join(CSRC, "gemm.hip")).read(), "gemm_walk_body")
+    struct = re.search(r"struct Walk \{(.*?)\n\};", open(os.path.join(CSRC, "gemm.hip")).read(), re.S).group(1)
+    places = re.search(r"const int row = p < n_first \? from \+ p \* 8 : p < n_first \+ n_second \? (\S+) \+ from \+ \(p - n_first\) \* 8 : -1;", text)
+    assert "dst = row >= 0 ? (unsigned)row * 128u" in text
+    reads = re.search(r"aoff\[kk\] = \(\(wm \? (\S+) : 0\) \+ li\) \* 8", text)
+    assert places and reads and places.group(1) == reads.group(1)
+    at = {"row1": lambda f: (f >> 1) * 16, "S::ROW1": lambda f: {"16 * MTX": 16 * 9}[re.search(r"ROW1 = VH \? (.*?) : BM / 2;", struct).group(1)]}[places.group(1)]
+    of_phase = ([set(), set()])
+    for f in (16, 17, 18):
+        first, second = f >> 1, f - (f >> 1)          # row fragments of the two wave rows, four of each in the first phase
+        for start, n in ((0, first), (at(f), second)):
+            for i in range(n):
+                of_phase[i >= 4] |= set(range(start + 16 * i, start + 16 * i + 16))
+    assert not of_phase[0] & of_phase[1]
+    assert max(of_phase[1]) < 288
