@@ -38,14 +38,14 @@ static inline int slab_gemm(const DecBuffers& b, const bf16_t* A, int lda, const
   *nsplit = s;
   return gemm_bf16(g, st);
 }
-// slab_gemm(A, W) and the SwiGLU product of the same rows (gate_up, into C), in one launch where that is to be had (17 to 64 rows); *paired: it was
+// slab_gemm(A, W) and the SwiGLU product of the same rows (gate_up, into C), in one launch where that is the faster one (17 to 64 rows: gemv_rows_pair_ok); *paired: it was
 static inline int slab_swiglu_gemm(const DecBuffers& b, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K, const bf16_t* gate_up, int N2, bf16_t* C, int ldc,
                                    int* nsplit, bool* paired, hipStream_t st) {
   GemmArgs g, s;
   g.A = A; g.lda = lda; g.W = W; g.ldw = K; g.w_packed = 1; g.M = M; g.N = N; g.K = K; g.partial = b.part;
   g.nsplit = std::min(std::min(gemv_num_splits(N, K), 8), (K + 63) / 64);
   s.A = A; s.lda = lda; s.W = gate_up; s.ldw = K; s.w_packed = 1; s.C = C; s.ldc = ldc; s.M = M; s.N = N2; s.K = K; s.epilogue = LCC_EPI_SWIGLU;
-  *paired = gate_up != nullptr && (size_t)g.nsplit * M * N <= b.part_cap && gemv_rows_pair_ok(g, s);
+  *paired = g_fused_decode && gate_up != nullptr && (size_t)g.nsplit * M * N <= b.part_cap && gemv_rows_pair_ok(g, s);
   if (!*paired) return slab_gemm(b, A, lda, W, M, N, K, nsplit, st);
   *nsplit = g.nsplit;
   return gemv_rows_pair(g, s, st);

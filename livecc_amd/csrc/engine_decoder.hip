@@ -83,7 +83,7 @@ int carve_bound(lcc_engine* e, DecBuffers* b) {
 }
 
 }  // namespace
-int g_fused_decode = 1;      // lcc_debug_set_decoder_fused: decode steps of up to 16 rows run the fused launches (6 per layer instead of 9)
+int g_fused_decode = 1;      // lcc_debug_set_decoder_fused: decode steps of up to 16 rows run the fused launches (6 per layer instead of 9), of 17 to 64 eight
 
 namespace {
 // S packed rows through every layer; pt null: a decode step over the streams `d_slots`.  On exit b.h holds the final norm of the residual.

@@ -28,7 +28,8 @@ enum LaunchCounter {
   LC_ATTN_VIT32 = 13,          // attn_vit32_kernel (vision attention on 32x32x16 MFMAs)
   LC_GEMM_VH = 14,             // gemm_walk_vh_kernel (row tiles of 256 / 272 / 288 rows), gemm_vh_kernel (small class 128 / 144; round 5 -- the slot of the retired gemm_pp_kernel)
   LC_GEMM_VIT_QKV = 15,        // gemm_vit_kernel: EPI_VIT_QK / EPI_VIT_V epilogues (RoPE / V transpose fused into the q|k|v projection; one EPI_VIT_QKV launch per tower block when E % 128 == 0, else a q|k launch + a V launch)
-  LC_COUNT = 16
+  LC_GEMV_ROWS_PAIR = 16,      // gemv_rows_pair_kernel (input projection and gate/up of 17 to 64 rows in one launch)
+  LC_COUNT = 17
 };
 extern long long g_launch_counts[LC_COUNT];
 

@@ -112,7 +112,7 @@ ATTN_DEFAULT_VARIANT = 3
 
 LAUNCH_COUNTERS = ("attn_decode", "attn_decode_combine", "attn_decode_fused", "attn_decode_fused_merge", "gemv_fused_tail", "dgemv_v2",
                    "attn_prefill_mfma32", "attn_prefill_shared", "attn_prefill_per_wave", "attn_prefill_combine", "last_decode_nsplit",
-                   "last_prefill_nsplit", "gemm_tall", "attn_vit32", "gemm_vh", "gemm_vit_qkv")
+                   "last_prefill_nsplit", "gemm_tall", "attn_vit32", "gemm_vh", "gemm_vit_qkv", "gemv_rows_pair")
 
 
 def attn_tile_rows(n_q_heads: int, n_kv_heads: int) -> int:
@@ -149,8 +149,8 @@ def gemm_plan(M: int, N: int, K: int, epilogue: int = EPI_NONE, nsplit: int = 0,
 def launch_counts(reset: bool = False) -> dict:
     """Host-side launch counters of the library (which kernel served the calls since the last reset): lcc_debug_launch_counts."""
     import numpy as np
-    buf = np.zeros(16, dtype=np.int64)
-    _lib.check(_lib.load().lcc_debug_launch_counts(buf.ctypes.data, 16, 1 if reset else 0), "lcc_debug_launch_counts")
+    buf = np.zeros(len(LAUNCH_COUNTERS), dtype=np.int64)
+    _lib.check(_lib.load().lcc_debug_launch_counts(buf.ctypes.data, len(LAUNCH_COUNTERS), 1 if reset else 0), "lcc_debug_launch_counts")
     return {k: int(buf[i]) for i, k in enumerate(LAUNCH_COUNTERS)}
 
 

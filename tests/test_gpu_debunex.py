@@ -497,6 +497,47 @@ def test_wide_feed_forward_beside_the_input_projection(dev, ff, n):
         assert U.error(got[i], U.oracle_logits(cfg, T, seqs[i])[[-1]]) < U.LIMIT
 
 
+@pytest.mark.parametrize("width,ff,n", [(200, 8300, 17), (200, 8300, 48), (200, 8300, 64), (704, 7900, 33), (1600, 8300, 40), (200, 2200, 64), (200, 100, 32)])
+def test_one_launch_and_two_give_the_same_bits(dev, lib, width, ff, n):
+    """Input projection and gate/up of 17 to 64 rows, in one launch (counted) and in two: two, four and six weight tiles a block, one split and several."""
+    from livecc_amd import ops
+    from livecc_amd.config import DebunexConfig
+    cfg = DebunexConfig(width, 100, [U.L(U.M(3, 40, 48, 72, 90, 0.2), ff), U.L(U.M(2, 64, 64, 800, 90, 0.2, 0), ff)], 1e-5, 20.0, name="pair")
+    T = U.make_weights(cfg, 8)
+    m = _model(cfg, T, dev, max_streams=n, max_kv_len=64, max_new_rows=512)
+    seqs = [U.ids_of(cfg, 3 + i % 5, 50 + i) for i in range(n)]
+    res = []
+    for on in (1, 0):
+        old = lib.lcc_debug_set_decoder_fused(on)
+        try:
+            st = [m.new_stream() for _ in seqs]
+            m.forward_step([(s, x[:-1], []) for s, x in zip(st, seqs)])
+            before = ops.launch_counts()["gemv_rows_pair"]
+            res.append([g.clone() for g in m.forward_step([(s, [x[-1]], [0]) for s, x in zip(st, seqs)])])
+            assert ops.launch_counts()["gemv_rows_pair"] - before == (2 if on else 0)
+            for s in st:
+                s.release()
+        finally:
+            lib.lcc_debug_set_decoder_fused(old)
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+
+
+def test_a_wide_input_projection_keeps_a_launch_of_its_own(dev):
+    """64 rows, a query rank of 5120 beside a feed-forward of 8192 at width 2048: the projection's blocks of one tile would take longer than the launch saved."""
+    from livecc_amd import ops
+    from livecc_amd.config import DebunexConfig
+    for rank, paired in ((5120, 0), (256, 1)):
+        cfg = DebunexConfig(64, 2048, [U.L(U.M(2, 64, 64, rank, 128, 0.1), 8192)], 1e-5, 20.0, name="wide-in")
+        T = U.make_weights(cfg, 3)
+        m = _model(cfg, T, dev, max_streams=64, max_kv_len=64, max_new_rows=512)
+        st = [m.new_stream() for _ in range(64)]
+        m.forward_step([(s, [1 + i % 7, 2], []) for i, s in enumerate(st)])
+        before = ops.launch_counts()["gemv_rows_pair"]
+        m.forward_step([(s, [3], [0]) for s in st])
+        assert ops.launch_counts()["gemv_rows_pair"] - before == paired
+
+
 def test_fused_and_separate_decode_launches_agree(dev, lib):
     cfg = U.configs()["full-heads"]
     T = U.make_weights(cfg, 4)
