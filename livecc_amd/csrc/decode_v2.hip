@@ -861,10 +861,12 @@ int dgemv_down_qkv(const DgArgs& down, const DgArgs& qkv, unsigned* flag, unsign
 // [RMSNorm] gate/up Linear [SwiGLU]
 int dgemv_norm_swiglu(const DgArgs& a, hipStream_t st) {
   if (int rc = dg_check(a, DG_PRO_NORM, DG_EPI_SWIGLU)) return rc;
-  // Weight chunks a stage: two where a unit's blocks are one at most, or more than three, and a wave has eight or more of them (the norm goes on under the
-  // first two stages); between, their bytes only wait for one another.  us, one / two: [37888, 3584] 48.7 / 47.3, [59136, 8192] 157 / 155, [28672, 2048] 23.5 / 23.2, [4736, 3584]
-  // 13.0 / 10.7;  [9472, 3584] 16.5 / 16.8, [9472, 8192] 32.7 / 34.4, [18944, 3584] 28.0 / 28.2, [17920, 1536] 13.2 / 13.4, [8960, 1536] 8.2 / 9.1
-  const bool two = a.K >= 2048 && (a.N > 768 * 32 || a.N <= 256 * 32);
+  // Weight chunks a stage: two where a unit's blocks are one at most and a wave has eight or more of them, or more than three and it has more than nine (the norm
+  // goes on under the first two stages); between, their bytes only wait for one another.  us, one / two: [37888, 3584] 48.7 / 47.3, [59136, 8192] 157 / 155, [28672, 2048] 23.5 / 23.2, [4736, 3584]
+  // 13.0 / 10.7;  [9472, 3584] 16.5 / 16.8, [9472, 8192] 32.7 / 34.4, [18944, 3584] 28.0 / 28.2, [17920, 1536] 13.2 / 13.4, [8960, 1536] 8.2 / 9.1;
+  // another card, one row and two: [37888, 3584] 43.2 / 41.9 and 43.1 / 42.1, [8192, 3584] 12.5 / 11.3 and 13.3 / 12.4, [8192, 2048] 8.2 / 7.8 and 8.2 / 7.9, [37888, 2432] 30.1 / 29.4
+  // and 30.7 / 29.8, [24640, 2304] 21.1 / 21.0 and 20.9 / 21.3, [37888, 2048] 25.2 / 25.9 and 25.3 / 26.1
+  const bool two = a.N > 768 * 32 ? a.K >= 2432 : a.N <= 256 * 32 && a.K >= 2048;
   hipEvent_t ev0 = g_swiglu_ev0, ev1 = g_swiglu_ev1;
   g_swiglu_ev0 = g_swiglu_ev1 = nullptr;
   if (ev0 != nullptr && ev1 != nullptr && a.wscale == nullptr && a.M <= 2) {      // the profiled launch of the bf16 one-/two-stream kernel

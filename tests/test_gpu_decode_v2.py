@@ -34,9 +34,9 @@ def test_norm_swiglu_gemv(dev, M, N, K):
     assert_bf16_close(got, ref, f"dgemv_norm_swiglu[{M}x{N}x{K}]", max_ulp=1.0, max_frac=1e-2, atol=atol)
 
 
-@pytest.mark.parametrize("M,K", [(1, 2048), (2, 2112), (1, 2240), (2, 3584), (1, 8192)])
+@pytest.mark.parametrize("M,K", [(1, 2048), (2, 2112), (1, 2240), (1, 2432), (2, 2496), (2, 3584), (1, 8192)])
 def test_norm_swiglu_gemv_chunks_a_stage_give_the_same_bits(dev, M, K):
-    """Two weight chunks a stage (at most 8,192 rows, or more than 24,576) and one (between): the first rows of all three are the same weights, each wave adds
+    """Two weight chunks a stage (at most 8,192 rows, or more than 24,576 of at least 2,432 columns) and one (else): the first rows of all three are the same weights, each wave adds
     its chunks up in the same order, so the outputs agree bit for bit; odd counts of chunks."""
     from livecc_amd import ops
     h, w, nw = _rand((M, K), dev, 2.0, 1), _rand((24608, K), dev, 0.03, 2), _rand((K,), dev, 1.0, 3)
