@@ -69,8 +69,9 @@ int lcc_debug_set_gemv_variant(int variant);
 /* tiled kernels: 0 = 4-wave register-staged double-buffered LDS, 1 = 4-wave LDS-DMA (global_load_lds) 3-stage ring, 2 = scored per
  * shape (default: 8-wave 256x256 / 128x256 LDS-DMA kernel where its grid fills the chip, else the 4-wave kernels), 3 / 4 = force the
  * 8-wave kernel with 256 / 128 rows where eligible, 5 / 6 = the same with the compiler's fragment-read schedule, 7 = 2 without the
- * 8-wave kernel, 8 = force the "tall" kernel (one block row covers all of M <= 448, 448x160 tiles; SwiGLU: as many rows as there are) wherever it is legal; the default
- * takes it when ceil(N/160) fills 75-100 % of one round of the chip (LiveCC-7B gate/up of a streaming chunk) and M > 256, or M > 64 (fp8 weights: 128) with N > 32768;
+ * 8-wave kernel, 8 = force the "tall" kernel (one block row covers all of M <= 448, 448x160 tiles; SwiGLU, and bf16 weights from 257 rows: as many rows as there are) wherever it is legal; the default
+ * takes it when ceil(N/160) fills 75-100 % of one round of the chip (LiveCC-7B gate/up of a streaming chunk) and M > 256 (fp8 weights without SwiGLU: 384), or, SwiGLU, M > 64
+ * (fp8 weights: 128) with N > 32768, and 448 rows of A fit a 32-bit byte offset;
  * 13 = the 192-row 8-wave tile wherever eligible; 14 = row tiles of variable height (256 / 272 / 288 rows: ceil(M/16) row fragments dealt
  * out over floor(ceil(M/16)/16) tiles, no ragged last tile; round 5) wherever legal, else as 3 -- the default picks them by score (e.g. the
  * gate/up GEMM of 8 co-scheduled chunks: 12 x 148 tiles instead of 13 x 148); 15 = the SMALL variable-height class (row tiles of 128 / 144
