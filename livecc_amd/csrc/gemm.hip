@@ -10,7 +10,8 @@
 //  * gemm_walk_vh_kernel : the walk over row tiles of 256 / 272 / 288 rows (no ragged last row tile).
 //  * gemm_vh_kernel      : row tiles of 128 / 144 rows, split-K slabs of one streaming chunk.
 //  * gemm_tall_kernel    : one block row covers all of M (up to 448 rows: gate/up of one streaming chunk or of a few short ones; wide products of 257 rows and more).
-//  * gemm_mid_kernel     : shapes with few 256-column tiles.  64x128x64 (128x128x64) tile, 8 waves, 6- (4-) stage LDS-DMA ring.
+//  * gemm_strip_kernel   : shapes with few 256-column tiles.  64x128x64 tile, 4 waves, weights straight into registers, idle compute units fetch them ahead.
+//  * gemm_mid_kernel     : the same shapes with more rows.  128x128x64 tile, 8 waves, 4-stage LDS-DMA ring.
 //  * gemm_glds_kernel /   : row-major W, K % 64 != 0.  64x128x64 (128x128x64) tile, 4 waves,
 //    gemm_tiled_kernel     LDS-DMA 3-stage ring / register-staged double buffer with an XOR swizzle, XCD-aware block remap.
 //  * gemv_skinny_kernel  : M <= 64 (decode, lm_head; MG = ceil(M / 16) activation fragments per weight fragment).  HBM-bound weight streaming.  4 waves per block share 16 (32, 64) W rows,
@@ -24,6 +25,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
+#include <utility>
 
 #include "common.h"
 #include "kernels.h"
@@ -31,6 +33,7 @@
 
 namespace lcc {
 
+constexpr int STRIP_STAGES = 6;      // k-tiles a block of gemm_strip_kernel holds
 __device__ unsigned int lcc_zero_page[256];  // 1 KB of zeros: operand source of absent K chunks (address select, no branch)
 
 // Grid cap (round 5): while it is set (engine_vit.hip sets it around a vision-tower call that runs on the side stream UNDER another turn's
@@ -583,24 +586,17 @@ __global__ __launch_bounds__(256) void gemm_glds_kernel(
 }
 
 // ------------------------------------------------------------------------------------------------
-// 64 x 128 x 64 (128 x 128 x 64) tile on EIGHT waves with a deep LDS-DMA ring: shapes whose 256-column tiles leave most of the chip idle
+// 128 x 128 x 64 tile on EIGHT waves with a four-stage LDS-DMA ring: shapes whose 256-column tiles leave most of the chip idle
 // ------------------------------------------------------------------------------------------------
-// One streaming chunk's vision fc2 / proj (M = 1456, N = 1280) is 230 tiles of 64 x 128, one per compute unit: the time is the chain of K / 64
-// steps of one block, and a split of K would give another summation order.  gemm_glds_kernel spent 0.92 us a step on it (four waves, two
-// stages in flight: DMA round trip, fragment reads and MFMAs one after the other).  Here
-//   * five stages (120 KB) are in flight, so a step never waits for a round trip that is longer than four steps;
+// The time is the chain of K / 64 steps of one block, and a split of K would give another summation order.
+//   * three stages (96 KB) are in flight;
 //   * the fragments of tile kt + 1 are read into a second register set under the MFMAs of tile kt, behind the same barrier;
-//   * eight waves, each 32 (BM 128: 64) rows x 32 columns.
-// What bounds it now: LDS.  A step of the 64-row tile reads 64 KB of fragments and takes 24 KB from the DMA = 704 clocks at 128 B/clk against
-// 256 clocks of MFMA per SIMD; measured 0.33 us a step with 120 blocks, 0.40 with 230.  The 128-row tile reads 96 KB for twice the work.
-// Same summation order as every other tile kernel of this file.  Measured (us, gemm_glds_kernel or the tile chosen before -> here):
-// 1456 x 1280, K 5120 73 -> 31 (36 between the other launches of a tower); K 1280 22 -> 12; 720 x 1280, K 5120 72 -> 28; 390 x 3584, K 3584 without a split 23 (128 x 256 tiles: 50);
-// 128-row tile: 1000 x 3584, K 22528 285 -> 196; 2000 x 1280, K 5120 55 -> 41.
-// NST 6 / 4 stages (64- / 128-row tile): one block on a compute unit.  NST 3 (72 KB, two blocks): more than 256 blocks of the 64-row tile
-// (2912 x 1280, K 5120: 57 us, gemm_glds_kernel 77).
+//   * eight waves, each 64 rows x 32 columns.
+// What bounds it: LDS (a step reads 96 KB of fragments and takes 32 KB from the DMA = 1,024 clocks at 128 B/clk against 512 of MFMA per SIMD) and lines
+// from beyond the L2 (gemm_strip_kernel).  Same summation order as every other tile kernel of this file.  Measured (us, the tile chosen before -> here): 1000 x 3584,
+// K 22528 285 -> 196; 2000 x 1280, K 5120 55 -> 41.
 // Requires packed W, K % 64 == 0.  W8: fp8 weights in their packed order, 1 KB a fragment's 64 k, converted in registers in front of the
-// MFMAs (the form before wrote the whole weight as bf16 first): 386 x 4608, K 3584 34.5 -> 25; 64 rows in four splits, [3584, 18944] 58 -> 29,
-// [3584, 3584] 20 -> 9.3; 128-row tile: 600 x 4608, K 3584 50 -> 34.
+// MFMAs (the form before wrote the whole weight as bf16 first): 600 x 4608, K 3584 50 -> 34.
 template <int BM, int EPI, int NST, bool W8>
 __global__ __launch_bounds__(512) void gemm_mid_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual,
@@ -718,6 +714,161 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(
     tile_epilogue_wide<EPI, MT, NT>(acc, m0 + wm * (BM / 2), n0 + wn * 32, lane, bias, residual, ldr, C, ldc, M, N, wscale,
                                     reinterpret_cast<unsigned char*>(dsmem) + wave * 4096);
   } else tile_epilogue<EPI, MT, NT>(acc, m0 + wm * (BM / 2), n0 + wn * 32, (n0 + wn * 32) / 2, li, g, bias, residual, ldr, C, ldc, M, N, partial, wscale);
+  if (vb + (int)gridDim.x < nblk) __syncthreads();     // the next tile's DMA reuses the stages
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// The 64 x 128 tile: FOUR waves, one a SIMD, each 64 rows x 32 columns; the weights go from memory into registers
+// ------------------------------------------------------------------------------------------------
+// With 32 columns of its own a wave is the only reader of its weight fragments: LDS holds the activations alone, and a k-step moves 32 + 8 KB through it instead
+// of 64 + 24 (gemm_mid_kernel's form: 32 x 32 a wave).  One step in source order: the activation fragments of tile kt + 1, a piece of what tile kt + D - 1 needs
+// and the MFMAs of tile kt by turns, so that a wave alone on its SIMD is never held by a burst of loads.
+// What bounds it then: what a compute unit takes from beyond its L2.  Lines that are there arrive at 135-150 B/ns, lines that the blocks of an XCD ask for
+// together and that come from memory at 45-58, whatever is in flight (2 to 8 steps measured the same): 24 KB a step are 0.16 us or 0.42.  So
+//   * compute units that get no tile read the weight ahead of the others into the memory-side cache (strip_fetch), whose lines come sooner than DRAM's;
+//   * nothing is requested past the last tile but what the full groups of D steps do.
+// Measured (us, weights from memory; the eight-wave form before -> these -> with fetching blocks): 1456 x 1280, K 5120 35.3 -> 33.0 -> 28.8, K 1280 10.6 -> 9.8;
+// 720 x 1280, K 5120 29.2 -> 28.7 -> 25.5; 390 x 3584, K 3584 23.7 -> 22.4 -> 20.5; 1120 x 1280, K 5184 30.9 -> 30.3 -> 25.4.
+// Not taken: weight loads past the caches (nt: 33 -> 40, the other blocks of the XCD fetch them again), 8 to 12 steps ahead (no faster), a dword of every line ahead of
+// its use by the block itself (loads return in order: slower), 128 rows x 32 columns a wave (2 to 4 % either way of gemm_mid_kernel<128>).
+// Same summation order as every other tile kernel of this file.  Requires packed W, K % 64 == 0.  W8: fp8 weights in their packed order, 1 KB a fragment's 64 k,
+// converted in registers in front of the MFMAs.
+// Blocks without a tile read 2 KB of every fragment row by turns, from piece c0 to c1 of the rows (`row` pieces of 16 bytes each), in the order in which the others will
+LCC_DEVICE void strip_fetch(const bf16_t* W, int row, int nfrag, int c0, int c1, int e, int ne) {
+  const u32x4* src = reinterpret_cast<const u32x4*>(W) + (threadIdx.x & 127);
+  const int half = threadIdx.x >> 7, pairs = (nfrag + 1) >> 1, items = (c1 - c0) * pairs;
+  for (int i0 = e; i0 < items; i0 += 8 * ne) {
+    u32x4 v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int i = min(i0 + u * ne, items - 1), c = i / pairs, fr = min((i - c * pairs) * 2 + half, nfrag - 1);
+      v[u] = src[(size_t)fr * row + (size_t)(c0 + c) * 128];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) asm volatile("" ::"v"(v[u]));
+  }
+}
+template <int... U, class F>
+LCC_DEVICE void strip_steps(std::integer_sequence<int, U...>, F f) { (f(std::integral_constant<int, U>{}), ...); }
+template <int EPI, bool W8>
+__global__ __launch_bounds__(256, 2) void gemm_strip_kernel(
+    const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual,
+    int ldr, bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n, float* __restrict__ partial, int kt_per_split,
+    const float* __restrict__ wscale, int raster, int fetch) {
+  constexpr int BM = 64, BK = 64, MT = BM / 16, NT = 2, D = STRIP_STAGES;
+  constexpr int WF = W8 ? 1 : 2;                                  // 1-KB weight sub-tiles of a fragment row
+  constexpr int STAGE = BM * 8;                                   // 16-byte units: [BM rows][8 chunks] (XOR-swizzled) = 8 KB
+  constexpr int APW = BM / 32, P = APW + WF * NT;                 // a wave's memory instructions of a k-tile: 8 activation rows each, then its weights
+  extern __shared__ __attribute__((aligned(16))) u32x4 dsmem[];
+  static_assert((D & 1) == 0 && P <= 2 * MT, "the two fragment sets alternate; a piece beside every fragment");
+
+  const int nkt_all = K / BK;
+  const int kt0 = (EPI == EPI_PARTIAL) ? blockIdx.y * kt_per_split : 0;
+  const int nkt = (EPI == EPI_PARTIAL) ? min(nkt_all, kt0 + kt_per_split) : nkt_all;
+  const int nblk = tiles_m * tiles_n;
+  if ((int)blockIdx.x >= nblk) {                  // the last `fetch` k-tiles of this split
+    strip_fetch(W, nkt_all * WF * 64, (N + 15) >> 4, max(kt0, nkt - fetch) * WF / 2, nkt * WF / 2, (int)blockIdx.x - nblk, (int)gridDim.x - nblk);
+    return;
+  }
+  for (int vb = blockIdx.x; vb < nblk; vb += gridDim.x) {     // one tile per block, or a persistent walk under the grid cap
+  int bid = vb;
+  {
+    const int q = nblk >> 3, r = nblk & 7, xcd = bid & 7, idx = bid >> 3;
+    bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
+  }
+  int tn, tm;                                     // tile order: see gemm_big_kernel
+  if (raster > 0) {
+    const int band = bid / (raster * tiles_m), rem = bid - band * raster * tiles_m;
+    const int bw = min(raster, tiles_n - band * raster);
+    tm = rem / bw;
+    tn = band * raster + (rem - tm * bw);
+  } else {
+    tn = bid / tiles_m;
+    tm = bid - tn * tiles_m;
+  }
+  const int m0 = tm * BM, n0 = tn * 128;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15, g = lane >> 4;
+  const int nfrag = (N + 15) >> 4;
+
+  const bf16_t* asrc[APW];
+#pragma unroll
+  for (int q = 0; q < APW; ++q) asrc[q] = A + (size_t)min(m0 + (wave + 4 * q) * 8 + (lane >> 3), M - 1) * lda + (((lane & 7) ^ (lane >> 3)) << 3);
+  const bf16_t* bsrc[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) bsrc[j] = W + (size_t)min((n0 >> 4) + wave * NT + j, nfrag - 1) * (nkt_all * WF) * 512 + lane * 8;
+  const unsigned lds0 = lds_addr(dsmem) + wave * 1024u;
+
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  int aoff[2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) aoff[kk] = li * 8 + ((W8 ? g * 2 + kk : kk * 4 + g) ^ (li & 7));
+  bf16x8 f[2][2][MT];                             // activation fragments of two k-tiles
+  u32x4 w[D][WF][NT];                             // weights of D
+  // piece q of k-tile k (in range) into stage and weight set u
+  auto issue = [&](int q, int k, auto uc) {
+    constexpr int u = decltype(uc)::value;
+    if (q < APW) glds16(asrc[q < APW ? q : 0] + (size_t)k * BK, lds0 + (unsigned)(u * STAGE * 16 + (q < APW ? q : 0) * 4096));
+    else if (q < P) {
+      const int h = (q - APW) / NT, j = (q - APW) % NT;
+      w[u][h % WF][j] = ld16(bsrc[j] + (size_t)k * (WF * 512) + h * 512);
+    }
+  };
+  // The stage and weight set of tile kt is u.  Tile kt + 1 has landed (the waits count every piece issued behind it: the barriers to the scheduler keep them in this
+  // order) -> block barrier -> its fragments are read, tile kt + D - 1 goes into the stage and the registers of tile kt - 1, whose fragments were in registers before
+  // the barrier, and tile kt is multiplied.  DRAIN > 0: the last steps, with nothing to request (past the last tile sources are clamped: stages nobody reads any more)
+  auto step = [&](int kt, auto uc, auto dc) {
+    constexpr int u = decltype(uc)::value, drain = decltype(dc)::value;
+    constexpr std::integral_constant<int, (u + D - 1) % D> un{};
+    const int k = min(kt + D - 1, nkt - 1);
+    const u32x4* s = dsmem + ((u + 1) % D) * STAGE;
+    constexpr int behind = drain == 0 ? D - 3 : D - 2 - drain;
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(behind > 0 ? P * behind : 0) : "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    bf16x8 b[2][NT];
+#pragma unroll
+    for (int q = 0; q < 2 * MT; ++q) {
+      const int kk = q / MT, i = q % MT;
+      f[(u + 1) & 1][kk][i] = as_bf16x8(s[aoff[kk] + i * 128]);
+      if (drain == 0) issue(q, k, un);
+      if (i == 0) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) b[kk][j] = W8 ? fp8x8_to_bf16x8(w[u][0][j][2 * kk], w[u][0][j][2 * kk + 1]) : as_bf16x8(w[u][kk % WF][j]);
+      }
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[i][j] = mfma16(b[kk][j], f[u & 1][kk][i], acc[i][j]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  __builtin_amdgcn_sched_barrier(0);
+  strip_steps(std::make_integer_sequence<int, D - 1>{}, [&](auto uc) {
+#pragma unroll
+    for (int q = 0; q < P; ++q) issue(q, min(kt0 + decltype(uc)::value, nkt - 1), uc);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(P * (D - 2)) : "memory");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int q = 0; q < 2 * MT; ++q) f[0][q / MT][q % MT] = as_bf16x8(dsmem[aoff[q / MT] + (q % MT) * 128]);
+  int kt = kt0;
+  for (; kt + D <= nkt; kt += D) strip_steps(std::make_integer_sequence<int, D>{}, [&](auto uc) { step(kt + decltype(uc)::value, uc, std::integral_constant<int, 0>{}); });
+  const int rem = nkt - kt;
+  strip_steps(std::make_integer_sequence<int, D - 1>{}, [&](auto uc) {
+    if (decltype(uc)::value < rem) step(kt + decltype(uc)::value, uc, std::integral_constant<int, decltype(uc)::value + 1>{});
+  });
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the clamped copies
+  if (wide_rows<EPI>(C, ldc, bias, residual, ldr)) {
+    __builtin_amdgcn_s_barrier();          // every wave is done with the stages, and its DMA pieces have landed
+    tile_epilogue_wide<EPI, MT, NT>(acc, m0, n0 + wave * 32, lane, bias, residual, ldr, C, ldc, M, N, wscale,
+                                    reinterpret_cast<unsigned char*>(dsmem) + wave * 4096);
+  } else tile_epilogue<EPI, MT, NT>(acc, m0, n0 + wave * 32, (n0 + wave * 32) / 2, li, g, bias, residual, ldr, C, ldc, M, N, partial, wscale);
   if (vb + (int)gridDim.x < nblk) __syncthreads();     // the next tile's DMA reuses the stages
   }
 }
@@ -1601,12 +1752,29 @@ static void launch_mid_w(const GemmArgs& a, hipStream_t st) {
 }
 template <int BM, int EPI, int NST>
 static void launch_mid(const GemmArgs& a, hipStream_t st) { a.w_fp8 ? launch_mid_w<BM, EPI, NST, true>(a, st) : launch_mid_w<BM, EPI, NST, false>(a, st); }
-// the 64 x 128 tile
-template <int EPI>
-static void launch_mid64(const GemmArgs& a, hipStream_t st) {
-  const long blocks = (long)capped_grid((long)((a.M + 63) / 64) * ((a.N + 127) / 128)) * (EPI == EPI_PARTIAL ? a.nsplit : 1);
-  return blocks <= 256 ? launch_mid<64, EPI, 6>(a, st) : launch_mid<64, EPI, 3>(a, st);
+// The 64 x 128 tile.  Compute units left over by its blocks fetch weights ahead of them (strip_fetch): a block passes on some 50 B/ns and a step of the others takes
+// 0.32 us, so that N / 60 blocks (fp8: N / 120) keep ahead of them from the first step on; fewer take the k-tiles at the end that they reach in time, under two
+// fifths of them none (1456 x 1280, K 5120, us: none 33.5, 16 blocks 32.2, 26 28.8; all of 390 x 3584, K 3584 on 16 blocks 42, on 60 20.5, none 22.4).
+static int strip_fetch_blocks(int tiles, int N, int S, int nkt, bool w8, int* fetch) {
+  const int idle = get_grid_cap() > 0 ? 0 : (256 - tiles * S) / S;
+  const long reach = (long)idle * (w8 ? 120 : 60) * nkt / N;      // k-tiles of a split
+  *fetch = (int)std::min<long>(reach, nkt);
+  return idle > 0 && *fetch * 5 >= nkt * 2 ? idle : 0;
 }
+template <int EPI, bool W8>
+static void launch_strip_w(const GemmArgs& a, hipStream_t st) {
+  const int tiles_m = (a.M + 63) / 64, tiles_n = (a.N + 127) / 128, S = (EPI == EPI_PARTIAL) ? a.nsplit : 1, nkt = (a.K / 64 + S - 1) / S;
+  const long tiles = (long)tiles_m * tiles_n;
+  int fetch = 0;
+  const int extra = tiles * S < 256 ? strip_fetch_blocks((int)tiles, a.N, S, nkt, W8, &fetch) : 0;
+  constexpr size_t lds = (size_t)STRIP_STAGES * 8192;
+  static DeviceOnce attr_set;   // per instantiation
+  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_strip_kernel<EPI, W8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  gemm_strip_kernel<EPI, W8><<<dim3(capped_grid(tiles) + extra, S), dim3(256), lds, st>>>(
+      a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.partial, nkt, a.wscale, raster_for(tiles_m), fetch);
+}
+template <int EPI>
+static void launch_mid64(const GemmArgs& a, hipStream_t st) { a.w_fp8 ? launch_strip_w<EPI, true>(a, st) : launch_strip_w<EPI, false>(a, st); }
 template <int BM, int EPI>
 static void launch_tiled(const GemmArgs& a, hipStream_t st) {
   if constexpr (BM == 64) {

@@ -244,7 +244,7 @@ def test_gemm_variable_height_tiles_are_bit_identical_to_the_256_row_tiles(dev, 
     (2912, 1280, 192, 3, 7), (1031, 2320, 256, 1, 7), (65, 144, 64, 0, 16), (129, 272, 128, 3, 16), (257, 144, 192, 2, 16), (720, 1280, 448, 1, 16),
     (100, 544, 320, 4, 16), (1000, 3584, 1536, 3, 2)])
 def test_gemm_128_column_tiles_are_bit_identical_to_the_256_row_tiles(dev, M, N, K, epi, variant):
-    """64 x 128 tiles (6 stages up to 256 tiles, 3 stages beyond: 2912 x 1280, 1031 x 2320) and 128 x 128 tiles (variant 16): one k-tile, fewer
+    """64 x 128 tiles (up to 256 of them, and more: 2912 x 1280, 1031 x 2320) and 128 x 128 tiles (variant 16): one k-tile, fewer
     k-tiles than stages, odd and even counts, one row past a tile, a ragged last column tile, every epilogue; the summation order is that of
     the 256-row tiles."""
     from livecc_amd import ops
@@ -261,6 +261,33 @@ def test_gemm_128_column_tiles_are_bit_identical_to_the_256_row_tiles(dev, M, N,
     finally:
         ops.set_gemm_variant(ops.GEMM_DEFAULT_VARIANT)
     assert torch.equal(got, ref), f"{int((got != ref).sum())} of {got.numel()} outputs differ from the 256-row tiles"
+
+
+@pytest.mark.parametrize("M,N", [(65, 144), (100, 272), (1456, 1280), (1500, 1280), (1600, 1280)])
+@pytest.mark.parametrize("nkt", [1, 2, 5, 6, 7, 11, 12, 13, 16, 20])
+@pytest.mark.parametrize("fp8", [False, True], ids=["bf16", "fp8"])
+def test_gemm_64_row_tile_every_remainder_of_its_stages(dev, M, N, nkt, fp8):
+    """64 x 128 tiles: one k-tile, every kind of remainder of the six that a block holds; blocks without a tile that read all of the weight ahead (an odd
+    number of fragment rows, of 64-k pieces), its last three quarters (1500 rows), none of it (1600); three splits.  The bits of the 256-row tiles."""
+    from livecc_amd import ops
+    K, S = 64 * nkt, min(3, nkt)
+    x, w, b = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.05, 2), _rand((N,), dev, 0.1, 3)
+    w8, sc = ops.quantize_fp8(w.float())
+    wp = ops.pack_weight(w)
+
+    def both():
+        if fp8:
+            return ops.linear_w8(x, w8, sc, b, ops.EPI_NONE), ops.linear_w8(x, w8, sc, None, ops.EPI_QUICK_GELU)
+        return ops.linear(x, wp, b, ops.EPI_NONE, packed_shape=(N, K)), ops.linear_partial(x, wp, S, packed_shape=(N, K))
+    try:
+        ops.set_gemm_variant(3)
+        ref = both()
+        ops.set_gemm_variant(7)
+        got = both()
+    finally:
+        ops.set_gemm_variant(ops.GEMM_DEFAULT_VARIANT)
+    for g, r in zip(got, ref):
+        assert torch.equal(g, r), f"{int((g != r).sum())} of {g.numel()} values differ from the 256-row tiles"
 
 
 @pytest.mark.parametrize("variant", [3, 4, 13, 14, 16, 7])
