@@ -128,8 +128,9 @@ class EngineModel:
         self.device = torch.device(device)
         if max_kv_len is None:
             max_kv_len = cfg.max_position_embeddings + max_history
+        self.max_patches = max_patches
         self.engine = Engine(cfg, weights, self.device, max_slots=max_streams, max_kv_len=max_kv_len,
-                             max_new_rows=max_new_rows, max_patches=max_patches, max_history=max_history)
+                             max_new_rows=max_new_rows, max_patches=max_patches + max_patches // 8, max_history=max_history)
         self._free_slots = list(range(max_streams - 1, -1, -1))
         self._lock = threading.RLock()          # every engine entry point below holds it for the whole call (see the module docstring)
         self.generation_config: dict = {}            # from_pretrained fills it from generation_config.json (do_sample / top_k ...)
@@ -428,7 +429,8 @@ class LiveCCForConditionalGeneration(EngineModel):
         max_new_rows    = rows of ONE prefill launch sequence -- longer prompts (the one-shot 24k-token video_qa / MCQ prefill)
                           are cut into pieces of at most this many rows over the carried KV (bit-identical to one pass);
         max_patches     = ViT patches of ONE encode launch sequence -- longer clips are encoded in groups of temporal slices
-                          (slices never attend to each other, Q2VL vision_utils.py:60-65);
+                          (slices never attend to each other, Q2VL vision_utils.py:60-65); the workspace has room for an eighth
+                          more, so that a short last group goes with the one before it;
         max_kv_len      = KV capacity per stream; default = the trained 32k window + max_history of generation headroom.
         text_offset_rule: "hf4" = transformers-4.5x M-RoPE text offset after a vision block (what the released checkpoints
         were trained with, ref README.md:30); "hf5" = the installed 5.15 oracle's rule.  Identical for every streaming chunk;
@@ -642,21 +644,21 @@ class LiveCCForConditionalGeneration(EngineModel):
                 T = f.shape[0]
                 H, W = (f.shape[1], f.shape[2]) if lay == "THWC" else (f.shape[2], f.shape[3])
                 per_slice = (H // cfg.patch_size) * (W // cfg.patch_size)
-                slices = max(1, eng.max_patches // per_slice)
-                if per_slice > eng.max_patches:
-                    raise ValueError(f"one {H}x{W} frame pair is {per_slice} patches > max_patches {eng.max_patches}")
+                slices = max(1, self.max_patches // per_slice)
+                if per_slice > self.max_patches:
+                    raise ValueError(f"one {H}x{W} frame pair is {per_slice} patches > max_patches {self.max_patches}")
                 step = slices * cfg.temporal_patch_size
                 for a in range(0, T, step):
                     pieces.append(dict(frames=f[a:a + step], layout=lay))
             else:
                 t, h, w = (int(x) for x in c["grid"])
                 per_slice = h * w
-                slices = max(1, eng.max_patches // per_slice)
+                slices = max(1, self.max_patches // per_slice)
                 pv = c["pixel_values"]
                 for a in range(0, t, slices):
                     b = min(t, a + slices)
                     pieces.append(dict(pixel_values=pv[a * per_slice:b * per_slice], grid=(b - a, h, w)))
-        groups, cur, cur_p = [], [], 0
+        groups, rows, cur, cur_p = [], [], [], 0
         for pc in pieces:
             if "frames" in pc:
                 f, lay = pc["frames"], pc["layout"]
@@ -664,11 +666,15 @@ class LiveCCForConditionalGeneration(EngineModel):
                 n = ((f.shape[0] + 1) // 2) * (H // cfg.patch_size) * (W // cfg.patch_size)
             else:
                 n = pc["grid"][0] * pc["grid"][1] * pc["grid"][2]
-            if cur and cur_p + n > eng.max_patches:
-                groups.append(cur); cur, cur_p = [], 0
+            if cur and cur_p + n > self.max_patches:
+                groups.append(cur); rows.append(cur_p); cur, cur_p = [], 0
             cur.append(pc); cur_p += n
         if cur:
-            groups.append(cur)
+            groups.append(cur); rows.append(cur_p)
+        # A last group of one slice walks the whole tower at a twentieth of the chip's rate: with the group before it where the workspace holds both (19 slices of
+        # 880 patches as 18 + 1 / together 27.6 / 25.0 ms; pieces of equal size instead were slower for other clips, 12 slices of 1,456 32.0 / 32.6)
+        if len(groups) > 1 and rows[-2] + rows[-1] <= eng.max_patches:
+            groups[-2:] = [groups[-2] + groups[-1]]
         # EVERY vision-tower launch goes through here: the tower has ONE private workspace + meta ring (lcc_engine_bind_vit_buffers),
         # so the issuing stream first waits for the previous ViT call -- wherever it ran (main stream, prefetch side stream,
         # get_video_features) -- and leaves an event behind for the next one.  Never two ViT calls in flight.

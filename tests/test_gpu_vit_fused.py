@@ -112,3 +112,18 @@ def test_tower_under_a_grid_cap_is_bit_identical(dev, streams, cap):
     assert torch.equal(ref, got), f"{int((ref != got).sum())} of {ref.numel()} embedding values differ under a cap of {cap} workgroups"
     assert torch.equal(ref, again)
     record(f"vit_tower_grid_cap[{streams} streams, {cap} CUs]", dict(tower_ms=min(ms)))
+
+
+@pytest.mark.parametrize("slices,calls", [(8, 1), (9, 1), (10, 2), (16, 2), (17, 2), (18, 3), (25, 3)])
+def test_a_short_last_group_of_a_clip_goes_with_the_one_before_it(dev, slices, calls, monkeypatch):
+    """max_patches of eight slices, room for nine: a ninth, 17th or 25th slice rides along, two do not.  The features are those of the slices by themselves up to
+    bf16 rounding (other products by the number of rows; a change of rounding in one layer of a random tower shows as 1.3e-2 of the norm behind the last)."""
+    from livecc_amd.config import tiny
+    native = _model(tiny(), dev, max_patches=8 * 24)
+    f = torch.randint(0, 256, (2 * slices - 1, 3, 56, 84), dtype=torch.uint8, generator=torch.Generator().manual_seed(slices)).to(dev)
+    seen, encode = [], native.engine.vit_encode
+    monkeypatch.setattr(native.engine, "vit_encode", lambda g, stream=None: seen.append(sum((c["frames"].shape[0] + 1) // 2 for c in g)) or encode(g, stream=stream))
+    got = native.get_video_features(frames=f).float()
+    assert len(seen) == calls and sum(seen) == slices and max(seen) <= 9
+    want = torch.cat([native.get_video_features(frames=f[2 * i:2 * i + 2]) for i in range(slices)]).float()
+    assert (got - want).norm() <= 2e-2 * want.norm()
