@@ -4,7 +4,8 @@
 // engine's (engine.hip, engine_llm.hip); this file is the launch sequence of the layers and what they need in memory.
 //
 // A layer is
-// (decode steps of up to 16 rows fuse "in" with "ff", the norms with "query", and "out" with the residual and the next norm: decode_v2.hip)
+// (decode steps of up to 16 rows fuse "in" with "ff", the norms with "query", and "out" with the residual and the next norm: decode_v2.hip; where a head's part of the
+// query projection is small, the norms, "query" and the absorption are one launch at any number of rows: latent_query)
 //   in      [Wdq | Wdkv | Wg] h           one GEMM, fp32 slabs
 //           norms -> query latent, c -> cache, gates          (latent_norm_append)
 //   query   Wuq cq                                            GEMM
@@ -83,7 +84,7 @@ int carve_bound(lcc_engine* e, DecBuffers* b) {
 }
 
 }  // namespace
-int g_fused_decode = 1;      // lcc_debug_set_decoder_fused: decode steps of up to 16 rows run the fused launches (6 per layer instead of 9), of 17 to 64 eight
+int g_fused_decode = 1;      // lcc_debug_set_decoder_fused: decode steps run the fused launches (up to 16 rows five or six per layer instead of nine, of 17 to 64 six to eight)
 
 namespace {
 // S packed rows through every layer; pt null: a decode step over the streams `d_slots`.  On exit b.h holds the final norm of the residual.
@@ -113,8 +114,9 @@ int run_decoder_layers(lcc_engine* e, const DecBuffers& b, int S, const PrefillT
     LatentInArgs in; in.part = b.part; in.nsplit = ns; in.rows = S; in.ldn = in_n; in.qp = L.q_rank_pad; in.rp = own ? rp : 0; in.q_rank = L.q_rank;
     in.kv_rank = L.kv_rank; in.heads = L.heads; in.eps = e->dc.norm_eps; in.q_norm = w.q_norm; in.kv_norm = w.kv_norm; in.cq = b.cq; in.gate = b.gate;
     in.tok_stream = pt ? pt->tok_stream : d_slots; in.tok_pos = pt ? pt->tok_pos : nullptr; in.kv_len = e->d_kv_len; in.kv_base = e->d_kv_base; in.kv_off = kv_off;
-    const bool fused_q = fused && dgemv_latent_q_ok(S, L.q_rank_pad);
-    if (!fused_q) LCC_TRY(latent_norm_append(in, st));
+    const bool query = !pt && g_fused_decode && latent_query_ok(S, L.heads, L.dim_pad, L.q_rank_pad);
+    const bool fused_q = !query && fused && dgemv_latent_q_ok(S, L.q_rank_pad);
+    if (!fused_q && !query) LCC_TRY(latent_norm_append(in, st));
     if (pt) {
       LCC_TRY(plain_gemm(b.cq, L.q_rank_pad, w.uq_w, b.q, L.heads * L.dim_pad, S, L.heads * L.dim_pad, L.q_rank_pad, LCC_EPI_NONE, st));
       for (const KeyGroup& kg : pt->groups) {
@@ -130,7 +132,9 @@ int run_decoder_layers(lcc_engine* e, const DecBuffers& b, int S, const PrefillT
       }
     } else {
       float* q32 = b.part;
-      if (fused_q) {
+      if (query) {
+        LCC_TRY(latent_query(in, w.uq_w, w.ukt_w, L.dim_pad, rp, b.lat_q, st));
+      } else if (fused_q) {
         q32 = b.part + align_up((size_t)S * in_n, 64);      // beside the input projection it reads
         DgArgs gq; gq.W = w.uq_w; gq.M = S; gq.N = L.heads * L.dim_pad; gq.K = L.q_rank_pad; gq.S32 = b.part; gq.lds32 = in_n; gq.rank = L.q_rank;
         gq.norm_w = w.q_norm; gq.eps = e->dc.norm_eps; gq.C32 = q32; gq.ldc = gq.N;
@@ -139,7 +143,7 @@ int run_decoder_layers(lcc_engine* e, const DecBuffers& b, int S, const PrefillT
       } else {
         LCC_TRY(slab_gemm(b, b.cq, L.q_rank_pad, w.uq_w, S, L.heads * L.dim_pad, L.q_rank_pad, &ns, st));
       }
-      LCC_TRY(latent_absorb(q32, ns, S, L.heads, L.dim_pad, w.ukt_w, rp, b.lat_q, st));
+      if (!query) LCC_TRY(latent_absorb(q32, ns, S, L.heads, L.dim_pad, w.ukt_w, rp, b.lat_q, st));
       LatentDecodeArgs a; a.q = b.lat_q; a.rows = S; a.heads = L.heads; a.rp = rp; a.nsplit = nsplit_attn; a.scale_log2e = scale_log2e; a.slots = d_slots;
       a.kv_len = e->d_kv_len; a.kv_base = e->d_kv_base; a.kv_off = kv_off; a.ws_o = b.ws_o; a.ws_ml = b.ws_ml; a.direct = direct;
       LCC_TRY(latent_attn_decode(a, st));

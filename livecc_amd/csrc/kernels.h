@@ -29,7 +29,8 @@ enum LaunchCounter {
   LC_GEMM_VH = 14,             // gemm_walk_vh_kernel (row tiles of 256 / 272 / 288 rows), gemm_vh_kernel (small class 128 / 144; round 5 -- the slot of the retired gemm_pp_kernel)
   LC_GEMM_VIT_QKV = 15,        // gemm_vit_kernel: EPI_VIT_QK / EPI_VIT_V epilogues (RoPE / V transpose fused into the q|k|v projection; one EPI_VIT_QKV launch per tower block when E % 128 == 0, else a q|k launch + a V launch)
   LC_GEMV_ROWS_PAIR = 16,      // gemv_rows_pair_kernel (input projection and gate/up of 17 to 64 rows in one launch)
-  LC_COUNT = 17
+  LC_LATENT_QUERY = 17,        // latent_query_kernel (query norm, up-projection and absorption in one launch)
+  LC_COUNT = 18
 };
 extern long long g_launch_counts[LC_COUNT];
 
@@ -291,6 +292,8 @@ struct MhaArgs {                 // causal multi-head attention of packed rows o
 constexpr int MHA_GROUP_ROWS = 256;
 int attn_mha(const MhaArgs& a, hipStream_t st);
 int attn_mha32_launch(const MhaArgs& a, hipStream_t st);      // dim, vdim in {64, 128}
+bool latent_query_ok(int rows, int heads, int dim, int qp);
+int latent_query(const LatentInArgs& a, const bf16_t* uq, const bf16_t* ukt, int dim, int rp, bf16_t* out, hipStream_t st);      // norms, q, absorb in one launch
 int latent_absorb(const float* q_part, int nsplit, int rows, int heads, int dim, const bf16_t* ukt, int rp, bf16_t* out, hipStream_t st);
 constexpr int LATENT_MAX_SPLIT = 128;
 struct LatentDecodeArgs {

@@ -196,6 +196,111 @@ int latent_absorb(const float* q_part, int nsplit, int rows, int heads, int dim,
 }
 
 // ------------------------------------------------------------------------------------------------------------------------------
+// Decode, norms and step 1 in one launch: the query latents' norm, q_h = Uq_h cq and a_h = Uk_h^T q_h; caches and gates beside them.  128 channels a head.
+// Block = (128 ranks, head, RG rows), 8 waves: each norms RG / 8 rows into LDS, forms 16 channels of the head over the whole query rank, then 16 ranks.  The head's Uq
+// is requested before the norm; the blocks of a head's other ranks and rows form q again from the same lines.  The blocks behind the ranks (blockIdx.x = parts) append
+// and gate, a row after another.
+// Bound by what one compute unit pulls, about 50 B/ns: Uq_h (query rank x 256 bytes), 32 KB of Uk_h and the rows' slabs.
+// ------------------------------------------------------------------------------------------------------------------------------
+constexpr int LATENT_Q_PIECES = 3;             // 256-channel pieces of the widest query rank
+template <int RG>
+__global__ __launch_bounds__(512, 2) void latent_query_kernel(LatentInArgs a, const bf16_t* __restrict__ uq, const bf16_t* __restrict__ ukt, int rp, int parts,
+                                                              bf16_t* __restrict__ out) {
+  constexpr int DIM = 128, PQ = LATENT_Q_PIECES, PITCH = PQ * 256 + 8, QP = DIM + 8, RW = RG / 8;
+  __shared__ __attribute__((aligned(16))) bf16_t s_x[RG * PITCH];       // normed latents, zeros beyond the rank
+  __shared__ __attribute__((aligned(16))) bf16_t s_q[RG * QP];
+  __shared__ float s_red[16];
+  const int h = blockIdx.y, b0 = blockIdx.z * RG, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, g = lane >> 4;
+  const int nrow = min(RG, a.rows - b0);
+  if ((int)blockIdx.x == parts) {
+    for (int r = h; r < nrow; r += gridDim.y) {
+      latent_row<512, false>(a, b0 + r, s_red);
+      __syncthreads();
+    }
+    return;
+  }
+  // this wave's rows: the first two slabs of a piece and its weight, in flight together
+  const size_t slab = (size_t)a.rows * a.ldn, second = a.nsplit > 1 ? slab : 0;
+  f32x4 v[RW][PQ], u[RW][PQ];
+  u32x2 nw[PQ];
+#pragma unroll
+  for (int p = 0; p < PQ; ++p) {
+    const int c = min(p * 256 + lane * 4, a.qp - 4);
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+      const float* src = a.part + (size_t)(b0 + min(wave * RW + r, nrow - 1)) * a.ldn + c;
+      v[r][p] = *reinterpret_cast<const f32x4*>(src);
+      u[r][p] = *reinterpret_cast<const f32x4*>(src + second);
+    }
+    nw[p] = ld8(a.q_norm + c);
+  }
+  __builtin_amdgcn_sched_barrier(0);          // ahead of the weights: loads return in order
+  const int KB = a.qp >> 5, tiles = rp >> 4, tile = (int)blockIdx.x * 8 + wave;
+  const bf16_t* wq = uq + (size_t)(h * (DIM / 16) + wave) * KB * 512 + lane * 8;
+  u32x4 wf[PQ][8], uk[4];
+#pragma unroll
+  for (int b = 0; b < PQ; ++b)
+#pragma unroll
+    for (int k = 0; k < 8; ++k) wf[b][k] = ld16(wq + (size_t)min(b * 8 + k, KB - 1) * 512);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) uk[k] = ld16(ukt + ((size_t)(h * tiles + min(tile, tiles - 1)) * 4 + k) * 512 + lane * 8);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int r = 0; r < RW; ++r) {
+    const int row = wave * RW + r;
+    const float* src = a.part + (size_t)(b0 + min(row, nrow - 1)) * a.ldn;
+    float ss = 0.f;
+#pragma unroll
+    for (int p = 0; p < PQ; ++p) {
+      const int c = p * 256 + lane * 4;
+      if (a.nsplit > 1) v[r][p] += u[r][p];
+      for (int s = 2; s < a.nsplit; ++s) v[r][p] += *reinterpret_cast<const f32x4*>(src + s * slab + min(c, a.qp - 4));
+      if (c >= a.qp) v[r][p] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      ss += (v[r][p][0] * v[r][p][0] + v[r][p][1] * v[r][p][1]) + (v[r][p][2] * v[r][p][2] + v[r][p][3] * v[r][p][3]);
+    }
+    const float inv = 1.f / sqrtf(wave_sum(ss) / (float)a.q_rank + a.eps);      // padding channels are zeros: the mean is over the real ones
+#pragma unroll
+    for (int p = 0; p < PQ; ++p)
+      st8(s_x + row * PITCH + p * 256 + lane * 4, (u32x2){pack2(v[r][p][0] * inv * lo2f(nw[p].x), v[r][p][1] * inv * hi2f(nw[p].x)),
+                                                          pack2(v[r][p][2] * inv * lo2f(nw[p].y), v[r][p][3] * inv * hi2f(nw[p].y))});
+  }
+  __syncthreads();
+  f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  const int xr = min(li, nrow - 1);
+#pragma unroll
+  for (int b = 0; b < PQ; ++b) {
+    if (b * 8 >= KB) continue;                // a piece that is there in part: its last fragment again, against zeros
+#pragma unroll
+    for (int k = 0; k < 8; ++k) acc[k & 1] = mfma16(as_bf16x8(wf[b][k]), as_bf16x8(ld16(s_x + xr * PITCH + (b * 8 + k) * 32 + g * 8)), acc[k & 1]);
+  }
+  acc[0] += acc[1];
+  if (li < RG) st8(s_q + li * QP + wave * 16 + g * 4, (u32x2){pack2(acc[0][0], acc[0][1]), pack2(acc[0][2], acc[0][3])});
+  __syncthreads();
+  if (tile >= tiles) return;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) o = mfma16(as_bf16x8(uk[k]), as_bf16x8(ld16(s_q + xr * QP + k * 32 + g * 8)), o);
+  if (li < nrow) st8(out + ((size_t)(b0 + li) * a.heads + h) * rp + tile * 16 + g * 4, (u32x2){pack2(o[0], o[1]), pack2(o[2], o[3])});
+}
+// In place of three launches (32 rows, 12 heads, ranks 768 and 512: 4.0 + 4.2 + 4.1 us; up to 8 rows two of 5.9 + 4.3).  A step of 28 such layers, us, apart / here: 1 row 1188 / 1134,
+// 8 1458 / 1406, 16 1692 / 1589, 24 1538 / 1430, 32 1594 / 1464 (with 16 rows and 256 ranks a block 1529).  A wider query rank is more than a unit should pull for a head: 28 heads of
+// rank 1536 3,568 / 3,713 with 32 rows, 2,811 / 2,955 with one.  Few heads would append many rows one after another.
+bool latent_query_ok(int rows, int heads, int dim, int qp) { return rows >= 1 && rows <= 64 && heads >= 8 && dim == 128 && qp <= LATENT_Q_PIECES * 256; }
+int latent_query(const LatentInArgs& a, const bf16_t* uq, const bf16_t* ukt, int dim, int rp, bf16_t* out, hipStream_t st) {
+  if (!latent_query_ok(a.rows, a.heads, dim, a.qp)) return LCC_ERR_SHAPE;
+  if ((a.qp & 63) || a.qp <= 0 || (rp & 63) || rp < 64 || (a.rp != 0 && a.rp != rp) || a.nsplit < 1 || (a.ldn & 3) || a.ldn < a.qp + a.rp + a.heads) return LCC_ERR_SHAPE;
+  if (!a.part || !a.q_norm || !a.gate || a.q_rank < 1 || !uq || !ukt || !out) return LCC_ERR_ARG;
+  if (a.rp > 0 && (!a.kv_norm || !a.tok_stream || (!a.tok_pos && !a.kv_len) || !a.kv_base || a.kv_rank < 1)) return LCC_ERR_ARG;
+  g_launch_counts[LC_LATENT_QUERY]++;
+  const int parts = (rp + 127) / 128;
+  // eight rows a block halve the slabs a unit pulls, while all blocks run at once
+  const int g8 = (a.rows + 7) / 8, g16 = (a.rows + 15) / 16;
+  if ((long)(parts + 1) * a.heads * g8 <= 256) latent_query_kernel<8><<<dim3(parts + 1, a.heads, g8), dim3(512), 0, st>>>(a, uq, ukt, rp, parts, out);
+  else latent_query_kernel<16><<<dim3(parts + 1, a.heads, g16), dim3(512), 0, st>>>(a, uq, ukt, rp, parts, out);
+  return 0;
+}
+
+// ------------------------------------------------------------------------------------------------------------------------------
 // Decode, step 2: attention over the cached latents, all heads of a row together.  rank = 64 RT.
 // Block = quads of 4 waves, one quad per 16 heads; 64 keys per iteration, staged once for all quads by LDS-DMA, double buffered.  Per iteration a wave multiplies its 16 keys with its quad's 16 queries
 // (S^T[key][head]: a lane owns 4 keys of one head), the quad agrees on the new maxima through LDS, and then each wave adds

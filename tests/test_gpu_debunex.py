@@ -523,6 +523,34 @@ def test_one_launch_and_two_give_the_same_bits(dev, lib, width, ff, n):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("n,rank,kv", [(1, 768, 512), (7, 700, 130), (8, 64, 64), (9, 256, 512), (16, 300, 1000), (17, 513, 64), (24, 768, 300), (33, 48, 512), (64, 768, 512)])
+def test_norms_query_and_absorption_in_one_launch(dev, lib, n, rank, kv):
+    """Query ranks of one channel to all that the kernel holds, eight rows a block and 16 (more blocks than units), short last groups, cache ranks of half a block's
+    to eight blocks'; a layer with a cache of its own and one that reads it; one split of the input projection and several (from nine rows on).  Both forms within the bound
+    of the tests around this one, and the next step reads what this one appended."""
+    from livecc_amd import ops
+    from livecc_amd.config import DebunexConfig
+    cfg = DebunexConfig(300, 200, [U.L(U.M(9, 120, 64, rank, kv, 0.15), 320), U.L(U.M(8, 128, 40, rank, kv, 0.15, 0), 100)], 1e-5, 20.0, name="query")
+    T = U.make_weights(cfg, 5)
+    m = _model(cfg, T, dev, max_streams=n, max_kv_len=128, max_new_rows=1024)
+    seqs = [U.ids_of(cfg, 4 + i % 9, 30 + i) for i in range(n)]
+    for on in (1, 0):
+        old = lib.lcc_debug_set_decoder_fused(on)
+        try:
+            st = [m.new_stream() for _ in seqs]
+            m.forward_step([(s, x[:-2], []) for s, x in zip(st, seqs)])
+            before = ops.launch_counts()["latent_query"]
+            m.forward_step([(s, [x[-2]], [0]) for s, x in zip(st, seqs)])
+            got = m.forward_step([(s, [x[-1]], [0]) for s, x in zip(st, seqs)])
+            assert ops.launch_counts()["latent_query"] - before == (4 if on else 0)
+            for i in sorted({0, n // 2, n - 1}):
+                assert U.error(got[i], U.oracle_logits(cfg, T, seqs[i])[[-1]]) < U.LIMIT
+            for s in st:
+                s.release()
+        finally:
+            lib.lcc_debug_set_decoder_fused(old)
+
+
 def test_a_wide_input_projection_keeps_a_launch_of_its_own(dev):
     """64 rows, a query rank of 5120 beside a feed-forward of 8192 at width 2048: the projection's blocks of one tile would take longer than the launch saved."""
     from livecc_amd import ops
