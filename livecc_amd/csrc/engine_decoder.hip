@@ -90,7 +90,9 @@ namespace {
 // S packed rows through every layer; pt null: a decode step over the streams `d_slots`.  On exit b.h holds the final norm of the residual.
 int run_decoder_layers(lcc_engine* e, const DecBuffers& b, int S, const PrefillTables* pt, const int32_t* d_slots, int nsplit_attn, const AttnDirect& direct,
                        hipStream_t st) {
-  const bool fused = !pt && S <= 16 && g_fused_decode;
+  // From nine rows on at widths up to 2,048 the launches of 17 to 64 rows are the faster ones: their blocks pull the activations once for six weight tiles.  us a step, 28 layers,
+  // 9 / 12 / 16 rows, these launches / those: width 1536 1418 / 1305, 1494 / 1346, 1584 / 1391; width 3584 3168 / 3243, 3284 / 3328, 3542 / 3523
+  const bool fused = !pt && S <= (e->c.hidden_size <= 2048 ? 8 : 16) && g_fused_decode;
   const int W = e->c.hidden_size, NL = (int)e->dl.size();
   if (e->llm_over) return fail(LCC_ERR_STATE, "per-layer input overrides are not available for this model family");
   LCC_TRY(tap(e, b, 0, S, st));

@@ -2361,7 +2361,7 @@ __global__ __launch_bounds__(256) void gemv_skinny_kernel(
   __shared__ u32x4 xs_all[gemv_rows_lds(MG)];
   gemv_skinny_body<NTILE, MODE, PACKED, UNR, PIPE, MG>(X, ldx, W, ldw, bias, out, ldo, M, N, K, chunks_per_split, tail, blockIdx.x, blockIdx.y, gridDim.y, red, xs_all);
 }
-// Two products of the same 17..64 rows in ONE launch: a gate/up projection (SwiGLU, NTILE tiles a block) and, behind its blocks, another one into fp32 slabs (a tile
+// Two products of the same 9..64 rows in ONE launch: a gate/up projection (SwiGLU, NTILE tiles a block) and, behind its blocks, another one into fp32 slabs (a tile
 // a block).  Alone, neither fills the chip (32 rows of the 2B layer-list decoder: 187 blocks of gate/up, 13.6 us; 162 of the input projection, 4.6 us): the
 // small one runs on the units that the large one leaves, and a launch of the step is gone.  Same sums, same bits.
 struct GemvPart { const bf16_t *X, *W; void* out; int ldx, ldo, N, K, cps; };
@@ -2459,13 +2459,15 @@ static void launch_gemv_rows(const GemmArgs& a, int S, void* out, int ldo, int c
   }
 }
 
+// (9 to 16 rows run as 17 here: the kernel has two groups of rows at least)
+static int pair_tiles(const GemmArgs& sw) { GemmArgs a = sw; a.M = std::max(sw.M, 17); return gemv_rows_tiles(a, 1); }
 // Whether one launch is the faster one.  Beside a small body (two tiles a block) it was in all shapes measured.  A large one leaves a unit to one block at a time,
 // the input projection's blocks of one tile among them: what the units pull (gemv_rows_tiles), apart with the tiles each would take alone and together, and a
 // launch's worth of it, 160, between them.  us a layer of a decode step, apart / together, width, feed-forward, query rank, rows:  1536, 8960, 768: 17 rows 59.8 / 56.4,
 // 64 79.1 / 75.1;  3584, 18944, 1536: 17 124.6 / 122.4, 32 136.7 / 131.3, 64 168.9 / 162.8;  8192, 28672, 1536: 64 400 / 392;  3584, 8192, 3584: 48 128.3 / 128.3,
 // 64 142.1 / 146.9;  8192, 14336, 4096: 32 191.3 / 189.4, 64 234.5 / 237.4;  8192, 8192, 4096: 17 134.9 / 134.7, 32 140.7 / 141.8, 64 172.1 / 181.0
 static bool gemv_rows_pair_pays(const GemmArgs& in, const GemmArgs& sw) {
-  const int nt = gemv_rows_tiles(sw, 1), alone = gemv_rows_tiles(in, in.nsplit);
+  const int nt = pair_tiles(sw), alone = gemv_rows_tiles(in, in.nsplit);
   if (nt == 2) return true;
   const float groups = (float)sw.M / 16.f;
   const long blocks_sw = (sw.N / 16 + nt - 1) / nt, blocks_in = (long)(in.N / 16) * in.nsplit, blocks_alone = (long)((in.N / 16 + alone - 1) / alone) * in.nsplit;
@@ -2476,10 +2478,10 @@ static bool gemv_rows_pair_pays(const GemmArgs& in, const GemmArgs& sw) {
   const float together = std::max(sw_alone, ((float)blocks_sw * block_sw + (float)blocks_in * block_in) / 256.f + block_in);
   return together - apart < 160.f;
 }
-// in: fp32 slabs (partial, nsplit); sw: SwiGLU.  Takes what the two calls of gemm_bf16 would take on the weight-streaming path with 17 to 64 rows, where it pays
+// in: fp32 slabs (partial, nsplit); sw: SwiGLU.  Takes what the two calls of gemm_bf16 would take on the weight-streaming path with 9 to 64 rows, where it pays
 bool gemv_rows_pair_ok(const GemmArgs& in, const GemmArgs& sw) {
   auto one = [](const GemmArgs& a) {
-    return a.w_packed && !a.w_fp8 && a.M > 16 && a.M <= 64 && a.N > 0 && gemm_routes_skinny(a.M, a.K, false) && (a.N & 15) == 0 && (a.lda & 7) == 0 &&
+    return a.w_packed && !a.w_fp8 && a.M > 8 && a.M <= 64 && a.N > 0 && gemm_routes_skinny(a.M, a.K, false) && (a.N & 15) == 0 && (a.lda & 7) == 0 &&
            (((uintptr_t)a.A | (uintptr_t)a.W) & 15) == 0 && a.bias == nullptr && a.tail.kind == 0;
   };
   return one(in) && one(sw) && in.M == sw.M && in.partial != nullptr && in.nsplit >= 1 && in.nsplit <= 8 && in.nsplit <= (in.K + 63) / 64 && in.epilogue == EPI_NONE &&
@@ -2497,7 +2499,7 @@ static void launch_rows_pair(const GemmArgs& in, const GemmArgs& sw, hipStream_t
 int gemv_rows_pair(const GemmArgs& in, const GemmArgs& sw, hipStream_t st) {
   if (!gemv_rows_pair_ok(in, sw)) return LCC_ERR_ARG;
   g_launch_counts[LC_GEMV_ROWS_PAIR]++;
-  switch (gemv_rows_tiles(sw, 1)) {
+  switch (pair_tiles(sw)) {
     case 6: launch_rows_pair<6>(in, sw, st); break;
     case 4: launch_rows_pair<4>(in, sw, st); break;
     default: launch_rows_pair<2>(in, sw, st);

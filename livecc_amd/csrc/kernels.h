@@ -28,7 +28,7 @@ enum LaunchCounter {
   LC_ATTN_VIT32 = 13,          // attn_vit32_kernel (vision attention on 32x32x16 MFMAs)
   LC_GEMM_VH = 14,             // gemm_walk_vh_kernel (row tiles of 256 / 272 / 288 rows), gemm_vh_kernel (small class 128 / 144; round 5 -- the slot of the retired gemm_pp_kernel)
   LC_GEMM_VIT_QKV = 15,        // gemm_vit_kernel: EPI_VIT_QK / EPI_VIT_V epilogues (RoPE / V transpose fused into the q|k|v projection; one EPI_VIT_QKV launch per tower block when E % 128 == 0, else a q|k launch + a V launch)
-  LC_GEMV_ROWS_PAIR = 16,      // gemv_rows_pair_kernel (input projection and gate/up of 17 to 64 rows in one launch)
+  LC_GEMV_ROWS_PAIR = 16,      // gemv_rows_pair_kernel (input projection and gate/up of 9 to 64 rows in one launch)
   LC_LATENT_QUERY = 17,        // latent_query_kernel (query norm, up-projection and absorption in one launch)
   LC_COUNT = 18
 };
@@ -81,7 +81,7 @@ struct GemmArgs {
   VitQkvEpi vq;                                 // epilogue == GEMM_EPI_VIT_QK / GEMM_EPI_VIT_V only
 };
 int gemm_bf16(const GemmArgs& a, hipStream_t st);
-bool gemv_rows_pair_ok(const GemmArgs& in, const GemmArgs& sw);                      // two products of the same 17..64 rows in one launch:
+bool gemv_rows_pair_ok(const GemmArgs& in, const GemmArgs& sw);                      // two products of the same 9..64 rows in one launch:
 int gemv_rows_pair(const GemmArgs& in, const GemmArgs& sw, hipStream_t st);          //   fp32 slabs and SwiGLU
 bool gemm_vit_qkv_eligible(int M, int E, int K);   // shapes the EPI_VIT_QK / EPI_VIT_V epilogues serve (8-wave kernel: K % 64 == 0; M > 64, M % 4 == 0, E % 32 == 0)
 int gemv_num_splits(int N, int K);

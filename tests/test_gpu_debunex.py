@@ -497,9 +497,9 @@ def test_wide_feed_forward_beside_the_input_projection(dev, ff, n):
         assert U.error(got[i], U.oracle_logits(cfg, T, seqs[i])[[-1]]) < U.LIMIT
 
 
-@pytest.mark.parametrize("width,ff,n", [(200, 8300, 17), (200, 8300, 48), (200, 8300, 64), (704, 7900, 33), (1600, 8300, 40), (200, 2200, 64), (200, 100, 32)])
+@pytest.mark.parametrize("width,ff,n", [(200, 8300, 9), (200, 8300, 16), (200, 8300, 17), (200, 8300, 48), (200, 8300, 64), (704, 7900, 33), (1600, 8300, 40), (200, 2200, 64), (200, 100, 32)])
 def test_one_launch_and_two_give_the_same_bits(dev, lib, width, ff, n):
-    """Input projection and gate/up of 17 to 64 rows, in one launch (counted) and in two: two, four and six weight tiles a block, one split and several."""
+    """Input projection and gate/up of 9 to 64 rows, in one launch (counted) and in two: two, four and six weight tiles a block, one split and several."""
     from livecc_amd import ops
     from livecc_amd.config import DebunexConfig
     cfg = DebunexConfig(width, 100, [U.L(U.M(3, 40, 48, 72, 90, 0.2), ff), U.L(U.M(2, 64, 64, 800, 90, 0.2, 0), ff)], 1e-5, 20.0, name="pair")
