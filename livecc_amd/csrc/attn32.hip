@@ -125,11 +125,21 @@ LCC_DEVICE void attn32_key_loop(unsigned char* alds, const Kv32& kv, const u32x4
   const float bias_raw = BIAS ? slope / scale_log2e : 0.f;
   const int col = lane & 31;
 
-  // DMA: this wave's pieces of a pair.  Surplus slots copy the last piece again (same bytes, same place).
+  // DMA: this wave's pieces of a pair.  Surplus slots copy the last piece again (same bytes, same place).  What a piece needs in every pair -- its operand, tiles from the
+  // pair's, row bytes and place in a slot -- is kept in scalar registers: formed anew, a pair of the tower kernel had 110 scalar instructions beside 190 others
+  struct Piece { const char* base; unsigned stride, row, at; int dt, lo; };
+  Piece pc[PWP];
   unsigned off[PWP], prow[CLAMP ? PWP : 1];
 #pragma unroll
   for (int j = 0; j < PWP; ++j) {
-    const int u = min(j * NWAVE + wave, 2 * NPD - 1), p = u >= NPD ? u - NPD : u;
+    const int u = min(j * NWAVE + wave, 2 * NPD - 1), r = u >= NPD ? 1 : 0, p = u - r * NPD;
+    const bool is_k = p < Im::KPD;
+    pc[j].base = is_k ? reinterpret_cast<const char*>(kv.k) : reinterpret_cast<const char*>(kv.v);
+    pc[j].stride = (unsigned)(is_k ? kv.k_tile : kv.v_tile);
+    pc[j].row = is_k ? kv.k_row : 0u;
+    pc[j].at = (unsigned)(r * Im::SLOT + (is_k ? p * (D == 128 ? 1040 : 1024) : Im::KB + (p - Im::KPD) * 1024));
+    pc[j].dt = is_k ? r + 2 : r - 2;
+    pc[j].lo = is_k ? 0 : tb;
     if (p < Im::KPD) {
       const int row = (p * 64 + lane) / Im::CR, c = (p * 64 + lane) % Im::CR;
       off[j] = (CLAMP ? 0u : (unsigned)row * kv.k_row) + (unsigned)((c ^ Im::kx(row)) * 16);
@@ -140,16 +150,13 @@ LCC_DEVICE void attn32_key_loop(unsigned char* alds, const Kv32& kv, const u32x4
       if (CLAMP) prow[j] = 0u;
     }
   }
-  auto piece = [&](int p, int tile, bool is_k, unsigned o_lane, unsigned row, unsigned slot) {      // p: of the slot; tile: in range
-    if (CLAMP) o_lane += __umul24(min(row, (unsigned)(kv.nkeys - 1 - tile * 32)), is_k ? kv.k_row : 0u);      // no branch: this is inside the pair's basic block
-    const char* base = is_k ? reinterpret_cast<const char*>(kv.k) + (size_t)tile * kv.k_tile : reinterpret_cast<const char*>(kv.v) + (size_t)tile * kv.v_tile;
-    glds16_base(base, o_lane, slot + (unsigned)(is_k ? p * (D == 128 ? 1040 : 1024) : Im::KB + (p - Im::KPD) * 1024));
+  auto piece = [&](const char* base, unsigned stride, int tile, unsigned row_bytes, unsigned o_lane, unsigned row, unsigned at) {      // tile: in range
+    if (CLAMP) o_lane += __umul24(min(row, (unsigned)(kv.nkeys - 1 - tile * 32)), row_bytes);      // no branch: this is inside the pair's basic block
+    glds16_base(base + (unsigned long long)stride * (unsigned)tile, o_lane, at);
   };
   auto issue = [&](int j, int t, int ps) {              // piece j of the pair (t, t + 1) into pair-stage ps
-    const int u = min(j * NWAVE + wave, 2 * NPD - 1), r = u >= NPD ? 1 : 0, p = u - r * NPD;
-    const bool is_k = p < Im::KPD;
-    const int tile = min(is_k ? t + r + 2 : max(t + r - 2, tb), kv.ntile - 1);
-    piece(p, tile, is_k, off[j], CLAMP ? prow[CLAMP ? j : 0] : 0u, lds0 + (unsigned)((2 * ps + r) * Im::SLOT));
+    const int tile = min(max(t + pc[j].dt, pc[j].lo), kv.ntile - 1);
+    piece(pc[j].base, pc[j].stride, tile, pc[j].row, off[j], CLAMP ? prow[CLAMP ? j : 0] : 0u, lds0 + (unsigned)(2 * ps * Im::SLOT) + pc[j].at);
   };
   // fragment addresses inside a slot: K row swap23(col), chunk 2 ks + hh; V^T row 32 dt + col, chunk 2 s + hh
   constexpr int NKA = D == 80 ? 1 : 4;
@@ -270,7 +277,8 @@ LCC_DEVICE void attn32_key_loop(unsigned char* alds, const Kv32& kv, const u32x4
 #pragma unroll
     for (int j = 0; j < PK; ++j) {
       const int p = min(j * NWAVE + wave, Im::KPD - 1), row = (p * 64 + lane) / Im::CR, c = (p * 64 + lane) % Im::CR;
-      piece(p, min(tb + r, kv.ntile - 1), true, (CLAMP ? 0u : (unsigned)row * kv.k_row) + (unsigned)((c ^ Im::kx(row)) * 16), row, lds0 + (unsigned)(4 + r) * Im::SLOT);
+      piece(reinterpret_cast<const char*>(kv.k), (unsigned)kv.k_tile, min(tb + r, kv.ntile - 1), kv.k_row,
+            (CLAMP ? 0u : (unsigned)row * kv.k_row) + (unsigned)((c ^ Im::kx(row)) * 16), row, lds0 + (unsigned)(4 + r) * Im::SLOT + (unsigned)p * (D == 128 ? 1040 : 1024));
     }
 #pragma unroll
   for (int k = 0; k < 2; ++k)
