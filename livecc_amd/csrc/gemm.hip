@@ -5,7 +5,7 @@
 //
 //  * gemm_walk_kernel    : M >= 17, packed W, K % 64 == 0 (LLM prefill, ViT).  MFMA-bound.  8 waves, BM x 256 x 64 tile
 //                          (BM 256 / 192 / 160 / 128), LDS-DMA for both operands; one block a compute unit, the DMA ring runs on from tile to tile.
-//  * gemm_vit_kernel     : the same pipeline, a tile a block, with the vision q|k|v epilogues.
+//  * gemm_vit_kernel     : the same pipeline, a tile a block, with the vision q|k|v epilogues (few patches: gemm_strip_kernel, gemm_mid_kernel).
 //  * gemm_big_kernel     : the same tiles one a block, both waves of a SIMD in step: 128-row tiles of one round.
 //  * gemm_walk_vh_kernel : the walk over row tiles of 256 / 272 / 288 rows (no ragged last row tile).
 //  * gemm_vh_kernel      : row tiles of 128 / 144 rows, split-K slabs of one streaming chunk.
@@ -268,7 +268,7 @@ LCC_DEVICE void tile_slab_wide(const f32x4 (&acc)[MT][NT], int mbase, int nbase,
 // EPI_VIT_QK / EPI_VIT_V (round 4): the vision tower's q|k|v projection writes what its attention kernels read -- q and k rotated (2-D
 // RoPE, HF modeling_qwen2_vl.py:225-248) at their natural columns of C, V blocked-transposed into vt[head][32-key block][80][32] -- instead
 // of a plain [P, 3E] tensor that vit_rope_vt_kernel re-reads and re-writes (52 us per tower block at 8 streams, 179 MB of traffic).
-// One launch of gemm_vit_kernel (two, q|k and V apart, where a column tile would hold both) over the `qkv_w_rope` copy of the weight (weights.py: vit_qkv_rope_row_permutation):
+// One launch of gemm_vit_kernel, or of the 128-column kernels (two of the first, q|k and V apart, where a column tile would hold both) over the `qkv_w_rope` copy of the weight (weights.py: vit_qkv_rope_row_permutation):
 //
 //  * q|k (N = 2E, EPI_VIT_QK): inside q and inside k every 32 stored rows are [16 first-half channels | their 16 rotation partners],
 //    first-half channels enumerated head-major (f = head * 40 + c, c < 40), so a lane's accumulators acc[i][j] / acc[i][j + 1] hold
@@ -597,34 +597,40 @@ __global__ __launch_bounds__(256) void gemm_glds_kernel(
 // K 22528 285 -> 196; 2000 x 1280, K 5120 55 -> 41.
 // Requires packed W, K % 64 == 0.  W8: fp8 weights in their packed order, 1 KB a fragment's 64 k, converted in registers in front of the
 // MFMAs (the form before wrote the whole weight as bf16 first): 600 x 4608, K 3584 50 -> 34.
+// The last part of a vision q|k|v tile of 32 columns a wave, NW waves: every wave is done with the stages (dsmem), and its DMA pieces have landed
+template <int EPI, int BM, int NW, int MT, int NT>
+LCC_DEVICE void vit_tile_end(const f32x4 (&acc)[MT][NT], u32x4* dsmem, int m0, int row0, int nbase, int lane, int wave, const bf16_t* bias, bf16_t* C, int ldc, int M, int N,
+                             const VitQkvEpi& vq) {
+  const int li = lane & 15, g = lane >> 4;
+  if constexpr (EPI == EPI_VIT_V) {
+    vit_v_epilogue<MT, NT>(acc, m0 + row0, nbase, li, g, bias, M, N, vq);
+  } else {
+    // cos / sin rows of this tile (gemm_walk_body): clamped reads past the last row belong to rows that are never stored
+    constexpr int UNITS = BM * 10;
+    const long first = (long)m0 * 10, last = (long)M * 10 - 1;
+    for (int t = wave; t * 64 < UNITS; t += NW) {
+      const long u = min(first + t * 64 + lane, last);
+      glds16(vq.cs + u * 4, lds_addr(dsmem + t * 64));
+      glds16(vq.sn + u * 4, lds_addr(dsmem + UNITS + t * 64));
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    const float* lcs = reinterpret_cast<const float*>(dsmem);
+    vit_qk_epilogue<MT, NT>(acc, m0 + row0, nbase, row0, li, g, bias, C, ldc, M, N, vq.E, lcs, lcs + UNITS * 4);
+  }
+}
+
 template <int BM, int EPI, int NST, bool W8>
-__global__ __launch_bounds__(512) void gemm_mid_kernel(
+LCC_DEVICE void gemm_mid_tile(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual,
-    int ldr, bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n, float* __restrict__ partial, int kt_per_split,
-    const float* __restrict__ wscale, int raster) {
+    int ldr, bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tm, int tn, float* __restrict__ partial, int kt_per_split,
+    const float* __restrict__ wscale, const VitQkvEpi& vq) {
   constexpr int BN = 128, BK = 64, MT = BM / 32, NT = 2;
   constexpr int WF = W8 ? 1 : 2;                                  // 1-KB weight sub-tiles of a fragment row
   constexpr int A_UNITS = BM * 8, STAGE = A_UNITS + 8 * WF * 64;  // 16-byte units: [BM rows][8 chunks] (XOR-swizzled) + 16 weight sub-tiles = 24 / 32 KB
   constexpr int APW = BM / 64, P = APW + WF;                      // DMA pieces of a wave per k-tile: 8 activation rows each, then the weights
   extern __shared__ __attribute__((aligned(16))) u32x4 dsmem[];
 
-  const int nblk = tiles_m * tiles_n;
-  for (int vb = blockIdx.x; vb < nblk; vb += gridDim.x) {     // one tile per block, or a persistent walk under the grid cap
-  int bid = vb;
-  {
-    const int q = nblk >> 3, r = nblk & 7, xcd = bid & 7, idx = bid >> 3;
-    bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
-  }
-  int tn, tm;                                     // tile order: see gemm_big_kernel
-  if (raster > 0) {
-    const int band = bid / (raster * tiles_m), rem = bid - band * raster * tiles_m;
-    const int bw = min(raster, tiles_n - band * raster);
-    tm = rem / bw;
-    tn = band * raster + (rem - tm * bw);
-  } else {
-    tn = bid / tiles_m;
-    tm = bid - tn * tiles_m;
-  }
   const int m0 = tm * BM, n0 = tn * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 2, wn = wave & 3;
@@ -679,7 +685,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(
 #pragma unroll
       for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) acc[i][j] = mfma16(b[j], f.a[kk][i], acc[i][j]);
+        for (int j = 0; j < NT; ++j) acc[i][j] = EPI == EPI_VIT_V ? mfma16(f.a[kk][i], b[j], acc[i][j]) : mfma16(b[j], f.a[kk][i], acc[i][j]);
     }
   };
   // tile kt + 1 has landed (this wave's pieces; NST - 3 newer tiles may stay in flight) -> barrier -> DMA of tile kt + NST - 1 into the stage
@@ -709,11 +715,43 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(
   }
   if (kt < nkt) mul(f0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the clamped copies
-  if (wide_rows<EPI>(C, ldc, bias, residual, ldr)) {
+  if constexpr (EPI == EPI_VIT_QK || EPI == EPI_VIT_V) {
+    __builtin_amdgcn_s_barrier();
+    vit_tile_end<EPI, BM, 8, MT, NT>(acc, dsmem, m0, wm * (BM / 2), n0 + wn * 32, lane, wave, bias, C, ldc, M, N, vq);
+  } else if (wide_rows<EPI>(C, ldc, bias, residual, ldr)) {
     __builtin_amdgcn_s_barrier();          // every wave is done with the stages, and its DMA pieces have landed
     tile_epilogue_wide<EPI, MT, NT>(acc, m0 + wm * (BM / 2), n0 + wn * 32, lane, bias, residual, ldr, C, ldc, M, N, wscale,
                                     reinterpret_cast<unsigned char*>(dsmem) + wave * 4096);
   } else tile_epilogue<EPI, MT, NT>(acc, m0 + wm * (BM / 2), n0 + wn * 32, (n0 + wn * 32) / 2, li, g, bias, residual, ldr, C, ldc, M, N, partial, wscale);
+}
+template <int BM, int EPI, int NST, bool W8>
+__global__ __launch_bounds__(512) void gemm_mid_kernel(
+    const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual,
+    int ldr, bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n, float* __restrict__ partial, int kt_per_split,
+    const float* __restrict__ wscale, int raster, VitQkvEpi vq) {
+  const int nblk = tiles_m * tiles_n;
+  for (int vb = blockIdx.x; vb < nblk; vb += gridDim.x) {     // one tile per block, or a persistent walk under the grid cap
+  int bid = vb;
+  {
+    const int q = nblk >> 3, r = nblk & 7, xcd = bid & 7, idx = bid >> 3;
+    bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
+  }
+  int tn, tm;                                     // tile order: see gemm_big_kernel
+  if (raster > 0) {
+    const int band = bid / (raster * tiles_m), rem = bid - band * raster * tiles_m;
+    const int bw = min(raster, tiles_n - band * raster);
+    tm = rem / bw;
+    tn = band * raster + (rem - tm * bw);
+  } else {
+    tn = bid / tiles_m;
+    tm = bid - tn * tiles_m;
+  }
+  if constexpr (EPI == EPI_VIT_QKV) {
+    const int qk_tiles = 2 * vq.E / 128;          // V: rows 2E.. of the packed weight
+    if (tn >= qk_tiles)
+      gemm_mid_tile<BM, EPI_VIT_V, NST, W8>(A, lda, W + (size_t)2 * vq.E * K, bias != nullptr ? bias + 2 * vq.E : nullptr, nullptr, 0, nullptr, 0, M, vq.E, K, tm, tn - qk_tiles, nullptr, 0, nullptr, vq);
+    else gemm_mid_tile<BM, EPI_VIT_QK, NST, W8>(A, lda, W, bias, nullptr, 0, C, ldc, M, 2 * vq.E, K, tm, tn, nullptr, 0, nullptr, vq);
+  } else gemm_mid_tile<BM, EPI, NST, W8>(A, lda, W, bias, residual, ldr, C, ldc, M, N, K, tm, tn, partial, kt_per_split, wscale, vq);
   if (vb + (int)gridDim.x < nblk) __syncthreads();     // the next tile's DMA reuses the stages
   }
 }
@@ -752,10 +790,10 @@ LCC_DEVICE void strip_fetch(const bf16_t* W, int row, int nfrag, int c0, int c1,
 template <int... U, class F>
 LCC_DEVICE void strip_steps(std::integer_sequence<int, U...>, F f) { (f(std::integral_constant<int, U>{}), ...); }
 template <int EPI, bool W8>
-__global__ __launch_bounds__(256, 2) void gemm_strip_kernel(
+LCC_DEVICE void gemm_strip_tile(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual,
-    int ldr, bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n, float* __restrict__ partial, int kt_per_split,
-    const float* __restrict__ wscale, int raster, int fetch) {
+    int ldr, bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tm, int tn, float* __restrict__ partial, int kt_per_split,
+    const float* __restrict__ wscale, const VitQkvEpi& vq) {
   constexpr int BM = 64, BK = 64, MT = BM / 16, NT = 2, D = STRIP_STAGES;
   constexpr int WF = W8 ? 1 : 2;                                  // 1-KB weight sub-tiles of a fragment row
   constexpr int STAGE = BM * 8;                                   // 16-byte units: [BM rows][8 chunks] (XOR-swizzled) = 8 KB
@@ -766,27 +804,6 @@ __global__ __launch_bounds__(256, 2) void gemm_strip_kernel(
   const int nkt_all = K / BK;
   const int kt0 = (EPI == EPI_PARTIAL) ? blockIdx.y * kt_per_split : 0;
   const int nkt = (EPI == EPI_PARTIAL) ? min(nkt_all, kt0 + kt_per_split) : nkt_all;
-  const int nblk = tiles_m * tiles_n;
-  if ((int)blockIdx.x >= nblk) {                  // the last `fetch` k-tiles of this split
-    strip_fetch(W, nkt_all * WF * 64, (N + 15) >> 4, max(kt0, nkt - fetch) * WF / 2, nkt * WF / 2, (int)blockIdx.x - nblk, (int)gridDim.x - nblk);
-    return;
-  }
-  for (int vb = blockIdx.x; vb < nblk; vb += gridDim.x) {     // one tile per block, or a persistent walk under the grid cap
-  int bid = vb;
-  {
-    const int q = nblk >> 3, r = nblk & 7, xcd = bid & 7, idx = bid >> 3;
-    bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
-  }
-  int tn, tm;                                     // tile order: see gemm_big_kernel
-  if (raster > 0) {
-    const int band = bid / (raster * tiles_m), rem = bid - band * raster * tiles_m;
-    const int bw = min(raster, tiles_n - band * raster);
-    tm = rem / bw;
-    tn = band * raster + (rem - tm * bw);
-  } else {
-    tn = bid / tiles_m;
-    tm = bid - tn * tiles_m;
-  }
   const int m0 = tm * BM, n0 = tn * 128;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, g = lane >> 4;
@@ -842,7 +859,7 @@ __global__ __launch_bounds__(256, 2) void gemm_strip_kernel(
         for (int j = 0; j < NT; ++j) b[kk][j] = W8 ? fp8x8_to_bf16x8(w[u][0][j][2 * kk], w[u][0][j][2 * kk + 1]) : as_bf16x8(w[u][kk % WF][j]);
       }
 #pragma unroll
-      for (int j = 0; j < NT; ++j) acc[i][j] = mfma16(b[kk][j], f[u & 1][kk][i], acc[i][j]);
+      for (int j = 0; j < NT; ++j) acc[i][j] = EPI == EPI_VIT_V ? mfma16(f[u & 1][kk][i], b[kk][j], acc[i][j]) : mfma16(b[kk][j], f[u & 1][kk][i], acc[i][j]);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -864,11 +881,51 @@ __global__ __launch_bounds__(256, 2) void gemm_strip_kernel(
     if (decltype(uc)::value < rem) step(kt + decltype(uc)::value, uc, std::integral_constant<int, decltype(uc)::value + 1>{});
   });
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the clamped copies
-  if (wide_rows<EPI>(C, ldc, bias, residual, ldr)) {
+  if constexpr (EPI == EPI_VIT_QK || EPI == EPI_VIT_V) {
+    __builtin_amdgcn_s_barrier();
+    vit_tile_end<EPI, BM, 4, MT, NT>(acc, dsmem, m0, 0, n0 + wave * 32, lane, wave, bias, C, ldc, M, N, vq);
+  } else if (wide_rows<EPI>(C, ldc, bias, residual, ldr)) {
     __builtin_amdgcn_s_barrier();          // every wave is done with the stages, and its DMA pieces have landed
     tile_epilogue_wide<EPI, MT, NT>(acc, m0, n0 + wave * 32, lane, bias, residual, ldr, C, ldc, M, N, wscale,
                                     reinterpret_cast<unsigned char*>(dsmem) + wave * 4096);
   } else tile_epilogue<EPI, MT, NT>(acc, m0, n0 + wave * 32, (n0 + wave * 32) / 2, li, g, bias, residual, ldr, C, ldc, M, N, partial, wscale);
+}
+template <int EPI, bool W8>
+__global__ __launch_bounds__(256, 2) void gemm_strip_kernel(
+    const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual,
+    int ldr, bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n, float* __restrict__ partial, int kt_per_split,
+    const float* __restrict__ wscale, int raster, int fetch, VitQkvEpi vq) {
+  constexpr int WF = W8 ? 1 : 2;
+  const int nkt_all = K / 64;
+  const int kt0 = (EPI == EPI_PARTIAL) ? blockIdx.y * kt_per_split : 0;
+  const int nkt = (EPI == EPI_PARTIAL) ? min(nkt_all, kt0 + kt_per_split) : nkt_all;
+  const int nblk = tiles_m * tiles_n;
+  if ((int)blockIdx.x >= nblk) {                  // the last `fetch` k-tiles of this split
+    strip_fetch(W, nkt_all * WF * 64, (N + 15) >> 4, max(kt0, nkt - fetch) * WF / 2, nkt * WF / 2, (int)blockIdx.x - nblk, (int)gridDim.x - nblk);
+    return;
+  }
+  for (int vb = blockIdx.x; vb < nblk; vb += gridDim.x) {     // one tile per block, or a persistent walk under the grid cap
+  int bid = vb;
+  {
+    const int q = nblk >> 3, r = nblk & 7, xcd = bid & 7, idx = bid >> 3;
+    bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
+  }
+  int tn, tm;                                     // tile order: see gemm_big_kernel
+  if (raster > 0) {
+    const int band = bid / (raster * tiles_m), rem = bid - band * raster * tiles_m;
+    const int bw = min(raster, tiles_n - band * raster);
+    tm = rem / bw;
+    tn = band * raster + (rem - tm * bw);
+  } else {
+    tn = bid / tiles_m;
+    tm = bid - tn * tiles_m;
+  }
+  if constexpr (EPI == EPI_VIT_QKV) {
+    const int qk_tiles = 2 * vq.E / 128;          // V: rows 2E.. of the packed weight
+    if (tn >= qk_tiles)
+      gemm_strip_tile<EPI_VIT_V, W8>(A, lda, W + (size_t)2 * vq.E * K, bias != nullptr ? bias + 2 * vq.E : nullptr, nullptr, 0, nullptr, 0, M, vq.E, K, tm, tn - qk_tiles, nullptr, 0, nullptr, vq);
+    else gemm_strip_tile<EPI_VIT_QK, W8>(A, lda, W, bias, nullptr, 0, C, ldc, M, 2 * vq.E, K, tm, tn, nullptr, 0, nullptr, vq);
+  } else gemm_strip_tile<EPI, W8>(A, lda, W, bias, residual, ldr, C, ldc, M, N, K, tm, tn, partial, kt_per_split, wscale, vq);
   if (vb + (int)gridDim.x < nblk) __syncthreads();     // the next tile's DMA reuses the stages
   }
 }
@@ -1748,7 +1805,7 @@ static void launch_mid_w(const GemmArgs& a, hipStream_t st) {
   static DeviceOnce attr_set;   // per instantiation
   if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_mid_kernel<BM, EPI, NST, W8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   gemm_mid_kernel<BM, EPI, NST, W8><<<dim3(capped_grid((long)tiles_m * tiles_n), S), dim3(512), lds, st>>>(
-      a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.partial, (nkt + S - 1) / S, a.wscale, raster_for(tiles_m));
+      a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.partial, (nkt + S - 1) / S, a.wscale, raster_for(tiles_m), a.vq);
 }
 template <int BM, int EPI, int NST>
 static void launch_mid(const GemmArgs& a, hipStream_t st) { a.w_fp8 ? launch_mid_w<BM, EPI, NST, true>(a, st) : launch_mid_w<BM, EPI, NST, false>(a, st); }
@@ -1771,7 +1828,7 @@ static void launch_strip_w(const GemmArgs& a, hipStream_t st) {
   static DeviceOnce attr_set;   // per instantiation
   if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_strip_kernel<EPI, W8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   gemm_strip_kernel<EPI, W8><<<dim3(capped_grid(tiles) + extra, S), dim3(256), lds, st>>>(
-      a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.partial, nkt, a.wscale, raster_for(tiles_m), fetch);
+      a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.partial, nkt, a.wscale, raster_for(tiles_m), fetch, a.vq);
 }
 template <int EPI>
 static void launch_mid64(const GemmArgs& a, hipStream_t st) { a.w_fp8 ? launch_strip_w<EPI, true>(a, st) : launch_strip_w<EPI, false>(a, st); }
@@ -2753,8 +2810,12 @@ int gemm_bf16(const GemmArgs& a, hipStream_t st) {
     g_launch_counts[LC_GEMM_VIT_QKV]++;
     int big = big_tile_rows(a, 1);
     if (big == 160) big = 192;
-    if (big == 272) big = 256;      // the rotation / transposed-V epilogues live on the fixed-height 256-column tiles (129: the 128-row one)
-    if (a.epilogue == EPI_VIT_QKV) launch_vit<EPI_VIT_QKV>(a, big, st);
+    if (big == 272) big = 256;      // the rotation / transposed-V epilogues live on the fixed-height 256-column tiles (129, 0: the 128-row one, or for q, k and V together the 128-column tiles)
+    // The narrow tiles where a product without these epilogues takes them (up to 1,024 patches at 1,280 channels).  A tower of 32 blocks, us, 128 x 256 tiles / here: 140 patches
+    // 2681 / 2370, 320 2896 / 2522, 560 3204 / 3004, 720 3387 / 3165, 880 3739 / 3501
+    if (all && big == 129) launch_mid_w<128, EPI_VIT_QKV, 4, false>(a, st);
+    else if (all && big == 0) launch_strip_w<EPI_VIT_QKV, false>(a, st);
+    else if (all) launch_vit<EPI_VIT_QKV>(a, big, st);
     else if (qk) launch_vit<EPI_VIT_QK>(a, big, st);
     else launch_vit<EPI_VIT_V>(a, big, st);
     return 0;

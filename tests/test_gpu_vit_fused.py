@@ -55,6 +55,32 @@ def test_fused_qkv_epilogue_is_bit_identical_to_the_separate_launches_small(dev,
     assert torch.equal(plain, fused)
 
 
+@pytest.mark.parametrize("shapes,tile", [([(2, 28, 476)], 64), ([(2, 140, 196)], 64), ([(2, 392, 252), (2, 28, 56)], 64), ([(2, 196, 532)], 129), ([(4, 280, 504), (2, 56, 56)], None),
+                                         ([(2, 280, 504)], 129), ([(2, 392, 504)], 129), ([(2, 392, 532)], 64), ([(2, 392, 728)], 128)])
+def test_fused_qkv_epilogue_of_the_128_column_tiles(dev, shapes, tile):
+    """E = 1280, few patches: the tower's epilogues on the 64 x 128 and 128 x 128 tiles, one row of a tile and all of it, with blocks that fetch the weight
+    ahead and without, several clips; under a cap on the workgroups, too.  The bits of the separate launches."""
+    import dataclasses
+    from livecc_amd import ops
+    from livecc_amd.config import small
+    cfg = dataclasses.replace(small(), vit_depth=2, vit_embed_dim=1280, vit_num_heads=16)
+    patches = sum(((T + 1) // 2) * (H // 14) * (W // 14) for T, H, W in shapes)
+    if tile is not None:
+        assert ops.gemm_plan(patches, 3 * 1280, 1280, ops.EPI_NONE)[0] == tile
+    native = _model(cfg, dev, max_patches=4096)
+    clips = _clips(shapes, dev, seed=17)
+    plain, fused, c0, c1 = _both(native, clips)
+    assert c0["gemm_vit_qkv"] == 0 and c1["gemm_vit_qkv"] == cfg.vit_depth
+    assert torch.isfinite(fused.float()).all() and torch.equal(plain, fused)
+    native.engine.set_vit_grid_cap(40)
+    try:
+        capped = native.engine.vit_encode(clips).clone()
+    finally:
+        native.engine.set_vit_grid_cap(0)
+    torch.cuda.synchronize()
+    assert torch.equal(capped, fused)
+
+
 @pytest.mark.parametrize("streams", [1, 8])
 def test_fused_qkv_epilogue_is_bit_identical_at_7b_shapes(dev, streams):
     """LiveCC-7B tower (E = 1280, 16 heads, 32 blocks) on the streaming chunk shape: 1 and 8 co-scheduled 2-frame 392x728 chunks
