@@ -2479,17 +2479,19 @@ static void launch_gemv_l(dim3 grid, const GemmArgs& a, void* out, int ldo, int 
   else launch_gemv<NTILE, MODE, false>(grid, a, out, ldo, cps, st);
 }
 
-// 17..64 rows: a block of one 16-row weight tile reads more activations than weights (32 rows: twice as many bytes, and a compute unit pulls about 40
+// 10..64 rows: a block of one 16-row weight tile reads more activations than weights (32 rows: twice as many bytes, and a compute unit pulls about 40
 // GB/s of either), so packed weights go up to six tiles to a block.  What a unit then pulls: rounds of blocks x (tiles + 16-row groups of
 // activations); more tiles only where that is clearly less, since their registers leave one or two waves a SIMD.  32 rows, [151936, 1536]: 116.5 us with
 // one tile, 80.8 with four (5.8 TB/s); [152064, 3584] 261 -> 182; 64 rows: 358 -> 239.  Three tiles against one, two, four at 32 rows (a row of launches
 // on weights from memory): [1536, 10496] in eight splits 9.7 / 11.7, 11.7, 10.3; [1536, 8960] in eight 9.0 / 12.0, 10.5, 9.6.  Six: [3584, 18944] in five
 // 30.3 against 35.6 with two and 37.4 with four, [4608, 3584] in four 10.7 / 12.4 with one, gate/up with SwiGLU [17920, 1536] 14.1 / 16.2 with two,
 // 64 rows of [37888, 3584] 68.6 / 76.0.  Where one tile's blocks fill a round at most it stays: [2048, 1536] in two splits 4.7 / 5.1.
+// 10 to 16 rows run as 17 do, two groups of rows (one, in fragment-shaped loads: 2 to 6 % slower a step).  us a step of 28 layers, one or two tiles / as many as here, 9 / 10 / 12 / 16 rows: 2B with
+// recurrence 1862 / 1900, 1904 / 1893, 1980 / 1958, 2077 / 2009; 7B with recurrence 4182 / 4148, 4277 / 4207, 4467 / 4297, 4882 / 4510; 2B (q, k, v) 1410 / 1420, -, 1452 / 1403, 1497 / 1426
 static int gemv_rows_tiles(const GemmArgs& a, int S) {
   const bool pairs = a.epilogue == EPI_SWIGLU;
   const int least = pairs ? 2 : 1;
-  if (!a.w_packed || a.M <= 16) return least;
+  if (!a.w_packed || a.M <= 9 || (a.M <= 16 && (a.K & 63) != 0)) return least;
   const int tiles = (a.N + 15) / 16;
   auto cost = [&](int nt) { return (float)(((long)((tiles + nt - 1) / nt) * S + 255) / 256) * ((float)nt + (float)a.M / 16.f); };
   int nt = least;

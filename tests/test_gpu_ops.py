@@ -263,6 +263,21 @@ def test_gemm_128_column_tiles_are_bit_identical_to_the_256_row_tiles(dev, M, N,
     assert torch.equal(got, ref), f"{int((got != ref).sum())} of {got.numel()} outputs differ from the 256-row tiles"
 
 
+@pytest.mark.parametrize("N,K,epi,S", [(17920, 1536, 4, 0), (17952, 576, 4, 0), (4624, 3584, 0, 4), (1536, 8960, 0, 8), (1552, 640, 0, 5), (40016, 512, 0, 0), (4608, 544, 0, 2)])
+@pytest.mark.parametrize("M", [10, 13, 16])
+def test_rows_up_to_16_in_one_tile_a_block_and_in_several_give_the_same_bits(dev, N, K, epi, S, M):
+    """From ten rows on a block of the weight-streaming kernel takes up to six weight tiles (a last block with fewer among them; a K of half a chunk keeps one): the rows' bits are
+    those that nine of them have."""
+    from livecc_amd import ops
+    x, w, b = _rand((M, K), dev, 1.0, 1), _rand((N, K), dev, 0.05, 2), _rand((N,), dev, 0.1, 3)
+    wp = ops.pack_weight(w)
+    product = lambda r: ops.linear_partial(r, wp, S, packed_shape=(N, K)) if S else ops.linear(r, wp, None if epi == 4 else b, epi, packed_shape=(N, K))[None]
+    got = product(x)
+    assert torch.isfinite(got.float()).all()
+    for r0 in (0, M - 9):
+        assert torch.equal(got[:, r0:r0 + 9], product(x[r0:r0 + 9].contiguous()))
+
+
 @pytest.mark.parametrize("M,N", [(65, 144), (100, 272), (1456, 1280), (1500, 1280), (1600, 1280)])
 @pytest.mark.parametrize("nkt", [1, 2, 5, 6, 7, 11, 12, 13, 16, 20])
 @pytest.mark.parametrize("fp8", [False, True], ids=["bf16", "fp8"])
