@@ -4,7 +4,7 @@
 // engine's (engine.hip, engine_llm.hip); this file is the launch sequence of the layers and what they need in memory.
 //
 // A layer is
-// (decode steps of up to 16 rows fuse "in" with "ff", the norms with "query", and "out" with the residual and the next norm: decode_v2.hip; where a head's part of the
+// (decode steps of up to eight or nine rows fuse "in" with "ff", the norms with "query", and "out" with the residual and the next norm: decode_v2.hip; where a head's part of the
 // query projection is small, the norms, "query" and the absorption are one launch at any number of rows: latent_query)
 //   in      [Wdq | Wdkv | Wg] h           one GEMM, fp32 slabs
 //           norms -> query latent, c -> cache, gates          (latent_norm_append)
@@ -84,15 +84,15 @@ int carve_bound(lcc_engine* e, DecBuffers* b) {
 }
 
 }  // namespace
-int g_fused_decode = 1;      // lcc_debug_set_decoder_fused: decode steps run the fused launches (up to 16 rows five or six per layer instead of nine, of 17 to 64 six to eight)
+int g_fused_decode = 1;      // lcc_debug_set_decoder_fused: decode steps run the fused launches (up to eight or nine rows five or six per layer instead of nine, of up to 64 six to eight)
 
 namespace {
 // S packed rows through every layer; pt null: a decode step over the streams `d_slots`.  On exit b.h holds the final norm of the residual.
 int run_decoder_layers(lcc_engine* e, const DecBuffers& b, int S, const PrefillTables* pt, const int32_t* d_slots, int nsplit_attn, const AttnDirect& direct,
                        hipStream_t st) {
-  // From nine rows on at widths up to 2,048 the launches of 17 to 64 rows are the faster ones: their blocks pull the activations once for six weight tiles.  us a step, 28 layers,
-  // 9 / 12 / 16 rows, these launches / those: width 1536 1418 / 1305, 1494 / 1346, 1584 / 1391; width 3584 3168 / 3243, 3284 / 3328, 3542 / 3523
-  const bool fused = !pt && S <= (e->c.hidden_size <= 2048 ? 8 : 16) && g_fused_decode;
+  // From nine rows on (ten above a width of 2,048) the launches of 17 to 64 rows are the faster ones: their blocks pull the activations once for up to six weight tiles.  us a step, 28
+  // layers, 9 / 10 / 12 / 16 rows, these launches / those: width 1536 1418 / 1296, -, 1494 / 1326, 1584 / 1355; width 3584 3191 / 3250, 3250 / 3216, 3289 / 3186, 3510 / 3270
+  const bool fused = !pt && S <= (e->c.hidden_size <= 2048 ? 8 : 9) && g_fused_decode;
   const int W = e->c.hidden_size, NL = (int)e->dl.size();
   if (e->llm_over) return fail(LCC_ERR_STATE, "per-layer input overrides are not available for this model family");
   LCC_TRY(tap(e, b, 0, S, st));
