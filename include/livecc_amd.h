@@ -243,7 +243,8 @@ int lcc_debug_bench_grid_barrier(int mode, int blocks, int iters, void* scratch,
  * (attn32.hip), 7 LDS-shared prefill attention, 8 per-wave prefill attention, 9 prefill split-merge launches, 10 / 11 = key splits of the
  * most recent decode / prefill attention launch (values, not counts), 12 tall-tile GEMM, 13 32x32x16 vision attention, 14 variable-height
  * GEMM tiles (gemm_walk_vh_kernel; small class: gemm_vh_kernel), 15 vision q|k|v projection with the RoPE / V-transpose epilogue,
- * 16 input projection and gate/up of a layer-list decoder's 17 to 64 rows in one launch. */
+ * 16 input projection and gate/up of a layer-list decoder's 9 to 64 rows in one launch, 17 query norm,
+ * up-projection and absorption of a latent layer in one. */
 int lcc_debug_launch_counts(int64_t* out, int n, int reset);
 int lcc_debug_set_fused_attn(int mode); /* bit 0 (default on): engine decode uses the fused kernel for batches of >= 16 (stream,
                                           KV head) pairs; bit 2: for every batch; bit 1: key splits merged in the same launch by the
@@ -461,9 +462,10 @@ typedef struct {
   int bigram_buckets;                           /* 0: none; else a second embedding, row (previous * mul_prev + current * mul_cur) mod buckets */
   long long bigram_mul_prev, bigram_mul_cur;
 } lcc_decoder_config;
-/* 1 (default): decode steps of up to 16 streams run the fused launches (input + gate/up projections in one; query norm, up-projection, cache
- * append and gates in one for up to 8 streams; output projection + residual + next norm in one), steps of 17 to 64 rows input + gate/up projections in one
- * (latent attention layers); 0: separate launches.  Returns the old value */
+/* 1 (default): decode steps of up to 8 streams (latent layers wider than 2,048: 9) run the fused launches (input + gate/up projections in one; query norm,
+ * up-projection, cache append and gates in one; output projection + residual + next norm in one), steps of up to 64 rows input + gate/up projections in one
+ * (latent attention layers); where a latent layer's query rank is small, norms, up-projection and absorption are one launch at any number of rows; 0: separate
+ * launches.  Returns the old value */
 int lcc_debug_set_decoder_fused(int on);
 lcc_engine* lcc_engine_create_decoder(const lcc_decoder_config* cfg, const lcc_decoder_layer* layers, const lcc_engine_limits* lim);
 void lcc_engine_destroy(lcc_engine* e);
