@@ -2048,7 +2048,8 @@ static int big_tile_rows(const GemmArgs& a, int S, bool wide_only = false) {
   // 128 rows: 0.85 us a step while all tiles run at once, 0.93 in several rounds (514 rows of [37888, 3584]: 192-row tiles 141 us, these 156; fp8 weights 136 / 160)
   const bool second_round = (long)((a.M + 127) / 128) * ((a.N + 255) / 256) * S > 256;
   const float s128 = tile_score(a.M, a.N, S, 128, 256, 256, second_round && !slabs && !wide_only ? 0.76f : a.w_fp8 ? 0.85f : 0.82f, true);
-  // gemm_mid_kernel: 0.38 / 0.52 us a step of 64 x 128 / 128 x 128 against 0.85 of 128 x 256, one tile a compute unit at a time (two 64-row
+  // gemm_strip_kernel / gemm_mid_kernel: 0.38 (0.33 since its waves read their own weights) / 0.52 us a step of 64 x 128 / 128 x 128 against 0.85 of 128 x 256, one tile a compute
+  // unit at a time.  With 0.33 the choice is within 4 % of the best in 223 of 230 shapes, 5 to 7 % off in the others: the weights stay (two 64-row
   // tiles side by side take twice as long).  Returned as 0 / 129.  The 128-row form wins where its blocks fill one round and the 64-row
   // form's need two; beyond a round the 256-column tiles do (shapes around the lines: 1000 x 3584, K 3584: 43 / 34 / 52 us for 64 x 128 /
   // 128 x 128 / 128 x 256; 1456 x 3584: 73 / 61 / 52; 520 x 3584: 25 / 33 / 50).  With fp8 weights the steps stand alike (4608, K 3584: 386 rows
