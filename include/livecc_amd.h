@@ -86,6 +86,9 @@ int lcc_debug_set_gemm_variant(int variant);
  * the engine's prefill asks for at this shape (what csrc/engine_llm.hip passes as nsplit for the o / down / q|k|v projections).
  * w_fp8 != 0: *tile_rows = 0 (fp8 weights route inside their own entry point), *engine_splits as for fp8 weights. */
 int lcc_debug_gemm_plan(int M, int N, int K, int epilogue, int nsplit, int w_fp8, int32_t* tile_rows, int32_t* engine_splits);
+/* Host logic only: 1 if the input projection [N_in, K] (fp32 slabs, nsplit of them) and the gate/up projection [N_gate_up, K] of the same M rows of a decode step go
+ * into one launch, 0 if they are two; negative: invalid arguments */
+int lcc_debug_gemv_pair_plan(int M, int N_in, int N_gate_up, int K, int nsplit);
 /* attention: 0 = per-wave kernels (operands straight from L2); 1 = prefill shares K/V tiles through an LDS-DMA ring,
  * ViT per-wave; 2 = LDS-shared for both; 3 (default) = 2 with the LLM prefill on the 32x32x16 MFMAs (csrc/attn32.hip; applies to
  * calls with tile_rows >= 32; the engine then builds tiles of 32 or lcc_debug_attn_tile_rows() rows) */

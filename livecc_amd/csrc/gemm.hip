@@ -2241,7 +2241,8 @@ LCC_DEVICE void gemv_skinny_body(
         if (MG == 1) {
           xv[u][h][0] = ld16(ok ? xp[0] + kbc * 32 : zp);
         } else {       // full lines of the 64-k chunk (both k-blocks): instruction i = h*MG + mg; a chunk whose second k-block is past K reads the
-                       // zero page for the whole chunk only when the chunk itself is absent (K % 64 == 32 never occurs with MG > 1: checked by the launcher)
+                       // zero page for the whole chunk only when the chunk itself is absent (K % 64 == 32 never occurs with MG > 1: gemm_routes_skinny
+                       // from 17 rows on, gemv_rows_tiles and gemv_rows_pair_ok below)
 #pragma unroll
           for (int mg = 0; mg < MG; ++mg) xv[u][h][mg] = ld16((cc < ce) ? xp[h * MG + mg] + min(cc, nchunk - 1) * 64 : zp);
         }
@@ -2541,7 +2542,7 @@ static bool gemv_rows_pair_pays(const GemmArgs& in, const GemmArgs& sw) {
 // in: fp32 slabs (partial, nsplit); sw: SwiGLU.  Takes what the two calls of gemm_bf16 would take on the weight-streaming path with 9 to 64 rows, where it pays
 bool gemv_rows_pair_ok(const GemmArgs& in, const GemmArgs& sw) {
   auto one = [](const GemmArgs& a) {
-    return a.w_packed && !a.w_fp8 && a.M > 8 && a.M <= 64 && a.N > 0 && gemm_routes_skinny(a.M, a.K, false) && (a.N & 15) == 0 && (a.lda & 7) == 0 &&
+    return a.w_packed && !a.w_fp8 && a.M > 8 && a.M <= 64 && a.N > 0 && gemm_routes_skinny(a.M, a.K, false) && (a.K & 63) == 0 && (a.N & 15) == 0 && (a.lda & 7) == 0 &&
            (((uintptr_t)a.A | (uintptr_t)a.W) & 15) == 0 && a.bias == nullptr && a.tail.kind == 0;
   };
   return one(in) && one(sw) && in.M == sw.M && in.partial != nullptr && in.nsplit >= 1 && in.nsplit <= 8 && in.nsplit <= (in.K + 63) / 64 && in.epilogue == EPI_NONE &&

@@ -54,6 +54,14 @@ extern "C" int lcc_debug_gemm_plan(int M, int N, int K, int epilogue, int nsplit
   *tile_rows = w_fp8 ? 0 : gemm_plan(M, N, K, epilogue, nsplit, false);      // fp8 weights route inside gemm_w8 (not modelled here)
   return 0;
 }
+extern "C" int lcc_debug_gemv_pair_plan(int M, int N_in, int N_gate_up, int K, int nsplit) {
+  if (M <= 0 || N_in <= 0 || N_gate_up <= 0 || K <= 0 || nsplit <= 0) return fail(LCC_ERR_ARG, "lcc_debug_gemv_pair_plan: invalid arguments");
+  GemmArgs in, sw;      // the addresses are looked at for their alignment alone
+  in.A = sw.A = (const bf16_t*)256; in.W = sw.W = (const bf16_t*)256; in.partial = (float*)256; sw.C = (bf16_t*)256;
+  in.lda = sw.lda = (K + 7) & ~7; in.ldw = sw.ldw = K; in.w_packed = sw.w_packed = 1; in.M = sw.M = M; in.K = sw.K = K;
+  in.N = N_in; in.nsplit = nsplit; sw.N = N_gate_up; sw.ldc = N_gate_up / 2; sw.epilogue = LCC_EPI_SWIGLU;
+  return gemv_rows_pair_ok(in, sw) ? 1 : 0;
+}
 extern "C" int lcc_debug_set_fused_tails(int on);
 extern "C" int lcc_gemm_bf16(const void* A, int lda, const void* W, int ldw, int w_layout, const void* bias, const void* residual,
                              int ldr, void* C, int ldc, int M, int N, int K, int epilogue, float* partial, int nsplit, void* stream) {

@@ -146,6 +146,14 @@ def gemm_plan(M: int, N: int, K: int, epilogue: int = EPI_NONE, nsplit: int = 0,
     return int(out[0]), int(out[1])
 
 
+def gemv_pair_plan(M: int, N_in: int, N_gate_up: int, K: int, nsplit: int) -> bool:
+    """Whether a decode step's input and gate/up projections of M rows go into one launch (lcc_debug_gemv_pair_plan: host logic, no GPU)."""
+    rc = _lib.load().lcc_debug_gemv_pair_plan(int(M), int(N_in), int(N_gate_up), int(K), int(nsplit))
+    if rc < 0:
+        _lib.check(rc, "lcc_debug_gemv_pair_plan")
+    return bool(rc)
+
+
 def launch_counts(reset: bool = False) -> dict:
     """Host-side launch counters of the library (which kernel served the calls since the last reset): lcc_debug_launch_counts."""
     import numpy as np

@@ -58,6 +58,17 @@ def test_the_switch_restores_the_128_row_slabs(built_lib):
     assert r.stdout.strip() == "4 128", r.stdout      # four slabs on the 128-row tiles: the round-4 form
 
 
+@pytest.mark.parametrize("M", [1, 8, 9, 13, 16, 17, 40, 64, 65])
+def test_input_and_gate_up_projections_in_one_launch_take_whole_64_k_chunks(built_lib, M):
+    """9 to 64 rows (lcc_debug_gemv_pair_plan).  The kernel reads whole 64-k chunks of the activations: at K = 64 n + 32 the last one would run into the next row
+    (behind the last one past the buffer) and meet the last 32 weights twice."""
+    from livecc_amd import ops
+    for K in (64, 192, 1536, 3584):
+        assert ops.gemv_pair_plan(M, 1296, 2 * 1024, K, 1) == (9 <= M <= 64)
+        assert not ops.gemv_pair_plan(M, 1296, 2 * 1024, K + 32, 1)
+        assert not ops.gemv_pair_plan(M, 1296, 2 * 1024, K + 16, 1)
+
+
 def test_prefill_attention_plan_at_the_engines_shapes(built_lib):
     """Tile height x key-split count of the LLM prefill attention (lcc_debug_attn_plan: the function lcc_llm_prefill itself calls, no launch):
     one block per CU and (tile, KV head, split), relative time = rounds of blocks x keys per block; measured in
