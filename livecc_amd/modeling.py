@@ -36,6 +36,7 @@ import numpy as np
 import torch
 
 from . import protocol
+from ._lib import LccError
 from .config import BemuzenConfig, DebunexConfig, LiveCCConfig, architecture_of, get_config
 from .engine import Engine, Sampling
 from .weights import WeightArena, from_hf_model as _arena_from_hf, from_pretrained as _arena_from_pretrained, make_arena
@@ -429,8 +430,9 @@ class LiveCCForConditionalGeneration(EngineModel):
         max_new_rows    = rows of ONE prefill launch sequence -- longer prompts (the one-shot 24k-token video_qa / MCQ prefill)
                           are cut into pieces of at most this many rows over the carried KV (bit-identical to one pass);
         max_patches     = ViT patches of ONE encode launch sequence -- longer clips are encoded in groups of temporal slices
-                          (slices never attend to each other, Q2VL vision_utils.py:60-65); the workspace has room for an eighth
-                          more, so that a short last group goes with the one before it;
+                          (slices never attend to each other, Q2VL vision_utils.py:60-65).  One slice has to fit.  The workspace has
+                          room for an eighth more (72 KB a patch, 147 MB with the default; unused where a slice is larger than
+                          it), so that a short last group goes with the one before it;
         max_kv_len      = KV capacity per stream; default = the trained 32k window + max_history of generation headroom.
         text_offset_rule: "hf4" = transformers-4.5x M-RoPE text offset after a vision block (what the released checkpoints
         were trained with, ref README.md:30); "hf5" = the installed 5.15 oracle's rule.  Identical for every streaming chunk;
@@ -653,6 +655,8 @@ class LiveCCForConditionalGeneration(EngineModel):
             else:
                 t, h, w = (int(x) for x in c["grid"])
                 per_slice = h * w
+                if per_slice > self.max_patches:          # the engine's limit is an eighth above
+                    raise LccError(f"one slice of {h} x {w} patches is {per_slice} > max_patches {self.max_patches}")
                 slices = max(1, self.max_patches // per_slice)
                 pv = c["pixel_values"]
                 for a in range(0, t, slices):

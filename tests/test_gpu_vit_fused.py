@@ -153,3 +153,21 @@ def test_a_short_last_group_of_a_clip_goes_with_the_one_before_it(dev, slices, c
     assert len(seen) == calls and sum(seen) == slices and max(seen) <= 9
     want = torch.cat([native.get_video_features(frames=f[2 * i:2 * i + 2]) for i in range(slices)]).float()
     assert (got - want).norm() <= 2e-2 * want.norm()
+
+
+@pytest.mark.parametrize("h,w,fits", [(12, 16, True), (12, 18, False), (14, 16, False)])
+def test_one_slice_above_max_patches_is_refused_whatever_holds_it(dev, h, w, fits):
+    """max_patches is the limit of both inputs; the room behind it (192 patches, room for 216) is for a short last group of slices alone."""
+    from livecc_amd import _lib
+    from livecc_amd.config import tiny
+    native = _model(tiny(), dev, max_patches=192)
+    pixels = torch.zeros(2 * h * w, native.cfg.patch_dim, device=dev)
+    frames = torch.zeros(3, 3, 14 * h, 14 * w, dtype=torch.uint8, device=dev)
+    grid = torch.tensor([[2, h, w]])
+    if fits:
+        assert native.get_video_features(pixel_values_videos=pixels, video_grid_thw=grid).shape[0] == native.get_video_features(frames=frames).shape[0] == h * w // 2
+        return
+    with pytest.raises(_lib.LccError, match="max_patches 192"):
+        native.get_video_features(pixel_values_videos=pixels, video_grid_thw=grid)
+    with pytest.raises(ValueError, match="max_patches 192"):
+        native.get_video_features(frames=frames)
