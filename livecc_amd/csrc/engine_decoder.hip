@@ -116,7 +116,7 @@ int run_decoder_layers(lcc_engine* e, const DecBuffers& b, int S, const PrefillT
     LatentInArgs in; in.part = b.part; in.nsplit = ns; in.rows = S; in.ldn = in_n; in.qp = L.q_rank_pad; in.rp = own ? rp : 0; in.q_rank = L.q_rank;
     in.kv_rank = L.kv_rank; in.heads = L.heads; in.eps = e->dc.norm_eps; in.q_norm = w.q_norm; in.kv_norm = w.kv_norm; in.cq = b.cq; in.gate = b.gate;
     in.tok_stream = pt ? pt->tok_stream : d_slots; in.tok_pos = pt ? pt->tok_pos : nullptr; in.kv_len = e->d_kv_len; in.kv_base = e->d_kv_base; in.kv_off = kv_off;
-    const bool query = !pt && g_fused_decode && latent_query_ok(S, L.heads, L.dim_pad, L.q_rank_pad);
+    const bool query = !pt && g_fused_decode && latent_query_ok(in, L.dim_pad, rp);
     const bool fused_q = !query && fused && dgemv_latent_q_ok(S, L.q_rank_pad);
     if (!fused_q && !query) LCC_TRY(latent_norm_append(in, st));
     if (pt) {

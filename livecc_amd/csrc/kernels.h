@@ -292,7 +292,7 @@ struct MhaArgs {                 // causal multi-head attention of packed rows o
 constexpr int MHA_GROUP_ROWS = 256;
 int attn_mha(const MhaArgs& a, hipStream_t st);
 int attn_mha32_launch(const MhaArgs& a, hipStream_t st);      // dim, vdim in {64, 128}
-bool latent_query_ok(int rows, int heads, int dim, int qp);
+bool latent_query_ok(const LatentInArgs& a, int dim, int rp);      // rp: cache rank, also where a.rp is 0
 int latent_query(const LatentInArgs& a, const bf16_t* uq, const bf16_t* ukt, int dim, int rp, bf16_t* out, hipStream_t st);      // norms, q, absorb in one launch
 int latent_absorb(const float* q_part, int nsplit, int rows, int heads, int dim, const bf16_t* ukt, int rp, bf16_t* out, hipStream_t st);
 constexpr int LATENT_MAX_SPLIT = 128;

@@ -283,20 +283,33 @@ __global__ __launch_bounds__(512, 2) void latent_query_kernel(LatentInArgs a, co
   if (li < nrow) st8(out + ((size_t)(b0 + li) * a.heads + h) * rp + tile * 16 + g * 4, (u32x2){pack2(o[0], o[1]), pack2(o[2], o[3])});
 }
 // In place of three launches (32 rows, 12 heads, ranks 768 and 512: 4.0 + 4.2 + 4.1 us; up to 8 rows two of 5.9 + 4.3).  A step of 28 such layers, us, apart / here: 1 row 1188 / 1134,
-// 8 1458 / 1406, 16 1692 / 1589, 24 1538 / 1430, 32 1594 / 1464 (with 16 rows and 256 ranks a block 1529).  A wider query rank is more than a unit should pull for a head: 28 heads of
-// rank 1536 3,568 / 3,713 with 32 rows, 2,811 / 2,955 with one.  Few heads would append many rows one after another.
-bool latent_query_ok(int rows, int heads, int dim, int qp) { return rows >= 1 && rows <= 64 && heads >= 8 && dim == 128 && qp <= LATENT_Q_PIECES * 256; }
+// 8 1458 / 1406, 16 1692 / 1589, 24 1538 / 1430, 32 1594 / 1464 (with 16 rows and 256 ranks a block 1529).  Few heads would append many rows one after another.
+// Each block forms its head's query anew, so the form pays while all of them run at once and none pulls much.  us a layer, apart / here, heads, query rank, cache rank (blocks; KB of one):
+//   12, 768, 512: 32 rows (240; 279) 43.0 / 38.1;  24, 768, 512: 16 rows (240; 328) 49.6 / 46.3;  32, 768, 256: 16 rows (192; 352) 51.7 / 49.2;  40, 768, 512: 9 rows (200; 257) 64.3 / 61.5
+//   more blocks:  28, 768, 1024: 1 row (252; 232) 51.5 / 52.0;  32, 256, 512: 24 rows (320; 180) 57.2 / 60.5;  64, 768, 512: 1 row (320; 232) 75.3 / 79.0, 64 rows (1280; 623) 130 / 202
+//   more of one:  32, 768, 512: 12 rows (160; 414) 54.2 / 55.1;  28, 768, 512: 16 rows (140; 426) 53.0 / 52.3;  40, 768, 512: 16 rows (200; 524) 65.0 / 66.8
+// A query rank above 768 is more than a unit should pull for a head whatever else there is: 28 heads of rank 1536 3,568 / 3,713 a step with 32 rows, 2,811 / 2,955 with one.
+constexpr int LATENT_Q_BLOCKS = 240, LATENT_Q_PULL = 360 * 1000;
+static int latent_query_rows(int rows, int heads, int parts) {      // eight rows a block halve the slabs a unit pulls, while all blocks run at once
+  return (long)(parts + 1) * heads * ((rows + 7) / 8) <= 256 ? 8 : 16;
+}
+bool latent_query_ok(const LatentInArgs& a, int dim, int rp) {
+  if (a.rows < 1 || a.rows > 64 || a.heads < 8 || dim != 128 || a.qp > LATENT_Q_PIECES * 256) return false;
+  const int parts = (rp + 127) / 128, rg = latent_query_rows(a.rows, a.heads, parts);
+  return (long)(parts + 1) * a.heads * ((a.rows + rg - 1) / rg) <= LATENT_Q_BLOCKS &&
+         (long)a.qp * 256 + 32 * 1024 + (long)std::min(rg, a.rows) * a.qp * 4 * a.nsplit <= LATENT_Q_PULL;
+}
 int latent_query(const LatentInArgs& a, const bf16_t* uq, const bf16_t* ukt, int dim, int rp, bf16_t* out, hipStream_t st) {
-  if (!latent_query_ok(a.rows, a.heads, dim, a.qp)) return LCC_ERR_SHAPE;
+  if (!latent_query_ok(a, dim, rp)) return LCC_ERR_SHAPE;
   if ((a.qp & 63) || a.qp <= 0 || (rp & 63) || rp < 64 || (a.rp != 0 && a.rp != rp) || a.nsplit < 1 || (a.ldn & 3) || a.ldn < a.qp + a.rp + a.heads) return LCC_ERR_SHAPE;
   if (!a.part || !a.q_norm || !a.gate || a.q_rank < 1 || !uq || !ukt || !out) return LCC_ERR_ARG;
   if (a.rp > 0 && (!a.kv_norm || !a.tok_stream || (!a.tok_pos && !a.kv_len) || !a.kv_base || a.kv_rank < 1)) return LCC_ERR_ARG;
   g_launch_counts[LC_LATENT_QUERY]++;
   const int parts = (rp + 127) / 128;
-  // eight rows a block halve the slabs a unit pulls, while all blocks run at once
-  const int g8 = (a.rows + 7) / 8, g16 = (a.rows + 15) / 16;
-  if ((long)(parts + 1) * a.heads * g8 <= 256) latent_query_kernel<8><<<dim3(parts + 1, a.heads, g8), dim3(512), 0, st>>>(a, uq, ukt, rp, parts, out);
-  else latent_query_kernel<16><<<dim3(parts + 1, a.heads, g16), dim3(512), 0, st>>>(a, uq, ukt, rp, parts, out);
+  const int rg = latent_query_rows(a.rows, a.heads, parts);
+  const dim3 grid(parts + 1, a.heads, (a.rows + rg - 1) / rg);
+  if (rg == 8) latent_query_kernel<8><<<grid, dim3(512), 0, st>>>(a, uq, ukt, rp, parts, out);
+  else latent_query_kernel<16><<<grid, dim3(512), 0, st>>>(a, uq, ukt, rp, parts, out);
   return 0;
 }
 

@@ -526,11 +526,24 @@ def test_one_launch_and_two_give_the_same_bits(dev, lib, width, ff, n):
 @pytest.mark.parametrize("n,rank,kv", [(1, 768, 512), (7, 700, 130), (8, 64, 64), (9, 256, 512), (16, 300, 1000), (17, 513, 64), (24, 768, 300), (33, 48, 512), (64, 768, 512)])
 def test_norms_query_and_absorption_in_one_launch(dev, lib, n, rank, kv):
     """Query ranks of one channel to all that the kernel holds, eight rows a block and 16 (more blocks than units), short last groups, cache ranks of half a block's
-    to eight blocks'; a layer with a cache of its own and one that reads it; one split of the input projection and several (from nine rows on).  Both forms within the bound
-    of the tests around this one, and the next step reads what this one appended."""
-    from livecc_amd import ops
+    to eight blocks'; a layer with a cache of its own and one that reads it.  Both forms within the bound of the tests around this one, and the next step reads what this
+    one appended."""
     from livecc_amd.config import DebunexConfig
     cfg = DebunexConfig(300, 200, [U.L(U.M(9, 120, 64, rank, kv, 0.15), 320), U.L(U.M(8, 128, 40, rank, kv, 0.15, 0), 100)], 1e-5, 20.0, name="query")
+    _latent_queries(cfg, dev, lib, n, 4)
+
+
+@pytest.mark.parametrize("width,heads,rank,kv,n,taken", [(1600, 24, 768, 512, 16, True), (1600, 25, 768, 512, 16, False), (200, 48, 64, 512, 1, True), (200, 49, 64, 512, 1, False),
+                                                         (2304, 9, 768, 512, 40, True), (2304, 9, 768, 512, 64, False), (2304, 9, 640, 512, 64, True)])
+def test_many_blocks_and_wide_ones_keep_the_launches_apart(dev, lib, width, heads, rank, kv, n, taken):
+    """Both sides of both lines: 240 blocks, 360 KB that one of them pulls (three splits of the input projection at width 2304, two at 1600)."""
+    from livecc_amd.config import DebunexConfig
+    cfg = DebunexConfig(200, width, [U.L(U.M(heads, 128, 16, rank, kv, 0.15), 64), U.L(U.M(heads, 120, 24, rank, kv, 0.15, 0), 0)], 1e-5, 20.0, name="lines")
+    _latent_queries(cfg, dev, lib, n, 4 if taken else 0)
+
+
+def _latent_queries(cfg, dev, lib, n, launches):
+    from livecc_amd import ops
     T = U.make_weights(cfg, 5)
     m = _model(cfg, T, dev, max_streams=n, max_kv_len=128, max_new_rows=1024)
     seqs = [U.ids_of(cfg, 4 + i % 9, 30 + i) for i in range(n)]
@@ -542,7 +555,7 @@ def test_norms_query_and_absorption_in_one_launch(dev, lib, n, rank, kv):
             before = ops.launch_counts()["latent_query"]
             m.forward_step([(s, [x[-2]], [0]) for s, x in zip(st, seqs)])
             got = m.forward_step([(s, [x[-1]], [0]) for s, x in zip(st, seqs)])
-            assert ops.launch_counts()["latent_query"] - before == (4 if on else 0)
+            assert ops.launch_counts()["latent_query"] - before == (launches if on else 0)
             for i in sorted({0, n // 2, n - 1}):
                 assert U.error(got[i], U.oracle_logits(cfg, T, seqs[i])[[-1]]) < U.LIMIT
             for s in st:
