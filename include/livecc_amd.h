@@ -86,6 +86,9 @@ int lcc_debug_set_gemm_variant(int variant);
  * the engine's prefill asks for at this shape (what csrc/engine_llm.hip passes as nsplit for the o / down / q|k|v projections).
  * w_fp8 != 0: *tile_rows = 0 (fp8 weights route inside their own entry point), *engine_splits as for fp8 weights. */
 int lcc_debug_gemm_plan(int M, int N, int K, int epilogue, int nsplit, int w_fp8, int32_t* tile_rows, int32_t* engine_splits);
+/* Host logic only: how many 16-row tiles of a packed bf16 weight a block of the weight-streaming kernel takes (1, 2, 3, 4 or 6; nsplit > 0: slabs); 0: the product
+ * takes another kernel; negative: invalid arguments */
+int lcc_debug_gemv_plan(int M, int N, int K, int epilogue, int nsplit);
 /* Host logic only: 1 if the input projection [N_in, K] (fp32 slabs, nsplit of them) and the gate/up projection [N_gate_up, K] of the same M rows of a decode step go
  * into one launch, 0 if they are two; negative: invalid arguments */
 int lcc_debug_gemv_pair_plan(int M, int N_in, int N_gate_up, int K, int nsplit);

@@ -152,6 +152,7 @@ def load():
         "lcc_debug_set_fused_attn": (i32, [i32]),
         "lcc_debug_launch_counts": (i32, [vp, i32, i32]),
         "lcc_debug_gemm_plan": (i32, [i32, i32, i32, i32, i32, i32, vp, vp]),
+        "lcc_debug_gemv_plan": (i32, [i32, i32, i32, i32, i32]),
         "lcc_debug_gemv_pair_plan": (i32, [i32, i32, i32, i32, i32]),
         "lcc_debug_attn_tile_rows": (i32, [i32, i32]),
         "lcc_debug_attn_decode_splits": (i32, [vp, i32, i32]),

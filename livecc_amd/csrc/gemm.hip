@@ -2488,8 +2488,11 @@ static void launch_gemv_l(dim3 grid, const GemmArgs& a, void* out, int ldo, int 
 // on weights from memory): [1536, 10496] in eight splits 9.7 / 11.7, 11.7, 10.3; [1536, 8960] in eight 9.0 / 12.0, 10.5, 9.6.  Six: [3584, 18944] in five
 // 30.3 against 35.6 with two and 37.4 with four, [4608, 3584] in four 10.7 / 12.4 with one, gate/up with SwiGLU [17920, 1536] 14.1 / 16.2 with two,
 // 64 rows of [37888, 3584] 68.6 / 76.0.  Where one tile's blocks fill a round at most it stays: [2048, 1536] in two splits 4.7 / 5.1.
-// 10 to 16 rows run as 17 do, two groups of rows (one, in fragment-shaped loads: 2 to 6 % slower a step).  us a step of 28 layers, one or two tiles / as many as here, 9 / 10 / 12 / 16 rows: 2B with
-// recurrence 1862 / 1900, 1904 / 1893, 1980 / 1958, 2077 / 2009; 7B with recurrence 4182 / 4148, 4277 / 4207, 4467 / 4297, 4882 / 4510; 2B (q, k, v) 1410 / 1420, -, 1452 / 1403, 1497 / 1426
+// 10 to 16 rows run as 17 do, two groups of rows (one, in fragment-shaped loads: 2 to 6 % slower a step), whose way through LDS and larger last sums have to be earned: what a unit pulls,
+// by the 64 k of a chunk, has to be less by 20 + 6 for each tile.  us, one tile / several (which), 10, 12, 14, 16 rows: [3584, 18944] in five (6) 26.8 / 25.3, 28.2 / 25.5, 29.4 / 25.6, 31.4 / 25.8;
+// [152064, 3584] (4) 178 / 165, 190 / 166, 204 / 167, 219 / 168; [4608, 3584] in four (6) 8.9 / 9.5, 9.2 / 9.5, 9.5 / 9.5, 9.9 / 9.5; [4096, 4096] in four (2, 2, 4, 4) 7.9 / 8.6, 8.2 / 8.6, 8.5 / 9.1,
+// 8.9 / 9.1; [2304, 1536] in two (2) 4.4 / 5.1, 4.6 / 5.1, 4.7 / 5.1, 4.9 / 5.1; of 216 such products (54 shapes) 56 were slower without this, by 2 to 18 %, five are with it, by 2 to 5.  With SwiGLU a
+// block has two tiles anyway and two groups of rows come with four: no such line ([17920, 1536] (6) 13.4 / 12.8, 13.9 / 12.7, 14.1 / 12.9, 14.0 / 12.4, [12288, 2048] (4) 16 rows 11.8 / 10.9)
 static int gemv_rows_tiles(const GemmArgs& a, int S) {
   const bool pairs = a.epilogue == EPI_SWIGLU;
   const int least = pairs ? 2 : 1;
@@ -2499,7 +2502,15 @@ static int gemv_rows_tiles(const GemmArgs& a, int S) {
   int nt = least;
   for (int c : {2, 3, 4, 6})
     if (c > least && !(pairs && (c & 1)) && cost(c) < (c == 2 ? 0.97f : 0.85f) * cost(nt)) nt = c;
+  const int chunks = ((a.K + 63) / 64 + S - 1) / S;
+  if (a.M <= 16 && !pairs && nt > least && (cost(least) - cost(nt)) * (float)chunks < 20.f + 6.f * (float)nt) return least;
   return nt;
+}
+// the weight tiles a block takes (0: another route), for packed weights; nsplit > 0: slabs
+int gemv_plan_tiles(int M, int N, int K, int epilogue, int nsplit) {
+  if (gemm_plan(M, N, K, epilogue, nsplit, false) != 16) return 0;
+  GemmArgs a; a.w_packed = 1; a.M = M; a.N = N; a.K = K; a.epilogue = epilogue;
+  return gemv_rows_tiles(a, std::max(nsplit, 1));
 }
 template <int NTILE, int MODE>
 static void launch_gemv_tiles(const GemmArgs& a, int S, void* out, int ldo, int cps, hipStream_t st) {

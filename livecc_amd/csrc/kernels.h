@@ -85,6 +85,7 @@ bool gemv_rows_pair_ok(const GemmArgs& in, const GemmArgs& sw);                 
 int gemv_rows_pair(const GemmArgs& in, const GemmArgs& sw, hipStream_t st);          //   fp32 slabs and SwiGLU
 bool gemm_vit_qkv_eligible(int M, int E, int K);   // shapes the EPI_VIT_QK / EPI_VIT_V epilogues serve (8-wave kernel: K % 64 == 0; M > 64, M % 4 == 0, E % 32 == 0)
 int gemv_num_splits(int N, int K);
+int gemv_plan_tiles(int M, int N, int K, int epilogue, int nsplit);      // weight tiles a block of the weight-streaming kernel takes, 0: another route
 int gemm_plan(int M, int N, int K, int epilogue, int nsplit, bool w_fp8);     // host logic: which kernel family would serve this GEMM
 int gemm_tiled_num_splits(int M, int N, int K, bool packed_bf16 = false);      // packed_bf16: the small variable-height tiles may serve it (more splits)
 void set_gemv_variant(int v);

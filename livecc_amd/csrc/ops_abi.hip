@@ -54,6 +54,10 @@ extern "C" int lcc_debug_gemm_plan(int M, int N, int K, int epilogue, int nsplit
   *tile_rows = w_fp8 ? 0 : gemm_plan(M, N, K, epilogue, nsplit, false);      // fp8 weights route inside gemm_w8 (not modelled here)
   return 0;
 }
+extern "C" int lcc_debug_gemv_plan(int M, int N, int K, int epilogue, int nsplit) {
+  if (M <= 0 || N <= 0 || K <= 0 || nsplit < 0) return fail(LCC_ERR_ARG, "lcc_debug_gemv_plan: invalid arguments");
+  return gemv_plan_tiles(M, N, K, epilogue, nsplit);
+}
 extern "C" int lcc_debug_gemv_pair_plan(int M, int N_in, int N_gate_up, int K, int nsplit) {
   if (M <= 0 || N_in <= 0 || N_gate_up <= 0 || K <= 0 || nsplit <= 0) return fail(LCC_ERR_ARG, "lcc_debug_gemv_pair_plan: invalid arguments");
   GemmArgs in, sw;      // the addresses are looked at for their alignment alone

@@ -146,6 +146,14 @@ def gemm_plan(M: int, N: int, K: int, epilogue: int = EPI_NONE, nsplit: int = 0,
     return int(out[0]), int(out[1])
 
 
+def gemv_plan(M: int, N: int, K: int, epilogue: int = EPI_NONE, nsplit: int = 0) -> int:
+    """Weight tiles a block of the weight-streaming kernel takes, 0 for a product of another kernel (lcc_debug_gemv_plan: host logic, no GPU)."""
+    rc = _lib.load().lcc_debug_gemv_plan(int(M), int(N), int(K), int(epilogue), int(nsplit))
+    if rc < 0:
+        _lib.check(rc, "lcc_debug_gemv_plan")
+    return rc
+
+
 def gemv_pair_plan(M: int, N_in: int, N_gate_up: int, K: int, nsplit: int) -> bool:
     """Whether a decode step's input and gate/up projections of M rows go into one launch (lcc_debug_gemv_pair_plan: host logic, no GPU)."""
     rc = _lib.load().lcc_debug_gemv_pair_plan(int(M), int(N_in), int(N_gate_up), int(K), int(nsplit))

@@ -58,6 +58,24 @@ def test_the_switch_restores_the_128_row_slabs(built_lib):
     assert r.stdout.strip() == "4 128", r.stdout      # four slabs on the 128-row tiles: the round-4 form
 
 
+def test_several_weight_tiles_a_block_where_they_save_more_than_they_cost(ops):
+    """10 to 16 rows: products whose blocks pull much take what 17 rows take, short ones (measured up to 18 % slower so) one tile, as up to nine rows do."""
+    slabs = lambda N, K: ops.gemv_num_splits(N, K)      # noqa: E731
+    for M in (10, 12, 16):
+        for N, K in ((3584, 18944), (8192, 29568), (3584, 22528)):
+            assert ops.gemv_plan(M, N, K, nsplit=slabs(N, K)) > 1, (M, N, K)
+        for N, K in ((2304, 1536), (2560, 2560), (1408, 3072), (1024, 4096), (2816, 1536)):
+            assert ops.gemv_plan(M, N, K, nsplit=slabs(N, K)) == 1, (M, N, K)
+        for N, K in ((152064, 3584), (151936, 1536), (32000, 4096)):
+            assert ops.gemv_plan(M, N, K) > 1, (M, N, K)
+        assert ops.gemv_plan(M, 3584, 3584) == 1
+        assert ops.gemv_plan(M, 17920, 1536, ops.EPI_SWIGLU) == 6
+    assert ops.gemv_plan(14, 4096, 4096, nsplit=4) == ops.gemv_plan(10, 5120, 5120, nsplit=4) == ops.gemv_plan(10, H, H, nsplit=4) == 1 and ops.gemv_plan(10, QKV, H, nsplit=4) == 1 and ops.gemv_plan(16, QKV, H, nsplit=4) == 1
+    for N, K in ((3584, 18944), (2304, 1536)):
+        assert ops.gemv_plan(9, N, K, nsplit=slabs(N, K)) == 1 and ops.gemv_plan(17, N, K, nsplit=slabs(N, K)) > 1
+    assert ops.gemv_plan(16, 3584, 18944 + 32) == 1 and ops.gemv_plan(17, 3584, 18944 + 32) == 0 and ops.gemv_plan(65, 3584, 18944) == 0
+
+
 @pytest.mark.parametrize("M", [1, 8, 9, 13, 16, 17, 40, 64, 65])
 def test_input_and_gate_up_projections_in_one_launch_take_whole_64_k_chunks(built_lib, M):
     """9 to 64 rows (lcc_debug_gemv_pair_plan).  The kernel reads whole 64-k chunks of the activations: at K = 64 n + 32 the last one would run into the next row
