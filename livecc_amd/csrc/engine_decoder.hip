@@ -4,7 +4,7 @@
 // engine's (engine.hip, engine_llm.hip); this file is the launch sequence of the layers and what they need in memory.
 //
 // A layer is
-// (decode steps of up to eight or nine rows fuse "in" with "ff", the norms with "query", and "out" with the residual and the next norm: decode_v2.hip; where a head's part of the
+// (decode steps of up to eight, nine or twelve rows fuse "in" with "ff", the norms with "query", and "out" with the residual and the next norm: decode_v2.hip; where a head's part of the
 // query projection is small, the norms, "query" and the absorption are one launch at any number of rows: latent_query)
 //   in      [Wdq | Wdkv | Wg] h           one GEMM, fp32 slabs
 //           norms -> query latent, c -> cache, gates          (latent_norm_append)
@@ -84,15 +84,12 @@ int carve_bound(lcc_engine* e, DecBuffers* b) {
 }
 
 }  // namespace
-int g_fused_decode = 1;      // lcc_debug_set_decoder_fused: decode steps run the fused launches (up to eight or nine rows five or six per layer instead of nine, of up to 64 six to eight)
+int g_fused_decode = 1;      // lcc_debug_set_decoder_fused: decode steps run the fused launches (up to eight, nine or twelve rows, by the width, five or six per layer instead of nine, of up to 64 six to eight)
 
 namespace {
 // S packed rows through every layer; pt null: a decode step over the streams `d_slots`.  On exit b.h holds the final norm of the residual.
 int run_decoder_layers(lcc_engine* e, const DecBuffers& b, int S, const PrefillTables* pt, const int32_t* d_slots, int nsplit_attn, const AttnDirect& direct,
                        hipStream_t st) {
-  // From nine rows on (ten above a width of 2,048) the launches of 17 to 64 rows are the faster ones: their blocks pull the activations once for up to six weight tiles.  us a step, 28
-  // layers, 9 / 10 / 12 / 16 rows, these launches / those: width 1536 1418 / 1296, -, 1494 / 1326, 1584 / 1355; width 3584 3191 / 3250, 3250 / 3216, 3289 / 3186, 3510 / 3270
-  const bool fused = !pt && S <= (e->c.hidden_size <= 2048 ? 8 : 9) && g_fused_decode;
   const int W = e->c.hidden_size, NL = (int)e->dl.size();
   if (e->llm_over) return fail(LCC_ERR_STATE, "per-layer input overrides are not available for this model family");
   LCC_TRY(tap(e, b, 0, S, st));
@@ -103,6 +100,12 @@ int run_decoder_layers(lcc_engine* e, const DecBuffers& b, int S, const PrefillT
     const int owner = own ? l : L.kv_from, rp = L.kv_rank_pad, in_n = lcc_engine::dec_in_rows(L), ldcat = L.heads * L.vdim_pad + L.ff_pad;
     const size_t kv_off = e->dec_off[owner].kv;
     const float scale_log2e = L.scale * 1.4426950408889634f;
+    // From nine rows on (ten above a width of 2,048) the launches of 17 to 64 rows are the faster ones: their blocks pull the activations once for up to six weight tiles.  Output
+    // products of 2,561 to 4,096 columns fill most of one round with a tile a block, and beside a feed-forward that is not large the launch saved weighs as much until 13 rows.  us a layer,
+    // width, feed-forward, these launches / those: 1536, 8960: 9 rows 53.1 / 45.3;  2560, 6912: 10 59.1 / 57.8;  3072, 8192: 10 66.8 / 68.6, 12 68.8 / 69.2, 14 70.4 / 69.7;
+    // 3072, 16384: 10 91.0 / 91.2, 12 94.3 / 92.1;  3584, 18944: 10 109.0 / 107.8, 12 112.7 / 108.9 (9, a step of 28: 3191 / 3250);  4096, 11008: 10 88.8 / 93.6, 12 91.4 / 94.3, 14 93.8 / 94.8, 16 96.8 / 95.5;
+    // 4096, 14336: 10 99.6 / 101.7, 12 102.2 / 102.3;  5120, 13824: 10 136.3 / 122.6;  8192, 28672: 10 284 / 278
+    const bool fused = !pt && g_fused_decode && S <= (W <= 2048 ? 8 : W > 2560 && W <= 4096 && (long)W * L.ff_pad < 64l << 20 ? 12 : 9);
     int ns = 1;
     bool paired = false;          // the feed-forward's first product went with the input projection
     if (fused) {

@@ -564,6 +564,34 @@ def _latent_queries(cfg, dev, lib, n, launches):
             lib.lcc_debug_set_decoder_fused(old)
 
 
+@pytest.mark.parametrize("width,ff,rows", [(2112, 500, 9), (2624, 500, 12), (4096, 100, 12), (2624, 26000, 9), (4160, 100, 9)])
+def test_wide_layers_up_to_the_last_row_of_the_fused_launches_and_behind(dev, lib, width, ff, rows):
+    """Widths above 2,048: a step of `rows` rows runs the launches of up to eight, one more row those of up to 64.  Layers with a cache of their own and without, with and
+    without a feed-forward, all launches apart as well; the next step reads what this one appended."""
+    from livecc_amd import ops
+    from livecc_amd.config import DebunexConfig
+    cfg = DebunexConfig(150, width, [U.L(U.M(3, 100, 48, 900, 200, 0.15), ff), U.L(U.M(2, 128, 64, 130, 200, 0.15, 0), ff)], 1e-5, 20.0, name="wide")
+    T = U.make_weights(cfg, 6)
+    m = _model(cfg, T, dev, max_streams=rows + 1, max_kv_len=64, max_new_rows=256)
+    for n in (rows, rows + 1):
+        seqs = [U.ids_of(cfg, 4 + i % 7, 60 + i) for i in range(n)]
+        for on in (1, 0):
+            old = lib.lcc_debug_set_decoder_fused(on)
+            try:
+                st = [m.new_stream() for _ in seqs]
+                m.forward_step([(s, x[:-2], []) for s, x in zip(st, seqs)])
+                m.forward_step([(s, [x[-2]], [0]) for s, x in zip(st, seqs)])
+                before = ops.launch_counts()["dgemv_v2"]
+                got = m.forward_step([(s, [x[-1]], [0]) for s, x in zip(st, seqs)])
+                assert ops.launch_counts()["dgemv_v2"] - before == (4 if on and n == rows else 0)      # input and feed-forward; output, residual and norm
+                for i in sorted({0, 1, n // 2, n - 1}):
+                    assert U.error(got[i], U.oracle_logits(cfg, T, seqs[i])[[-1]]) < U.LIMIT
+                for s in st:
+                    s.release()
+            finally:
+                lib.lcc_debug_set_decoder_fused(old)
+
+
 def test_a_wide_input_projection_keeps_a_launch_of_its_own(dev):
     """64 rows, a query rank of 5120 beside a feed-forward of 8192 at width 2048: the projection's blocks of one tile would take longer than the launch saved."""
     from livecc_amd import ops
