@@ -250,7 +250,7 @@ int lcc_debug_bench_grid_barrier(int mode, int blocks, int iters, void* scratch,
  * most recent decode / prefill attention launch (values, not counts), 12 tall-tile GEMM, 13 32x32x16 vision attention, 14 variable-height
  * GEMM tiles (gemm_walk_vh_kernel; small class: gemm_vh_kernel), 15 vision q|k|v projection with the RoPE / V-transpose epilogue,
  * 16 input projection and gate/up of a layer-list decoder's 9 to 64 rows in one launch, 17 query norm,
- * up-projection and absorption of a latent layer in one. */
+ * up-projection and absorption of a latent layer in one, 18 = those of 15 on 128-column tiles. */
 int lcc_debug_launch_counts(int64_t* out, int n, int reset);
 int lcc_debug_set_fused_attn(int mode); /* bit 0 (default on): engine decode uses the fused kernel for batches of >= 16 (stream,
                                           KV head) pairs; bit 2: for every batch; bit 1: key splits merged in the same launch by the

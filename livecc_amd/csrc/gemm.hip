@@ -2827,10 +2827,14 @@ int gemm_bf16(const GemmArgs& a, hipStream_t st) {
     if (big == 160) big = 192;
     if (big == 272) big = 256;      // the rotation / transposed-V epilogues live on the fixed-height 256-column tiles (129, 0: the 128-row one, or for q, k and V together the 128-column tiles)
     // The narrow tiles where a product without these epilogues takes them (up to 1,024 patches at 1,280 channels).  A tower of 32 blocks, us, 128 x 256 tiles / here: 140 patches
-    // 2681 / 2370, 320 2896 / 2522, 560 3204 / 3004, 720 3387 / 3165, 880 3739 / 3501
-    if (all && big == 129) launch_mid_w<128, EPI_VIT_QKV, 4, false>(a, st);
-    else if (all && big == 0) launch_strip_w<EPI_VIT_QKV, false>(a, st);
-    else if (all) launch_vit<EPI_VIT_QKV>(a, big, st);
+    // 2681 / 2370, 320 2896 / 2522, 560 3204 / 3004, 720 3387 / 3165, 880 3739 / 3501.  Under a cap on the workgroups only while their tiles all run at once: a unit gets less done with them
+    // (128 units: 140 patches, 90 tiles, 3004 / 2617; 560, 270 tiles, 3842 / 3983; 768, 360, 4014 / 4238; 40 units: 560 8337 / 8623)
+    const long tiles = (long)(big == 129 ? (a.M + 127) / 128 : (a.M + 63) / 64) * ((a.N + 127) / 128);
+    const bool narrow = all && (big == 129 || big == 0) && (get_grid_cap() <= 0 || tiles <= get_grid_cap());
+    if (narrow) {
+      g_launch_counts[LC_GEMM_VIT_QKV_NARROW]++;
+      big == 129 ? launch_mid_w<128, EPI_VIT_QKV, 4, false>(a, st) : launch_strip_w<EPI_VIT_QKV, false>(a, st);
+    } else if (all) launch_vit<EPI_VIT_QKV>(a, big, st);
     else if (qk) launch_vit<EPI_VIT_QK>(a, big, st);
     else launch_vit<EPI_VIT_V>(a, big, st);
     return 0;

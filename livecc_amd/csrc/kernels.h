@@ -30,7 +30,8 @@ enum LaunchCounter {
   LC_GEMM_VIT_QKV = 15,        // gemm_vit_kernel: EPI_VIT_QK / EPI_VIT_V epilogues (RoPE / V transpose fused into the q|k|v projection; one EPI_VIT_QKV launch per tower block when E % 128 == 0, else a q|k launch + a V launch)
   LC_GEMV_ROWS_PAIR = 16,      // gemv_rows_pair_kernel (input projection and gate/up of 9 to 64 rows in one launch)
   LC_LATENT_QUERY = 17,        // latent_query_kernel (query norm, up-projection and absorption in one launch)
-  LC_COUNT = 18
+  LC_GEMM_VIT_QKV_NARROW = 18, // ... of these, on the 64 x 128 and 128 x 128 tiles (gemm_strip_kernel, gemm_mid_kernel)
+  LC_COUNT = 19
 };
 extern long long g_launch_counts[LC_COUNT];
 

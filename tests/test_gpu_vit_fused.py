@@ -71,14 +71,21 @@ def test_fused_qkv_epilogue_of_the_128_column_tiles(dev, shapes, tile):
     clips = _clips(shapes, dev, seed=17)
     plain, fused, c0, c1 = _both(native, clips)
     assert c0["gemm_vit_qkv"] == 0 and c1["gemm_vit_qkv"] == cfg.vit_depth
+    assert tile is None or c1["gemm_vit_qkv_narrow"] == (cfg.vit_depth if tile in (64, 129) else 0)
     assert torch.isfinite(fused.float()).all() and torch.equal(plain, fused)
-    native.engine.set_vit_grid_cap(40)
-    try:
-        capped = native.engine.vit_encode(clips).clone()
-    finally:
-        native.engine.set_vit_grid_cap(0)
-    torch.cuda.synchronize()
-    assert torch.equal(capped, fused)
+    # under a cap on the workgroups the narrow tiles are for products whose tiles all run at once
+    for cap in (40, 128, 248):
+        blocks = 30 * ((patches + 63) // 64 if tile == 64 else (patches + 127) // 128)
+        native.engine.set_vit_grid_cap(cap)
+        ops.launch_counts(reset=True)
+        try:
+            capped = native.engine.vit_encode(clips).clone()
+        finally:
+            native.engine.set_vit_grid_cap(0)
+        torch.cuda.synchronize()
+        assert torch.equal(capped, fused)
+        if tile is not None:
+            assert ops.launch_counts()["gemm_vit_qkv_narrow"] == (cfg.vit_depth if tile in (64, 129) and blocks <= cap else 0)
 
 
 @pytest.mark.parametrize("streams", [1, 8])
