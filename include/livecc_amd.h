@@ -468,10 +468,10 @@ typedef struct {
   int bigram_buckets;                           /* 0: none; else a second embedding, row (previous * mul_prev + current * mul_cur) mod buckets */
   long long bigram_mul_prev, bigram_mul_cur;
 } lcc_decoder_config;
-/* 1 (default): decode steps of up to 8 streams (latent layers wider than 2,048: 9) run the fused launches (input + gate/up projections in one; query norm,
- * up-projection, cache append and gates in one; output projection + residual + next norm in one), steps of up to 64 rows input + gate/up projections in one
- * (latent attention layers); where a latent layer's query rank is small, norms, up-projection and absorption are one launch at any number of rows; 0: separate
- * launches.  Returns the old value */
+/* 1 (default): decode steps of up to 8 streams (latent layers wider than 2,048: 9, of 2,561 to 4,096 with a feed-forward that is not large: 12) run the fused
+ * launches (input + gate/up projections in one; query norm, up-projection, cache append and gates in one; output projection + residual + next norm in one), steps
+ * of up to 64 rows input + gate/up projections in one (latent attention layers); where a latent layer has a small query rank and few blocks of heads, cache ranks
+ * and rows, norms, up-projection and absorption are one launch at any number of rows; 0: separate launches.  Returns the old value */
 int lcc_debug_set_decoder_fused(int on);
 lcc_engine* lcc_engine_create_decoder(const lcc_decoder_config* cfg, const lcc_decoder_layer* layers, const lcc_engine_limits* lim);
 void lcc_engine_destroy(lcc_engine* e);
@@ -576,9 +576,9 @@ int lcc_llm_prefill(lcc_engine* e, int n_streams, const int32_t* slots, const in
                     const int32_t* vit_index, const void* vit_embeds, const int32_t* pos3, const lcc_sampling* sp,
                     void* stream);
 /* n_steps further decode steps for the same streams without any host round trip.  n_streams <= LCC_MAX_DECODE_BATCH (and
- * <= max_new_rows): up to 16 streams are one activation fragment per weight fragment of the weight-streaming GEMVs; 17..64 streams run the
- * same kernels with 2-4 activation fragments per weight fragment (bf16 weights; lcc_debug_set_skinny_rows lowers the limit) or, with fp8
- * weights, the 64-row GEMM tiles -- either way the weights are streamed once per step for the whole batch.  Larger batches: call once
+ * <= max_new_rows): up to 9 streams (fp8 weights: 16) are one activation fragment per weight fragment of the weight-streaming GEMVs, 10..16 one or
+ * two; 17..64 streams run the same kernels with 2-4 activation fragments per weight fragment (bf16 weights; lcc_debug_set_skinny_rows lowers the
+ * limit) or, with fp8 weights, the 64-row GEMM tiles -- either way the weights are streamed once per step for the whole batch.  Larger batches: call once
  * per group. */
 #define LCC_MAX_DECODE_BATCH 64
 int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots, int n_steps, int first_step_index,

@@ -126,7 +126,8 @@ LCC_DEVICE void attn32_key_loop(unsigned char* alds, const Kv32& kv, const u32x4
   const int col = lane & 31;
 
   // DMA: this wave's pieces of a pair.  Surplus slots copy the last piece again (same bytes, same place).  What a piece needs in every pair -- its operand, tiles from the
-  // pair's, row bytes and place in a slot -- is kept in scalar registers: formed anew, a pair of the tower kernel had 110 scalar instructions beside 190 others
+  // pair's, row bytes and place in a slot -- is kept in scalar registers: formed anew, a pair of the four-wave tower kernel had 101 scalar instructions
+  // beside 202 others, now 68 (eight waves 60 / 42, LLM prefill 63 / 45); one chunk's tower 4,079 / 4,042 us in turn on one card, eight chunks' the same
   struct Piece { const char* base; unsigned stride, row, at; int dt, lo; };
   Piece pc[PWP];
   unsigned off[PWP], prow[CLAMP ? PWP : 1];

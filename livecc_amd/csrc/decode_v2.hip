@@ -696,7 +696,7 @@ static int dg_check(const DgArgs& a, int pro, int epi) {
 
 int dgemv_in_swiglu(const DgArgs& in, const DgArgs& sw, hipStream_t st) {
   g_launch_counts[LC_DGEMV_V2]++;
-  if (in.M < 1 || in.M > 16 || sw.M != in.M || (in.N & 15) || (sw.N & 31) || (in.K & 31) || (sw.K & 31) || (in.ldx & 7) || (sw.ldx & 7) || (in.ldc & 3) || (sw.ldc & 3))
+  if (in.M < 1 || in.M > DGEMV_DECODER_ROWS || sw.M != in.M || (in.N & 15) || (sw.N & 31) || (in.K & 31) || (sw.K & 31) || (in.ldx & 7) || (sw.ldx & 7) || (in.ldc & 3) || (sw.ldc & 3))
     return LCC_ERR_SHAPE;
   if (!in.W || !in.X || !in.C32 || in.wscale || (sw.N > 0 && (!sw.W || !sw.X || !sw.C || sw.wscale))) return LCC_ERR_ARG;
   dgemv_in_swiglu_kernel<<<dim3(in.N / 16 + sw.N / 32), dim3(256), 0, st>>>(in, sw, in.N / 16);
@@ -704,7 +704,7 @@ int dgemv_in_swiglu(const DgArgs& in, const DgArgs& sw, hipStream_t st) {
 }
 static int dg_f32_check(const DgArgs& a) {
   g_launch_counts[LC_DGEMV_V2]++;
-  if (a.M < 1 || a.M > 16 || a.N < 16 || (a.N & 15) || (a.K & 31) || a.K < 32 || (a.ldx & 7) || (a.ldc & 3)) return LCC_ERR_SHAPE;
+  if (a.M < 1 || a.M > DGEMV_MIXER_ROWS || a.N < 16 || (a.N & 15) || (a.K & 31) || a.K < 32 || (a.ldx & 7) || (a.ldc & 3)) return LCC_ERR_SHAPE;
   return !a.W || !a.X || !a.C32 || a.wscale ? LCC_ERR_ARG : 0;
 }
 int dgemv_f32(const DgArgs& a, hipStream_t st) {
@@ -725,7 +725,7 @@ int dgemv_f32_pair(const DgArgs& a, const DgArgs& b, hipStream_t st) {
 // gate/up Linear [SwiGLU] of rows that are normed already
 int dgemv_swiglu(const DgArgs& a, hipStream_t st) {
   if (int rc = dg_check(a, DG_PRO_PLAIN, DG_EPI_SWIGLU)) return rc;
-  if (a.wscale) return LCC_ERR_ARG;
+  if (a.wscale || a.M > DGEMV_MIXER_ROWS) return LCC_ERR_ARG;
   dgemv_kernel<2, DG_PRO_PLAIN, DG_EPI_SWIGLU, 4, 1, 2><<<dim3(a.N / 32), dim3(256), 0, st>>>(a);
   return 0;
 }
@@ -740,7 +740,7 @@ int dgemv_latent_q(const DgArgs& a, const LatentInArgs& row, hipStream_t st) {
 // fp32 residual += Linear(x), h = next norm
 int dgemv_resid_dyt(const DgArgs& a, hipStream_t st) {
   g_launch_counts[LC_DGEMV_V2]++;
-  if (a.M < 1 || a.M > 16 || (a.N & 15) || (a.K & 31) || (a.ldx & 7)) return LCC_ERR_SHAPE;
+  if (a.M < 1 || a.M > DGEMV_DECODER_ROWS || (a.N & 15) || (a.K & 31) || (a.ldx & 7)) return LCC_ERR_SHAPE;
   if (!a.W || !a.X || !a.X32 || !a.C || !a.dyt.w || !a.dyt.b || !a.dyt.alpha || a.wscale) return LCC_ERR_ARG;
   if (dgemv_rows8_ok(a.M, a.N, a.K, nullptr)) { launch_rows8<DG_EPI_RESID_DYT>(a, st); return 0; }
   if (a.K >= 8192) dgemv_kernel<1, DG_PRO_PLAIN, DG_EPI_RESID_DYT, 16, 3><<<dim3(a.N / 16), dim3(1024), 0, st>>>(a);

@@ -38,7 +38,7 @@ static inline int slab_gemm(const DecBuffers& b, const bf16_t* A, int lda, const
   *nsplit = s;
   return gemm_bf16(g, st);
 }
-// slab_gemm(A, W) and the SwiGLU product of the same rows (gate_up, into C), in one launch where that is the faster one (17 to 64 rows: gemv_rows_pair_ok); *paired: it was
+// slab_gemm(A, W) and the SwiGLU product of the same rows (gate_up, into C), in one launch where that is the faster one (9 to 64 rows: gemv_rows_pair_ok); *paired: it was
 static inline int slab_swiglu_gemm(const DecBuffers& b, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K, const bf16_t* gate_up, int N2, bf16_t* C, int ldc,
                                    int* nsplit, bool* paired, hipStream_t st) {
   GemmArgs g, s;

@@ -105,7 +105,7 @@ int run_decoder_layers(lcc_engine* e, const DecBuffers& b, int S, const PrefillT
     // width, feed-forward, these launches / those: 1536, 8960: 9 rows 53.1 / 45.3;  2560, 6912: 10 59.1 / 57.8;  3072, 8192: 10 66.8 / 68.6, 12 68.8 / 69.2, 14 70.4 / 69.7;
     // 3072, 16384: 10 91.0 / 91.2, 12 94.3 / 92.1;  3584, 18944: 10 109.0 / 107.8, 12 112.7 / 108.9 (9, a step of 28: 3191 / 3250);  4096, 11008: 10 88.8 / 93.6, 12 91.4 / 94.3, 14 93.8 / 94.8, 16 96.8 / 95.5;
     // 4096, 14336: 10 99.6 / 101.7, 12 102.2 / 102.3;  5120, 13824: 10 136.3 / 122.6;  8192, 28672: 10 284 / 278
-    const bool fused = !pt && g_fused_decode && S <= (W <= 2048 ? 8 : W > 2560 && W <= 4096 && (long)W * L.ff_pad < 64l << 20 ? 12 : 9);
+    const bool fused = !pt && g_fused_decode && S <= (W <= 2048 ? 8 : W > 2560 && W <= 4096 && (long)W * L.ff_pad < 64l << 20 ? DGEMV_DECODER_ROWS : 9);
     int ns = 1;
     bool paired = false;          // the feed-forward's first product went with the input projection
     if (fused) {

@@ -195,7 +195,9 @@ bool decode_v2_ok(const lcc_engine* e) {
 // v2 normalises rows in every block for one or two streams and uses row-scaled products for 3 to 16 (one / two streams: 7B 2.81 / 2.90 ms a
 // step against 2.81 / 2.93 row-scaled, 2B 1.17 / 1.18 against 1.19 / 1.19; three: 3.02 -> 2.85 against the sequence with norm launches).
 // More than eight rows do not fit the 8-row residual blocks, and 16-row ones leave most of the chip idle at 2,048 hidden channels and
-// below: 2B, 12 / 16 streams 1.48 / 1.56 ms with norm launches against 1.52 / 1.66 (nine: 1.44 against 1.41).
+// below: 2B, 12 / 16 streams 1.48 / 1.56 ms with norm launches against 1.52 / 1.66 (nine: 1.44 against 1.41).  (7B in bf16: since products of 10 to 16 rows take
+// several weight tiles a block the sequence with norm launches is as fast with 12 streams, 3.28 ms a step against 3.26, and faster with 16, 3.39-3.42 against 3.50;
+// 10 3.21 / 3.10.  The line stands at 16 as below; fp8, 16: 2.91 / 2.71.)
 // What it saves is two norm launches and the slabs of a layer, what it costs is slower products, by their bytes and their rows: it serves while a
 // layer's weight bytes x rows stay below 8e9.  Eight layers at 2,000 keys, row-scaled / with norm launches, us: 7B (466 MB a layer) 16 streams
 // 1,271 / 1,284; 72B (1.76 GB) 3 / 4 / 5 / 8 / 16 streams 2,736 / 2,765 / 2,805 / 2,934 / 3,489 against 2,742 / 2,759 / 2,784 / 2,889 / 3,349; 72B in
@@ -467,9 +469,9 @@ extern "C" int lcc_llm_decode(lcc_engine* e, int n_streams, const int32_t* slots
   CallScope in_flight;
   std::lock_guard<std::mutex> lk(e->mu_llm);
   if (n_streams <= 0 || !slots || n_steps < 0) return fail(LCC_ERR_ARG, "bad argument");
-  // <= 16 streams: one activation fragment per weight fragment of the weight-streaming GEMVs.  17..64 (bf16 weights): the same kernels with
-  // 2-4 activation fragments per weight fragment (gemv_skinny_kernel<..., MG>, round 4); fp8 weights above 16 rows: the GEMM tiles
-  // of the prefill path.  One predicate decides (gemm.hip: gemm_routes_skinny).  Beyond 64 the caller splits.
+  // Up to 9 streams: one activation fragment per weight fragment of the weight-streaming GEMVs.  bf16 weights, up to 64: the same kernels with 2-4 activation
+  // fragments per weight fragment (gemv_skinny_kernel<..., MG>; up to 16 streams where that is the faster form: gemv_rows_tiles); fp8 weights above 16
+  // rows: the GEMM tiles of the prefill path.  One predicate decides (gemm.hip: gemm_routes_skinny).  Beyond 64 the caller splits.
   if (n_streams > LCC_MAX_DECODE_BATCH)
     return fail(LCC_ERR_SHAPE, "decode batches of more than %d streams are not supported", LCC_MAX_DECODE_BATCH);
   if (n_streams > e->lim.max_new_rows) return fail(LCC_ERR_STATE, "%d streams > max_new_rows %d", n_streams, e->lim.max_new_rows);

@@ -585,18 +585,6 @@ __global__ __launch_bounds__(256) void gemm_glds_kernel(
   }
 }
 
-// ------------------------------------------------------------------------------------------------
-// 128 x 128 x 64 tile on EIGHT waves with a four-stage LDS-DMA ring: shapes whose 256-column tiles leave most of the chip idle
-// ------------------------------------------------------------------------------------------------
-// The time is the chain of K / 64 steps of one block, and a split of K would give another summation order.
-//   * three stages (96 KB) are in flight;
-//   * the fragments of tile kt + 1 are read into a second register set under the MFMAs of tile kt, behind the same barrier;
-//   * eight waves, each 64 rows x 32 columns.
-// What bounds it: LDS (a step reads 96 KB of fragments and takes 32 KB from the DMA = 1,024 clocks at 128 B/clk against 512 of MFMA per SIMD) and lines
-// from beyond the L2 (gemm_strip_kernel).  Same summation order as every other tile kernel of this file.  Measured (us, the tile chosen before -> here): 1000 x 3584,
-// K 22528 285 -> 196; 2000 x 1280, K 5120 55 -> 41.
-// Requires packed W, K % 64 == 0.  W8: fp8 weights in their packed order, 1 KB a fragment's 64 k, converted in registers in front of the
-// MFMAs (the form before wrote the whole weight as bf16 first): 600 x 4608, K 3584 50 -> 34.
 // The last part of a vision q|k|v tile of 32 columns a wave, NW waves: every wave is done with the stages (dsmem), and its DMA pieces have landed
 template <int EPI, int BM, int NW, int MT, int NT>
 LCC_DEVICE void vit_tile_end(const f32x4 (&acc)[MT][NT], u32x4* dsmem, int m0, int row0, int nbase, int lane, int wave, const bf16_t* bias, bf16_t* C, int ldc, int M, int N,
@@ -620,14 +608,27 @@ LCC_DEVICE void vit_tile_end(const f32x4 (&acc)[MT][NT], u32x4* dsmem, int m0, i
   }
 }
 
-template <int BM, int EPI, int NST, bool W8>
+// ------------------------------------------------------------------------------------------------
+// 128 x 128 x 64 tile on EIGHT waves with a four-stage LDS-DMA ring: shapes whose 256-column tiles leave most of the chip idle
+// ------------------------------------------------------------------------------------------------
+// The time is the chain of K / 64 steps of one block, and a split of K would give another summation order.
+//   * three stages (96 KB) are in flight;
+//   * the fragments of tile kt + 1 are read into a second register set under the MFMAs of tile kt, behind the same barrier;
+//   * eight waves, each 64 rows x 32 columns.
+// What bounds it: LDS (a step reads 96 KB of fragments and takes 32 KB from the DMA = 1,024 clocks at 128 B/clk against 512 of MFMA per SIMD) and lines
+// from beyond the L2 (gemm_strip_kernel).  Same summation order as every other tile kernel of this file.  Measured (us, the tile chosen before -> here): 1000 x 3584,
+// K 22528 285 -> 196; 2000 x 1280, K 5120 55 -> 41.
+// Requires packed W, K % 64 == 0.  W8: fp8 weights in their packed order, 1 KB a fragment's 64 k, converted in registers in front of the
+// MFMAs (the form before wrote the whole weight as bf16 first): 600 x 4608, K 3584 50 -> 34.
+constexpr int MID_STAGES = 4;
+template <int EPI, bool W8>
 LCC_DEVICE void gemm_mid_tile(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual,
     int ldr, bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tm, int tn, float* __restrict__ partial, int kt_per_split,
     const float* __restrict__ wscale, const VitQkvEpi& vq) {
-  constexpr int BN = 128, BK = 64, MT = BM / 32, NT = 2;
+  constexpr int BM = 128, BN = 128, BK = 64, MT = BM / 32, NT = 2, NST = MID_STAGES;
   constexpr int WF = W8 ? 1 : 2;                                  // 1-KB weight sub-tiles of a fragment row
-  constexpr int A_UNITS = BM * 8, STAGE = A_UNITS + 8 * WF * 64;  // 16-byte units: [BM rows][8 chunks] (XOR-swizzled) + 16 weight sub-tiles = 24 / 32 KB
+  constexpr int A_UNITS = BM * 8, STAGE = A_UNITS + 8 * WF * 64;  // 16-byte units: [BM rows][8 chunks] (XOR-swizzled) + 16 weight sub-tiles = 32 KB (fp8 weights: 24)
   constexpr int APW = BM / 64, P = APW + WF;                      // DMA pieces of a wave per k-tile: 8 activation rows each, then the weights
   extern __shared__ __attribute__((aligned(16))) u32x4 dsmem[];
 
@@ -724,7 +725,7 @@ LCC_DEVICE void gemm_mid_tile(
                                     reinterpret_cast<unsigned char*>(dsmem) + wave * 4096);
   } else tile_epilogue<EPI, MT, NT>(acc, m0 + wm * (BM / 2), n0 + wn * 32, (n0 + wn * 32) / 2, li, g, bias, residual, ldr, C, ldc, M, N, partial, wscale);
 }
-template <int BM, int EPI, int NST, bool W8>
+template <int EPI, bool W8>
 __global__ __launch_bounds__(512) void gemm_mid_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual,
     int ldr, bf16_t* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n, float* __restrict__ partial, int kt_per_split,
@@ -749,9 +750,9 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(
   if constexpr (EPI == EPI_VIT_QKV) {
     const int qk_tiles = 2 * vq.E / 128;          // V: rows 2E.. of the packed weight
     if (tn >= qk_tiles)
-      gemm_mid_tile<BM, EPI_VIT_V, NST, W8>(A, lda, W + (size_t)2 * vq.E * K, bias != nullptr ? bias + 2 * vq.E : nullptr, nullptr, 0, nullptr, 0, M, vq.E, K, tm, tn - qk_tiles, nullptr, 0, nullptr, vq);
-    else gemm_mid_tile<BM, EPI_VIT_QK, NST, W8>(A, lda, W, bias, nullptr, 0, C, ldc, M, 2 * vq.E, K, tm, tn, nullptr, 0, nullptr, vq);
-  } else gemm_mid_tile<BM, EPI, NST, W8>(A, lda, W, bias, residual, ldr, C, ldc, M, N, K, tm, tn, partial, kt_per_split, wscale, vq);
+      gemm_mid_tile<EPI_VIT_V, W8>(A, lda, W + (size_t)2 * vq.E * K, bias != nullptr ? bias + 2 * vq.E : nullptr, nullptr, 0, nullptr, 0, M, vq.E, K, tm, tn - qk_tiles, nullptr, 0, nullptr, vq);
+    else gemm_mid_tile<EPI_VIT_QK, W8>(A, lda, W, bias, nullptr, 0, C, ldc, M, 2 * vq.E, K, tm, tn, nullptr, 0, nullptr, vq);
+  } else gemm_mid_tile<EPI, W8>(A, lda, W, bias, residual, ldr, C, ldc, M, N, K, tm, tn, partial, kt_per_split, wscale, vq);
   if (vb + (int)gridDim.x < nblk) __syncthreads();     // the next tile's DMA reuses the stages
   }
 }
@@ -766,10 +767,10 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(
 // together and that come from memory at 45-58, whatever is in flight (2 to 8 steps measured the same): 24 KB a step are 0.16 us or 0.42.  So
 //   * compute units that get no tile read the weight ahead of the others into the memory-side cache (strip_fetch), whose lines come sooner than DRAM's;
 //   * nothing is requested past the last tile but what the full groups of D steps do.
-// Measured (us, weights from memory; the eight-wave form before -> these -> with fetching blocks): 1456 x 1280, K 5120 35.3 -> 33.0 -> 28.8, K 1280 10.6 -> 9.8;
-// 720 x 1280, K 5120 29.2 -> 28.7 -> 25.5; 390 x 3584, K 3584 23.7 -> 22.4 -> 20.5; 1120 x 1280, K 5184 30.9 -> 30.3 -> 25.4.
+// Measured (us, weights from memory; the eight-wave form before -> these -> with fetching blocks): 1456 x 1280, K 5120 35.3 -> 33.0 -> 28.1, K 1280 10.6 -> 9.8;
+// 720 x 1280, K 5120 29.2 -> 28.7 -> 25.4; 390 x 3584, K 3584 23.7 -> 22.4 -> 20.6; 1120 x 1280, K 5184 30.9 -> 30.3 -> 25.1.
 // Not taken: weight loads past the caches (nt: 33 -> 40, the other blocks of the XCD fetch them again), 8 to 12 steps ahead (no faster), a dword of every line ahead of
-// its use by the block itself (loads return in order: slower), 128 rows x 32 columns a wave (2 to 4 % either way of gemm_mid_kernel<128>).
+// its use by the block itself (loads return in order: slower), 128 rows x 32 columns a wave (2 to 4 % either way of gemm_mid_kernel).
 // Same summation order as every other tile kernel of this file.  Requires packed W, K % 64 == 0.  W8: fp8 weights in their packed order, 1 KB a fragment's 64 k,
 // converted in registers in front of the MFMAs.
 // Blocks without a tile read 2 KB of every fragment row by turns, from piece c0 to c1 of the rows (`row` pieces of 16 bytes each), in the order in which the others will
@@ -1798,20 +1799,20 @@ static int g_gemm_sched = 1;   // fragment-read schedule of gemm_big_kernel: 0 c
 void set_gemm_variant(int v);
 
 static inline int raster_for(int tiles_m);
-template <int BM, int EPI, int NST, bool W8>
+template <int EPI, bool W8>
 static void launch_mid_w(const GemmArgs& a, hipStream_t st) {
-  const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + 127) / 128, nkt = a.K / 64, S = (EPI == EPI_PARTIAL) ? a.nsplit : 1;
-  constexpr size_t lds = (size_t)NST * (BM * 128 + (W8 ? 8192 : 16384));
+  const int tiles_m = (a.M + 127) / 128, tiles_n = (a.N + 127) / 128, nkt = a.K / 64, S = (EPI == EPI_PARTIAL) ? a.nsplit : 1;
+  constexpr size_t lds = (size_t)MID_STAGES * (16384 + (W8 ? 8192 : 16384));
   static DeviceOnce attr_set;   // per instantiation
-  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_mid_kernel<BM, EPI, NST, W8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  gemm_mid_kernel<BM, EPI, NST, W8><<<dim3(capped_grid((long)tiles_m * tiles_n), S), dim3(512), lds, st>>>(
+  if (attr_set.first()) (void)hipFuncSetAttribute((const void*)gemm_mid_kernel<EPI, W8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  gemm_mid_kernel<EPI, W8><<<dim3(capped_grid((long)tiles_m * tiles_n), S), dim3(512), lds, st>>>(
       a.A, a.lda, a.W, a.bias, a.residual, a.ldr, a.C, a.ldc, a.M, a.N, a.K, tiles_m, tiles_n, a.partial, (nkt + S - 1) / S, a.wscale, raster_for(tiles_m), a.vq);
 }
-template <int BM, int EPI, int NST>
-static void launch_mid(const GemmArgs& a, hipStream_t st) { a.w_fp8 ? launch_mid_w<BM, EPI, NST, true>(a, st) : launch_mid_w<BM, EPI, NST, false>(a, st); }
+template <int EPI>
+static void launch_mid(const GemmArgs& a, hipStream_t st) { a.w_fp8 ? launch_mid_w<EPI, true>(a, st) : launch_mid_w<EPI, false>(a, st); }
 // The 64 x 128 tile.  Compute units left over by its blocks fetch weights ahead of them (strip_fetch): a block passes on some 50 B/ns and a step of the others takes
 // 0.32 us, so that N / 60 blocks (fp8: N / 120) keep ahead of them from the first step on; fewer take the k-tiles at the end that they reach in time, under two
-// fifths of them none (1456 x 1280, K 5120, us: none 33.5, 16 blocks 32.2, 26 28.8; all of 390 x 3584, K 3584 on 16 blocks 42, on 60 20.5, none 22.4).
+// fifths of them none (a run of its own, 1456 x 1280, K 5120, us: none 33.5, 16 blocks 32.2, 26 28.8; all of 390 x 3584, K 3584 on 16 blocks 42, on 60 20.5, none 22.4).
 static int strip_fetch_blocks(int tiles, int N, int S, int nkt, bool w8, int* fetch) {
   const int idle = get_grid_cap() > 0 ? 0 : (256 - tiles * S) / S;
   const long reach = (long)idle * (w8 ? 120 : 60) * nkt / N;      // k-tiles of a split
@@ -2137,7 +2138,7 @@ static void launch_tiled_bm(const GemmArgs& a, hipStream_t st) {
     if (tall_wanted(a)) return launch_tall<EPI>(a, st);
   }
   const int big = big_tile_rows(a, 1);
-  if (big == 129) return launch_mid<128, EPI, 4>(a, st);
+  if (big == 129) return launch_mid<EPI>(a, st);
   if (big == 272) return launch_vh<EPI>(a, st);
   if (big == 256) return launch_big<256, EPI>(a, st);
   if (big == 192) return launch_big<192, EPI>(a, st);
@@ -2165,7 +2166,7 @@ int gemm_plan(int M, int N, int K, int epilogue, int nsplit, bool w_fp8) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// skinny GEMV-like kernel (M <= 16; 17..64 rows with MG = 2..4 activation fragments per weight fragment): HBM-bound weight streaming
+// skinny GEMV-like kernel (M <= 64; MG = 1..4 activation fragments per weight fragment, two from ten rows on where a block takes several tiles): HBM-bound weight streaming
 // ------------------------------------------------------------------------------------------------
 // Block = 4 waves.  The block owns NTILE*16 consecutive W rows and the 64-element K chunks [c_begin, c_end) of split
 // blockIdx.y; wave w takes chunks c_begin + w, + 4, ...  W fragments go HBM -> VGPR -> MFMA (no LDS: each byte is used
@@ -2453,7 +2454,7 @@ void set_gemv_variant(int v) { g_gemv_variant = v; }
 
 template <int NTILE, int MODE, bool PACKED, int MG>
 static void launch_gemv_mg(dim3 grid, const GemmArgs& a, void* out, int ldo, int cps, hipStream_t st) {
-  if constexpr (MG > 1) {     // 17..64 rows: the two-stage pipeline with one chunk per stage (register budget: NTILE x MG accumulators + MG x fragments)
+  if constexpr (MG > 1) {     // 10..64 rows (the pair kernel: 9..64): the two-stage pipeline with one chunk per stage (register budget: NTILE x MG accumulators + MG x fragments)
     gemv_skinny_kernel<NTILE, MODE, PACKED, 1, 1, MG><<<grid, dim3(256), 0, st>>>(a.A, a.lda, a.W, a.ldw, a.bias, out, ldo, a.M, a.N, a.K, cps, a.tail);
     return;
   } else switch (g_gemv_variant) {
@@ -2790,7 +2791,7 @@ static int gemm_w8(const GemmArgs& a, hipStream_t st) {
   const bool tall = !part && !odd && tall_wanted(c);
   const int big = (g_gemm_variant == 7) ? 0 : big_tile_rows(c, part ? a.nsplit : 1, odd);
   if (odd && big != 256 && big != 128) return (a.ldc & 3) != 0 ? LCC_ERR_SHAPE : LCC_ERR_ALIGN;
-#define LCC_W8_TILE(EPI) (big == 256 ? launch_big<256, EPI>(c, st) : big == 192 ? launch_big<192, EPI>(c, st) : big == 160 ? launch_big<160, EPI>(c, st) : big == 128 ? launch_big<128, EPI>(c, st) : big == 129 ? launch_mid<128, EPI, 4>(c, st) : launch_mid64<EPI>(c, st))
+#define LCC_W8_TILE(EPI) (big == 256 ? launch_big<256, EPI>(c, st) : big == 192 ? launch_big<192, EPI>(c, st) : big == 160 ? launch_big<160, EPI>(c, st) : big == 128 ? launch_big<128, EPI>(c, st) : big == 129 ? launch_mid<EPI>(c, st) : launch_mid64<EPI>(c, st))
 #define LCC_W8(EPI) (tall ? launch_tall<EPI>(c, st) : LCC_W8_TILE(EPI))
   if (part) { LCC_W8_TILE(EPI_PARTIAL); return 0; }
   switch (a.epilogue) {
@@ -2833,7 +2834,7 @@ int gemm_bf16(const GemmArgs& a, hipStream_t st) {
     const bool narrow = all && (big == 129 || big == 0) && (get_grid_cap() <= 0 || tiles <= get_grid_cap());
     if (narrow) {
       g_launch_counts[LC_GEMM_VIT_QKV_NARROW]++;
-      big == 129 ? launch_mid_w<128, EPI_VIT_QKV, 4, false>(a, st) : launch_strip_w<EPI_VIT_QKV, false>(a, st);
+      big == 129 ? launch_mid_w<EPI_VIT_QKV, false>(a, st) : launch_strip_w<EPI_VIT_QKV, false>(a, st);
     } else if (all) launch_vit<EPI_VIT_QKV>(a, big, st);
     else if (qk) launch_vit<EPI_VIT_QK>(a, big, st);
     else launch_vit<EPI_VIT_V>(a, big, st);
@@ -2872,7 +2873,7 @@ int gemm_bf16(const GemmArgs& a, hipStream_t st) {
     else if (big == 192) launch_big<192, EPI_PARTIAL>(a, st);
     else if (big == 160) launch_big<160, EPI_PARTIAL>(a, st);
     else if (big == 128) launch_big<128, EPI_PARTIAL>(a, st);
-    else if (big == 129) launch_mid<128, EPI_PARTIAL, 4>(a, st);
+    else if (big == 129) launch_mid<EPI_PARTIAL>(a, st);
     else launch_tiled<64, EPI_PARTIAL>(a, st);
     return 0;
   }

@@ -271,8 +271,9 @@ struct LatentInArgs {            // behind the fused input projection: norms, ca
   bf16_t* const* kv_base = nullptr; size_t kv_off = 0;
 };
 int latent_norm_append(const LatentInArgs& a, hipStream_t st);
-// fused decode forms (decode_v2.hip; M <= 16): input projection + gate/up in one launch (sw.N = 0: none); query norm + up-projection with the rows'
+// fused decode forms (decode_v2.hip; M <= 12): input projection + gate/up in one launch (sw.N = 0: none); query norm + up-projection with the rows'
 // cache appends and gates behind it (dgemv_latent_q_ok: M <= 8, query rank <= 2048); output projection + fp32 residual + next norm
+constexpr int DGEMV_DECODER_ROWS = 12, DGEMV_MIXER_ROWS = 8;      // the most rows the layer-list decoders bring to these forms (the others: dgemv_f32 and below)
 int dgemv_in_swiglu(const DgArgs& in, const DgArgs& sw, hipStream_t st);
 bool dgemv_latent_q_ok(int M, int K);
 int dgemv_latent_q(const DgArgs& a, const LatentInArgs& row, hipStream_t st);
@@ -370,7 +371,7 @@ struct RecNormArgs {             // y -> gated norm over norm_groups equal parts
 };
 int rec_norm(const RecNormArgs& a, hipStream_t st);
 int gqa_merge_rec_norm(const GqaDecodeArgs& m, const RecNormArgs& a, hipStream_t st);
-// decode GEMVs with fp32 output (decode_v2.hip; M <= 16): one product, two independent products in one launch, gate/up with SwiGLU
+// decode GEMVs with fp32 output (decode_v2.hip; M <= 8): one product, two independent products in one launch, gate/up with SwiGLU
 int dgemv_f32(const DgArgs& a, hipStream_t st);
 int dgemv_f32_pair(const DgArgs& a, const DgArgs& b, hipStream_t st);
 int dgemv_swiglu(const DgArgs& a, hipStream_t st);

@@ -499,10 +499,10 @@ def test_wide_feed_forward_beside_the_input_projection(dev, ff, n):
 
 @pytest.mark.parametrize("width,ff,n", [(200, 8300, 9), (200, 8300, 16), (200, 8300, 17), (200, 8300, 48), (200, 8300, 64), (704, 7900, 33), (1600, 8300, 40), (200, 2200, 64), (200, 100, 32)])
 def test_one_launch_and_two_give_the_same_bits(dev, lib, width, ff, n):
-    """Input projection and gate/up of 9 to 64 rows, in one launch (counted) and in two: two, four and six weight tiles a block, one split and several."""
+    """Input projection and gate/up of 9 to 64 rows, in one launch (counted) and in two: two, four and six weight tiles a block, one split and two (width 1600)."""
     from livecc_amd import ops
     from livecc_amd.config import DebunexConfig
-    cfg = DebunexConfig(width, 100, [U.L(U.M(3, 40, 48, 72, 90, 0.2), ff), U.L(U.M(2, 64, 64, 800, 90, 0.2, 0), ff)], 1e-5, 20.0, name="pair")
+    cfg = DebunexConfig(100, width, [U.L(U.M(3, 40, 48, 72, 90, 0.2), ff), U.L(U.M(2, 64, 64, 800, 90, 0.2, 0), ff)], 1e-5, 20.0, name="pair")
     T = U.make_weights(cfg, 8)
     m = _model(cfg, T, dev, max_streams=n, max_kv_len=64, max_new_rows=512)
     seqs = [U.ids_of(cfg, 3 + i % 5, 50 + i) for i in range(n)]
