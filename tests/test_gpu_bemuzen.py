@@ -805,7 +805,7 @@ def test_many_streams_decode_in_groups(dev):
         got = m.forward_step([(s, [x[-j]], [0]) for s, x in zip(st, seqs)])
         for g, w in zip(got, wants):
             assert U.error(g, w[[-j]]) < U.LIMIT
-    for n in (17, 33, 48):                       # other batch sizes of the unfused decode step, from the middle of the streams
+    for n in (8, 9, 12, 16, 17, 33, 48):                       # other batch sizes: the last of the fused decode step, of the unfused one
         st2 = st[:n]
         got = m.forward_step([(s, [5], [0]) for s in st2])
         for k in range(n):
