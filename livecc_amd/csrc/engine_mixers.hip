@@ -161,7 +161,7 @@ int mixers_resolve_weights(lcc_engine* e, std::string* missing) {
 // S packed rows through every layer; pt null: a decode step over the streams `d_slots`.  On exit b.h holds the final norm of the residual.
 int run_mixer_layers(lcc_engine* e, const DecBuffers& b, int S, const PrefillTables* pt, const int32_t* d_slots, int nsplit_attn, const AttnDirect& direct, hipStream_t st) {
   // From nine rows on the products of 17 to 64 rows are the faster ones, launch for launch: their blocks pull the activations once for up to six weight tiles.  us a step, 28 layers, these
-  // launches / those, 9 / 12 / 16 rows: width 1536 1950 / 1865, 2114 / 1957, 2255 / 2009; width 3584 4172 / 4178, 4482 / 4298, 4898 / 4512
+  // launches / those, 9 / 12 / 16 rows: width 1536 1980 / 1898, 2127 / 1940, 2269 / 2027; width 3584 4164 / 4176, 4479 / 4302, 4902 / 4548
   const bool fused = !pt && S <= DGEMV_MIXER_ROWS && g_fused_decode;
   const int W = e->c.hidden_size, NL = (int)e->dl.size();
   if (e->llm_over) return fail(LCC_ERR_STATE, "per-layer input overrides are not available for this model family");
